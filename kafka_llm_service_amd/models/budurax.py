@@ -564,12 +564,16 @@ class BuduraxLM:
         xbc = torch.empty(T, C, dtype=dt, device=dev)
         hops.conv_silu(proj, inner, lw.conv, lw.conv_b, m.tok_seg, m.seg, state.conv[i], xbc)
         y = torch.empty(T, inner, dtype=torch.float32, device=dev)
-        plan = self._chunk_plan(m, Hh) if dev.type == "cuda" else None
-        if plan is not None:  # long prompt portions, few sequences: chunk-parallel scan
-            hops.ssm_scan_chunked(xbc, proj, inner + C, lw.dt_bias, lw.A_log, lw.D, Hh, P, N, G, plan, state.ssm[i], y)
+        a = (xbc, proj, inner + C, lw.dt_bias, lw.A_log, lw.D, Hh, P, N, G)
+        if hops.ssd_ok(xbc, Hh, P, N, G):
+            chunks, short = m.chunks(hops.SSD_CHUNK, hops.SSD_CHUNK_MIN)
+            hops.ssm_scan(*a, m.tok_seg, m.seg, state.ssm[i], y, chunks, short)
         else:
-            hops.ssm_scan(xbc, proj, inner + C, lw.dt_bias, lw.A_log, lw.D, Hh, P, N, G, m.tok_seg, m.seg,
-                          state.ssm[i], y)
+            plan = self._chunk_plan(m, Hh) if dev.type == "cuda" else None
+            if plan is not None:  # long prompt portions, few sequences: chunk-parallel scan
+                hops.ssm_scan_chunked(*a, plan, state.ssm[i], y)
+            else:
+                hops.ssm_scan(*a, m.tok_seg, m.seg, state.ssm[i], y)
         yn = torch.empty(T, inner, dtype=dt, device=dev)
         hops.gated_norm(y, proj, lw.mnorm, int(mm["norm_groups"]), self.cfg.norm_eps, yn)
         return self._lin(yn, lw.o, getattr(lw, "o_t", None))

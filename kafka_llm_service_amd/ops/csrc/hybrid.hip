@@ -870,7 +870,7 @@ template <typename AT, int RN, int RP, int TB>
 __global__ __launch_bounds__(256) void ssm_scan_kernel(const AT* __restrict__ xbc, int64_t xs, const AT* __restrict__ proj, int64_t ps,
                                 int dt_off, const float* __restrict__ dt_bias, const float* __restrict__ A_log,
                                 const float* __restrict__ Dp, int heads, int P, int N, int G, int TN, int TP, int NPS,
-                                const int* __restrict__ seg, float* __restrict__ state,
+                                const int* __restrict__ seg, int min_n, int max_n, float* __restrict__ state,
                                 float* __restrict__ y, int64_t ys) {
   extern __shared__ float sm[];
   const int nthr = blockDim.x, tid = threadIdx.x;
@@ -880,6 +880,7 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(const AT* __restrict__ xb
   b /= NPS;
   const int h = b % heads, sgi = b / heads;
   const int q0 = seg[4 * sgi], n = seg[4 * sgi + 1], p0s = seg[4 * sgi + 2], slot = seg[4 * sgi + 3];
+  if (n < min_n || n > max_n) return;   // (uniform)
   const int tp = tid % TP, tn = tid / TP;
   const bool active = tn < TN;
   const int pbase = psl * W, pw = min(W, P - pbase);
@@ -1030,7 +1031,7 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(const AT* __restrict__ xb
   }
 }
 
-// The recurrence for a step of single tokens (every segment one row: a decode step): one workgroup per (segment,
+// The recurrence for segments of one row (decoded tokens; longer segments are left alone): one workgroup per (segment,
 // head) streams the head's state through once - thread (g, p) owns column p and the rows n = g, g + NG, ... (the
 // state's rows are read and written as consecutive columns: coalesced) - and the NG partial outputs per column are
 // summed through LDS. No staging, no token loop: the state traffic is the whole cost.
@@ -1045,6 +1046,7 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(const AT* __restrict__ xb
   __shared__ float part[256];
   const int sgi = blockIdx.x / heads, h = blockIdx.x - sgi * heads;
   const int64_t row = seg[4 * sgi];
+  if (seg[4 * sgi + 1] != 1) return;   // (uniform)
   const int p0s = seg[4 * sgi + 2], slot = seg[4 * sgi + 3];
   const int tid = threadIdx.x, p = tid % P, g = tid / P;
   const int grp = h / (heads / G), inner = heads * P;
@@ -1381,21 +1383,24 @@ int kafka_hy_scan_groups(int P, int N) {
 
 hipError_t kafka_hy_ssm_scan(int f32, const void* xbc, int64_t xs, const void* proj, int64_t ps, int dt_off,
                              const float* dt_bias, const float* A_log, const float* Dp, int heads, int P, int N, int G,
-                             const int* seg, int R, int single, float* state, float* y, int64_t ys, hipStream_t st) {
+                             const int* seg, int R, int min_n, int max_n, float* state, float* y, int64_t ys,
+                             hipStream_t st) {
   if (R <= 0) return hipSuccess;
-  if (single && P <= 256) {  // every segment one row
+  if (min_n <= 1 && P <= 256) {  // the segments of one row
     const int NG = std::max(1, std::min(256 / P, N));
     DISPATCH_AT(f32, ssm_step_kernel<AT><<<R * heads, P * NG, 0, st>>>((const AT*)xbc, xs, (const AT*)proj, ps, dt_off,
                                                                       dt_bias, A_log, Dp, heads, P, N, G, NG, seg,
                                                                       state, y, ys));
-    return hipGetLastError();
+    min_n = 2;
   }
+  if (max_n < min_n) return hipGetLastError();
   ScanPlan sp;
   if (!scan_plan(P, N, (int64_t)R * heads, &sp)) return hipErrorInvalidValue;
   DISPATCH_AT(f32, {
     auto a = [&](auto k) {
       k<<<R * heads * sp.NPS, sp.threads, sp.lds, st>>>((const AT*)xbc, xs, (const AT*)proj, ps, dt_off, dt_bias, A_log,
-                                                        Dp, heads, P, N, G, sp.TN, sp.TP, sp.NPS, seg, state, y, ys);
+                                                        Dp, heads, P, N, G, sp.TN, sp.TP, sp.NPS, seg, min_n, max_n, state, y,
+                                                        ys);
     };
     if (sp.TB == 8) a(ssm_scan_kernel<AT, 8, 4, 8>);
     else if (sp.TB == 4) a(ssm_scan_kernel<AT, 8, 4, 4>);

@@ -41,7 +41,14 @@ hipError_t kafka_hy_short_conv(int f32, const void* proj, int64_t ps, int c0, co
 int kafka_hy_scan_groups(int P, int N);
 hipError_t kafka_hy_ssm_scan(int f32, const void* xbc, int64_t xs, const void* proj, int64_t ps, int dt_off,
                              const float* dt_bias, const float* A_log, const float* Dp, int heads, int P, int N, int G,
-                             const int* seg, int R, int single, float* state, float* y, int64_t ys, hipStream_t st);
+                             const int* seg, int R, int min_n, int max_n, float* state, float* y, int64_t ys,
+                             hipStream_t st);
+int kafka_hy_ssd_chunk();
+int kafka_hy_ssd_ok(int H, int P, int N, int G, int64_t xs);
+int64_t kafka_hy_ssd_scratch(int P, int N);
+hipError_t kafka_hy_ssd_scan(const void* xbc, int64_t xs, const void* dt, int64_t ds, const float* dt_bias,
+                             const float* A_log, const float* Dp, int H, int P, int N, int G, const int* vseg, int n_chunks,
+                             const int* cs, int R, float* scratch, float* state, float* y, int64_t ys, hipStream_t st);
 hipError_t kafka_hy_ssm_combine(int f32, const void* proj, int64_t ps, int dt_off, const float* dt_bias,
                                 const float* A_log, int heads, int NP_, const int* vseg, const int* cs, int S,
                                 float* tmp, float* state, hipStream_t st);
@@ -484,12 +491,15 @@ void short_conv(at::Tensor proj, int64_t c0, at::Tensor w, OptT b, at::Tensor to
                              (int)residual, stream()));
 }
 
+// ``cs`` given: ``seg`` is the chunk table of the segments of ``cs``, which run on the matrix cores; else the segments of
+// min_n .. max_n rows, token by token
 void ssm_scan(at::Tensor xbc, at::Tensor proj, int64_t dt_off, at::Tensor dt_bias, at::Tensor A_log, at::Tensor D,
-              int64_t heads, int64_t P, int64_t N, int64_t G, at::Tensor seg, at::Tensor state, at::Tensor y) {
+              int64_t heads, int64_t P, int64_t N, int64_t G, at::Tensor seg, at::Tensor state, at::Tensor y, int64_t min_n,
+              int64_t max_n, OptT cs) {
   rows2d(xbc, "xbc"); rows2d(proj, "proj"); rows2d(y, "y");
   const int f32 = act_f32(xbc);
   same_act(f32, {&proj});
-  const int64_t T = xbc.size(0);
+  const int64_t T = xbc.size(0), R = seg.size(0);
   TORCH_CHECK(heads > 0 && G > 0 && heads % G == 0 && xbc.size(1) == heads * P + 2 * G * N && proj.size(0) == T &&
                   dt_off >= 0 && dt_off + heads <= proj.size(1), "ssm_scan: sizes");
   for (const at::Tensor* t : {&dt_bias, &A_log, &D})
@@ -500,13 +510,28 @@ void ssm_scan(at::Tensor xbc, at::Tensor proj, int64_t dt_off, at::Tensor dt_bia
   TORCH_CHECK(state.is_cuda() && state.scalar_type() == at::kFloat && state.is_contiguous() && state.dim() == 4 &&
                   state.size(1) == heads && state.size(2) == N && state.size(3) == P,
               "ssm_scan: state fp32 [slots, heads, N, P]");
-  TORCH_CHECK(y.scalar_type() == at::kFloat && y.size(0) == T && y.size(1) == heads * P, "ssm_scan: y fp32 [T, inner]");
+  TORCH_CHECK(y.is_cuda() && y.scalar_type() == at::kFloat && y.size(0) == T && y.size(1) == heads * P,
+              "ssm_scan: y fp32 [T, inner]");
+  float *Sp = state.data_ptr<float>(), *yp = y.data_ptr<float>();
+  if (cs.has_value()) {
+    TORCH_CHECK(cs->is_cuda() && cs->scalar_type() == at::kInt && cs->is_contiguous() && cs->dim() == 2 &&
+                    cs->size(1) == 4, "ssm_scan: cs int32 [n, 4]");
+    TORCH_CHECK(!f32 && kafka_hy_ssd_ok((int)heads, (int)P, (int)N, (int)G, xbc.stride(0)) && y.stride(0) % 4 == 0 &&
+                    (reinterpret_cast<uintptr_t>(xbc.data_ptr()) & 15) == 0 && (reinterpret_cast<uintptr_t>(yp) & 15) == 0,
+                "ssm_scan: sizes not supported in chunks");
+    at::Tensor scratch = at::empty({R * heads * kafka_hy_ssd_scratch((int)P, (int)N)}, state.options());
+    HY_HIP(kafka_hy_ssd_scan(xbc.data_ptr(), xbc.stride(0), (const at::BFloat16*)proj.data_ptr() + dt_off, proj.stride(0),
+                             dt_bias.data_ptr<float>(), A_log.data_ptr<float>(), D.data_ptr<float>(), (int)heads, (int)P,
+                             (int)N, (int)G, seg.data_ptr<int>(), (int)R, cs->data_ptr<int>(), (int)cs->size(0),
+                             scratch.data_ptr<float>(), Sp, yp, y.stride(0), stream()));
+    return;
+  }
   TORCH_CHECK(kafka_hy_scan_groups((int)P, (int)N) > 0, "ssm_scan: state of ", N, " x ", P, " per head is not supported");
+  if (T == R) max_n = std::min<int64_t>(max_n, 1);   // every segment one row
   HY_HIP(kafka_hy_ssm_scan(f32, xbc.data_ptr(), xbc.stride(0), proj.data_ptr(), proj.stride(0), (int)dt_off,
                            dt_bias.data_ptr<float>(), A_log.data_ptr<float>(), D.data_ptr<float>(), (int)heads, (int)P,
-                           (int)N, (int)G, seg.data_ptr<int>(), (int)seg.size(0), (int)(T == seg.size(0)),
-                           state.data_ptr<float>(),
-                           y.data_ptr<float>(), y.stride(0), stream()));
+                           (int)N, (int)G, seg.data_ptr<int>(), (int)R, (int)min_n,
+                           (int)std::min<int64_t>(max_n, 0x7fffffff), Sp, yp, y.stride(0), stream()));
 }
 
 // vseg int32 [V, 4] chunk table (first row, rows, -, scratch slot); cs int32 [S, 4] = (first chunk, chunks, first
@@ -1317,7 +1342,11 @@ void kafka_bind_hybrid(pybind11::module_& m) {
         py::arg("tok_seg"), py::arg("positions"), py::arg("scale"), py::arg("out"), py::arg("window") = 0,
         py::arg("sink") = py::none());
   m.def("hy_short_conv", &short_conv);
-  m.def("hy_ssm_scan", &ssm_scan);
+  m.def("hy_ssm_scan", &ssm_scan, py::arg("xbc"), py::arg("proj"), py::arg("dt_off"), py::arg("dt_bias"), py::arg("A_log"),
+        py::arg("D"), py::arg("heads"), py::arg("P"), py::arg("N"), py::arg("G"), py::arg("seg"), py::arg("state"),
+        py::arg("y"), py::arg("min_n") = 1, py::arg("max_n") = 0x7fffffff, py::arg("cs") = py::none());
+  m.def("hy_ssd_chunk", []() { return kafka_hy_ssd_chunk(); });
+  m.def("hy_ssd_ok", [](int H, int P, int N, int G, int64_t xs) { return kafka_hy_ssd_ok(H, P, N, G, xs) != 0; });
   m.def("hy_ssm_combine", &ssm_combine);
   m.def("hy_gated_norm", &gated_norm);
   m.def("hy_scan_groups", [](int P, int N) { return kafka_hy_scan_groups(P, N); });

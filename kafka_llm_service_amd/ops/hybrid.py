@@ -177,14 +177,38 @@ def short_conv(u, c0: int, w, b, tok_seg, seg, state, out, act: str = "none", re
         ref.short_conv(u, c0, w, b, tok_seg, seg, state, out, act, residual)
 
 
-def ssm_scan(xbc, proj, dt_off: int, dt_bias, A_log, D, heads, P, N, G, tok_seg, seg, state, y) -> None:
+SSD_CHUNK = 128         # tokens of a chunk (the kernels' constant)
+# segments of at least this many rows are scanned in chunks: 128 heads of 128 x 64, one segment of 16 / 24 / 32 / 128 rows,
+# chunks against token by token: 34 / 35 / 35 / 43 us against 32 / 41 / 50 / 155 us; four segments 61 / 62 / 63 / 73 against
+# 57 / 71 / 86 / 305 us
+SSD_CHUNK_MIN = 24
+
+
+def ssd_ok(xbc, heads: int, P: int, N: int, G: int) -> bool:
+    """bf16 GPU rows of sizes the chunked state-space kernels take (state rows a multiple of 16 up to 256, columns of 8)."""
+    return xbc.is_cuda and xbc.dtype == torch.bfloat16 and xbc.data_ptr() % 16 == 0 and \
+        bool(ext().hy_ssd_ok(int(heads), int(P), int(N), int(G), xbc.stride(0)))
+
+
+def ssm_scan(xbc, proj, dt_off: int, dt_bias, A_log, D, heads, P, N, G, tok_seg, seg, state, y, chunks=None,
+             rows=(1, 1 << 30)) -> None:
     """Mamba-2 recurrence per (segment, head): S <- exp(-exp(A_log) dt) S + dt B x^T, y = S^T C + D x, with
-    dt = softplus(raw dt + bias); fp32 state [slots, heads, N, P] read (unless the segment starts at 0) and left."""
-    if _gpu(xbc):
-        ext().hy_ssm_scan(xbc, proj, int(dt_off), dt_bias, A_log, D, int(heads), int(P), int(N), int(G), seg, state,
-                          y)
-    else:
+    dt = softplus(raw dt + bias); fp32 state [slots, heads, N, P] read (unless the segment starts at 0) and left.
+    ``chunks``: device tensors of ``chunk_tables(seg_host, SSD_CHUNK, SSD_CHUNK_MIN)`` - where the sizes allow (``ssd_ok``)
+    their segments run in chunks (the same recurrence as matrix products, re-associated: fp32 rounding only), the others
+    token by token. ``rows``: the shortest and the longest of those others (None: there are none)."""
+    if not _gpu(xbc):
         ref.ssm_scan(xbc, proj, dt_off, dt_bias, A_log, D, heads, P, N, G, tok_seg, seg, state, y)
+        return
+    a = (xbc, proj, int(dt_off), dt_bias, A_log, D, int(heads), int(P), int(N), int(G))
+    if chunks is not None:
+        if ssd_ok(xbc, heads, P, N, G):
+            ext().hy_ssm_scan(*a, chunks[0], state, y, cs=chunks[1])
+            rows = (rows[0], min(rows[1], SSD_CHUNK_MIN - 1)) if rows is not None else None
+        else:
+            rows = (1, 1 << 30)
+    if rows is not None:
+        ext().hy_ssm_scan(*a, seg, state, y, int(rows[0]), int(rows[1]))
 
 
 def chunk_tables(seg_host, chunk: int, min_rows: int):

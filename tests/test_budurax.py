@@ -716,3 +716,64 @@ def test_trace_runner_command_line(tmp_path):
     assert rel_err(got[0], b.oracle(t)[[0, 8]]) < TOL["float32"]
     assert rel_err(got[1], b.oracle(u)[[5]]) < TOL["float32"]
     assert rel_err(got[2], b.oracle(t)[[20]]) < TOL["float32"]
+
+
+def _ssm_want(xbc, raw, dt_bias, A_log, D, Hh, P, N, G, S):
+    """The recurrence in float64 over one sequence from state S [Hh, N, P]: (rows [T, Hh P], last state)."""
+    grp, rows = torch.arange(Hh) // (Hh // G), []
+    x, B, C = (t.double() for t in xbc.split([Hh * P, G * N, G * N], 1))
+    dt = torch.nn.functional.softplus(raw.double() + dt_bias.double(), threshold=1e9)
+    for t in range(xbc.shape[0]):
+        Bt, Ct, xt = B[t].view(G, N)[grp], C[t].view(G, N)[grp], x[t].view(Hh, P)
+        S = torch.exp(-torch.exp(A_log.double()) * dt[t])[:, None, None] * S + dt[t][:, None, None] * Bt[:, :, None] * xt[:, None]
+        rows.append((torch.einsum("hnp,hn->hp", S, Ct) + D.double()[:, None] * xt).reshape(-1))
+    return torch.stack(rows), S
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hh,P,N,G", [(4, 64, 128, 2), (2, 8, 16, 1), (6, 72, 144, 3), (2, 40, 256, 2), (3, 136, 80, 1)])
+@pytest.mark.parametrize("fast", [False, True])
+def test_scan_in_matrix_core_chunks(Hh, P, N, G, fast):
+    """Segments of 1 .. 300 rows, fresh in slots of NaN and from stored states, in one launch: those of at least
+    SSD_CHUNK_MIN rows in chunks on the matrix cores, the others token by token. ``fast``: decays of up to e^-40 a token, a
+    chunk's running sum in the thousands. The fp32 factors of the products keep all their bits, so a row's error is bounded by
+    the fp32 additions of up to 300 terms: 300 * 2^-24 = 1.8e-5 of the row's largest partial sum, which the bound 2e-5 of the
+    head's largest value stands for - and it is no larger than twice the token-by-token kernel's (plus 1e-6)."""
+    device = "cuda:0"
+    torch.manual_seed(P + N)
+    runs = [(300, 0, 0), (1, 0, 1), (hops.SSD_CHUNK_MIN, 0, 2), (hops.SSD_CHUNK_MIN - 1, 7, 3), (128, 3, 4), (129, 0, 5),
+            (127, 9, 6), (1, 5, 7)]
+    T, inner = sum(r[0] for r in runs), Hh * P
+    xbc = (torch.randn(T, inner + 2 * G * N) / 2).bfloat16()
+    proj = torch.randn(T, Hh + 3).bfloat16()
+    A_log, D = torch.rand(Hh) * 2 + (1.5 if fast else -1.0), torch.randn(Hh)
+    dt_bias = torch.randn(Hh) / 2 + (0.0 if fast else -3.0)
+    state0 = torch.full((8, Hh, N, P), float("nan"))
+    for _, p0, slot in runs:
+        if p0:
+            state0[slot] = torch.randn(Hh, N, P)
+    seg, ts = _seg("cpu", runs)
+    want_y, want_S, at = [], [], 0
+    for n, p0, slot in runs:
+        S = state0[slot].double() if p0 else torch.zeros(Hh, N, P, dtype=torch.float64)
+        y, S = _ssm_want(xbc[at:at + n], proj[at:at + n, 3:], dt_bias, A_log, D, Hh, P, N, G, S)
+        want_y.append(y)
+        want_S.append(S)
+        at += n
+    want_y = torch.cat(want_y).view(T, Hh, P)
+    tabs = tuple(torch.from_numpy(t).to(device) for t in hops.chunk_tables(seg.numpy(), hops.SSD_CHUNK, hops.SSD_CHUNK_MIN))
+    xg = xbc.to(device)
+    assert hops.ssd_ok(xg, Hh, P, N, G)
+    errs = []
+    for chunks, rows in ((tabs, (1, hops.SSD_CHUNK_MIN - 1)), (None, (1, 1 << 30))):
+        state, y = state0.clone().to(device), torch.full((T, inner), float("nan"), device=device)
+        hops.ssm_scan(xg, proj.to(device), 3, dt_bias.to(device), A_log.to(device), D.to(device), Hh, P, N, G, ts.to(device),
+                      seg.to(device), state, y, chunks, rows)
+        d = (y.cpu().double().view(T, Hh, P) - want_y).abs().amax(-1) / want_y.abs().amax((0, 2))
+        ds = max(((state[slot].cpu().double() - S).abs().amax() / S.abs().amax()).item()
+                 for (_, _, slot), S in zip(runs, want_S))
+        errs.append((d.max().item(), ds))
+        assert not torch.isnan(y).any()
+    print(errs)
+    assert errs[0][0] < 2e-5 and errs[0][1] < 2e-5
+    assert errs[0][0] < 2 * errs[1][0] + 1e-6 and errs[0][1] < 2 * errs[1][1] + 1e-6

@@ -32,6 +32,7 @@ import math
 from dataclasses import dataclass, field
 from pathlib import Path
 
+import numpy as np
 import torch
 import torch.nn.functional as F
 
@@ -249,11 +250,27 @@ class SegMeta:
                     rows = rows[rows < min_rows]
                 short = (int(rows.min()), int(rows.max())) if len(rows) else None
                 if tabs is not None:
-                    n = tabs[0].size
-                    up = torch.cat([torch.from_numpy(t).view(-1) for t in tabs]).to(self.seg.device)
-                    tabs = (up[:n].view(-1, 4), up[n:].view(-1, 4))
+                    tabs = self.upload(tabs)
             self.cache[key] = (tabs, short)
         return self.cache[key]
+
+    def portions(self, window: int):
+        """``hops.portion_tables`` of the step with its tables on the device, built once per step."""
+        key = ("portions", window)
+        if key not in self.cache:
+            t = hops.portion_tables(self.seg_host, window)
+            self.cache[key] = None if t is None else t[:2] + self.upload(t[2:])
+        return self.cache[key]
+
+    def upload(self, tables) -> tuple:
+        """int32 numpy tables on the step's device, by one copy that the host does not wait for."""
+        up = torch.from_numpy(np.concatenate([t.reshape(-1) for t in tables])).pin_memory().to(self.seg.device,
+                                                                                               non_blocking=True)
+        out, at = [], 0
+        for t in tables:
+            out.append(up[at:at + t.size].view(t.shape))
+            at += t.size
+        return tuple(out)
 
 
 @dataclass
@@ -270,6 +287,31 @@ class RecurrentState:
 
 class _Layer:
     pass
+
+
+def latent_mix(q, q_rot, cache, cache_t, lw, inp, m: SegMeta, ao, window: int = 0, sink=None, gate=None) -> None:
+    """Latent attention of a step's rows: ao [T, H vdim] from q [T, H, dim] and the rotated q_rot [T, H, rot_dim], times
+    sigmoid(gate) when given. Decoded tokens attend in the latent space (q_lat = W_uk^T q, out = W_uv (sum p c)), prompt
+    portions on expanded keys and values where the sizes allow."""
+    T, H, D = q.shape
+    R, Dv = lw.uk_h.shape[2], lw.uv_ht.shape[2]
+    tables = m.portions(window) if cache_t is not None and lw.scale > 0 and hops.latent_rows_ok(q, q_rot, cache, Dv) else None
+    n = T if tables is None else tables[0]        # rows that stay in the latent space
+    if n:
+        q_lat = torch.bmm(q[:n].transpose(0, 1), lw.uk_h)                         # [H, n, R]
+        o_lat = torch.empty(H, n, R, dtype=q.dtype, device=q.device)
+        tiles, keys = m.tiles.get(hops.tile_tokens(H)), m.max_keys
+        if n < T:
+            tiles, keys = tiles[:n], int(m.seg_host[:n, 2].max()) + 1             # (single tokens: a tile each)
+        hops.latent_attn(q_lat, q_rot[:n], cache, m.block_tables, m.tok_seg[:n], m.seg, inp.positions[:n], lw.scale, o_lat,
+                         cache_t, tiles, keys, window=window, sink=sink)
+        if gate is None:
+            torch.bmm(o_lat, lw.uv_ht, out=ao[:n].view(n, H, Dv).transpose(0, 1))  # head h -> its vdim columns
+        else:
+            hops.sigmoid_mul(torch.bmm(o_lat, lw.uv_ht), gate[:n], ao[:n])
+    if n < T:
+        hops.latent_attn_portions(q, q_rot, cache, lw.uk_h.view(H * D, R), lw.uv, tables, m.block_tables, lw.scale, ao, window,
+                                  sink, gate)
 
 
 class BuduraxLM:
@@ -402,6 +444,7 @@ class BuduraxLM:
                 t = W[p + "mix.uv"].to(device=dev, dtype=dt).view(H, vd, R).transpose(1, 2).contiguous()
                 self._tensors.append(t)
                 lw.uv_ht = t                                                       # out = o_lat @ uv_ht (per head)
+                lw.uv = act(p + "mix.uv")                                          # v = c @ uv^T (prompt portions)
                 lw.o = act(p + "mix.o")
                 lw.scale = float(m["scale"])
                 lw.rot_dims = int(m["rot"]["dims"])
@@ -531,14 +574,9 @@ class BuduraxLM:
         q_rot = torch.empty(T, H, rd, dtype=dt, device=dev)
         hops.latent_prep(qgd, H, D, rd, R, lw.dkv_off, lw.dkv_norm, self.cfg.norm_eps, inp.positions, lw.cos_sin,
                          lw.rot_dims, cache, inp.slot_mapping, q_rot, cache_t if lw.kv_from is None else None)
-        q_u = qgd[:, :H * (D + rd)].view(T, H, D + rd)[:, :, :D].transpose(0, 1)  # [H, T, dim] (strided view)
-        q_lat = torch.bmm(q_u, lw.uk_h)                                           # [H, T, R]
-        o_lat = torch.empty(H, T, R, dtype=dt, device=dev)
-        hops.latent_attn(q_lat, q_rot, cache, m.block_tables, m.tok_seg, m.seg, inp.positions, lw.scale, o_lat,
-                         cache_t, m.tiles.get(hops.tile_tokens(H)), m.max_keys)
-        a = torch.bmm(o_lat, lw.uv_ht)                                            # [H, T, vdim]
         ao = torch.empty(T, H * vd, dtype=dt, device=dev)
-        hops.sigmoid_mul(a, qgd[:, lw.g_off:lw.g_off + H * vd], ao)
+        latent_mix(qgd[:, :H * (D + rd)].view(T, H, D + rd)[:, :, :D], q_rot, cache, cache_t, lw, inp, m, ao,
+                   gate=qgd[:, lw.g_off:lw.g_off + H * vd])
         return self._lin(ao, lw.o, getattr(lw, "o_t", None))
 
     def _chunk_plan(self, m: SegMeta, heads: int):

@@ -46,7 +46,7 @@ import torch
 import torch.nn.functional as F
 
 from kafka_llm_service_amd import ops
-from kafka_llm_service_amd.models.budurax import SegMeta, rotary_table
+from kafka_llm_service_amd.models.budurax import SegMeta, latent_mix, rotary_table
 from kafka_llm_service_amd.ops import hybrid as hops
 
 PAGE = 16
@@ -347,6 +347,7 @@ class FurapelLM:
                 lw.dkv_norm = act(q + "dkv.norm")
                 lw.uk_h = act(q + "uk").view(H, D, R)                              # q_lat = q @ uk_h  (per head)
                 lw.uv_ht = keep(W[q + "uv"].to(device=dev, dtype=dt).view(H, Dv, R).transpose(1, 2))
+                lw.uv = act(q + "uv")
                 lw.scale = float(m["scale"])
                 tiles.add(hops.tile_tokens(H))
             else:
@@ -507,13 +508,8 @@ class FurapelLM:
         q_rot = torch.empty(T, H, 0, dtype=dt, device=dev)                         # (no rotated part in this family)
         hops.latent_prep(qd, H, D, 0, R, H * D, lw.dkv_norm, self.cfg.norm_eps, inp.positions, None, 0, cache,
                          inp.slot_mapping, q_rot, cache_t)
-        q_u = qd[:, :H * D].view(T, H, D).transpose(0, 1)                          # [H, T, dim] (strided view)
-        q_lat = torch.bmm(q_u, lw.uk_h)                                            # [H, T, R]
-        o_lat = torch.empty(H, T, R, dtype=dt, device=dev)
-        hops.latent_attn(q_lat, q_rot, cache, m.block_tables, m.tok_seg, m.seg, inp.positions, lw.scale, o_lat,
-                         cache_t, m.tiles.get(hops.tile_tokens(H)), m.max_keys, window=lw.window)
         ao = torch.empty(T, H * Dv, dtype=dt, device=dev)
-        torch.bmm(o_lat, lw.uv_ht, out=ao.view(T, H, Dv).transpose(0, 1))          # head h -> its vdim columns
+        latent_mix(qd[:, :H * D].view(T, H, D), q_rot, cache, cache_t, lw, inp, m, ao, window=lw.window)
         return self._lin(ao, lw.o, getattr(lw, "o_t", None), slabs=True)
 
     def _mlstm(self, lw, h, m: SegMeta, st: dict) -> torch.Tensor:

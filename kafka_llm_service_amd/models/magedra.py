@@ -58,7 +58,7 @@ import torch
 import torch.nn.functional as F
 
 from kafka_llm_service_amd import ops
-from kafka_llm_service_amd.models.budurax import SegMeta, rotary_table
+from kafka_llm_service_amd.models.budurax import SegMeta, latent_mix, rotary_table
 from kafka_llm_service_amd.ops import hybrid as hops
 
 PAGE = 16
@@ -410,6 +410,7 @@ class MagedraLM:
                 lw.dkv_norm = act(p + "mix.dkv.norm")
                 lw.uk_h = act(p + "mix.uk").view(H, D, R)                          # q_lat = q @ uk_h  (per head)
                 lw.uv_ht = keep(W[p + "mix.uv"].to(device=dev, dtype=dt).view(H, Dv, R).transpose(1, 2))
+                lw.uv = act(p + "mix.uv")
                 lw.o = act(p + "mix.o")
                 lw.scale = float(m["scale"])
                 lw.cos_sin = self._rot_table(rot)
@@ -596,13 +597,8 @@ class MagedraLM:
                          inp.slot_mapping, q_rot)
         hops.latent_prep(first, 0, D, rd, R, Rq, lw.dkv_norm, self.cfg.norm_eps, inp.positions, lw.cos_sin,
                          lw.rot_dims, cache, inp.slot_mapping, q_rot[:, :0], cache_t)
-        q_u = q.view(T, H, D + rd)[:, :, :D].transpose(0, 1)                      # [H, T, dim] (strided view)
-        q_lat = torch.bmm(q_u, lw.uk_h)                                           # [H, T, R]
-        o_lat = torch.empty(H, T, R, dtype=dt, device=dev)
-        hops.latent_attn(q_lat, q_rot, cache, m.block_tables, m.tok_seg, m.seg, inp.positions, lw.scale, o_lat,
-                         cache_t, m.tiles.get(hops.tile_tokens(H)), m.max_keys)
         ao = torch.empty(T, H * Dv, dtype=dt, device=dev)
-        torch.bmm(o_lat, lw.uv_ht, out=ao.view(T, H, Dv).transpose(0, 1))         # head h -> its vdim columns
+        latent_mix(q.view(T, H, D + rd)[:, :, :D], q_rot, cache, cache_t, lw, inp, m, ao)
         return self._lin(ao, lw.o, getattr(lw, "o_t", None))
 
 

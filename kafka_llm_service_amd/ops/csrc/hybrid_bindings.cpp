@@ -43,6 +43,13 @@ hipError_t kafka_hy_ssm_scan(int f32, const void* xbc, int64_t xs, const void* p
                              const float* dt_bias, const float* A_log, const float* Dp, int heads, int P, int N, int G,
                              const int* seg, int R, int min_n, int max_n, float* state, float* y, int64_t ys,
                              hipStream_t st);
+int kafka_hy_latent_rows_ok(int R, int rd, int D, int Dv);
+hipError_t kafka_hy_latent_gather(const void* cache, int R, int rd, const int* bt, int bt_stride, const int* px,
+                                  const int* blocks, int n_blocks, void* ck, void* kr, hipStream_t st);
+hipError_t kafka_hy_latent_rows(const void* q, int64_t q_t, int64_t q_h, const void* q_rot, int64_t qr_t, int64_t qr_h,
+                                const void* K, const void* kr, const void* Vt, int64_t M, const int* px, const int* tiles,
+                                int n_tiles, int H, int rd, float scale, int window, const float* sink, const void* gate,
+                                int64_t gs, void* out, int64_t os, hipStream_t st);
 int kafka_hy_ssd_chunk();
 int kafka_hy_ssd_ok(int H, int P, int N, int G, int64_t xs);
 int64_t kafka_hy_ssd_scratch(int P, int N);
@@ -468,6 +475,62 @@ void latent_attn_mfma(at::Tensor q_lat, at::Tensor q_rot, at::Tensor cache, at::
                                    (int)items.size(0), positions.data_ptr<int64_t>(), (float)scale, out.data_ptr(),
                                    out.stride(0), out.stride(1), (int)H, (int)nsplit, pop, pmlp, (int)T, (int)window,
                                    sink_ptr(sink, H), stream()));
+}
+
+// latent attention of prompt portions on expanded keys and values: px int32 [n, 8], blocks int32 [M / 64], tiles int32 [m, 4]
+void i32_table(const at::Tensor& t, int64_t cols, const char* what) {
+  TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::kInt && t.is_contiguous() &&
+                  (cols ? t.dim() == 2 && t.size(1) == cols : t.dim() == 1), what, ": int32 table");
+}
+
+void latent_gather(at::Tensor cache, int64_t rd, at::Tensor bt, at::Tensor px, at::Tensor blocks, at::Tensor ck,
+                   at::Tensor kr) {
+  for (const at::Tensor* t : {&cache, &ck, &kr})
+    TORCH_CHECK(t->is_cuda() && t->scalar_type() == at::kBFloat16 && t->is_contiguous(), "latent_gather: bf16 GPU tensors");
+  i32_table(px, 8, "portions"); i32_table(blocks, 0, "blocks");
+  const int64_t M = ck.size(0);
+  TORCH_CHECK(cache.dim() == 3 && cache.size(1) == 16 && rd >= 0 && rd % 8 == 0 && cache.size(2) % 8 == 0 && ck.dim() == 2 &&
+                  ck.size(1) == cache.size(2) - rd && kr.dim() == 2 && kr.size(0) == M && kr.size(1) == rd &&
+                  M == 64 * blocks.size(0), "latent_gather: shapes");
+  TORCH_CHECK(bt.is_cuda() && bt.scalar_type() == at::kInt && bt.dim() == 2 && bt.stride(1) == 1, "latent_gather: block table");
+  HY_HIP(kafka_hy_latent_gather(cache.data_ptr(), (int)ck.size(1), (int)rd, bt.data_ptr<int>(), (int)bt.stride(0),
+                                px.data_ptr<int>(), blocks.data_ptr<int>(), (int)blocks.size(0), ck.data_ptr(),
+                                kr.data_ptr(), stream()));
+}
+
+void latent_rows(at::Tensor q, at::Tensor q_rot, at::Tensor k, at::Tensor kr, at::Tensor vt, at::Tensor px, at::Tensor tiles,
+                 double scale, int64_t window, OptT sink, OptT gate, at::Tensor out) {
+  for (const at::Tensor* t : {&q, &q_rot, &k, &kr, &vt, &out})
+    TORCH_CHECK(t->is_cuda() && t->scalar_type() == at::kBFloat16, "latent_rows: bf16 GPU tensors");
+  auto al = [](const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; };
+  TORCH_CHECK(q.dim() == 3 && q_rot.dim() == 3 && q.stride(2) == 1, "latent_rows: q [T, H, dim], q_rot [T, H, rot_dim]");
+  const int64_t T = q.size(0), H = q.size(1), D = q.size(2), rd = q_rot.size(2), M = k.size(0);
+  rows2d(out, "out");
+  i32_table(px, 8, "portions"); i32_table(tiles, 4, "tiles");
+  TORCH_CHECK(vt.dim() == 2 && vt.is_contiguous() && vt.size(1) == M && vt.size(0) % H == 0 && k.is_contiguous() &&
+                  k.dim() == 2 && k.size(1) == H * D && kr.is_contiguous() && kr.dim() == 2 && kr.size(0) == M &&
+                  kr.size(1) == rd && q_rot.size(0) == T && q_rot.size(1) == H && M % 64 == 0, "latent_rows: shapes");
+  const int64_t Dv = vt.size(0) / H;
+  TORCH_CHECK(kafka_hy_latent_rows_ok(32, (int)rd, (int)D, (int)Dv), "latent_rows: sizes not supported");
+  TORCH_CHECK(out.size(0) == T && out.size(1) == H * Dv && out.stride(0) % 8 == 0 && al(out) && al(q) && al(k) && al(vt) &&
+                  q.stride(0) % 8 == 0 && q.stride(1) % 8 == 0, "latent_rows: output shape or alignment");
+  TORCH_CHECK(rd == 0 || (q_rot.stride(2) == 1 && q_rot.stride(0) % 8 == 0 && q_rot.stride(1) % 8 == 0 && al(q_rot) && al(kr)),
+              "latent_rows: rotated part alignment");
+  TORCH_CHECK(window >= 0 && scale > 0.0, "latent_rows: window, scale");
+  const void* gp = nullptr;
+  int64_t gs = 0;
+  if (gate.has_value()) {
+    rows2d(*gate, "gate");
+    TORCH_CHECK(gate->scalar_type() == at::kBFloat16 && gate->is_cuda() && gate->size(0) == T && gate->size(1) >= H * Dv &&
+                    gate->stride(0) % 4 == 0 && (reinterpret_cast<uintptr_t>(gate->data_ptr()) & 7) == 0,
+                "latent_rows: gate");
+    gp = gate->data_ptr();
+    gs = gate->stride(0);
+  }
+  HY_HIP(kafka_hy_latent_rows(q.data_ptr(), q.stride(0), q.stride(1), q_rot.data_ptr(), q_rot.stride(0), q_rot.stride(1),
+                              k.data_ptr(), kr.data_ptr(), vt.data_ptr(), M, px.data_ptr<int>(), tiles.data_ptr<int>(),
+                              (int)tiles.size(0), (int)H, (int)rd, (float)scale, (int)window, sink_ptr(sink, H), gp, gs,
+                              out.data_ptr(), out.stride(0), stream()));
 }
 
 void short_conv(at::Tensor proj, int64_t c0, at::Tensor w, OptT b, at::Tensor tok_seg, at::Tensor seg,
@@ -1345,6 +1408,9 @@ void kafka_bind_hybrid(pybind11::module_& m) {
   m.def("hy_ssm_scan", &ssm_scan, py::arg("xbc"), py::arg("proj"), py::arg("dt_off"), py::arg("dt_bias"), py::arg("A_log"),
         py::arg("D"), py::arg("heads"), py::arg("P"), py::arg("N"), py::arg("G"), py::arg("seg"), py::arg("state"),
         py::arg("y"), py::arg("min_n") = 1, py::arg("max_n") = 0x7fffffff, py::arg("cs") = py::none());
+  m.def("hy_latent_rows_ok", [](int R, int rd, int D, int Dv) { return kafka_hy_latent_rows_ok(R, rd, D, Dv) != 0; });
+  m.def("hy_latent_gather", &latent_gather);
+  m.def("hy_latent_rows", &latent_rows);
   m.def("hy_ssd_chunk", []() { return kafka_hy_ssd_chunk(); });
   m.def("hy_ssd_ok", [](int H, int P, int N, int G, int64_t xs) { return kafka_hy_ssd_ok(H, P, N, G, xs) != 0; });
   m.def("hy_ssm_combine", &ssm_combine);

@@ -150,6 +150,82 @@ def latent_attn(q_lat, q_rot, cache, block_tables, tok_seg, seg, positions, scal
         ref.latent_attn(q_lat, q_rot, cache, block_tables, tok_seg, seg, positions, scale, out, window, sink)
 
 
+# Rows of a step's longest portion from which its portions attend on expanded keys and values (H = 32, 512 / 64 / 128 / 128,
+# us with the products around it, expanded against latent space): fresh portions of 128 / 512 / 2048 rows 52 / 74 / 178 against
+# 50 / 140 / 1170; behind 2000 keys 64 / 128 / 512 rows 176 / 189 / 201 against 132 / 304 / 632; behind 8000 keys 64 rows 539
+# against 313 (a tile walks its keys alone). With a window of 1024 keys the two are level at 64 rows.
+LATENT_ROWS_MIN = 96
+LATENT_ROWS_CHAIN = 2048  # keys that a portion of fewer rows may walk beside it, if more than the long portions' own
+LATENT_ROWS_KEYS = 64   # (kernel constants) keys of a block ...
+LATENT_ROWS_TILE = 128  # ... and rows of a workgroup
+LATENT_ROWS_MAX = 1 << 17   # gathered rows of a step beyond which it stays in the latent space (the expanded keys' memory)
+
+
+def latent_rows_ok(q, q_rot, cache, Dv: int) -> bool:
+    """Whether prompt portions can attend on expanded keys and values (``latent_attn_portions``): bf16 GPU rows q [T, H, dim]
+    and q_rot [T, H, rot_dim] in 16-byte pieces, dim = vdim = 128, rot_dim 0 or 64."""
+    if not (q.is_cuda and q.dtype == torch.bfloat16 and cache.dtype == torch.bfloat16 and cache.shape[1] == 16):
+        return False
+    D, rd = q.shape[2], q_rot.shape[2]
+    return all(t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 and t.stride(2) == 1
+               for t in ((q, q_rot) if rd else (q,))) and bool(ext().hy_latent_rows_ok(cache.shape[2] - rd, rd, D, int(Dv)))
+
+
+def portion_tables(seg_host, window: int):
+    """Tables of ``latent_attn_portions`` for a step: (rows in front of them, gathered rows, portions int32 [n, 8], portion of
+    every 64 gathered rows, tiles int32 [m, 4]) as numpy, or None when the step has no portion of LATENT_ROWS_MIN rows. The
+    single tokens in front (a plan's decoded rows) are left to ``latent_attn``."""
+    import numpy as np
+
+    if seg_host is None or not len(seg_host):
+        return None
+    rows = seg_host[:, 1]
+    first = int(np.argmax(rows > 1)) if (rows > 1).any() else len(rows)
+    if first == len(rows) or int(rows[first:].max()) < LATENT_ROWS_MIN:
+        return None
+    keys = seg_host[first:, 1] + seg_host[first:, 2]
+    if window:
+        keys = np.minimum(keys, rows[first:] + window)
+    if int(keys.max()) > max(LATENT_ROWS_CHAIN, int(keys[rows[first:] >= LATENT_ROWS_MIN].max())):
+        return None
+    px, blocks, tiles, at = [], [], [], 0
+    for j, (q0, n, p0, _) in enumerate(seg_host[first:].tolist()):
+        klo = max(0, p0 - window + 1) // LATENT_ROWS_KEYS * LATENT_ROWS_KEYS if window else 0
+        nb = -(-(p0 + n - klo) // LATENT_ROWS_KEYS)
+        px.append((q0, n, p0, klo, at, first + j, p0 + n, 0))
+        blocks += [j] * nb
+        at += nb * LATENT_ROWS_KEYS
+        for r in range(0, n, LATENT_ROWS_TILE):
+            e = p0 + min(n, r + LATENT_ROWS_TILE)
+            tiles.append((max(0, p0 + r - window + 1) - e if window else -e, j, r))
+    if at > LATENT_ROWS_MAX:
+        return None
+    tiles.sort(key=lambda t: t[0])   # most keys first
+    return (int(seg_host[first, 0]), at, np.asarray(px, dtype=np.int32), np.asarray(blocks, dtype=np.int32),
+            np.asarray([(j, r, 0, 0) for _, j, r in tiles], dtype=np.int32))
+
+
+def latent_attn_portions(q, q_rot, cache, w_k, w_v, tables, block_tables, scale: float, out, window: int = 0, sink=None,
+                         gate=None) -> None:
+    """Attention of a step's prompt portions over their sequences' cached [latent | rotated key] rows with the heads' keys and
+    values expanded: k = W_k c, v = W_v c (W_k [H dim, kv_rank], W_v [H vdim, kv_rank]),
+    out[t, h] = sum_j softmax_j((q[t, h] . k_j + q_rot[t, h] . kr_j) scale) v_j over the keys j <= position[t] (with ``window``
+    the last so many of them), times sigmoid(gate[t]) when given. q [T, H, dim], q_rot [T, H, rot_dim], out and gate
+    [T, >= H vdim]; ``tables``: ``portion_tables`` on the device - only their rows are read and written. ``sink`` as in
+    ``latent_attn``.
+
+    Against the latent space (2 kv_rank + rot_dim channels a score and kv_rank a value, 3.4 times the products at 512 / 64 /
+    128 / 128) a portion pays kv_rank x (dim + vdim) per key of its context once."""
+    _, M, px, blocks, tiles = tables
+    rd, R = q_rot.shape[2], w_k.shape[1]
+    ck = torch.empty(M, R, dtype=q.dtype, device=q.device)
+    kr = torch.empty(M, rd, dtype=q.dtype, device=q.device)
+    ext().hy_latent_gather(cache, rd, block_tables, px, blocks, ck, kr)
+    k = torch.nn.functional.linear(ck, w_k)       # [M, H dim]
+    vt = torch.nn.functional.linear(w_v, ck)      # [H vdim, M]
+    ext().hy_latent_rows(q, q_rot, k, kr, vt, px, tiles, float(scale), int(window), sink, gate, out)
+
+
 def sigmoid_mul(a, g, out) -> None:
     if _gpu(a):
         ext().hy_sigmoid_mul(a, g, out)

@@ -777,3 +777,83 @@ def test_scan_in_matrix_core_chunks(Hh, P, N, G, fast):
     print(errs)
     assert errs[0][0] < 2e-5 and errs[0][1] < 2e-5
     assert errs[0][0] < 2 * errs[1][0] + 1e-6 and errs[0][1] < 2 * errs[1][1] + 1e-6
+
+
+def test_portion_tables():
+    """Which rows attend on expanded keys: none without a portion of LATENT_ROWS_MIN rows, else everything behind the leading
+    single tokens; blocks of 64 gathered rows per portion, tiles of 128 rows with the most keys first."""
+    seg = _seg("cpu", [(1, 5, 0), (1, 9, 1), (200, 0, 2), (3, 1000, 3), (1, 77, 4)])[0].numpy()
+    first, M, px, blocks, tiles = hops.portion_tables(seg, 0)
+    assert (first, M) == (2, 64 * (4 + 16 + 2))
+    assert px.tolist() == [[2, 200, 0, 0, 0, 2, 200, 0], [202, 3, 1000, 0, 256, 3, 1003, 0], [205, 1, 77, 0, 1280, 4, 78, 0]]
+    assert blocks.tolist() == [0] * 4 + [1] * 16 + [2] * 2
+    assert tiles.tolist() == [[1, 0, 0, 0], [0, 128, 0, 0], [0, 0, 0, 0], [2, 0, 0, 0]]
+    first, M, px, blocks, tiles = hops.portion_tables(seg, 100)
+    assert px[:, 3].tolist() == [0, 896, 0] and M == 64 * (4 + 2 + 2) and tiles[0].tolist() == [0, 128, 0, 0]
+    short = _seg("cpu", [(1, 5, 0), (hops.LATENT_ROWS_MIN - 1, 0, 1)])[0].numpy()
+    assert hops.portion_tables(short, 0) is None and hops.portion_tables(seg[:2], 0) is None
+    assert hops.portion_tables(None, 0) is None
+    # a few rows behind a long history beside it: the whole step stays in the latent space
+    far = hops.LATENT_ROWS_CHAIN
+    for p0, none in ((far - 3, False), (far - 2, True)):
+        seg = _seg("cpu", [(hops.LATENT_ROWS_MIN, 0, 0), (3, p0, 1)])[0].numpy()
+        assert (hops.portion_tables(seg, 0) is None) == none and hops.portion_tables(seg, 50) is not None
+    assert hops.portion_tables(_seg("cpu", [(hops.LATENT_ROWS_MIN, far, 0), (3, far, 1)])[0].numpy(), 0) is not None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,rd,window,extras", [(8, 64, 0, True), (3, 0, 0, False), (16, 0, 70, True), (5, 64, 200, False),
+                                                (8, 0, 1, False)])
+def test_attention_of_portions_on_expanded_keys(H, rd, window, extras):
+    """Portions whose rows and keys end inside, at and one past a tile (128 rows) and a block (64 keys), fresh and behind
+    histories, scattered pages, beside single tokens that must stay untouched; with a sink and a gate. Against float64 on the
+    same bf16 keys and values: the weights' and the output's rounding to bf16 move a value by at most 2^-9 of the largest |v|
+    each (a gate shrinks both), the fp32 sums by far less."""
+    device, R, D, Dv = "cuda:0", 96, 128, 128
+    torch.manual_seed(H + window)
+    runs = [(1, 40, 0), (129, 0, 1), (64, 0, 2), (33, 95, 3), (128, 64, 4), (1, 130, 5), (300, 37, 6)]
+    T = sum(r[0] for r in runs)
+    seg, _ = _seg("cpu", runs)
+    W = -(-max(n + p for n, p, _ in runs) // 16)
+    bt = torch.randperm(len(runs) * W).view(len(runs), W).int()
+    cache = torch.full((len(runs) * W, 16, R + rd), float("nan"), dtype=torch.bfloat16)
+    rows = []
+    for j, (n, p0, _) in enumerate(runs):
+        c = torch.randn(p0 + n, R + rd).bfloat16()
+        c[-1] *= 3
+        rows.append(c)
+        for i in range(p0 + n):
+            cache[bt[j, i // 16], i % 16] = c[i]
+    q, q_rot = torch.randn(T, H, D).bfloat16(), torch.randn(T, H, rd).bfloat16()
+    w_k, w_v = (torch.randn(H * D, R) / R ** 0.5).bfloat16(), (torch.randn(H * Dv, R) / R ** 0.5).bfloat16()
+    sink = torch.randn(H) * 3 if extras else None
+    gate = torch.randn(T, H * Dv + 8).bfloat16() if extras else None
+    scale = (D + rd) ** -0.5
+    want, vmax, at = torch.zeros(T, H, Dv, dtype=torch.float64), 0.0, 0
+    for j, (n, p0, _) in enumerate(runs):
+        c = rows[j][:, :R].to(device)
+        k = torch.nn.functional.linear(c, w_k.to(device)).cpu().double().view(-1, H, D)
+        v = torch.nn.functional.linear(c, w_v.to(device)).cpu().double().view(-1, H, Dv)
+        kr = rows[j][:, R:].double()
+        s = torch.einsum("thd,shd->hts", q[at:at + n].double(), k) + torch.einsum("thd,sd->hts", q_rot[at:at + n].double(), kr)
+        dist = torch.arange(p0, p0 + n)[:, None] - torch.arange(p0 + n)
+        s = (s * scale).masked_fill((dist < 0) | (dist >= window if window else dist < 0), float("-inf"))
+        if sink is not None:
+            s = torch.cat([s, sink.double()[:, None, None].expand(H, n, 1)], 2)
+            v = torch.cat([v, torch.zeros(1, H, Dv, dtype=torch.float64)])
+        want[at:at + n] = torch.einsum("hts,shd->thd", torch.softmax(s, -1), v)
+        vmax = max(vmax, v.abs().max().item())
+        at += n
+    if gate is not None:
+        want = want * torch.sigmoid(gate[:, :H * Dv].double()).view(T, H, Dv)
+    t = hops.portion_tables(seg.numpy(), window)
+    tabs = t[:2] + tuple(torch.from_numpy(x).to(device) for x in t[2:])
+    assert t[0] == 1
+    out = torch.full((T, H * Dv), 7.0, dtype=torch.bfloat16, device=device)
+    qg, qr = q.to(device), q_rot.to(device)
+    assert hops.latent_rows_ok(qg, qr, cache.to(device), Dv)
+    hops.latent_attn_portions(qg, qr, cache.to(device), w_k.to(device), w_v.to(device), tabs, bt.to(device), scale, out,
+                              window, sink.to(device) if extras else None, gate.to(device)[:, :H * Dv] if extras else None)
+    got = out.cpu().double().view(T, H, Dv)
+    assert (got[:1] == 7).all()
+    assert (got[1:] - want[1:]).abs().max().item() < 1.1 * 2 ** -8 * vmax

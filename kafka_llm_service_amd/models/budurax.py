@@ -370,7 +370,7 @@ class BuduraxLM:
                 ops.stream_plan(M, w.shape[0], w.shape[1]) is not None:
             y = ops.linear_stream(x, wt)
             return ops.slab_reduce(y) if ops.is_slab(y) else y
-        return F.linear(x, w)
+        return ops.linear_dense(x, w)
 
     def weight_bytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self._tensors)

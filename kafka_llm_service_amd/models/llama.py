@@ -210,7 +210,7 @@ class TransformerLM:
                 return ops.linear_stream(x, wt, max_splits)
             if kind in SKINNY and ops.skinny_plan(M, wt.shape[0] * 32, x.shape[1], max_splits):
                 return ops.linear_skinny(x, wt, max_splits)
-        return F.linear(x, self._dense(w, wt))
+        return ops.linear_dense(x, self._dense(w, wt))
 
     @staticmethod
     def _dense(w: torch.Tensor | None, wt: torch.Tensor | None, glu: bool = False) -> torch.Tensor:

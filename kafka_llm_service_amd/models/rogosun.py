@@ -305,7 +305,7 @@ class RogosunLM:
         if self._streams(x.shape[0], w, wt):
             y = ops.linear_stream(x, wt)
             return ops.slab_reduce(y) if ops.is_slab(y) and not slabs else y
-        return F.linear(x, w)
+        return ops.linear_dense(x, w)
 
     def weight_bytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self._tensors)

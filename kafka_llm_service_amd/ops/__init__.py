@@ -236,6 +236,25 @@ def untile_weight(wt: torch.Tensor, glu: bool = False) -> torch.Tensor:
     return wt.reshape(nb, kb, 2, 32, 8).permute(0, 3, 1, 2, 4).reshape(nb * 32, kb * 16)
 
 
+# A library product of up to this many output columns is cut into blocks of this many rows: 4096 x 4096 outputs are one round
+# of 256 x 256 tiles over the 256 CUs, and the few tiles of the rows beyond it are a second round that takes as long as the
+# first. Library alone against blocks, N = 4096, us: K = 14336, 4099 rows 722 / 328, 5500 rows 852 / 457, 7000 rows 656 / 558;
+# K = 8192, 4099 rows 244 / 194; K = 4096, 4099 rows 131 / 111, 7000 rows 160 / 168; 8192 rows level. Wider outputs gain
+# nothing on average (28672 columns: 692 / 715 at 4099 rows).
+DENSE_BLOCK = 4096
+
+
+def linear_dense(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ w^T (bf16 [M, K] x [N, K], prefill-sized M) on hipBLASLt, in row blocks where one call would leave the chip idle."""
+    M, N = x.shape[0], w.shape[0]
+    if not _gpu(x) or M <= DENSE_BLOCK or N > DENSE_BLOCK or x.dtype != torch.bfloat16:
+        return torch.nn.functional.linear(x, w)
+    y = torch.empty(M, N, dtype=x.dtype, device=x.device)
+    for a in range(0, M, DENSE_BLOCK):
+        torch.mm(x[a:a + DENSE_BLOCK], w.t(), out=y[a:a + DENSE_BLOCK])
+    return y
+
+
 # Steps of up to this many rows run the dense projections on the weight-streaming kernel (csrc/wstream_gemm.hip).
 # The kernel takes up to 256 rows: one 192-row tile (MT = 6) up to 192, beyond that two row tiles of 128 sharing each
 # weight slice through the MALL, where it loses to hipBLASLt (gate_up 101 vs 66 us at 168..248 rows; bench 7,359 vs

@@ -840,3 +840,15 @@ def test_cascade_pass_with_new_turn_rows(cuda):
             p_ = torch.softmax(s_, -1)
             o_ref[t, h * G:(h + 1) * G] = p_ @ vv[:pos + 1, h].float()
     _close(out, o_ref, atol=0.02, msg="new-turn rows through the cascade pass")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N", [(ops.DENSE_BLOCK, 256), (ops.DENSE_BLOCK + 1, 256), (2 * ops.DENSE_BLOCK + 3, 64)])
+def test_linear_dense_blocks(M, N):
+    """Row blocks give the rows of the whole product: bf16 results of the same fp32 sums, so each lies within half an ulp
+    (2^-9 of itself) of the fp32 product, plus its sums' rounding over K = 512 terms of size ~1 (2^-24 * 512 / 2)."""
+    torch.manual_seed(M)
+    x, w = torch.randn(M, 512, device="cuda:0").bfloat16(), torch.randn(N, 512, device="cuda:0").bfloat16()
+    want = x.float() @ w.float().t()
+    got = ops.linear_dense(x, w).float()
+    assert ((got - want).abs() <= 2 ** -8 * want.abs() + 1e-2).all()

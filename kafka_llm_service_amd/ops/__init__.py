@@ -576,8 +576,9 @@ def grouped_stream_combine(a: torch.Tensor, wt: torch.Tensor, r: "MoERouting", T
 
 
 def grouped_wide(x: torch.Tensor, wt: torch.Tensor, r: "MoERouting", epilogue: str, gather: bool,
-                 out: torch.Tensor | None = None, limit: float = 0.0, alpha: float = 1.0) -> torch.Tensor:
-    """The expert products of a long step on wave-tiled expert weights (128-row tiles; K % 128 == 0, N % 64 == 0).
+                 out: torch.Tensor | None = None, limit: float = 0.0, alpha: float = 1.0, tile: int = 0) -> torch.Tensor:
+    """The expert products of a long step on wave-tiled expert weights (K % 128 == 0, N % 64 == 0). ``tile``: rows of a tile,
+    128 or (N % 128 == 0) 256; 0 = by the sizes.
     ``epilogue``: "glu" (``tile_experts(w13, glu=True)``; silu(gate) * up, or with a limit the clamped form, [n_ent,
     N/2]), "relu2" (relu squared, [n_ent, N]), "combine" (out[token] += w * row, out f32 [T, N] zeroed by the caller) or
     "rows" (w * row, [n_ent, N], entry order).
@@ -589,7 +590,7 @@ def grouped_wide(x: torch.Tensor, wt: torch.Tensor, r: "MoERouting", epilogue: s
         y = torch.empty(n_ent, N // 2 if epilogue == "glu" else N, dtype=x.dtype, device=x.device)
     if _gpu(x):
         ext().grouped_wide(x, wt, r.perm_tok, r.perm_w, r.expert_off, bool(gather),
-                           ("glu", "relu2", "combine", "rows").index(epilogue), y, out, float(limit), float(alpha))
+                           ("glu", "relu2", "combine", "rows").index(epilogue), y, out, float(limit), float(alpha), int(tile))
         return out if y is None else y
     if epilogue == "combine":
         ref.grouped_gemm(x, untile_experts(wt), r.perm_tok, r.perm_w, r.expert_off, 0, gather, None, out)

@@ -88,7 +88,7 @@ hipError_t kafka_launch_moe_sort(const float* topk_w, const int* topk_e, int n, 
 hipError_t kafka_launch_grouped_wide(const bf16* X, int64_t ldx, const bf16* Wt, int E, int N, int K,
                                      const int* perm_tok, const float* perm_w, const int* expert_off, int n_ent,
                                      int gather, int epi, bf16* Y, int64_t ldy, float* out, int64_t ldo,
-                                     float glu_limit, float glu_alpha, hipStream_t st);
+                                     float glu_limit, float glu_alpha, int bm, hipStream_t st);
 int kafka_narrow_ok(int N, int K, int64_t xs);
 int kafka_narrow_max_k();
 hipError_t kafka_launch_narrow_linear(const bf16* x, int64_t xs, const bf16* w, const float* bias, int N, int K,
@@ -758,7 +758,7 @@ static void wstream_grouped(at::Tensor x, at::Tensor wt, at::Tensor perm_tok, at
 // Expert ids were in [0, E) when the entries were sorted, so perm_tok / expert_off stay inside x and wt.
 static void grouped_wide(at::Tensor x, at::Tensor wt, at::Tensor perm_tok, at::Tensor perm_w, at::Tensor expert_off,
                          bool gather, int64_t epi, c10::optional<at::Tensor> y, c10::optional<at::Tensor> out,
-                         double glu_limit, double glu_alpha) {
+                         double glu_limit, double glu_alpha, int64_t bm) {
   CHECK_CUDA(x); CHECK_DT(x, at::kBFloat16); CHECK_DT(wt, at::kBFloat16); CHECK_LASTDIM(x);
   CHECK_DT(perm_tok, at::kInt); CHECK_DT(perm_w, at::kFloat); CHECK_DT(expert_off, at::kInt);
   TORCH_CHECK(x.dim() == 2 && x.stride(0) % 8 == 0 && (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) == 0,
@@ -783,7 +783,7 @@ static void grouped_wide(at::Tensor x, at::Tensor wt, at::Tensor perm_tok, at::T
   }
   CHECK_HIP(kafka_launch_grouped_wide(bptr(x), x.stride(0), bptr(wt), (int)E, (int)N, (int)K, perm_tok.data_ptr<int>(),
                                       perm_w.data_ptr<float>(), expert_off.data_ptr<int>(), (int)n_ent, gather ? 1 : 0,
-                                      (int)epi, yp, ldy, op, ldo, (float)glu_limit, (float)glu_alpha, cur_stream()));
+                                      (int)epi, yp, ldy, op, ldo, (float)glu_limit, (float)glu_alpha, (int)bm, cur_stream()));
 }
 
 static void narrow_args(const at::Tensor& x, const at::Tensor& w) {
@@ -1159,7 +1159,9 @@ PYBIND11_MODULE(_kafka_ops, m) {
   m.def("ep_dispatch", &ep_dispatch);
   m.def("ep_recv_route", &ep_recv_route);
   m.def("ep_combine", &ep_combine);
-  m.def("grouped_wide", &grouped_wide);
+  m.def("grouped_wide", &grouped_wide, py::arg("x"), py::arg("wt"), py::arg("perm_tok"), py::arg("perm_w"),
+        py::arg("expert_off"), py::arg("gather"), py::arg("epi"), py::arg("y"), py::arg("out"), py::arg("glu_limit"),
+        py::arg("glu_alpha"), py::arg("bm") = 0);
   m.def("narrow_linear", &narrow_linear);
   m.def("narrow_route", &narrow_route);
   m.def("narrow_ok", [](int N, int K, int64_t xs) { return kafka_narrow_ok(N, K, xs) != 0; });

@@ -10,6 +10,7 @@
 //                  Epilogues: silu(gate) * up or its clamped form on GLU-interleaved tiles (a wave holds both tiles of a
 //                  pair), relu squared, the weighted combine into fp32 rows, or the weighted rows as they are (in entry
 //                  order; their consumer gathers a token's rows through the sort's inverse, no atomics).
+//   grouped_ring   the same for experts of more rows: 256 x 256 tiles, both operands through a ring in LDS
 //   moe_sort       stable sort of (token, choice) entries by expert, one workgroup: every wave counts and then places
 //                  its stretch of the entries 64 at a time, equal experts found by ballots over the bits of their ids
 //   narrow         fp32 products of bf16 rows with up to 64 bf16 weight rows (router logits, gate projections): 16 rows a
@@ -32,7 +33,7 @@ enum { EPI_GLU = 0, EPI_RELU2 = 1, EPI_COMBINE = 2, EPI_ROWS = 3 };
 __device__ __forceinline__ int xoff(int r, int c) { return r * BK + 8 * (c ^ (r & 7)); }
 
 // item -> (expert, row tile, column tile) over the experts' segments; false past the last item. Every wave does this.
-__device__ __forceinline__ bool find_item(const int* expert_off, int E, int ntn, int& e, int& rt, int& nt) {
+__device__ __forceinline__ bool find_item(const int* expert_off, int E, int ntn, int BM, int& e, int& rt, int& nt) {
   const int lane = threadIdx.x & 63;
   // all items, in waves of 64 experts: the total first, then this workgroup's place
   int total = 0;
@@ -62,8 +63,11 @@ __device__ __forceinline__ bool find_item(const int* expert_off, int E, int ntn,
       const int before = base + __shfl(incl - t, l, 64), tiles = __shfl(t, l, 64) / ntn;
       e = __builtin_amdgcn_readfirstlane(b + l);
       const int i = __builtin_amdgcn_readfirstlane(item - before), ti = __builtin_amdgcn_readfirstlane(tiles);
-      nt = i / ti;
-      rt = i - nt * ti;
+      // row tiles of up to 2048 rows side by side, then the next column tile, then the next 2048 rows: what an XCD's 32
+      // CUs work on at once is about as many rows as columns
+      const int gr = 2048 / BM, g = i / (gr * ntn), j = i - g * gr * ntn, in_g = min(gr, ti - g * gr);
+      nt = j / in_g;
+      rt = g * gr + (j - nt * in_g);
       return true;
     }
     base += __shfl(incl, 63, 64);
@@ -82,7 +86,7 @@ __global__ __launch_bounds__(256, 2) void grouped_wide_kernel(const bf16* __rest
                                                               float glu_alpha) {
   __shared__ __attribute__((aligned(16))) bf16 xs[2][BM * BK];
   int e, rt, nt;
-  if (!find_item(expert_off, E, (N + BN - 1) / BN, e, rt, nt)) return;   // (uniform)
+  if (!find_item(expert_off, E, (N + BN - 1) / BN, BM, e, rt, nt)) return;   // (uniform)
   const int seg0 = expert_off[e] + rt * BM, rows = min(BM, expert_off[e + 1] - seg0);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 31, h = lane >> 5;
   const int nb = (nt * 4 + w) * 2;                 // this wave's two 32-column tiles
@@ -184,6 +188,210 @@ __global__ __launch_bounds__(256, 2) void grouped_wide_kernel(const bf16* __rest
           al = glu_alpha;
         }
         Y[(int64_t)ent * ldy + (nb >> 1) * 32 + r] = (bf16)(g / (1.0f + __expf(-al * g)) * u);
+      }
+    }
+}
+
+// ---- the same on 256 x 256 tiles through a ring in LDS ---------------------------------------------------------------
+// Four waves of 128 x 128 (one workgroup per CU): an operand byte read from LDS feeds four products instead of the two of
+// the kernel above, and a byte from the cache twice as many. Activations and weights arrive by LDS-DMA, 32 deep, in a ring of
+// five stages: three or four are in flight while one is multiplied (a miss under load takes longer than a stage), one counted
+// wait and one barrier per stage; a wave reads a stage's fragments while it multiplies the one before. 16x16x32 products: the
+// matrix cores alone reach 1.89 PFLOP/s on them at one wave per SIMD, 1.47 on 32x32x16. A weight piece is a whole 1 KB tile of
+// 32 x 16 in lane order; the activations' 16-byte pieces are permuted at the source so that eight neighbouring rows of a
+// fragment lie in different banks.
+// Measured, us against the kernel above (random routing and values): 32768 entries of 16 experts, 4096 -> 5376 relu2 1303 /
+// 1654, 5376 -> 4096 rows 1306 / 1682 (1.1 PFLOP/s); 3800 of 8, 4096 -> 2 x 14336 glu 855 / 1007, 14336 -> 4096 combine
+// 450 / 564; 5386 of 8, 4096 -> 2 x 4608 glu 462 / 533, 4608 -> 4096 rows 264 / 284; one product of 8192^3 859 / 1186 (1.28
+// PFLOP/s). With the loads and reads of a stage in front of its products instead of between them 1507 and 1575 us for the first
+// two; 32x32x16 products the same way 1568 and 1646.
+namespace ring {
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_t;
+constexpr int BM = 256, BK = 32, NS = 5, KB = BK / 16;
+constexpr int XB = BM * BK * 2, STAGE = XB + BN * BK * 2;   // bytes
+constexpr int DX = XB / 1024 / 4, DW = BN * BK * 2 / 1024 / 4, DPS = DX + DW;   // 1 KB pieces a wave moves per stage
+constexpr int LGKM0 = 0xC07F;   // s_waitcnt lgkmcnt(0) alone, in a form that the compiler counts too
+
+__device__ __forceinline__ int xslot(int row, int c) { return c ^ ((row >> 1) & 3); }
+
+// c += a b in an accumulation register: left to itself the compiler moves sums between the two register files in the loop.
+// (Operands come from LDS, so their waits are the compiler's; two products on one sum are 64 products apart.)
+__device__ __forceinline__ void mfma16(f32x4v& c, bf16x8 a, bf16x8 b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+
+template <bool B>
+struct Full {
+  static constexpr bool value = B;
+};
+
+template <int N>
+__device__ __forceinline__ void vmcnt() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+}  // namespace ring
+
+template <bool GATHER, int EPI>
+__global__ __launch_bounds__(256, 1) void grouped_ring_kernel(const bf16* __restrict__ X, int64_t ldx,
+                                                              const bf16x8* __restrict__ Wt, int E, int N, int K,
+                                                              const int* __restrict__ perm_tok,
+                                                              const float* __restrict__ perm_w,
+                                                              const int* __restrict__ expert_off,
+                                                              bf16* __restrict__ Y, int64_t ldy,
+                                                              float* __restrict__ out, int64_t ldo, float glu_limit,
+                                                              float glu_alpha) {
+  using namespace ring;
+  __shared__ __attribute__((aligned(1024))) char smem[NS * STAGE];
+  int e, rt, nt;
+  if (!find_item(expert_off, E, (N + BN - 1) / BN, ring::BM, e, rt, nt)) return;   // (uniform)
+  const int seg0 = expert_off[e] + rt * ring::BM, rows = min(ring::BM, expert_off[e + 1] - seg0);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, q = lane >> 4;
+  const int wr = w >> 1, wc = w & 1;
+  const int nb = nt * 8 + 4 * wc;                  // this wave's first 32-column tile (N is a multiple of 128)
+  const int K16 = K >> 4, nst = K / ring::BK;
+  const bf16* xsrc[DX];
+  const bf16x8* wsrc[DW];
+#pragma unroll
+  for (int u = 0; u < DX; ++u) {
+    const int row = 16 * (DX * w + u) + (lane >> 2);
+    const int ent = seg0 + min(row, rows - 1);     // rows past the segment reload a valid row, never stored
+    xsrc[u] = X + (GATHER ? (int64_t)perm_tok[ent] : (int64_t)ent) * ldx + 8 * xslot(row, lane & 3);
+  }
+#pragma unroll
+  for (int u = 0; u < DW; ++u) {
+    const int j = DW * w + u, t = min(nt * 8 + j / KB, (N >> 5) - 1);   // (tiles past N reload the last, never stored)
+    wsrc[u] = Wt + (((int64_t)e * (N >> 5) + t) * K16 + j % KB) * 64 + lane;
+  }
+  auto issue_piece = [&](int s, int slot, int u) {
+    char* base = smem + slot * STAGE;
+    if (u < DX)
+      __builtin_amdgcn_global_load_lds(xsrc[u] + (int64_t)s * ring::BK, (lds_t*)(base + (DX * w + u) * 1024), 16, 0, 0);
+    else
+      __builtin_amdgcn_global_load_lds(wsrc[u - DX] + (int64_t)s * KB * 64,
+                                       (lds_t*)(base + XB + (DW * w + u - DX) * 1024), 16, 0, 0);
+  };
+  auto issue = [&](int s, int slot) {
+#pragma unroll
+    for (int u = 0; u < DPS; ++u) issue_piece(s, slot, u);
+  };
+  f32x4v acc[8][8];
+#pragma unroll
+  for (int a = 0; a < 8; ++a)
+#pragma unroll
+    for (int b = 0; b < 8; ++b) acc[a][b] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  // where this lane's fragments lie in a stage: rows 16 i + r, 8-deep piece q; columns 16 j + r, piece q of tile j / 2
+  const int xa = (128 * wr + r) * (2 * ring::BK) + 16 * xslot(r, q);   // (row bits above 2 leave the slot alone)
+  const int wa = XB + (4 * wc * KB + (q >> 1)) * 1024 + ((q & 1) * 32 + r) * 16;
+  auto read_pair = [&](bf16x8& a, bf16x8& b, int slot, int i) {
+    const char* base = smem + slot * STAGE;
+    a = *reinterpret_cast<const bf16x8*>(base + xa + i * 16 * 2 * ring::BK);
+    b = *reinterpret_cast<const bf16x8*>(base + wa + (i >> 1) * KB * 1024 + (i & 1) * 256);
+  };
+  // stage s has been read by this wave; stage s + 1 arrives, the ring takes stage s + NS in stage s's place
+  auto turn = [&](int s) {
+    const int later = min(NS - 2, nst - 2 - s);    // stages behind s + 1 that may be in flight
+    if (later >= 3) vmcnt<3 * DPS>();
+    else if (later == 2) vmcnt<2 * DPS>();
+    else if (later == 1) vmcnt<DPS>();
+    else vmcnt<0>();
+    asm volatile("s_barrier" ::: "memory");
+  };
+  bf16x8 a0[8], b0[8], a1[8], b1[8];
+  // (K is a multiple of 128: an even number of stages, at least NS - 1)
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s) issue(s, s);
+  turn(-1);
+  if (NS - 1 < nst) issue(NS - 1, NS - 1);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) read_pair(a0[i], b0[i], 0, i);
+  int slot = 0;
+  // Between the eight groups of eight products go the next stage's reads and the ring's next pieces, one of each: a wave
+  // issues in order, and all of them in front of the products would leave the matrix core waiting for the load path.
+  // ``full``: the ring stays full (s + NS < nst), no conditions in the way.
+  auto step = [&](auto full, int s, const bf16x8(&a)[8], const bf16x8(&b)[8], bf16x8(&an)[8], bf16x8(&bn)[8]) {
+    const int next = slot == NS - 1 ? 0 : slot + 1;
+    __builtin_amdgcn_s_waitcnt(LGKM0);             // (this stage's fragments: requested a stage ago)
+    const bool more = full.value || s + 1 < nst, load = full.value;
+    if constexpr (full.value) {
+      vmcnt<(NS - 2) * DPS>();
+      asm volatile("s_barrier" ::: "memory");
+    } else {
+      if (more) turn(s);
+      if (s + NS < nst) issue(s + NS, slot);
+    }
+    const char* nx = smem + next * STAGE;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (load) issue_piece(s + NS, slot, i);
+      __builtin_amdgcn_sched_barrier(0);
+      mfma16(acc[i][0], a[i], b[0]);
+      mfma16(acc[i][1], a[i], b[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) an[i] = *reinterpret_cast<const bf16x8*>(nx + xa + i * 16 * 2 * ring::BK);
+      __builtin_amdgcn_sched_barrier(0);
+      mfma16(acc[i][2], a[i], b[2]);
+      mfma16(acc[i][3], a[i], b[3]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) bn[i] = *reinterpret_cast<const bf16x8*>(nx + wa + (i >> 1) * KB * 1024 + (i & 1) * 256);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 4; j < 8; ++j) mfma16(acc[i][j], a[i], b[j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    slot = next;
+  };
+  static_assert(DPS == 8, "a piece per group");
+  int s = 0;
+  for (; s + 1 + NS < nst; s += 2) {
+    step(Full<true>(), s, a0, b0, a1, b1);
+    step(Full<true>(), s + 1, a1, b1, a0, b0);
+  }
+  for (; s < nst; s += 2) {
+    step(Full<false>(), s, a0, b0, a1, b1);
+    step(Full<false>(), s + 1, a1, b1, a0, b0);
+  }
+  // the last products' results are complete before anything reads them behind a branch
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_nop 15");
+  __builtin_amdgcn_sched_barrier(0);
+  if (nb >= (N >> 5)) return;
+#pragma unroll
+  for (int mt = 0; mt < 8; ++mt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = 128 * wr + mt * 16 + 4 * q + i;
+      if (m >= rows) continue;
+      const int ent = seg0 + m;
+      if constexpr (EPI == EPI_COMBINE || EPI == EPI_ROWS) {
+        const float pw = perm_w[ent];
+        float* o = EPI == EPI_COMBINE ? out + (int64_t)perm_tok[ent] * ldo + nb * 32 + r : nullptr;
+        bf16* y = EPI == EPI_ROWS ? Y + (int64_t)ent * ldy + nb * 32 + r : nullptr;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          if constexpr (EPI == EPI_COMBINE) atomicAdd(o + 16 * j, pw * acc[mt][j][i]);
+          else y[16 * j] = (bf16)(pw * acc[mt][j][i]);
+        }
+      } else if constexpr (EPI == EPI_RELU2) {
+        bf16* y = Y + (int64_t)ent * ldy + nb * 32 + r;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float a = fmaxf(acc[mt][j][i], 0.f);
+          y[16 * j] = (bf16)(a * a);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          if (j & 2) continue;                     // tiles of 32: gate, up, gate, up
+          float g = acc[mt][j][i], u = acc[mt][j + 2][i], al = 1.0f;
+          if (glu_limit > 0.f) {   // (uniform) the clamped form
+            g = fminf(g, glu_limit);
+            u = fminf(fmaxf(u, -glu_limit), glu_limit) + 1.0f;
+            al = glu_alpha;
+          }
+          Y[(int64_t)ent * ldy + ((nb + (j >> 1)) >> 1) * 32 + 16 * (j & 1) + r] =
+              (bf16)(g / (1.0f + __expf(-al * g)) * u);
+        }
       }
     }
 }
@@ -438,29 +646,39 @@ hipError_t kafka_launch_moe_sort(const float* topk_w, const int* topk_e, int n, 
 hipError_t kafka_launch_grouped_wide(const bf16* X, int64_t ldx, const bf16* Wt, int E, int N, int K,
                                      const int* perm_tok, const float* perm_w, const int* expert_off, int n_ent,
                                      int gather, int epi, bf16* Y, int64_t ldy, float* out, int64_t ldo,
-                                     float glu_limit, float glu_alpha, hipStream_t st) {
+                                     float glu_limit, float glu_alpha, int bm, hipStream_t st) {
   if (n_ent < 1 || E < 1) return hipSuccess;
+  if (bm == 0) {
+    // Which tiles, from the mean rows of an expert. A round of the chip is 256 tiles of 256 x 256 or 512 of 128 x 256, the same
+    // products; the ring kernel does them 1.3 times as fast, but in whole rounds, the other one's last round thins out
+    // (a quarter of one on average).
+    const int64_t r = ((int64_t)n_ent + E - 1) / E, ct = (N + BN - 1) / BN * (int64_t)E;
+    const double ring_rounds = (double)(((r + 255) / 256 * ct + 255) / 256) / 1.3;
+    const double wide_rounds = (double)((r + 127) / 128 * ct) / 512 + 0.25;
+    bm = N % 128 == 0 && ring_rounds < wide_rounds ? 256 : 128;
+  }
+  if ((bm != 128 && bm != 256) || (bm == 256 && N % 128)) return hipErrorInvalidValue;
   if (N % 64 || K % (2 * BK) || N < 64 || K < 2 * BK || epi < 0 || epi > 3 || (epi == EPI_COMBINE) != (out != nullptr) ||
       (epi != EPI_COMBINE) != (Y != nullptr))
     return hipErrorInvalidValue;
-  const int64_t items = ((int64_t)n_ent / BM + E) * ((N + BN - 1) / BN);   // an upper bound over all routings
+  const int64_t items = ((int64_t)n_ent / bm + E) * ((N + BN - 1) / BN);   // an upper bound over all routings
   if (items > 0x0fffffff) return hipErrorInvalidValue;
   const unsigned grid = (unsigned)((items + 7) / 8 * 8);
   const auto* wt = reinterpret_cast<const bf16x8*>(Wt);
   auto a = [&](auto kern) {
     kern<<<grid, 256, 0, st>>>(X, ldx, wt, E, N, K, perm_tok, perm_w, expert_off, Y, ldy, out, ldo, glu_limit, glu_alpha);
   };
-  if (gather) {
-    if (epi == EPI_GLU) a(grouped_wide_kernel<true, EPI_GLU>);
-    else if (epi == EPI_RELU2) a(grouped_wide_kernel<true, EPI_RELU2>);
-    else if (epi == EPI_ROWS) a(grouped_wide_kernel<true, EPI_ROWS>);
-    else a(grouped_wide_kernel<true, EPI_COMBINE>);
-  } else {
-    if (epi == EPI_GLU) a(grouped_wide_kernel<false, EPI_GLU>);
-    else if (epi == EPI_RELU2) a(grouped_wide_kernel<false, EPI_RELU2>);
-    else if (epi == EPI_ROWS) a(grouped_wide_kernel<false, EPI_ROWS>);
-    else a(grouped_wide_kernel<false, EPI_COMBINE>);
-  }
+#define GW_BM(G, EPI) (bm == 256 ? a(grouped_ring_kernel<G, EPI>) : a(grouped_wide_kernel<G, EPI>))
+#define GW_EPI(G)                                       \
+  do {                                                  \
+    if (epi == EPI_GLU) GW_BM(G, EPI_GLU);              \
+    else if (epi == EPI_RELU2) GW_BM(G, EPI_RELU2);     \
+    else if (epi == EPI_ROWS) GW_BM(G, EPI_ROWS);       \
+    else GW_BM(G, EPI_COMBINE);                         \
+  } while (0)
+  if (gather) GW_EPI(true); else GW_EPI(false);
+#undef GW_EPI
+#undef GW_BM
   return hipGetLastError();
 }
 

@@ -998,3 +998,46 @@ def test_trace_runner_command_line(tmp_path):
     assert rel_err(got[0], b.oracle(t)[[0, 8]]) < TOL["float32"]
     assert rel_err(got[1], b.oracle(u)[[5]]) < TOL["float32"]
     assert rel_err(got[2], b.oracle(t)[[20]]) < TOL["float32"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,N,K", [((255, 256, 257, 0, 1), 128, 128), ((2300, 0, 700), 384, 256), ((511,), 640, 640),
+                                      ((5, 513, 300), 256, 1152)])
+def test_wide_expert_products_on_256_row_tiles(rows, N, K):
+    """Every epilogue of the 256 x 256 tiles: experts whose rows end inside, at and one past a tile, experts without rows,
+    column tiles that end inside a workgroup, fewer stages than the ring holds, more than one group of row tiles. Against the
+    fp32 product of the same bf16 operands: sums of K terms of size ~1/sqrt(K) differ by far less than the results' rounding
+    to bf16, 2^-9 of a value (the combine's fp32 adds by less still)."""
+    from kafka_llm_service_amd import ops
+
+    g = torch.Generator().manual_seed(N)
+    E, n = len(rows), sum(rows)
+    te = torch.cat([torch.full((r,), e) for e, r in enumerate(rows)])[torch.randperm(n, generator=g)].int()[:, None]
+    tw = torch.rand(n, 1, generator=g)
+    x = torch.randn(n, K, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(E, N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
+    r = ops.moe_sort(tw.cuda(), te.cuda(), E)
+    tok = r.perm_tok.long()
+    want = torch.empty(n, N, device="cuda")
+    for e in range(E):
+        a, b = int(r.expert_off[e]), int(r.expert_off[e + 1])
+        want[a:b] = x[tok[a:b]].float() @ w[e].float().t()
+    wt, tol = ops.tile_experts(w), 2 ** -8
+
+    def same(got, ref):
+        return ((got.float() - ref).abs() <= tol * ref.abs() + 1e-3).all()
+
+    assert same(ops.grouped_wide(x, wt, r, "rows", True, tile=256), want * r.perm_w[:, None])
+    assert same(ops.grouped_wide(x[tok], wt, r, "rows", False, tile=256), want * r.perm_w[:, None])
+    assert same(ops.grouped_wide(x, wt, r, "relu2", True, tile=256), want.relu() ** 2)
+    out = torch.zeros(n, N, device="cuda")
+    ops.grouped_wide(x, wt, r, "combine", True, out, tile=256)
+    assert same(out[tok], want * r.perm_w[:, None])
+    gt = ops.tile_experts(w, glu=True)
+    for kw in ({}, {"limit": 1.5, "alpha": 1.7}):
+        gate, up = want[:, :N // 2], want[:, N // 2:]
+        if kw:
+            gate, up = gate.clamp(max=1.5), up.clamp(-1.5, 1.5) + 1
+        ref = gate * torch.sigmoid(kw.get("alpha", 1.0) * gate) * up
+        assert same(ops.grouped_wide(x, gt, r, "glu", True, tile=256, **kw), ref)
+        assert same(ops.grouped_wide(x, gt, r, "glu", True, tile=128, **kw), ref)

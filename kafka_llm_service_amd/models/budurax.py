@@ -530,10 +530,13 @@ class BuduraxLM:
             stack[0].copy_(x)
         h = torch.empty(T, d, dtype=dt, device=dev)
         h2 = torch.empty(T, d, dtype=dt, device=dev)
-        last = torch.empty(m.num_segs, d, dtype=torch.float32, device=dev)
+        # the slots' shift rows: written in place unless a portion of several rows goes on from its slot
+        sh = m.seg_host
+        last = None if sh is not None and bool(((sh[:, 1] == 1) | (sh[:, 2] == 0)).all()) else \
+            torch.empty(m.num_segs, d, dtype=torch.float32, device=dev)
         for i, lw in enumerate(self.layers):
             hops.ln_shift(x, lw.norm1, lw.norm1_b, eps, h, lw.shift, m.tok_seg, m.seg, state.shift[i], last)
-            if lw.shift is not None:
+            if lw.shift is not None and last is not None:
                 hops.scatter_rows(state.shift[i], m.seg, last)
             if lw.type == "latent_attention":
                 y = self._latent_attention(i, lw, h, inp, m, pages)

@@ -33,8 +33,9 @@ __device__ __forceinline__ float ldf(const T* p) { return (float)(*p); }
 template <typename T>
 __device__ __forceinline__ void stf(T* p, float v) { *p = (T)v; }
 
+// z (1 + tanh(u)) / 2 = z / (1 + e^(-2u)): one exponential and no cancellation for negative z
 __device__ __forceinline__ float gelu_tanh(float z) {
-  return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+  return z / (1.0f + expf(-1.5957691216057308f * (z + 0.044715f * z * z * z)));
 }
 __device__ __forceinline__ float sigmoidf(float z) { return 1.0f / (1.0f + expf(-z)); }
 __device__ __forceinline__ float inv_sqrt(float v) { return 1.0f / sqrtf(v); }
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(NT) void ln_shift_kernel(const float* __restrict__ 
                                                       const AT* __restrict__ b, float eps, AT* __restrict__ out,
                                                       int64_t os, int d, const AT* __restrict__ mu,
                                                       const int* __restrict__ tok_seg, const int* __restrict__ seg,
-                                                      const float* __restrict__ state, float* __restrict__ last) {
+                                                      float* state, float* __restrict__ last) {
   __shared__ float red[NT / 64];
   const int64_t t = blockIdx.x;
   const float* xr = x + t * xs;
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(NT) void ln_shift_kernel(const float* __restrict__ 
     else
       prev = (xp[i] - mean2) * rstd2 * wi + bi;
     stf(out + t * os + i, h + (prev - h) * ldf(mu + i));
-    if (is_last) last[(int64_t)sg * d + i] = h;
+    if (is_last) (last != nullptr ? last + (int64_t)sg * d : state + (int64_t)slot * d)[i] = h;
   }
 }
 
@@ -127,36 +128,88 @@ __global__ __launch_bounds__(NT) void add_ln_kernel(float* __restrict__ x, int64
   }
 }
 
-// ---- the same three row kernels with the row held in registers (d <= NV * 256) -------------------------------------
-// A step of few rows (a decode step) has few workgroups, so these kernels are latency-bound: every pass over a row
-// that goes back to memory is a dependent round trip. Here each row is loaded once (all its loads in flight together,
-// the previous row's and the second operand's too) and the statistics, the second norm and the outputs come from
-// registers. The sums run over the same elements in the same order as in the generic kernels above.
-template <int NV>
-__device__ __forceinline__ void reg_stats(const float (&v)[NV], int d, float eps, float* red, float& mean, float& rstd) {
+// ---- the same three row kernels with the row held in registers ---------------------------------------------------------
+// A step of few rows (a decode step) has few workgroups, so these kernels are latency-bound: every pass over a row that goes
+// back to memory is a dependent round trip. Here each row is loaded once (all its loads in flight together, the previous
+// row's and the second operand's too) and the statistics, the second norm and the outputs come from registers. A thread holds
+// NV pieces of VEC neighbouring elements: four where rows are 16-byte pieces, else one. NTH threads a row: steps of few rows
+// take 1024 (one piece a thread at 4096 elements: the loads of a row are as few round trips as they can be), long ones 256.
+// 64 rows of 4096, one element a load on 256 threads -> four on 1024: ln_shift 16 -> 6 us, add_ln with a second norm 22 -> 6,
+// side_dwa (mean over three layers) 27 -> 5; 2048 rows, four a load on 256: 35 -> 22, 47 -> 24, 45 -> 33 (4 TB/s).
+template <int VEC>
+__device__ __forceinline__ void ldv(const float* p, float (&o)[VEC]) {
+  if constexpr (VEC == 4) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(p);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = v[e];
+  } else {
+    o[0] = *p;
+  }
+}
+template <int VEC>
+__device__ __forceinline__ void ldv(const bf16* p, float (&o)[VEC]) {
+  if constexpr (VEC == 4) {
+    typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    const bf16x4 v = *reinterpret_cast<const bf16x4*>(p);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (float)v[e];
+  } else {
+    o[0] = (float)*p;
+  }
+}
+template <int VEC>
+__device__ __forceinline__ void stv(float* p, const float (&v)[VEC]) {
+  if constexpr (VEC == 4) *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
+  else *p = v[0];
+}
+template <int VEC>
+__device__ __forceinline__ void stv(bf16* p, const float (&v)[VEC]) {
+  if constexpr (VEC == 4) {
+    typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    *reinterpret_cast<bf16x4*>(p) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
+  } else {
+    *p = (bf16)v[0];
+  }
+}
+template <int VEC>
+__device__ __forceinline__ void zero(float (&v)[VEC]) {
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) v[e] = 0.f;
+}
+
+// piece k of this thread starts at element (threadIdx.x + k NTH) VEC (d is a multiple of VEC)
+template <int VEC, int NTH, int NV>
+__device__ __forceinline__ void reg_stats(const float (&v)[NV][VEC], int d, float eps, float* red, float& mean,
+                                          float& rstd) {
   float s = 0.f;
 #pragma unroll
   for (int k = 0; k < NV; ++k)
-    if ((int)threadIdx.x + k * NT < d) s += v[k];
-  mean = block_sum<NT>(s, red) / (float)d;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) s += v[k][e];   // (zeros past d)
+  mean = block_sum<NTH>(s, red) / (float)d;
   float q = 0.f;
 #pragma unroll
   for (int k = 0; k < NV; ++k)
-    if ((int)threadIdx.x + k * NT < d) {
-      const float c = v[k] - mean;
-      q += c * c;
+    if (((int)threadIdx.x + k * NTH) * VEC < d) {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        const float c = v[k][e] - mean;
+        q += c * c;
+      }
     }
-  rstd = inv_sqrt(block_sum<NT>(q, red) / (float)d + eps);
+  rstd = inv_sqrt(block_sum<NTH>(q, red) / (float)d + eps);
 }
 
-template <typename AT, int NV>
-__global__ __launch_bounds__(NT) void ln_shift_reg_kernel(const float* __restrict__ x, int64_t xs,
-                                                          const AT* __restrict__ w, const AT* __restrict__ b, float eps,
-                                                          AT* __restrict__ out, int64_t os, int d,
-                                                          const AT* __restrict__ mu, const int* __restrict__ tok_seg,
-                                                          const int* __restrict__ seg, const float* __restrict__ state,
-                                                          float* __restrict__ last) {
-  __shared__ float red[NT / 64];
+// last == nullptr: a segment's last normed row goes straight to its slot (the caller knows that no row of another workgroup
+// reads it: segments of one row, or fresh ones)
+template <typename AT, int VEC, int NTH, int NV>
+__global__ __launch_bounds__(NTH) void ln_shift_reg_kernel(const float* __restrict__ x, int64_t xs,
+                                                           const AT* __restrict__ w, const AT* __restrict__ b, float eps,
+                                                           AT* __restrict__ out, int64_t os, int d,
+                                                           const AT* __restrict__ mu, const int* __restrict__ tok_seg,
+                                                           const int* __restrict__ seg, float* state,
+                                                           float* __restrict__ last) {
+  __shared__ float red[NTH / 64];
   const int64_t t = blockIdx.x;
   const float* xr = x + t * xs;
   bool first = true, is_last = false;
@@ -169,127 +222,202 @@ __global__ __launch_bounds__(NT) void ln_shift_reg_kernel(const float* __restric
     first = (t == q0);
     is_last = (t == q0 + n - 1);
   }
-  float v[NV], pv[NV], wv[NV], bv[NV];
+  float v[NV][VEC], pv[NV][VEC], wv[NV][VEC], bv[NV][VEC];
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const int i = threadIdx.x + k * NT;
-    const bool in = i < d;
-    v[k] = in ? xr[i] : 0.f;
-    wv[k] = in ? ldf(w + i) : 0.f;
-    bv[k] = in ? ldf(b + i) : 0.f;
-    pv[k] = 0.f;
-    if (mu != nullptr && in) pv[k] = first ? (p0 > 0 ? state[(int64_t)slot * d + i] : 0.f) : xr[i - xs];
+    const int i = (threadIdx.x + k * NTH) * VEC;
+    zero<VEC>(v[k]);
+    zero<VEC>(pv[k]);
+    zero<VEC>(wv[k]);
+    zero<VEC>(bv[k]);
+    if (i < d) {
+      ldv<VEC>(xr + i, v[k]);
+      ldv<VEC>(w + i, wv[k]);
+      ldv<VEC>(b + i, bv[k]);
+      if (mu != nullptr) {
+        if (!first) ldv<VEC>(xr + i - xs, pv[k]);
+        else if (p0 > 0) ldv<VEC>(state + (int64_t)slot * d + i, pv[k]);
+      }
+    }
   }
   float mean, rstd, mean2 = 0.f, rstd2 = 0.f;
-  reg_stats<NV>(v, d, eps, red, mean, rstd);
-  if (mu != nullptr && !first) reg_stats<NV>(pv, d, eps, red, mean2, rstd2);  // (uniform per workgroup)
+  reg_stats<VEC, NTH, NV>(v, d, eps, red, mean, rstd);
+  if (mu != nullptr && !first) reg_stats<VEC, NTH, NV>(pv, d, eps, red, mean2, rstd2);  // (uniform per workgroup)
+  float* keep = last != nullptr ? last + (int64_t)sg * d : state + (int64_t)slot * d;
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const int i = threadIdx.x + k * NT;
+    const int i = (threadIdx.x + k * NTH) * VEC;
     if (i < d) {
-      const float h = (v[k] - mean) * rstd * wv[k] + bv[k];
+      float h[VEC], m[VEC];
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) h[e] = (v[k][e] - mean) * rstd * wv[k][e] + bv[k][e];
       if (mu == nullptr) {
-        stf(out + t * os + i, h);
+        stv<VEC>(out + t * os + i, h);
       } else {
-        const float prev = first ? pv[k] : (pv[k] - mean2) * rstd2 * wv[k] + bv[k];
-        stf(out + t * os + i, h + (prev - h) * ldf(mu + i));
-        if (is_last) last[(int64_t)sg * d + i] = h;
+        ldv<VEC>(mu + i, m);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          const float prev = first ? pv[k][e] : (pv[k][e] - mean2) * rstd2 * wv[k][e] + bv[k][e];
+          m[e] = h[e] + (prev - h[e]) * m[e];
+        }
+        stv<VEC>(out + t * os + i, m);
+        if (is_last) stv<VEC>(keep + i, h);
       }
     }
   }
 }
 
-template <typename AT, int NV, int MODE>
-__global__ __launch_bounds__(NT) void add_ln_reg_kernel(float* __restrict__ x, int64_t xs, const AT* __restrict__ y,
-                                                        int64_t ys, const AT* __restrict__ w,
-                                                        const AT* __restrict__ b, float eps, int d,
-                                                        AT* __restrict__ out2, int64_t os, const AT* __restrict__ w2,
-                                                        const AT* __restrict__ b2) {
-  __shared__ float red[NT / 64];
+template <typename AT, int VEC, int NTH, int NV, int MODE>
+__global__ __launch_bounds__(NTH) void add_ln_reg_kernel(float* __restrict__ x, int64_t xs, const AT* __restrict__ y,
+                                                         int64_t ys, const AT* __restrict__ w,
+                                                         const AT* __restrict__ b, float eps, int d,
+                                                         AT* __restrict__ out2, int64_t os, const AT* __restrict__ w2,
+                                                         const AT* __restrict__ b2) {
+  __shared__ float red[NTH / 64];
   const int64_t t = blockIdx.x;
-  float yv[NV], xv[NV];
+  float yv[NV][VEC], xv[NV][VEC], wv[NV][VEC], bv[NV][VEC];
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const int i = threadIdx.x + k * NT;
-    yv[k] = i < d ? ldf(y + t * ys + i) : 0.f;
-    xv[k] = i < d ? x[t * xs + i] : 0.f;
+    const int i = (threadIdx.x + k * NTH) * VEC;
+    zero<VEC>(yv[k]);
+    zero<VEC>(xv[k]);
+    if (i < d) {
+      ldv<VEC>(y + t * ys + i, yv[k]);
+      ldv<VEC>(x + t * xs + i, xv[k]);
+      ldv<VEC>(w + i, wv[k]);
+      ldv<VEC>(b + i, bv[k]);
+    }
   }
   float mean, rstd;
-  reg_stats<NV>(yv, d, eps, red, mean, rstd);
+  reg_stats<VEC, NTH, NV>(yv, d, eps, red, mean, rstd);
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const int i = threadIdx.x + k * NT;
+    const int i = (threadIdx.x + k * NTH) * VEC;
     if (i < d) {
-      xv[k] = xv[k] + ((yv[k] - mean) * rstd * ldf(w + i) + ldf(b + i));
-      x[t * xs + i] = xv[k];
-      if constexpr (MODE == 2) stf(out2 + t * os + i, xv[k]);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) xv[k][e] = xv[k][e] + ((yv[k][e] - mean) * rstd * wv[k][e] + bv[k][e]);
+      stv<VEC>(x + t * xs + i, xv[k]);
+      if constexpr (MODE == 2) stv<VEC>(out2 + t * os + i, xv[k]);
+      if constexpr (MODE == 1) {
+        ldv<VEC>(w2 + i, wv[k]);
+        ldv<VEC>(b2 + i, bv[k]);
+      }
     }
   }
   if constexpr (MODE == 1) {
     float m2, r2;
-    reg_stats<NV>(xv, d, eps, red, m2, r2);
+    reg_stats<VEC, NTH, NV>(xv, d, eps, red, m2, r2);
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      const int i = threadIdx.x + k * NT;
-      if (i < d) stf(out2 + t * os + i, (xv[k] - m2) * r2 * ldf(w2 + i) + ldf(b2 + i));
+      const int i = (threadIdx.x + k * NTH) * VEC;
+      if (i < d) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) xv[k][e] = (xv[k][e] - m2) * r2 * wv[k][e] + bv[k][e];
+        stv<VEC>(out2 + t * os + i, xv[k]);
+      }
     }
   }
 }
 
-template <typename AT, int NV>
-__global__ __launch_bounds__(NT) void side_dwa_reg_kernel(float* __restrict__ x, const AT* __restrict__ y, int64_t ys,
-                                                          const AT* __restrict__ sw, float eps,
-                                                          float* __restrict__ stack, int layer,
-                                                          const float* __restrict__ dwa, int64_t T, int d) {
-  __shared__ float red[NT / 64];
+template <typename AT, int VEC, int NTH, int NV>
+__global__ __launch_bounds__(NTH) void side_dwa_reg_kernel(float* __restrict__ x, const AT* __restrict__ y, int64_t ys,
+                                                           const AT* __restrict__ sw, float eps,
+                                                           float* __restrict__ stack, int layer,
+                                                           const float* __restrict__ dwa, int64_t T, int d) {
+  __shared__ float red[NTH / 64];
   const int64_t t = blockIdx.x;
   const int64_t plane = T * d;
-  float xv[NV], yv[NV];
+  float xv[NV][VEC], yv[NV][VEC], a[NV][VEC];
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const int i = threadIdx.x + k * NT;
-    xv[k] = i < d ? x[t * d + i] : 0.f;
-    yv[k] = (y != nullptr && i < d) ? ldf(y + t * ys + i) : 0.f;
+    const int i = (threadIdx.x + k * NTH) * VEC;
+    zero<VEC>(xv[k]);
+    zero<VEC>(yv[k]);
+    zero<VEC>(a[k]);
+    if (i < d) {
+      ldv<VEC>(x + t * d + i, xv[k]);
+      if (y != nullptr) ldv<VEC>(y + t * ys + i, yv[k]);
+    }
+  }
+  if (stack != nullptr && dwa != nullptr) {
+#pragma unroll 4
+    for (int j = 0; j <= layer; ++j) {  // the earlier planes of the row, in flight under the statistics of y
+      const float c = dwa[j];
+      const float* pj = stack + (int64_t)j * plane + t * d;
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        const int i = (threadIdx.x + k * NTH) * VEC;
+        if (i < d) {
+          float p[VEC];
+          ldv<VEC>(pj + i, p);
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) a[k][e] += c * p[e];
+        }
+      }
+    }
   }
   if (y != nullptr) {
     float s = 0.f;
 #pragma unroll
-    for (int k = 0; k < NV; ++k) s += yv[k] * yv[k];  // (zeros beyond d)
-    const float r = inv_sqrt(block_sum<NT>(s, red) / (float)d + eps);
+    for (int k = 0; k < NV; ++k)
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) s += yv[k][e] * yv[k][e];  // (zeros beyond d)
+    const float r = inv_sqrt(block_sum<NTH>(s, red) / (float)d + eps);
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      const int i = threadIdx.x + k * NT;
-      if (i < d) xv[k] += yv[k] * r * ldf(sw + i);
-    }
-  }
-  if (stack != nullptr) {
-    float a[NV];
+      const int i = (threadIdx.x + k * NTH) * VEC;
+      if (i < d) {
+        float g[VEC];
+        ldv<VEC>(sw + i, g);
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      const int i = threadIdx.x + k * NT;
-      if (i < d) stack[(int64_t)(layer + 1) * plane + t * d + i] = xv[k];
-      a[k] = 0.f;
-    }
-    if (dwa != nullptr) {
-      for (int j = 0; j <= layer; ++j) {  // one plane per turn, the row's NV loads of it in flight together
-        const float c = dwa[j];
-        const float* pj = stack + (int64_t)j * plane + t * d;
-#pragma unroll
-        for (int k = 0; k < NV; ++k) {
-          const int i = threadIdx.x + k * NT;
-          if (i < d) a[k] += c * pj[i];
-        }
+        for (int e = 0; e < VEC; ++e) xv[k][e] += yv[k][e] * r * g[e];
       }
-      const float c = dwa[layer + 1];
-#pragma unroll
-      for (int k = 0; k < NV; ++k) xv[k] = a[k] + c * xv[k];
     }
   }
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const int i = threadIdx.x + k * NT;
-    if (i < d) x[t * d + i] = xv[k];
+    const int i = (threadIdx.x + k * NTH) * VEC;
+    if (i < d) {
+      if (stack != nullptr) {
+        stv<VEC>(stack + (int64_t)(layer + 1) * plane + t * d + i, xv[k]);
+        if (dwa != nullptr) {
+          const float c = dwa[layer + 1];
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) xv[k][e] = a[k][e] + c * xv[k][e];
+        }
+      }
+      stv<VEC>(x + t * d + i, xv[k]);
+    }
   }
+}
+
+// launch shape of the register kernels: l(vec, threads, pieces) for rows of d elements, false: the generic kernel
+template <typename F>
+static inline bool row_shape(int64_t T, int d, bool vec4, F l) {
+  using std::integral_constant;
+  if (vec4 && d <= 1024) l(integral_constant<int, 4>(), integral_constant<int, 256>(), integral_constant<int, 1>());
+  else if (vec4 && d <= 4096 && T <= 512)
+    l(integral_constant<int, 4>(), integral_constant<int, 1024>(), integral_constant<int, 1>());
+  else if (vec4 && d <= 4096) l(integral_constant<int, 4>(), integral_constant<int, 256>(), integral_constant<int, 4>());
+  else if (d <= 1024) l(integral_constant<int, 1>(), integral_constant<int, 256>(), integral_constant<int, 4>());
+  else if (d <= 4096) l(integral_constant<int, 1>(), integral_constant<int, 256>(), integral_constant<int, 16>());
+  else return false;
+  return true;
+}
+static inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// the same on bf16 rows in 16-byte pieces: 2048 x 2 x 14336 in 34 us (176 MB at 5.2 TB/s; an element a thread took 99)
+__global__ void gelu_mul_vec8_kernel(const bf16* __restrict__ gu, int64_t gs, bf16* __restrict__ out, int64_t T, int F) {
+  const int F8 = F >> 3;
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= T * F8) return;
+  const int64_t t = i / F8;
+  const int f = (int)(i - t * F8) << 3;
+  const bf16x8 g = load_bf16x8(gu + t * gs + f), u = load_bf16x8(gu + t * gs + F + f);
+  bf16x8 o;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = (bf16)(gelu_tanh((float)g[e]) * (float)u[e]);
+  store_bf16x8(out + t * F + f, o);
 }
 
 template <typename AT>
@@ -780,10 +908,12 @@ __global__ void short_conv_kernel(const AT* __restrict__ proj, int64_t ps, int c
 // The same on bf16 rows whose sizes, offsets, strides and bases are multiples of 8 elements: a thread takes 8 channels of
 // TB consecutive rows and slides the window over them (a row is loaded once per thread; a row that starts a segment
 // takes its window from the slot's tail, or zeros).
-template <int TAPS, int TB>
+// STEP: every segment is one row; its thread also moves the slot's tail on (no other thread reads it): 64 x 10240 in 6 us, 7 + 11
+// with the tails in a launch of their own.
+template <int TAPS, int TB, bool STEP>
 __global__ void short_conv_vec8_kernel(const bf16* __restrict__ proj, int64_t ps, int c0, const bf16* __restrict__ w,
                                        const bf16* __restrict__ b, int C, const int* __restrict__ tok_seg,
-                                       const int* __restrict__ seg, const bf16* __restrict__ state,
+                                       const int* __restrict__ seg, bf16* state,
                                        bf16* __restrict__ out, int64_t T, int silu, int residual) {
   const int C8 = C >> 3;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -792,11 +922,15 @@ __global__ void short_conv_vec8_kernel(const bf16* __restrict__ proj, int64_t ps
   const int64_t ta = blk * TB;
   if (ta >= T) return;
   float wt[TAPS][8], bias[8];
+  bf16x8 wr[TAPS], br = {0, 0, 0, 0, 0, 0, 0, 0};   // 8 channels' taps: 8 TAPS neighbouring elements
+#pragma unroll
+  for (int k = 0; k < TAPS; ++k) wr[k] = load_bf16x8(w + (int64_t)c * TAPS + 8 * k);
+  if (b) br = load_bf16x8(b + c);
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    bias[e] = b ? (float)b[c + e] : 0.f;
+    bias[e] = (float)br[e];
 #pragma unroll
-    for (int k = 0; k < TAPS; ++k) wt[k][e] = (float)w[(int64_t)(c + e) * TAPS + k];
+    for (int k = 0; k < TAPS; ++k) wt[k][e] = (float)wr[(e * TAPS + k) >> 3][(e * TAPS + k) & 7];
   }
   bf16x8 win[TAPS];   // inputs of rows t - TAPS + 1 .. t
   const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -833,6 +967,11 @@ __global__ void short_conv_vec8_kernel(const bf16* __restrict__ proj, int64_t ps
       o[e] = (bf16)a;
     }
     store_bf16x8(out + t * C + c, o);
+    if constexpr (STEP) {
+#pragma unroll
+      for (int k = 0; k < TAPS - 1; ++k)
+        store_bf16x8(state + ((int64_t)seg[4 * sg + 3] * (TAPS - 1) + k) * C + c, win[k + 1]);
+    }
   }
 }
 
@@ -1145,6 +1284,46 @@ __global__ __launch_bounds__(NT) void gated_norm_kernel(const float* __restrict_
   }
 }
 
+// The same on rows in 4-element pieces, parts of up to 4096 elements in registers (y and z are read once): 2048 x 8192 in 29
+// us, 53 in the form above.
+template <typename AT, int NV>
+__global__ __launch_bounds__(NT) void gated_norm_reg_kernel(const float* __restrict__ y, int64_t ys,
+                                                            const AT* __restrict__ z, int64_t zs,
+                                                            const AT* __restrict__ w, int gs, float eps,
+                                                            AT* __restrict__ out, int64_t os) {
+  __shared__ float red[NT / 64];
+  const int64_t t = blockIdx.x;
+  const int c0 = blockIdx.y * gs;
+  float v[NV][4], s = 0.f;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int i = (threadIdx.x + k * NT) * 4;
+    zero<4>(v[k]);
+    if (i < gs) {
+      float zv[4];
+      ldv<4>(y + t * ys + c0 + i, v[k]);
+      ldv<4>(z + t * zs + c0 + i, zv);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[k][e] *= zv[e] / (1.0f + expf(-zv[e]));
+        s += v[k][e] * v[k][e];
+      }
+    }
+  }
+  const float r = inv_sqrt(block_sum<NT>(s, red) / (float)gs + eps);
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int i = (threadIdx.x + k * NT) * 4;
+    if (i < gs) {
+      float wv[4];
+      ldv<4>(w + c0 + i, wv);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[k][e] = v[k][e] * r * wv[e];
+      stv<4>(out + t * os + c0 + i, v[k]);
+    }
+  }
+}
+
 static inline int ew_grid(int64_t n) { return (int)std::min<int64_t>((n + 255) / 256, 65535 * 4); }
 
 }  // namespace hy
@@ -1165,16 +1344,17 @@ extern "C" {
 
 hipError_t kafka_hy_ln_shift(int f32, const float* x, int64_t xs, const void* w, const void* b, float eps, void* out,
                              int64_t os, int T, int d, const void* mu, const int* tok_seg, const int* seg,
-                             const float* state, float* last, hipStream_t st) {
+                             float* state, float* last, hipStream_t st) {
   if (T <= 0) return hipSuccess;
   DISPATCH_AT(f32, {
-    auto a = [&](auto k) {
-      k<<<T, NT, 0, st>>>(x, xs, (const AT*)w, (const AT*)b, eps, (AT*)out, os, d, (const AT*)mu, tok_seg, seg, state,
-                          last);
-    };
-    if (d <= 4 * NT) a(ln_shift_reg_kernel<AT, 4>);
-    else if (d <= 16 * NT) a(ln_shift_reg_kernel<AT, 16>);
-    else a(ln_shift_kernel<AT>);
+    const bool v4 = d % 4 == 0 && xs % 4 == 0 && os % 4 == 0 && al16(x) && al16(w) && al16(b) && al16(out) && al16(mu) &&
+                    al16(state) && al16(last);
+    if (!row_shape(T, d, v4, [&](auto V, auto N, auto K) {
+          ln_shift_reg_kernel<AT, V.value, N.value, K.value><<<T, N.value, 0, st>>>(
+              x, xs, (const AT*)w, (const AT*)b, eps, (AT*)out, os, d, (const AT*)mu, tok_seg, seg, state, last);
+        }))
+      ln_shift_kernel<AT><<<T, NT, 0, st>>>(x, xs, (const AT*)w, (const AT*)b, eps, (AT*)out, os, d, (const AT*)mu, tok_seg,
+                                            seg, state, last);
   });
   return hipGetLastError();
 }
@@ -1191,27 +1371,35 @@ hipError_t kafka_hy_add_ln(int f32, float* x, int64_t xs, const void* y, int64_t
   if (T <= 0) return hipSuccess;
   const int mode = out2 == nullptr ? 0 : (w2 != nullptr ? 1 : 2);
   DISPATCH_AT(f32, {
+    const bool v4 = d % 4 == 0 && xs % 4 == 0 && ys % 4 == 0 && os % 4 == 0 && al16(x) && al16(y) && al16(w) && al16(b) &&
+                    al16(out2) && al16(w2) && al16(b2);
+    auto reg = [&](auto M) {
+      return row_shape(T, d, v4, [&](auto V, auto N, auto K) {
+        add_ln_reg_kernel<AT, V.value, N.value, K.value, M.value><<<T, N.value, 0, st>>>(
+            x, xs, (const AT*)y, ys, (const AT*)w, (const AT*)b, eps, d, (AT*)out2, os, (const AT*)w2, (const AT*)b2);
+      });
+    };
     auto a = [&](auto k) {
       k<<<T, NT, 0, st>>>(x, xs, (const AT*)y, ys, (const AT*)w, (const AT*)b, eps, d, (AT*)out2, os, (const AT*)w2,
                           (const AT*)b2);
     };
-    if (d <= 4 * NT) {
-      if (mode == 0) a(add_ln_reg_kernel<AT, 4, 0>);
-      else if (mode == 1) a(add_ln_reg_kernel<AT, 4, 1>);
-      else a(add_ln_reg_kernel<AT, 4, 2>);
-    } else if (d <= 16 * NT) {
-      if (mode == 0) a(add_ln_reg_kernel<AT, 16, 0>);
-      else if (mode == 1) a(add_ln_reg_kernel<AT, 16, 1>);
-      else a(add_ln_reg_kernel<AT, 16, 2>);
-    } else if (mode == 0) a(add_ln_kernel<AT, 0>);
-    else if (mode == 1) a(add_ln_kernel<AT, 1>);
-    else a(add_ln_kernel<AT, 2>);
+    if (mode == 0) {
+      if (!reg(std::integral_constant<int, 0>())) a(add_ln_kernel<AT, 0>);
+    } else if (mode == 1) {
+      if (!reg(std::integral_constant<int, 1>())) a(add_ln_kernel<AT, 1>);
+    } else if (!reg(std::integral_constant<int, 2>())) {
+      a(add_ln_kernel<AT, 2>);
+    }
   });
   return hipGetLastError();
 }
 
 hipError_t kafka_hy_gelu_mul(int f32, const void* gu, int64_t gs, void* out, int64_t T, int F, hipStream_t st) {
   if (T * F <= 0) return hipSuccess;
+  if (!f32 && F % 8 == 0 && gs % 8 == 0 && al16(gu) && al16(out)) {
+    gelu_mul_vec8_kernel<<<(unsigned)((T * (F / 8) + 255) / 256), 256, 0, st>>>((const bf16*)gu, gs, (bf16*)out, T, F);
+    return hipGetLastError();
+  }
   DISPATCH_AT(f32, gelu_mul_kernel<AT><<<ew_grid(T * F), 256, 0, st>>>((const AT*)gu, gs, (AT*)out, T, F));
   return hipGetLastError();
 }
@@ -1228,10 +1416,12 @@ hipError_t kafka_hy_side_dwa(int f32, float* x, const void* y, int64_t ys, const
                              int layer, const float* dwa, int64_t T, int d, hipStream_t st) {
   if (T <= 0) return hipSuccess;
   DISPATCH_AT(f32, {
-    auto a = [&](auto k) { k<<<(int)T, NT, 0, st>>>(x, (const AT*)y, ys, (const AT*)sw, eps, stack, layer, dwa, T, d); };
-    if (d <= 4 * NT) a(side_dwa_reg_kernel<AT, 4>);
-    else if (d <= 16 * NT) a(side_dwa_reg_kernel<AT, 16>);
-    else a(side_dwa_kernel<AT>);
+    const bool v4 = d % 4 == 0 && ys % 4 == 0 && al16(x) && al16(y) && al16(sw) && al16(stack);
+    if (!row_shape(T, d, v4, [&](auto V, auto N, auto K) {
+          side_dwa_reg_kernel<AT, V.value, N.value, K.value><<<(unsigned)T, N.value, 0, st>>>(
+              x, (const AT*)y, ys, (const AT*)sw, eps, stack, layer, dwa, T, d);
+        }))
+      side_dwa_kernel<AT><<<(int)T, NT, 0, st>>>(x, (const AT*)y, ys, (const AT*)sw, eps, stack, layer, dwa, T, d);
   });
   return hipGetLastError();
 }
@@ -1327,18 +1517,27 @@ hipError_t kafka_hy_short_conv(int f32, const void* proj, int64_t ps, int c0, co
                                int silu, int residual, hipStream_t st) {
   if (T <= 0 || C <= 0 || taps > 16 || taps < 1) return (taps > 16 || taps < 1) ? hipErrorInvalidValue : hipSuccess;
   auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (!f32 && taps >= 2 && taps <= 4 && C % 8 == 0 && c0 % 8 == 0 && ps % 8 == 0 && al(proj) && al(state) && al(out)) {
+  if (!f32 && taps >= 2 && taps <= 4 && C % 8 == 0 && c0 % 8 == 0 && ps % 8 == 0 && al(proj) && al(state) && al(out) &&
+      al(w) && al(b)) {
     const bool runs = T >= 2048;   // few rows: a thread per row, many: a thread per eight
-    const int64_t n = (runs ? (T + 7) / 8 : T) * (C / 8);
+    const bool step = T == R;      // every segment one row
+    const int64_t n = (runs && !step ? (T + 7) / 8 : T) * (C / 8);
     auto a = [&](auto k) {
       k<<<(unsigned)((n + 255) / 256), 256, 0, st>>>((const bf16*)proj, ps, c0, (const bf16*)w, (const bf16*)b, C, tok_seg,
-                                                     seg, (const bf16*)state, (bf16*)out, T, silu, residual);
+                                                     seg, (bf16*)state, (bf16*)out, T, silu, residual);
     };
-    if (taps == 2) runs ? a(short_conv_vec8_kernel<2, 8>) : a(short_conv_vec8_kernel<2, 1>);
-    else if (taps == 3) runs ? a(short_conv_vec8_kernel<3, 8>) : a(short_conv_vec8_kernel<3, 1>);
-    else runs ? a(short_conv_vec8_kernel<4, 8>) : a(short_conv_vec8_kernel<4, 1>);
-    conv_state_kernel<bf16><<<(int)(((int64_t)R * C + 255) / 256), 256, 0, st>>>((const bf16*)proj, ps, c0, C, taps, seg,
-                                                                                 (bf16*)state, R);
+    auto taps_of = [&](auto TB, auto ST) {
+      if (taps == 2) a(short_conv_vec8_kernel<2, TB.value, ST.value>);
+      else if (taps == 3) a(short_conv_vec8_kernel<3, TB.value, ST.value>);
+      else a(short_conv_vec8_kernel<4, TB.value, ST.value>);
+    };
+    using std::integral_constant;
+    if (step) taps_of(integral_constant<int, 1>(), integral_constant<bool, true>());
+    else if (runs) taps_of(integral_constant<int, 8>(), integral_constant<bool, false>());
+    else taps_of(integral_constant<int, 1>(), integral_constant<bool, false>());
+    if (!step)
+      conv_state_kernel<bf16><<<(int)(((int64_t)R * C + 255) / 256), 256, 0, st>>>((const bf16*)proj, ps, c0, C, taps, seg,
+                                                                                  (bf16*)state, R);
     return hipGetLastError();
   }
   DISPATCH_AT(f32, {
@@ -1422,6 +1621,17 @@ hipError_t kafka_hy_ssm_combine(int f32, const void* proj, int64_t ps, int dt_of
 hipError_t kafka_hy_gated_norm(int f32, const float* y, int64_t ys, const void* z, int64_t zs, const void* w, int inner,
                                int groups, float eps, void* out, int64_t os, int64_t T, hipStream_t st) {
   if (T <= 0) return hipSuccess;
+  const int gw = inner / groups;
+  if (gw % 4 == 0 && gw <= 4096 && ys % 4 == 0 && zs % 4 == 0 && os % 4 == 0 && al16(y) && al16(z) && al16(w) && al16(out)) {
+    DISPATCH_AT(f32, {
+      auto a = [&](auto k) {
+        k<<<dim3((unsigned)T, (unsigned)groups), NT, 0, st>>>(y, ys, (const AT*)z, zs, (const AT*)w, gw, eps, (AT*)out, os);
+      };
+      if (gw <= 1024) a(gated_norm_reg_kernel<AT, 1>);
+      else a(gated_norm_reg_kernel<AT, 4>);
+    });
+    return hipGetLastError();
+  }
   DISPATCH_AT(f32, gated_norm_kernel<AT><<<dim3((unsigned)T, (unsigned)groups), NT, 0, st>>>(
                        y, ys, (const AT*)z, zs, (const AT*)w, inner / groups, eps, (AT*)out, os));
   return hipGetLastError();

@@ -7,7 +7,7 @@
 extern "C" {
 hipError_t kafka_hy_ln_shift(int f32, const float* x, int64_t xs, const void* w, const void* b, float eps, void* out,
                              int64_t os, int T, int d, const void* mu, const int* tok_seg, const int* seg,
-                             const float* state, float* last, hipStream_t st);
+                             float* state, float* last, hipStream_t st);
 hipError_t kafka_hy_scatter_rows(float* dst, const int* seg, const float* src, int R, int d, hipStream_t st);
 hipError_t kafka_hy_add_ln(int f32, float* x, int64_t xs, const void* y, int64_t ys, const void* w, const void* b,
                            float eps, int T, int d, void* out2, int64_t os, const void* w2, const void* b2,
@@ -244,19 +244,18 @@ void ln_shift(at::Tensor x, at::Tensor w, at::Tensor b, double eps, at::Tensor o
   same_act(f32, {&w, &b});
   vec(w, d, "w"); vec(b, d, "b");
   TORCH_CHECK(out.size(0) == T && out.size(1) == d, "ln_shift: out shape");
-  const void* mup = nullptr; const int *tsp = nullptr, *sgp = nullptr; const float* stp = nullptr; float* lp = nullptr;
+  const void* mup = nullptr; const int *tsp = nullptr, *sgp = nullptr; float *stp = nullptr, *lp = nullptr;
   if (mu.has_value()) {
-    TORCH_CHECK(tok_seg.has_value() && seg.has_value() && state.has_value() && last.has_value(),
-                "ln_shift: a shift needs tok_seg, seg, state and last");
+    TORCH_CHECK(tok_seg.has_value() && seg.has_value() && state.has_value(), "ln_shift: a shift needs tok_seg, seg and state");
     same_act(f32, {&*mu}); vec(*mu, d, "mu");
     segs(*tok_seg, *seg, T);
     TORCH_CHECK(state->is_cuda() && state->scalar_type() == at::kFloat && state->is_contiguous() && state->dim() == 2 &&
                     state->size(1) == d, "ln_shift: state fp32 [slots, d]");
-    TORCH_CHECK(last->is_cuda() && last->scalar_type() == at::kFloat && last->is_contiguous() && last->dim() == 2 &&
-                    last->size(0) >= seg->size(0) && last->size(1) == d, "ln_shift: last fp32 [R, d]");
+    TORCH_CHECK(!last.has_value() || (last->is_cuda() && last->scalar_type() == at::kFloat && last->is_contiguous() && last->dim() == 2 &&
+                    last->size(0) >= seg->size(0) && last->size(1) == d), "ln_shift: last fp32 [R, d]");
     TORCH_CHECK(x.stride(0) >= d, "ln_shift: rows must not overlap");
     mup = mu->data_ptr(); tsp = tok_seg->data_ptr<int>(); sgp = seg->data_ptr<int>();
-    stp = state->data_ptr<float>(); lp = last->data_ptr<float>();
+    stp = state->data_ptr<float>(); lp = last.has_value() ? last->data_ptr<float>() : nullptr;
   }
   HY_HIP(kafka_hy_ln_shift(f32, x.data_ptr<float>(), x.stride(0), w.data_ptr(), b.data_ptr(), (float)eps,
                            out.data_ptr(), out.stride(0), (int)T, (int)d, mup, tsp, sgp, stp, lp, stream()));

@@ -24,9 +24,14 @@ def _gpu(t: torch.Tensor) -> bool:
 def ln_shift(x, w, b, eps, out, mu=None, tok_seg=None, seg=None, state=None, last=None) -> None:
     """out = layer_norm(x) (x fp32 [T, d]); with ``mu`` each row is then moved towards the previous row's normed
     value (the slot's ``state`` row for a segment's first row) by mu, and every segment's last normed row lands in
-    ``last`` [R, d] (``scatter_rows`` stores it once all rows have read the old state)."""
+    ``last`` [R, d] (``scatter_rows`` stores it once all rows have read the old state), or without ``last`` in the slots:
+    only where every segment is one row or starts its sequence (nobody else reads its slot in this step)."""
     if _gpu(x):
         ext().hy_ln_shift(x, w, b, float(eps), out, mu, tok_seg, seg, state, last)
+    elif mu is not None and last is None:
+        last = torch.empty(seg.shape[0], x.shape[1], dtype=torch.float32)
+        ref.ln_shift(x, w, b, eps, out, mu, tok_seg, seg, state, last)
+        ref.scatter_rows(state, seg, last)
     else:
         ref.ln_shift(x, w, b, eps, out, mu, tok_seg, seg, state, last)
 

@@ -857,3 +857,99 @@ def test_attention_of_portions_on_expanded_keys(H, rd, window, extras):
     got = out.cpu().double().view(T, H, Dv)
     assert (got[:1] == 7).all()
     assert (got[1:] - want[1:]).abs().max().item() < 1.1 * 2 ** -8 * vmax
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d,T", [(4, 3), (1024, 3), (1028, 5), (1030, 5), (4096, 7), (4096, 600), (4100, 3), (1022, 2)])
+def test_row_kernels_over_widths(dtype, d, T):
+    """Layer norm with the token shift, add + norm, token input + depth average and the grouped gated norm at the widths
+    where their forms change (pieces of four elements or single ones, 256 or 1024 threads, registers or not), and views whose
+    rows are not in 16-byte pieces, against the CPU functions: fp32 sums in another order (d * 2^-24 of the row's size, 2.4e-4
+    at 4096), results rounded to the activation type: two fp32 values on either side of a boundary end one bf16 step apart, at
+    most 2^-7 of the value."""
+    from kafka_llm_service_amd.ops import hybrid_reference as href
+
+    dev = "cuda:0"
+    g = torch.Generator().manual_seed(d + T)
+
+    def rn(*s):
+        return torch.randn(*s, generator=g)
+
+    def same(got, want, acc=d * 2.0 ** -24 + 1e-5):
+        got, want = got.float().cpu(), want.float()
+        tol = acc + (2 ** -7 if dtype == torch.bfloat16 else 0)
+        assert ((got - want).abs() <= tol * (want.abs() + 1)).all(), (got - want).abs().max()
+
+    for off in (0, 1):   # rows of a wider buffer, from its first or its second column on
+        wide = rn(T, d + 8)
+        x, w, b, mu = wide[:, off:off + d], rn(d).to(dtype), rn(d).to(dtype), torch.rand(d, generator=g).to(dtype)
+        xd = wide.to(dev)[:, off:off + d]
+        seg, ts = _seg("cpu", [(1, 5, 2), (T - 1, 0, 0)])
+        state = rn(3, d)
+        for direct in (False, True):
+            want, out = torch.empty(T, d, dtype=dtype), torch.empty(T, d, dtype=dtype, device=dev)
+            s0, s1 = state.clone(), state.to(dev)
+            last = None if direct else torch.empty(2, d)
+            hops.ln_shift(x, w, b, 1e-5, want, mu, ts, seg, s0, last)
+            ld = None if direct else torch.empty(2, d, device=dev)
+            hops.ln_shift(xd, w.to(dev), b.to(dev), 1e-5, out, mu.to(dev), ts.to(dev), seg.to(dev), s1, ld)
+            same(out, want)
+            same(s1, s0)
+            if not direct:
+                same(ld, last)
+        out = torch.empty(T, d, dtype=dtype, device=dev)
+        hops.ln_shift(xd, w.to(dev), b.to(dev), 1e-5, out)
+        href.ln_shift(x, w, b, 1e-5, want)
+        same(out, want)
+        y = rn(T, d).to(dtype)
+        for w2 in (None, w):
+            x0, x1 = x.clone(), wide.to(dev)[:, off:off + d]
+            o0, o1 = torch.empty(T, d, dtype=dtype), torch.empty(T, d, dtype=dtype, device=dev)
+            b2 = None if w2 is None else b
+            hops.add_ln(x0, y, w, b, 1e-5, o0, w2, b2)
+            hops.add_ln(x1, y.to(dev), w.to(dev), b.to(dev), 1e-5, o1, None if w2 is None else w2.to(dev),
+                        None if b2 is None else b2.to(dev))
+            same(x1, x0)
+            same(o1, o0)
+    x = rn(T, d)
+    stack = rn(4, T, d)
+    for layer in (0, 2):
+        dwa = torch.rand(layer + 2, generator=g)
+        x0, x1, s0, s1 = x.clone(), x.to(dev), stack.clone(), stack.to(dev)
+        hops.side_dwa(x0, y, w, 1e-5, s0, layer, dwa)
+        hops.side_dwa(x1, y.to(dev), w.to(dev), 1e-5, s1, layer, dwa.to(dev))
+        same(x1, x0)
+        same(s1, s0)
+    for groups in (1, 2):
+        yv, z, o0 = rn(T, d), rn(T, d + 4).to(dtype), torch.empty(T, d, dtype=dtype)
+        o1 = torch.empty(T, d, dtype=dtype, device=dev)
+        hops.gated_norm(yv, z, w, groups, 1e-5, o0)
+        hops.gated_norm(yv.to(dev), z.to(dev), w.to(dev), groups, 1e-5, o1)
+        same(o1, o0)
+    gu = (rn(T, 2 * d) * 3).to(dtype)
+    o0, o1 = torch.empty(T, d, dtype=dtype), torch.empty(T, d, dtype=dtype, device=dev)
+    hops.gelu_mul(gu, o0)
+    hops.gelu_mul(gu.to(dev), o1)
+    same(o1, o0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("taps", [2, 3, 4])
+def test_conv_of_single_tokens(taps):
+    """A step of single tokens (fresh ones in slots of NaN, others going on): one kernel for the rows and the slots' tails,
+    against the CPU function; bf16 results of fp32 sums of up to four products: at most one bf16 step (2^-7) apart."""
+    g = torch.Generator().manual_seed(taps)
+    C, R = 40, 7
+    proj = torch.randn(R, C + 8, generator=g).bfloat16()
+    w, b = torch.randn(C, taps, generator=g).bfloat16(), torch.randn(C, generator=g).bfloat16()
+    seg, ts = _seg("cpu", [(1, 0 if r % 3 == 0 else r, R - 1 - r) for r in range(R)])
+    state = torch.randn(R, taps - 1, C, generator=g).bfloat16()
+    for r in range(0, R, 3):
+        state[R - 1 - r] = float("nan")
+    s0, s1 = state.clone(), state.to("cuda:0")
+    o0, o1 = torch.empty(R, C, dtype=torch.bfloat16), torch.empty(R, C, dtype=torch.bfloat16, device="cuda:0")
+    hops.conv_silu(proj, 8, w, b, ts, seg, s0, o0)
+    hops.conv_silu(proj.cuda(), 8, w.cuda(), b.cuda(), ts.cuda(), seg.cuda(), s1, o1)
+    assert torch.equal(s1.cpu(), s0)
+    assert ((o1.cpu().float() - o0.float()).abs() <= 2 ** -7 * o0.float().abs() + 1e-5).all()

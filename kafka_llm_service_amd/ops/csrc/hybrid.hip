@@ -847,28 +847,42 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   }
 }
 
-// out[h][t] = sum_z 2^(m_z - m) O_z / sum_z 2^(m_z - m) l_z over the key-range splits of latent_attn_mfma_kernel
-__global__ void latent_merge_kernel(const float* __restrict__ po, const float* __restrict__ pml, int nsplit, int H,
-                                    int T, int R, bf16* __restrict__ out, int64_t o_h, int64_t o_t,
-                                    const float* __restrict__ sink) {
-  const int64_t ht = blockIdx.x;  // h * T + t
-  const int h = (int)(ht / T), t = (int)(ht - (int64_t)h * T);
-  float mx = -INFINITY;
-  for (int z = 0; z < nsplit; ++z) mx = fmaxf(mx, pml[2 * ((int64_t)z * H * T + ht)]);
-  float den = 0.f;
-  for (int z = 0; z < nsplit; ++z) {
-    const float mz = pml[2 * ((int64_t)z * H * T + ht)];
-    if (mz != -INFINITY) den += fast_exp2(mz - mx) * pml[2 * ((int64_t)z * H * T + ht) + 1];
-  }
+// out[h][t] = sum_z 2^(m_z - m) O_z / sum_z 2^(m_z - m) l_z over the (at most 64) key-range splits. Bound by latency: lane z
+// holds split z's maximum and sum, and a thread's partials of four splits are in flight at a time (one after the other, 16 splits
+// of 512 rows took 15 us more).
+__global__ __launch_bounds__(128) void latent_merge_kernel(const float* __restrict__ po, const float* __restrict__ pml,
+                                                           int nsplit, int H, int T, int R, bf16* __restrict__ out,
+                                                           int64_t o_h, int64_t o_t, const float* __restrict__ sink) {
+  const int64_t ht = blockIdx.x, HT = (int64_t)H * T;  // h * T + t
+  const int h = (int)(ht / T), t = (int)(ht - (int64_t)h * T), lane = threadIdx.x & 63;
+  const float mz = lane < nsplit ? pml[2 * (lane * HT + ht)] : -INFINITY;
+  const float lz = lane < nsplit ? pml[2 * (lane * HT + ht) + 1] : 0.f;
+  float mx = mz;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  const float wz = mz == -INFINITY ? 0.f : fast_exp2(mz - mx);
+  float den = wz * lz;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) den += __shfl_xor(den, o, 64);
   if (sink != nullptr) den += fast_exp2(sink[h] * 1.4426950408889634f - mx);
   const float inv = 1.0f / den;
-  for (int d = threadIdx.x; d < R; d += blockDim.x) {
-    float a = 0.f;
+  for (int d0 = 0; d0 < R; d0 += 512) {   // (threadIdx.x + 128 k: R is a multiple of 32)
+    float a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
     for (int z = 0; z < nsplit; ++z) {
-      const float mz = pml[2 * ((int64_t)z * H * T + ht)];
-      if (mz != -INFINITY) a += fast_exp2(mz - mx) * po[((int64_t)z * H * T + ht) * R + d];
+      const float f = __shfl(wz, z, 64);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int d = d0 + threadIdx.x + 128 * k;
+        const float v = d < R ? po[(z * HT + ht) * R + d] : 0.f;
+        a[k] += f == 0.f ? 0.f : f * v;
+      }
     }
-    out[(int64_t)h * o_h + (int64_t)t * o_t + d] = (bf16)(a * inv);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int d = d0 + threadIdx.x + 128 * k;
+      if (d < R) out[(int64_t)h * o_h + (int64_t)t * o_t + d] = (bf16)(a[k] * inv);
+    }
   }
 }
 
@@ -1342,6 +1356,13 @@ using namespace kafka::hy;
 
 extern "C" {
 
+// attention in the latent space at kv_rank 512 (hybrid_latent.hip); scale in log2 units, partials as latent_merge_kernel's
+int kafka_hy_latent_decode_ok(const void* cache, int R, int rd, const void* out, int64_t o_h, int64_t o_t);
+hipError_t kafka_hy_latent_decode(const void* q_lat, int64_t ql_h, int64_t ql_t, const void* q_rot, int64_t qr_t, int64_t qr_h,
+                                  const void* cache, int rd, const int* bt, int bt_stride, const int* items, int n_items,
+                                  const int64_t* positions, float scale_log2e, void* out, int64_t o_h, int64_t o_t, int H,
+                                  int nsplit, float* po, float* pml, int T, int window, const float* sink, hipStream_t st);
+
 hipError_t kafka_hy_ln_shift(int f32, const float* x, int64_t xs, const void* w, const void* b, float eps, void* out,
                              int64_t os, int T, int d, const void* mu, const int* tok_seg, const int* seg,
                              float* state, float* last, hipStream_t st) {
@@ -1499,12 +1520,15 @@ hipError_t kafka_hy_latent_attn_mfma(const void* q_lat, int64_t ql_h, int64_t ql
                               po, pml, T, window, sink);
   };
   const int nks = Dk / 16;
-  if (tw == 1 && nks <= 12) a(latent_attn_mfma_kernel<1, 12>);
+  if (kafka_hy_latent_decode_ok(cache, R, rd, out, o_h, o_t)) {
+    const hipError_t e = kafka_hy_latent_decode(q_lat, ql_h, ql_t, q_rot, qr_t, qr_h, cache, rd, bt, bt_stride, items, n_items,
+                                                positions, sl, out, o_h, o_t, H, nsplit, po, pml, T, window, sink, st);
+    if (e != hipSuccess) return e;
+  } else if (tw == 1 && nks <= 12) a(latent_attn_mfma_kernel<1, 12>);
   else if (tw == 1) a(latent_attn_mfma_kernel<1, 40>);
   else if (tw == 2 && nks <= 24) a(latent_attn_mfma_kernel<2, 24>);
   else if (tw == 2) a(latent_attn_mfma_kernel<2, 40>);
   else if (tw == 3) a(latent_attn_mfma_kernel<3, 40>);
-  else if (nks <= 36) a(latent_attn_mfma_kernel<4, 36>);
   else a(latent_attn_mfma_kernel<4, 40>);
   if (nsplit > 1)
     latent_merge_kernel<<<(unsigned)((int64_t)H * T), 128, 0, st>>>(po, pml, nsplit, H, T, R, (bf16*)out, o_h, o_t,

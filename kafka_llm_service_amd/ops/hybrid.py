@@ -110,25 +110,26 @@ def tile_tokens(heads: int) -> int:
     return max(1, MFMA_ROWS // heads)
 
 
-ATTN_SPLIT_WGS = 256   # workgroups a matrix-core attention launch should reach before its key ranges are left whole
-ATTN_SPLIT_MAX = 16
+# Workgroups a matrix-core attention launch should reach before its key ranges are left whole, and the most ranges of a tile.
+# kv_rank 512, us by ranges: 64 sequences x 1706 keys 1: 95, 2: 60, 4: 44, 8: 59; 16 x 1706 4: 36, 8: 29, 16: 30; one x 1706 4: 35,
+# 8: 26, 16: 23, 32: 25; one x 8000 8: 63, 16: 41, 32: 34.
+ATTN_SPLIT_WGS = 256
+ATTN_SPLIT_MAX = 32
 
 
 def attn_splits(n_tiles: int, heads: int, max_keys: int) -> int:
     """Key-range splits of a matrix-core attention launch: few tiles (a decode step's one tile per sequence) against
-    long contexts are dealt over more workgroups, each at least two 128-key blocks long; a merge pass combines them."""
+    long contexts are dealt over more workgroups, each at least 128 keys long; a merge pass combines them."""
     wgs = n_tiles * -(-heads // MFMA_ROWS)
     blocks = -(-max_keys // 128)
-    if wgs >= ATTN_SPLIT_WGS // 2 or blocks < 4:
-        return 1
-    return max(1, min(ATTN_SPLIT_MAX, ATTN_SPLIT_WGS // wgs, blocks // 2))
+    return max(1, min(ATTN_SPLIT_MAX, ATTN_SPLIT_WGS // wgs, blocks))
 
 
 def latent_attn(q_lat, q_rot, cache, block_tables, tok_seg, seg, positions, scale, out, cache_t=None,
                 tiles=None, max_keys: int = 0, window: int = 0, sink=None) -> None:
     """Causal softmax attention of every row's heads over its sequence's cached [latent | rotated key] rows:
     out[h, t] = sum_j softmax_j((q_lat[h, t] . c_j + q_rot[t, h] . k_j) scale) c_j over the keys j <= position[t].
-    With the transposed latent copy ``cache_t`` and ``tiles`` (int32 [n, 4] = (first row, tokens, segment, 0), at
+    With the transposed latent copy ``cache_t`` (not read at kv_rank 512 with 0 or 64 rotated channels) and ``tiles`` (int32 [n, 4] = (first row, tokens, segment, 0), at
     most ``tile_tokens(H)`` tokens of one segment each) bf16 runs on the matrix cores; else one wave per (row, 4
     heads) on the vector units (fp32, odd sizes). ``max_keys`` (the step's longest context) lets a launch of few
     tiles split its key ranges over more workgroups (``attn_splits``).
@@ -399,6 +400,9 @@ def sigmoid_attn_mfma_ok(q, k_cache, v_cache_t, H: int, G: int) -> bool:
                                               H // G))
 
 
+SIG_SPLIT_MAX = 16
+
+
 def sig_splits(wgs: int, max_keys: int, target: int = ATTN_SPLIT_WGS) -> int:
     """Key-range splits of a matrix-core sigmoid attention launch: few workgroups (a decode step has one tile per
     sequence and key/value head) against long contexts are dealt over more (up to ``target`` in all), each at least
@@ -406,7 +410,7 @@ def sig_splits(wgs: int, max_keys: int, target: int = ATTN_SPLIT_WGS) -> int:
     blocks = -(-max_keys // 128)
     if wgs >= target // 2 or blocks < 4:
         return 1
-    return max(1, min(ATTN_SPLIT_MAX, target // max(1, wgs), blocks // 2))
+    return max(1, min(SIG_SPLIT_MAX, target // max(1, wgs), blocks // 2))
 
 
 def sigmoid_attn(q, q_off: int, k_cache, v_cache_t, block_tables, tok_seg, positions, H: int, G: int, scale: float,

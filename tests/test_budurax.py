@@ -355,6 +355,54 @@ def test_latent_attention_split_key_ranges(R, rd, H):
         assert torch.allclose(out[:, 0].float().cpu(), kvs[0][j, :R].float().expand(H, R), atol=6e-3), j
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,rd", [(32, 64), (16, 0), (40, 64), (1, 0)])
+@pytest.mark.parametrize("window,sink", [(0, False), (70, True)])
+def test_latent_decode_block_edges(H, rd, window, sink):
+    """kv_rank 512: contexts around the edges of pages and 64-key blocks, a tile of two tokens where the heads allow, several
+    splits (some empty), windows and sinks; what lies in the pages behind the last position is NaN. Latents of unit length: the
+    scores are up to 4.5 in bf16 products (relative 2^-9 each way, 0.02), weights rounded to bf16 (2^-9), outputs below 1."""
+    device, R, page = "cuda:0", 512, 16
+    torch.manual_seed(11)
+    lens = [1, 2, 16, 17, 63, 64, 65, 80, 127, 128, 129, 193, 300]
+    new = 2 if H <= 16 else 1
+    pages = [-(-(n + new - 1) // page) for n in lens]
+    cache = torch.full((sum(pages), page, R + rd), float("nan"), dtype=torch.bfloat16, device=device)
+    perm, at, kvs = torch.randperm(sum(pages)).tolist(), 0, []
+    bt = torch.zeros(len(lens), max(pages), dtype=torch.int32, device=device)
+    pos, tiles = [], []
+    for r, n in enumerate(lens):
+        kv = torch.nn.functional.normalize(torch.randn(n + new - 1, R + rd), dim=-1).bfloat16()
+        kvs.append(kv)
+        ids = perm[at:at + pages[r]]
+        at += pages[r]
+        bt[r, :pages[r]] = torch.tensor(ids)
+        for j in range(0, len(kv), page):
+            cache[ids[j // page], :len(kv[j:j + page])] = kv[j:j + page].to(device)
+        tiles.append((len(pos), new, r, 0))
+        pos += [n - 1 + i for i in range(new)]
+    T = len(pos)
+    q_lat, q_rot = torch.randn(H, T, R).bfloat16(), torch.randn(T, H, rd).bfloat16()
+    sk = torch.randn(H) if sink else None
+    cache_t = cache[:, :, :R].transpose(1, 2).contiguous()
+    g = [t.to(device) for t in (q_lat, q_rot)]
+    tt, ps = torch.tensor(tiles, dtype=torch.int32, device=device), torch.tensor(pos, device=device)
+    for ns in (1, 3):
+        out = torch.empty(T, H, R, dtype=torch.bfloat16, device=device).transpose(0, 1)
+        po, pml = (torch.empty(ns, H, T, w, device=device) for w in (R, 2))
+        hops.ext().hy_latent_attn_mfma(*g, cache, cache_t, bt, tt, hops.tile_tokens(H), ps, 0.3, out, ns,
+                                       po if ns > 1 else None, pml if ns > 1 else None, window,
+                                       sk.to(device) if sink else None)
+        for i, p in enumerate(pos):
+            lo = max(0, p - window + 1) if window else 0
+            kv = kvs[i // new][lo:p + 1].double()
+            s = (q_lat[:, i].double() @ kv[:, :R].T + q_rot[i].double() @ kv[:, R:].T) * 0.3
+            if sink:
+                s = torch.cat([s, sk.double()[:, None]], 1)
+            want = torch.softmax(s, -1)[:, :len(kv)] @ kv[:, :R]
+            assert torch.allclose(out[:, i].double().cpu(), want, atol=3e-3), (ns, i, p)
+
+
 def cfg_m():
     """Sizes the matrix-core attention kernel takes (latent 64, rotary part 16), two attention layers sharing a cache."""
     ff = {"kind": "dense", "ff": 96}

@@ -1,11 +1,11 @@
 // Latent attention for gfx950 (bf16): prompt portions on expanded keys and values; single tokens at kv_rank 512.
 //
 // A latent-attention layer caches one latent row c (and one rotated key part) per token; head h's key and value are
-// W_uk,h c and W_uv,h c. A decoded token attends in the latent space (latent_decode, for other ranks
-// hybrid.hip): its cost is the cache, read once for all heads, and nothing per head is materialised. A portion of many rows is bound by its products instead, and there the
-// latent space is the dear one: 2 (kv_rank + rot_dim) + 2 kv_rank multiply-adds per (row, key, head) against
-// 2 (dim + rot_dim) + 2 vdim on the heads' own keys and values (2176 against 640 at 512 / 64 / 128 / 128), which cost one
-// product of kv_rank x (dim + vdim) per key and head, however many rows follow.
+// W_uk,h c and W_uv,h c. A decoded token attends in the latent space (latent_decode, for other ranks hybrid.hip): its cost is the
+// cache, read once for all heads, and nothing per head is materialised. A portion of many rows is bound by its products
+// instead, and there the latent space is the dear one: 2 (kv_rank + rot_dim) + 2 kv_rank multiply-adds per (row, key, head)
+// against 2 (dim + rot_dim) + 2 vdim on the heads' own keys and values (2176 against 640 at 512 / 64 / 128 / 128), which cost
+// one product of kv_rank x (dim + vdim) per key and head, however many rows follow.
 //   latent_gather  the context's cache rows (all of it, or what the window reaches) one below the other: latents [M, kv_rank]
 //                  for the two products K = C W_uk^T and V^T = W_uv C^T, rotated parts [M, rot_dim]
 //   latent_rows    softmax attention of one head's rows against them

@@ -700,6 +700,223 @@ __global__ __launch_bounds__(256, NKS * 4 + NVT * 16 <= 96 ? 2 : 1) void window_
     }
 }
 
+// ---- the same for long portions, 128 channels: eight items share their keys in LDS -----------------------------------------
+// A workgroup takes eight neighbouring items of one key/value head, a wave each (as above: S^T = K Q^T, the weights stay in
+// registers, O^T += V^T P^T), and walks the union of their keys 64 at a time: K and V^T pages go to a ring of three slots in LDS
+// without a register on the way, two tiles ahead. Chunk c (16 bytes) of key row k lies at c ^ k of its page, the halves of
+// channels 8 .. 15 of every 16 in a V^T page are swapped: every operand read meets all banks once. Items of different segments
+// go one segment after the other, the rest of the workgroup helps loading. The accumulators are rescaled only when a row's
+// maximum has grown by more than 2^WT_THR.
+// What bounds it: products and softmax of two waves a SIMD; above, each wave's operands came through the caches. 8192 fresh rows
+// x 32 heads over 8 1287 -> 649 us (0.85 PFLOP/s), 3 x 1100 rows, 32 over 2, 108 -> 65, 4096 rows with a window of 1024 175 -> 97.
+constexpr int WT_WAVES = 8, WT_KEYS = 64, WT_SLOTS = 3, WT_RUN = 512;   // WT_RUN: tiles whose page ids lie in LDS at a time
+constexpr int WT_KB = WT_KEYS * 256, WT_SLOT = 2 * WT_KB;
+constexpr float WT_THR = 8.f;
+// Items x key/value heads from which it runs: a wave each on 256 CUs, fewer leave whole CUs idle that the form above still uses.
+// us there / here: 1000 waves (1000 rows) 33 / 40, 1024 (2048 rows, 4 heads) 62 / 66, 1200 47 / 45, 1500 63 / 60, 2048 with a
+// window of 1024 85 / 45.
+constexpr int WT_MIN_WAVES = 1280;
+
+typedef __attribute__((address_space(3))) void wt_lds_t;
+template <int OFF>
+__device__ __forceinline__ void wt_dma16(const void* g, void* lds) {
+  __builtin_amdgcn_global_load_lds(g, (wt_lds_t*)lds, 16, OFF, 0);
+}
+__device__ __forceinline__ float wt_max(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+
+__global__ __launch_bounds__(512, 2) void window_attn_tile_kernel(
+    const bf16* __restrict__ q, int64_t qs, const bf16* __restrict__ kc, const bf16* __restrict__ vt,
+    const int* __restrict__ bt, int bt_stride, const int* __restrict__ items, int n_items,
+    const int64_t* __restrict__ positions, int H, int G, int Ck, int kstep, float scale_log2e, int window,
+    const float* __restrict__ sink, const bf16* __restrict__ gate, int64_t gs, bf16* __restrict__ out, int64_t os,
+    float out_scale, int min_tok, bool vec4) {
+  constexpr int D = 128, Dv = 128, NKS = 8, NVT = 4;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[WT_SLOTS * WT_SLOT + 4 * WT_RUN * 4 + WT_WAVES * 16];
+  int* pg_s = reinterpret_cast<int*>(smem + WT_SLOTS * WT_SLOT);   // [4 WT_RUN]
+  int4* who = reinterpret_cast<int4*>(pg_s + 4 * WT_RUN);          // [waves] (segment or -1, first tile, end tile, last page)
+  const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int item = n_items - 1 - ((int)blockIdx.y * WT_WAVES + w);
+  int t0 = 0, ntok = 0, sg = -1;
+  if (item >= 0) {
+    t0 = items[4 * item];
+    ntok = items[4 * item + 1];
+    sg = ntok >= min_tok ? items[4 * item + 2] : -1;
+  }
+  const bool mine = sg >= 0;   // (uniform per wave)
+  const int g = blockIdx.x, rep = H / G, nrows = max(ntok, 1) * rep, Cv = G * Dv;
+  const int row = min(lr, nrows - 1), h = g * rep + row % rep;
+  const int64_t t = t0 + row / rep;
+  int p = -1, minpos = 0, maxpos = -1;
+  bf16x8 qf[NKS];
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks) qf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  if (mine) {
+    p = (int)positions[t];
+    minpos = (int)positions[t0];
+    maxpos = (int)positions[t0 + ntok - 1];
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) qf[ks] = load_bf16x8(q + t * qs + (int64_t)h * D + 16 * ks + 8 * lh);
+  }
+  const int jb = window > 0 ? max(0, minpos - window + 1) / WT_KEYS : 0, je = maxpos / WT_KEYS + 1;   // tiles of this wave
+  if (lane == 0) who[w] = int4{sg, jb, je, maxpos >> 4};
+  const int krow = (lr & 19) | ((lr & 4) << 1) | ((lr & 8) >> 1), kk = krow & 15;   // bits 2 and 3 swapped
+  int kat[NKS], vat[NVT];   // operands' places in a slot
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks) kat[ks] = (krow >> 4) * 4096 + kk * 256 + 16 * ((2 * ks + lh) ^ kk);
+#pragma unroll
+  for (int v = 0; v < NVT; ++v) vat[v] = WT_KB + (32 * v + lr) * 32 + 16 * (lh ^ ((lr >> 3) & 1));
+  // wave w copies half w & 1 of page w >> 1 of a tile: two 1-KiB pieces of K and of V^T
+  const int pw = w >> 1, c0 = (w & 1) * 2048;
+  const int vsrc = c0 + (lane ^ ((lane >> 4) & 1)) * 16;
+  int ksrc[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int k = 8 * (w & 1) + 4 * c + (lane >> 4);
+    ksrc[c] = k * Ck * 2 + 16 * ((lane & 15) ^ k);
+  }
+  auto issue = [&](int j) {   // tile j of the run
+    const int64_t pg = __builtin_amdgcn_readfirstlane(pg_s[4 * j + pw]);
+    const char* kp = reinterpret_cast<const char*>(kc + pg * PAGE * Ck + (int64_t)g * kstep);
+    const char* vp = reinterpret_cast<const char*>(vt + (pg * Cv + (int64_t)g * Dv) * PAGE);
+    unsigned char* dst = smem + (j % WT_SLOTS) * WT_SLOT + pw * 4096 + c0;
+    wt_dma16<0>(kp + ksrc[0], dst);
+    wt_dma16<0>(kp + ksrc[1], dst + 1024);
+    wt_dma16<0>(vp + vsrc, dst + WT_KB);
+    wt_dma16<1024>(vp + vsrc, dst + WT_KB);
+  };
+  float m = -INFINITY, l = 0.f;
+  f32x16 O[NVT];
+#pragma unroll
+  for (int v = 0; v < NVT; ++v)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) O[v][i] = 0.f;
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // (vmcnt(0): left open, the queries' loads are waited for, with the tiles', in every step)
+  lds_barrier();
+  for (int a = 0; a < WT_WAVES;) {   // (uniform) waves a .. b - 1 walk one segment
+    const int4 wa = who[a];
+    const int seg = __builtin_amdgcn_readfirstlane(wa.x);
+    int b = a + 1, lo = __builtin_amdgcn_readfirstlane(wa.y), hi = __builtin_amdgcn_readfirstlane(wa.z),
+        lastpg = __builtin_amdgcn_readfirstlane(wa.w);
+    for (; b < WT_WAVES; ++b) {
+      const int4 wb = who[b];
+      if (__builtin_amdgcn_readfirstlane(wb.x) != seg) break;
+      lo = min(lo, __builtin_amdgcn_readfirstlane(wb.y));
+      hi = max(hi, __builtin_amdgcn_readfirstlane(wb.z));
+      lastpg = max(lastpg, __builtin_amdgcn_readfirstlane(wb.w));
+    }
+    const bool on = w >= a && w < b;
+    a = b;
+    if (seg < 0) continue;
+    const int* btr = bt + (int64_t)seg * bt_stride;
+    for (int run = lo; run < hi; run += WT_RUN) {
+      const int n = min(hi - run, WT_RUN);
+      for (int i = threadIdx.x; i < 4 * n; i += 512) pg_s[i] = btr[min(4 * run + i, lastpg)];   // (past the last page: it again)
+      lds_barrier();
+      issue(0);
+      if (n > 1) issue(1);
+      for (int j = 0; j < n; ++j) {
+        // this wave's pieces of the tile have landed (the next tile's stay on their way), then everyone's; everyone has left
+        // the tile before, whose slot the one after next takes
+        if (j + 1 < n)
+          asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        else
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        lds_barrier();
+        if (j + 2 < n) issue(j + 2);
+        const int key0 = (run + j) * WT_KEYS;
+        if (!on || run + j < jb || run + j >= je) continue;
+        const unsigned char* sl = smem + (j % WT_SLOTS) * WT_SLOT;
+        f32x16 S[2];
+#pragma unroll
+        for (int sb = 0; sb < 2; ++sb) {
+          bf16x8 kf[NKS];
+#pragma unroll
+          for (int ks = 0; ks < NKS; ++ks) kf[ks] = *reinterpret_cast<const bf16x8*>(sl + kat[ks] + sb * 8192);
+          f32x16 acc = {};
+#pragma unroll
+          for (int ks = 0; ks < NKS; ++ks) acc = mfma32(kf[ks], qf[ks], acc);
+          S[sb] = acc;
+        }
+        // (uniform) a tile that every row sees whole needs no mask
+        if (key0 + WT_KEYS - 1 > minpos || (window > 0 && key0 <= maxpos - window)) {
+#pragma unroll
+          for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const int key = key0 + 32 * sb + 16 * (i >> 3) + 8 * lh + (i & 7);
+              if (key > p || (window > 0 && key <= p - window)) S[sb][i] = -INFINITY;
+            }
+        }
+        float ma = wt_max(S[0][0], S[1][0]), mb = wt_max(S[0][1], S[1][1]);
+#pragma unroll
+        for (int i = 2; i < 16; i += 2) {
+          ma = wt_max(wt_max(ma, S[0][i]), S[1][i]);
+          mb = wt_max(wt_max(mb, S[0][i + 1]), S[1][i + 1]);
+        }
+        float mx = wt_max(ma, mb);
+        {
+          const auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+          mx = wt_max(__uint_as_float(r2[0]), __uint_as_float(r2[1])) * scale_log2e;   // (the scale is positive)
+        }
+        if (__any(!(mx <= m + WT_THR))) {
+          const float mn = fmaxf(m, mx);
+          const float corr = mn == -INFINITY ? 1.f : fast_exp2(m - mn);
+          l *= corr;
+#pragma unroll
+          for (int v = 0; v < NVT; ++v) O[v] *= corr;
+          m = mn;
+        }
+        const float base = m == -INFINITY ? 0.f : m;   // nothing visible yet: every weight is 2^-inf = 0
+#pragma unroll
+        for (int sb = 0; sb < 2; ++sb) {
+          bf16x8 vf[2][NVT];
+#pragma unroll
+          for (int pg = 0; pg < 2; ++pg)
+#pragma unroll
+            for (int v = 0; v < NVT; ++v) vf[pg][v] = *reinterpret_cast<const bf16x8*>(sl + vat[v] + sb * 8192 + pg * 4096);
+          bf16x8 pf[2];
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const float e = fast_exp2(fmaf(S[sb][i], scale_log2e, -base));
+            l += e;
+            pf[i >> 3][i & 7] = (bf16)e;
+          }
+#pragma unroll
+          for (int pg = 0; pg < 2; ++pg)
+#pragma unroll
+            for (int v = 0; v < NVT; ++v) O[v] = mfma32(vf[pg][v], pf[pg], O[v]);
+        }
+      }
+      lds_barrier();   // (the run's page ids and slots have been read)
+    }
+  }
+  // the last products' results are complete before anything reads them behind a branch
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_nop 15");
+  __builtin_amdgcn_sched_barrier(0);
+  l += __shfl_xor(l, 32, 64);
+  if (!mine || lr >= nrows) return;
+  if (sink != nullptr) l += fast_exp2(sink[h] * LOG2E - m);
+  float inv = out_scale / l;
+  if (gate != nullptr) inv *= head_gate(gate + t * gs + h);
+  bf16* op = out + t * os + (int64_t)h * Dv;
+#pragma unroll
+  for (int v = 0; v < NVT; ++v)
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      const int c = 32 * v + 8 * i4 + 4 * lh;
+      typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
+      const bf16x4 o = {(bf16)(O[v][4 * i4] * inv), (bf16)(O[v][4 * i4 + 1] * inv), (bf16)(O[v][4 * i4 + 2] * inv),
+                        (bf16)(O[v][4 * i4 + 3] * inv)};
+      if (vec4) {
+        *reinterpret_cast<bf16x4*>(op + c) = o;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) op[c + e] = o[e];
+      }
+    }
+}
+
 // out[t][h] = sum_z 2^(m_z - m) O_z / (sum_z 2^(m_z - m) l_z + 2^(sink_h - m)) over the key-range splits
 __global__ void window_merge_kernel(const float* __restrict__ po, const float* __restrict__ pml, int nsplit, int64_t T,
                                     int H, int Dv, const float* __restrict__ sink, const bf16* __restrict__ gate,
@@ -996,7 +1213,12 @@ hipError_t kafka_hy_window_attn_mfma(const void* q, int64_t qs, const void* kc, 
                                    positions, H, G, D, Dv, Ck, kstep, scale * LOG2E, window, sink, (const bf16*)gate, gs,
                                    (bf16*)out, os, out_scale, min_rows_tok, vec4);
     };
-    if (D <= 64) {
+    const bool al = ((reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vt)) & 15) == 0;
+    if (D == 128 && Dv == 128 && al && scale > 0.f && (int64_t)n_items * G >= WT_MIN_WAVES) {
+      window_attn_tile_kernel<<<dim3((unsigned)G, (unsigned)((n_items + WT_WAVES - 1) / WT_WAVES)), 64 * WT_WAVES, 0, st>>>(
+          (const bf16*)q, qs, (const bf16*)kc, (const bf16*)vt, bt, bt_stride, items, n_items, positions, H, G, Ck, kstep,
+          scale * LOG2E, window, sink, (const bf16*)gate, gs, (bf16*)out, os, out_scale, min_rows_tok, vec4);
+    } else if (D <= 64) {
       if (Dv <= 64) b(window_attn_rows_kernel<4, 2>);
       else if (Dv <= 128) b(window_attn_rows_kernel<4, 4>);
       else b(window_attn_rows_kernel<4, 8>);

@@ -1041,3 +1041,48 @@ def test_wide_expert_products_on_256_row_tiles(rows, N, K):
         ref = gate * torch.sigmoid(kw.get("alpha", 1.0) * gate) * up
         assert same(ops.grouped_wide(x, gt, r, "glu", True, tile=256, **kw), ref)
         assert same(ops.grouped_wide(x, gt, r, "glu", True, tile=128, **kw), ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("window,sink,cols", [(0, False, 0), (100, True, 3)])
+def test_window_attention_of_long_portions(window, sink, cols):
+    """Enough prompt rows for the kernel whose eight items share their keys in LDS: segments of odd lengths that end within a
+    workgroup, some behind a history, outputs in rows that are no multiple of 8 bytes. Values up to 4.5: a weight's rounding to
+    bf16 (2^-9 of each term) and the result's (2^-9) move an output by up to 0.018."""
+    dev, H, G, D = "cuda:0", 64, 2, 128
+    torch.manual_seed(23)
+    segs = [(1, 40), (37, 0), (64, 0), (65, 31), (200, 0), (290, 75)]     # rows, history
+    pages = [-(-(n + p0) // 16) for n, p0 in segs]
+    perm = torch.randperm(sum(pages))
+    kc, vt = torch.randn(sum(pages), 16, G * D).bfloat16(), torch.randn(sum(pages), G * D, 16).clamp(-4.5, 4.5).bfloat16()
+    bt = torch.zeros(len(segs), max(pages), dtype=torch.int32)
+    tiles, pos, at = [], [], 0
+    for r, (n, p0) in enumerate(segs):
+        bt[r, :pages[r]] = perm[at:at + pages[r]]
+        at += pages[r]
+        tiles += [(len(pos) + i, 1, r, 0) for i in range(n)]
+        pos += list(range(p0, p0 + n))
+    T = len(pos)
+    assert T * G >= 1280
+    q, sk = torch.randn(T, H * D).bfloat16(), torch.randn(H)
+    gate = torch.randn(T, H + 1).bfloat16()
+    out = torch.empty(T, H * D + cols, dtype=torch.bfloat16, device=dev)[:, cols:]
+    g = [t.to(dev) for t in (q, kc, vt, bt)]
+    hops.window_attn(*g, None, torch.tensor(pos, device=dev), H, G, D ** -0.5, window, sk.to(dev) if sink else None, out,
+                     torch.tensor(tiles, dtype=torch.int32, device=dev), 365, gate=gate.to(dev), gate_off=1, kinds=(False, True))
+    at = 0
+    for r, (n, p0) in enumerate(segs):
+        pg = bt[r, :pages[r]].long()
+        k = kc[pg].reshape(-1, G, D).double()[:p0 + n]
+        v = vt[pg].view(-1, G, D, 16).permute(0, 3, 1, 2).reshape(-1, G, D).double()[:p0 + n]
+        qq = q[at:at + n].view(n, G, H // G, D).double()
+        s = torch.einsum("ngrd,kgd->ngrk", qq, k) * D ** -0.5
+        j, p = torch.arange(p0 + n), torch.arange(p0, p0 + n)[:, None]
+        see = (j <= p) & (j > p - window if window else torch.ones_like(j, dtype=torch.bool))
+        s = s.masked_fill(~see[:, None, None], float("-inf"))
+        if sink:
+            s = torch.cat([s, sk.double().view(1, G, H // G, 1).expand(n, -1, -1, -1)], -1)
+        want = torch.einsum("ngrk,kgd->ngrd", torch.softmax(s, -1)[..., :p0 + n], v).reshape(n, H, D)
+        want = want * torch.sigmoid(gate[at:at + n, 1:].double())[..., None]
+        assert torch.allclose(out[at:at + n].double().cpu().view(n, H, D), want, atol=2e-2), r
+        at += n

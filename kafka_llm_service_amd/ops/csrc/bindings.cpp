@@ -83,8 +83,9 @@ hipError_t kafka_launch_moe_route(const bf16* logits, int64_t ld, int T, int E, 
                                   int* topk_e, int* perm_tok, float* perm_w, int* expert_off, int* tile_off,
                                   hipStream_t st);
 int kafka_moe_sort_max_e();
+int kafka_moe_sort_parts(int n, int E);
 hipError_t kafka_launch_moe_sort(const float* topk_w, const int* topk_e, int n, int k, int E, int bm, int* perm_tok,
-                                 float* perm_w, int* expert_off, int* tile_off, int* inv, hipStream_t st);
+                                 float* perm_w, int* expert_off, int* tile_off, int* inv, int* counts, hipStream_t st);
 hipError_t kafka_launch_grouped_wide(const bf16* X, int64_t ldx, const bf16* Wt, int E, int N, int K,
                                      const int* perm_tok, const float* perm_w, const int* expert_off, int n_ent,
                                      int gather, int epi, bf16* Y, int64_t ldy, float* out, int64_t ldo,
@@ -870,9 +871,12 @@ static void moe_sort(at::Tensor topk_w, at::Tensor topk_e, int64_t E, int64_t bm
     ip = inv->data_ptr<int>();
   }
   if (E <= kafka_moe_sort_max_e() && T * k < (int64_t)1 << 30) {
+    const int parts = kafka_moe_sort_parts((int)(T * k), (int)E);
+    const at::Tensor counts = parts > 1 ? at::empty({64 * parts}, topk_e.options()) : at::Tensor();
     CHECK_HIP(kafka_launch_moe_sort(topk_w.data_ptr<float>(), topk_e.data_ptr<int>(), (int)(T * k), (int)k, (int)E,
                                     (int)bm, perm_tok.data_ptr<int>(), perm_w.data_ptr<float>(),
-                                    expert_off.data_ptr<int>(), tile_off.data_ptr<int>(), ip, cur_stream()));
+                                    expert_off.data_ptr<int>(), tile_off.data_ptr<int>(), ip,
+                                    parts > 1 ? counts.data_ptr<int>() : nullptr, cur_stream()));
     return;
   }
   CHECK_HIP(kafka_launch_moe_route(nullptr, 0, (int)T, (int)E, (int)k, (int)bm, topk_w.data_ptr<float>(),

@@ -16,7 +16,7 @@
 //   narrow         fp32 products of bf16 rows with up to 64 bf16 weight rows (router logits, gate projections): 16 rows a
 //                  workgroup, its 16 (or 8) waves split K, 16x16x32 products; with a bias, or followed in place by the
 //                  choice of the k largest scores, a wave per row
-#include "common.h"
+#include "moe_sort.h"
 
 namespace kafka {
 namespace mw {
@@ -397,7 +397,6 @@ __global__ __launch_bounds__(256, 1) void grouped_ring_kernel(const bf16* __rest
 }
 
 // ---- stable sort by expert --------------------------------------------------------------------------------------------
-constexpr int SORT_NT = 1024, SORT_W = SORT_NT / 64;
 constexpr int SORT_MAXE = 512;
 
 // lanes of the wave whose (valid) entry has this lane's expert
@@ -410,6 +409,33 @@ __device__ __forceinline__ unsigned long long same_expert(int e, bool valid, int
   return m;
 }
 
+__global__ __launch_bounds__(SORT_NT) void moe_sort_few_kernel(const float* __restrict__ topk_w, const int* __restrict__ topk_e,
+                                                               int n, int k, int E, int bits, int bm,
+                                                               int* __restrict__ perm_tok, float* __restrict__ perm_w,
+                                                               int* __restrict__ expert_off, int* __restrict__ tile_off,
+                                                               int* __restrict__ inv, const int* __restrict__ counts) {
+  __shared__ int cnt[SORT_W][64];
+  const int lo = gridDim.x > 1 ? blockIdx.x * SORT_PART : 0, hi = gridDim.x > 1 ? min(n, lo + SORT_PART) : n;
+  sort_few_experts(topk_w, topk_e, lo, hi, k, E, bits, bm, perm_tok, perm_w, expert_off, tile_off, inv, counts, blockIdx.x,
+                   gridDim.x, cnt);
+}
+
+// how many of the part's entries go to expert `lane`
+__global__ __launch_bounds__(SORT_NT) void moe_sort_count_kernel(const int* __restrict__ topk_e, int n, int E, int bits,
+                                                                 int* __restrict__ counts) {
+  __shared__ int cnt[SORT_W][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lo = blockIdx.x * SORT_PART;
+  const int c = sort_count(topk_e, sort_stretch(lo, min(n, lo + SORT_PART), w), bits);
+  cnt[w][lane] = lane < E ? c : 0;
+  __syncthreads();
+  if (w > 0) return;
+  int tot = 0;
+#pragma unroll
+  for (int i = 0; i < SORT_W; ++i) tot += cnt[i][lane];
+  counts[64 * blockIdx.x + lane] = tot;
+}
+
+// more experts: a counter in LDS per wave and expert
 __global__ __launch_bounds__(SORT_NT) void moe_sort_kernel(const float* __restrict__ topk_w,
                                                            const int* __restrict__ topk_e, int n, int k, int E, int bits,
                                                            int bm, int* __restrict__ perm_tok,
@@ -575,6 +601,20 @@ __global__ __launch_bounds__(64 * nr_waves(TN)) void narrow_linear_kernel(const 
   }
 }
 
+// lane exchange within 16 lanes: the neighbour, the pair's neighbour, the mirrored half, the mirrored 16
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+template <typename OP>
+__device__ __forceinline__ float row16(float v, OP op) {
+  v = op(v, dpp<0xB1>(v));
+  v = op(v, dpp<0x4E>(v));
+  v = op(v, dpp<0x141>(v));
+  return op(v, dpp<0x140>(v));
+}
+
+// up to 16 experts live in the first 16 lanes (the others run along): exchanges without LDS, 16 rows of 4096 12.2 -> 10.9 us
 // softmax over all N experts, the k largest (ties: the lower index), their scores as weights (norm: divided by their sum)
 // times scale; lane = expert
 template <int TN>
@@ -590,20 +630,30 @@ __global__ __launch_bounds__(64 * nr_waves(TN)) void narrow_route_kernel(const b
     const int64_t t = (int64_t)blockIdx.x * NR_ROWS + row;
     if (t >= T) break;   // (uniform)
     const float z = lane < N ? part[0][row][lane] : -INFINITY;
-    const float mx = wave_max(z), ex = lane < N ? expf(z - mx) : 0.f;
-    const float s = ex / wave_sum(ex);
+    const float mx = TN == 1 ? row16(z, [](float a, float b) { return fmaxf(a, b); }) : wave_max(z);
+    const float ex = lane < N ? expf(z - mx) : 0.f;
+    const float s = ex / (TN == 1 ? row16(ex, [](float a, float b) { return a + b; }) : wave_sum(ex));
     float c = lane < N ? s : -1.f, mine = 0.f, sum = 0.f;
     int me = 0;
     for (int j = 0; j < k; ++j) {
       float bv = c;
       int bi = lane;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(bv, o, 64);
-        const int oi = __shfl_xor(bi, o, 64);
+      auto take = [&](float ov, int oi) {
         if (ov > bv || (ov == bv && oi < bi)) {
           bv = ov;
           bi = oi;
+        }
+      };
+      if constexpr (TN == 1) {
+        take(dpp<0xB1>(bv), __float_as_int(dpp<0xB1>(__int_as_float(bi))));
+        take(dpp<0x4E>(bv), __float_as_int(dpp<0x4E>(__int_as_float(bi))));
+        take(dpp<0x141>(bv), __float_as_int(dpp<0x141>(__int_as_float(bi))));
+        take(dpp<0x140>(bv), __float_as_int(dpp<0x140>(__int_as_float(bi))));
+      } else {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+          const float ov = __shfl_xor(bv, o, 64);
+          take(ov, __shfl_xor(bi, o, 64));
         }
       }
       if (lane == j) {
@@ -630,14 +680,23 @@ extern "C" {
 
 int kafka_moe_sort_max_e() { return SORT_MAXE; }
 
+// workgroups of a sort (its scratch: 64 counts each): one up to 4096 entries, where a second launch costs what it saves
+int kafka_moe_sort_parts(int n, int E) { return E > 64 || n <= 2 * SORT_PART ? 1 : (n + SORT_PART - 1) / SORT_PART; }
+
 hipError_t kafka_launch_moe_sort(const float* topk_w, const int* topk_e, int n, int k, int E, int bm, int* perm_tok,
-                                 float* perm_w, int* expert_off, int* tile_off, int* inv, hipStream_t st) {
+                                 float* perm_w, int* expert_off, int* tile_off, int* inv, int* counts, hipStream_t st) {
   if (n < 1) return hipSuccess;
   if (E < 1 || E > SORT_MAXE || k < 1 || bm < 1) return hipErrorInvalidValue;
   int bits = 0;
   while ((1 << bits) < E) ++bits;
-  moe_sort_kernel<<<1, SORT_NT, 0, st>>>(topk_w, topk_e, n, k, E, bits, bm, perm_tok, perm_w, expert_off, tile_off,
-                                        inv);
+  if (E > 64) {
+    moe_sort_kernel<<<1, SORT_NT, 0, st>>>(topk_w, topk_e, n, k, E, bits, bm, perm_tok, perm_w, expert_off, tile_off, inv);
+    return hipGetLastError();
+  }
+  const int parts = counts != nullptr ? kafka_moe_sort_parts(n, E) : 1;
+  if (parts > 1) moe_sort_count_kernel<<<parts, SORT_NT, 0, st>>>(topk_e, n, E, bits, counts);
+  moe_sort_few_kernel<<<parts, SORT_NT, 0, st>>>(topk_w, topk_e, n, k, E, bits, bm, perm_tok, perm_w, expert_off, tile_off, inv,
+                                                 counts);
   return hipGetLastError();
 }
 

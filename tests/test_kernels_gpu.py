@@ -852,3 +852,18 @@ def test_linear_dense_blocks(M, N):
     want = x.float() @ w.float().t()
     got = ops.linear_dense(x, w).float()
     assert ((got - want).abs() <= 2 ** -8 * want.abs() + 1e-2).all()
+
+
+@pytest.mark.parametrize("T,k", [(1, 1), (63, 1), (65, 1), (1024, 4), (4097, 1), (683, 6), (2731, 3)])
+@pytest.mark.parametrize("E", [1, 5, 64, 65])
+def test_moe_sort_sizes(cuda, T, k, E):
+    """The sort by expert where its forms meet: full and ragged waves, one workgroup or parts of 2048 entries, 64 experts and
+    more, experts without entries (only the odd ones get any from 5 on)."""
+    torch.manual_seed(T + E)
+    k = min(k, E)   # (more choices than experts are refused)
+    te = torch.randint(0, E, (T, k), dtype=torch.int32) | (1 if E > 1 else 0)
+    te = te.clamp(max=E - 1)
+    tw = torch.rand(T, k)
+    r, c = ops.moe_sort(tw.to(cuda), te.to(cuda), E, inverse=True), ops.moe_sort(tw, te, E, inverse=True)
+    for a in ("perm_tok", "perm_w", "expert_off", "tile_off", "inv"):
+        assert torch.equal(getattr(r, a).cpu(), getattr(c, a)), a

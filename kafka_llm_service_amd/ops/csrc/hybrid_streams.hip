@@ -26,6 +26,8 @@
 //                       their two largest) by corrected score, weights normalised or as they are, times a scale
 #include "common.h"
 
+#include <type_traits>
+
 namespace kafka {
 namespace hs {
 
@@ -383,7 +385,23 @@ __global__ __launch_bounds__(NT) void window_attn_kernel(const AT* __restrict__ 
 // gridDim.z > 1 the tile's key blocks are dealt to gridDim.z workgroups in contiguous ranges; each leaves its
 // unnormalised accumulators in po [z][T][H Dv] and (row maximum, row sum) in pml [z][T][H][2] for window_merge.
 // Needs 16-token pages, D % 16 == 0, at most 32 query heads per key/value head.
+// What bounds it: a block's chain of key loads, maxima, weights and value loads. A decoded token fills few of the 32 rows, and
+// the others' softmax is left out (their weights in LDS stay zero); maxima go lane to lane without LDS. With the merge, before / now,
+// us: 16 sequences x 1700 keys, 32 heads over 8, 40 / 31, 64 sequences 120 / 103, one x 8000 43 / 27,
+// 16 sequences, 32 over 2, 25 / 19.
 constexpr int WM_ROWS = 32;
+
+// the largest of a lane half's 32 values, in each of its lanes: neighbours, pairs, mirrored eights and sixteens, the other sixteen
+__device__ __forceinline__ float max32(float v) {
+  auto dpp = [](float x, auto c) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(c)::value, 0xf, 0xf, false));
+  };
+  v = fmaxf(v, dpp(v, std::integral_constant<int, 0xB1>()));
+  v = fmaxf(v, dpp(v, std::integral_constant<int, 0x4E>()));
+  v = fmaxf(v, dpp(v, std::integral_constant<int, 0x141>()));
+  v = fmaxf(v, dpp(v, std::integral_constant<int, 0x140>()));
+  return fmaxf(v, __shfl_xor(v, 16, 64));
+}
 
 template <int TW, int NKSC>
 __global__ __launch_bounds__(256) void window_attn_mfma_kernel(
@@ -404,6 +422,7 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(
   if (ntok > max_tok) return;   // (uniform) an item of window_attn_rows
   const int g = blockIdx.y, rep = H / G;
   const int nrows = ntok * rep;
+  for (int i = threadIdx.x; i < WM_ROWS * 136 / 8; i += 256) store_bf16x8(Ps + 8 * i, bf16x8{0, 0, 0, 0, 0, 0, 0, 0});
   for (int i = threadIdx.x; i < WM_ROWS * (D >> 3); i += 256) {
     const int r = i / (D >> 3), d0 = (i - r * (D >> 3)) << 3;
     bf16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -459,34 +478,33 @@ __global__ __launch_bounds__(256) void window_attn_mfma_kernel(
     float s[16], mx[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
+      if (8 * (i >> 2) >= nrows) break;   // (uniform) a decoded token has few rows
       s[i] = (any && key <= prow[i] && (window == 0 || key > prow[i] - window)) ? S[i] * scale_log2e : -INFINITY;
-      float v = s[i];
-#pragma unroll
-      for (int o = 16; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-      mx[i] = v;
+      mx[i] = max32(s[i]);
     }
     if (lr == 0) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mloc[w * 32 + (i & 3) + 8 * (i >> 2) + 4 * lh] = mx[i];
+      for (int i = 0; i < 16; ++i) {
+        if (8 * (i >> 2) >= nrows) break;
+        mloc[w * 32 + (i & 3) + 8 * (i >> 2) + 4 * lh] = mx[i];
+      }
     }
     lds_barrier();
-    float corr[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
+      if (8 * (i >> 2) >= nrows) break;
       const int r = (i & 3) + 8 * (i >> 2) + 4 * lh;
       const float mn = fmaxf(fmaxf(m[i], fmaxf(mloc[r], mloc[32 + r])), fmaxf(mloc[64 + r], mloc[96 + r]));
       // first block: m = -inf -> corr 0. A range may lie wholly outside a row's window: then mn is still -inf and
       // the row stays empty (the guards keep inf - inf out)
-      corr[i] = mn == -INFINITY ? 0.f : fast_exp2(m[i] - mn);
+      const float corr = mn == -INFINITY ? 0.f : fast_exp2(m[i] - mn);
       const float p = mn == -INFINITY ? 0.f : fast_exp2(s[i] - mn);
-      lsum[i] = lsum[i] * corr[i] + p;
+      lsum[i] = lsum[i] * corr + p;
       m[i] = mn;
       Ps[r * 136 + 32 * w + lr] = (bf16)p;
+#pragma unroll
+      for (int tw = 0; tw < TW; ++tw) O[tw][i] *= corr;
     }
-#pragma unroll
-    for (int tw = 0; tw < TW; ++tw)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) O[tw][i] *= corr[i];
     lds_barrier();
     // ---- values: one page (16 keys) per step
 #pragma unroll
@@ -917,31 +935,45 @@ __global__ __launch_bounds__(512, 2) void window_attn_tile_kernel(
     }
 }
 
-// out[t][h] = sum_z 2^(m_z - m) O_z / (sum_z 2^(m_z - m) l_z + 2^(sink_h - m)) over the key-range splits
-__global__ void window_merge_kernel(const float* __restrict__ po, const float* __restrict__ pml, int nsplit, int64_t T,
-                                    int H, int Dv, const float* __restrict__ sink, const bf16* __restrict__ gate,
-                                    int64_t gs, bf16* __restrict__ out, int64_t os, float out_scale) {
+// out[t][h] = sum_z 2^(m_z - m) O_z / (sum_z 2^(m_z - m) l_z + 2^(sink_h - m)) over the (at most 64) key-range splits: lane z holds
+// split z's maximum and sum, four splits' partials are in flight at a time
+__global__ __launch_bounds__(64) void window_merge_kernel(const float* __restrict__ po, const float* __restrict__ pml, int nsplit,
+                                                          int64_t T, int H, int Dv, const float* __restrict__ sink,
+                                                          const bf16* __restrict__ gate, int64_t gs, bf16* __restrict__ out,
+                                                          int64_t os, float out_scale) {
   const int64_t th = blockIdx.x;  // t * H + h
   const int64_t t = th / H;
-  const int h = (int)(th - t * H);
+  const int h = (int)(th - t * H), lane = threadIdx.x;
   const int64_t zs = T * H;
-  float mx = -INFINITY;
-  for (int z = 0; z < nsplit; ++z) mx = fmaxf(mx, pml[2 * (z * zs + th)]);
-  float den = 0.f;
-  for (int z = 0; z < nsplit; ++z) {
-    const float mz = pml[2 * (z * zs + th)];
-    if (mz != -INFINITY) den += fast_exp2(mz - mx) * pml[2 * (z * zs + th) + 1];
-  }
+  const float mz = lane < nsplit ? pml[2 * (lane * zs + th)] : -INFINITY;
+  const float lz = lane < nsplit ? pml[2 * (lane * zs + th) + 1] : 0.f;
+  float mx = mz;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  const float wz = mz == -INFINITY ? 0.f : fast_exp2(mz - mx);
+  float den = wz * lz;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) den += __shfl_xor(den, o, 64);
   if (sink != nullptr) den += fast_exp2(sink[h] * LOG2E - mx);
   float inv = out_scale / den;
   if (gate != nullptr) inv *= head_gate(gate + t * gs + h);
-  for (int d = threadIdx.x; d < Dv; d += blockDim.x) {
-    float a = 0.f;
+  for (int d0 = 0; d0 < Dv; d0 += 128) {
+    float a[2] = {0.f, 0.f};
+#pragma unroll 4
     for (int z = 0; z < nsplit; ++z) {
-      const float mz = pml[2 * (z * zs + th)];
-      if (mz != -INFINITY) a += fast_exp2(mz - mx) * po[(z * zs + th) * Dv + d];
+      const float f = __shfl(wz, z, 64);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int d = d0 + lane + 64 * k;
+        const float v = d < Dv ? po[(z * zs + th) * Dv + d] : 0.f;
+        a[k] += f == 0.f ? 0.f : f * v;
+      }
     }
-    out[t * os + (int64_t)h * Dv + d] = (bf16)(a * inv);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int d = d0 + lane + 64 * k;
+      if (d < Dv) out[t * os + (int64_t)h * Dv + d] = (bf16)(a[k] * inv);
+    }
   }
 }
 

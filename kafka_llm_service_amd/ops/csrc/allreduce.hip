@@ -50,11 +50,26 @@ struct ARPtrs {
 
 typedef int ar_i32x4 __attribute__((ext_vector_type(4)));
 
-// system-coherent 16-B load, issued without a wait (the caller waits once for all peers' loads)
-__device__ __forceinline__ ar_i32x4 load_sys16_nowait(const bf16* p) {
-  ar_i32x4 r;
-  asm volatile("global_load_dwordx4 %0, %1, off sc0 sc1" : "=v"(r) : "v"(p) : "memory");
-  return r;
+// One system-coherent 16-B load per peer, all in flight at once (one per xGMI link), and their wait: one block, because the
+// compiler takes an asm's outputs as written at its end - with the wait in a block of its own it may read (or move) them before.
+template <int NR>
+__device__ __forceinline__ void load_peers16(const bf16* const (&q)[NR], ar_i32x4 (&r)[NR]) {
+  static_assert(NR == 2 || NR == 4 || NR == 8, "");
+  if constexpr (NR == 2) {
+    asm volatile("global_load_dwordx4 %0, %2, off sc0 sc1\n\tglobal_load_dwordx4 %1, %3, off sc0 sc1\n\ts_waitcnt vmcnt(0)"
+                 : "=&v"(r[0]), "=&v"(r[1]) : "v"(q[0]), "v"(q[1]) : "memory");
+  } else if constexpr (NR == 4) {
+    asm volatile("global_load_dwordx4 %0, %4, off sc0 sc1\n\tglobal_load_dwordx4 %1, %5, off sc0 sc1\n\t"
+                 "global_load_dwordx4 %2, %6, off sc0 sc1\n\tglobal_load_dwordx4 %3, %7, off sc0 sc1\n\ts_waitcnt vmcnt(0)"
+                 : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]) : "v"(q[0]), "v"(q[1]), "v"(q[2]), "v"(q[3]) : "memory");
+  } else {
+    asm volatile("global_load_dwordx4 %0, %8, off sc0 sc1\n\tglobal_load_dwordx4 %1, %9, off sc0 sc1\n\t"
+                 "global_load_dwordx4 %2, %10, off sc0 sc1\n\tglobal_load_dwordx4 %3, %11, off sc0 sc1\n\t"
+                 "global_load_dwordx4 %4, %12, off sc0 sc1\n\tglobal_load_dwordx4 %5, %13, off sc0 sc1\n\t"
+                 "global_load_dwordx4 %6, %14, off sc0 sc1\n\tglobal_load_dwordx4 %7, %15, off sc0 sc1\n\ts_waitcnt vmcnt(0)"
+                 : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7])
+                 : "v"(q[0]), "v"(q[1]), "v"(q[2]), "v"(q[3]), "v"(q[4]), "v"(q[5]), "v"(q[6]), "v"(q[7]) : "memory");
+  }
 }
 
 // This block's epoch for this call: its device counter + 1 (advanced here; one block per counter, stream-ordered
@@ -117,10 +132,10 @@ __device__ __forceinline__ void ar_exchange(const ARPtrs& ptrs, int rank, int e)
 template <int NR>
 __device__ __forceinline__ void ar_sum8(const ARPtrs& ptrs, int64_t half, int64_t c, float (&v)[8]) {
   ar_i32x4 raw[NR];
+  const bf16* q[NR];
 #pragma unroll
-  for (int p = 0; p < NR; ++p)  // all peers' loads in flight at once (one per xGMI link)
-    raw[p] = load_sys16_nowait(reinterpret_cast<const bf16*>(ptrs.base[p] + AR_HEADER + half) + c * 8);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  for (int p = 0; p < NR; ++p) q[p] = reinterpret_cast<const bf16*>(ptrs.base[p] + AR_HEADER + half) + c * 8;
+  load_peers16<NR>(q, raw);
 #pragma unroll
   for (int j = 0; j < 8; ++j) v[j] = 0.f;
 #pragma unroll
@@ -342,9 +357,14 @@ __global__ __launch_bounds__(256) void a2a_pull_kernel(ARPtrs ptrs, int rank, co
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int64_t cc = min(c + (int64_t)u * blockDim.x, z - 1);  // clamp, don't branch (stores are guarded)
-        v[p][u] = load_sys16_nowait(reinterpret_cast<const bf16*>(ptrs.base[p] + AR_HEADER + half) + cc * 8);
+        asm volatile("global_load_dwordx4 %0, %1, off sc0 sc1"
+                     : "=v"(v[p][u]) : "v"(reinterpret_cast<const bf16*>(ptrs.base[p] + AR_HEADER + half) + cc * 8) : "memory");
       }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int p = 0; p < NR; ++p)
+#pragma unroll
+      for (int u = 0; u < U; ++u) asm volatile("" : "+v"(v[p][u]));   // (read behind the wait)
 #pragma unroll
     for (int p = 0; p < NR; ++p)
 #pragma unroll

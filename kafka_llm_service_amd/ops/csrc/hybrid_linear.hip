@@ -686,8 +686,12 @@ __global__ __launch_bounds__(NT) void lin_chunk_prep_kernel(LinIn<AT> in, const 
 // (Q e^b) S over the wave's rows; the waves' parts of W S are summed through LDS to U; the state's update; a quarter of
 // P U per wave; the waves' parts of the output summed through LDS. The operands of the next two chunks are in flight.
 // The column tiles of a head are given to workgroups of one XCD where the heads divide by 8: they read the same operands.
+// What bounds it: half the time fp32 products, else a chunk's chain of loads and exchanges. Up to 128 channels without the delta rule
+// three workgroups fit a CU when the registers are held to 160 (2529 rows of three segments, 32 heads: 156 -> 117 us; left
+// to itself the compiler aims at two); with it that costs 34 spilled registers (181 -> 244), so two.
 template <typename AT, int NTL, bool FULL, bool DELTA>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, NTL > 2 ? 1 : 2))) void lin_chunk_scan_kernel(
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NTL > 2 || DELTA ? 1 : 3, NTL > 2 ? 1 : DELTA ? 2 : 3)))
+void lin_chunk_scan_kernel(
     LinIn<AT> in, const int* __restrict__ vseg, const int* __restrict__ cs, ChunkBuf cb, float* __restrict__ Sst,
     float* __restrict__ out, int64_t os) {
   __shared__ f32x4 red[4][2][64];

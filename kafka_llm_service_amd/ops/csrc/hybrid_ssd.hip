@@ -12,7 +12,8 @@
 // x, B and C are bf16; every fp32 factor of a product (B times its weight, the weights of the rows, the entry state) is
 // split into three bf16 parts that hold all its bits, one matrix product each, fp32 accumulation - as exact as the fp32
 // multiply-adds of the token-by-token kernels. The running sums are formed in fp64 and kept as two floats, so that the
-// difference of two of them is good to its own last bit however long the chunk's sum has become.
+// difference of two of them is good to its own last bit however long the chunk's sum has become. A token's exponent is held
+// at SSD_FLOOR or above: every decay over such a token is zero in fp32 either way, and the sums stay finite where A or dt do not.
 //
 // What bounds it: the chunks' contributions and entry states through memory (67 MB written, read and written by the
 // carry, read at 2048 tokens x 128 heads of 128 x 64) and the LDS reads of the split products. Measured there, one layer:
@@ -37,6 +38,8 @@ struct SsdIn {
   float* dec;           // [chunks][H]: e^(c_end)
 };
 
+constexpr double SSD_FLOOR = -1000.0;   // (e^-1000 is far below the smallest fp32 number)
+
 // The chunk's step sizes and running sums (times log2 e, as a float and what the float leaves out) by one wave; rows past n:
 // dt = 0, the sum stays.
 __device__ __forceinline__ void ssd_sums(const SsdIn& in, int row0, int n, int h, int lane, float* dt_s, float* ch_s,
@@ -47,12 +50,14 @@ __device__ __forceinline__ void ssd_sums(const SsdIn& in, int row0, int n, int h
   for (int k = 0; k < 2; ++k) {
     const int t = 64 * k + lane;
     float dt = 0.f;
+    double a = 0.0;
     if (t < n) {
       const float raw = (float)in.dt[(int64_t)(row0 + t) * in.ds + h] + bias;
       dt = raw > 20.f ? raw : log1pf(expf(raw));
+      a = (double)A * (double)dt;
     }
     dt_s[t] = dt;
-    c[k] = (double)A * (double)dt;
+    c[k] = a < SSD_FLOOR ? SSD_FLOOR : a;   // (NaN stays NaN)
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const double u = __shfl_up(c[k], o, 64);
@@ -65,7 +70,7 @@ __device__ __forceinline__ void ssd_sums(const SsdIn& in, int row0, int n, int h
     const double v = c[k] * 1.4426950408889634;
     const float hi = (float)v;
     ch_s[64 * k + lane] = hi;
-    cl_s[64 * k + lane] = hi > -INFINITY ? (float)(v - (double)hi) : 0.f;
+    cl_s[64 * k + lane] = (float)(v - (double)hi);
   }
 }
 
@@ -243,7 +248,45 @@ __global__ __launch_bounds__(NT) void ssd_out_kernel(SsdIn in, int n_chunks, int
   stage_transposed(rows + (int64_t)h * P, in.xs, n, v0, VSL, P, buf, tid);
   __syncthreads();
   if (32 * w >= n) return;   // (uniform per wave; no barrier follows)
-  const float th = ch_s[t], tl = cl_s[t], g0 = fast_exp2(th + tl);
+  const float th = ch_s[t], tl = cl_s[t], g0 = fast_exp2(th + tl), Dh = Dp[h];
+  unsigned odd = 0;   // (two values a word: a full exponent carries)
+#pragma unroll
+  for (int vt = 0; vt < 2; ++vt)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+      const u32x4 x = *reinterpret_cast<const u32x4*>(buf + (32 * vt + lr) * LDJ + 32 * w + 16 * lh + 8 * e);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) odd |= (x[i] & 0x7f807f80u) + 0x00800080u;
+    }
+  if (__any(odd & 0x80008000u)) {
+    // (uniform per wave, never with finite inputs) In the products below a row has the weight 0 for the rows behind it in its
+    // tile, and 0 times what is not finite is not 0. A tile that holds such values is summed row by row, up to the row itself.
+    if (t >= n) return;
+    const bf16 *ct = crow - 8 * lh, *b0 = Bc - 8 * lh;
+    const float* Uh = in.U + ((int64_t)item * P + v0 + 32 * lh) * N;
+    const int nv = min(32, P - v0 - 32 * lh);   // this lane's columns
+    float yv[32];
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      float a = 0.f;
+      if (i < nv)
+        for (int d = 0; d < N; ++d) a += Uh[(int64_t)i * N + d] * (float)ct[d];
+      yv[i] = a * g0;
+    }
+    for (int j = 0; j <= t; ++j) {
+      float wj = 0.f;
+      for (int d = 0; d < N; ++d) wj += (float)b0[(int64_t)j * in.xs + d] * (float)ct[d];
+      wj *= ssd_decay(th, tl, ch_s[j], cl_s[j]) * dt_s[j];
+#pragma unroll
+      for (int i = 0; i < 32; ++i) yv[i] += wj * (float)buf[(32 * lh + i) * LDJ + j];
+    }
+#pragma unroll
+    for (int i = 0; i < 32; ++i)
+      if (i < nv)
+        y[(int64_t)(row0 + t) * ys + (int64_t)h * P + v0 + 32 * lh + i] = yv[i] + Dh * (float)buf[(32 * lh + i) * LDJ + t];
+    return;
+  }
 #pragma unroll
   for (int vt = 0; vt < 2; ++vt)
 #pragma unroll
@@ -280,7 +323,6 @@ __global__ __launch_bounds__(NT) void ssd_out_kernel(SsdIn in, int n_chunks, int
   }
   mfma_settle();
   if (t >= n) return;
-  const float Dh = Dp[h];
   const bf16* xr = rows + (int64_t)t * in.xs + (int64_t)h * P + v0;
   float* op = y + (int64_t)(row0 + t) * ys + (int64_t)h * P + v0;
 #pragma unroll

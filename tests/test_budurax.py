@@ -827,6 +827,42 @@ def test_scan_in_matrix_core_chunks(Hh, P, N, G, fast):
     assert errs[0][0] < 2 * errs[1][0] + 1e-6 and errs[0][1] < 2 * errs[1][1] + 1e-6
 
 
+@pytest.mark.gpu
+def test_chunked_scan_of_rates_and_rows_without_bound():
+    """The chunked scan where A_log is past the largest exponent (A = -inf: the state of a token is gone with the next one), and
+    with a row whose x is infinite and one whose x is NaN: whatever stands before such a row comes out as it does without it
+    (portions that end inside a chunk of 128 and a tile of 32 rows; the same error bound as above)."""
+    device = "cuda:0"
+    torch.manual_seed(9)
+    Hh, P, N, G, n = 4, 64, 32, 2, 173
+    inner = Hh * P
+    xbc = (torch.randn(n, inner + 2 * G * N) / 2).bfloat16()
+    proj = torch.randn(n, Hh).bfloat16()
+    A_log = torch.tensor([0.3, 89.0, 200.0, 1.0])
+    dt_bias, D = torch.randn(Hh) / 2, torch.randn(Hh)
+    seg, ts = _seg("cpu", [(n, 0, 0)])
+    tabs = tuple(torch.from_numpy(t).to(device) for t in hops.chunk_tables(seg.numpy(), hops.SSD_CHUNK, hops.SSD_CHUNK_MIN))
+
+    def scan(xb):
+        state, y = torch.full((1, Hh, N, P), float("nan"), device=device), torch.full((n, inner), float("nan"), device=device)
+        hops.ssm_scan(xb.to(device), proj.to(device), 0, dt_bias.to(device), A_log.to(device), D.to(device), Hh, P, N, G,
+                      ts.to(device), seg.to(device), state, y, tabs, None)
+        return y.cpu().view(n, Hh, P), state.cpu()
+
+    want, S = _ssm_want(xbc, proj, dt_bias, A_log, D, Hh, P, N, G, torch.zeros(Hh, N, P, dtype=torch.float64))
+    want = want.view(n, Hh, P)
+    y, state = scan(xbc)
+    assert ((y.double() - want).abs().amax((0, 2)) < 2e-5 * want.abs().amax((0, 2))).all()
+    assert ((state[0].double() - S).abs().amax((1, 2)) < 2e-5 * S.abs().amax((1, 2))).all()
+    for row, bad in ((5, float("inf")), (63, float("nan")), (130, float("-inf")), (172, float("nan"))):
+        xb = xbc.clone()
+        xb[row, 0:3] = bad                  # three channels of the first head ...
+        xb[row, inner - 1] = bad            # ... and one of the last
+        y, _ = scan(xb)
+        assert ((y[:row].double() - want[:row]).abs().amax((0, 2)) < 2e-5 * want.abs().amax((0, 2))).all()
+        assert not torch.isfinite(y[row, 0, :3]).any() and torch.isfinite(y[row, 1:3]).all()
+
+
 def test_portion_tables():
     """Which rows attend on expanded keys: none without a portion of LATENT_ROWS_MIN rows, else everything behind the leading
     single tokens; blocks of 64 gathered rows per portion, tiles of 128 rows with the most keys first."""

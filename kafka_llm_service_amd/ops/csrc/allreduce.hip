@@ -332,7 +332,9 @@ extern "C" hipError_t kafka_launch_car_allreduce_add_rmsnorm(char* const* bases,
 
 // Pull-mode all-to-all (bcast = 0: part q of the image, at q * bpd, goes to rank q; recv part p = peer p's part for
 // this rank) or all-gather (bcast = 1: the image is one part of bpd bytes; recv part p = peer p's image).
-// nbytes = image bytes (ep * bpd, or bpd); bpd % 16 == 0.
+// nbytes = image bytes (ep * bpd, or bpd); bpd % 16 == 0. The peers' parts are read by builtin loads (system-coherent, U per peer in
+// flight): more of them than one asm block has operands for, and a wait outside the block that loads is none to the compiler.
+constexpr int SYS_COHERENT = 1 | 16;   // sc0 sc1
 template <int NR>
 __global__ __launch_bounds__(256) void a2a_pull_kernel(ARPtrs ptrs, int rank, const ar_i32x4* __restrict__ send,
                                                        int64_t n16, ar_i32x4* __restrict__ recv, int64_t bpd16,
@@ -342,7 +344,7 @@ __global__ __launch_bounds__(256) void a2a_pull_kernel(ARPtrs ptrs, int rank, co
   const int b = blockIdx.x, nb = gridDim.x;
   const int64_t per = (n16 + nb - 1) / nb;
   const int64_t c0 = min(n16, (int64_t)b * per), c1 = min(n16, c0 + per);
-  const int64_t half = (int64_t)(e & 1) * max_bytes;
+  const int64_t half = (int64_t)(__builtin_amdgcn_readfirstlane(e) & 1) * max_bytes;
   ar_i32x4* mine = reinterpret_cast<ar_i32x4*>(ptrs.base[rank] + AR_HEADER + half);
   for (int64_t c = c0 + threadIdx.x; c < c1; c += blockDim.x) mine[c] = send[c];
   ar_exchange<NR>(ptrs, rank, e);
@@ -350,21 +352,18 @@ __global__ __launch_bounds__(256) void a2a_pull_kernel(ARPtrs ptrs, int rank, co
   const int64_t lo = bcast ? 0 : rank * bpd16, hi = lo + bpd16;
   const int64_t a = max(lo, c0), z = min(hi, c1);
   constexpr int U = 4;  // loads in flight per thread and peer
+  const int64_t at = half + (int64_t)__builtin_amdgcn_readfirstlane((int)a) * 16;   // (uniform, but computed per lane)
   for (int64_t c = a + threadIdx.x; c < z; c += (int64_t)blockDim.x * U) {
     ar_i32x4 v[NR][U];
 #pragma unroll
-    for (int p = 0; p < NR; ++p)
+    for (int p = 0; p < NR; ++p) {
+      const auto rs = buf_rsrc(ptrs.base[p] + AR_HEADER + at);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int64_t cc = min(c + (int64_t)u * blockDim.x, z - 1);  // clamp, don't branch (stores are guarded)
-        asm volatile("global_load_dwordx4 %0, %1, off sc0 sc1"
-                     : "=v"(v[p][u]) : "v"(reinterpret_cast<const bf16*>(ptrs.base[p] + AR_HEADER + half) + cc * 8) : "memory");
+        v[p][u] = __builtin_bit_cast(ar_i32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(cc - a) * 16, 0, SYS_COHERENT));
       }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-    for (int p = 0; p < NR; ++p)
-#pragma unroll
-      for (int u = 0; u < U; ++u) asm volatile("" : "+v"(v[p][u]));   // (read behind the wait)
+    }
 #pragma unroll
     for (int p = 0; p < NR; ++p)
 #pragma unroll

@@ -243,10 +243,15 @@ __device__ __forceinline__ void ld_dma16(const void* g, void* lds) {
 __device__ __forceinline__ f32x4 ld_mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
-// c += a b in c's own vector registers (the compiler keeps it in accumulation registers and moves it for every rescale). It does
-// not know that these products take 16 passes: the next reader of c comes behind the scores' products, or mfma_settle().
-__device__ __forceinline__ void ld_mfma32(f32x16& c, bf16x8 a, bf16x8 b) {
-  asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+// c[j] += a b[j] in the sums' own vector registers (the compiler keeps them in accumulation registers and moves them for every
+// rescale). One statement, wait included: the compiler does not know that these products take eight passes, nor of a wait that
+// stands elsewhere, and may copy a statement's outputs as soon as it ends.
+__device__ __forceinline__ void ld_mfma32(f32x16 (&c)[4], bf16x8 a, const bf16x8 (&b)[4]) {
+  asm volatile(
+      "s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %4, %5, %0\n\tv_mfma_f32_32x32x16_bf16 %1, %4, %6, %1\n\t"
+      "v_mfma_f32_32x32x16_bf16 %2, %4, %7, %2\n\tv_mfma_f32_32x32x16_bf16 %3, %4, %8, %3\n\ts_nop 11"
+      : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3])
+      : "v"(a), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]));
 }
 // the value of the lane n places on in its 16
 template <int N>
@@ -415,17 +420,19 @@ __global__ __launch_bounds__(256, 2) void latent_decode_kernel(
           if (kb * LD_KEYS + 16 * st + 8 * lh + k > maxpos) v[st][k] = ld_u2{0u, 0u};
     }
 #pragma unroll
-    for (int st = 0; st < 2; ++st)
+    for (int st = 0; st < 2; ++st) {
+      bf16x8 b[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        ld_u4 b;
+        ld_u4 p;
 #pragma unroll
         for (int x4 = 0; x4 < 4; ++x4)
-          b[x4] = __builtin_amdgcn_perm(v[st][2 * x4 + 1][j >> 1], v[st][2 * x4][j >> 1], j & 1 ? 0x07060302u : 0x05040100u);
-        ld_mfma32(O[j], a[st], __builtin_bit_cast(bf16x8, b));
+          p[x4] = __builtin_amdgcn_perm(v[st][2 * x4 + 1][j >> 1], v[st][2 * x4][j >> 1], j & 1 ? 0x07060302u : 0x05040100u);
+        b[j] = __builtin_bit_cast(bf16x8, p);
       }
+      ld_mfma32(O, a[st], b);
+    }
    }
-   mfma_settle();
    lds_barrier();   // (the run's page ids, slots and corr_s are read until here)
   }
   // ---- row sums: across the lanes of a row, then the two pages

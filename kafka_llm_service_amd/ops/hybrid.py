@@ -164,7 +164,9 @@ LATENT_ROWS_MIN = 96
 LATENT_ROWS_CHAIN = 2048  # keys that a portion of fewer rows may walk beside it, if more than the long portions' own
 LATENT_ROWS_KEYS = 64   # (kernel constants) keys of a block ...
 LATENT_ROWS_TILE = 128  # ... and rows of a workgroup
-LATENT_ROWS_MAX = 1 << 17   # gathered rows of a step beyond which it stays in the latent space (the expanded keys' memory)
+LATENT_ROWS_MAX = 1 << 17   # gathered rows of a step beyond which it stays in the latent space
+LATENT_BYTES = 1 << 29      # most bytes of expanded keys and values at a time: what the latent space's queries and outputs of a
+                            # portion of 8192 rows x 32 heads take; more heads follow group by group
 
 
 def latent_rows_ok(q, q_rot, cache, Dv: int) -> bool:
@@ -227,9 +229,20 @@ def latent_attn_portions(q, q_rot, cache, w_k, w_v, tables, block_tables, scale:
     ck = torch.empty(M, R, dtype=q.dtype, device=q.device)
     kr = torch.empty(M, rd, dtype=q.dtype, device=q.device)
     ext().hy_latent_gather(cache, rd, block_tables, px, blocks, ck, kr)
-    k = torch.nn.functional.linear(ck, w_k)       # [M, H dim]
-    vt = torch.nn.functional.linear(w_v, ck)      # [H vdim, M]
-    ext().hy_latent_rows(q, q_rot, k, kr, vt, px, tiles, float(scale), int(window), sink, gate, out)
+    H, D = q.shape[1:]
+    Dv = w_v.shape[0] // H
+    hg = max(1, min(H, LATENT_BYTES // (M * (D + Dv) * q.element_size())))   # heads at a time
+    if 8 < hg < H:
+        hg = hg // 8 * 8
+    k = vt = None
+    for a in range(0, H, hg):
+        b = min(H, a + hg)
+        del k, vt         # (before the next group's are made)
+        k = torch.nn.functional.linear(ck, w_k[a * D:b * D])         # [M, (b - a) dim]
+        vt = torch.nn.functional.linear(w_v[a * Dv:b * Dv], ck)      # [(b - a) vdim, M]
+        ext().hy_latent_rows(q[:, a:b], q_rot[:, a:b], k, kr, vt, px, tiles, float(scale), int(window),
+                             None if sink is None else sink[a:b], None if gate is None else gate[:, a * Dv:b * Dv],
+                             out[:, a * Dv:b * Dv])
 
 
 def sigmoid_mul(a, g, out) -> None:

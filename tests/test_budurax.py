@@ -944,6 +944,38 @@ def test_attention_of_portions_on_expanded_keys(H, rd, window, extras):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H", [48, 7])
+def test_expanded_keys_by_groups_of_heads(H, monkeypatch):
+    """Expanded keys and values past LATENT_BYTES: groups of heads one after the other give what one group gives (library
+    products of other widths: keys and values a bf16 rounding apart, 2^-8 of the largest value at most in an average of values
+    and again in the weights' exponents), and no more memory is held than the bound, the gathered rows and the allocator's
+    rounding to 2 MiB."""
+    device, R, rd, D, n, p0 = "cuda:0", 256, 64, 128, 150, 3000
+    torch.manual_seed(H)
+    W = -(-(n + p0) // 16)
+    bt = torch.randperm(W, device=device).view(1, W).int()
+    cache = torch.randn(W, 16, R + rd, device=device).bfloat16()
+    q, q_rot = (torch.randn(n, H, d, device=device).bfloat16() for d in (D, rd))
+    w_k, w_v = ((torch.randn(H * D, R, device=device) / R ** 0.5).bfloat16() for _ in range(2))
+    sink, gate = torch.randn(H, device=device), torch.randn(n, H * D, device=device).bfloat16()
+    t = hops.portion_tables(_seg("cpu", [(n, p0, 0)])[0].numpy(), 0)
+    tabs = t[:2] + tuple(torch.from_numpy(x).to(device) for x in t[2:])
+    outs, peaks, M = [], [], t[1]
+    for most in (1 << 29, M * 2 * D * 2 * 20):
+        monkeypatch.setattr(hops, "LATENT_BYTES", most)
+        out = torch.full((n, H * D), float("nan"), dtype=torch.bfloat16, device=device)
+        torch.cuda.reset_peak_memory_stats()
+        held = torch.cuda.memory_allocated()
+        hops.latent_attn_portions(q, q_rot, cache, w_k, w_v, tabs, bt, 192 ** -0.5, out, 0, sink, gate)
+        peaks.append(torch.cuda.max_memory_allocated() - held)
+        outs.append(out.float())
+    top = (cache[:, :, :R].float().reshape(-1, R) @ w_v.float().t()).abs().max().item()
+    assert (outs[0] - outs[1]).abs().max().item() <= 2 ** -7 * top
+    if H > 20:
+        assert peaks[1] <= M * 2 * D * 2 * 20 + M * (R + rd) * 2 + (8 << 20) < peaks[0]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("d,T", [(4, 3), (1024, 3), (1028, 5), (1030, 5), (4096, 7), (4096, 600), (4100, 3), (1022, 2)])
 def test_row_kernels_over_widths(dtype, d, T):

@@ -255,11 +255,11 @@ class SegMeta:
             self.cache[key] = (tabs, short)
         return self.cache[key]
 
-    def portions(self, window: int):
+    def portions(self, window: int, heads: int, kv_rank: int, rot_dim: int):
         """``hops.portion_tables`` of the step with its tables on the device, built once per step."""
-        key = ("portions", window)
+        key = ("portions", window, heads, kv_rank, rot_dim)
         if key not in self.cache:
-            t = hops.portion_tables(self.seg_host, window)
+            t = hops.portion_tables(self.seg_host, window, heads, kv_rank, rot_dim)
             self.cache[key] = None if t is None else t[:2] + self.upload(t[2:])
         return self.cache[key]
 
@@ -296,7 +296,8 @@ def latent_mix(q, q_rot, cache, cache_t, lw, inp, m: SegMeta, ao, window: int = 
     portions on expanded keys and values where the sizes allow."""
     T, H, D = q.shape
     R, Dv = lw.uk_h.shape[2], lw.uv_ht.shape[2]
-    tables = m.portions(window) if cache_t is not None and lw.scale > 0 and hops.latent_rows_ok(q, q_rot, cache, Dv) else None
+    tables = m.portions(window, H, R, q_rot.shape[2]) if cache_t is not None and lw.scale > 0 and \
+        hops.latent_rows_ok(q, q_rot, cache, Dv) else None
     n = T if tables is None else tables[0]        # rows that stay in the latent space
     if n:
         q_lat = torch.bmm(q[:n].transpose(0, 1), lw.uk_h)                         # [H, n, R]

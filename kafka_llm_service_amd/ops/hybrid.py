@@ -156,11 +156,9 @@ def latent_attn(q_lat, q_rot, cache, block_tables, tok_seg, seg, positions, scal
         ref.latent_attn(q_lat, q_rot, cache, block_tables, tok_seg, seg, positions, scale, out, window, sink)
 
 
-# Rows of a step's longest portion from which its portions attend on expanded keys and values (H = 32, 512 / 64 / 128 / 128,
-# us with the products around it, expanded against latent space): fresh portions of 128 / 512 / 2048 rows 52 / 74 / 178 against
-# 50 / 140 / 1170; behind 2000 keys 64 / 128 / 512 rows 176 / 189 / 201 against 132 / 304 / 632; behind 8000 keys 64 rows 539
-# against 313 (a tile walks its keys alone). With a window of 1024 keys the two are level at 64 rows.
-LATENT_ROWS_MIN = 96
+# Below these no step gained from expanded keys and values, whatever the rest of ``expanded_pays`` (128 rows of 32 heads, kv_rank 512 /
+# 256 / 128: 62 / 46 / 38 us against 44 / 45 / 36 in the latent space)
+LATENT_ROWS_MIN = 96      # rows of a step's longest portion
 LATENT_ROWS_CHAIN = 2048  # keys that a portion of fewer rows may walk beside it, if more than the long portions' own
 LATENT_ROWS_KEYS = 64   # (kernel constants) keys of a block ...
 LATENT_ROWS_TILE = 128  # ... and rows of a workgroup
@@ -179,10 +177,41 @@ def latent_rows_ok(q, q_rot, cache, Dv: int) -> bool:
                for t in ((q, q_rot) if rd else (q,))) and bool(ext().hy_latent_rows_ok(cache.shape[2] - rd, rd, D, int(Dv)))
 
 
-def portion_tables(seg_host, window: int):
+def expanded_pays(portions, window: int, heads: int, kv_rank: int, rot_dim: int) -> bool:
+    """Whether portions (rows, first position) attend faster on expanded keys and values than in the latent space, from what
+    either was measured to take (us, operands from memory; kv_rank 128 .. 512, 8 .. 64 heads, 48 .. 1024 rows behind 0 .. 8000 keys):
+      latent    its tiles of 32 (row, head) pairs in rounds of 256 workgroups, a round as long as a tile's keys; less than
+                a round is divided by key ranges;
+      expanded  the longest tile's walk over its keys (a workgroup of 128 rows) or, with many tiles, their rounds of 512; the
+                products of every key of a context; both products' and the gather's launches.
+    Latent / expanded, 32 heads of 512 + 64: 128 / 256 / 512 fresh rows 44 / 56 / 91 against 62 / 72 / 86; behind 2000 keys 100 / 155 /
+    290 against 207 / 197 / 219; behind 8000 keys 249 / 447 / 868 against 591 / 671 / 658; 512 + 0 with a window of 1024 71 / 95 /
+    156 against 92 / 92 / 107; 16 heads, 512 rows behind 2000 keys 164 / 204; 64 heads, 256 rows 280 / 252; 32 heads of 256 + 64, 192
+    and 512 rows behind 2000 keys 231 / 195 and 415 / 203. The choice was the faster one, or within 15 % of it, at all of 256 points."""
+    r = work = walk = turns = ctx = 0
+    for n, p0 in portions:
+        last = min(p0 + n, window + LATENT_ROWS_TILE) if window else p0 + n
+        mean = min(p0 + n / 2, window) if window else p0 + n / 2
+        r += n
+        work += n * mean
+        walk = max(walk, last)
+        turns += -(-n // LATENT_ROWS_TILE) * heads * mean
+        ctx += min(p0, window) + n if window else p0 + n
+    rounds = r * heads / MFMA_ROWS / 256
+    rounds = float(-(-rounds // 1)) if rounds > 1 else 1 / (1 / rounds // 1)
+    # a key of a tile and a tile, by kernel
+    key_us, tile_us = (0.052, 18) if kv_rank == 512 and rot_dim in (0, 64) else (0.03 + 0.00025 * kv_rank, 25)
+    latent = 20 + rounds * (work / r * key_us + tile_us)
+    expanded = (25 if rot_dim else 15) + 0.045 * kv_rank + max(walk, turns / 512) * (0.052 if rot_dim else 0.035) + \
+        ctx * heads * kv_rank * 4.6e-7
+    return latent > expanded
+
+
+def portion_tables(seg_host, window: int, heads: int = 0, kv_rank: int = 512, rot_dim: int = 0):
     """Tables of ``latent_attn_portions`` for a step: (rows in front of them, gathered rows, portions int32 [n, 8], portion of
-    every 64 gathered rows, tiles int32 [m, 4]) as numpy, or None when the step has no portion of LATENT_ROWS_MIN rows. The
-    single tokens in front (a plan's decoded rows) are left to ``latent_attn``."""
+    every 64 gathered rows, tiles int32 [m, 4]) as numpy, or None when the step has no portion of LATENT_ROWS_MIN rows or, with
+    ``heads`` given, is faster in the latent space (``expanded_pays``). The single tokens in front (a plan's decoded rows) are left
+    to ``latent_attn``."""
     import numpy as np
 
     if seg_host is None or not len(seg_host):
@@ -195,6 +224,8 @@ def portion_tables(seg_host, window: int):
     if window:
         keys = np.minimum(keys, rows[first:] + window)
     if int(keys.max()) > max(LATENT_ROWS_CHAIN, int(keys[rows[first:] >= LATENT_ROWS_MIN].max())):
+        return None
+    if heads and not expanded_pays(seg_host[first:, 1:3].tolist(), window, heads, kv_rank, rot_dim):
         return None
     px, blocks, tiles, at = [], [], [], 0
     for j, (q0, n, p0, _) in enumerate(seg_host[first:].tolist()):

@@ -885,6 +885,23 @@ def test_portion_tables():
     assert hops.portion_tables(_seg("cpu", [(hops.LATENT_ROWS_MIN, far, 0), (3, far, 1)])[0].numpy(), 0) is not None
 
 
+def test_where_expanded_keys_pay():
+    """The choice between the latent space and expanded keys and values at measured points of both sides (us in the latent space /
+    expanded), and its effect on a step's tables."""
+    for H, R, rd, hist, rows, window, latent, expanded in (
+            (8, 512, 64, 0, 512, 0, 53, 80), (16, 512, 64, 8000, 512, 0, 457, 595), (32, 512, 64, 0, 128, 0, 44, 62),
+            (32, 512, 64, 0, 512, 0, 91, 86), (32, 512, 64, 2000, 256, 0, 155, 197), (32, 512, 64, 2000, 384, 0, 280, 223),
+            (32, 512, 64, 8000, 128, 0, 249, 591), (32, 512, 64, 8000, 512, 0, 868, 658), (32, 512, 0, 4000, 384, 1024, 158, 96),
+            (64, 512, 64, 2000, 128, 0, 147, 261), (64, 512, 64, 8000, 192, 0, 831, 732), (32, 256, 64, 2000, 192, 0, 231, 195),
+            (32, 256, 64, 2000, 96, 0, 137, 178), (16, 256, 0, 4000, 192, 1024, 91, 68), (32, 128, 64, 2000, 512, 0, 273, 189)):
+        assert hops.expanded_pays([(rows, hist)], window, H, R, rd) == (expanded < latent), (H, R, rd, hist, rows, window)
+    # many portions fill the chip together
+    assert not hops.expanded_pays([(120, 500)], 0, 32, 512, 64) and hops.expanded_pays([(120, 500)] * 8, 0, 32, 512, 64)
+    seg = _seg("cpu", [(1, 5, 0), (200, 2000, 1)])[0].numpy()
+    assert hops.portion_tables(seg, 0) is not None and hops.portion_tables(seg, 0, 32, 512, 64) is None
+    assert hops.portion_tables(seg, 0, 64, 512, 64)[:2] == (1, 64 * 35)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,rd,window,extras", [(8, 64, 0, True), (3, 0, 0, False), (16, 0, 70, True), (5, 64, 200, False),
                                                 (8, 0, 1, False)])

@@ -110,27 +110,37 @@ def tile_tokens(heads: int) -> int:
     return max(1, MFMA_ROWS // heads)
 
 
-# Workgroups a matrix-core attention launch should reach before its key ranges are left whole, and the most ranges of a tile.
-# kv_rank 512, us by ranges: 64 sequences x 1706 keys 1: 95, 2: 60, 4: 44, 8: 59; 16 x 1706 4: 36, 8: 29, 16: 30; one x 1706 4: 35,
-# 8: 26, 16: 23, 32: 25; one x 8000 8: 63, 16: 41, 32: 34.
+# Workgroups a matrix-core attention launch should reach before its key ranges are left whole, and the most ranges of a tile
 ATTN_SPLIT_WGS = 256
 ATTN_SPLIT_MAX = 32
 
 
-def attn_splits(n_tiles: int, heads: int, max_keys: int) -> int:
-    """Key-range splits of a matrix-core attention launch: few tiles (a decode step's one tile per sequence) against
-    long contexts are dealt over more workgroups, each at least 128 keys long; a merge pass combines them."""
-    wgs = n_tiles * -(-heads // MFMA_ROWS)
-    blocks = -(-max_keys // 128)
-    return max(1, min(ATTN_SPLIT_MAX, ATTN_SPLIT_WGS // wgs, blocks))
+def attn_splits(n_tiles: int, heads: int, max_keys: int, kv_rank: int = 0, rot_dim: int = 0, seqs: int = 0) -> int:
+    """Key-range splits of a matrix-core attention launch: few tiles (a decode step's one tile per sequence) against long contexts are
+    dealt over more workgroups, each at least 128 keys long; a merge pass combines them, and costs the host another launch: contexts
+    whose ranges would gain less than that stay whole. ``seqs``: sequences the tiles belong to (0: a tile each).
+
+    us by ranges, single tokens, 32 heads, operands from memory. kv_rank 512 (``latent_decode``): one sequence x 256 keys 1: 26, 2: 23;
+    512 1: 39, 4: 24; 1706 1: 98, 8: 30, 16: 30; 8000 16: 48, 32: 42. There the cache's rows from memory bound some dozens of
+    sequences, and more ranges than their walk needs only add traffic: 16 x 8000 8: 77, 16: 83; 32 x 1706 4: 45, 8: 47, 16: 63; 64 x 1706
+    1: 100, 2: 67, 4: 68, 8: 81; 100 x 700 1: 52, 2: 51; 128 x 1706 1: 107, 2: 113; 128 x 4000 1: 219, 2: 191; 200 x 1706 1: 139, 2: 168.
+    kv_rank 256 + 32: one x 130 1: 32, 2: 30; one x 256 1: 39, 2: 30; 64 x 1000 1: 116, 2: 74, 4: 55, 8: 69; 128 x 200 1: 39, 2: 37;
+    128 x 1000 1: 125, 2: 86, 4: 99."""
+    wgs = max(1, n_tiles * -(-heads // MFMA_ROWS))
+    ns = min(ATTN_SPLIT_MAX, ATTN_SPLIT_WGS // wgs, -(-max_keys // 128))
+    if kv_rank == 512 and rot_dim in (0, 64):
+        if max_keys <= 256:
+            return 1
+        ns = min(ns, max(-(-100 // max(1, seqs or n_tiles)), 2 if max_keys >= 2000 else 1))
+    return 1 if max_keys <= 160 else max(1, ns)
 
 
 def latent_attn(q_lat, q_rot, cache, block_tables, tok_seg, seg, positions, scale, out, cache_t=None,
                 tiles=None, max_keys: int = 0, window: int = 0, sink=None) -> None:
     """Causal softmax attention of every row's heads over its sequence's cached [latent | rotated key] rows:
     out[h, t] = sum_j softmax_j((q_lat[h, t] . c_j + q_rot[t, h] . k_j) scale) c_j over the keys j <= position[t].
-    With the transposed latent copy ``cache_t`` (not read at kv_rank 512 with 0 or 64 rotated channels) and ``tiles`` (int32 [n, 4] = (first row, tokens, segment, 0), at
-    most ``tile_tokens(H)`` tokens of one segment each) bf16 runs on the matrix cores; else one wave per (row, 4
+    With the transposed latent copy ``cache_t`` (not read at kv_rank 512 with 0 or 64 rotated channels) and ``tiles`` (int32 [n, 4] =
+    (first row, tokens, segment, 0), at most ``tile_tokens(H)`` tokens of one segment each) bf16 runs on the matrix cores; else one wave per (row, 4
     heads) on the vector units (fp32, odd sizes). ``max_keys`` (the step's longest context) lets a launch of few
     tiles split its key ranges over more workgroups (``attn_splits``).
     ``window`` > 0: a row at position p sees only the keys p - window < j <= p. ``sink`` fp32 [H]: a per-head logit
@@ -142,7 +152,8 @@ def latent_attn(q_lat, q_rot, cache, block_tables, tok_seg, seg, positions, scal
             H, T, R = q_lat.shape
             if window:  # a key range is at most the window long
                 max_keys = min(max_keys, window + tile_tokens(H))
-            ns = attn_splits(tiles.shape[0], H, max_keys) if max_keys else 1
+            seqs = 0 if seg is None else min(tiles.shape[0], seg.shape[0])
+            ns = attn_splits(tiles.shape[0], H, max_keys, R, q_rot.shape[2], seqs) if max_keys else 1
             po = pml = None
             if ns > 1:
                 po = torch.empty(ns, H, T, R, dtype=torch.float32, device=q_lat.device)

@@ -236,18 +236,28 @@ def untile_weight(wt: torch.Tensor, glu: bool = False) -> torch.Tensor:
     return wt.reshape(nb, kb, 2, 32, 8).permute(0, 3, 1, 2, 4).reshape(nb * 32, kb * 16)
 
 
-# A library product of up to this many output columns is cut into blocks of this many rows: 4096 x 4096 outputs are one round
-# of 256 x 256 tiles over the 256 CUs, and the few tiles of the rows beyond it are a second round that takes as long as the
-# first. Library alone against blocks, N = 4096, us: K = 14336, 4099 rows 722 / 328, 5500 rows 852 / 457, 7000 rows 656 / 558;
-# K = 8192, 4099 rows 244 / 194; K = 4096, 4099 rows 131 / 111, 7000 rows 160 / 168; 8192 rows level. Wider outputs gain
-# nothing on average (28672 columns: 692 / 715 at 4099 rows).
+# Rows and output columns that are one round of the library's 256 x 256 tiles over the 256 CUs: the few tiles of the rows beyond it are
+# a second round that takes as long as the first. A product of that many columns is cut into blocks of that many rows. Library alone
+# against blocks, N = 4096, us, operands from memory: K = 14336, 4099 rows 753 / 356, 5500 873 / 496, 7000 674 / 576, 8200 1047 / 639,
+# 10000 1130 / 805; K = 8192, 4099 264 / 192, 7000 336 / 324, 8200 569 / 364; K = 4096, 4099 145 / 115, 7000 175 / 176, 10000 377 / 244;
+# K = 2048, 4099 80 / 66, 4500 79 / 74, 8200 141 / 120, but 5500 87 / 92; whole blocks (8192, 12288, 16384 rows) gain nothing (-1 %).
+# Fewer columns fill no round with a block: N = 2048, 4099 / 5500 / 10000 rows of K = 4096 72 / 84, 82 / 102, 144 / 172; N = 3072 83 / 98,
+# 141 / 129, 184 / 215; N = 1024 51 / 61, 62 / 73, 82 / 120. Wider outputs gain nothing on average (28672: 692 / 715 at 4099 rows).
 DENSE_BLOCK = 4096
+
+
+def dense_cut(M: int, N: int, K: int) -> bool:
+    """Whether x [M, K] @ w^T [N, K] goes in blocks of DENSE_BLOCK rows (the figures above)."""
+    tail = M % DENSE_BLOCK
+    if M <= DENSE_BLOCK or tail == 0 or not DENSE_BLOCK - 256 < N <= DENSE_BLOCK:
+        return False
+    return K >= 4096 or M > 2 * DENSE_BLOCK or tail <= 1024
 
 
 def linear_dense(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w^T (bf16 [M, K] x [N, K], prefill-sized M) on hipBLASLt, in row blocks where one call would leave the chip idle."""
     M, N = x.shape[0], w.shape[0]
-    if not _gpu(x) or M <= DENSE_BLOCK or N > DENSE_BLOCK or x.dtype != torch.bfloat16:
+    if not _gpu(x) or x.dtype != torch.bfloat16 or x.dim() != 2 or not dense_cut(M, N, x.shape[1]):
         return torch.nn.functional.linear(x, w)
     y = torch.empty(M, N, dtype=x.dtype, device=x.device)
     for a in range(0, M, DENSE_BLOCK):

@@ -336,6 +336,19 @@ def test_stream_plan_rules(monkeypatch):
     assert ops.stream_plan(300, 4096, 4096) is None and ops.stream_plan(64, 4100, 4096) is None
 
 
+def test_where_dense_products_are_cut():
+    """Row blocks where a block of 4096 rows is a round of the chip's tiles and a few rows lie beyond it, at measured points of both
+    sides (us, whole / in blocks)."""
+    from kafka_llm_service_amd import ops
+
+    for M, N, K, whole, cut in ((4099, 4096, 14336, 753, 356), (5500, 4096, 8192, 281, 270), (4099, 4096, 2048, 80, 66),
+                                (10000, 4096, 2048, 166, 140), (5500, 4096, 2048, 87, 92), (8192, 4096, 4096, 183, 186),
+                                (16384, 4096, 8192, 688, 696), (4099, 2048, 4096, 72, 84), (10000, 2048, 7168, 240, 287),
+                                (4099, 3072, 4096, 83, 98), (4500, 3072, 8192, 165, 199), (4099, 1024, 4096, 51, 61),
+                                (4096, 4096, 4096, 1, 1), (4099, 28672, 4096, 692, 715)):
+        assert ops.dense_cut(M, N, K) == (cut < whole), (M, N, K)
+
+
 def test_tiled_only_weights_match_stream():
     """Tiled-only mode (the row-major dense weights dropped after tiling, prefill untiles per projection — what a
     model whose second weight copy does not fit gets) generates exactly what the two-copy stream mode does."""

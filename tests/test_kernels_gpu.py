@@ -854,6 +854,19 @@ def test_linear_dense_blocks(M, N):
     assert ((got - want).abs() <= 2 ** -8 * want.abs() + 1e-2).all()
 
 
+@pytest.mark.parametrize("M", [ops.DENSE_BLOCK + 1, 2 * ops.DENSE_BLOCK + 3])
+def test_linear_dense_in_blocks(cuda, M):
+    """As above at a width that is cut (3841 columns), and rows of a wider buffer; three-dimensional inputs go whole."""
+    torch.manual_seed(M)
+    N = ops.DENSE_BLOCK - 255
+    x, w = torch.randn(M, 4096 + 8, device=cuda).bfloat16()[:, :4096], torch.randn(N, 4096, device=cuda).bfloat16()
+    assert ops.dense_cut(M, N, 4096)
+    want = x.float() @ w.float().t()
+    # fp32 sums of 4096 terms of size ~1: 2^-24 * 4096 / 2 of the sum of their sizes, 4096 * 0.64
+    assert ((ops.linear_dense(x, w).float() - want).abs() <= 2 ** -8 * want.abs() + 0.32).all()
+    assert ops.linear_dense(x.unsqueeze(1), w).shape == (M, 1, N)
+
+
 @pytest.mark.parametrize("T,k", [(1, 1), (63, 1), (65, 1), (1024, 4), (4097, 1), (683, 6), (2731, 3)])
 @pytest.mark.parametrize("E", [1, 5, 64, 65])
 def test_moe_sort_sizes(cuda, T, k, E):

@@ -315,10 +315,12 @@ def short_conv(u, c0: int, w, b, tok_seg, seg, state, out, act: str = "none", re
 
 
 SSD_CHUNK = 128         # tokens of a chunk (the kernels' constant)
-# segments of at least this many rows are scanned in chunks: 128 heads of 128 x 64, one segment of 16 / 24 / 32 / 128 rows,
-# chunks against token by token: 34 / 35 / 35 / 43 us against 32 / 41 / 50 / 155 us; four segments 61 / 62 / 63 / 73 against
-# 57 / 71 / 86 / 305 us
-SSD_CHUNK_MIN = 24
+# Segments of at least this many rows are scanned in chunks. The kernels alone are level at 24 rows (128 heads of 128 x 64, one segment of
+# 24 / 32 / 128 rows, chunks against token by token: 35 / 35 / 43 us against 41 / 50 / 155), but chunks cost the host three launches a
+# layer and a table, 60 .. 100 us a step of three layers, and steps of few rows wait for the host: beside 8 .. 13 decoded tokens, width
+# 2048, a portion of 45 rows 739 us a step in chunks / 615 without, 2 x 25 rows 754 / 615, one of 64 694 / 755, of 80 741 / 749; width
+# 4096, 2 x 25 rows 906 / 829, 45 rows 821 / 865, 64 rows 737 / 863.
+SSD_CHUNK_MIN = 64
 
 
 def ssd_ok(xbc, heads: int, P: int, N: int, G: int) -> bool:

@@ -827,6 +827,14 @@ def test_scan_in_matrix_core_chunks(Hh, P, N, G, fast):
     assert errs[0][0] < 2 * errs[1][0] + 1e-6 and errs[0][1] < 2 * errs[1][1] + 1e-6
 
 
+def test_short_portions_are_scanned_token_by_token():
+    """A few dozen rows beside decoded tokens make a step that waits for the host: no chunk tables, no launches for them."""
+    for runs, chunks in (([(1, 9, 0), (45, 800, 1)], 0), ([(1, 9, 0), (25, 0, 1), (63, 7, 2)], 0), ([(64, 0, 0)], 1),
+                         ([(1, 3, 0), (300, 5, 1), (40, 0, 2)], 3)):
+        t = hops.chunk_tables(_seg("cpu", runs)[0].numpy(), hops.SSD_CHUNK, hops.SSD_CHUNK_MIN)
+        assert (0 if t is None else len(t[0])) == chunks
+
+
 @pytest.mark.gpu
 def test_chunked_scan_of_rates_and_rows_without_bound():
     """The chunked scan where A_log is past the largest exponent (A = -inf: the state of a token is gone with the next one), and

@@ -730,7 +730,7 @@ __global__ __launch_bounds__(256, NKS * 4 + NVT * 16 <= 96 ? 2 : 1) void window_
 constexpr int WT_WAVES = 8, WT_KEYS = 64, WT_SLOTS = 3, WT_RUN = 512;   // WT_RUN: tiles whose page ids lie in LDS at a time
 constexpr int WT_KB = WT_KEYS * 256, WT_SLOT = 2 * WT_KB;
 constexpr float WT_THR = 8.f;
-// Items x key/value heads from which it runs: a wave each on 256 CUs, fewer leave whole CUs idle that the form above still uses.
+// Items (those that it works on, not the single tokens between them) x key/value heads from which it runs: a wave each on 256 CUs, fewer leave whole CUs idle that the form above still uses.
 // us there / here: 1000 waves (1000 rows) 33 / 40, 1024 (2048 rows, 4 heads) 62 / 66, 1200 47 / 45, 1500 63 / 60, 2048 with a
 // window of 1024 85 / 45.
 constexpr int WT_MIN_WAVES = 1280;
@@ -1228,8 +1228,10 @@ hipError_t kafka_hy_window_attn_mfma(const void* q, int64_t qs, const void* kc, 
                                      int bt_stride, const int* items, int n_items, const int64_t* positions, int H,
                                      int G, int D, int Dv, float scale, int window, const float* sink,
                                      const void* gate, int64_t gs, void* out, int64_t os, int nsplit, float* po,
-                                     float* pml, int64_t T, int shared_keys, float out_scale, int max_tok, int min_rows_tok, hipStream_t st) {
-  // items of up to max_tok tokens here (0: none), those of at least min_rows_tok tokens a wave each (0: none)
+                                     float* pml, int64_t T, int shared_keys, float out_scale, int max_tok, int min_rows_tok,
+                                     int tile_items, hipStream_t st) {
+  // items of up to max_tok tokens here (0: none), those of at least min_rows_tok tokens a wave each (0: none), about tile_items of
+  // which have something to share (window_attn_tile)
   if (n_items <= 0) return hipSuccess;
   const int Ck = shared_keys ? D : G * D, kstep = shared_keys ? 0 : D;
   if (G < 1 || H % G || window < 0 || !kafka_hy_window_attn_mfma_ok(PAGE, D, Dv, H / G)) return hipErrorInvalidValue;
@@ -1246,7 +1248,7 @@ hipError_t kafka_hy_window_attn_mfma(const void* q, int64_t qs, const void* kc, 
                                    (bf16*)out, os, out_scale, min_rows_tok, vec4);
     };
     const bool al = ((reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vt)) & 15) == 0;
-    if (D == 128 && Dv == 128 && al && scale > 0.f && (int64_t)n_items * G >= WT_MIN_WAVES) {
+    if (D == 128 && Dv == 128 && al && scale > 0.f && (int64_t)tile_items * G >= WT_MIN_WAVES) {
       window_attn_tile_kernel<<<dim3((unsigned)G, (unsigned)((n_items + WT_WAVES - 1) / WT_WAVES)), 64 * WT_WAVES, 0, st>>>(
           (const bf16*)q, qs, (const bf16*)kc, (const bf16*)vt, bt, bt_stride, items, n_items, positions, H, G, Ck, kstep,
           scale * LOG2E, window, sink, (const bf16*)gate, gs, (bf16*)out, os, out_scale, min_rows_tok, vec4);

@@ -778,6 +778,23 @@ def window_attn_mfma_ok(q, k_cache, v_cache_t, H: int, G: int, shared_keys: bool
                                              v_cache_t.shape[1] // G, H // G))
 
 
+WINDOW_SHARE_KEYS = 128   # keys of the longest context from which items share them in LDS
+
+
+def shared_items(tokens: int, items: int, tile_tokens: int, kinds, max_keys: int) -> int:
+    """About how many of a step's attention items, of up to ``tile_tokens`` of its ``tokens`` rows each, are tiles of prompt portions
+    that gain from keys shared in LDS (window_attn_tile; it runs from 1280 items x key/value heads on). Beside decoded tokens those
+    are counted from the rows that are more than one an item; items of one token each cannot be told apart then, and a workgroup
+    that meets eight sequences walks one after the other (64 decoded tokens behind 1500 keys beside 2 x 600 rows, 64 heads over 2:
+    268 us, a wave each 135). Nor is there much to share in short contexts: 100 portions of 30 rows, 32 heads over 8, 33 us a wave
+    each / 39 shared, 40 of 64 rows 31 / 34, 20 of 100 26 / 28, 10 of 200 30 / 28, 20 of 100 behind 1000 keys 141 / 78."""
+    if max_keys and max_keys < WINDOW_SHARE_KEYS:
+        return 0
+    if not kinds[0]:
+        return items
+    return -(-(tokens - items) // (tile_tokens - 1)) if tile_tokens > 1 else 0
+
+
 def window_attn(q, k_cache, v_cache_t, block_tables, tok_seg, positions, H: int, G: int, scale: float, window: int,
                 sink, out, tiles=None, max_keys: int = 0, shared_keys: bool = False, out_scale: float = 1.0, gate=None,
                 gate_off: int = 0, kinds=(True, False)) -> None:
@@ -801,6 +818,7 @@ def window_attn(q, k_cache, v_cache_t, block_tables, tok_seg, positions, H: int,
     if _gpu(q):
         if tiles is not None and window_attn_mfma_ok(q, k_cache, v_cache_t, H, G, shared_keys):
             tt = sig_tile_tokens(H, G)
+            share = shared_items(q.shape[0], tiles.shape[0], tt, kinds, max_keys) if kinds[1] else 0
             if window and max_keys:  # a tile's key range is at most the window and its own tokens long
                 max_keys = min(max_keys, window + tt)
             # (shared keys: few key/value heads, every workgroup walks the whole key row - more, shorter ranges)
@@ -814,7 +832,7 @@ def window_attn(q, k_cache, v_cache_t, block_tables, tok_seg, positions, H: int,
                 pml = torch.empty(ns, q.shape[0], H, 2, dtype=torch.float32, device=q.device)
             ext().hy_window_attn_mfma(q, k_cache, v_cache_t, block_tables, tiles, tt, positions, int(H), int(G),
                                       float(scale), int(window), sink, out, ns, po, pml, bool(shared_keys),
-                                      float(out_scale), gate, int(gate_off), mt, mt + 1 if kinds[1] else 0)
+                                      float(out_scale), gate, int(gate_off), mt, mt + 1 if kinds[1] else 0, share)
         else:
             ext().hy_window_attn(q, k_cache, v_cache_t, block_tables, tok_seg, positions, int(H), int(G), float(scale),
                                  int(window), sink, out, bool(shared_keys), float(out_scale), gate, int(gate_off))

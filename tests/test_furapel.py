@@ -1043,6 +1043,18 @@ def test_wide_expert_products_on_256_row_tiles(rows, N, K):
         assert same(ops.grouped_wide(x, gt, r, "glu", True, tile=128, **kw), ref)
 
 
+def test_items_that_share_keys():
+    """Which of a step's attention items count for the kernel that shares keys among eight of them: all of prompt portions, those of
+    more than one token beside decoded ones (160 of one token and 2 portions of 5 items of 8: 10), none where items of one token
+    each cannot be told apart or no context has 128 keys."""
+    assert hops.shared_items(1100, 138, 8, (False, True), 1100) == 138
+    assert hops.shared_items(160 + 2 * 40, 160 + 2 * 5, 8, (True, True), 2000) == 10
+    assert hops.shared_items(160 + 2 * 37, 160 + 2 * 5, 8, (True, True), 2000) == 10
+    assert hops.shared_items(64 + 1200, 64 + 1200, 1, (True, True), 1500) == 0
+    assert hops.shared_items(300, 300, 1, (False, True), 300) == 300
+    assert hops.shared_items(3000, 400, 8, (False, True), 30) == 0 and hops.shared_items(3000, 400, 8, (False, True), 0) == 400
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("window,sink,cols", [(0, False, 0), (100, True, 3)])
 def test_window_attention_of_long_portions(window, sink, cols):

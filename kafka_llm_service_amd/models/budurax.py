@@ -488,8 +488,7 @@ class BuduraxLM:
     def page_bytes(self) -> int:
         """Bytes of one 16-token page over every layer that owns a latent cache."""
         es = torch.empty(0, dtype=self.dtype).element_size()
-        # (the latent part is kept twice where the matrix-core kernel runs: row-major and page-wise transposed)
-        return sum(PAGE * (2 * int(L["mixer"]["kv_rank"]) + int(L["mixer"]["rot_dim"])) * es
+        return sum(PAGE * hops.latent_page_channels(int(L["mixer"]["kv_rank"]), int(L["mixer"]["rot_dim"]), self.dtype, self.device) * es
                    for L in self.cfg.layers
                    if L["type"] == "latent_attention" and L["mixer"].get("kv_from") is None) or 1
 
@@ -498,15 +497,13 @@ class BuduraxLM:
         a masked key's row is never read, but fresh memory must not hold NaN patterns for the debug checks."""
         dev, dt, d = self.device, self.dtype, self.cfg.hidden_size
         pages, shift, conv, ssm = [], [], [], []
-        self.pages_t = []  # page-wise transposed latent copies [blocks, kv_rank, 16] where the MFMA kernel applies
+        self.pages_t = []  # page-wise transposed latent copies (hops.latent_pool_t) where the MFMA kernel applies
         for lw in self.layers:
             m = lw.m
             own = lw.type == "latent_attention" and lw.kv_from is None
             pages.append(torch.zeros(num_blocks, PAGE, int(m["kv_rank"]) + int(m["rot_dim"]), dtype=dt, device=dev)
                          if own else None)
-            self.pages_t.append(torch.zeros(num_blocks, int(m["kv_rank"]), PAGE, dtype=dt, device=dev)
-                                if own and hops.latent_mfma_ok(pages[-1], int(m["kv_rank"]), int(m["rot_dim"]))
-                                else None)
+            self.pages_t.append(hops.latent_pool_t(pages[-1], int(m["kv_rank"]), int(m["rot_dim"])) if own else None)
             shift.append(torch.zeros(num_slots, d, dtype=torch.float32, device=dev) if lw.shift is not None else None)
             if lw.type == "mamba2":
                 Hh, P, N, G = (int(m[k]) for k in ("heads", "vdim", "state", "groups"))

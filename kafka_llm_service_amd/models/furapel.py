@@ -391,8 +391,7 @@ class FurapelLM:
             if L["type"] == "attention":
                 n += int(m["kv_heads"]) * (int(m["dim"]) + int(m["vdim"]))
             elif L["type"] == "latent_attention":
-                # (the latent is kept twice where the matrix-core kernel runs: row-major and page-wise transposed)
-                n += 2 * int(m["kv_rank"])
+                n += hops.latent_page_channels(int(m["kv_rank"]), 0, self.dtype, self.device)
         return PAGE * n * es or 1
 
     def alloc_cache(self, num_blocks: int, num_slots: int):
@@ -401,7 +400,7 @@ class FurapelLM:
         is never used, but fresh memory must not hold NaN patterns for the debug checks."""
         dev, dt = self.device, self.dtype
         pages, state = [], LayerState()
-        self.pages_t = []  # page-wise transposed latent copies [blocks, kv_rank, 16] for the matrix-core kernel
+        self.pages_t = []  # page-wise transposed latent copies (hops.latent_pool_t) for the matrix-core kernel
         for i, _ in self.runs:
             lw = self.layers[i]
             m, st, pt = lw.m, {}, None
@@ -412,8 +411,7 @@ class FurapelLM:
             elif lw.type == "latent_attention":
                 R = int(m["kv_rank"])
                 pages.append(torch.zeros(num_blocks, PAGE, R, dtype=dt, device=dev))
-                if hops.latent_mfma_ok(pages[-1], R, 0):
-                    pt = torch.zeros(num_blocks, R, PAGE, dtype=dt, device=dev)
+                pt = hops.latent_pool_t(pages[-1], R, 0)
             else:
                 H, D, Dv = (int(m[k]) for k in ("heads", "dim", "vdim"))
                 pages.append(None)

@@ -448,8 +448,7 @@ class MagedraLM:
             if L["type"] == "parallel":
                 n += int(m["left"]["kv_heads"]) * (int(m["left"]["dim"]) + int(m["left"]["vdim"]))
             elif L["type"] == "latent_attention":
-                # (the latent is kept twice where the matrix-core kernel runs: row-major and page-wise transposed)
-                n += 2 * int(m["kv_rank"]) + int(m["rot_dim"])
+                n += hops.latent_page_channels(int(m["kv_rank"]), int(m["rot_dim"]), self.dtype, self.device)
         return PAGE * n * es or 1
 
     def alloc_cache(self, num_blocks: int, num_slots: int):
@@ -459,7 +458,7 @@ class MagedraLM:
         hold NaN patterns for the debug checks."""
         dev, dt = self.device, self.dtype
         pages, state = [], LayerState()
-        self.pages_t = []  # page-wise transposed latent copies [blocks, kv_rank, 16] for the matrix-core kernel
+        self.pages_t = []  # page-wise transposed latent copies (hops.latent_pool_t) for the matrix-core kernel
         for lw in self.layers:
             m, st, pt = lw.m, {}, None
             if lw.type == "parallel":
@@ -471,8 +470,7 @@ class MagedraLM:
             elif lw.type == "latent_attention":
                 R, rd = int(m["kv_rank"]), int(m["rot_dim"])
                 pages.append(torch.zeros(num_blocks, PAGE, R + rd, dtype=dt, device=dev))
-                if hops.latent_mfma_ok(pages[-1], R, rd):
-                    pt = torch.zeros(num_blocks, R, PAGE, dtype=dt, device=dev)
+                pt = hops.latent_pool_t(pages[-1], R, rd)
             else:
                 pages.append(None)
                 st["rnn"] = torch.zeros(num_slots, int(m["width"]), dtype=torch.float32, device=dev)

@@ -416,8 +416,8 @@ class MozidraLM:
             m = L["mixer"]
             if L["type"] == "attention":
                 n += int(m["kv_heads"]) * (int(m["dim"]) + int(m["vdim"]))
-            else:  # (the latent is kept twice where the matrix-core kernel runs: row-major and page-wise transposed)
-                n += 2 * int(m["kv_rank"])
+            else:
+                n += hops.latent_page_channels(int(m["kv_rank"]), 0, self.dtype, self.device)
         return PAGE * n * es or 1
 
     def alloc_cache(self, num_blocks: int, num_slots: int):
@@ -426,7 +426,7 @@ class MozidraLM:
         patterns for the debug checks."""
         dev, dt = self.device, self.dtype
         pages = []
-        self.pages_t = []  # page-wise transposed latent copies [blocks, kv_rank, 16] for the matrix-core kernel
+        self.pages_t = []  # page-wise transposed latent copies (hops.latent_pool_t) for the matrix-core kernel
         for lw in self.layers:
             m = lw.m
             if lw.type == "attention":
@@ -437,8 +437,7 @@ class MozidraLM:
             else:
                 R = int(m["kv_rank"])
                 pages.append(torch.zeros(num_blocks, PAGE, R, dtype=dt, device=dev))
-                self.pages_t.append(torch.zeros(num_blocks, R, PAGE, dtype=dt, device=dev)
-                                    if hops.latent_mfma_ok(pages[-1], R, 0) else None)
+                self.pages_t.append(hops.latent_pool_t(pages[-1], R, 0))
         return pages, PageState()
 
     # one step ---------------------------------------------------------------------------------------------------

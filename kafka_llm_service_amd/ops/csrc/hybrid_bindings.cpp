@@ -43,6 +43,7 @@ hipError_t kafka_hy_ssm_scan(int f32, const void* xbc, int64_t xs, const void* p
                              const float* dt_bias, const float* A_log, const float* Dp, int heads, int P, int N, int G,
                              const int* seg, int R, int min_n, int max_n, float* state, float* y, int64_t ys,
                              hipStream_t st);
+int kafka_hy_latent_decode_ok(const void* cache, int R, int rd, const void* out, int64_t o_h, int64_t o_t);
 int kafka_hy_latent_rows_ok(int R, int rd, int D, int Dv);
 hipError_t kafka_hy_latent_gather(const void* cache, int R, int rd, const int* bt, int bt_stride, const int* px,
                                   const int* blocks, int n_blocks, void* ck, void* kr, hipStream_t st);
@@ -442,8 +443,11 @@ void latent_attn_mfma(at::Tensor q_lat, at::Tensor q_rot, at::Tensor cache, at::
   const int64_t H = q_lat.size(0), T = q_lat.size(1), R = q_lat.size(2), rd = q_rot.size(2);
   TORCH_CHECK(q_rot.size(0) == T && q_rot.size(1) == H && out.size(0) == H && out.size(1) == T && out.size(2) == R,
               "latent_attn_mfma: shapes");
+  // (a copy of no pages where the kernel that runs does not read it)
+  const bool rows_only = cache_t.dim() == 3 && cache_t.size(0) == 0 && cache.dim() == 3 &&
+                         kafka_hy_latent_decode_ok(cache.data_ptr(), (int)R, (int)rd, out.data_ptr(), out.stride(0), out.stride(1));
   TORCH_CHECK(cache.is_contiguous() && cache.dim() == 3 && cache.size(2) == R + rd && cache_t.is_contiguous() &&
-                  cache_t.dim() == 3 && cache_t.size(0) == cache.size(0) && cache_t.size(1) == R &&
+                  cache_t.dim() == 3 && (rows_only || cache_t.size(0) == cache.size(0)) && cache_t.size(1) == R &&
                   cache_t.size(2) == cache.size(1), "latent_attn_mfma: cache [pages, 16, R + rd] and [pages, R, 16]");
   TORCH_CHECK(kafka_hy_latent_mfma_ok((int)cache.size(1), (int)R, (int)rd), "latent_attn_mfma: sizes not supported");
   // 16-byte loads: every row start must be a multiple of 8 elements

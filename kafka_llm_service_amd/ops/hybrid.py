@@ -81,7 +81,9 @@ def latent_prep(qgd, H, dim, rd, R, dkv_off, dkv_w, eps, positions, cos_sin, rot
                 q_rot, cache_t=None) -> None:
     """RMS norm of the latent and rotary on the shared key part of the fused projection row -> the row's cache slot
     ([latent | rotated key]; with ``cache_t`` [pages, kv_rank, page] also the latent page-wise transposed, the value
-    operand of the matrix-core attention kernel); rotary on every head's query part -> ``q_rot``."""
+    operand of the matrix-core attention kernel, see ``latent_pool_t``); rotary on every head's query part -> ``q_rot``."""
+    if cache_t is not None and cache_t.shape[0] == 0:
+        cache_t = None
     if rd == 0 and (rot_dims or cos_sin is not None):
         raise ValueError("latent_prep: a rotation needs a rotated part")
     if _gpu(qgd):
@@ -103,6 +105,25 @@ MFMA_ROWS = 32  # (token, head) rows of one tile of the matrix-core attention ke
 def latent_mfma_ok(cache: torch.Tensor, R: int, rd: int) -> bool:
     """bf16 GPU caches of sizes the matrix-core kernel takes (16-token pages, kv_rank % 32 == 0, rot_dim % 16 == 0)."""
     return cache.is_cuda and cache.dtype == torch.bfloat16 and bool(ext().hy_latent_mfma_ok(cache.shape[1], R, rd))
+
+
+def latent_direct(R: int, rd: int) -> bool:
+    """Sizes whose matrix-core kernels read the latent rows as they are cached: no transposed copy of them."""
+    return R == 512 and rd in (0, 64)
+
+
+def latent_page_channels(R: int, rd: int, dtype: torch.dtype, device) -> int:
+    """Channels a latent cache keeps per token: the row and, where the matrix-core kernel wants one, the transposed copy."""
+    once = latent_direct(R, rd) and dtype == torch.bfloat16 and torch.device(device).type == "cuda"
+    return R + rd + (0 if once else R)
+
+
+def latent_pool_t(cache: torch.Tensor, R: int, rd: int):
+    """The transposed copy [pages, kv_rank, page] beside a latent cache: of no pages where the matrix-core kernels do without it, None
+    where they do not run."""
+    if not latent_mfma_ok(cache, R, rd):
+        return None
+    return torch.zeros(0 if latent_direct(R, rd) else cache.shape[0], R, cache.shape[1], dtype=cache.dtype, device=cache.device)
 
 
 def tile_tokens(heads: int) -> int:
@@ -128,7 +149,7 @@ def attn_splits(n_tiles: int, heads: int, max_keys: int, kv_rank: int = 0, rot_d
     128 x 1000 1: 125, 2: 86, 4: 99."""
     wgs = max(1, n_tiles * -(-heads // MFMA_ROWS))
     ns = min(ATTN_SPLIT_MAX, ATTN_SPLIT_WGS // wgs, -(-max_keys // 128))
-    if kv_rank == 512 and rot_dim in (0, 64):
+    if latent_direct(kv_rank, rot_dim):
         if max_keys <= 256:
             return 1
         ns = min(ns, max(-(-100 // max(1, seqs or n_tiles)), 2 if max_keys >= 2000 else 1))
@@ -139,7 +160,7 @@ def latent_attn(q_lat, q_rot, cache, block_tables, tok_seg, seg, positions, scal
                 tiles=None, max_keys: int = 0, window: int = 0, sink=None) -> None:
     """Causal softmax attention of every row's heads over its sequence's cached [latent | rotated key] rows:
     out[h, t] = sum_j softmax_j((q_lat[h, t] . c_j + q_rot[t, h] . k_j) scale) c_j over the keys j <= position[t].
-    With the transposed latent copy ``cache_t`` (not read at kv_rank 512 with 0 or 64 rotated channels) and ``tiles`` (int32 [n, 4] =
+    With the transposed latent copy ``cache_t`` (``latent_pool_t``: of no pages where nothing reads it) and ``tiles`` (int32 [n, 4] =
     (first row, tokens, segment, 0), at most ``tile_tokens(H)`` tokens of one segment each) bf16 runs on the matrix cores; else one wave per (row, 4
     heads) on the vector units (fp32, odd sizes). ``max_keys`` (the step's longest context) lets a launch of few
     tiles split its key ranges over more workgroups (``attn_splits``).
@@ -148,6 +169,9 @@ def latent_attn(q_lat, q_rot, cache, block_tables, tok_seg, seg, positions, scal
     if window < 0:
         raise ValueError("latent_attn: window must be positive (0 = every earlier position)")
     if _gpu(q_lat):
+        rows_only = cache_t is not None and cache_t.shape[0] == 0   # (its kernel reads 16-byte pieces and writes 8-byte ones)
+        if rows_only and (cache.data_ptr() % 16 or out.data_ptr() % 8 or out.stride(0) % 4 or out.stride(1) % 4):
+            cache_t = None
         if cache_t is not None and tiles is not None and q_lat.dtype == torch.bfloat16:
             H, T, R = q_lat.shape
             if window:  # a key range is at most the window long
@@ -211,7 +235,7 @@ def expanded_pays(portions, window: int, heads: int, kv_rank: int, rot_dim: int)
     rounds = r * heads / MFMA_ROWS / 256
     rounds = float(-(-rounds // 1)) if rounds > 1 else 1 / (1 / rounds // 1)
     # a key of a tile and a tile, by kernel
-    key_us, tile_us = (0.052, 18) if kv_rank == 512 and rot_dim in (0, 64) else (0.03 + 0.00025 * kv_rank, 25)
+    key_us, tile_us = (0.052, 18) if latent_direct(kv_rank, rot_dim) else (0.03 + 0.00025 * kv_rank, 25)
     latent = 20 + rounds * (work / r * key_us + tile_us)
     expanded = (25 if rot_dim else 15) + 0.045 * kv_rank + max(walk, turns / 512) * (0.052 if rot_dim else 0.035) + \
         ctx * heads * kv_rank * 4.6e-7

@@ -907,6 +907,53 @@ def test_key_ranges_by_size():
     assert hops.attn_splits(64, 32, 8000, 512, 64, 1) == 4 and hops.attn_splits(64, 32, 8000, 512, 64, 64) == 2
 
 
+def cfg_direct():
+    """kv_rank 512 with 64 rotated channels and heads of 128: the sizes whose kernels read the cached rows alone."""
+    ff = {"kind": "dense", "ff": 96}
+    return {"architecture": "Budurax", "vocab": 173, "width": 80, "norm": {"eps": 1e-5}, "token_side": {"dim": 4},
+            "layers": [{"type": "latent_attention", "mixer": _attn(3, 128, 64, 64, 128, 512), "mlp": ff},
+                       {"type": "mamba2", "mixer": _mamba(2, 16, 8, 1, 2, 4), "mlp": ff},
+                       {"type": "latent_attention", "mixer": _attn(3, 128, 64, 64, 128, 512), "mlp": ff}]}
+
+
+def test_channels_of_latent_pages():
+    """What a cached token takes: the row, and a transposed copy except in bf16 on the GPU at the sizes that do without."""
+    for R, rd, dtype, dev, want in ((512, 64, torch.bfloat16, "cuda", 576), (512, 0, torch.bfloat16, "cuda:0", 512),
+                                    (512, 32, torch.bfloat16, "cuda", 1056), (256, 64, torch.bfloat16, "cuda", 576),
+                                    (512, 64, torch.float32, "cuda", 1088), (512, 64, torch.bfloat16, "cpu", 1088)):
+        assert hops.latent_page_channels(R, rd, dtype, dev) == want, (R, rd, dtype, dev)
+
+
+@pytest.mark.gpu
+def test_latent_rows_are_cached_once():
+    """kv_rank 512 in the engine: no transposed copy is allocated or charged, and portions, single tokens and a mixed step agree
+    with the plain model; an output that the row kernel cannot write goes the vector kernel's way."""
+    b = Bench(cfg_direct(), seed=11)
+    t, u = toks(200, 173, 1), toks(41, 173, 2)
+    eng = b.engine("cuda:0", "bfloat16", blocks=40)
+    assert all(p is None or p.shape == (0, 512, 16) for p in eng.model.pages_t) and eng.model.pages_t[0] is not None
+    assert eng.model.page_bytes() == 2 * 16 * 576 * 2
+    assert rel_err(feed_all(eng, "c", t, [130, 2, 61, 1]), b.oracle(t)) < TOL["bfloat16"]
+    got = [eng.feed([("u", u[:40], list(range(40)))])]
+    got.append(eng.feed([("u", u[40:], [0]), ("v", t[:50], list(range(50)))], ["u", "v"]))
+    assert rel_err(torch.cat([got[0], got[1][:1]]), b.oracle(u)) < TOL["bfloat16"]
+    # 40 keys, a row of the output one element off its 8 bytes
+    dev = "cuda:0"
+    cache = torch.randn(3, 16, 576, device=dev).bfloat16()
+    bt, pos = torch.tensor([[2, 0, 1]], dtype=torch.int32, device=dev), torch.tensor([39], device=dev)
+    seg, ts = _seg(dev, [(1, 39, 0)])
+    q, qr = torch.randn(4, 1, 512, device=dev).bfloat16(), torch.randn(1, 4, 64, device=dev).bfloat16()
+    tiles = torch.tensor([(0, 1, 0, 0)], dtype=torch.int32, device=dev)
+    outs = []
+    for off in (0, 1):
+        out = torch.empty(4, 1, 516, device=dev, dtype=torch.bfloat16)[:, :, off:off + 512]
+        hops.latent_attn(q, qr, cache, bt, ts, seg, pos, 0.05, out, torch.empty(0, 512, 16, dtype=torch.bfloat16, device=dev),
+                         tiles, 40)
+        outs.append(out.float())
+    # weights and results in bf16 on one side only: 2^-8 of the largest value
+    assert (outs[0] - outs[1]).abs().max().item() <= 2 ** -8 * 1.1 * cache.float().abs().max().item()
+
+
 def test_where_expanded_keys_pay():
     """The choice between the latent space and expanded keys and values at measured points of both sides (us in the latent space /
     expanded), and its effect on a step's tables."""

@@ -1062,6 +1062,62 @@ def test_expanded_keys_by_groups_of_heads(H, monkeypatch):
 
 
 @pytest.mark.gpu
+def test_decoded_tokens_beside_expanded_portions(monkeypatch):
+    """A step of two decoded tokens, a portion of 130 rows and one of 7 in the engine, the portions on expanded keys and values and the
+    single tokens in the latent space beside them, into the same rows; histories behind all of them, against the plain model."""
+    b = Bench(cfg_direct(), seed=5)
+    eng = b.engine("cuda:0", "bfloat16", blocks=60, seqs=4)
+    t = {k: toks(n, 173, i) for i, (k, n) in enumerate((("a", 71), ("b", 34), ("p", 200), ("s", 27)))}
+    cut = {"a": 70, "b": 33, "p": 70, "s": 20}
+    got = {k: [eng.feed([(k, t[k][:n], list(range(n)))])] for k, n in cut.items()}
+    monkeypatch.setattr(hops, "expanded_pays", lambda *a: True)
+    calls, orig = [], hops.latent_attn_portions
+
+    def spy(*a):
+        calls.append(a[5][0])      # the rows in front of the portions
+        return orig(*a)
+
+    monkeypatch.setattr(hops, "latent_attn_portions", spy)
+    order = ["a", "b", "p", "s"]
+    out = eng.feed([(k, t[k][cut[k]:], list(range(len(t[k]) - cut[k]))) for k in order], order)
+    assert calls == [2, 2]         # (two layers)
+    at = 0
+    for k in order:
+        n = len(t[k]) - cut[k]
+        assert rel_err(torch.cat([got[k][0], out[at:at + n]]), b.oracle(t[k])) < TOL["bfloat16"], k
+        at += n
+
+
+@pytest.mark.gpu
+def test_single_token_behind_more_pages_than_a_run():
+    """kv_rank 512, one range over 16400 keys: page ids are kept for 16384 keys at a time. Single keys on both sides of that line, the
+    first and the last carry the result (queries of 80 times a unit key: every other key's score is at least 40 lower), and a flat
+    softmax over all of them: an average of unit vectors, weights in bf16 (2^-9 of it)."""
+    device, H, R, rd, n = "cuda:0", 4, 512, 64, 16400
+    torch.manual_seed(3)
+    kv = torch.nn.functional.normalize(torch.randn(n, R + rd, device=device), dim=-1).bfloat16()
+    perm = torch.randperm(n // 16, device=device)
+    cache = torch.empty(n // 16, 16, R + rd, dtype=torch.bfloat16, device=device)
+    cache[perm] = kv.view(-1, 16, R + rd)
+    bt, pos = perm.int()[None].contiguous(), torch.tensor([n - 1], device=device)
+    tiles = torch.tensor([(0, 1, 0, 0)], dtype=torch.int32, device=device)
+    cache_t = torch.empty(0, R, 16, dtype=torch.bfloat16, device=device)
+
+    def attend(q, scale):
+        out = torch.empty(H, 1, R, dtype=torch.bfloat16, device=device)
+        hops.ext().hy_latent_attn_mfma(q[:R].expand(H, 1, R).contiguous(), q[R:].expand(1, H, rd).contiguous(), cache, cache_t, bt,
+                                       tiles, hops.tile_tokens(H), pos, scale, out, 1, None, None, 0, None)
+        return out[:, 0].float()
+
+    for j in (0, 16351, 16383, 16384, 16399):
+        got = attend((kv[j].float() * 80).bfloat16(), 1.0)
+        assert (got - kv[j, :R].float()).abs().max().item() < 2 ** -8
+    flat = attend(torch.zeros(R + rd, dtype=torch.bfloat16, device=device), 1.0)
+    want = kv[:, :R].double().mean(0)
+    assert (flat.double() - want).abs().max().item() < 2 ** -8 * want.abs().max().item() + 1e-6
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("d,T", [(4, 3), (1024, 3), (1028, 5), (1030, 5), (4096, 7), (4096, 600), (4100, 3), (1022, 2)])
 def test_row_kernels_over_widths(dtype, d, T):

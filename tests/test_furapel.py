@@ -1098,3 +1098,85 @@ def test_window_attention_of_long_portions(window, sink, cols):
         want = want * torch.sigmoid(gate[at:at + n, 1:].double())[..., None]
         assert torch.allclose(out[at:at + n].double().cpu().view(n, H, D), want, atol=2e-2), r
         at += n
+
+
+def _paged(segs, G, D, seed):
+    """Caches of the segments (rows, history) on scattered pages: keys, transposed values, block table, and each segment's keys and
+    values [tokens, G, D] in order."""
+    g = torch.Generator().manual_seed(seed)
+    pages = [-(-(n + p0) // 16) for n, p0 in segs]
+    perm = torch.randperm(sum(pages), generator=g)
+    kc = torch.randn(sum(pages), 16, G * D, generator=g).bfloat16()
+    vt = torch.randn(sum(pages), G * D, 16, generator=g).clamp(-4.5, 4.5).bfloat16()
+    bt = torch.zeros(len(segs), max(pages), dtype=torch.int32)
+    kv, at = [], 0
+    for r, (n, p0) in enumerate(segs):
+        ids = perm[at:at + pages[r]]
+        bt[r, :pages[r]] = ids
+        at += pages[r]
+        kv.append((kc[ids].reshape(-1, G, D)[:p0 + n],
+                   vt[ids].view(-1, G, D, 16).permute(0, 3, 1, 2).reshape(-1, G, D)[:p0 + n]))
+    return kc, vt, bt, kv
+
+
+def _attend(q, kv, p, window):
+    """float64 softmax attention of rows q [n, G, rep, D] at positions p over a segment's keys and values."""
+    k, v = (x.to(q.device).double() for x in kv)
+    s = torch.einsum("ngrd,kgd->ngrk", q.double(), k) * q.shape[-1] ** -0.5
+    j = torch.arange(k.shape[0], device=q.device)
+    see = (j <= p[:, None]) & (j > p[:, None] - window if window else True)
+    return torch.einsum("ngrk,kgd->ngrd", torch.softmax(s.masked_fill(~see[:, None, None], float("-inf")), -1), v)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("window", [0, 130])
+@pytest.mark.parametrize("H,G", [(32, 8), (16, 8), (32, 2)])
+def test_window_attention_on_shared_keys(H, G, window):
+    """Items of several tokens (8, 16 and 2) that share their keys eight at a time: portions that are no multiple of an item, with one
+    token left over or fewer than a workgroup's items, behind histories and fresh; decoded tokens in front of and between them, whose
+    items the kernel passes by (the other kernel of the step takes them). Values up to 4.5: a weight's rounding to bf16 (2^-9 of each
+    term) and the result's (2^-9) move an output by up to 0.018."""
+    dev, D = "cuda:0", 128
+    tt = hops.sig_tile_tokens(H, G)
+    segs = [(1, 40), (1, 700), (3 * tt + 1, 0), (1, 17), (411, 0), (2 * tt, 333), (1, 129), (1, 0), (500, 61), (tt - 1 or 1, 64), (399, 1)]
+    segs += [(1000, 0)] if tt == 16 else [(301, 0)]
+    if tt == 16:
+        segs.append((640, 10))
+    kc, vt, bt, kv = _paged(segs, G, D, H + G)
+    tiles, pos = [], []
+    for r, (n, p0) in enumerate(segs):
+        tiles += [(len(pos) + a, min(tt, n - a), r, 0) for a in range(0, n, tt)]
+        pos += list(range(p0, p0 + n))
+    T, longest = len(pos), max(n + p0 for n, p0 in segs)
+    assert hops.shared_items(T, len(tiles), tt, (True, True), longest) * G >= 1280
+    torch.manual_seed(H)
+    q = torch.randn(T, H * D, device=dev).bfloat16()
+    out = torch.full((T, H * D), float("nan"), dtype=torch.bfloat16, device=dev)
+    hops.window_attn(q, kc.to(dev), vt.to(dev), bt.to(dev), None, torch.tensor(pos, device=dev), H, G, D ** -0.5, window, None, out,
+                     torch.tensor(tiles, dtype=torch.int32, device=dev), longest, kinds=(True, True))
+    at = 0
+    for r, (n, p0) in enumerate(segs):
+        want = _attend(q[at:at + n].view(n, G, H // G, D), kv[r], torch.arange(p0, p0 + n, device=dev), window)
+        assert torch.allclose(out[at:at + n].double().view_as(want), want, atol=2e-2), (r, n, p0)
+        at += n
+
+
+@pytest.mark.gpu
+def test_shared_keys_past_a_run_of_pages():
+    """Shared keys of a portion that goes on behind more than 32768 keys, for which page ids are kept at a time: rows in front of, at and
+    behind that line, the keys around it loud in some of them (their weight is one), the same bound as above."""
+    dev, H, G, D, p0, n = "cuda:0", 64, 2, 128, 32500, 660
+    kc, vt, bt, kv = _paged([(n, p0)], G, D, 7)
+    torch.manual_seed(7)
+    q = (torch.randn(n, G, H // G, D) / 4).bfloat16()
+    rows = [0, 200, 267, 268, 269, 400, 659]
+    for r, j in ((268, 32768), (269, 32767), (400, 32768), (659, 32767)):
+        q[r] = (kv[0][0][j, :, None] * 4).expand(G, H // G, D)
+    qg = q.view(n, H * D).to(dev)
+    out = torch.full((n, H * D), float("nan"), dtype=torch.bfloat16, device=dev)
+    assert hops.shared_items(n, n, 1, (False, True), p0 + n) * G >= 1280
+    hops.window_attn(qg, kc.to(dev), vt.to(dev), bt.to(dev), None, torch.arange(p0, p0 + n, device=dev), H, G, D ** -0.5, 0, None,
+                     out, torch.tensor([(i, 1, 0, 0) for i in range(n)], dtype=torch.int32, device=dev), p0 + n, kinds=(False, True))
+    assert not torch.isnan(out).any()
+    want = _attend(q[rows].to(dev), kv[0], torch.tensor([p0 + r for r in rows], device=dev), 0)
+    assert torch.allclose(out[rows].double().view_as(want), want, atol=2e-2)

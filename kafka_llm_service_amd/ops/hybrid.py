@@ -136,24 +136,20 @@ ATTN_SPLIT_WGS = 256
 ATTN_SPLIT_MAX = 32
 
 
-def attn_splits(n_tiles: int, heads: int, max_keys: int, kv_rank: int = 0, rot_dim: int = 0, seqs: int = 0) -> int:
+def attn_splits(n_tiles: int, heads: int, max_keys: int, kv_rank: int = 0, rot_dim: int = 0) -> int:
     """Key-range splits of a matrix-core attention launch: few tiles (a decode step's one tile per sequence) against long contexts are
     dealt over more workgroups, each at least 128 keys long; a merge pass combines them, and costs the host another launch: contexts
-    whose ranges would gain less than that stay whole. ``seqs``: sequences the tiles belong to (0: a tile each).
+    whose ranges would gain less than that stay whole.
 
-    us by ranges, single tokens, 32 heads, operands from memory. kv_rank 512 (``latent_decode``): one sequence x 256 keys 1: 26, 2: 23;
-    512 1: 39, 4: 24; 1706 1: 98, 8: 30, 16: 30; 8000 16: 48, 32: 42. There the cache's rows from memory bound some dozens of
-    sequences, and more ranges than their walk needs only add traffic: 16 x 8000 8: 77, 16: 83; 32 x 1706 4: 45, 8: 47, 16: 63; 64 x 1706
-    1: 100, 2: 67, 4: 68, 8: 81; 100 x 700 1: 52, 2: 51; 128 x 1706 1: 107, 2: 113; 128 x 4000 1: 219, 2: 191; 200 x 1706 1: 139, 2: 168.
-    kv_rank 256 + 32: one x 130 1: 32, 2: 30; one x 256 1: 39, 2: 30; 64 x 1000 1: 116, 2: 74, 4: 55, 8: 69; 128 x 200 1: 39, 2: 37;
-    128 x 1000 1: 125, 2: 86, 4: 99."""
+    Whole steps of three layers, us by ranges, contexts of unequal lengths (the longest walk counts) up to: 64 sequences x 2048, kv_rank
+    512 + 64, 1: 1021, 2: 975, 4: 964, 8: 975; 16 x 8000 1: 1103, 8: 756, 16: 743; 32 x 3000 1: 886, 4: 777, 8: 771, 16: 785; 100 x 1200
+    1: 1222, 2: 1205, 4: 1219. The launch alone, single tokens of 32 heads, operands from memory: one x 130 keys 1: 25, 2: 23; one x 256
+    1: 26, 2: 23; 512 1: 39, 4: 24; 8000 16: 48, 32: 42; kv_rank 256 + 32: one x 130 1: 32, 2: 30; one x 256 1: 39, 2: 30; 64 x 1000
+    1: 116, 2: 74, 4: 55, 8: 69; 128 x 200 1: 39, 2: 37; 128 x 1000 1: 125, 2: 86, 4: 99."""
+    if max_keys <= (256 if latent_direct(kv_rank, rot_dim) else 160):
+        return 1
     wgs = max(1, n_tiles * -(-heads // MFMA_ROWS))
-    ns = min(ATTN_SPLIT_MAX, ATTN_SPLIT_WGS // wgs, -(-max_keys // 128))
-    if latent_direct(kv_rank, rot_dim):
-        if max_keys <= 256:
-            return 1
-        ns = min(ns, max(-(-100 // max(1, seqs or n_tiles)), 2 if max_keys >= 2000 else 1))
-    return 1 if max_keys <= 160 else max(1, ns)
+    return max(1, min(ATTN_SPLIT_MAX, ATTN_SPLIT_WGS // wgs, -(-max_keys // 128)))
 
 
 def latent_attn(q_lat, q_rot, cache, block_tables, tok_seg, seg, positions, scale, out, cache_t=None,
@@ -176,8 +172,7 @@ def latent_attn(q_lat, q_rot, cache, block_tables, tok_seg, seg, positions, scal
             H, T, R = q_lat.shape
             if window:  # a key range is at most the window long
                 max_keys = min(max_keys, window + tile_tokens(H))
-            seqs = 0 if seg is None else min(tiles.shape[0], seg.shape[0])
-            ns = attn_splits(tiles.shape[0], H, max_keys, R, q_rot.shape[2], seqs) if max_keys else 1
+            ns = attn_splits(tiles.shape[0], H, max_keys, R, q_rot.shape[2]) if max_keys else 1
             po = pml = None
             if ns > 1:
                 po = torch.empty(ns, H, T, R, dtype=torch.float32, device=q_lat.device)

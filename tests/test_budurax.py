@@ -895,16 +895,14 @@ def test_portion_tables():
 
 def test_key_ranges_by_size():
     """Key ranges of single tokens' latent attention at measured points: whole where a merge costs what it saves, as many as fill the
-    chip otherwise and, at kv_rank 512, no more than the rows' way from memory leaves room for; steps without tiles too."""
+    chip otherwise, of at least 128 keys; launches without tiles too."""
     for n, heads, keys, rank, rot, want in ((1, 32, 130, 512, 64, 1), (1, 32, 256, 512, 0, 1), (1, 32, 512, 512, 64, 4),
-                                            (1, 32, 1706, 512, 64, 14), (1, 32, 8000, 512, 64, 32), (16, 32, 8000, 512, 64, 7),
-                                            (64, 32, 1706, 512, 64, 2), (128, 32, 1706, 512, 64, 1), (128, 32, 4000, 512, 64, 2),
-                                            (200, 32, 8000, 512, 64, 1), (64, 64, 1706, 512, 64, 2), (128, 32, 1000, 256, 32, 2),
-                                            (1, 32, 130, 256, 32, 1), (1, 32, 256, 256, 32, 2), (64, 32, 1000, 384, 64, 4),
-                                            (48, 16, 1706, 512, 32, 5), (0, 32, 8000, 512, 64, 32), (0, 32, 100, 256, 0, 1)):
+                                            (1, 32, 1706, 512, 64, 14), (1, 32, 8000, 512, 64, 32), (16, 32, 8000, 512, 64, 16),
+                                            (64, 32, 2048, 512, 64, 4), (100, 32, 1200, 512, 64, 2), (200, 32, 8000, 512, 64, 1),
+                                            (64, 64, 2048, 512, 64, 2), (128, 32, 1000, 256, 32, 2), (1, 32, 130, 256, 32, 1),
+                                            (1, 32, 256, 256, 32, 2), (64, 32, 1000, 384, 64, 4), (48, 16, 1706, 512, 32, 5),
+                                            (0, 32, 8000, 512, 64, 32), (0, 32, 100, 256, 0, 1)):
         assert hops.attn_splits(n, heads, keys, rank, rot) == want, (n, heads, keys, rank, rot)
-    # 64 rows of one portion read the same rows
-    assert hops.attn_splits(64, 32, 8000, 512, 64, 1) == 4 and hops.attn_splits(64, 32, 8000, 512, 64, 64) == 2
 
 
 def cfg_direct():

@@ -293,7 +293,7 @@ class _Layer:
 def latent_mix(q, q_rot, cache, cache_t, lw, inp, m: SegMeta, ao, window: int = 0, sink=None, gate=None) -> None:
     """Latent attention of a step's rows: ao [T, H vdim] from q [T, H, dim] and the rotated q_rot [T, H, rot_dim], times
     sigmoid(gate) when given. Decoded tokens attend in the latent space (q_lat = W_uk^T q, out = W_uv (sum p c)), prompt
-    portions on expanded keys and values where the sizes allow."""
+    portions on expanded keys and values where the sizes allow and it is faster (``hops.expanded_pays``)."""
     T, H, D = q.shape
     R, Dv = lw.uk_h.shape[2], lw.uv_ht.shape[2]
     tables = m.portions(window, H, R, q_rot.shape[2]) if cache_t is not None and lw.scale > 0 and \

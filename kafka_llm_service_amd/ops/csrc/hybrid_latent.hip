@@ -55,8 +55,9 @@ __global__ __launch_bounds__(NT) void latent_gather_kernel(const bf16* __restric
 //   values   O^T += V^T P^T: the weights are the right operand as they lie in the registers, the left one is a channel's 8
 //            consecutive keys.
 // What bounds it: a wave's chain of scores, softmax and values (two waves per SIMD hide part of it), and half the LDS rate
-// for the operands; K and V of a head come from its XCD's cache. 2048 fresh rows x 32 heads with
-// the products around it 178 us (latent space: 1170), 8192 rows with a window of 1024 216 us alone, 0.6 PFLOP/s (4550).
+// for the operands; K and V of a head come from its XCD's cache. With the gather and the products around it, operands from
+// memory, 32 heads: 2048 fresh rows of 128 + 64 channels 192 us (in the latent space 626), 8192 rows of 128 + 0 with a window of
+// 1024 310 (2120; this kernel alone 209 of them, 0.6 PFLOP/s).
 // ND, NR: steps of 16 channels of a head's own and rotated key part; NV: tiles of 32 value channels.
 template <int ND, int NR, int NV, bool GATE>
 __global__ __launch_bounds__(NT, 2) void latent_rows_kernel(
@@ -228,8 +229,8 @@ __global__ __launch_bounds__(NT, 2) void latent_rows_kernel(
 //            four operands by byte permutes.
 // What bounds it: a block's chain of waits, softmax and products (1.5 us; Q's scores want 72 registers and one workgroup fits a
 // CU), with many sequences the rows' way to the CUs as well. The walk for other ranks (hybrid.hip) reads keys in 32-byte pieces
-// and the values from a second, transposed copy; here, with the launch's merge, 32 heads: 64 sequences x 1706 keys 134 -> 44 us
-// (126 MB), 16 sequences 68 -> 28, one 52 -> 23, one x 8000 109 -> 34.
+// and the values from a second, transposed copy; here, with the launch's merge, 32 heads, operands from memory: 64 sequences x 1706
+// keys 168 -> 70 us (126 MB; from a warm cache 131 -> 51), 16 sequences 93 -> 38, one 80 -> 28, one x 8000 136 -> 41.
 // Rows past the tile's last position are masked as keys and zeroed as values: what a page holds there does not matter.
 constexpr int LD_R = 512, LD_KEYS = 32, LD_SLOTS = 4;
 constexpr int LD_RUN = 512;   // blocks whose page ids lie in LDS at a time (16k tokens)

@@ -16,8 +16,8 @@
 // at SSD_FLOOR or above: every decay over such a token is zero in fp32 either way, and the sums stay finite where A or dt do not.
 //
 // What bounds it: the chunks' contributions and entry states through memory (67 MB written, read and written by the
-// carry, read at 2048 tokens x 128 heads of 128 x 64) and the LDS reads of the split products. Measured there, one layer:
-// 53 + 33 + 102 us; the token-by-token form in two passes over chunks of 256 took 2 x 1196 + 87 us.
+// carry, read at 2048 tokens x 128 heads of 128 x 64) and the LDS reads of the split products. Measured there, one layer of a
+// step: 55 + 33 + 108 us; the token-by-token form in two passes over chunks of 256 took 2 x 1196 + 87 us.
 #include "chunk_common.h"
 
 namespace kafka {

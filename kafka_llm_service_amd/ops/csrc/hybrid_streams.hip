@@ -386,9 +386,9 @@ __global__ __launch_bounds__(NT) void window_attn_kernel(const AT* __restrict__ 
 // unnormalised accumulators in po [z][T][H Dv] and (row maximum, row sum) in pml [z][T][H][2] for window_merge.
 // Needs 16-token pages, D % 16 == 0, at most 32 query heads per key/value head.
 // What bounds it: a block's chain of key loads, maxima, weights and value loads. A decoded token fills few of the 32 rows, and
-// the others' softmax is left out (their weights in LDS stay zero); maxima go lane to lane without LDS. With the merge, before / now,
-// us: 16 sequences x 1700 keys, 32 heads over 8, 40 / 31, 64 sequences 120 / 103, one x 8000 43 / 27,
-// 16 sequences, 32 over 2, 25 / 19.
+// the others' softmax is left out (their weights in LDS stay zero); maxima go lane to lane without LDS. With the merge, operands from
+// memory, before / now, us: 16 sequences x 1700 keys, 32 heads over 8, 61 / 57, 64 sequences 159 / 153, one x 8000 50 / 37,
+// 16 sequences, 32 over 2, 32 / 27 (from a warm cache 43 / 34, 111 / 105, 45 / 28, 27 / 22).
 constexpr int WM_ROWS = 32;
 
 // the largest of a lane half's 32 values, in each of its lanes: neighbours, pairs, mirrored eights and sixteens, the other sixteen

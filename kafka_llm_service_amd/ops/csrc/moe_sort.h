@@ -1,4 +1,5 @@
-// Stable sort of a step's routed entries by expert, one workgroup of 1024 threads (moe.hip, moe_wide.hip).
+// Stable sort of a step's routed entries by expert, one workgroup of 1024 threads or one per part of the entries (moe.hip,
+// moe_wide.hip).
 #pragma once
 #include "common.h"
 

@@ -4,15 +4,16 @@
 //                  whose experts have many rows. The weights come in the wave-tiled order of the weight-streaming
 //                  kernels (Wt[E][N/32][K/16][64][8]): a wave owns 64 columns and loads its operands straight from
 //                  memory in 1 KB pieces; only the activations go through LDS (64-deep steps, double buffered, next
-//                  step's loads in flight), where all four waves share them. Work items are ordered row tile first, then
-//                  column tile, then expert, and every XCD takes one contiguous stretch of them: the row tiles of a
-//                  column tile run side by side on one L2 and its weights leave memory once.
+//                  step's loads in flight), where all four waves share them. Work items are ordered row tile first (up to 2048
+//                  rows), then column tile, then the next rows, then expert, and every XCD takes one contiguous stretch of
+//                  them: the row tiles of a column tile run side by side on one L2 and its weights leave memory once.
 //                  Epilogues: silu(gate) * up or its clamped form on GLU-interleaved tiles (a wave holds both tiles of a
 //                  pair), relu squared, the weighted combine into fp32 rows, or the weighted rows as they are (in entry
 //                  order; their consumer gathers a token's rows through the sort's inverse, no atomics).
 //   grouped_ring   the same for experts of more rows: 256 x 256 tiles, both operands through a ring in LDS
-//   moe_sort       stable sort of (token, choice) entries by expert, one workgroup: every wave counts and then places
-//                  its stretch of the entries 64 at a time, equal experts found by ballots over the bits of their ids
+//   moe_sort       stable sort of (token, choice) entries by expert: every wave counts and then places its stretch of the
+//                  entries 64 at a time, equal experts found by ballots over the bits of their ids; one workgroup, or for
+//                  more than 4096 entries of up to 64 experts one per 2048 behind a launch that counts
 //   narrow         fp32 products of bf16 rows with up to 64 bf16 weight rows (router logits, gate projections): 16 rows a
 //                  workgroup, its 16 (or 8) waves split K, 16x16x32 products; with a bias, or followed in place by the
 //                  choice of the k largest scores, a wave per row
@@ -202,8 +203,8 @@ __global__ __launch_bounds__(256, 2) void grouped_wide_kernel(const bf16* __rest
 // fragment lie in different banks.
 // Measured, us against the kernel above (random routing and values): 32768 entries of 16 experts, 4096 -> 5376 relu2 1303 /
 // 1654, 5376 -> 4096 rows 1306 / 1682 (1.1 PFLOP/s); 3800 of 8, 4096 -> 2 x 14336 glu 855 / 1007, 14336 -> 4096 combine
-// 450 / 564; 5386 of 8, 4096 -> 2 x 4608 glu 462 / 533, 4608 -> 4096 rows 264 / 284; one product of 8192^3 859 / 1186 (1.28
-// PFLOP/s). With the loads and reads of a stage in front of its products instead of between them 1507 and 1575 us for the first
+// 450 / 564; 5386 of 8, 4096 -> 2 x 4608 glu 462 / 533, 4608 -> 4096 rows 264 / 284; one product of 8192^3 933 / 1023 (1.18
+// PFLOP/s; 859, 1.28, on a card that held its clock better; the library there 808). With the loads and reads of a stage in front of its products instead of between them 1507 and 1575 us for the first
 // two; 32x32x16 products the same way 1568 and 1646.
 namespace ring {
 typedef float f32x4v __attribute__((ext_vector_type(4)));

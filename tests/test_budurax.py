@@ -836,13 +836,14 @@ def test_short_portions_are_scanned_token_by_token():
 
 
 @pytest.mark.gpu
-def test_chunked_scan_of_rates_and_rows_without_bound():
+@pytest.mark.parametrize("P,N", [(64, 32), (72, 144), (8, 256)])
+def test_chunked_scan_of_rates_and_rows_without_bound(P, N):
     """The chunked scan where A_log is past the largest exponent (A = -inf: the state of a token is gone with the next one), and
     with a row whose x is infinite and one whose x is NaN: whatever stands before such a row comes out as it does without it
     (portions that end inside a chunk of 128 and a tile of 32 rows; the same error bound as above)."""
     device = "cuda:0"
     torch.manual_seed(9)
-    Hh, P, N, G, n = 4, 64, 32, 2, 173
+    Hh, G, n = 4, 2, 173
     inner = Hh * P
     xbc = (torch.randn(n, inner + 2 * G * N) / 2).bfloat16()
     proj = torch.randn(n, Hh).bfloat16()

@@ -89,7 +89,7 @@ hipError_t kafka_launch_moe_sort(const float* topk_w, const int* topk_e, int n, 
 hipError_t kafka_launch_grouped_wide(const bf16* X, int64_t ldx, const bf16* Wt, int E, int N, int K,
                                      const int* perm_tok, const float* perm_w, const int* expert_off, int n_ent,
                                      int gather, int epi, bf16* Y, int64_t ldy, float* out, int64_t ldo,
-                                     float glu_limit, float glu_alpha, int bm, hipStream_t st);
+                                     float glu_limit, float glu_alpha, int bm, int64_t xrows, hipStream_t st);
 int kafka_narrow_ok(int N, int K, int64_t xs);
 int kafka_narrow_max_k();
 hipError_t kafka_launch_narrow_linear(const bf16* x, int64_t xs, const bf16* w, const float* bias, int N, int K,
@@ -784,7 +784,7 @@ static void grouped_wide(at::Tensor x, at::Tensor wt, at::Tensor perm_tok, at::T
   }
   CHECK_HIP(kafka_launch_grouped_wide(bptr(x), x.stride(0), bptr(wt), (int)E, (int)N, (int)K, perm_tok.data_ptr<int>(),
                                       perm_w.data_ptr<float>(), expert_off.data_ptr<int>(), (int)n_ent, gather ? 1 : 0,
-                                      (int)epi, yp, ldy, op, ldo, (float)glu_limit, (float)glu_alpha, (int)bm, cur_stream()));
+                                      (int)epi, yp, ldy, op, ldo, (float)glu_limit, (float)glu_alpha, (int)bm, x.size(0), cur_stream()));
 }
 
 static void narrow_args(const at::Tensor& x, const at::Tensor& w) {

@@ -10,14 +10,17 @@
 //                  Epilogues: silu(gate) * up or its clamped form on GLU-interleaved tiles (a wave holds both tiles of a
 //                  pair), relu squared, the weighted combine into fp32 rows, or the weighted rows as they are (in entry
 //                  order; their consumer gathers a token's rows through the sort's inverse, no atomics).
-//   grouped_ring   the same for experts of more rows: 256 x 256 tiles, both operands through a ring in LDS
+//   grouped_ring   the same on 256 x 256 tiles (lower ones for an expert's last rows), both operands through a ring in LDS
 //   moe_sort       stable sort of (token, choice) entries by expert: every wave counts and then places its stretch of the
 //                  entries 64 at a time, equal experts found by ballots over the bits of their ids; one workgroup, or for
 //                  more than 4096 entries of up to 64 experts one per 2048 behind a launch that counts
 //   narrow         fp32 products of bf16 rows with up to 64 bf16 weight rows (router logits, gate projections): 16 rows a
 //                  workgroup, its 16 (or 8) waves split K, 16x16x32 products; with a bias, or followed in place by the
 //                  choice of the k largest scores, a wave per row
+#include <type_traits>
+
 #include "moe_sort.h"
+#include "ring.h"
 
 namespace kafka {
 namespace mw {
@@ -194,44 +197,102 @@ __global__ __launch_bounds__(256, 2) void grouped_wide_kernel(const bf16* __rest
 }
 
 // ---- the same on 256 x 256 tiles through a ring in LDS ---------------------------------------------------------------
-// Four waves of 128 x 128 (one workgroup per CU): an operand byte read from LDS feeds four products instead of the two of
-// the kernel above, and a byte from the cache twice as many. Activations and weights arrive by LDS-DMA, 32 deep, in a ring of
-// five stages: three or four are in flight while one is multiplied (a miss under load takes longer than a stage), one counted
-// wait and one barrier per stage; a wave reads a stage's fragments while it multiplies the one before. 16x16x32 products: the
-// matrix cores alone reach 1.89 PFLOP/s on them at one wave per SIMD, 1.47 on 32x32x16. A weight piece is a whole 1 KB tile of
-// 32 x 16 in lane order; the activations' 16-byte pieces are permuted at the source so that eight neighbouring rows of a
-// fragment lie in different banks.
-// Measured, us against the kernel above (random routing and values): 32768 entries of 16 experts, 4096 -> 5376 relu2 1303 /
-// 1654, 5376 -> 4096 rows 1306 / 1682 (1.1 PFLOP/s); 3800 of 8, 4096 -> 2 x 14336 glu 855 / 1007, 14336 -> 4096 combine
-// 450 / 564; 5386 of 8, 4096 -> 2 x 4608 glu 462 / 533, 4608 -> 4096 rows 264 / 284; one product of 8192^3 933 / 1023 (1.18
-// PFLOP/s; 859, 1.28, on a card that held its clock better; the library there 808). With the loads and reads of a stage in front of its products instead of between them 1507 and 1575 us for the first
-// two; 32x32x16 products the same way 1568 and 1646.
-namespace ring {
-typedef float f32x4v __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void lds_t;
-constexpr int BM = 256, BK = 32, NS = 5, KB = BK / 16;
-constexpr int XB = BM * BK * 2, STAGE = XB + BN * BK * 2;   // bytes
-constexpr int DX = XB / 1024 / 4, DW = BN * BK * 2 / 1024 / 4, DPS = DX + DW;   // 1 KB pieces a wave moves per stage
-constexpr int LGKM0 = 0xC07F;   // s_waitcnt lgkmcnt(0) alone, in a form that the compiler counts too
-
-__device__ __forceinline__ int xslot(int row, int c) { return c ^ ((row >> 1) & 3); }
-
-// c += a b in an accumulation register: left to itself the compiler moves sums between the two register files in the loop.
-// (Operands come from LDS, so their waits are the compiler's; two products on one sum are 64 products apart.)
-__device__ __forceinline__ void mfma16(f32x4v& c, bf16x8 a, bf16x8 b) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-}
-
-template <bool B>
-struct Full {
-  static constexpr bool value = B;
+// Four waves of 128 x 128 (ring.h; one workgroup per CU): an operand byte read from LDS feeds four products instead of the two of
+// the kernel above, and a byte from the cache twice as many. Results
+// leave in 16-byte pieces. An expert's last rows go on a tile of 64 or 128 rows where they fit one (the weights' way is then what it
+// takes, a third of a whole tile). What bounds it: the card lowers its clock to 1.9 - 2.0 GHz under these products, and the last
+// round of the chip.
+// Measured, us, before (stages of 32 for both operands, 64-bit addresses, whole tiles only, 2-byte stores) / now (random routing
+// and values, rows of 128 bytes a piece): 32768 entries of 16 experts, 4096 -> 5376 relu2 1325 / 1260, 5376 -> 4096 rows 1295 /
+// 1147; 3800 of 8, 4096 -> 2 x 14336 glu 887 / 847, 14336 -> 4096 rows 660 / 606; 5386 of 8, 4096 -> 2 x 4608 glu 423 / 404, 4608 -> 4096
+// rows 223 / 211. Activations in 64-byte pieces alone (half a cache line: twice the lines asked of the cache) 1303 and 1254 for the first
+// two. A workgroup that goes on to its next tile with the ring kept full gained nothing (the clock), its branches in the loop cost 5 %.
+struct RingArgs {
+  const bf16* X;
+  int64_t ldx;
+  const bf16x8* Wt;
+  int N, K;
+  const int* perm_tok;
+  const float* perm_w;
+  bf16* Y;
+  int64_t ldy;
+  float* out;
+  int64_t ldo;
+  float glu_limit, glu_alpha;
 };
 
-template <int N>
-__device__ __forceinline__ void vmcnt() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+// rows (at most 32 MT) entries from seg0 on of expert e, 256 columns from 256 nt on
+template <int MT, bool GATHER, int EPI>
+__device__ __forceinline__ void ring_tile(const RingArgs& A, char* smem, int e, int seg0, int rows, int nt) {
+  using R = ring::Ring<MT, 8, EPI != EPI_COMBINE>;   // (sums added to memory: lanes along the columns of a row)
+  const int N = A.N, K = A.K;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, q = lane >> 4;
+  const int nb = nt * 8 + 4 * (w & 1);             // this wave's first 32-column tile (N is a multiple of 128)
+  unsigned xo[2 * R::DX], wo[R::DW];
+#pragma unroll
+  for (int u = 0; u < 2 * R::DX; ++u) {
+    const int row = R::xrow(w, u, lane), m = min(row, rows - 1);   // rows past the segment reload a valid row, never stored
+    const unsigned at = GATHER ? (unsigned)A.perm_tok[seg0 + m] : (unsigned)m;
+    xo[u] = at * (unsigned)(A.ldx * 2) + R::xbyte(row, lane);
+  }
+#pragma unroll
+  for (int u = 0; u < R::DW; ++u)                  // (tiles past N reload the last, never stored)
+    wo[u] = (unsigned)(min(nt * 8 + R::wtile(w, u), (N >> 5) - 1) * (K >> 4) + R::wblock(w, u)) * 1024u;
+  ring::f32x4v acc[MT][8];
+#pragma unroll
+  for (int a = 0; a < MT; ++a)
+#pragma unroll
+    for (int b = 0; b < 8; ++b) acc[a][b] = ring::f32x4v{0.f, 0.f, 0.f, 0.f};
+  R::multiply(acc, smem, ring::buffer(GATHER ? A.X : A.X + (int64_t)seg0 * A.ldx), xo,
+              ring::buffer(A.Wt + (int64_t)e * (N >> 5) * (K >> 4) * 64), R::wlane(lane), wo, K / ring::BK, lane, w);
+  if (nb >= (N >> 5)) return;
+  if constexpr (EPI == EPI_COMBINE) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = 16 * (MT * (w >> 1) + mt) + 4 * q + i;
+        if (m >= rows) continue;
+        const float pw = A.perm_w[seg0 + m];
+        float* o = A.out + (int64_t)A.perm_tok[seg0 + m] * A.ldo + nb * 32 + r;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) atomicAdd(o + 16 * j, pw * acc[mt][j][i]);
+      }
+  } else {
+    // this lane: row 16 mt + r, columns 8 q .. of every tile
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int m = 16 * (MT * (w >> 1) + mt) + r;
+      if (m >= rows) continue;
+      bf16* y = A.Y + (int64_t)(seg0 + m) * A.ldy + 8 * q;
+      const float pw = EPI == EPI_ROWS ? A.perm_w[seg0 + m] : 1.0f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if (EPI == EPI_GLU && (t & 1)) continue;   // tiles of 32: gate, up, gate, up
+        bf16x8 o;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float v = acc[mt][2 * t + (i >> 2)][i & 3];
+          if constexpr (EPI == EPI_ROWS) {
+            o[i] = (bf16)(pw * v);
+          } else if constexpr (EPI == EPI_RELU2) {
+            const float a = fmaxf(v, 0.f);
+            o[i] = (bf16)(a * a);
+          } else {
+            float g = v, u = acc[mt][(2 * t + 2 + (i >> 2)) & 7][i & 3], al = 1.0f;
+            if (A.glu_limit > 0.f) {   // (uniform) the clamped form
+              g = fminf(g, A.glu_limit);
+              u = fminf(fmaxf(u, -A.glu_limit), A.glu_limit) + 1.0f;
+              al = A.glu_alpha;
+            }
+            o[i] = (bf16)(g / (1.0f + __expf(-al * g)) * u);
+          }
+        }
+        *reinterpret_cast<bf16x8*>(y + (EPI == EPI_GLU ? (nb + t) >> 1 : nb + t) * 32) = o;
+      }
+    }
+  }
 }
-}  // namespace ring
 
 template <bool GATHER, int EPI>
 __global__ __launch_bounds__(256, 1) void grouped_ring_kernel(const bf16* __restrict__ X, int64_t ldx,
@@ -242,159 +303,17 @@ __global__ __launch_bounds__(256, 1) void grouped_ring_kernel(const bf16* __rest
                                                               bf16* __restrict__ Y, int64_t ldy,
                                                               float* __restrict__ out, int64_t ldo, float glu_limit,
                                                               float glu_alpha) {
-  using namespace ring;
-  __shared__ __attribute__((aligned(1024))) char smem[NS * STAGE];
+  constexpr int BM = ring::Ring<8, 8, true>::BM;
+  __shared__ __attribute__((aligned(1024))) char smem[ring::Ring<8, 8, true>::LDS];
   int e, rt, nt;
-  if (!find_item(expert_off, E, (N + BN - 1) / BN, ring::BM, e, rt, nt)) return;   // (uniform)
-  const int seg0 = expert_off[e] + rt * ring::BM, rows = min(ring::BM, expert_off[e + 1] - seg0);
-  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, q = lane >> 4;
-  const int wr = w >> 1, wc = w & 1;
-  const int nb = nt * 8 + 4 * wc;                  // this wave's first 32-column tile (N is a multiple of 128)
-  const int K16 = K >> 4, nst = K / ring::BK;
-  const bf16* xsrc[DX];
-  const bf16x8* wsrc[DW];
-#pragma unroll
-  for (int u = 0; u < DX; ++u) {
-    const int row = 16 * (DX * w + u) + (lane >> 2);
-    const int ent = seg0 + min(row, rows - 1);     // rows past the segment reload a valid row, never stored
-    xsrc[u] = X + (GATHER ? (int64_t)perm_tok[ent] : (int64_t)ent) * ldx + 8 * xslot(row, lane & 3);
-  }
-#pragma unroll
-  for (int u = 0; u < DW; ++u) {
-    const int j = DW * w + u, t = min(nt * 8 + j / KB, (N >> 5) - 1);   // (tiles past N reload the last, never stored)
-    wsrc[u] = Wt + (((int64_t)e * (N >> 5) + t) * K16 + j % KB) * 64 + lane;
-  }
-  auto issue_piece = [&](int s, int slot, int u) {
-    char* base = smem + slot * STAGE;
-    if (u < DX)
-      __builtin_amdgcn_global_load_lds(xsrc[u] + (int64_t)s * ring::BK, (lds_t*)(base + (DX * w + u) * 1024), 16, 0, 0);
-    else
-      __builtin_amdgcn_global_load_lds(wsrc[u - DX] + (int64_t)s * KB * 64,
-                                       (lds_t*)(base + XB + (DW * w + u - DX) * 1024), 16, 0, 0);
-  };
-  auto issue = [&](int s, int slot) {
-#pragma unroll
-    for (int u = 0; u < DPS; ++u) issue_piece(s, slot, u);
-  };
-  f32x4v acc[8][8];
-#pragma unroll
-  for (int a = 0; a < 8; ++a)
-#pragma unroll
-    for (int b = 0; b < 8; ++b) acc[a][b] = f32x4v{0.f, 0.f, 0.f, 0.f};
-  // where this lane's fragments lie in a stage: rows 16 i + r, 8-deep piece q; columns 16 j + r, piece q of tile j / 2
-  const int xa = (128 * wr + r) * (2 * ring::BK) + 16 * xslot(r, q);   // (row bits above 2 leave the slot alone)
-  const int wa = XB + (4 * wc * KB + (q >> 1)) * 1024 + ((q & 1) * 32 + r) * 16;
-  auto read_pair = [&](bf16x8& a, bf16x8& b, int slot, int i) {
-    const char* base = smem + slot * STAGE;
-    a = *reinterpret_cast<const bf16x8*>(base + xa + i * 16 * 2 * ring::BK);
-    b = *reinterpret_cast<const bf16x8*>(base + wa + (i >> 1) * KB * 1024 + (i & 1) * 256);
-  };
-  // stage s has been read by this wave; stage s + 1 arrives, the ring takes stage s + NS in stage s's place
-  auto turn = [&](int s) {
-    const int later = min(NS - 2, nst - 2 - s);    // stages behind s + 1 that may be in flight
-    if (later >= 3) vmcnt<3 * DPS>();
-    else if (later == 2) vmcnt<2 * DPS>();
-    else if (later == 1) vmcnt<DPS>();
-    else vmcnt<0>();
-    asm volatile("s_barrier" ::: "memory");
-  };
-  bf16x8 a0[8], b0[8], a1[8], b1[8];
-  // (K is a multiple of 128: an even number of stages, at least NS - 1)
-#pragma unroll
-  for (int s = 0; s < NS - 1; ++s) issue(s, s);
-  turn(-1);
-  if (NS - 1 < nst) issue(NS - 1, NS - 1);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) read_pair(a0[i], b0[i], 0, i);
-  int slot = 0;
-  // Between the eight groups of eight products go the next stage's reads and the ring's next pieces, one of each: a wave
-  // issues in order, and all of them in front of the products would leave the matrix core waiting for the load path.
-  // ``full``: the ring stays full (s + NS < nst), no conditions in the way.
-  auto step = [&](auto full, int s, const bf16x8(&a)[8], const bf16x8(&b)[8], bf16x8(&an)[8], bf16x8(&bn)[8]) {
-    const int next = slot == NS - 1 ? 0 : slot + 1;
-    __builtin_amdgcn_s_waitcnt(LGKM0);             // (this stage's fragments: requested a stage ago)
-    const bool more = full.value || s + 1 < nst, load = full.value;
-    if constexpr (full.value) {
-      vmcnt<(NS - 2) * DPS>();
-      asm volatile("s_barrier" ::: "memory");
-    } else {
-      if (more) turn(s);
-      if (s + NS < nst) issue(s + NS, slot);
-    }
-    const char* nx = smem + next * STAGE;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (load) issue_piece(s + NS, slot, i);
-      __builtin_amdgcn_sched_barrier(0);
-      mfma16(acc[i][0], a[i], b[0]);
-      mfma16(acc[i][1], a[i], b[1]);
-      __builtin_amdgcn_sched_barrier(0);
-      if (more) an[i] = *reinterpret_cast<const bf16x8*>(nx + xa + i * 16 * 2 * ring::BK);
-      __builtin_amdgcn_sched_barrier(0);
-      mfma16(acc[i][2], a[i], b[2]);
-      mfma16(acc[i][3], a[i], b[3]);
-      __builtin_amdgcn_sched_barrier(0);
-      if (more) bn[i] = *reinterpret_cast<const bf16x8*>(nx + wa + (i >> 1) * KB * 1024 + (i & 1) * 256);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 4; j < 8; ++j) mfma16(acc[i][j], a[i], b[j]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    slot = next;
-  };
-  static_assert(DPS == 8, "a piece per group");
-  int s = 0;
-  for (; s + 1 + NS < nst; s += 2) {
-    step(Full<true>(), s, a0, b0, a1, b1);
-    step(Full<true>(), s + 1, a1, b1, a0, b0);
-  }
-  for (; s < nst; s += 2) {
-    step(Full<false>(), s, a0, b0, a1, b1);
-    step(Full<false>(), s + 1, a1, b1, a0, b0);
-  }
-  // the last products' results are complete before anything reads them behind a branch
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_nop 15");
-  __builtin_amdgcn_sched_barrier(0);
-  if (nb >= (N >> 5)) return;
-#pragma unroll
-  for (int mt = 0; mt < 8; ++mt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = 128 * wr + mt * 16 + 4 * q + i;
-      if (m >= rows) continue;
-      const int ent = seg0 + m;
-      if constexpr (EPI == EPI_COMBINE || EPI == EPI_ROWS) {
-        const float pw = perm_w[ent];
-        float* o = EPI == EPI_COMBINE ? out + (int64_t)perm_tok[ent] * ldo + nb * 32 + r : nullptr;
-        bf16* y = EPI == EPI_ROWS ? Y + (int64_t)ent * ldy + nb * 32 + r : nullptr;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          if constexpr (EPI == EPI_COMBINE) atomicAdd(o + 16 * j, pw * acc[mt][j][i]);
-          else y[16 * j] = (bf16)(pw * acc[mt][j][i]);
-        }
-      } else if constexpr (EPI == EPI_RELU2) {
-        bf16* y = Y + (int64_t)ent * ldy + nb * 32 + r;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float a = fmaxf(acc[mt][j][i], 0.f);
-          y[16 * j] = (bf16)(a * a);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          if (j & 2) continue;                     // tiles of 32: gate, up, gate, up
-          float g = acc[mt][j][i], u = acc[mt][j + 2][i], al = 1.0f;
-          if (glu_limit > 0.f) {   // (uniform) the clamped form
-            g = fminf(g, glu_limit);
-            u = fminf(fmaxf(u, -glu_limit), glu_limit) + 1.0f;
-            al = glu_alpha;
-          }
-          Y[(int64_t)ent * ldy + ((nb + (j >> 1)) >> 1) * 32 + 16 * (j & 1) + r] =
-              (bf16)(g / (1.0f + __expf(-al * g)) * u);
-        }
-      }
-    }
+  if (!find_item(expert_off, E, (N + 255) / 256, BM, e, rt, nt)) return;   // (uniform)
+  const int seg0 = expert_off[e] + rt * BM, rows = min(BM, expert_off[e + 1] - seg0);
+  const RingArgs A{X, ldx, Wt, N, K, perm_tok, perm_w, Y, ldy, out, ldo, glu_limit, glu_alpha};
+  // an expert's last rows on a lower tile where they fit one: the weights' way is then what it takes, a third of a whole tile
+  // (sums added to memory take as long either way)
+  if (rows > 128 || EPI == EPI_COMBINE) ring_tile<8, GATHER, EPI>(A, smem, e, seg0, rows, nt);
+  else if (rows > 64) ring_tile<4, GATHER, EPI>(A, smem, e, seg0, rows, nt);
+  else ring_tile<2, GATHER, EPI>(A, smem, e, seg0, rows, nt);
 }
 
 // ---- stable sort by expert --------------------------------------------------------------------------------------------
@@ -706,18 +625,26 @@ hipError_t kafka_launch_moe_sort(const float* topk_w, const int* topk_e, int n, 
 hipError_t kafka_launch_grouped_wide(const bf16* X, int64_t ldx, const bf16* Wt, int E, int N, int K,
                                      const int* perm_tok, const float* perm_w, const int* expert_off, int n_ent,
                                      int gather, int epi, bf16* Y, int64_t ldy, float* out, int64_t ldo,
-                                     float glu_limit, float glu_alpha, int bm, hipStream_t st) {
+                                     float glu_limit, float glu_alpha, int bm, int64_t xrows, hipStream_t st) {
   if (n_ent < 1 || E < 1) return hipSuccess;
+  // what the ring kernel addresses with 32 bits (all rows of X where they are gathered, a tile's otherwise, and an expert's weights)
+  // and stores in 16-byte pieces
+  const bool ring_ok = N % 128 == 0 && (gather ? xrows : 256) * ldx * 2 < (int64_t)0xffff0000 &&
+                       (int64_t)N * K * 2 < (int64_t)0xffff0000 &&
+                       (epi == EPI_COMBINE || (ldy % 8 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0));
   if (bm == 0) {
-    // Which tiles, from the mean rows of an expert. A round of the chip is 256 tiles of 256 x 256 or 512 of 128 x 256, the same
-    // products; the ring kernel does them 1.3 times as fast, but in whole rounds, the other one's last round thins out
-    // (a quarter of one on average).
+    // Which tiles, from the mean rows of an expert. Up to 128 rows the ring kernel's low tiles (us, 128-row kernel / ring, 40 - 100 rows
+    // of each of 8 experts: 4096 -> 2 x 4608 148 - 154 / 142 - 158, 4608 -> 4096 79 - 86 / 68 - 82, 2048 -> 2 x 2304 39 / 30,
+    // 2304 -> 2048 42 / 26). Beyond, by rounds: one is 256 tiles of 256 x 256 or 512 of 128 x 256, the same products; the ring
+    // kernel does them 1.4 times as fast, but in whole rounds, the other one's last round thins out (a quarter of one on
+    // average): 2048 -> 2 x 2304 280 rows 63 / 99, 600 rows 100 / 100, 1300 rows 218 / 208; 4096 -> 2 x 14336 140 rows 504 / 446, 600 rows 1143 / 1025.
     const int64_t r = ((int64_t)n_ent + E - 1) / E, ct = (N + BN - 1) / BN * (int64_t)E;
-    const double ring_rounds = (double)(((r + 255) / 256 * ct + 255) / 256) / 1.3;
+    const double ring_rounds = (double)(((r + 255) / 256 * ct + 255) / 256) / 1.4;
     const double wide_rounds = (double)((r + 127) / 128 * ct) / 512 + 0.25;
-    bm = N % 128 == 0 && ring_rounds < wide_rounds ? 256 : 128;
+    bm = ring_ok && (r <= 128 || ring_rounds < wide_rounds) ? 256 : 128;
   }
   if ((bm != 128 && bm != 256) || (bm == 256 && N % 128)) return hipErrorInvalidValue;
+  if (bm == 256 && !ring_ok) bm = 128;
   if (N % 64 || K % (2 * BK) || N < 64 || K < 2 * BK || epi < 0 || epi > 3 || (epi == EPI_COMBINE) != (out != nullptr) ||
       (epi != EPI_COMBINE) != (Y != nullptr))
     return hipErrorInvalidValue;

@@ -1043,6 +1043,14 @@ def test_wide_expert_products_on_256_row_tiles(rows, N, K):
         assert same(ops.grouped_wide(x, gt, r, "glu", True, tile=128, **kw), ref)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,N,K", [((64, 65, 128, 129, 1), 256, 128), ((320, 321, 384, 385), 384, 256), ((63, 127), 640, 384)])
+def test_wide_expert_products_on_low_row_tiles(rows, N, K):
+    """An expert's last rows on tiles of 64 and 128 rows: at, and one past, the height of each, alone and behind a whole tile;
+    four, eight and twelve stages of the ring (it holds four). Bounds as above."""
+    test_wide_expert_products_on_256_row_tiles(rows, N, K)
+
+
 def test_items_that_share_keys():
     """Which of a step's attention items count for the kernel that shares keys among eight of them: all of prompt portions, those of
     more than one token beside decoded ones (160 of one token and 2 portions of 5 items of 8: 10), none where items of one token

@@ -264,13 +264,13 @@ class FurapelLM:
 
     def _lin(self, x, w, wt=None, slabs: bool = False):
         """x @ w^T: the weight-streaming kernel for decode-sized steps when the weight has a tiled copy, else
-        hipBLASLt. ``slabs``: the caller takes the split-K slabs [S, T, N] as they are."""
+        the tile kernel or the library (ops.linear_long). ``slabs``: the caller takes the split-K slabs [S, T, N] as they are."""
         M = x.shape[0]
         if self.stream and wt is not None and 0 < M <= self.stream_max_m and \
                 ops.stream_plan(M, w.shape[0], w.shape[1]) is not None:
             y = ops.linear_stream(x, wt)
             return ops.slab_reduce(y) if ops.is_slab(y) and not slabs else y
-        return ops.linear_dense(x, w)
+        return ops.linear_long(x, w, wt if self.stream else None, slabs)
 
     def weight_bytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self._tensors)

@@ -6,9 +6,9 @@ Per layer (SURVEY.md §3.2 "Target equivalent"):
     -> fused_add_rmsnorm -> gate_up GEMM (column-parallel) -> silu_mul (HIP) -> down GEMM (row-parallel)
     -> [TP all-reduce]                                     (Mixtral: router -> expert MLPs, models/moe.py)
 Decode-sized steps (T <= 128) run every projection on the weight-streaming MFMA kernel (``ops/csrc/wstream_gemm.hip``,
-wave-tiled weight copies, SwiGLU fused into gate_up; the grouped variant for Mixtral's experts); 129..256-row mixed
-steps run qkv / o / down on the skinny MFMA GEMM (``ops/csrc/skinny_gemm.hip``, SKINNY below); other prefill-sized
-steps use hipBLASLt through ``torch.nn.functional.linear`` (bf16, fp32 accumulate). Norm / RoPE / attention / sampling run
+wave-tiled weight copies, SwiGLU fused into gate_up; the grouped variant for Mixtral's experts); longer
+steps on the tile kernel (``ops/csrc/tile_gemm.hip``, the same weights; SwiGLU in its epilogue), shapes it does not take on
+hipBLASLt through ``torch.nn.functional.linear`` (bf16, fp32 accumulate). Norm / RoPE / attention / sampling run
 in the hand-written kernels of ``ops/csrc``.
 
 Weights are stored HF-style ``[out, in]`` so safetensors checkpoints load without transposes; random init (seeded,
@@ -37,17 +37,17 @@ from kafka_llm_service_amd.parallel import state as pstate
 TP_OVERLAP = os.environ.get("KAFKA_TP_OVERLAP", "0") == "1"
 
 # Projections of 129..256-row steps (decode + a new turn's prefill) that run on the skinny MFMA GEMM
-# (ops.linear_skinny, csrc/skinny_gemm.hip) instead of hipBLASLt: env KAFKA_SKINNY, a comma list of qkv / o / down
-# ("" = none; "+" also separates). gate_up stays on hipBLASLt (faster there). Same-box A/B, 2 interleaved rounds:
-# 7,857 (none) -> 7,924 tok/s (o+down or all three), profiles/r03/skinny_gemm/bench_ab_wired.jsonl.
+# (ops.linear_skinny, csrc/skinny_gemm.hip) instead of the tile kernel: env KAFKA_SKINNY, a comma list of qkv / o / down / gate_up
+# ("" = none, the default; "+" also separates). us at 200 rows, weights from memory, skinny / tile kernel: qkv 23.4 / 22.4, o 16.4 /
+# 16.0, down 38.4 / 37.4, gate_up 79.9 / 60.2.
 # Prefill-sized TP seams whose message exceeds the custom all-reduce's buffer (RCCL): the row-parallel GEMM and the
 # all-reduce are pipelined over row blocks of at least PIPE_ROWS tokens, at most PIPE_CHUNKS blocks
 # (comm.pipelined_linear_all_reduce; env KAFKA_TP_PIPE_CHUNKS, 1 = off). At Llama-3-70B TP = 8 a 2k-token chunk has
 # 160 such seams of 32 MiB each; with the pipeline only the last block's all-reduce is left exposed.
 PIPE_CHUNKS = max(1, int(os.environ.get("KAFKA_TP_PIPE_CHUNKS", "4")))
 PIPE_ROWS = 256
-SKINNY = frozenset(p for p in os.environ.get("KAFKA_SKINNY", "qkv,o,down").replace("+", ",").split(",")
-                   if p in ("qkv", "o", "down", "gate_up"))  # gate_up: fused SwiGLU epilogue (A/B, not default)
+SKINNY = frozenset(p for p in os.environ.get("KAFKA_SKINNY", "").replace("+", ",").split(",")
+                   if p in ("qkv", "o", "down", "gate_up"))
 # Fused decode layer (forward -> _forward_fused; env KAFKA_FUSED_DECODE=1): 6 launches per layer instead of 9 —
 # deferred RMSNorm and RoPE + KV write inside the streaming GEMMs' split-K finishers. Correct (fp32-reference and
 # buffer-reuse tests) but OFF by default: each finisher is one workgroup reducing its column block's slabs at the
@@ -202,15 +202,16 @@ class TransformerLM:
 
     def _linear(self, x: torch.Tensor, w: torch.Tensor, wt: torch.Tensor | None, max_splits: int = 8,
                 kind: str = ""):
-        """x @ w^T: the weight-streaming kernel for decode-sized x (bf16 or a split-K slab out), the skinny MFMA GEMM
-        for 129..256 rows of the projections in SKINNY, else hipBLASLt."""
+        """x @ w^T: the weight-streaming kernel for decode-sized x (bf16 or a split-K slab out), else the tile kernel
+        (the same) or the library; 129..256 rows of the projections in SKINNY on the skinny MFMA GEMM."""
         M = x.shape[0]
         if self.stream and wt is not None:
             if 0 < M <= self.stream_max_m:
                 return ops.linear_stream(x, wt, max_splits)
             if kind in SKINNY and ops.skinny_plan(M, wt.shape[0] * 32, x.shape[1], max_splits):
                 return ops.linear_skinny(x, wt, max_splits)
-        return ops.linear_dense(x, self._dense(w, wt))
+        # (under TP slabs of more rows would be reduced to bf16 ahead of the collective)
+        return ops.linear_long(x, w, wt if self.stream else None, slabs=max_splits > 1 and (self.tp == 1 or M <= 256))
 
     @staticmethod
     def _dense(w: torch.Tensor | None, wt: torch.Tensor | None, glu: bool = False) -> torch.Tensor:
@@ -277,7 +278,9 @@ class TransformerLM:
                 if ops.is_slab(a):
                     a = ops.silu_mul(a)
             else:
-                a = ops.silu_mul(F.linear(x, self._dense(lw.gate_up, lw.gate_up_t, bool(lw.glu))))
+                a = ops.linear_glu_long(x, lw.gate_up_t) if self.stream and lw.glu else None
+                if a is None:
+                    a = ops.silu_mul(F.linear(x, self._dense(lw.gate_up, lw.gate_up_t, bool(lw.glu))))
             if tp and self._can_overlap(T, lw.down_t) and i + 1 < len(self.layers):
                 # the next layer's input RMSNorm is the seam's normalisation: delta is consumed here
                 self._overlapped_seam(a, lw.down_t, residual, self.layers[i + 1].input_norm, eps, x)

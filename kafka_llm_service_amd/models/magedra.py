@@ -285,13 +285,15 @@ class MagedraLM:
 
     def _lin(self, x, w, wt=None, bias=None):
         """x @ w^T (+ bias): the weight-streaming kernel for decode-sized steps when the weight has a tiled copy, else
-        hipBLASLt."""
+        the tile kernel or the library (ops.linear_long; a bias is the library's, added before the rounding)."""
         M = x.shape[0]
         if self.stream and wt is not None and 0 < M <= self.stream_max_m and \
                 ops.stream_plan(M, w.shape[0], w.shape[1]) is not None:
             y = ops.linear_stream(x, wt)
             y = ops.slab_reduce(y) if ops.is_slab(y) else y
             return y if bias is None else y.add_(bias)
+        if self.stream and wt is not None and bias is None and x.is_cuda:
+            return ops.linear_long(x, w, wt)
         return F.linear(x, w, bias)
 
     def weight_bytes(self) -> int:

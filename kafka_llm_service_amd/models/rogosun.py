@@ -301,11 +301,11 @@ class RogosunLM:
 
     def _lin(self, x, w, wt=None, slabs: bool = False):
         """x @ w^T: the weight-streaming kernel for decode-sized steps when the weight has a tiled copy, else
-        hipBLASLt. ``slabs``: the caller takes the split-K slabs [S, T, N] as they are."""
+        the tile kernel or the library (ops.linear_long). ``slabs``: the caller takes the split-K slabs [S, T, N] as they are."""
         if self._streams(x.shape[0], w, wt):
             y = ops.linear_stream(x, wt)
             return ops.slab_reduce(y) if ops.is_slab(y) and not slabs else y
-        return ops.linear_dense(x, w)
+        return ops.linear_long(x, w, wt if self.stream else None, slabs)
 
     def weight_bytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self._tensors)
@@ -547,8 +547,11 @@ class RogosunLM:
         if self._streams(T, lw.sh_gu, getattr(lw, "sh_gu_t", None)):
             a = ops.linear_glu(h, lw.sh_gu_t)
         else:
-            a = torch.empty(T, z["shared_ff"], dtype=dt, device=dev)
-            hops.silu_mul(F.linear(h, lw.sh_gu), a)
+            wt = getattr(lw, "sh_gu_t", None)
+            a = ops.linear_glu_long(h, wt) if self.stream and wt is not None else None
+            if a is None:
+                a = torch.empty(T, z["shared_ff"], dtype=dt, device=dev)
+                hops.silu_mul(F.linear(h, lw.sh_gu), a)
         return out, self._lin(a, lw.sh_down, getattr(lw, "sh_down_t", None))
 
 

@@ -12,6 +12,7 @@ Kernel inventory:
 from __future__ import annotations
 
 import os
+from functools import lru_cache
 
 import numpy as np
 import torch
@@ -302,6 +303,98 @@ def skinny_plan(M: int, N: int, K: int, max_splits: int = 8) -> int:
     while s * 2 <= max_splits and nx * s < 192 and K % (64 * s * 2) == 0 and K // (s * 2) >= 256:
         s *= 2
     return s
+
+
+# ---- dense products of long steps on wave-tiled weights (csrc/tile_gemm.hip) -------------------------------------------
+# (16-row parts, 16-column parts) of a wave's tile, 2 x 2 waves a workgroup -> us: of a launch, of a round of 256 workgroups, of 64 of K
+# in it, and of a MB/us of what is written, over 4.5. Fitted to 6200 timings (19 shapes of width 2048 and 4096, 136 - 4099 rows,
+# every tile, one to eight splits; weights from memory): a time is off by 5 % (the worst by a third), the tile and split that the
+# figures pick by 0.5 % on average from the best.
+TILES = {(8, 8): (3.3, 7.6, 1.24, 0.64), (8, 6): (3.7, 4.6, 0.96, 0.82), (6, 8): (2.9, 7.5, 0.94, 0.55), (6, 6): (2.9, 5.9, 0.75, 0.73), (8, 4): (2.8, 3.6, 0.71, 1.00), (4, 8): (3.1, 4.4, 0.76, 0.81), (4, 6): (2.8, 3.9, 0.61, 0.98), (4, 4): (4.9, 0.2, 0.45, 1.01)}
+TILE_SPLITS = (1, 2, 4, 8)      # what the consumers of slabs load with all slabs in flight
+TILE_SLAB_BYTES = 1 << 28
+TILE_LIBRARY_N, TILE_MAX_M = 24576, 2560
+
+
+@lru_cache(maxsize=4096)
+def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) -> tuple[int, int, int] | None:
+    """(16-row parts, 16-column parts, splits) of the tile kernel for x [M, K] @ W^T [N, K], None where it does not take the shape or
+    the library is as fast. ``form``: "slabs" (the consumer sums the split-K slabs as it loads them), "bf16" (slabs go
+    through slab_reduce, a launch) or "glu" (silu(gate) * up, in the epilogue or from slabs). ``library``: there is a row-major weight for it.
+
+    Against the library (us, library / this kernel): 450 rows of 14336 -> 4096 89 / 55, 2048 rows 202 / 178; 2048 rows of 4096 -> 18560 350 / 277,
+    200 rows 57 / 45; 900 rows of 2048 -> 9344 45 / 36; 450 rows of 2048 -> 2048 19 / 11; over all timed shapes 13 % less time with slabs,
+    9 % as bf16. The library's: very wide outputs of 257 - 1024 rows (28672 columns: 320 rows 74 / 78, 640 135 / 149); beyond
+    them, where its 256 x 256 tiles (1.42 us a round and 64 of K) fill their rounds (28672: 1536 rows 264 / 293, 4099 722 / 774; 2048 -> 7168,
+    2048 rows 49 / 62), which ragged columns (no multiple of 256) do not (10816: 2048 rows 164 / 151); and beyond 2560 rows: the
+    longer the card is busy the lower its clock, and the library takes less power (a step of 4099 rows 6387 / 6587, of 8192 its products
+    2935 / 3276, of 2750 the same)."""
+    if M < 1 or N % 32 or N < 32 or K % 64 or K < 128 or N * K * 2 > 0xffff0000 or (form == "glu" and N % 64):
+        return None
+    if library and (M > TILE_MAX_M or form == "bf16" and N > TILE_LIBRARY_N and 256 < M <= 1024):
+        return None
+    best = None
+    for (mt, nt), (launch, rnd, unit, out) in TILES.items():
+        if form == "glu" and nt % 4:
+            continue                # (a wave holds whole gate, up pairs)
+        items = -(-M // (32 * mt)) * -(-N // (32 * nt))
+        for s in TILE_SPLITS:
+            if K // 64 < 2 * s or (s > 1 and 4 * s * M * N > TILE_SLAB_BYTES):
+                break
+            mb = M * N / 4.5e6
+            t = launch + -(-items * s // 256) * (rnd + unit * (K // 64) / s) + out * mb * (4 * s if s > 1 else 2)
+            if s > 1:               # the slabs' way back in, beside that of a bf16 output; a launch of its own but for "slabs"
+                t += mb * (4 * s - 2) if form == "slabs" else 6 + mb * (4 * s + 2)
+            if best is None or t < best[0]:
+                best = (t, (mt, nt, s))
+    if library and M > 1024:
+        rows = M // DENSE_BLOCK * DENSE_BLOCK if dense_cut(M, N, K) else M
+        lib = 4 + -(-(-(-rows // 256) * -(-N // 256)) // 256) * 1.42 * (K // 64) + (20 if rows < M else 0)
+        if form == "glu":           # (the activation's launch and its way to memory and back)
+            lib += 5 + 3 * M * N / 4.5e6
+        if best[0] > lib * (1.25 if N % 256 else 0.95):
+            return None
+    return best[1]
+
+
+def tile_ok(x: torch.Tensor, wt: torch.Tensor | None) -> bool:
+    """Whether the tile kernel takes these operands (its rows in 16-byte pieces, a row tile within 4 GB)."""
+    return wt is not None and wt.is_cuda and _gpu(x) and x.dtype == torch.bfloat16 and wt.dtype == torch.bfloat16 and x.dim() == 2 and \
+        wt.dim() == 4 and x.shape[0] > 0 and x.shape[1] == wt.shape[1] * 16 and x.stride(1) == 1 and x.stride(0) >= x.shape[1] and \
+        x.stride(0) % 8 == 0 and x.stride(0) < 1 << 22 and x.data_ptr() % 16 == 0 and wt.is_contiguous()
+
+
+def linear_tile(x: torch.Tensor, wt: torch.Tensor, plan: tuple[int, int, int], glu: bool = False) -> torch.Tensor:
+    """x @ W^T from the wave-tiled weight: bf16 [M, N] for a plan of one split (``glu``: W tiled with glu=True, silu(gate) * up
+    [M, N / 2]), else fp32 slabs [S, M, N] (gate | up order)."""
+    M, N, (mt, nt, s) = x.shape[0], wt.shape[0] * 32, plan
+    if s == 1:
+        y = torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
+        ext().tile_gemm(x, wt, y, None, mt, nt, 1, glu)
+        return y
+    p = torch.empty(s, M, N, dtype=torch.float32, device=x.device)
+    ext().tile_gemm(x, wt, None, p, mt, nt, s, glu)
+    return p
+
+
+def linear_long(x: torch.Tensor, w: torch.Tensor | None, wt: torch.Tensor | None, slabs: bool = False) -> torch.Tensor:
+    """x @ w^T of a long step: on the tile kernel where the weight has a tiled copy ``wt`` (or is only that) and the plan says so, else
+    the library. bf16, or with ``slabs`` maybe the split-K slabs (is_slab)."""
+    if tile_ok(x, wt):
+        plan = tile_plan(x.shape[0], wt.shape[0] * 32, x.shape[1], "slabs" if slabs else "bf16", w is not None)
+        if plan is not None:
+            y = linear_tile(x, wt, plan)
+            return y if slabs or plan[2] == 1 else slab_reduce(y)
+    return linear_dense(x, w if w is not None else untile_weight(wt))
+
+
+def linear_glu_long(x: torch.Tensor, wt: torch.Tensor) -> torch.Tensor | None:
+    """silu(x @ Wg^T) * (x @ Wu^T) of a long step from GLU-tiled weights, None where the tile kernel does not take it."""
+    plan = tile_plan(x.shape[0], wt.shape[0] * 32, x.shape[1], "glu") if tile_ok(x, wt) else None
+    if plan is None:
+        return None
+    y = linear_tile(x, wt, plan, glu=True)
+    return y if plan[2] == 1 else silu_mul(y)
 
 
 def linear_skinny(x: torch.Tensor, wt: torch.Tensor, max_splits: int = 8, glu: bool = False) -> torch.Tensor:

@@ -118,6 +118,8 @@ hipError_t kafka_launch_ep_recv_route(const bf16* img, int ep, int C, int MR, in
                                       float* perm_w, int* expert_off, int* tile_off, hipStream_t st);
 hipError_t kafka_launch_ep_combine(const bf16* back, const int* slot_map, const float* topk_w, int lo, int n_own,
                                    int k, int d, bf16* out, int64_t ldo, hipStream_t st);
+hipError_t kafka_launch_tile_gemm(const bf16* X, int64_t ldx, const bf16* Wt, int M, int N, int K, int mt, int nt, int splits,
+                                  int glu, bf16* Y, int64_t ldy, float* P, hipStream_t st);
 int kafka_skinny_plan(int M, int N, int K, int max_splits, int* splits);
 hipError_t kafka_launch_skinny_gemm(const bf16* X, int64_t ldx, const bf16* Wt, int M, int N, int K, int splits,
                                     int glu, bf16* Y, int64_t ldy, float* P, hipStream_t st);
@@ -661,6 +663,32 @@ static int64_t skinny_plan(int64_t M, int64_t N, int64_t K, int64_t max_splits) 
   return kafka_skinny_plan((int)M, (int)N, (int)K, (int)max_splits, &s) == 0 ? s : 0;
 }
 
+// Dense products of long steps (csrc/tile_gemm.hip) on tiles of 32 mt x 32 nt: y bf16 [M, N] (glu: [M, N / 2] activated) or
+// fp32 split-K slabs p [splits, M, N]
+static void tile_gemm(at::Tensor x, at::Tensor wt, c10::optional<at::Tensor> y, c10::optional<at::Tensor> p, int64_t mt,
+                      int64_t nt, int64_t splits, bool glu) {
+  CHECK_CUDA(x); CHECK_DT(x, at::kBFloat16); CHECK_CUDA(wt); CHECK_DT(wt, at::kBFloat16); CHECK_LASTDIM(x);
+  TORCH_CHECK(x.dim() == 2, "tile_gemm: x must be [M, K]");
+  TORCH_CHECK(wt.dim() == 4 && wt.is_contiguous() && wt.size(2) == 64 && wt.size(3) == 8,
+              "tile_gemm: wt must be contiguous [N/32, K/16, 64, 8]");
+  const int64_t M = x.size(0), K = x.size(1), N = wt.size(0) * 32;
+  TORCH_CHECK(wt.size(1) * 16 == K && M < (1 << 28) && (M < 2 || x.stride(0) >= K), "tile_gemm: shape");
+  TORCH_CHECK(y.has_value() != p.has_value(), "tile_gemm: one output");
+  bf16* yp = nullptr; float* pp = nullptr; int64_t ldy = 0;
+  if (y.has_value()) {
+    CHECK_DT(y.value(), at::kBFloat16); CHECK_CUDA(y.value()); CHECK_LASTDIM(y.value());
+    TORCH_CHECK(y->dim() == 2 && y->size(0) == M && y->size(1) == (glu ? N / 2 : N), "tile_gemm: y shape");
+    yp = bptr(y.value()); ldy = y->stride(0);
+  } else {
+    CHECK_DT(p.value(), at::kFloat); CHECK_CUDA(p.value());
+    TORCH_CHECK(p->is_contiguous() && p->dim() == 3 && p->size(0) == splits && p->size(1) == M && p->size(2) == N,
+                "tile_gemm: slabs must be [splits, M, N]");
+    pp = p->data_ptr<float>();
+  }
+  CHECK_HIP(kafka_launch_tile_gemm(bptr(x), x.stride(0), bptr(wt), (int)M, (int)N, (int)K, (int)mt, (int)nt, (int)splits,
+                                   glu ? 1 : 0, yp, ldy, pp, cur_stream()));
+}
+
 static void skinny_gemm(at::Tensor x, at::Tensor wt, c10::optional<at::Tensor> y, c10::optional<at::Tensor> p,
                         int64_t splits, bool glu) {
   CHECK_CUDA(x); CHECK_DT(x, at::kBFloat16); CHECK_DT(wt, at::kBFloat16); CHECK_LASTDIM(x);
@@ -1136,6 +1164,7 @@ PYBIND11_MODULE(_kafka_ops, m) {
         py::arg("v_cache"), py::arg("slots"), py::arg("Hq"), py::arg("Hkv"), py::arg("max_splits"),
         py::arg("stamps") = py::none());
   m.def("skinny_plan", &skinny_plan);
+  m.def("tile_gemm", &tile_gemm);
   m.def("skinny_gemm", &skinny_gemm);
   m.def("wstream_gemm_cfg", &wstream_gemm_cfg);
   m.def("slab_reduce", &slab_reduce);

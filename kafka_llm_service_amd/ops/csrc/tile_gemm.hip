@@ -1,0 +1,113 @@
+// Dense products of long steps on wave-tiled weights: Y[M, N] = X[M, K] W[N, K]^T, bf16, fp32 sums (gfx950).
+//
+// Tiles of 128, 192 and 256 rows and columns (ring.h), K split over workgroups into fp32 slabs where a step has few rows: the host
+// picks by a model of the launch (ops.tile_plan). What bounds it: a whole round of 256 x 256 tiles takes 1.24 us per 64 of K
+// (1.7 PFLOP/s) and 7.6 us for its start and its results; smaller tiles are bound by what the L2s give the CUs, 65 - 72 GB/s each
+// whatever the tile (17 - 18 TB/s): 192 x 192 0.75 us per 64 of K, 256 x 128 0.71, 128 x 128 (two workgroups a CU) 0.45 each. So a tile is as
+// large as leaves no round of the chip half empty, and sizes between 128 and 256 pay: 2048 rows of 4096 -> 6144 on 256 x 256 91 us, on
+// 256 x 192 78; 2800 rows on 192 x 192 120, on 256 x 256 150. Tried: two of the four waves moving the weights alone, eight stages ahead
+// (3 % more: their latency is not what a step of 136 - 256 rows waits for).
+#include "ring.h"
+
+namespace kafka {
+namespace tg {
+
+enum { OUT_BF16 = 0, OUT_SLAB = 1, OUT_GLU = 2, OUT_SLAB_GLU = 3 };
+
+// MT, NT: 16-row and 16-column parts of a wave's tile (2 x 2 waves); OCC workgroups on a CU
+template <int MT, int NT, int OCC>
+__global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const bf16* __restrict__ X, int64_t ldx,
+                                                             const bf16x8* __restrict__ Wt, int M, int N, int K, int S,
+                                                             bf16* __restrict__ Y, int64_t ldy, float* __restrict__ P,
+                                                             int mode) {
+  using R = ring::Ring<MT, NT, true>;
+  __shared__ __attribute__((aligned(1024))) char smem[R::LDS];
+  // item -> (split, rows, columns): an XCD takes one contiguous stretch of them: of a split the row tiles of up to 2048 rows
+  // side by side, then the next column tile, so that its weights leave memory once
+  const int rts = (M + R::BM - 1) / R::BM, nts = (N + R::BN - 1) / R::BN, tiles = rts * nts, total = tiles * S;
+  const int per = (total + 7) >> 3, k8 = blockIdx.x >> 3, item = (blockIdx.x & 7) * per + k8;
+  if (k8 >= per || item >= total) return;          // (uniform)
+  constexpr int GR = 2048 / R::BM;
+  const int sp = item / tiles, it = item - sp * tiles, g = it / (GR * nts), j = it - g * GR * nts, in_g = min(GR, rts - g * GR);
+  const int nt = j / in_g, row0 = (g * GR + j - nt * in_g) * R::BM, rows = min(R::BM, M - row0);
+  // K in units of 64, split as evenly as they go
+  const int units = K >> 6, u0 = (int)((int64_t)units * sp / S), u1 = (int)((int64_t)units * (sp + 1) / S);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, q = lane >> 4;
+  unsigned xo[2 * R::DX], wo[R::DW];
+#pragma unroll
+  for (int u = 0; u < 2 * R::DX; ++u) {            // rows past M reload the last, never stored
+    const int row = R::xrow(w, u, lane);
+    xo[u] = (unsigned)min(row, rows - 1) * (unsigned)(ldx * 2) + R::xbyte(row, lane);
+  }
+#pragma unroll
+  for (int u = 0; u < R::DW; ++u)                  // (tiles past N reload the last, never stored)
+    wo[u] = (unsigned)(min(nt * NT + R::wtile(w, u), (N >> 5) - 1) * (K >> 4) + R::wblock(w, u)) * 1024u;
+  ring::f32x4v acc[MT][NT];
+#pragma unroll
+  for (int a = 0; a < MT; ++a)
+#pragma unroll
+    for (int b = 0; b < NT; ++b) acc[a][b] = ring::f32x4v{0.f, 0.f, 0.f, 0.f};
+  R::multiply(acc, smem, ring::buffer(X + (int64_t)row0 * ldx + 64 * u0), xo, ring::buffer(Wt + (int64_t)u0 * 4 * 64),
+              R::wlane(lane), wo, 2 * (u1 - u0), lane, w);
+  // this lane: row 16 mt + r, columns 8 q .. of every 32-column tile
+  const int nb = nt * NT + NT / 2 * (w & 1), nall = N >> 5;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const int m = 16 * (MT * (w >> 1) + mt) + r;
+    if (m >= rows) continue;
+#pragma unroll
+    for (int t = 0; t < NT / 2; ++t) {
+      if (nb + t >= nall) continue;
+      if (mode == OUT_BF16) {
+        bf16x8 o;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = (bf16)acc[mt][2 * t + (i >> 2)][i & 3];
+        *reinterpret_cast<bf16x8*>(Y + (int64_t)(row0 + m) * ldy + (nb + t) * 32 + 8 * q) = o;
+      } else if (mode == OUT_GLU) {                // tiles of 32: gate, up, gate, up
+        if (t & 1) continue;
+        bf16x8 o;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float a = acc[mt][2 * t + (i >> 2)][i & 3], b = acc[mt][(2 * t + 2 + (i >> 2)) % NT][i & 3];
+          o[i] = (bf16)(a / (1.0f + __expf(-a)) * b);
+        }
+        *reinterpret_cast<bf16x8*>(Y + (int64_t)(row0 + m) * ldy + ((nb + t) >> 1) * 32 + 8 * q) = o;
+      } else {
+        // (gate | up order of interleaved tiles)
+        const int c = mode == OUT_SLAB ? (nb + t) * 32 : (((nb + t) & 1) ? N >> 1 : 0) + ((nb + t) >> 1) * 32;
+        float* p = P + ((int64_t)sp * M + row0 + m) * N + c + 8 * q;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) *reinterpret_cast<ring::f32x4v*>(p + 4 * h) = acc[mt][2 * t + h];
+      }
+    }
+  }
+}
+
+extern "C" hipError_t kafka_launch_tile_gemm(const bf16* X, int64_t ldx, const bf16* Wt, int M, int N, int K, int mt, int nt,
+                                             int splits, int glu, bf16* Y, int64_t ldy, float* P, hipStream_t st) {
+  if (M <= 0) return hipSuccess;
+  if (N < 32 || N % 32 || K % 64 || splits < 1 || K / 64 < 2 * splits || ldx % 8 || (glu && N % 64)) return hipErrorInvalidValue;
+  if ((Y != nullptr) == (P != nullptr) || (Y && (splits != 1 || ldy % 8 || reinterpret_cast<uintptr_t>(Y) % 16)))
+    return hipErrorInvalidValue;
+  if (reinterpret_cast<uintptr_t>(X) % 16 || 256 * ldx * 2 > (int64_t)0xffff0000 || (int64_t)N * K * 2 > (int64_t)0xffff0000)
+    return hipErrorInvalidValue;
+  const int mode = P ? (glu ? OUT_SLAB_GLU : OUT_SLAB) : (glu ? OUT_GLU : OUT_BF16);
+  const int64_t total = (int64_t)((M + 32 * mt - 1) / (32 * mt)) * ((N + 32 * nt - 1) / (32 * nt)) * splits;
+  if (total > 0x0fffffff) return hipErrorInvalidValue;
+  const unsigned grid = (unsigned)((total + 7) / 8 * 8);
+  const auto* wt = reinterpret_cast<const bf16x8*>(Wt);
+  auto a = [&](auto kern) { kern<<<grid, 256, 0, st>>>(X, ldx, wt, M, N, K, splits, Y, ldy, P, mode); };
+  if (mt == 8 && nt == 8) a(tile_gemm_kernel<8, 8, 1>);
+  else if (mt == 8 && nt == 4) a(tile_gemm_kernel<8, 4, 1>);
+  else if (mt == 8 && nt == 6) a(tile_gemm_kernel<8, 6, 1>);
+  else if (mt == 6 && nt == 8) a(tile_gemm_kernel<6, 8, 1>);
+  else if (mt == 6 && nt == 6) a(tile_gemm_kernel<6, 6, 1>);
+  else if (mt == 4 && nt == 6) a(tile_gemm_kernel<4, 6, 1>);
+  else if (mt == 4 && nt == 8) a(tile_gemm_kernel<4, 8, 1>);
+  else if (mt == 4 && nt == 4) a(tile_gemm_kernel<4, 4, 2>);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+}  // namespace tg
+}  // namespace kafka

@@ -1,0 +1,90 @@
+"""Dense products of long steps on wave-tiled weights (csrc/tile_gemm.hip, ops.linear_tile / linear_long / tile_plan)."""
+import random
+
+import pytest
+import torch
+
+from kafka_llm_service_amd import ops
+
+
+def test_plans_are_launches():
+    """Every plan is one that the kernel takes: at least two units of 64 of K a split, whole gate, up pairs a wave, slabs within
+    their bound; what it cannot take has no plan."""
+    rng = random.Random(3)
+    for _ in range(300):
+        M, N, K = rng.randint(1, 9000), 32 * rng.randint(1, 900), 64 * rng.randint(2, 230)
+        form = rng.choice(["slabs", "bf16", "glu"])
+        plan = ops.tile_plan(M, N, K, form, library=False)
+        if form == "glu" and N % 64:
+            assert plan is None
+            continue
+        mt, nt, s = plan
+        assert (mt, nt) in ops.TILES and K // 64 >= 2 * s and (form != "glu" or nt % 4 == 0)
+        assert s == 1 or 4 * s * M * N <= ops.TILE_SLAB_BYTES
+    assert ops.tile_plan(300, 4100, 4096) is None and ops.tile_plan(300, 4096, 64) is None and ops.tile_plan(300, 4096, 4112) is None
+    assert ops.tile_plan(0, 4096, 4096) is None and ops.tile_plan(300, 32800, 65536, library=False) is None   # 4 GB of weights
+    assert ops.tile_plan(300, 28672, 4096) is None and ops.tile_plan(300, 28672, 4096, "glu") is not None
+
+
+def test_long_products_on_the_cpu():
+    """Without a GPU linear_long is the plain product, from either weight, whatever the strides of x."""
+    w = torch.randn(96, 128)
+    wt = ops.tile_weight(w)
+    for x in (torch.randn(150, 128), torch.randn(128, 150).t(), torch.randn(150, 256)[:, ::2], torch.randn(1, 128).expand(150, 128)):
+        for y in (ops.linear_long(x, w, wt, slabs=True), ops.linear_long(x, None, wt), ops.linear_long(x, w, None)):
+            torch.testing.assert_close(y, x @ w.t())
+    assert ops.linear_glu_long(torch.randn(150, 128), ops.tile_weight(torch.randn(128, 128), glu=True)) is None
+
+
+def _close(got, want, K):
+    # sums of K terms of size ~ 1 / sqrt(K) in fp32 (errors of 1e-6 of them) rounded to bf16, 2^-9 of a value
+    assert ((got.float() - want).abs() <= 2 ** -8 * want.abs() + 1e-3).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mt,nt", sorted(ops.TILES))
+def test_tiles_against_fp32(mt, nt):
+    """Rows and columns that end inside, at and past a tile, one row, one 32-column tile, more than a group of row tiles; K of two and
+    three units a split (four and six stages; the ring holds four) and of uneven splits; wide rows of x; both outputs of either order
+    of weights. Rows of a padded output stay as they were."""
+    g = torch.Generator().manual_seed(mt * 10 + nt)
+    bm, bn = 32 * mt, 32 * nt
+    for M, N, K, s in ((1, 32, 128, 1), (bm - 1, bn, 192, 1), (bm, bn + 32, 256, 2), (bm + 1, 3 * bn - 32, 448, 3), (2100, 64, 320, 2),
+                       (200, 2 * bn + 64, 1088, 8), (65, 192, 1024, 8)):
+        x = torch.randn(M, K + 24, generator=g).to(torch.bfloat16).cuda()[:, 8:8 + K]
+        w = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
+        want = x.float() @ w.float().t()
+        wt = ops.tile_weight(w)
+        assert ops.tile_ok(x, wt)
+        ext = ops.ext()
+        y = torch.full((M + 1, N + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+        ext.tile_gemm(x, wt, y[:M, :N], None, mt, nt, 1, False)
+        _close(y[:M, :N], want, K)
+        assert (y[M:] == 7).all() and (y[:, N:] == 7).all()
+        if s > 1:
+            p = ops.linear_tile(x, wt, (mt, nt, s))
+            assert p.shape == (s, M, N) and ((p.sum(0) - want).abs() <= 1e-4).all()
+        if N % 64 == 0 and nt % 4 == 0:
+            gt, F = ops.tile_weight(w, glu=True), N // 2
+            _close(ops.linear_tile(x, gt, (mt, nt, 1), glu=True), torch.nn.functional.silu(want[:, :F]) * want[:, F:], K)
+            if s > 1:
+                assert ((ops.linear_tile(x, gt, (mt, nt, s), glu=True).sum(0) - want).abs() <= 1e-4).all()
+
+
+@pytest.mark.gpu
+def test_long_products_by_their_plans():
+    """linear_long and linear_glu_long over sizes of every route (tiles with and without splits, the library) and forms of x that the
+    kernel leaves to the library (odd strides, a shifted start)."""
+    g = torch.Generator().manual_seed(0)
+    for M, N, K in ((131, 2048, 2048), (300, 4096, 1024), (700, 96, 4096), (1300, 6176, 512), (257, 24608, 128), (3000, 1024, 256)):
+        w = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
+        wt = ops.tile_weight(w)
+        base = torch.randn(M, K + 16, generator=g).to(torch.bfloat16).cuda()
+        for x in (base[:, :K].contiguous(), base[:, 8:8 + K], base[:, 1:1 + K], base[:, :K].t().contiguous().t()):
+            want = x.float() @ w.float().t()
+            for y in (ops.linear_long(x, w, wt), ops.linear_long(x, None, wt), ops.linear_long(x, w, wt, slabs=True)):
+                _close(y.sum(0) if ops.is_slab(y) else y, want, K)
+            if N % 64 == 0:
+                a = ops.linear_glu_long(x, ops.tile_weight(w, glu=True))
+                if a is not None:
+                    _close(a, torch.nn.functional.silu(want[:, :N // 2]) * want[:, N // 2:], K)

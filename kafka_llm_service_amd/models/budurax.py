@@ -290,6 +290,19 @@ class _Layer:
     pass
 
 
+HEAD_ROWS = 64   # rows up to which the heads' products run on the kernel for small products (figures: csrc/small_gemm.hip)
+
+
+def head_product(x, w, wt, out=None):
+    """Per head x [H, n, K] @ w [H, N, K]^T; ``wt``: the same weights [H, K, N], ``w`` None: those alone."""
+    if w is not None and ops.small_ok(x, w, HEAD_ROWS) and (out is None or out.stride(0) % 4 == 0 and out.stride(1) % 4 == 0 and out.data_ptr() % 8 == 0):
+        if out is None:
+            out = torch.empty(x.shape[0], x.shape[1], w.shape[1], dtype=x.dtype, device=x.device)
+        ops.ext().small_gemm(x, w, out)
+        return out
+    return torch.bmm(x, wt) if out is None else torch.bmm(x, wt, out=out)
+
+
 def latent_mix(q, q_rot, cache, cache_t, lw, inp, m: SegMeta, ao, window: int = 0, sink=None, gate=None) -> None:
     """Latent attention of a step's rows: ao [T, H vdim] from q [T, H, dim] and the rotated q_rot [T, H, rot_dim], times
     sigmoid(gate) when given. Decoded tokens attend in the latent space (q_lat = W_uk^T q, out = W_uv (sum p c)), prompt
@@ -300,7 +313,7 @@ def latent_mix(q, q_rot, cache, cache_t, lw, inp, m: SegMeta, ao, window: int = 
         hops.latent_rows_ok(q, q_rot, cache, Dv) else None
     n = T if tables is None else tables[0]        # rows that stay in the latent space
     if n:
-        q_lat = torch.bmm(q[:n].transpose(0, 1), lw.uk_h)                         # [H, n, R]
+        q_lat = head_product(q[:n].transpose(0, 1), lw.uk_n, lw.uk_h)             # [H, n, R]
         o_lat = torch.empty(H, n, R, dtype=q.dtype, device=q.device)
         tiles, keys = m.tiles.get(hops.tile_tokens(H)), m.max_keys
         if n < T:
@@ -308,9 +321,9 @@ def latent_mix(q, q_rot, cache, cache_t, lw, inp, m: SegMeta, ao, window: int = 
         hops.latent_attn(q_lat, q_rot[:n], cache, m.block_tables, m.tok_seg[:n], m.seg, inp.positions[:n], lw.scale, o_lat,
                          cache_t, tiles, keys, window=window, sink=sink)
         if gate is None:
-            torch.bmm(o_lat, lw.uv_ht, out=ao[:n].view(n, H, Dv).transpose(0, 1))  # head h -> its vdim columns
+            head_product(o_lat, lw.uv.view(H, Dv, R), lw.uv_ht, ao[:n].view(n, H, Dv).transpose(0, 1))  # head h -> its vdim columns
         else:
-            hops.sigmoid_mul(torch.bmm(o_lat, lw.uv_ht), gate[:n], ao[:n])
+            hops.sigmoid_mul(head_product(o_lat, lw.uv.view(H, Dv, R), lw.uv_ht), gate[:n], ao[:n])
     if n < T:
         hops.latent_attn_portions(q, q_rot, cache, lw.uk_h.view(H * D, R), lw.uv, tables, m.block_tables, lw.scale, ao, window,
                                   sink, gate)
@@ -443,6 +456,10 @@ class BuduraxLM:
                 lw.dkv_off = lw.g_off + H * vd if lw.kv_from is None else -1
                 lw.dkv_norm = act(p + "mix.dkv.norm") if lw.kv_from is None else None
                 lw.uk_h = act(p + "mix.uk").view(H, D, R)                          # q_lat = q_u @ uk_h  (per head)
+                lw.uk_n = None
+                if dt == torch.bfloat16:
+                    lw.uk_n = lw.uk_h.transpose(1, 2).contiguous()                 # the same, [H, R, D] (head_product)
+                    self._tensors.append(lw.uk_n)
                 t = W[p + "mix.uv"].to(device=dev, dtype=dt).view(H, vd, R).transpose(1, 2).contiguous()
                 self._tensors.append(t)
                 lw.uv_ht = t                                                       # out = o_lat @ uv_ht (per head)
@@ -553,8 +570,8 @@ class BuduraxLM:
             if lw.side_gate is not None:
                 hops.add_ln(x, y, nw, nb, eps, h2)  # h2 = the new x in the model dtype (the gate GEMM's input)
                 g = torch.empty(T, cfg.token_side_dim, dtype=dt, device=dev)
-                hops.side_gate(F.linear(h2, lw.side_gate), inp.tokens, self.side_embed, i * cfg.token_side_dim, g)
-                ys = F.linear(g, lw.side_proj)
+                hops.side_gate(ops.linear_small(h2, lw.side_gate), inp.tokens, self.side_embed, i * cfg.token_side_dim, g)
+                ys = ops.linear_small(g, lw.side_proj)
             else:
                 hops.add_ln(x, y, nw, nb, eps)
             if ys is not None or stack is not None:

@@ -346,6 +346,7 @@ class FurapelLM:
                 lw.w_in = fused([q + "q", q + "dkv"], multiple=32)                  # row = [q heads | latent]
                 lw.dkv_norm = act(q + "dkv.norm")
                 lw.uk_h = act(q + "uk").view(H, D, R)                              # q_lat = q @ uk_h  (per head)
+                lw.uk_n = keep(lw.uk_h.transpose(1, 2)) if dt == torch.bfloat16 else None   # the same, [H, R, D] (head_product)
                 lw.uv_ht = keep(W[q + "uv"].to(device=dev, dtype=dt).view(H, Dv, R).transpose(1, 2))
                 lw.uv = act(q + "uv")
                 lw.scale = float(m["scale"])

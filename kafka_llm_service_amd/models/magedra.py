@@ -411,6 +411,7 @@ class MagedraLM:
                 lw.dq_norm = f32(p + "mix.dq.norm")
                 lw.dkv_norm = act(p + "mix.dkv.norm")
                 lw.uk_h = act(p + "mix.uk").view(H, D, R)                          # q_lat = q @ uk_h  (per head)
+                lw.uk_n = keep(lw.uk_h.transpose(1, 2)) if dt == torch.bfloat16 else None   # the same, [H, R, D] (head_product)
                 lw.uv_ht = keep(W[p + "mix.uv"].to(device=dev, dtype=dt).view(H, Dv, R).transpose(1, 2))
                 lw.uv = act(p + "mix.uv")
                 lw.o = act(p + "mix.o")

@@ -55,7 +55,7 @@ class MoEBlock:
 
     def __call__(self, x: torch.Tensor, lw) -> torch.Tensor:
         T, d = x.shape
-        logits = F.linear(x, lw.router)
+        logits = ops.linear_small(x, lw.router)
         r = ops.moe_route(logits, self.k)
         if self.ep > 1 and self.a2a:
             return self._a2a(x, lw, r)

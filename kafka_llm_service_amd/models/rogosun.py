@@ -412,6 +412,8 @@ class RogosunLM:
                     raise ValueError(f"layer {i}: {z['top']} of {E} experts in {z['keep']} of {z['groups']} groups")
                 lw.z = z
                 lw.router = f32(p + "mlp.router")
+                low = lw.router.to(dt)                                # where it is exact: the kernel for small products
+                lw.router_a = keep(low) if dt != torch.float32 and torch.equal(low.float(), lw.router) else None
                 lw.w_gu = keep(torch.stack([torch.cat([W[f"{p}mlp.e{e}.gate"], W[f"{p}mlp.e{e}.up"]], 0)
                                             for e in range(E)]).to(device=dev, dtype=dt))       # [E, 2 ff, d]
                 lw.w_down = keep(torch.stack([W[f"{p}mlp.e{e}.down"] for e in range(E)]).to(device=dev, dtype=dt))
@@ -499,7 +501,7 @@ class RogosunLM:
         H, D, Dv = (int(lw.m[k]) for k in ("heads", "dim", "vdim"))
         T, dt, dev, off = h.shape[0], self.dtype, self.device, lw.off
         proj = self._lin(h, lw.w_in, getattr(lw, "w_in_t", None))                 # [q | k | v | g | a1]
-        z = F.linear(proj[:, off["a1"]:off["a1"] + lw.low.shape[1]], lw.low)      # raw decays
+        z = ops.linear_small(proj[:, off["a1"]:off["a1"] + lw.low.shape[1]], lw.low)      # raw decays
         o = torch.empty(T, H * Dv, dtype=torch.float32, device=dev)
         chunks, short = m.chunks(hops.LIN_CHUNK, hops.LIN_CHUNK_MIN)
         hops.lin_scan(proj, off["q"], off["k"], proj[:, off["v"]:off["v"] + H * Dv], z, lw.z_bias, H, H, D, Dv,
@@ -525,7 +527,7 @@ class RogosunLM:
                          out_scale=lw.left_scale, kinds=m.tile_kinds(hops.sig_tile_tokens(H, G)))
         qkv = torch.empty(T, lw.conv.shape[0], dtype=dt, device=dev)
         hops.short_conv(proj, off["conv"], lw.conv, None, m.tok_seg, m.seg, st["conv"], qkv, act="silu")
-        low = F.linear(proj[:, off["low"]:off["low"] + lw.low.shape[1]], lw.low)  # raw decays | output gate
+        low = ops.linear_small(proj[:, off["low"]:off["low"] + lw.low.shape[1]], lw.low)  # raw decays | output gate
         o = torch.empty(T, Hr * Dvr, dtype=torch.float32, device=dev)
         chunks, short = m.chunks(hops.LIN_CHUNK, hops.LIN_CHUNK_MIN)
         hops.lin_scan(qkv, 0, Gr * Dr, qkv[:, 2 * Gr * Dr:], low[:, :Hr * Dr], lw.z_bias, Hr, Gr, Dr, Dvr, m.tok_seg,
@@ -539,7 +541,7 @@ class RogosunLM:
         z = lw.z
         T, d, dt, dev = h.shape[0], self.cfg.hidden_size, self.dtype, self.device
         tw, te, _ = hops.moe_router_grouped(h, lw.router, None, z["top"], z["groups"], z["keep"], score="sigmoid",
-                                            group_score="top2", norm=False, scale=z["scale"])
+                                            group_score="top2", norm=False, scale=z["scale"], w_act=lw.router_a)
         out = torch.empty(T, d, dtype=torch.float32, device=dev)
         hops.moe_experts(h, lw.w_gu, lw.w_down, tw, te, out, getattr(lw, "w_gu_t", None), getattr(lw, "w_down_t", None))
         if lw.sh_gu is None:

@@ -305,6 +305,34 @@ def skinny_plan(M: int, N: int, K: int, max_splits: int = 8) -> int:
     return s
 
 
+# ---- small products (csrc/small_gemm.hip) -----------------------------------------------------------------------------
+def small_ok(x: torch.Tensor, w: torch.Tensor, rows: int) -> bool:
+    """Whether x [.., M, K] @ w [.., N, K]^T of up to ``rows`` rows runs on the kernel for small products: bf16 operands of one
+    order, whole 16-byte pieces."""
+    d, K = x.dim(), x.shape[-1]
+    return x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and d == w.dim() and w.shape[-1] == K and \
+        0 < x.shape[-2] <= rows and K % 8 == 0 and K > 0 and w.shape[-2] % 4 == 0 and w.shape[-2] > 0 and \
+        x.stride(-1) == 1 and w.stride(-1) == 1 and x.stride(-2) % 8 == 0 and w.stride(-2) % 8 == 0 and \
+        (d == 2 or d == 3 and x.shape[0] == w.shape[0] and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0) and \
+        x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+
+
+def small_rows(N: int, K: int) -> int:
+    """Rows up to which a small product runs on the kernel instead of the library (figures: csrc/small_gemm.hip)."""
+    if K >= 1024:
+        return 1024 if N <= 64 else 0   # (a workgroup per 16 columns reads the rows again)
+    return 4096 if K <= 32 else 256
+
+
+def linear_small(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x [M, K] @ w [N, K]^T: gates, routers, low-rank projections - long rows and few columns, or short rows."""
+    if x.dim() == 2 and small_ok(x, w, small_rows(w.shape[0], w.shape[1])):
+        y = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
+        ext().small_gemm(x, w, y)
+        return y
+    return torch.nn.functional.linear(x, w)
+
+
 # ---- dense products of long steps on wave-tiled weights (csrc/tile_gemm.hip) -------------------------------------------
 # (16-row parts, 16-column parts) of a wave's tile, 2 x 2 waves a workgroup -> us: of a launch, of a round of 256 workgroups, of 64 of K
 # in it, and of a MB/us of what is written, over 4.5. Fitted to 6200 timings (19 shapes of width 2048 and 4096, 136 - 4099 rows,

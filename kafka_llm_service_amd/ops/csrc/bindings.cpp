@@ -118,6 +118,8 @@ hipError_t kafka_launch_ep_recv_route(const bf16* img, int ep, int C, int MR, in
                                       float* perm_w, int* expert_off, int* tile_off, hipStream_t st);
 hipError_t kafka_launch_ep_combine(const bf16* back, const int* slot_map, const float* topk_w, int lo, int n_own,
                                    int k, int d, bf16* out, int64_t ldo, hipStream_t st);
+hipError_t kafka_launch_small_gemm(const bf16* X, const bf16* W, int B, int M, int N, int K, int64_t xb, int64_t xm, int64_t wb,
+                                   int64_t wn, const float* bias, int f32, void* Y, int64_t yb, int64_t ym, hipStream_t st);
 hipError_t kafka_launch_tile_gemm(const bf16* X, int64_t ldx, const bf16* Wt, int M, int N, int K, int mt, int nt, int splits,
                                   int glu, bf16* Y, int64_t ldy, float* P, hipStream_t st);
 int kafka_skinny_plan(int M, int N, int K, int max_splits, int* splits);
@@ -663,6 +665,26 @@ static int64_t skinny_plan(int64_t M, int64_t N, int64_t K, int64_t max_splits) 
   return kafka_skinny_plan((int)M, (int)N, (int)K, (int)max_splits, &s) == 0 ? s : 0;
 }
 
+// Small products (csrc/small_gemm.hip): out[b, m, n] = x[b, m, :] . w[b, n, :] of 2-D or 3-D operands, bf16 rows, out bf16 or fp32
+static void small_gemm(at::Tensor x, at::Tensor w, at::Tensor out, c10::optional<at::Tensor> bias) {
+  CHECK_CUDA(x); CHECK_DT(x, at::kBFloat16); CHECK_LASTDIM(x);
+  CHECK_CUDA(w); CHECK_DT(w, at::kBFloat16); CHECK_LASTDIM(w);
+  CHECK_CUDA(out); CHECK_LASTDIM(out);
+  const int64_t d = x.dim(), B = d == 3 ? x.size(0) : 1, M = x.size(-2), K = x.size(-1), N = w.size(-2);
+  const bool f32 = out.scalar_type() == at::kFloat;
+  TORCH_CHECK((d == 2 || d == 3) && w.dim() == d && out.dim() == d && (f32 || out.scalar_type() == at::kBFloat16), "small_gemm: operands");
+  TORCH_CHECK(w.size(-1) == K && out.size(-2) == M && out.size(-1) == N && (d == 2 || (w.size(0) == B && out.size(0) == B)) &&
+                  M < (1 << 28) && N < (1 << 20) && K < (1 << 20), "small_gemm: shape");
+  if (bias.has_value()) {
+    CHECK_DT(bias.value(), at::kFloat);
+    TORCH_CHECK(bias->is_cuda() && bias->is_contiguous() && bias->numel() == N && f32, "small_gemm: bias [N] of an fp32 result");
+  }
+  CHECK_HIP(kafka_launch_small_gemm(bptr(x), bptr(w), (int)B, (int)M, (int)N, (int)K, d == 3 ? x.stride(0) : 0, x.stride(-2),
+                                    d == 3 ? w.stride(0) : 0, w.stride(-2),
+                                    bias.has_value() ? bias->data_ptr<float>() : nullptr, f32 ? 1 : 0, out.data_ptr(),
+                                    d == 3 ? out.stride(0) : 0, out.stride(-2), cur_stream()));
+}
+
 // Dense products of long steps (csrc/tile_gemm.hip) on tiles of 32 mt x 32 nt: y bf16 [M, N] (glu: [M, N / 2] activated) or
 // fp32 split-K slabs p [splits, M, N]
 static void tile_gemm(at::Tensor x, at::Tensor wt, c10::optional<at::Tensor> y, c10::optional<at::Tensor> p, int64_t mt,
@@ -1165,6 +1187,7 @@ PYBIND11_MODULE(_kafka_ops, m) {
         py::arg("stamps") = py::none());
   m.def("skinny_plan", &skinny_plan);
   m.def("tile_gemm", &tile_gemm);
+  m.def("small_gemm", &small_gemm, py::arg("x"), py::arg("w"), py::arg("out"), py::arg("bias") = c10::nullopt);
   m.def("skinny_gemm", &skinny_gemm);
   m.def("wstream_gemm_cfg", &wstream_gemm_cfg);
   m.def("slab_reduce", &slab_reduce);

@@ -1,0 +1,118 @@
+// Small products of bf16 rows with row-major weights: Y[b][m][n] = sum_k X[b][m][k] W[b][n][k], fp32 sums, bf16 or fp32 results
+// (gfx950). Gates and routers (few columns, long rows), low-rank projections (short rows, many columns) and the products of
+// latent attention's heads (a small product per head): what has neither a tiled copy nor the size for one.
+//
+// What bounds it: a round trip to memory, a launch, and with long rows of a power of two that all 16 of a load lie in one cache
+// channel. So the loads of a wave's whole share of K (16 waves share it) are in flight together. The library's kernels take as long here, but
+// its call costs the host 17 us and this one 3, which is what steps of few rows wait for.
+// us, library on the GPU / this kernel: 64 columns of K = 4096, 64 rows 7.6 / 8.8, 900 8.1 / 9.4, 2048 15.2 / 16.9, 4096 15.9 / 31.9; 4096 columns of
+// K = 64, 64 rows 3.6 / 3.3, 300 5.4 / 4.7, 900 5.8 / 8.4; 2048 of K = 16, 64 rows 4.0 / 2.8, 4096 10.1 / 8.9; 8192 of K = 128, 128 rows
+// 4.7 / 4.6, 300 6.3 / 9.8; 32 heads of 128 -> 512, 64 rows 4.6 / 4.6, 128 5.5 / 7.9, of 512 -> 128, 64 rows 8.6 / 4.7, 300 15.3 / 16.1.
+#include "common.h"
+
+namespace kafka {
+namespace sg {
+
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+struct Strides {
+  int64_t xb, xm, wb, wn, yb, ym;
+};
+
+// A wave: 16 rows x 16 NT columns over its share of K. KW waves of a workgroup share K (their sums meet in LDS), the other
+// 4 / KW (KW up to 4) take further columns. Products are taken with the weights first: a lane holds four columns of one row.
+template <int NT, int KW, bool F32>
+__global__ __launch_bounds__(64 * (KW > 4 ? KW : 4)) void small_gemm_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W,
+                                                                            int M, int N, int K, const float* __restrict__ bias,
+                                                                            void* __restrict__ Y, Strides st) {
+  constexpr int NW = KW > 4 ? KW : 4, CW = NW / KW;   // waves; column parts
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, q = lane >> 4;
+  const int kw = w % KW, m0 = blockIdx.x * 16, n0 = (blockIdx.y * CW + w / KW) * 16 * NT, b = blockIdx.z;
+  // shares of K in whole steps of 32
+  const int steps = (K + 31) >> 5, s0 = steps * kw / KW, s1 = steps * (kw + 1) / KW;
+  const bf16* x = X + b * st.xb + (int64_t)min(m0 + r, M - 1) * st.xm + 8 * q;
+  const bf16* wp[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) wp[t] = W + b * st.wb + (int64_t)min(n0 + 16 * t + r, N - 1) * st.wn + 8 * q;
+  f32x4v acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  const bf16x8 zero = {};
+  auto step = [&](int s, bool in) {
+    const bf16x8 xv = in ? load_bf16x8(x + 32 * s) : zero;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(in ? load_bf16x8(wp[t] + 32 * s) : zero, xv, acc[t], 0, 0, 0);
+  };
+  const int whole = min(s1, K >> 5);                 // (a last step of 8, 16 or 24: the lanes past K bring zeros)
+  int s = s0;
+  constexpr int U = KW == 16 ? 8 : 4;                // steps whose loads are in flight together
+  for (; s + U <= whole; s += U) {
+    bf16x8 xv[U], wv[U][NT];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      xv[j] = load_bf16x8(x + 32 * (s + j));
+#pragma unroll
+      for (int t = 0; t < NT; ++t) wv[j][t] = load_bf16x8(wp[t] + 32 * (s + j));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[j][t], xv[j], acc[t], 0, 0, 0);
+  }
+  for (; s < whole; ++s) step(s, true);
+  if (s < s1) step(s, 32 * s + 8 * q < K);
+  if constexpr (KW > 1) {
+    __shared__ f32x4v part[NW][NT][64];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) part[w][t][lane] = acc[t];
+    __syncthreads();
+    if (kw) return;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int j = 1; j < KW; ++j) acc[t] += part[w + j][t][lane];
+  }
+  const int m = m0 + r;
+  if (m >= M) return;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int n = n0 + 16 * t + 4 * q;               // (N is a multiple of 4)
+    if (n >= N) continue;
+    const int64_t at = b * st.yb + (int64_t)m * st.ym + n;
+    if constexpr (F32) {
+      if (bias) acc[t] += *reinterpret_cast<const f32x4v*>(bias + n);
+      *reinterpret_cast<f32x4v*>(reinterpret_cast<float*>(Y) + at) = acc[t];
+    } else {
+      bf16x4 o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = (bf16)acc[t][i];
+      *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(Y) + at) = o;
+    }
+  }
+}
+
+extern "C" hipError_t kafka_launch_small_gemm(const bf16* X, const bf16* W, int B, int M, int N, int K, int64_t xb, int64_t xm,
+                                              int64_t wb, int64_t wn, const float* bias, int f32, void* Y, int64_t yb, int64_t ym, hipStream_t st) {
+  if (B < 1 || M < 1 || N < 1) return hipSuccess;
+  const uintptr_t ya = reinterpret_cast<uintptr_t>(Y);
+  if (N % 4 || K < 8 || K % 8 || xb % 8 || xm % 8 || wb % 8 || wn % 8 || yb % 4 || ym % 4 || reinterpret_cast<uintptr_t>(X) % 16 ||
+      reinterpret_cast<uintptr_t>(W) % 16 || ya % (f32 ? 16 : 8) || B > 65535 ||
+      (bias && (!f32 || reinterpret_cast<uintptr_t>(bias) % 16)) || (N + 15) / 16 > 65535)
+    return hipErrorInvalidValue;
+  const Strides s{xb, xm, wb, wn, yb, ym};
+  const int rows = (M + 15) / 16;
+  auto go = [&](auto kern, int nt, int kw) {
+    const int cols = 16 * nt * (kw >= 4 ? 1 : 4 / kw);
+    kern<<<dim3(rows, (N + cols - 1) / cols, B), 64 * (kw > 4 ? kw : 4), 0, st>>>(X, W, M, N, K, bias, Y, s);
+    return hipGetLastError();
+  };
+  // Long K: 16 waves share it, a workgroup per 16 columns (64 columns of 4096 in one workgroup of 8 waves 19.7 us at 64 rows, so 8.8);
+  // in between 4 waves; short K: a wave takes 64 columns alone.
+  if (K >= 1024) return f32 ? go(small_gemm_kernel<1, 16, true>, 1, 16) : go(small_gemm_kernel<1, 16, false>, 1, 16);
+  if (K >= 256) return f32 ? go(small_gemm_kernel<2, 4, true>, 2, 4) : go(small_gemm_kernel<2, 4, false>, 2, 4);
+  return f32 ? go(small_gemm_kernel<4, 1, true>, 4, 1) : go(small_gemm_kernel<4, 1, false>, 4, 1);
+}
+
+}  // namespace sg
+}  // namespace kafka

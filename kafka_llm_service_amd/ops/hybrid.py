@@ -871,7 +871,8 @@ def moe_router_grouped(h, w, correction, k: int, groups: int, keep: int, eps: fl
     ``scale``. With ``extra_gate`` the last row of ``w`` is a gate vector and sigmoid of its product is returned per
     row. Returns (weights fp32 [T, k], experts int32 [T, k], gate fp32 [T] or None).
     ``w_act``: the same weights in h's dtype when they are exact in it - then a plain choice (softmax, no groups, no
-    correction) of up to 64 experts is one kernel, product included (bf16 products, fp32 sums: the same logits)."""
+    correction) of up to 64 experts is one kernel, product included (bf16 products, fp32 sums: the same logits); other choices
+    take the logits of steps of few rows from the kernel for small products."""
     T = h.shape[0]
     E = w.shape[0] - (1 if extra_gate else 0)
     if E < 1 or groups < 1 or E % groups or not 1 <= keep <= groups or not 1 <= k <= keep * (E // groups):
@@ -889,7 +890,14 @@ def moe_router_grouped(h, w, correction, k: int, groups: int, keep: int, eps: fl
     elif _gpu(h):
         # logits as one full-precision fp32 matrix product (the engine switches reduced-precision matrix modes off),
         # then the choice kernel
-        ext().hy_moe_topk_grouped(torch.mm(h.float(), w.t()), int(E), correction, int(groups), int(keep), float(eps),
+        from kafka_llm_service_amd import ops
+
+        if w_act is not None and ops.small_ok(h, w_act, 1024) and h.shape[1] >= 1024 and w_act.shape[0] <= 64:
+            z = torch.empty(T, w_act.shape[0], dtype=torch.float32, device=h.device)   # (the same products and sums)
+            ext().small_gemm(h, w_act, z)
+        else:
+            z = torch.mm(h.float(), w.t())
+        ext().hy_moe_topk_grouped(z, int(E), correction, int(groups), int(keep), float(eps),
                                   tw, te, gate, score == "sigmoid", group_score == "top2", bool(norm), float(scale))
     else:
         ref.moe_router_grouped(h, w, E, correction, k, groups, keep, eps, tw, te, gate, score, group_score, norm, scale)
@@ -1091,10 +1099,22 @@ def narrow_ok(x, w) -> bool:
         bool(ext().narrow_ok(w.shape[0], w.shape[1], x.stride(0)))
 
 
+# Gate products of long rows: the kernel for small products gives 16 columns a workgroup, the narrow one all of them to one, which
+# waits longer for few rows and reads the rows once (32 columns of K = 4096, us, narrow / small: 16 rows 12.3 / 8.6, 2048 12.8 /
+# 9.4, 4096 13.3 / 16.4).
+SMALL_F32_ROWS = 2048
+
+
 def linear_f32(x, w, bias=None) -> torch.Tensor:
     """x @ w^T (+ bias fp32) with an fp32 result for operands in the activation dtype: one matrix product, nothing rounded
     to it. Few weight rows (gate projections) have a kernel of their own."""
     if _gpu(x) and x.dtype == torch.bfloat16:
+        from kafka_llm_service_amd import ops
+
+        if x.dim() == 2 and ops.small_ok(x, w, SMALL_F32_ROWS) and 1024 <= w.shape[1] and w.shape[0] <= 64:
+            out = torch.empty(x.shape[0], w.shape[0], dtype=torch.float32, device=x.device)
+            ext().small_gemm(x, w, out, bias)
+            return out
         if narrow_ok(x, w):
             out = torch.empty(x.shape[0], w.shape[0], dtype=torch.float32, device=x.device)
             ext().narrow_linear(x, w, bias, out)

@@ -1,0 +1,80 @@
+"""Small products (csrc/small_gemm.hip, ops.linear_small, hybrid.linear_f32, the heads' products of latent attention)."""
+import pytest
+import torch
+
+from kafka_llm_service_amd import ops
+from kafka_llm_service_amd.models.budurax import head_product
+from kafka_llm_service_amd.ops import hybrid as hops
+
+
+def _close(got, want):
+    # sums of K terms of size ~ 1 / sqrt(K) in fp32 (errors of 1e-6 of them) rounded to bf16, 2^-9 of a value
+    assert ((got.float() - want).abs() <= 2 ** -8 * want.abs() + 1e-4).all()
+
+
+def test_on_the_cpu():
+    """Without a GPU the plain products, whatever the strides."""
+    x, w = torch.randn(5, 24)[:, ::2], torch.randn(7, 12)
+    torch.testing.assert_close(ops.linear_small(x, w), x @ w.t())
+    a, h = torch.randn(6, 3, 8), torch.randn(3, 10, 8)
+    for n in (h, None):
+        torch.testing.assert_close(head_product(a.transpose(0, 1), n, h.transpose(1, 2)), torch.einsum("tha,hna->htn", a, h))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [8, 16, 40, 64, 128, 256, 264, 1016, 1024, 1032, 4096])
+def test_against_fp32(K):
+    """Rows and columns that end inside, at and past the 16 of a tile; K that ends inside a step of 32, of one step and of shares that
+    differ by one; rows and results in wider buffers (what lies beside them stays); fp32 results and their bias."""
+    g = torch.Generator().manual_seed(K)
+    for M, N in ((1, 4), (15, 8), (16, 16), (17, 64), (33, 68), (200, 260)):
+        x = torch.randn(M, K + 16, generator=g).to(torch.bfloat16).cuda()[:, 8:8 + K]
+        w = (torch.randn(N, K + 8, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()[:, :K]
+        b = torch.randn(N, generator=g).cuda()
+        want = x.float() @ w.float().t()
+        y = torch.full((M + 1, N + 4), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.ext().small_gemm(x, w, y[:M, :N])
+        _close(y[:M, :N], want)
+        assert (y[M:] == 7).all() and (y[:, N:] == 7).all()
+        f = torch.empty(M, N, device="cuda")
+        ops.ext().small_gemm(x, w, f)
+        assert ((f - want).abs() <= 2e-5).all()
+        ops.ext().small_gemm(x, w, f, b)
+        assert ((f - want - b).abs() <= 2e-5).all()
+        assert ((hops.linear_f32(x, w.contiguous(), b) - want - b).abs() <= 2e-5).all()
+        _close(ops.linear_small(x, w), want)
+
+
+@pytest.mark.gpu
+def test_rows_beyond_and_forms_of_the_library():
+    """One row past each limit, and operands that the kernel does not take (odd columns, odd strides, a shifted start)."""
+    g = torch.Generator().manual_seed(1)
+    for N, K in ((64, 1024), (68, 1024), (32, 16), (512, 128)):
+        n = ops.small_rows(N, K)
+        for M in (n, n + 1):
+            x, w = torch.randn(max(M, 1), K, generator=g).to(torch.bfloat16).cuda(), (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
+            assert ops.small_ok(x, w, n) == (0 < M <= n)
+            _close(ops.linear_small(x, w), x.float() @ w.float().t())
+    x = torch.randn(20, 72, generator=g).to(torch.bfloat16).cuda()
+    w = torch.randn(18, 64, generator=g).to(torch.bfloat16).cuda() / 8
+    for a, b in ((x[:, :64], w), (x[:, 1:65], w[:16]), (x[:, :64].t().contiguous().t(), w[:16]), (x[:, :60], w[:16, :60])):
+        assert not ops.small_ok(a, b, 4096)
+        _close(ops.linear_small(a, b), a.float() @ b.float().t())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 16, 63, 64, 65])
+def test_heads(n):
+    """Products per head into the head's columns of a wider row and into rows of their own, queries as slices of a fused row."""
+    g = torch.Generator().manual_seed(n)
+    H, D, R = 6, 128, 192
+    q = torch.randn(n, H, D + 64, generator=g).to(torch.bfloat16).cuda()[:, :, :D]
+    uk = (torch.randn(H, D, R, generator=g) / D ** 0.5).to(torch.bfloat16).cuda()
+    want = torch.stack([q[:, h].float() @ uk[h].float() for h in range(H)])
+    _close(head_product(q.transpose(0, 1), uk.transpose(1, 2).contiguous(), uk), want)
+    o = torch.randn(H, n, R, generator=g).to(torch.bfloat16).cuda()
+    uv = (torch.randn(H, D, R, generator=g) / R ** 0.5).to(torch.bfloat16).cuda()
+    ao = torch.empty(n, H * D, dtype=torch.bfloat16, device="cuda")
+    head_product(o, uv, uv.transpose(1, 2).contiguous(), ao.view(n, H, D).transpose(0, 1))
+    for h in range(H):
+        _close(ao[:, h * D:(h + 1) * D], o[h].float() @ uv[h].float().t())

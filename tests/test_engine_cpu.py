@@ -494,6 +494,20 @@ def test_plan_prefill_items_balances_causal_tiles():
     assert 200 <= len(items) * 8 <= 256, len(items) * 8
 
 
+def test_whole_prefill_tiles_come_longest_first():
+    """Tiles of a launch without splits are ordered by the keys they attend, not by their chunk's bound, which they share: two
+    portions of different lengths, and the many tiles of a long prompt."""
+    from kafka_llm_service_amd.engine.model_runner import plan_prefill_items
+
+    for tiles in ([(64 * i, 64, 0, 64 * (i + 1), 8192) for i in range(128)],
+                  [(64 * i, 64, 0, 64 * (i + 1), 320) for i in range(5)] + [(320 + 64 * i, 64, 1, 3000 + 64 * i, 3256) for i in range(60)]):
+        items, splits, ranges = plan_prefill_items(tiles, 8, 256, 256)
+        ext = {t[0]: t[3] for t in tiles}
+        assert splits == 0 and not ranges and sorted(it[0] for it in items) == sorted(ext)
+        order = [ext[it[0]] for it in items]
+        assert order == sorted(order, reverse=True)
+
+
 def test_padded_mixed_steps_match_unpadded(base_engine, monkeypatch):
     """Steps beyond the streaming GEMM's rows (up to 256) padded with inert rows (pad_step_rows) produce the same
     greedy tokens (checked with the streaming bound at 128, so a 150-row step is padded)."""

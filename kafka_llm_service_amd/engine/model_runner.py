@@ -168,6 +168,18 @@ MIN_DECODE_KEYS = 256      # smallest key range of one decode work item
 # profiles/r02/decode_items_ab.jsonl)
 ROWS_BUCKETS = (64, 96, 128, 256, 1 << 30)  # step-size histogram buckets (decode GEMM row-tile plans, skinny, BLAS)
 DECODE_TARGET_ITEMS = 1344  # (768 / 1536 / 2304 lose to it: profiles/r04/bench_ab_decode_target_blas.jsonl)
+# Rows that leave room in two (three) workgroups a CU get pieces for one whole round of them: a piece is a chain of waits (item, page ids,
+# keys, its partial's merge) beside its bytes, and a round that is not whole leaves CUs idle. us a step, pieces for 1344 workgroups / one round:
+# 64 rows of 1344 keys 844 / 818 (592 workgroups 833, 736 830), 16 of 3000 608 / 585, fp8 29 of 7900 768 / 745 (376 workgroups 787, 752 775), fp8 8 of 8000 611 / 570,
+# 90 of 700 793 / 775 (three a CU); 128 rows are more than that either way (1333 / 1336 on one piece each).
+DECODE_ROUNDS = (512, 768)
+
+
+def decode_round(n: int) -> int:
+    """Workgroups of the round that n rows x heads get their pieces for, 0 = more than one."""
+    return next((r for r in DECODE_ROUNDS if n <= r), 0)
+
+
 MAX_PARTIALS = 64           # partial slots per row that the decode kernel's fused merge reads (one lane each)
 MAX_PREFIX_CHUNKS = 32
 
@@ -323,6 +335,12 @@ def decode_items(seq_lens: np.ndarray, kv_start: np.ndarray, npre: np.ndarray, h
     ns = np.minimum(np.maximum(1, -(-suffix // ch)), MAX_PARTIALS - npre)
     bps = -(-nb // ns)
     ns = -(-nb // bps)  # no empty trailing piece
+    whole = decode_round(B * hkv) if target > 0 else 0
+    while whole and int(ns.sum()) * hkv > whole:     # (rounding up gave the rows more pieces than the round has)
+        ch += max(32, ch // 16 // 32 * 32)
+        ns = np.minimum(np.maximum(1, -(-suffix // ch)), MAX_PARTIALS - npre)
+        bps = -(-nb // ns)
+        ns = -(-nb // bps)
     rows = np.repeat(np.arange(B), ns)
     first = np.cumsum(ns) - ns
     split = np.arange(rows.shape[0]) - np.repeat(first, ns)
@@ -819,7 +837,8 @@ class ModelRunner:
     def _plan_decode_items(self, h: HostStep, seq_lens: np.ndarray, kv_start: np.ndarray, npre: np.ndarray,
                            i32_parts: list) -> None:
         if self.graphs is not None or self.fixed_decode_items:  # graph replay: the decode grid depends on B alone
-            ditems = decode_items_fixed(seq_lens, kv_start, npre, self.model.hkv)
+            ditems = decode_items_fixed(seq_lens, kv_start, npre, self.model.hkv,
+                                        decode_round(len(seq_lens) * self.model.hkv) or DECODE_TARGET_ITEMS)
         else:
             ditems = decode_items(seq_lens, kv_start, npre, self.model.hkv)
         h.n_dec_items = int(ditems.shape[0])

@@ -34,7 +34,6 @@ from pathlib import Path
 
 import numpy as np
 import torch
-import torch.nn.functional as F
 
 from kafka_llm_service_amd import ops
 from kafka_llm_service_amd.ops import hybrid as hops
@@ -539,7 +538,7 @@ class BuduraxLM:
         cfg, dt, dev = self.cfg, self.dtype, self.device
         m: SegMeta = inp.attn
         T, d, eps = inp.tokens.shape[0], cfg.hidden_size, cfg.norm_eps
-        x = F.embedding(inp.tokens, self.embed)  # fp32 [T, d] residual stream
+        x = ops.gather_rows(self.embed, inp.tokens)  # fp32 [T, d] residual stream
         stack = None
         if self.has_dwa:
             stack = torch.empty(len(self.layers) + 1, T, d, dtype=torch.float32, device=dev)
@@ -578,7 +577,7 @@ class BuduraxLM:
                 hops.side_dwa(x, ys, lw.side_norm, eps, stack, i, lw.dwa)
             if layers_out is not None:
                 layers_out.append(x.clone())
-        xs = x.index_select(0, inp.logit_rows)
+        xs = ops.gather_rows(x, inp.logit_rows)
         hf = torch.empty(xs.shape[0], d, dtype=dt, device=dev)
         hops.ln_shift(xs, self.final_norm, self.final_norm_b, eps, hf)
         return self._lin(hf, self.head, getattr(self, "head_t", None)).float()[:, :cfg.vocab_size]

@@ -43,7 +43,6 @@ from dataclasses import dataclass, field
 from pathlib import Path
 
 import torch
-import torch.nn.functional as F
 
 from kafka_llm_service_amd import ops
 from kafka_llm_service_amd.models.budurax import SegMeta, latent_mix, rotary_table
@@ -431,7 +430,7 @@ class FurapelLM:
         cfg, dt, dev = self.cfg, self.dtype, self.device
         m: SegMeta = inp.attn
         T, d = inp.tokens.shape[0], cfg.hidden_size
-        x = F.embedding(inp.tokens, self.embed)       # fp32 [T, d] residual (the table holds the scale)
+        x = ops.gather_rows(self.embed, inp.tokens)       # fp32 [T, d] residual (the table holds the scale)
         h1, h2 = (torch.empty(T, d, dtype=dt, device=dev) for _ in range(2))
         both = None                                   # the loop product's input [residual | embedding rows]
         if self.loop_in is not None:
@@ -466,7 +465,7 @@ class FurapelLM:
             hops.add_tanh_norm(x, y, ye, **outputs(r + 1))
             if layers_out is not None:
                 layers_out.append(x.clone())
-        xs = x.index_select(0, inp.logit_rows)
+        xs = ops.gather_rows(x, inp.logit_rows)
         hf = torch.empty(xs.shape[0], d, dtype=dt, device=dev)
         hops.add_tanh_norm(xs, norms=[self.final_norm], outs=[hf])
         logits = self._lin(hf, self.head, getattr(self, "head_t", None)).float()

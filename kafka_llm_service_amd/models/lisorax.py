@@ -428,7 +428,7 @@ class LisoraxLM:
         cfg, dt, dev = self.cfg, self.dtype, self.device
         m: SegMeta = inp.attn
         T, d, eps = inp.tokens.shape[0], cfg.hidden_size, cfg.norm_eps
-        x = F.embedding(inp.tokens, self.embed)  # fp32 [T, d] residual stream (the table holds the scale)
+        x = ops.gather_rows(self.embed, inp.tokens)  # fp32 [T, d] residual stream (the table holds the scale)
         h = torch.empty(T, d, dtype=dt, device=dev)
         hm = torch.empty(T, d, dtype=dt, device=dev) if cfg.canon_taps >= 1 else h
         if self.layers:
@@ -448,7 +448,7 @@ class LisoraxLM:
             hops.add2(x, y, ye, nxt, eps, h if nxt is not None else None)
             if layers_out is not None:
                 layers_out.append(x.clone())
-        xs = x.index_select(0, inp.logit_rows)
+        xs = ops.gather_rows(x, inp.logit_rows)
         hf = torch.empty(xs.shape[0], d, dtype=dt, device=dev)
         hops.rms_norm(xs, self.final_norm, eps, hf)
         return self._lin(hf, self.head, getattr(self, "head_t", None)).float()[:, :cfg.vocab_size]

@@ -56,7 +56,7 @@ SKINNY = frozenset(p for p in os.environ.get("KAFKA_SKINNY", "").replace("+", ",
 # (profiles/r06/fused/README.md).
 FUSED = os.environ.get("KAFKA_FUSED_DECODE", "0") == "1"
 _OVL: dict = {}
-_SEAM_DONE = object()  # forward(): the previous layer's overlapped seam already produced this layer's input
+_SEAM_DONE = object()  # forward(): residual and x are this layer's already (the embedding, an overlapped seam)
 
 
 def _overlap_stream(dev: torch.device):
@@ -231,22 +231,24 @@ class TransformerLM:
         T = inp.tokens.shape[0]
         if self._fused_ok(T, k_caches):
             return self._forward_fused(inp, k_caches, v_caches, gather)
-        h = self._embed(inp.tokens)
-        residual = h
-        x = torch.empty_like(h)
+        delta, pending = None, False
+        if self.tp == 1:  # (the embedding is a fresh tensor, which the residual stream owns)
+            residual, x = ops.embed_rmsnorm(self.embed, inp.tokens, self.layers[0].input_norm, cfg.rms_norm_eps)
+            delta = _SEAM_DONE
+        else:
+            h = self._embed(inp.tokens)
+            residual = h
+            x = torch.empty_like(h)
         q = torch.empty(T, self.hq, self.D, dtype=self.dtype, device=self.device)
         attn_out = torch.empty(T, self.hq, self.D, dtype=self.dtype, device=self.device)
         eps = cfg.rms_norm_eps
         tp = self.tp > 1
-        delta, pending = None, False
         for i, lw in enumerate(self.layers):
             if delta is _SEAM_DONE:
-                pass  # the previous layer's overlapped down seam already wrote residual and x
+                pass  # the embedding or the previous layer's overlapped down seam already wrote residual and x
             elif delta is None:
                 ops.rmsnorm(h, lw.input_norm, eps, out=x)
-                # the embedding is a fresh tensor at TP = 1 (the residual stream can own it); under TP it may be the
-                # all-reduce's persistent buffer
-                residual = h if self.tp == 1 else h.clone()
+                residual = h.clone()  # (the embedding may be the all-reduce's persistent buffer)
             elif pending:
                 pstate.tp_all_reduce_add_rmsnorm(delta, residual, lw.input_norm, eps, out=x)
             else:
@@ -293,10 +295,7 @@ class TransformerLM:
                 pending = tp
         if pending:
             delta = pstate.tp_all_reduce(delta)
-        rows = inp.logit_rows
-        d_sel = delta.index_select(1 if ops.is_slab(delta) else 0, rows)
-        r_sel = residual.index_select(0, rows)
-        hf = ops.fused_add_rmsnorm(d_sel, r_sel, self.final_norm, eps)
+        hf = ops.rows_add_rmsnorm(delta, residual, inp.logit_rows, self.final_norm, eps)
         logits = self._linear(hf, self.lm_head, self.lm_head_t, max_splits=1)
         if not gather:
             return logits

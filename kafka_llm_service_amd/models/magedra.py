@@ -490,7 +490,7 @@ class MagedraLM:
         m: SegMeta = inp.attn
         T, d, eps, S = inp.tokens.shape[0], cfg.hidden_size, cfg.norm_eps, self.S
         xs = torch.empty(S, T, d, dtype=torch.float32, device=dev)      # fp32 streams
-        e = F.embedding(inp.tokens, self.embed).unsqueeze(0)
+        e = ops.gather_rows(self.embed, inp.tokens).unsqueeze(0)
         hops.stream_step(e, read=self.one, norm_w=self.embed_norm, eps=eps, out=xs[0], center=True)
         if S > 1:
             xs[1:] = xs[0]

@@ -451,7 +451,7 @@ class MozidraLM:
         cfg, dt, dev = self.cfg, self.dtype, self.device
         m: SegMeta = inp.attn
         T, d, eps, S = inp.tokens.shape[0], cfg.hidden_size, cfg.norm_eps, self.S
-        xs = F.embedding(inp.tokens, self.embed).unsqueeze(0).repeat(S, 1, 1)   # fp32 [S, T, d] streams
+        xs = ops.gather_rows(self.embed, inp.tokens).unsqueeze(0).repeat(S, 1, 1)   # fp32 [S, T, d] streams
         h = torch.empty(T, d, dtype=dt, device=dev)
         step = {}   # what later layers of this step read from earlier ones (the first value-mixing layer's values)
         if self.layers:

@@ -473,7 +473,7 @@ class RogosunLM:
         cfg, dt, dev = self.cfg, self.dtype, self.device
         m: SegMeta = inp.attn
         d, eps = cfg.hidden_size, cfg.norm_eps
-        x = F.embedding(inp.tokens, self.embed)       # fp32 [T, d] residual
+        x = ops.gather_rows(self.embed, inp.tokens)       # fp32 [T, d] residual
         h = torch.empty(x.shape, dtype=dt, device=dev)
         h.copy_(x)                                    # what the sublayers read: x in the model dtype
         for i, lw in enumerate(self.layers):
@@ -492,7 +492,7 @@ class RogosunLM:
                 hops.norm_add(x, y1, y2, lw.norm2, eps, None if last else h)
             if layers_out is not None:
                 layers_out.append(x.clone())
-        xs = x.index_select(0, inp.logit_rows)
+        xs = ops.gather_rows(x, inp.logit_rows)
         hf = torch.empty(xs.shape[0], d, dtype=dt, device=dev)
         hops.rms_norm(xs, self.final_norm, eps, hf)
         return self._lin(hf, self.head, getattr(self, "head_t", None)).float()[:, :cfg.vocab_size]

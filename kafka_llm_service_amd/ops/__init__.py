@@ -67,6 +67,46 @@ def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, w: torch.Tensor, 
     return out
 
 
+def _whole_rows(t: torch.Tensor) -> bool:
+    """GPU rows of whole, aligned 16-byte pieces."""
+    e = t.element_size()
+    return t.is_cuda and t.dim() >= 2 and t.stride(-1) == 1 and t.shape[-1] * e % 16 == 0 and t.stride(-2) * e % 16 == 0 and \
+        t.data_ptr() % 16 == 0
+
+
+def embed_rmsnorm(table: torch.Tensor, tokens: torch.Tensor, w: torch.Tensor, eps: float) -> tuple[torch.Tensor, torch.Tensor]:
+    """(rows = table[tokens], rmsnorm(rows) * w), both new: a step's residual stream and its first layer's input."""
+    n, d = tokens.shape[0], table.shape[1]
+    if n and _whole_rows(table) and table.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and d <= 16384:
+        r = torch.empty(n, d, dtype=table.dtype, device=table.device)
+        x = torch.empty_like(r)
+        ext().rows_norm(x, table, r, tokens, w, float(eps), True)
+        return r, x
+    r = torch.nn.functional.embedding(tokens, table)
+    return r, rmsnorm(r, w, eps)
+
+
+def rows_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, rows: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
+    """rmsnorm(x[rows] + residual[rows]) * w (``x`` bf16 or a slab); neither is written."""
+    slab = is_slab(x)
+    if rows.shape[0] and _whole_rows(x) and _whole_rows(residual) and residual.shape[1] <= 16384 and \
+            residual.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and (slab or x.dtype == torch.bfloat16):
+        out = torch.empty(rows.shape[0], residual.shape[1], dtype=residual.dtype, device=x.device)
+        ext().rows_norm(out, x, residual, rows, w, float(eps), False)
+        return out
+    return fused_add_rmsnorm(x.index_select(1 if slab else 0, rows), residual.index_select(0, rows), w, eps)
+
+
+def gather_rows(table: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
+    """table[idx] for rows of a matrix (fp32 or bf16) and int64 indices."""
+    if idx.shape[0] and table.dim() == 2 and _whole_rows(table) and table.dtype in (torch.float32, torch.bfloat16) and \
+            table.shape[1] * table.element_size() < 1 << 24:
+        out = torch.empty(idx.shape[0], table.shape[1], dtype=table.dtype, device=table.device)
+        ext().gather_rows(out, table, idx)
+        return out
+    return table.index_select(0, idx)
+
+
 def silu_mul(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """silu(x[..., :F]) * x[..., F:] (bf16 out); ``x`` may be a split-K slab [S, T, 2F]."""
     F = x.shape[-1] // 2

@@ -14,6 +14,11 @@ hipError_t kafka_launch_fused_add_rmsnorm(bf16* out, int64_t os, const bf16* x, 
                                     const bf16* w, int T, int d, float eps, hipStream_t st);
 hipError_t kafka_launch_fused_add_rmsnorm_slab(bf16* out, int64_t os, const float* xp, int S, int64_t ps, bf16* resid,
                                                int64_t rs, const bf16* w, int T, int d, float eps, hipStream_t st);
+hipError_t kafka_launch_rows_norm(bf16* out, int64_t os, const bf16* x, int64_t xs, const float* xp, int S, int64_t ps, bf16* resid,
+                                  int64_t rs, const int64_t* idx, int64_t n_src, const bf16* w, int n, int d, float eps, int embed,
+                                  hipStream_t st);
+hipError_t kafka_launch_gather_rows(void* out, int64_t out_bytes, const void* src, int64_t src_bytes, const int64_t* idx,
+                                    int64_t n_src, int n, int row_bytes, hipStream_t st);
 hipError_t kafka_launch_silu_mul(bf16* out, const bf16* x, int64_t xs, int T, int F, hipStream_t st);
 hipError_t kafka_launch_silu_mul_slab(bf16* out, const float* xp, int S, int64_t ps, int T, int F, hipStream_t st);
 hipError_t kafka_launch_rope_kv(const bf16* qkv, const float* qp, int S, int64_t ps, int64_t qkv_stride,
@@ -181,6 +186,41 @@ static void fused_add_rmsnorm(at::Tensor out, at::Tensor x, at::Tensor residual,
   else
     CHECK_HIP(kafka_launch_fused_add_rmsnorm(bptr(out), out.stride(0), bptr(x), x.stride(0), bptr(residual),
                                               residual.stride(0), bptr(w), T, d, eps, cur_stream()));
+}
+
+// Rows picked by idx (int64 [n]) with a norm. embed: residual[i] = x[idx[i]] (x a table [V, d]), out[i] = norm of it; else
+// out[i] = norm(x[idx[i]] + residual[idx[i]]), x bf16 [T, d] or slab [S, T, d], residual [T, d]
+static void rows_norm(at::Tensor out, at::Tensor x, at::Tensor residual, at::Tensor idx, at::Tensor w, double eps, bool embed) {
+  CHECK_CUDA(x); CHECK_CUDA(out); CHECK_CUDA(residual); CHECK_CUDA(idx);
+  CHECK_DT(residual, at::kBFloat16); CHECK_DT(w, at::kBFloat16); CHECK_DT(out, at::kBFloat16); CHECK_DT(idx, at::kLong);
+  CHECK_LASTDIM(x); CHECK_LASTDIM(out); CHECK_LASTDIM(residual);
+  const bool slab = is_slab(x);
+  if (slab) check_slab(x); else CHECK_DT(x, at::kBFloat16);
+  TORCH_CHECK((slab || x.dim() == 2) && residual.dim() == 2 && out.dim() == 2 && idx.dim() == 1 && idx.is_contiguous() &&
+                  w.is_contiguous() && !(embed && slab), "rows_norm: operands");
+  const int64_t n_src = x.size(slab ? 1 : 0), n = idx.size(0);
+  const int d = x.size(slab ? 2 : 1);
+  auto al = [](const at::Tensor& t) { return t.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  TORCH_CHECK(d % 8 == 0 && d <= 16384 && w.numel() == d && residual.size(1) == d && residual.size(0) == (embed ? n : n_src) &&
+                  out.size(0) == n && out.size(1) == d && al(out) && al(residual) && (slab || al(x)) &&
+                  reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 && n_src > 0, "rows_norm: bad shapes");
+  CHECK_HIP(kafka_launch_rows_norm(bptr(out), out.stride(0), slab ? nullptr : bptr(x), slab ? d : x.stride(0),
+                                   slab ? x.data_ptr<float>() : nullptr, slab ? (int)x.size(0) : 0, n_src * d, bptr(residual),
+                                   residual.stride(0), idx.data_ptr<int64_t>(), n_src, bptr(w), (int)n, d, eps, embed ? 1 : 0,
+                                   cur_stream()));
+}
+
+// out[i] = src[idx[i]]: fp32 or bf16 rows of whole 16-byte pieces
+static void gather_rows(at::Tensor out, at::Tensor src, at::Tensor idx) {
+  CHECK_CUDA(src); CHECK_CUDA(out); CHECK_CUDA(idx); CHECK_DT(idx, at::kLong); CHECK_LASTDIM(src); CHECK_LASTDIM(out);
+  TORCH_CHECK(src.dim() == 2 && out.dim() == 2 && idx.dim() == 1 && idx.is_contiguous() && src.scalar_type() == out.scalar_type() &&
+                  (src.scalar_type() == at::kFloat || src.scalar_type() == at::kBFloat16) && out.size(0) == idx.size(0) &&
+                  out.size(1) == src.size(1) && src.size(0) > 0, "gather_rows: operands");
+  const int64_t e = src.element_size(), row = src.size(1) * e;
+  auto al = [&](const at::Tensor& t) { return t.stride(0) * e % 16 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  TORCH_CHECK(row % 16 == 0 && row > 0 && row < (1 << 24) && al(src) && al(out), "gather_rows: rows of whole 16-byte pieces");
+  CHECK_HIP(kafka_launch_gather_rows(out.data_ptr(), out.stride(0) * e, src.data_ptr(), src.stride(0) * e, idx.data_ptr<int64_t>(),
+                                     src.size(0), (int)idx.size(0), (int)row, cur_stream()));
 }
 
 // x: bf16 [T, 2F] or slab [S, T, 2F]
@@ -1162,6 +1202,8 @@ PYBIND11_MODULE(_kafka_ops, m) {
   kafka_bind_hybrid(m);
   m.def("rmsnorm", &rmsnorm);
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
+  m.def("rows_norm", &rows_norm);
+  m.def("gather_rows", &gather_rows);
   m.def("silu_mul", &silu_mul);
   m.def("rope_kv_write", &rope_kv_write);
   m.def("attn_decode", &attn_decode, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),

@@ -1,0 +1,43 @@
+"""Rows picked by an index, with and without a norm (csrc/norm_act.hip: ops.embed_rmsnorm, rows_add_rmsnorm, gather_rows)."""
+import pytest
+import torch
+
+from kafka_llm_service_amd import ops
+
+
+def _check(dev, dtype):
+    """The same as the separate operations, to the last bit (on the GPU the same sums and roundings)."""
+    g = torch.Generator().manual_seed(2)
+    for d, n in ((64, 3), (2048, 1), (4096, 7), (5120, 2), (16384, 2)):
+        table = torch.randn(11, d, generator=g).to(dtype).to(dev)
+        w = torch.rand(d, generator=g).to(dtype).to(dev)
+        idx = torch.randint(0, 11, (n,), generator=g).to(dev)
+        r, x = ops.embed_rmsnorm(table, idx, w, 1e-5)
+        assert torch.equal(r, table[idx]) and torch.equal(x, ops.rmsnorm(table[idx], w, 1e-5))
+        res = torch.randn(11, d, generator=g).to(dtype).to(dev)
+        for delta in [torch.randn(11, d, generator=g).to(dtype)] + [torch.randn(s, 11, d, generator=g) for s in (1, 2, 3, 8)]:
+            delta, keep = delta.to(dev), res.clone()
+            slab = ops.is_slab(delta)
+            want = ops.fused_add_rmsnorm(delta.index_select(1 if slab else 0, idx), res.index_select(0, idx), w, 1e-5)
+            assert torch.equal(ops.rows_add_rmsnorm(delta, res, idx, w, 1e-5), want) and torch.equal(res, keep)
+        for t in (table, table.float(), torch.randn(11, d + 8, generator=g).to(dev)[:, :d], torch.randn(11, d + 1, generator=g).to(dev)[:, 1:]):
+            assert torch.equal(ops.gather_rows(t, idx), t[idx])
+    none = torch.zeros(0, dtype=torch.int64, device=dev)
+    assert ops.gather_rows(table, none).shape == (0, 16384) and ops.rows_add_rmsnorm(table, res, none, w, 1e-5).shape == (0, 16384)
+
+
+def test_on_the_cpu():
+    _check("cpu", torch.float32)
+
+
+@pytest.mark.gpu
+def test_on_the_gpu():
+    _check("cuda", torch.bfloat16)
+    table, w = torch.randn(5, 4096, device="cuda").to(torch.bfloat16), torch.ones(4096, device="cuda", dtype=torch.bfloat16)
+    idx = torch.tensor([4, 5, -1, 0], device="cuda")    # rows outside the table come out as NaN, the others as they are
+    r, x = ops.embed_rmsnorm(table, idx, w, 1e-5)
+    f = ops.gather_rows(table.float(), idx)
+    y = ops.rows_add_rmsnorm(table, table, idx, w, 1e-5)
+    for t in (r, x, f, y):
+        assert torch.isnan(t[1:3]).all() and torch.isfinite(t[0]).all() and torch.isfinite(t[3]).all()
+    assert torch.equal(r[[0, 3]], table[[4, 0]])

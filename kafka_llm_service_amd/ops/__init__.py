@@ -67,17 +67,17 @@ def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, w: torch.Tensor, 
     return out
 
 
-def _whole_rows(t: torch.Tensor) -> bool:
-    """GPU rows of whole, aligned 16-byte pieces."""
+def _whole_rows(t: torch.Tensor, idx: torch.Tensor) -> bool:
+    """GPU rows of whole, aligned 16-byte pieces, and an index that the row kernels read as it lies."""
     e = t.element_size()
-    return t.is_cuda and t.dim() >= 2 and t.stride(-1) == 1 and t.shape[-1] * e % 16 == 0 and t.stride(-2) * e % 16 == 0 and \
+    return t.is_cuda and idx.is_cuda and idx.dtype == torch.int64 and idx.dim() == 1 and idx.is_contiguous() and t.dim() >= 2 and t.stride(-1) == 1 and t.shape[-1] * e % 16 == 0 and t.stride(-2) * e % 16 == 0 and \
         t.data_ptr() % 16 == 0
 
 
 def embed_rmsnorm(table: torch.Tensor, tokens: torch.Tensor, w: torch.Tensor, eps: float) -> tuple[torch.Tensor, torch.Tensor]:
     """(rows = table[tokens], rmsnorm(rows) * w), both new: a step's residual stream and its first layer's input."""
     n, d = tokens.shape[0], table.shape[1]
-    if n and _whole_rows(table) and table.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and d <= 16384:
+    if n and _whole_rows(table, tokens) and table.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and d <= 16384:
         r = torch.empty(n, d, dtype=table.dtype, device=table.device)
         x = torch.empty_like(r)
         ext().rows_norm(x, table, r, tokens, w, float(eps), True)
@@ -89,7 +89,7 @@ def embed_rmsnorm(table: torch.Tensor, tokens: torch.Tensor, w: torch.Tensor, ep
 def rows_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, rows: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     """rmsnorm(x[rows] + residual[rows]) * w (``x`` bf16 or a slab); neither is written."""
     slab = is_slab(x)
-    if rows.shape[0] and _whole_rows(x) and _whole_rows(residual) and residual.shape[1] <= 16384 and \
+    if rows.shape[0] and _whole_rows(x, rows) and _whole_rows(residual, rows) and residual.shape[1] <= 16384 and \
             residual.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and (slab or x.dtype == torch.bfloat16):
         out = torch.empty(rows.shape[0], residual.shape[1], dtype=residual.dtype, device=x.device)
         ext().rows_norm(out, x, residual, rows, w, float(eps), False)
@@ -98,8 +98,8 @@ def rows_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, rows: torch.Tensor
 
 
 def gather_rows(table: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
-    """table[idx] for rows of a matrix (fp32 or bf16) and int64 indices."""
-    if idx.shape[0] and table.dim() == 2 and _whole_rows(table) and table.dtype in (torch.float32, torch.bfloat16) and \
+    """table[idx] for rows of a matrix."""
+    if idx.shape[0] and table.dim() == 2 and _whole_rows(table, idx) and table.dtype in (torch.float32, torch.bfloat16) and \
             table.shape[1] * table.element_size() < 1 << 24:
         out = torch.empty(idx.shape[0], table.shape[1], dtype=table.dtype, device=table.device)
         ext().gather_rows(out, table, idx)

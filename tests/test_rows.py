@@ -22,6 +22,9 @@ def _check(dev, dtype):
             assert torch.equal(ops.rows_add_rmsnorm(delta, res, idx, w, 1e-5), want) and torch.equal(res, keep)
         for t in (table, table.float(), torch.randn(11, d + 8, generator=g).to(dev)[:, :d], torch.randn(11, d + 1, generator=g).to(dev)[:, 1:]):
             assert torch.equal(ops.gather_rows(t, idx), t[idx])
+    for i in (idx.int(), idx.repeat_interleave(2)[::2]):     # indices that the kernels do not read
+        assert torch.equal(ops.gather_rows(table, i), table[idx]) and torch.equal(ops.embed_rmsnorm(table, i, w, 1e-5)[0], table[idx])
+        assert torch.equal(ops.rows_add_rmsnorm(table, res, i, w, 1e-5), ops.rows_add_rmsnorm(table, res, idx, w, 1e-5))
     none = torch.zeros(0, dtype=torch.int64, device=dev)
     assert ops.gather_rows(table, none).shape == (0, 16384) and ops.rows_add_rmsnorm(table, res, none, w, 1e-5).shape == (0, 16384)
 

@@ -42,6 +42,8 @@ def test_against_fp32(K):
         ops.ext().small_gemm(x, w, f, b)
         assert ((f - want - b).abs() <= 2e-5).all()
         assert ((hops.linear_f32(x, w.contiguous(), b) - want - b).abs() <= 2e-5).all()
+        o = torch.randn(N + 1, generator=g).cuda()[1:]      # (a bias that starts between two 16-byte pieces)
+        assert ((hops.linear_f32(x, w.contiguous(), o) - want - o).abs() <= 2e-5).all()
         _close(ops.linear_small(x, w), want)
 
 

@@ -382,6 +382,7 @@ TILES = {(8, 8): (3.3, 7.6, 1.24, 0.64), (8, 6): (3.7, 4.6, 0.96, 0.82), (6, 8):
 TILE_SPLITS = (1, 2, 4, 8)      # what the consumers of slabs load with all slabs in flight
 TILE_SLAB_BYTES = 1 << 28
 TILE_LIBRARY_N, TILE_MAX_M = 24576, 2560
+TILE_GLU_M, TILE_EVEN_M, TILE_RAGGED_M = 3600, 5600, 8448
 
 
 @lru_cache(maxsize=4096)
@@ -394,13 +395,26 @@ def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) 
     200 rows 57 / 45; 900 rows of 2048 -> 9344 45 / 36; 450 rows of 2048 -> 2048 19 / 11; over all timed shapes 13 % less time with slabs,
     9 % as bf16. The library's: very wide outputs of 257 - 1024 rows (28672 columns: 320 rows 74 / 78, 640 135 / 149); beyond
     them, where its 256 x 256 tiles (1.42 us a round and 64 of K) fill their rounds (28672: 1536 rows 264 / 293, 4099 722 / 774; 2048 -> 7168,
-    2048 rows 49 / 62), which ragged columns (no multiple of 256) do not (10816: 2048 rows 164 / 151); and beyond 2560 rows: the
-    longer the card is busy the lower its clock, and the library takes less power (a step of 4099 rows 6387 / 6587, of 8192 its products
-    2935 / 3276, of 2750 the same)."""
+    2048 rows 49 / 62), which ragged columns (no multiple of 256) do not (10816: 2048 rows 164 / 151).
+
+    Beyond 2560 rows the library's choice of kernel decides. Where its tiles are one round or less it is as fast or faster (4096 -> 4096: 2716 rows
+    73 / 74, 4096 91 / 100). Beyond a round ragged columns take this kernel (4096 -> 18560: 3182 rows 500 / 378, 4096 560 / 461; 12320: 2593 333 /
+    221, 7583 538 / 576; 2048 -> 9344: 4096 180 / 155; over 130 sizes up to 8192 rows 9 % less time), whole ones up to 5600 rows where the model says
+    a fifth less (6144: 2716 rows 205 / 120, 4096 158 / 156; over 28 sizes 9 % less, the others 6 % more). Gate and up with their
+    activation: up to 3600 rows from two rounds on (28672: 2716 rows 593 / 508, 3182 716 / 596, 3600 - 4200 3 % more; 4096 -> 9216, less
+    than two rounds, 5 % more). Steps: llama 2700 rows 5030 -> 4400, 3000 4930 -> 4790, 3300 6050 -> 5480; rogosun 4000 8740 -> 8570, width 2048 2700
+    2925 -> 2860; budurax width 2048 2700 2280 -> 2208; furapel 6400 15235 -> 15020."""
     if M < 1 or N % 32 or N < 32 or K % 64 or K < 128 or N * K * 2 > 0xffff0000 or (form == "glu" and N % 64):
         return None
-    if library and (M > TILE_MAX_M or form == "bf16" and N > TILE_LIBRARY_N and 256 < M <= 1024):
+    if library and form == "bf16" and N > TILE_LIBRARY_N and 256 < M <= 1024:
         return None
+    gain = 1.25 if N % 256 else 0.95
+    if library and M > TILE_MAX_M:
+        tiles = -(-M // 256) * -(-N // 256)
+        if M > (TILE_GLU_M if form == "glu" else TILE_RAGGED_M if N % 256 else TILE_EVEN_M) or tiles <= (512 if form == "glu" else 256):
+            return None
+        if form != "glu" and N % 256 == 0:
+            gain = 0.8
     best = None
     for (mt, nt), (launch, rnd, unit, out) in TILES.items():
         if form == "glu" and nt % 4:
@@ -420,7 +434,7 @@ def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) 
         lib = 4 + -(-(-(-rows // 256) * -(-N // 256)) // 256) * 1.42 * (K // 64) + (20 if rows < M else 0)
         if form == "glu":           # (the activation's launch and its way to memory and back)
             lib += 5 + 3 * M * N / 4.5e6
-        if best[0] > lib * (1.25 if N % 256 else 0.95):
+        if best[0] > lib * gain:
             return None
     return best[1]
 

@@ -23,6 +23,12 @@ def test_plans_are_launches():
         assert s == 1 or 4 * s * M * N <= ops.TILE_SLAB_BYTES
     assert ops.tile_plan(300, 4100, 4096) is None and ops.tile_plan(300, 4096, 64) is None and ops.tile_plan(300, 4096, 4112) is None
     assert ops.tile_plan(0, 4096, 4096) is None and ops.tile_plan(300, 32800, 65536, library=False) is None   # 4 GB of weights
+    for M, N, form, taken in ((2561, 6176, "bf16", True), (8448, 6176, "slabs", True), (8449, 6176, "bf16", False),   # ragged columns
+                              (2561, 6144, "bf16", True), (5600, 9216, "bf16", False), (2700, 28672, "bf16", False),   # whole ones: a fifth less
+                              (4096, 4064, "bf16", False), (2816, 5920, "bf16", True),      # one round of 256 x 256 tiles, and a bit more
+                              (2561, 28672, "glu", True), (3600, 28672, "glu", True), (3601, 28672, "glu", False),
+                              (2816, 11776, "glu", False)):                             # two rounds
+        assert (ops.tile_plan(M, N, 4096, form) is not None) == taken, (M, N, form)
     assert ops.tile_plan(300, 28672, 4096) is None and ops.tile_plan(300, 28672, 4096, "glu") is not None
 
 
@@ -76,7 +82,8 @@ def test_long_products_by_their_plans():
     """linear_long and linear_glu_long over sizes of every route (tiles with and without splits, the library) and forms of x that the
     kernel leaves to the library (odd strides, a shifted start)."""
     g = torch.Generator().manual_seed(0)
-    for M, N, K in ((131, 2048, 2048), (300, 4096, 1024), (700, 96, 4096), (1300, 6176, 512), (257, 24608, 128), (3000, 1024, 256)):
+    for M, N, K in ((131, 2048, 2048), (300, 4096, 1024), (700, 96, 4096), (1300, 6176, 512), (257, 24608, 128), (3000, 1024, 256),
+                    (2561, 6176, 256), (2600, 6144, 512)):
         w = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
         wt = ops.tile_weight(w)
         base = torch.randn(M, K + 16, generator=g).to(torch.bfloat16).cuda()

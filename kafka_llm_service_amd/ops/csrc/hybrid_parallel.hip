@@ -16,6 +16,7 @@
 //                   optional mix of the queries over the heads (so that one product with the whole key row gives the
 //                   head-mixed score), paged key / transposed value store; the values may be the raw key columns
 #include "common.h"
+#include "page_values.h"
 
 namespace kafka {
 namespace hp {
@@ -498,65 +499,97 @@ __global__ __launch_bounds__(NT) void rope_kv_store_kernel(
   }
 }
 
-// The same for bf16 rows whose values are the key columns, without a head mix: L = D / 8 lanes per (row, query or key
-// head), a lane holds 8 consecutive elements in registers; the rotation's partner is dims / 16 lanes away. Everything in
-// 16-byte pieces (the page-wise transposed values element by element). D = 8 L with L a power of two, dims % 16 == 0.
-template <int L>
+// The same for bf16 rows without a head mix, values as wide as keys: L = D / 8 lanes per (row, U heads), a lane holds 8
+// consecutive elements of each in registers; the rotation's partner is dims / 16 lanes away. Heads are the query heads, the key heads
+// and the value heads: the key heads again where keys double as values (VH false), columns of their own from v_off on (VH). Everything in 16-byte
+// pieces, but the page-wise transposed values element by element. With ``pages`` a wave per row (the last blocks) stores
+// the values by whole pages instead (page_values.h). D = 8 L with L a power of two, dims % 16 == 0.
+// us, 32 + 8 heads of 128, LDS kernel / this one: 4 rows 7.9 / 5.6, 200 9.1 / 5.8, 700 14.8 / 7.6, 1100 16.4 / 8.9, 8192 116 / 34 (5 TB/s); 32 + 2 heads whose keys double as
+// values, one head a lane and values one by one / this one: 2805 rows 16.6 / 14.0, 8192 51.6 / 33.8.
+template <int L, int U, bool VH>
 __global__ __launch_bounds__(NT) void rope_kv_store_vec8_kernel(
     const bf16* __restrict__ qkv, int64_t qs, int H, int G, const int64_t* __restrict__ positions,
     const float* __restrict__ cos_sin, int dims, const float* __restrict__ qn, const float* __restrict__ kn, float eps,
-    bf16* __restrict__ kc, bf16* __restrict__ vt, const int64_t* __restrict__ slots, bf16* __restrict__ q_out,
-    int64_t qos, int64_t T) {
+    int v_off, bf16* __restrict__ kc, bf16* __restrict__ vt, const int64_t* __restrict__ slots, bf16* __restrict__ q_out,
+    int64_t qos, int64_t T, unsigned rope_blocks) {
   constexpr int D = 8 * L;
-  const int64_t u = (int64_t)blockIdx.x * (NT / L) + threadIdx.x / L;
-  if (u >= T * (H + G)) return;   // (whole groups of L lanes leave)
-  const int64_t t = u / (H + G);
-  const int hd = (int)(u - t * (H + G)), l = threadIdx.x % L;
-  const bf16x8 raw = load_bf16x8(qkv + t * qs + (int64_t)hd * D + 8 * l);
-  float x[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) x[j] = (float)raw[j];
-  if (qn != nullptr) {
-    const float* nw = (hd < H ? qn : kn) + 8 * l;
-    float s = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s += x[j] * x[j];
-#pragma unroll
-    for (int o = L / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, L);
-    const float rs = 1.0f / sqrtf(s / (float)D + eps);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = x[j] * rs * nw[j];
-  }
-  if (dims > 0) {   // (uniform)
-    const int hl = dims >> 4;   // lanes of a half
-    const bool lo = l < hl, in = l < 2 * hl;
-    const int pl = lo ? l + hl : in ? l - hl : l;
-    const float* cs = cos_sin + positions[t] * dims + 8 * (in ? (lo ? l : l - hl) : 0);
-    float y[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) y[j] = __shfl(x[j], pl, L);
-    if (in) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float c = cs[j], sn = cs[(dims >> 1) + j];
-        x[j] = lo ? x[j] * c - y[j] * sn : x[j] * c + y[j] * sn;
-      }
+  constexpr bool PAGES = U > 1;
+  if constexpr (PAGES) {
+    __shared__ __attribute__((aligned(16))) kafka::pv::Turn turn[NT / 64];
+    if (blockIdx.x >= rope_blocks) {
+      const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+      const int64_t t = (int64_t)(blockIdx.x - rope_blocks) * (NT / 64) + w;
+      if (t >= T) return;
+      const int64_t slot = slots[t], around = kafka::pv::near(slots, (int)t, (int)T, lane);
+      if (slot >= 0)
+        kafka::pv::store(qkv + v_off, qs, G * D, (int)t, (int)T, slot, around, vt, turn[w], lane, [](int k) { return k; });
+      return;
     }
   }
-  bf16x8 r;
+  const int nh = H + G + (VH && !PAGES ? G : 0), ng = (nh + U - 1) / U;
+  const int64_t u = (int64_t)blockIdx.x * (NT / L) + threadIdx.x / L;
+  if (u >= T * ng) return;   // (whole groups of L lanes leave)
+  const int64_t t = u / ng;
+  const int g = (int)(u - t * ng), l = threadIdx.x % L;
+  const bf16* row = qkv + t * qs + 8 * l;
+  bf16x8 raw[U];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) r[j] = (bf16)x[j];
-  if (hd < H) {
-    store_bf16x8(q_out + t * qos + (int64_t)hd * D + 8 * l, r);
-    return;
+  for (int i = 0; i < U; ++i) {
+    const int hd = min(g + i * ng, nh - 1);
+    raw[i] = load_bf16x8(row + (hd >= H + G ? v_off + (hd - H - G) * D : hd * D));
+  }
+  const int hl = dims >> 4;   // lanes of a half
+  const bool lo = l < hl, in = l < 2 * hl;
+  const int pl = lo ? l + hl : in ? l - hl : l;
+  float c[8], sn[8];
+  if (in) {
+    const float* cs = cos_sin + positions[t] * dims + 8 * (lo ? l : l - hl);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) c[j] = cs[j], sn[j] = cs[(dims >> 1) + j];
   }
   const int64_t slot = slots[t];
-  if (slot < 0) return;
-  const int c0 = (hd - H) * D + 8 * l;
-  store_bf16x8(kc + slot * ((int64_t)G * D) + c0, r);
-  bf16* vd = vt + ((slot / PAGE) * ((int64_t)G * D) + c0) * PAGE + (slot % PAGE);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) vd[(int64_t)j * PAGE] = raw[j];
+  for (int i = 0; i < U; ++i) {
+    const int hd = g + i * ng;   // (one head for the L lanes)
+    if (hd >= nh) break;
+    const bool value = hd >= H + G;
+    const int c0 = (hd - H - (value ? G : 0)) * D + 8 * l;
+    if (!value) {
+      float x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = (float)raw[i][j];
+      if (qn != nullptr) {
+        const float* nw = (hd < H ? qn : kn) + 8 * l;
+        float s = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s += x[j] * x[j];
+#pragma unroll
+        for (int o = L / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, L);
+        const float rs = 1.0f / sqrtf(s / (float)D + eps);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = x[j] * rs * nw[j];
+      }
+      if (dims > 0) {   // (uniform)
+        float y[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) y[j] = __shfl(x[j], pl, L);
+        if (in) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) x[j] = lo ? x[j] * c[j] - y[j] * sn[j] : x[j] * c[j] + y[j] * sn[j];
+        }
+      }
+      bf16x8 r;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) r[j] = (bf16)x[j];
+      if (hd < H) store_bf16x8(q_out + t * qos + (int64_t)hd * D + 8 * l, r);
+      else if (slot >= 0) store_bf16x8(kc + slot * ((int64_t)G * D) + c0, r);
+    }
+    if (!PAGES && hd >= (VH ? H + G : H) && slot >= 0) {
+      bf16* vd = vt + ((slot / PAGE) * ((int64_t)G * D) + c0) * PAGE + (slot % PAGE);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) vd[(int64_t)j * PAGE] = raw[i][j];
+    }
+  }
 }
 
 }  // namespace hp
@@ -671,6 +704,8 @@ hipError_t kafka_hy_hgrn2_combine(const int* cs, int R, const float* F, int HD, 
 
 int kafka_hy_rope_store_max_q() { return 15360; }   // floats of LDS: H D + G D + rot dims (+ H H with a head mix)
 
+constexpr int64_t ROPE_FEW = 1 << 18;
+
 hipError_t kafka_hy_rope_kv_store(int f32, const void* qkv, int64_t qs, int H, int G, int D, int Dv,
                                   const int64_t* positions, const float* cos_sin, int dims, int pairs,
                                   const float* talk, const float* qn, const float* kn, float eps, int v_off, void* kc,
@@ -682,22 +717,33 @@ hipError_t kafka_hy_rope_kv_store(int f32, const void* qkv, int64_t qs, int H, i
   {
     auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     const int L = D / 8;
-    if (!f32 && talk == nullptr && !pairs && v_off == H * D && Dv == D && D % 8 == 0 && L <= 64 && (L & (L - 1)) == 0 &&
+    const bool vh = v_off != H * D;   // (values in columns of their own)
+    if (!f32 && talk == nullptr && !pairs && v_off % 8 == 0 && Dv == D && D % 8 == 0 && L <= 64 && (L & (L - 1)) == 0 &&
         dims % 16 == 0 && qs % 8 == 0 && qos % 8 == 0 && al(qkv) && al(q_out) && al(kc)) {
-      const unsigned grid = (unsigned)((T * (H + G) * L + NT - 1) / NT);
-      auto a = [&](auto k) {
-        k<<<grid, NT, 0, st>>>((const bf16*)qkv, qs, H, G, positions, cos_sin, dims, qn, kn, eps, (bf16*)kc, (bf16*)vt,
-                               slots, (bf16*)q_out, qos, T);
+      // four heads a lane and values by pages from where one head a lane is half as many waves as the chip has places for; where keys double as
+      // values, that many (one / four heads a lane: 700 rows of 32 + 2 heads 6.9 / 8.0 us, 1100 9.0 / 8.5)
+      const bool few = T * (H + G) * L < (vh ? ROPE_FEW : 2 * ROPE_FEW) || !al(vt) || T > 1 << 28;
+      auto a = [&](auto k, int u) {
+        const int64_t ng = (H + G + (vh && few ? G : 0) + u - 1) / u;
+        const unsigned blocks = (unsigned)((T * ng * L + NT - 1) / NT), values = few ? 0 : (unsigned)((T + NT / 64 - 1) / (NT / 64));
+        k<<<blocks + values, NT, 0, st>>>((const bf16*)qkv, qs, H, G, positions, cos_sin, dims, qn, kn, eps, v_off, (bf16*)kc,
+                                          (bf16*)vt, slots, (bf16*)q_out, qos, T, blocks);
       };
+#define ROPE_L(L_)                                                                                                    \
+  case L_:                                                                                                            \
+    if (few) vh ? a(rope_kv_store_vec8_kernel<L_, 1, true>, 1) : a(rope_kv_store_vec8_kernel<L_, 1, false>, 1);  \
+    else a(rope_kv_store_vec8_kernel<L_, 4, false>, 4);                                                              \
+    break
       switch (L) {
-        case 1: a(rope_kv_store_vec8_kernel<1>); break;
-        case 2: a(rope_kv_store_vec8_kernel<2>); break;
-        case 4: a(rope_kv_store_vec8_kernel<4>); break;
-        case 8: a(rope_kv_store_vec8_kernel<8>); break;
-        case 16: a(rope_kv_store_vec8_kernel<16>); break;
-        case 32: a(rope_kv_store_vec8_kernel<32>); break;
-        default: a(rope_kv_store_vec8_kernel<64>); break;
+        ROPE_L(1);
+        ROPE_L(2);
+        ROPE_L(4);
+        ROPE_L(8);
+        ROPE_L(16);
+        ROPE_L(32);
+        ROPE_L(64);
       }
+#undef ROPE_L
       return hipGetLastError();
     }
   }

@@ -27,6 +27,7 @@
 #include <cstdlib>
 
 #include "common.h"
+#include "page_values.h"
 
 namespace kafka {
 
@@ -100,6 +101,68 @@ __global__ __launch_bounds__(1024) void rope_kv_kernel(const bf16* __restrict__ 
       for (int j = 0; j < 8; ++j) dst[(int64_t)(c + j) * block_size] = (bf16)x[j];
     }
   }
+}
+
+// The same for long steps of bf16 rows, pages of 16: a wave per row, which reads its position's cos and sin once and asks for five
+// heads a lane together; values by whole pages (page_values.h). What bounds the kernel above at such sizes is its seven
+// waves a row (28700 of one wave each at 4099 rows, 3.5 rounds of the chip's places, each a chain of three round trips) and the
+// two-byte stores. us, 32 + 8 heads of 128: 512 rows 8.2 / 5.8, 1100 13.9 / 9.2, 1900 21.0 / 10.7, 4099 50.6 / 22.0 (4.6 TB/s; 35.8 with values
+// one by one), 8192 106 / 37; 16 + 4 heads: 512 6.3 / 4.8, 4099 21.7 / 10.4.
+template <int D>
+__global__ __launch_bounds__(256) void rope_kv_rows_kernel(const bf16* __restrict__ qkv, int64_t qkv_stride,
+                                                           const int64_t* __restrict__ positions,
+                                                           const float* __restrict__ cos_sin, bf16* __restrict__ q_out,
+                                                           int64_t q_stride, bf16* __restrict__ k_cache,
+                                                           bf16* __restrict__ v_cache, const int64_t* __restrict__ slot_mapping,
+                                                           int T, int Hq, int Hkv) {
+  constexpr int HALF = D / 2, RU = HALF / 8, HW = 64 / RU, HB = 5;
+  __shared__ __attribute__((aligned(16))) pv::Turn turn[4];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int t = blockIdx.x * 4 + w;
+  if (t >= T) return;
+  const int64_t pos = positions[t], slot = slot_mapping ? slot_mapping[t] : -1;
+  const int64_t around = slot_mapping ? pv::near(slot_mapping, t, T, lane) : -1;
+  const bf16* row = qkv + (int64_t)t * qkv_stride;
+  const int n = Hq + Hkv, c = (lane % RU) * 8;
+  const int64_t blk = slot >= 0 ? slot >> 4 : 0;
+  const int off = slot >= 0 ? (int)(slot & 15) : 0;
+  const float* cs = cos_sin + pos * D + c;
+  const f32x4 c0 = *reinterpret_cast<const f32x4*>(cs), c1 = *reinterpret_cast<const f32x4*>(cs + 4);
+  const f32x4 s0 = *reinterpret_cast<const f32x4*>(cs + HALF), s1 = *reinterpret_cast<const f32x4*>(cs + HALF + 4);
+  const float cv[8] = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
+  const float sv[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
+  for (int h0 = lane / RU; h0 < n; h0 += HB * HW) {
+    bf16x8 x1[HB], x2[HB];
+#pragma unroll
+    for (int i = 0; i < HB; ++i) {
+      const bf16* p = row + min(h0 + i * HW, n - 1) * D + c;
+      x1[i] = load_bf16x8(p);
+      x2[i] = load_bf16x8(p + HALF);
+    }
+#pragma unroll
+    for (int i = 0; i < HB; ++i) {
+      const int head = h0 + i * HW;
+      if (head >= n) break;
+      bf16x8 o1, o2;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float a = (float)x1[i][j], b = (float)x2[i][j];
+        o1[j] = (bf16)(a * cv[j] - b * sv[j]);
+        o2[j] = (bf16)(b * cv[j] + a * sv[j]);
+      }
+      if (head < Hq) {
+        bf16* dst = q_out + t * q_stride + head * D;
+        store_bf16x8(dst + c, o1);
+        store_bf16x8(dst + HALF + c, o2);
+      } else if (slot >= 0) {
+        bf16* dst = k_cache + (blk * Hkv + head - Hq) * (int64_t)16 * D + off * 8;
+        store_bf16x8(dst + (c >> 3) * 128, o1);
+        store_bf16x8(dst + ((HALF + c) >> 3) * 128, o2);
+      }
+    }
+  }
+  if (slot >= 0)
+    pv::store(qkv + n * D, qkv_stride, Hkv * D, t, T, slot, around, v_cache, turn[w], lane, [](int k) { return vt_pos(k); });
 }
 
 constexpr int KPAGE8 = 16 * 128 + 32;
@@ -239,6 +302,8 @@ extern "C" hipError_t kafka_launch_rope_kv_fp8(const bf16* qkv, const float* qp,
   return hipGetLastError();
 }
 
+constexpr int ROWS_MIN = 384;   // (of few rows a wave each leaves CUs idle; 512 rows 8.2 / 5.8 us)
+
 // qp != nullptr: the input is S fp32 slabs [S][T][(Hq + 2 Hkv) D] (slab stride ps) instead of bf16 qkv
 extern "C" hipError_t kafka_launch_rope_kv(const bf16* qkv, const float* qp, int S, int64_t ps, int64_t qkv_stride,
                                           const int64_t* positions, const float* cos_sin, bf16* q_out,
@@ -260,6 +325,13 @@ extern "C" hipError_t kafka_launch_rope_kv(const bf16* qkv, const float* qp, int
     const char* e = getenv("KAFKA_SC1_ROPE");
     return e == nullptr || e[0] != '0';
   }();
+  if (qp == nullptr && T >= ROWS_MIN && block_size == 16 && reinterpret_cast<uintptr_t>(v_cache) % 16 == 0) {
+    auto go = [&](auto kern) {
+      kern<<<(T + 3) / 4, 256, 0, st>>>(qkv, qkv_stride, positions, cos_sin, q_out, q_stride, k_cache, v_cache, slot_mapping, T, Hq, Hkv);
+      return hipGetLastError();
+    };
+    return D == 64 ? go(rope_kv_rows_kernel<64>) : go(rope_kv_rows_kernel<128>);
+  }
   if (D == 128 && sc1 && q_stride % 8 == 0)
     rope_kv_kernel<128, true><<<grid, nt, 0, st>>>(qkv, qp, S, ps, qkv_stride, positions, cos_sin, q_out, q_stride,
                                                 k_cache, v_cache, slot_mapping, Hq, Hkv, block_size);

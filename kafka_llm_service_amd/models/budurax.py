@@ -376,15 +376,16 @@ class BuduraxLM:
         self.stream_max_m = ops.STREAM_MAX_M
         return added
 
-    def _lin(self, x, w, wt=None):
+    def _lin(self, x, w, wt=None, slabs: bool = False):
         """x @ w^T: the weight-streaming kernel for decode-sized steps when the weight has a tiled copy (its split-K
-        slabs summed to bf16 by slab_reduce), else the tile kernel or the library (ops.linear_long)."""
+        slabs summed to bf16 by slab_reduce), else the tile kernel or the library (ops.linear_long). ``slabs``: the caller
+        takes the split-K slabs [S, T, N] as they are."""
         M = x.shape[0]
         if self.stream and wt is not None and 0 < M <= self.stream_max_m and \
                 ops.stream_plan(M, w.shape[0], w.shape[1]) is not None:
             y = ops.linear_stream(x, wt)
-            return ops.slab_reduce(y) if ops.is_slab(y) else y
-        return ops.linear_long(x, w, wt if self.stream else None)
+            return ops.slab_reduce(y) if ops.is_slab(y) and not slabs else y
+        return ops.linear_long(x, w, wt if self.stream else None, slabs)
 
     def weight_bytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self._tensors)
@@ -561,7 +562,7 @@ class BuduraxLM:
                 hops.add_ln(x, y, lw.norm1b, lw.norm1b_b, eps, h2, lw.norm2, lw.norm2_b)
                 a = torch.empty(T, lw.ff, dtype=dt, device=dev)
                 hops.gelu_mul(self._lin(h2, lw.gate_up, getattr(lw, "gate_up_t", None)), a)
-                y = self._lin(a, lw.down, getattr(lw, "down_t", None))
+                y = self._lin(a, lw.down, getattr(lw, "down_t", None), slabs=True)
                 nw, nb = lw.norm2b, lw.norm2b_b
             else:
                 nw, nb = lw.norm1b, lw.norm1b_b
@@ -595,7 +596,7 @@ class BuduraxLM:
         ao = torch.empty(T, H * vd, dtype=dt, device=dev)
         latent_mix(qgd[:, :H * (D + rd)].view(T, H, D + rd)[:, :, :D], q_rot, cache, cache_t, lw, inp, m, ao,
                    gate=qgd[:, lw.g_off:lw.g_off + H * vd])
-        return self._lin(ao, lw.o, getattr(lw, "o_t", None))
+        return self._lin(ao, lw.o, getattr(lw, "o_t", None), slabs=True)
 
     def _chunk_plan(self, m: SegMeta, heads: int):
         """Device chunk tables of this step for layers of ``heads`` heads (built once per step), None = plain scan."""
@@ -632,7 +633,7 @@ class BuduraxLM:
                 hops.ssm_scan(*a, m.tok_seg, m.seg, state.ssm[i], y)
         yn = torch.empty(T, inner, dtype=dt, device=dev)
         hops.gated_norm(y, proj, lw.mnorm, int(mm["norm_groups"]), self.cfg.norm_eps, yn)
-        return self._lin(yn, lw.o, getattr(lw, "o_t", None))
+        return self._lin(yn, lw.o, getattr(lw, "o_t", None), slabs=True)
 
 
 def load_checkpoint(model: BuduraxLM, path: str | Path) -> BuduraxLM:

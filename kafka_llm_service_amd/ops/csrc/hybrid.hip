@@ -267,9 +267,32 @@ __global__ __launch_bounds__(NTH) void ln_shift_reg_kernel(const float* __restri
   }
 }
 
-template <typename AT, int VEC, int NTH, int NV, int MODE>
-__global__ __launch_bounds__(NTH) void add_ln_reg_kernel(float* __restrict__ x, int64_t xs, const AT* __restrict__ y,
-                                                         int64_t ys, const AT* __restrict__ w,
+// VEC neighbouring elements summed over S fp32 slabs, all loads in flight together
+template <int VEC, int S>
+__device__ __forceinline__ void sum_slabs(const float* p, int64_t slab, float (&o)[VEC]) {
+  float t[S][VEC];
+#pragma unroll
+  for (int s = 0; s < S; ++s) ldv<VEC>(p + s * slab, t[s]);
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) o[e] += t[s][e];
+}
+template <int VEC>
+__device__ __forceinline__ void ld_slabs(const float* p, int S, int64_t slab, float (&o)[VEC]) {
+  switch (S) {  // (uniform)
+    case 2: sum_slabs<VEC, 2>(p, slab, o); break;
+    case 4: sum_slabs<VEC, 4>(p, slab, o); break;
+    case 8: sum_slabs<VEC, 8>(p, slab, o); break;
+    default:
+      for (int s = 0; s < S; ++s) sum_slabs<VEC, 1>(p + s * slab, slab, o);
+  }
+}
+
+// SLABS: y is the S fp32 split-K slabs of a projection (a launch of their own to bf16 took 4.6 us of a step of 64 rows)
+template <typename AT, int VEC, int NTH, int NV, int MODE, bool SLABS>
+__global__ __launch_bounds__(NTH) void add_ln_reg_kernel(float* __restrict__ x, int64_t xs, const void* __restrict__ yp,
+                                                         int64_t ys, int S, int64_t slab, const AT* __restrict__ w,
                                                          const AT* __restrict__ b, float eps, int d,
                                                          AT* __restrict__ out2, int64_t os, const AT* __restrict__ w2,
                                                          const AT* __restrict__ b2) {
@@ -282,7 +305,8 @@ __global__ __launch_bounds__(NTH) void add_ln_reg_kernel(float* __restrict__ x, 
     zero<VEC>(yv[k]);
     zero<VEC>(xv[k]);
     if (i < d) {
-      ldv<VEC>(y + t * ys + i, yv[k]);
+      if constexpr (SLABS) ld_slabs<VEC>(reinterpret_cast<const float*>(yp) + t * ys + i, S, slab, yv[k]);
+      else ldv<VEC>(reinterpret_cast<const AT*>(yp) + t * ys + i, yv[k]);
       ldv<VEC>(x + t * xs + i, xv[k]);
       ldv<VEC>(w + i, wv[k]);
       ldv<VEC>(b + i, bv[k]);
@@ -1386,18 +1410,25 @@ hipError_t kafka_hy_scatter_rows(float* dst, const int* seg, const float* src, i
   return hipGetLastError();
 }
 
-hipError_t kafka_hy_add_ln(int f32, float* x, int64_t xs, const void* y, int64_t ys, const void* w, const void* b,
+// S > 0: y is S fp32 slabs, `slab` elements apart (bf16 weights, rows of the register kernels: d up to 4096)
+hipError_t kafka_hy_add_ln(int f32, float* x, int64_t xs, const void* y, int64_t ys, int S, int64_t slab, const void* w, const void* b,
                            float eps, int T, int d, void* out2, int64_t os, const void* w2, const void* b2,
                            hipStream_t st) {
   if (T <= 0) return hipSuccess;
+  if (S < 0 || (S > 0 && (f32 || d > 4096))) return hipErrorInvalidValue;
   const int mode = out2 == nullptr ? 0 : (w2 != nullptr ? 1 : 2);
   DISPATCH_AT(f32, {
-    const bool v4 = d % 4 == 0 && xs % 4 == 0 && ys % 4 == 0 && os % 4 == 0 && al16(x) && al16(y) && al16(w) && al16(b) &&
+    const bool v4 = d % 4 == 0 && xs % 4 == 0 && ys % 4 == 0 && os % 4 == 0 && slab % 4 == 0 && al16(x) && al16(y) && al16(w) && al16(b) &&
                     al16(out2) && al16(w2) && al16(b2);
     auto reg = [&](auto M) {
       return row_shape(T, d, v4, [&](auto V, auto N, auto K) {
-        add_ln_reg_kernel<AT, V.value, N.value, K.value, M.value><<<T, N.value, 0, st>>>(
-            x, xs, (const AT*)y, ys, (const AT*)w, (const AT*)b, eps, d, (AT*)out2, os, (const AT*)w2, (const AT*)b2);
+        auto go = [&](auto k) {
+          k<<<T, N.value, 0, st>>>(x, xs, y, ys, S, slab, (const AT*)w, (const AT*)b, eps, d, (AT*)out2, os, (const AT*)w2, (const AT*)b2);
+        };
+        if constexpr (std::is_same<AT, bf16>::value) {
+          if (S > 0) return go(add_ln_reg_kernel<AT, V.value, N.value, K.value, M.value, true>);
+        }
+        go(add_ln_reg_kernel<AT, V.value, N.value, K.value, M.value, false>);
       });
     };
     auto a = [&](auto k) {

@@ -9,7 +9,7 @@ hipError_t kafka_hy_ln_shift(int f32, const float* x, int64_t xs, const void* w,
                              int64_t os, int T, int d, const void* mu, const int* tok_seg, const int* seg,
                              float* state, float* last, hipStream_t st);
 hipError_t kafka_hy_scatter_rows(float* dst, const int* seg, const float* src, int R, int d, hipStream_t st);
-hipError_t kafka_hy_add_ln(int f32, float* x, int64_t xs, const void* y, int64_t ys, const void* w, const void* b,
+hipError_t kafka_hy_add_ln(int f32, float* x, int64_t xs, const void* y, int64_t ys, int S, int64_t slab, const void* w, const void* b,
                            float eps, int T, int d, void* out2, int64_t os, const void* w2, const void* b2,
                            hipStream_t st);
 hipError_t kafka_hy_gelu_mul(int f32, const void* gu, int64_t gs, void* out, int64_t T, int F, hipStream_t st);
@@ -272,14 +272,22 @@ void scatter_rows(at::Tensor dst, at::Tensor seg, at::Tensor src) {
                                (int)dst.size(1), stream()));
 }
 
+// y: rows of the activation dtype, or the fp32 split-K slabs [S, T, d] of a projection beside bf16 weights
 void add_ln(at::Tensor x, at::Tensor y, at::Tensor w, at::Tensor b, double eps, OptT out2, OptT w2, OptT b2) {
-  rows2d(x, "x"); rows2d(y, "y");
+  rows2d(x, "x");
   TORCH_CHECK(x.scalar_type() == at::kFloat, "add_ln: x is the fp32 stream");
-  const int f32 = act_f32(y);
   const int64_t T = x.size(0), d = x.size(1);
+  const bool slabs = y.dim() == 3;
+  if (slabs) {
+    TORCH_CHECK(y.is_cuda() && y.scalar_type() == at::kFloat && y.is_contiguous() && y.size(0) > 0 && d <= 4096 &&
+                    w.scalar_type() == at::kBFloat16, "add_ln: slabs fp32 [S, T, d], d up to 4096, bf16 weights");
+  } else {
+    rows2d(y, "y");
+  }
+  const int f32 = slabs ? 0 : act_f32(y);
   same_act(f32, {&w, &b});
   vec(w, d, "w"); vec(b, d, "b");
-  TORCH_CHECK(y.size(0) == T && y.size(1) == d && x.stride(0) >= d, "add_ln: shapes");
+  TORCH_CHECK(y.size(-2) == T && y.size(-1) == d && x.stride(0) >= d, "add_ln: shapes");
   void* o2 = nullptr; int64_t os = 0; const void *w2p = nullptr, *b2p = nullptr;
   if (out2.has_value()) {
     rows2d(*out2, "out2"); same_act(f32, {&*out2});
@@ -291,7 +299,7 @@ void add_ln(at::Tensor x, at::Tensor y, at::Tensor w, at::Tensor b, double eps, 
       w2p = w2->data_ptr(); b2p = b2->data_ptr();
     }
   }
-  HY_HIP(kafka_hy_add_ln(f32, x.data_ptr<float>(), x.stride(0), y.data_ptr(), y.stride(0), w.data_ptr(), b.data_ptr(),
+  HY_HIP(kafka_hy_add_ln(f32, x.data_ptr<float>(), x.stride(0), y.data_ptr(), y.stride(-2), slabs ? (int)y.size(0) : 0, slabs ? T * d : 0, w.data_ptr(), b.data_ptr(),
                          (float)eps, (int)T, (int)d, o2, os, w2p, b2p, stream()));
 }
 

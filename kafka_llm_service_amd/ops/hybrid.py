@@ -46,7 +46,10 @@ def scatter_rows(dst, seg, src) -> None:
 
 def add_ln(x, y, w, b, eps, out2=None, w2=None, b2=None) -> None:
     """x += layer_norm(y; w, b) in place (x fp32); with ``out2`` also out2 = layer_norm(x; w2, b2), or the new x in
-    out2's dtype when no second norm is given."""
+    out2's dtype when no second norm is given. y [T, d] in the weights' dtype, or the fp32 split-K slabs [S, T, d] of a
+    projection (summed here)."""
+    if y.dim() == 3 and not (_gpu(x) and x.shape[1] <= 4096 and w.dtype == torch.bfloat16 and y.is_contiguous()):
+        y = y.sum(0).to(w.dtype)
     if _gpu(x):
         ext().hy_add_ln(x, y, w, b, float(eps), out2, w2, b2)
     else:

@@ -1116,6 +1116,30 @@ def test_single_token_behind_more_pages_than_a_run():
     assert (flat.double() - want).abs().max().item() < 2 ** -8 * want.abs().max().item() + 1e-6
 
 
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("d,T", [(4, 3), (1022, 3), (1028, 513), (1030, 5), (4096, 7), (4096, 520), (4100, 3)])
+def test_add_norm_of_slabs(device, d, T):
+    """A projection's split-K slabs in place of its rows: the forms of the row kernels, slab counts with loops of their own and
+    without, against 64 bits: fp32 sums (d * 2^-24 of a value's size), results in bf16 (half a step, 2^-8), and the
+    widths beyond the register kernels and the CPU, where the sum is rounded to bf16 first (2^-8 of a y of up to 5 sizes)."""
+    g = torch.Generator().manual_seed(d + T)
+    w, b, w2, b2 = ((torch.randn(d, generator=g)).to(torch.bfloat16) for _ in range(4))
+    for S in (1, 2, 3, 4, 8):
+        x, y = torch.randn(T, d, generator=g), torch.randn(S, T, d, generator=g)
+        x1 = x.double() + plain.layer_norm(y.double().sum(0), w.double(), b.double(), 1e-5)
+        low = device == "cpu" or d > 4096
+        for second in (None, (w2, b2)):
+            xd, o = x.clone().to(device), torch.empty(T, d, dtype=torch.bfloat16, device=device)
+            hops.add_ln(xd, y.to(device), w.to(device), b.to(device), 1e-5, o, *(t.to(device) for t in second or ()))
+            tol = d * 2.0 ** -24 + 1e-5 + (2 ** -7 * 5 if low else 0)
+            size = w.double().abs() + x1.abs() + 1
+            assert ((xd.cpu().double() - x1).abs() <= tol * size).all()
+            want = xd.cpu().double()
+            if second:
+                want = plain.layer_norm(want, w2.double(), b2.double(), 1e-5)
+            assert ((o.cpu().double() - want).abs() <= (2 ** -8 + d * 2.0 ** -24 + 1e-5) * (want.abs() + 1)).all()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("d,T", [(4, 3), (1024, 3), (1028, 5), (1030, 5), (4096, 7), (4096, 600), (4100, 3), (1022, 2)])

@@ -56,26 +56,24 @@ class MoEBlock:
     def __call__(self, x: torch.Tensor, lw) -> torch.Tensor:
         T, d = x.shape
         logits = ops.linear_small(x, lw.router)
-        r = ops.moe_route(logits, self.k)
         if self.ep > 1 and self.a2a:
-            return self._a2a(x, lw, r)
+            return self._a2a(x, lw, ops.moe_route(logits, self.k))
+        out = torch.empty(T, d, dtype=torch.float32, device=x.device)
+        r = ops.moe_route(logits, self.k, zero=out)
         if self.model.stream and lw.w13_t is not None and T <= MOE_STREAM_MAX_T:
             # decode-sized steps: expert weights streamed from their wave-tiled copies, SwiGLU fused into the gate_up
             # epilogue, weighted combine fused into the down epilogue (csrc/wstream_gemm.hip, grouped variant)
             a = ops.grouped_stream_glu(x, lw.w13_t, r, e_lo=self.e0)
-            out = torch.zeros(T, d, dtype=torch.float32, device=x.device)
             ops.grouped_stream_combine(a, lw.w2_t, r, T, out, e_lo=self.e0)
             return self._finish(out, x.dtype)
         if self.model.stream and lw.w13_t is not None and self.ep == 1 and d % 128 == 0 and self.F % 128 == 0:
             # long steps on the same tiled weights: 128-row tiles (csrc/moe_wide.hip)
             a = ops.grouped_wide(x, lw.w13_t, r, "glu", True)
-            out = torch.zeros(T, d, dtype=torch.float32, device=x.device)
             return self._finish(ops.grouped_wide(a, lw.w2_t, r, "combine", False, out), x.dtype)
         # gate_up for every (token, expert) entry routed to a local expert, rows gathered from x by the kernel
         h = ops.grouped_gemm(x, lw.w13, r, gather=True, e_lo=self.e0)
         a = ops.silu_mul(h)
         # down projection with the routing-weighted scatter-combine fused into the epilogue
-        out = torch.zeros(T, d, dtype=torch.float32, device=x.device)
         ops.grouped_gemm(a, lw.w2, r, gather=False, e_lo=self.e0, combine_out=out)
         return self._finish(out, x.dtype)
 

@@ -830,8 +830,9 @@ class MoERouting:
 GG_BM = 64  # row tile of the grouped GEMM (a routing bound the kernel and the host agree on)
 
 
-def moe_route(logits: torch.Tensor, k: int) -> MoERouting:
-    """softmax -> top-k -> renormalise, then a stable sort of the T*k entries by expert (token order inside)."""
+def moe_route(logits: torch.Tensor, k: int, zero: torch.Tensor | None = None) -> MoERouting:
+    """softmax -> top-k -> renormalise, then a stable sort of the T*k entries by expert (token order inside). ``zero`` fp32:
+    cleared by the same launch (the sums that the experts add to)."""
     T, E = logits.shape
     dev = logits.device
     if _gpu(logits):
@@ -841,15 +842,18 @@ def moe_route(logits: torch.Tensor, k: int) -> MoERouting:
         pw = torch.empty(T * k, dtype=torch.float32, device=dev)
         eo = torch.empty(E + 1, dtype=torch.int32, device=dev)
         to = torch.empty(E + 1, dtype=torch.int32, device=dev)
-        ext().moe_route(logits, int(k), GG_BM, tw, te, pt, pw, eo, to)
+        ext().moe_route(logits, int(k), GG_BM, tw, te, pt, pw, eo, to, zero)
         return MoERouting(tw, te, pt, pw, eo, to, E)
+    if zero is not None:
+        zero.zero_()
     tw, te, pt, pw, eo, to = ref.moe_route(logits, k, GG_BM)
     return MoERouting(tw, te, pt, pw, eo, to, E)
 
 
-def moe_sort(topk_w: torch.Tensor, topk_e: torch.Tensor, num_experts: int, inverse: bool = False) -> MoERouting:
+def moe_sort(topk_w: torch.Tensor, topk_e: torch.Tensor, num_experts: int, inverse: bool = False,
+             zero: torch.Tensor | None = None) -> MoERouting:
     """MoERouting of entries routed elsewhere (weights fp32 [T, k], expert ids int32 [T, k]): the stable sort by expert
-    of ``moe_route`` alone, for any number of experts and choices. ``inverse``: also ``inv`` (up to 512 experts)."""
+    of ``moe_route`` alone, for any number of experts and choices. ``inverse``: also ``inv`` (up to 512 experts). ``zero`` as in ``moe_route``."""
     T, k = topk_e.shape
     dev = topk_e.device
     inv = torch.empty(T, k, dtype=torch.int32, device=dev) if inverse else None
@@ -858,8 +862,10 @@ def moe_sort(topk_w: torch.Tensor, topk_e: torch.Tensor, num_experts: int, inver
         pw = torch.empty(T * k, dtype=torch.float32, device=dev)
         eo = torch.empty(num_experts + 1, dtype=torch.int32, device=dev)
         to = torch.empty(num_experts + 1, dtype=torch.int32, device=dev)
-        ext().moe_sort(topk_w, topk_e, int(num_experts), GG_BM, pt, pw, eo, to, inv)
+        ext().moe_sort(topk_w, topk_e, int(num_experts), GG_BM, pt, pw, eo, to, inv, zero)
         return MoERouting(topk_w, topk_e, pt, pw, eo, to, num_experts, inv)
+    if zero is not None:
+        zero.zero_()
     flat = topk_e.reshape(-1).long()
     perm = torch.argsort(flat, stable=True)
     counts = torch.bincount(flat, minlength=num_experts)

@@ -86,11 +86,11 @@ hipError_t kafka_launch_wstream_grouped(const bf16* X, int64_t ldx, const bf16* 
                                         int pin, int relu2, float glu_limit, float glu_alpha, hipStream_t st);
 hipError_t kafka_launch_moe_route(const bf16* logits, int64_t ld, int T, int E, int K, int BM, float* topk_w,
                                   int* topk_e, int* perm_tok, float* perm_w, int* expert_off, int* tile_off,
-                                  hipStream_t st);
+                                  float* zero, int64_t nzero, hipStream_t st);
 int kafka_moe_sort_max_e();
 int kafka_moe_sort_parts(int n, int E);
 hipError_t kafka_launch_moe_sort(const float* topk_w, const int* topk_e, int n, int k, int E, int bm, int* perm_tok,
-                                 float* perm_w, int* expert_off, int* tile_off, int* inv, int* counts, hipStream_t st);
+                                 float* perm_w, int* expert_off, int* tile_off, int* inv, int* counts, float* zero, int64_t nzero, hipStream_t st);
 hipError_t kafka_launch_grouped_wide(const bf16* X, int64_t ldx, const bf16* Wt, int E, int N, int K,
                                      const int* perm_tok, const float* perm_w, const int* expert_off, int n_ent,
                                      int gather, int epi, bf16* Y, int64_t ldy, float* out, int64_t ldo,
@@ -922,8 +922,19 @@ static void slab_reduce(at::Tensor p, at::Tensor y) {
 }
 
 // softmax -> top-k -> renormalise + stable expert sort (one kernel, no host sync)
+// an fp32 tensor that a routing launch clears: its 16-byte pieces, 0 where it has to be cleared by itself (and is, here)
+static int64_t clear_pieces(const c10::optional<at::Tensor>& zero, bool in_launch) {
+  if (!zero.has_value()) return 0;
+  CHECK_CUDA(zero.value()); CHECK_DT(zero.value(), at::kFloat);
+  if (in_launch && zero->numel() > 0 && zero->is_contiguous() && zero->numel() % 4 == 0 && reinterpret_cast<uintptr_t>(zero->data_ptr()) % 16 == 0)
+    return zero->numel() / 4;
+  zero->zero_();
+  return 0;
+}
+
 static void moe_route(at::Tensor logits, int64_t k, int64_t bm, at::Tensor topk_w, at::Tensor topk_e,
-                      at::Tensor perm_tok, at::Tensor perm_w, at::Tensor expert_off, at::Tensor tile_off) {
+                      at::Tensor perm_tok, at::Tensor perm_w, at::Tensor expert_off, at::Tensor tile_off,
+                      c10::optional<at::Tensor> zero) {
   CHECK_CUDA(logits); CHECK_DT(logits, at::kBFloat16); CHECK_LASTDIM(logits);
   CHECK_DT(topk_w, at::kFloat); CHECK_DT(perm_w, at::kFloat);
   CHECK_DT(topk_e, at::kInt); CHECK_DT(perm_tok, at::kInt); CHECK_DT(expert_off, at::kInt); CHECK_DT(tile_off, at::kInt);
@@ -935,15 +946,18 @@ static void moe_route(at::Tensor logits, int64_t k, int64_t bm, at::Tensor topk_
               "moe_route: output sizes");
   TORCH_CHECK(topk_w.is_contiguous() && topk_e.is_contiguous() && perm_tok.is_contiguous() && perm_w.is_contiguous(),
               "moe_route: contiguous outputs");
+  const int64_t nz = clear_pieces(zero, true);
   CHECK_HIP(kafka_launch_moe_route(bptr(logits), logits.stride(0), T, E, (int)k, (int)bm, topk_w.data_ptr<float>(),
                                    topk_e.data_ptr<int>(), perm_tok.data_ptr<int>(), perm_w.data_ptr<float>(),
-                                   expert_off.data_ptr<int>(), tile_off.data_ptr<int>(), cur_stream()));
+                                   expert_off.data_ptr<int>(), tile_off.data_ptr<int>(), nz ? zero->data_ptr<float>() : nullptr, nz,
+                                   cur_stream()));
 }
 
 // the sort of moe_route alone, for entries routed elsewhere (topk_w / topk_e [T, k] are inputs; expert ids in [0, E));
 // inv [T, k]: every entry's place in the sorted order
 static void moe_sort(at::Tensor topk_w, at::Tensor topk_e, int64_t E, int64_t bm, at::Tensor perm_tok,
-                     at::Tensor perm_w, at::Tensor expert_off, at::Tensor tile_off, c10::optional<at::Tensor> inv) {
+                     at::Tensor perm_w, at::Tensor expert_off, at::Tensor tile_off, c10::optional<at::Tensor> inv,
+                     c10::optional<at::Tensor> zero) {
   CHECK_CUDA(topk_w); CHECK_DT(topk_w, at::kFloat); CHECK_DT(perm_w, at::kFloat);
   CHECK_DT(topk_e, at::kInt); CHECK_DT(perm_tok, at::kInt); CHECK_DT(expert_off, at::kInt); CHECK_DT(tile_off, at::kInt);
   TORCH_CHECK(topk_w.dim() == 2 && topk_e.sizes() == topk_w.sizes() && topk_w.is_contiguous() && topk_e.is_contiguous(),
@@ -960,18 +974,20 @@ static void moe_sort(at::Tensor topk_w, at::Tensor topk_e, int64_t E, int64_t bm
                 "moe_sort: inv [T, k], up to ", kafka_moe_sort_max_e(), " experts");
     ip = inv->data_ptr<int>();
   }
+  const int64_t nz = clear_pieces(zero, E <= 64 && T * k < (int64_t)1 << 30);
   if (E <= kafka_moe_sort_max_e() && T * k < (int64_t)1 << 30) {
     const int parts = kafka_moe_sort_parts((int)(T * k), (int)E);
     const at::Tensor counts = parts > 1 ? at::empty({64 * parts}, topk_e.options()) : at::Tensor();
     CHECK_HIP(kafka_launch_moe_sort(topk_w.data_ptr<float>(), topk_e.data_ptr<int>(), (int)(T * k), (int)k, (int)E,
                                     (int)bm, perm_tok.data_ptr<int>(), perm_w.data_ptr<float>(),
                                     expert_off.data_ptr<int>(), tile_off.data_ptr<int>(), ip,
-                                    parts > 1 ? counts.data_ptr<int>() : nullptr, cur_stream()));
+                                    parts > 1 ? counts.data_ptr<int>() : nullptr, nz ? zero->data_ptr<float>() : nullptr, nz,
+                                    cur_stream()));
     return;
   }
   CHECK_HIP(kafka_launch_moe_route(nullptr, 0, (int)T, (int)E, (int)k, (int)bm, topk_w.data_ptr<float>(),
                                    topk_e.data_ptr<int>(), perm_tok.data_ptr<int>(), perm_w.data_ptr<float>(),
-                                   expert_off.data_ptr<int>(), tile_off.data_ptr<int>(), cur_stream()));
+                                   expert_off.data_ptr<int>(), tile_off.data_ptr<int>(), nullptr, 0, cur_stream()));
 }
 
 // Y (or out += w * Y) = X_e . W_e^T per expert segment of the routed entries; W = [e_n, N, K] local experts
@@ -1237,8 +1253,9 @@ PYBIND11_MODULE(_kafka_ops, m) {
         py::arg("expert_off"), py::arg("e_lo"), py::arg("max_rows"), py::arg("gather"), py::arg("y"), py::arg("out"),
         py::arg("pin") = true, py::arg("glu_limit") = 0.0, py::arg("glu_alpha") = 1.0, py::arg("relu2") = false);
   m.def("moe_sort", &moe_sort, py::arg("topk_w"), py::arg("topk_e"), py::arg("E"), py::arg("bm"), py::arg("perm_tok"),
-        py::arg("perm_w"), py::arg("expert_off"), py::arg("tile_off"), py::arg("inv") = py::none());
-  m.def("moe_route", &moe_route);
+        py::arg("perm_w"), py::arg("expert_off"), py::arg("tile_off"), py::arg("inv") = py::none(), py::arg("zero") = py::none());
+  m.def("moe_route", &moe_route, py::arg("logits"), py::arg("k"), py::arg("bm"), py::arg("topk_w"), py::arg("topk_e"), py::arg("perm_tok"),
+        py::arg("perm_w"), py::arg("expert_off"), py::arg("tile_off"), py::arg("zero") = py::none());
   m.def("cu_mask_stream", &cu_mask_stream);
   m.def("stream_cu_mask", &stream_cu_mask);
   m.def("car_alloc", &car_alloc);

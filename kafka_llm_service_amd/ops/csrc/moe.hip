@@ -1,6 +1,6 @@
 // Sparse-MoE kernels for gfx950 (Mixtral: E = 8 experts, top-2; SURVEY.md §2.6 `moe_router_topk`, `grouped_gemm`).
 //
-// moe_route_kernel — ONE workgroup of 1024 threads does the whole routing of a step (T <= 32k tokens):
+// moe_route_kernel — ONE workgroup of 1024 threads (further ones clear the experts' sums) does the whole routing of a step (T <= 32k tokens):
 //   softmax over the E router logits -> top-k -> renormalise (Mixtral), then a stable expert sort of the T*k
 //   (token, slot) entries: every entry's position is its rank among its expert's, so the permutation is deterministic
 //   (token order inside each expert). Outputs:
@@ -42,6 +42,7 @@ namespace kafka {
 constexpr int MOE_MAXE = 16;
 constexpr int MOE_MAXK = 4;
 constexpr int MOE_NT = 1024;
+static_assert(MOE_NT == mw::SORT_NT, "the sort's threads");
 
 // softmax + top-k + renormalise of a thread's tokens in registers, then the sort. Bound by latency: the logits' round trip, the
 // sort's two. 1900 tokens x 8 experts 35 -> 15 us, 128 tokens 12 -> 6.5, 8192 194 -> 43 (probabilities in indexed memory and a block scan per
@@ -50,8 +51,12 @@ __global__ __launch_bounds__(MOE_NT) void moe_route_kernel(const bf16* __restric
                                                             int K, int bits, int BM, float* __restrict__ topk_w,
                                                             int* __restrict__ topk_e, int* __restrict__ perm_tok,
                                                             float* __restrict__ perm_w, int* __restrict__ expert_off,
-                                                            int* __restrict__ tile_off) {
+                                                            int* __restrict__ tile_off, float* __restrict__ zero, int64_t nzero) {
   __shared__ int cnt[mw::SORT_W][64];
+  if (blockIdx.x > 0) {
+    mw::clear(zero, nzero, blockIdx.x - 1, gridDim.x - 1);
+    return;
+  }
   for (int t = threadIdx.x; t < T; t += MOE_NT) {
     float p[MOE_MAXE];
     float m = -INFINITY;
@@ -278,12 +283,14 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(const bf16* __restric
 
 extern "C" hipError_t kafka_launch_moe_route(const bf16* logits, int64_t ld, int T, int E, int K, int BM,
                                             float* topk_w, int* topk_e, int* perm_tok, float* perm_w,
-                                            int* expert_off, int* tile_off, hipStream_t st) {
+                                            int* expert_off, int* tile_off, float* zero, int64_t nzero, hipStream_t st) {
+  if (zero != nullptr && logits == nullptr) return hipErrorInvalidValue;
   if (K > E || K < 1 || (logits != nullptr && (E > MOE_MAXE || K > MOE_MAXK))) return hipErrorInvalidValue;
   int bits = 0;
   while ((1 << bits) < E) ++bits;
   if (logits != nullptr)
-    moe_route_kernel<<<1, MOE_NT, 0, st>>>(logits, ld, T, E, K, bits, BM, topk_w, topk_e, perm_tok, perm_w, expert_off, tile_off);
+    moe_route_kernel<<<1 + (zero != nullptr ? mw::clear_blocks(nzero) : 0), MOE_NT, 0, st>>>(
+        logits, ld, T, E, K, bits, BM, topk_w, topk_e, perm_tok, perm_w, expert_off, tile_off, zero, nzero);
   else   // (the caller has routed: topk_w / topk_e are inputs)
     moe_sort_any_kernel<<<1, MOE_NT, 0, st>>>(T, E, K, BM, topk_w, topk_e, perm_tok, perm_w, expert_off, tile_off);
   return hipGetLastError();

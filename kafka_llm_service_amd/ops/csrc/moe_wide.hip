@@ -333,11 +333,16 @@ __global__ __launch_bounds__(SORT_NT) void moe_sort_few_kernel(const float* __re
                                                                int n, int k, int E, int bits, int bm,
                                                                int* __restrict__ perm_tok, float* __restrict__ perm_w,
                                                                int* __restrict__ expert_off, int* __restrict__ tile_off,
-                                                               int* __restrict__ inv, const int* __restrict__ counts) {
+                                                               int* __restrict__ inv, const int* __restrict__ counts, int parts,
+                                                               float* __restrict__ zero, int64_t nzero) {
   __shared__ int cnt[SORT_W][64];
-  const int lo = gridDim.x > 1 ? blockIdx.x * SORT_PART : 0, hi = gridDim.x > 1 ? min(n, lo + SORT_PART) : n;
+  if ((int)blockIdx.x >= parts) {
+    clear(zero, nzero, blockIdx.x - parts, gridDim.x - parts);
+    return;
+  }
+  const int lo = parts > 1 ? blockIdx.x * SORT_PART : 0, hi = parts > 1 ? min(n, lo + SORT_PART) : n;
   sort_few_experts(topk_w, topk_e, lo, hi, k, E, bits, bm, perm_tok, perm_w, expert_off, tile_off, inv, counts, blockIdx.x,
-                   gridDim.x, cnt);
+                   parts, cnt);
 }
 
 // how many of the part's entries go to expert `lane`
@@ -603,10 +608,12 @@ int kafka_moe_sort_max_e() { return SORT_MAXE; }
 // workgroups of a sort (its scratch: 64 counts each): one up to 4096 entries, where a second launch costs what it saves
 int kafka_moe_sort_parts(int n, int E) { return E > 64 || n <= 2 * SORT_PART ? 1 : (n + SORT_PART - 1) / SORT_PART; }
 
+// zero: nzero 16-byte pieces that the launch clears (up to 64 experts)
 hipError_t kafka_launch_moe_sort(const float* topk_w, const int* topk_e, int n, int k, int E, int bm, int* perm_tok,
-                                 float* perm_w, int* expert_off, int* tile_off, int* inv, int* counts, hipStream_t st) {
+                                 float* perm_w, int* expert_off, int* tile_off, int* inv, int* counts, float* zero, int64_t nzero,
+                                 hipStream_t st) {
   if (n < 1) return hipSuccess;
-  if (E < 1 || E > SORT_MAXE || k < 1 || bm < 1) return hipErrorInvalidValue;
+  if (E < 1 || (zero != nullptr && E > 64) || E > SORT_MAXE || k < 1 || bm < 1) return hipErrorInvalidValue;
   int bits = 0;
   while ((1 << bits) < E) ++bits;
   if (E > 64) {
@@ -615,8 +622,8 @@ hipError_t kafka_launch_moe_sort(const float* topk_w, const int* topk_e, int n, 
   }
   const int parts = counts != nullptr ? kafka_moe_sort_parts(n, E) : 1;
   if (parts > 1) moe_sort_count_kernel<<<parts, SORT_NT, 0, st>>>(topk_e, n, E, bits, counts);
-  moe_sort_few_kernel<<<parts, SORT_NT, 0, st>>>(topk_w, topk_e, n, k, E, bits, bm, perm_tok, perm_w, expert_off, tile_off, inv,
-                                                 counts);
+  moe_sort_few_kernel<<<parts + (zero != nullptr ? clear_blocks(nzero) : 0), SORT_NT, 0, st>>>(
+      topk_w, topk_e, n, k, E, bits, bm, perm_tok, perm_w, expert_off, tile_off, inv, counts, parts, zero, nzero);
   return hipGetLastError();
 }
 

@@ -686,8 +686,7 @@ def moe_experts(h, w_gu, w_down, topk_w, topk_e, out, w_gu_t=None, w_down_t=None
     T = h.shape[0]
     glu = act != "relu2"
     if T and moe_grouped_ok(h, w_gu, w_down, glu):
-        r = ops.moe_sort(topk_w, topk_e, w_gu.shape[0])
-        out.zero_()
+        r = ops.moe_sort(topk_w, topk_e, w_gu.shape[0], zero=out)
         if w_gu_t is not None and w_down_t is not None:
             lim, al = _glu_act(act, limit, alpha) if glu else (0.0, 1.0)
             if moe_wide(T, topk_e.shape[1], w_gu.shape[0]):

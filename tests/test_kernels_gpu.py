@@ -867,6 +867,23 @@ def test_linear_dense_in_blocks(cuda, M):
     assert ops.linear_dense(x.unsqueeze(1), w).shape == (M, 1, N)
 
 
+@pytest.mark.parametrize("T,k,E", [(1, 1, 1), (16, 4, 16), (5000, 2, 8), (9, 3, 65), (7, 2, 600)])
+def test_routing_clears_the_sums(cuda, T, k, E):
+    """The launch that sorts a step's entries (one workgroup, several, the kernels for many experts) and the one that routes them
+    clear the given sums and nothing beside them, whatever their size, place and strides."""
+    te = torch.stack([torch.randperm(E)[:k] for _ in range(T)]).to(torch.int32).to(cuda)
+    tw, lg = torch.rand(T, k, device=cuda), torch.randn(T, min(E, 16), device=cuda).to(torch.bfloat16)
+    want = ops.moe_sort(tw, te, E)
+    for d, at, wide in ((4096, 0, 0), (64, 4, 0), (5, 0, 0), (64, 1, 0), (64, 0, 8)):
+        for f in (lambda z: ops.moe_sort(tw, te, E, zero=z), lambda z: ops.moe_route(lg, min(k, 4, lg.shape[1]), zero=z)):
+            buf = torch.full((at + T * (d + wide) + 7,), 7.0, device=cuda)
+            z = buf[at:at + T * (d + wide)].view(T, d + wide)[:, :d]
+            r = f(z)
+            assert (z == 0).all() and (buf == 7).sum() == buf.numel() - T * d
+    r = ops.moe_sort(tw, te, E, zero=torch.empty(T, 64, device=cuda))
+    assert all(torch.equal(getattr(r, n), getattr(want, n)) for n in ("perm_tok", "perm_w", "expert_off", "tile_off"))
+
+
 @pytest.mark.parametrize("T,k", [(1, 1), (63, 1), (65, 1), (1024, 4), (4097, 1), (683, 6), (2731, 3)])
 @pytest.mark.parametrize("E", [1, 5, 64, 65])
 def test_moe_sort_sizes(cuda, T, k, E):

@@ -359,8 +359,8 @@ def small_ok(x: torch.Tensor, w: torch.Tensor, rows: int) -> bool:
 
 def small_rows(N: int, K: int) -> int:
     """Rows up to which a small product runs on the kernel instead of the library (figures: csrc/small_gemm.hip)."""
-    if K >= 1024:
-        return 1024 if N <= 64 else 0   # (a workgroup per 16 columns reads the rows again)
+    if K >= 1024:   # (a workgroup per 16 columns reads the rows again)
+        return 8192 if N <= 16 else 2048 if N <= 32 else 1024 if N <= 64 else 0
     return 4096 if K <= 32 else 256
 
 

@@ -5,7 +5,8 @@
 // What bounds it: a round trip to memory, a launch, and with long rows of a power of two that all 16 of a load lie in one cache
 // channel. So the loads of a wave's whole share of K (16 waves share it) are in flight together. The library's kernels take as long here, but
 // its call costs the host 17 us and this one 3, which is what steps of few rows wait for.
-// us, library on the GPU / this kernel: 64 columns of K = 4096, 64 rows 7.6 / 8.8, 900 8.1 / 9.4, 2048 15.2 / 16.9, 4096 15.9 / 31.9; 4096 columns of
+// us, library on the GPU / this kernel: 64 columns of K = 4096, 64 rows 7.6 / 8.8, 900 8.1 / 9.4, 2048 15.2 / 16.9, 4096 15.9 / 31.9; 8 columns 1900 rows 15.3 / 7.9,
+// with the call 18.8 / 7.9, 8192 21 / 15.6; 32 columns 1900 rows 20 / 9.5, 2805 20 / 17; 4096 columns of
 // K = 64, 64 rows 3.6 / 3.3, 300 5.4 / 4.7, 900 5.8 / 8.4; 2048 of K = 16, 64 rows 4.0 / 2.8, 4096 10.1 / 8.9; 8192 of K = 128, 128 rows
 // 4.7 / 4.6, 300 6.3 / 9.8; 32 heads of 128 -> 512, 64 rows 4.6 / 4.6, 128 5.5 / 7.9, of 512 -> 128, 64 rows 8.6 / 4.7, 300 15.3 / 16.1.
 #include "common.h"

@@ -874,7 +874,7 @@ def moe_router_grouped(h, w, correction, k: int, groups: int, keep: int, eps: fl
     row. Returns (weights fp32 [T, k], experts int32 [T, k], gate fp32 [T] or None).
     ``w_act``: the same weights in h's dtype when they are exact in it - then a plain choice (softmax, no groups, no
     correction) of up to 64 experts is one kernel, product included (bf16 products, fp32 sums: the same logits); other choices
-    take the logits of steps of few rows from the kernel for small products."""
+    take their logits from the kernels for small products."""
     T = h.shape[0]
     E = w.shape[0] - (1 if extra_gate else 0)
     if E < 1 or groups < 1 or E % groups or not 1 <= keep <= groups or not 1 <= k <= keep * (E // groups):
@@ -892,11 +892,8 @@ def moe_router_grouped(h, w, correction, k: int, groups: int, keep: int, eps: fl
     elif _gpu(h):
         # logits as one full-precision fp32 matrix product (the engine switches reduced-precision matrix modes off),
         # then the choice kernel
-        from kafka_llm_service_amd import ops
-
-        if w_act is not None and ops.small_ok(h, w_act, 1024) and h.shape[1] >= 1024 and w_act.shape[0] <= 64:
-            z = torch.empty(T, w_act.shape[0], dtype=torch.float32, device=h.device)   # (the same products and sums)
-            ext().small_gemm(h, w_act, z)
+        if w_act is not None and T and narrow_ok(h, w_act):   # (the same products and sums; 2805 rows of 4096, 8 experts 28 / 8 us)
+            z = linear_f32(h, w_act)
         else:
             z = torch.mm(h.float(), w.t())
         ext().hy_moe_topk_grouped(z, int(E), correction, int(groups), int(keep), float(eps),

@@ -51,7 +51,7 @@ def test_against_fp32(K):
 def test_rows_beyond_and_forms_of_the_library():
     """One row past each limit, and operands that the kernel does not take (odd columns, odd strides, a shifted start)."""
     g = torch.Generator().manual_seed(1)
-    for N, K in ((64, 1024), (68, 1024), (32, 16), (512, 128)):
+    for N, K in ((64, 1024), (68, 1024), (32, 1024), (16, 1024), (32, 16), (512, 128)):
         n = ops.small_rows(N, K)
         for M in (n, n + 1):
             x, w = torch.randn(max(M, 1), K, generator=g).to(torch.bfloat16).cuda(), (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
@@ -80,3 +80,20 @@ def test_heads(n):
     head_product(o, uv, uv.transpose(1, 2).contiguous(), ao.view(n, H, D).transpose(0, 1))
     for h in range(H):
         _close(ao[:, h * D:(h + 1) * D], o[h].float() @ uv[h].float().t())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,K,gate", [(8, 1024, False), (8, 1024, True), (63, 2048, True), (64, 96, False), (65, 1024, False)])
+def test_router_logits_of_long_steps(E, K, gate):
+    """Choices other than the plain one, whose logits come from the kernels for small products where the weights are exact in bf16:
+    against the same with fp32 weights (sums of K products of size 1 in another order, far below the scores' distances)."""
+    g = torch.Generator().manual_seed(E)
+    w = torch.randn(E + gate, K, generator=g).to(torch.bfloat16).cuda() / 8
+    for T in (1, 1030, 2049):
+        h = torch.randn(T, K, generator=g).to(torch.bfloat16).cuda()
+        got, want = (hops.moe_router_grouped(h, w.float(), None, 2, 1, 1, extra_gate=gate, score="sigmoid", norm=False, w_act=a) for a in (w, None))
+        assert (got[1] == want[1]).float().mean() >= 0.999
+        same = got[1] == want[1]
+        assert ((got[0] - want[0]).abs()[same] <= 1e-4).all()
+        if gate:
+            assert ((got[2] - want[2]).abs() <= 1e-4).all()

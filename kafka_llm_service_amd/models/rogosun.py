@@ -482,9 +482,12 @@ class RogosunLM:
             y = self._gla(lw, h, m, st) if lw.type == "gla" else self._parallel(i, lw, h, inp, m, pages, st)
             hops.norm_add(x, y, None, lw.norm1, eps, None if last and not lw.ff else h)
             if lw.ff == "dense":
-                u = self._lin(h, lw.up, getattr(lw, "up_t", None))
-                a = torch.empty_like(u)
-                hops.relu2(u, a)
+                up_t = getattr(lw, "up_t", None)
+                a = ops.linear_relu2_long(h, up_t) if self.stream and up_t is not None and not self._streams(h.shape[0], lw.up, up_t) else None
+                if a is None:
+                    u = self._lin(h, lw.up, up_t)
+                    a = torch.empty_like(u)
+                    hops.relu2(u, a)
                 hops.norm_add(x, self._lin(a, lw.down, getattr(lw, "down_t", None), slabs=True), None, lw.norm2, eps,
                               None if last else h)
             elif lw.ff == "moe":

@@ -389,7 +389,7 @@ TILE_GLU_M, TILE_EVEN_M, TILE_RAGGED_M = 3600, 5600, 8448
 def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) -> tuple[int, int, int] | None:
     """(16-row parts, 16-column parts, splits) of the tile kernel for x [M, K] @ W^T [N, K], None where it does not take the shape or
     the library is as fast. ``form``: "slabs" (the consumer sums the split-K slabs as it loads them), "bf16" (slabs go
-    through slab_reduce, a launch) or "glu" (silu(gate) * up, in the epilogue or from slabs). ``library``: there is a row-major weight for it.
+    through slab_reduce, a launch), "glu" (silu(gate) * up, in the epilogue or from slabs) or "relu2" (relu squared, in the epilogue). ``library``: there is a row-major weight for it.
 
     Against the library (us, library / this kernel): 450 rows of 14336 -> 4096 89 / 55, 2048 rows 202 / 178; 2048 rows of 4096 -> 18560 350 / 277,
     200 rows 57 / 45; 900 rows of 2048 -> 9344 45 / 36; 450 rows of 2048 -> 2048 19 / 11; over all timed shapes 13 % less time with slabs,
@@ -408,12 +408,12 @@ def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) 
         return None
     if library and form == "bf16" and N > TILE_LIBRARY_N and 256 < M <= 1024:
         return None
-    gain = 1.25 if N % 256 else 0.95
+    gain, act = 1.25 if N % 256 else 0.95, form in ("glu", "relu2")
     if library and M > TILE_MAX_M:
         tiles = -(-M // 256) * -(-N // 256)
-        if M > (TILE_GLU_M if form == "glu" else TILE_RAGGED_M if N % 256 else TILE_EVEN_M) or tiles <= (512 if form == "glu" else 256):
+        if M > (TILE_GLU_M if act else TILE_RAGGED_M if N % 256 else TILE_EVEN_M) or tiles <= (512 if act else 256):
             return None
-        if form != "glu" and N % 256 == 0:
+        if not act and N % 256 == 0:
             gain = 0.8
     best = None
     for (mt, nt), (launch, rnd, unit, out) in TILES.items():
@@ -421,7 +421,7 @@ def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) 
             continue                # (a wave holds whole gate, up pairs)
         items = -(-M // (32 * mt)) * -(-N // (32 * nt))
         for s in TILE_SPLITS:
-            if K // 64 < 2 * s or (s > 1 and 4 * s * M * N > TILE_SLAB_BYTES):
+            if K // 64 < 2 * s or s > 1 and (form == "relu2" or 4 * s * M * N > TILE_SLAB_BYTES):
                 break
             mb = M * N / 4.5e6
             t = launch + -(-items * s // 256) * (rnd + unit * (K // 64) / s) + out * mb * (4 * s if s > 1 else 2)
@@ -432,8 +432,8 @@ def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) 
     if library and M > 1024:
         rows = M // DENSE_BLOCK * DENSE_BLOCK if dense_cut(M, N, K) else M
         lib = 4 + -(-(-(-rows // 256) * -(-N // 256)) // 256) * 1.42 * (K // 64) + (20 if rows < M else 0)
-        if form == "glu":           # (the activation's launch and its way to memory and back)
-            lib += 5 + 3 * M * N / 4.5e6
+        if act:                     # (the activation's launch and its way to memory and back)
+            lib += 5 + (3 if form == "glu" else 4) * M * N / 4.5e6
         if best[0] > lib * gain:
             return None
     return best[1]
@@ -446,13 +446,13 @@ def tile_ok(x: torch.Tensor, wt: torch.Tensor | None) -> bool:
         x.stride(0) % 8 == 0 and x.stride(0) < 1 << 22 and x.data_ptr() % 16 == 0 and wt.is_contiguous()
 
 
-def linear_tile(x: torch.Tensor, wt: torch.Tensor, plan: tuple[int, int, int], glu: bool = False) -> torch.Tensor:
+def linear_tile(x: torch.Tensor, wt: torch.Tensor, plan: tuple[int, int, int], glu: bool = False, relu2: bool = False) -> torch.Tensor:
     """x @ W^T from the wave-tiled weight: bf16 [M, N] for a plan of one split (``glu``: W tiled with glu=True, silu(gate) * up
-    [M, N / 2]), else fp32 slabs [S, M, N] (gate | up order)."""
+    [M, N / 2]; ``relu2``: relu squared), else fp32 slabs [S, M, N] (gate | up order)."""
     M, N, (mt, nt, s) = x.shape[0], wt.shape[0] * 32, plan
     if s == 1:
         y = torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
-        ext().tile_gemm(x, wt, y, None, mt, nt, 1, glu)
+        ext().tile_gemm(x, wt, y, None, mt, nt, 1, glu, relu2)
         return y
     p = torch.empty(s, M, N, dtype=torch.float32, device=x.device)
     ext().tile_gemm(x, wt, None, p, mt, nt, s, glu)
@@ -477,6 +477,12 @@ def linear_glu_long(x: torch.Tensor, wt: torch.Tensor) -> torch.Tensor | None:
         return None
     y = linear_tile(x, wt, plan, glu=True)
     return y if plan[2] == 1 else silu_mul(y)
+
+
+def linear_relu2_long(x: torch.Tensor, wt: torch.Tensor) -> torch.Tensor | None:
+    """relu(x @ W^T)^2 of a long step, None where the tile kernel does not take it."""
+    plan = tile_plan(x.shape[0], wt.shape[0] * 32, x.shape[1], "relu2") if tile_ok(x, wt) else None
+    return None if plan is None else linear_tile(x, wt, plan, relu2=True)
 
 
 def linear_skinny(x: torch.Tensor, wt: torch.Tensor, max_splits: int = 8, glu: bool = False) -> torch.Tensor:

@@ -726,16 +726,16 @@ static void small_gemm(at::Tensor x, at::Tensor w, at::Tensor out, c10::optional
 }
 
 // Dense products of long steps (csrc/tile_gemm.hip) on tiles of 32 mt x 32 nt: y bf16 [M, N] (glu: [M, N / 2] activated) or
-// fp32 split-K slabs p [splits, M, N]
+// fp32 split-K slabs p [splits, M, N]; relu2: y's elements through relu, squared
 static void tile_gemm(at::Tensor x, at::Tensor wt, c10::optional<at::Tensor> y, c10::optional<at::Tensor> p, int64_t mt,
-                      int64_t nt, int64_t splits, bool glu) {
+                      int64_t nt, int64_t splits, bool glu, bool relu2) {
   CHECK_CUDA(x); CHECK_DT(x, at::kBFloat16); CHECK_CUDA(wt); CHECK_DT(wt, at::kBFloat16); CHECK_LASTDIM(x);
   TORCH_CHECK(x.dim() == 2, "tile_gemm: x must be [M, K]");
   TORCH_CHECK(wt.dim() == 4 && wt.is_contiguous() && wt.size(2) == 64 && wt.size(3) == 8,
               "tile_gemm: wt must be contiguous [N/32, K/16, 64, 8]");
   const int64_t M = x.size(0), K = x.size(1), N = wt.size(0) * 32;
   TORCH_CHECK(wt.size(1) * 16 == K && M < (1 << 28) && (M < 2 || x.stride(0) >= K), "tile_gemm: shape");
-  TORCH_CHECK(y.has_value() != p.has_value(), "tile_gemm: one output");
+  TORCH_CHECK(y.has_value() != p.has_value() && !(relu2 && (glu || p.has_value())), "tile_gemm: one output, one activation");
   bf16* yp = nullptr; float* pp = nullptr; int64_t ldy = 0;
   if (y.has_value()) {
     CHECK_DT(y.value(), at::kBFloat16); CHECK_CUDA(y.value()); CHECK_LASTDIM(y.value());
@@ -748,7 +748,7 @@ static void tile_gemm(at::Tensor x, at::Tensor wt, c10::optional<at::Tensor> y, 
     pp = p->data_ptr<float>();
   }
   CHECK_HIP(kafka_launch_tile_gemm(bptr(x), x.stride(0), bptr(wt), (int)M, (int)N, (int)K, (int)mt, (int)nt, (int)splits,
-                                   glu ? 1 : 0, yp, ldy, pp, cur_stream()));
+                                   glu ? 1 : relu2 ? 2 : 0, yp, ldy, pp, cur_stream()));
 }
 
 static void skinny_gemm(at::Tensor x, at::Tensor wt, c10::optional<at::Tensor> y, c10::optional<at::Tensor> p,
@@ -1244,7 +1244,8 @@ PYBIND11_MODULE(_kafka_ops, m) {
         py::arg("v_cache"), py::arg("slots"), py::arg("Hq"), py::arg("Hkv"), py::arg("max_splits"),
         py::arg("stamps") = py::none());
   m.def("skinny_plan", &skinny_plan);
-  m.def("tile_gemm", &tile_gemm);
+  m.def("tile_gemm", &tile_gemm, py::arg("x"), py::arg("wt"), py::arg("y"), py::arg("p"), py::arg("mt"), py::arg("nt"), py::arg("splits"),
+        py::arg("glu"), py::arg("relu2") = false);
   m.def("small_gemm", &small_gemm, py::arg("x"), py::arg("w"), py::arg("out"), py::arg("bias") = c10::nullopt);
   m.def("skinny_gemm", &skinny_gemm);
   m.def("wstream_gemm_cfg", &wstream_gemm_cfg);

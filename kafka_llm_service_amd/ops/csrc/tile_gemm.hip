@@ -12,7 +12,7 @@
 namespace kafka {
 namespace tg {
 
-enum { OUT_BF16 = 0, OUT_SLAB = 1, OUT_GLU = 2, OUT_SLAB_GLU = 3 };
+enum { OUT_BF16 = 0, OUT_SLAB = 1, OUT_GLU = 2, OUT_SLAB_GLU = 3, OUT_RELU2 = 4 };
 
 // MT, NT: 16-row and 16-column parts of a wave's tile (2 x 2 waves); OCC workgroups on a CU
 template <int MT, int NT, int OCC>
@@ -58,10 +58,13 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const bf16* __restr
 #pragma unroll
     for (int t = 0; t < NT / 2; ++t) {
       if (nb + t >= nall) continue;
-      if (mode == OUT_BF16) {
+      if (mode == OUT_BF16 || mode == OUT_RELU2) {
         bf16x8 o;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = (bf16)acc[mt][2 * t + (i >> 2)][i & 3];
+        for (int i = 0; i < 8; ++i) {
+          const float a = acc[mt][2 * t + (i >> 2)][i & 3], p = a < 0.f ? 0.f : a;   // (not a number stays)
+          o[i] = (bf16)(mode == OUT_RELU2 ? p * p : a);
+        }
         *reinterpret_cast<bf16x8*>(Y + (int64_t)(row0 + m) * ldy + (nb + t) * 32 + 8 * q) = o;
       } else if (mode == OUT_GLU) {                // tiles of 32: gate, up, gate, up
         if (t & 1) continue;
@@ -83,15 +86,18 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const bf16* __restr
   }
 }
 
+// act: 1 W tiled as gate, up pairs (silu(gate) * up into Y, slabs in gate | up order), 2 relu squared into Y
 extern "C" hipError_t kafka_launch_tile_gemm(const bf16* X, int64_t ldx, const bf16* Wt, int M, int N, int K, int mt, int nt,
-                                             int splits, int glu, bf16* Y, int64_t ldy, float* P, hipStream_t st) {
+                                             int splits, int act, bf16* Y, int64_t ldy, float* P, hipStream_t st) {
   if (M <= 0) return hipSuccess;
+  const bool glu = act == 1;
+  if (act < 0 || act > 2 || (act == 2 && P)) return hipErrorInvalidValue;
   if (N < 32 || N % 32 || K % 64 || splits < 1 || K / 64 < 2 * splits || ldx % 8 || (glu && N % 64)) return hipErrorInvalidValue;
   if ((Y != nullptr) == (P != nullptr) || (Y && (splits != 1 || ldy % 8 || reinterpret_cast<uintptr_t>(Y) % 16)))
     return hipErrorInvalidValue;
   if (reinterpret_cast<uintptr_t>(X) % 16 || 256 * ldx * 2 > (int64_t)0xffff0000 || (int64_t)N * K * 2 > (int64_t)0xffff0000)
     return hipErrorInvalidValue;
-  const int mode = P ? (glu ? OUT_SLAB_GLU : OUT_SLAB) : (glu ? OUT_GLU : OUT_BF16);
+  const int mode = P ? (glu ? OUT_SLAB_GLU : OUT_SLAB) : (glu ? OUT_GLU : act ? OUT_RELU2 : OUT_BF16);
   const int64_t total = (int64_t)((M + 32 * mt - 1) / (32 * mt)) * ((N + 32 * nt - 1) / (32 * nt)) * splits;
   if (total > 0x0fffffff) return hipErrorInvalidValue;
   const unsigned grid = (unsigned)((total + 7) / 8 * 8);

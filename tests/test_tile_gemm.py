@@ -13,20 +13,21 @@ def test_plans_are_launches():
     rng = random.Random(3)
     for _ in range(300):
         M, N, K = rng.randint(1, 9000), 32 * rng.randint(1, 900), 64 * rng.randint(2, 230)
-        form = rng.choice(["slabs", "bf16", "glu"])
+        form = rng.choice(["slabs", "bf16", "glu", "relu2"])
         plan = ops.tile_plan(M, N, K, form, library=False)
         if form == "glu" and N % 64:
             assert plan is None
             continue
         mt, nt, s = plan
         assert (mt, nt) in ops.TILES and K // 64 >= 2 * s and (form != "glu" or nt % 4 == 0)
-        assert s == 1 or 4 * s * M * N <= ops.TILE_SLAB_BYTES
+        assert s == 1 or form != "relu2" and 4 * s * M * N <= ops.TILE_SLAB_BYTES
     assert ops.tile_plan(300, 4100, 4096) is None and ops.tile_plan(300, 4096, 64) is None and ops.tile_plan(300, 4096, 4112) is None
     assert ops.tile_plan(0, 4096, 4096) is None and ops.tile_plan(300, 32800, 65536, library=False) is None   # 4 GB of weights
     for M, N, form, taken in ((2561, 6176, "bf16", True), (8448, 6176, "slabs", True), (8449, 6176, "bf16", False),   # ragged columns
                               (2561, 6144, "bf16", True), (5600, 9216, "bf16", False), (2700, 28672, "bf16", False),   # whole ones: a fifth less
                               (4096, 4064, "bf16", False), (2816, 5920, "bf16", True),      # one round of 256 x 256 tiles, and a bit more
                               (2561, 28672, "glu", True), (3600, 28672, "glu", True), (3601, 28672, "glu", False),
+                              (2561, 14336, "relu2", True), (3601, 14336, "relu2", False), (2816, 11776, "relu2", False),
                               (2816, 11776, "glu", False)):                             # two rounds
         assert (ops.tile_plan(M, N, 4096, form) is not None) == taken, (M, N, form)
     assert ops.tile_plan(300, 28672, 4096) is None and ops.tile_plan(300, 28672, 4096, "glu") is not None
@@ -39,6 +40,7 @@ def test_long_products_on_the_cpu():
     for x in (torch.randn(150, 128), torch.randn(128, 150).t(), torch.randn(150, 256)[:, ::2], torch.randn(1, 128).expand(150, 128)):
         for y in (ops.linear_long(x, w, wt, slabs=True), ops.linear_long(x, None, wt), ops.linear_long(x, w, None)):
             torch.testing.assert_close(y, x @ w.t())
+    assert ops.linear_relu2_long(torch.randn(150, 128), wt) is None
     assert ops.linear_glu_long(torch.randn(150, 128), ops.tile_weight(torch.randn(128, 128), glu=True)) is None
 
 
@@ -67,6 +69,7 @@ def test_tiles_against_fp32(mt, nt):
         ext.tile_gemm(x, wt, y[:M, :N], None, mt, nt, 1, False)
         _close(y[:M, :N], want, K)
         assert (y[M:] == 7).all() and (y[:, N:] == 7).all()
+        _close(ops.linear_tile(x, wt, (mt, nt, 1), relu2=True), want.relu() ** 2, K)
         if s > 1:
             p = ops.linear_tile(x, wt, (mt, nt, s))
             assert p.shape == (s, M, N) and ((p.sum(0) - want).abs() <= 1e-4).all()
@@ -78,8 +81,17 @@ def test_tiles_against_fp32(mt, nt):
 
 
 @pytest.mark.gpu
+def test_relu_squared_of_what_is_not_finite():
+    """NaN stays, minus infinity is zero, plus infinity infinite."""
+    x = torch.ones(200, 128, dtype=torch.bfloat16, device="cuda")
+    x[0, 0], x[1, 0], x[2, 0] = float("nan"), float("inf"), float("-inf")
+    y = ops.linear_tile(x, ops.tile_weight(torch.ones(64, 128, dtype=torch.bfloat16, device="cuda")), (4, 4, 1), relu2=True)
+    assert y[0].isnan().all() and (y[1] == float("inf")).all() and (y[2] == 0).all() and (y[3:] == 128 ** 2).all()
+
+
+@pytest.mark.gpu
 def test_long_products_by_their_plans():
-    """linear_long and linear_glu_long over sizes of every route (tiles with and without splits, the library) and forms of x that the
+    """linear_long, linear_relu2_long and linear_glu_long over sizes of every route (tiles with and without splits, the library) and forms of x that the
     kernel leaves to the library (odd strides, a shifted start)."""
     g = torch.Generator().manual_seed(0)
     for M, N, K in ((131, 2048, 2048), (300, 4096, 1024), (700, 96, 4096), (1300, 6176, 512), (257, 24608, 128), (3000, 1024, 256),
@@ -91,6 +103,9 @@ def test_long_products_by_their_plans():
             want = x.float() @ w.float().t()
             for y in (ops.linear_long(x, w, wt), ops.linear_long(x, None, wt), ops.linear_long(x, w, wt, slabs=True)):
                 _close(y.sum(0) if ops.is_slab(y) else y, want, K)
+            a = ops.linear_relu2_long(x, wt)
+            if a is not None:
+                _close(a, want.relu() ** 2, K)
             if N % 64 == 0:
                 a = ops.linear_glu_long(x, ops.tile_weight(w, glu=True))
                 if a is not None:

@@ -383,6 +383,7 @@ TILE_SPLITS = (1, 2, 4, 8)      # what the consumers of slabs load with all slab
 TILE_SLAB_BYTES = 1 << 28
 TILE_LIBRARY_N, TILE_MAX_M = 24576, 2560
 TILE_GLU_M, TILE_EVEN_M, TILE_RAGGED_M = 3600, 5600, 8448
+TILE_WHOLE_GAIN = 0.8
 
 
 @lru_cache(maxsize=4096)
@@ -394,13 +395,15 @@ def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) 
     Against the library (us, library / this kernel): 450 rows of 14336 -> 4096 89 / 55, 2048 rows 202 / 178; 2048 rows of 4096 -> 18560 350 / 277,
     200 rows 57 / 45; 900 rows of 2048 -> 9344 45 / 36; 450 rows of 2048 -> 2048 19 / 11; over all timed shapes 13 % less time with slabs,
     9 % as bf16. The library's: very wide outputs of 257 - 1024 rows (28672 columns: 320 rows 74 / 78, 640 135 / 149); beyond
-    them, where its 256 x 256 tiles (1.42 us a round and 64 of K) fill their rounds (28672: 1536 rows 264 / 293, 4099 722 / 774; 2048 -> 7168,
-    2048 rows 49 / 62), which ragged columns (no multiple of 256) do not (10816: 2048 rows 164 / 151).
+    768, where its 256 x 256 tiles (1.42 us a round and 64 of K) fill their rounds: past one round whole columns (multiples of 256) take this
+    kernel only where the model says a fifth less (28672: 1536 rows 264 / 293, with the activation 272 / 304, 900 rows 189 / 198, 4099 722 / 774; 14336:
+    1903 rows 162 / 190; where the model says a fifth to a twentieth less, 11 % more over 20 sizes), ragged ones mostly (10816: 2048 rows
+    164 / 151).
 
     Beyond 2560 rows the library's choice of kernel decides. Where its tiles are one round or less it is as fast or faster (4096 -> 4096: 2716 rows
     73 / 74, 4096 91 / 100). Beyond a round ragged columns take this kernel (4096 -> 18560: 3182 rows 500 / 378, 4096 560 / 461; 12320: 2593 333 /
-    221, 7583 538 / 576; 2048 -> 9344: 4096 180 / 155; over 130 sizes up to 8192 rows 9 % less time), whole ones up to 5600 rows where the model says
-    a fifth less (6144: 2716 rows 205 / 120, 4096 158 / 156; over 28 sizes 9 % less, the others 6 % more). Gate and up with their
+    221, 7583 538 / 576; 2048 -> 9344: 4096 180 / 155; over 130 sizes up to 8192 rows 9 % less time), whole ones up to 5600 rows by the rule above
+    (6144: 2716 rows 205 / 120, 4096 158 / 156; over 28 sizes 9 % less, the others 6 % more). Gate and up with their
     activation: up to 3600 rows from two rounds on (28672: 2716 rows 593 / 508, 3182 716 / 596, 3600 - 4200 3 % more; 4096 -> 9216, less
     than two rounds, 5 % more). Steps: llama 2700 rows 5030 -> 4400, 3000 4930 -> 4790, 3300 6050 -> 5480; rogosun 4000 8740 -> 8570, width 2048 2700
     2925 -> 2860; budurax width 2048 2700 2280 -> 2208; furapel 6400 15235 -> 15020."""
@@ -408,13 +411,11 @@ def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) 
         return None
     if library and form == "bf16" and N > TILE_LIBRARY_N and 256 < M <= 1024:
         return None
-    gain, act = 1.25 if N % 256 else 0.95, form in ("glu", "relu2")
-    if library and M > TILE_MAX_M:
-        tiles = -(-M // 256) * -(-N // 256)
-        if M > (TILE_GLU_M if act else TILE_RAGGED_M if N % 256 else TILE_EVEN_M) or tiles <= (512 if act else 256):
-            return None
-        if not act and N % 256 == 0:
-            gain = 0.8
+    act, tiles = form in ("glu", "relu2"), -(-M // 256) * -(-N // 256)
+    gain = 1.25 if N % 256 else 0.95 if tiles <= 256 or act and M > TILE_MAX_M else TILE_WHOLE_GAIN
+    if library and M > TILE_MAX_M and \
+            (M > (TILE_GLU_M if act else TILE_RAGGED_M if N % 256 else TILE_EVEN_M) or tiles <= (512 if act else 256)):
+        return None
     best = None
     for (mt, nt), (launch, rnd, unit, out) in TILES.items():
         if form == "glu" and nt % 4:
@@ -429,7 +430,7 @@ def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) 
                 t += mb * (4 * s - 2) if form == "slabs" else 6 + mb * (4 * s + 2)
             if best is None or t < best[0]:
                 best = (t, (mt, nt, s))
-    if library and M > 1024:
+    if library and M > (768 if tiles > 256 else 1024):
         rows = M // DENSE_BLOCK * DENSE_BLOCK if dense_cut(M, N, K) else M
         lib = 4 + -(-(-(-rows // 256) * -(-N // 256)) // 256) * 1.42 * (K // 64) + (20 if rows < M else 0)
         if act:                     # (the activation's launch and its way to memory and back)

@@ -367,7 +367,9 @@ class BuduraxLM:
             for n in self.STREAMED:
                 w = getattr(lw, n, None)
                 if self._streamable(w):
-                    setattr(lw, n + "_t", ops.tile_weight(w))
+                    if n == "gate_up":
+                        lw.gated = lw.ff % 32 == 0   # (gate, up tiles in turn)
+                    setattr(lw, n + "_t", ops.tile_weight(w, glu=n == "gate_up" and lw.gated))
                     added += w.numel() * w.element_size()
         if self._streamable(self.head):
             self.head_t = ops.tile_weight(self.head)
@@ -386,6 +388,19 @@ class BuduraxLM:
             y = ops.linear_stream(x, wt)
             return ops.slab_reduce(y) if ops.is_slab(y) and not slabs else y
         return ops.linear_long(x, w, wt if self.stream else None, slabs)
+
+    def _gelu_up(self, lw, h):
+        """gelu(h @ gate^T) * (h @ up^T): in the epilogue of the weight-streaming and the tile kernel, beside the library's
+        product and kernels for other tilings a launch of its own."""
+        M, wt, a = h.shape[0], getattr(lw, "gate_up_t", None), None
+        if self.stream and wt is not None and getattr(lw, "gated", False):
+            if 0 < M <= self.stream_max_m and ops.stream_plan(M, lw.gate_up.shape[0], lw.gate_up.shape[1]) is not None:
+                return ops.linear_glu(h, wt, act="gelu")
+            a, wt = ops.linear_glu_long(h, wt, act="gelu"), None
+        if a is None:
+            a = torch.empty(M, lw.ff, dtype=h.dtype, device=h.device)
+            hops.gelu_mul(self._lin(h, lw.gate_up, wt), a)
+        return a
 
     def weight_bytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self._tensors)
@@ -560,9 +575,7 @@ class BuduraxLM:
                 y = self._mamba2(i, lw, h, m, state)
             if lw.gate_up is not None:
                 hops.add_ln(x, y, lw.norm1b, lw.norm1b_b, eps, h2, lw.norm2, lw.norm2_b)
-                a = torch.empty(T, lw.ff, dtype=dt, device=dev)
-                hops.gelu_mul(self._lin(h2, lw.gate_up, getattr(lw, "gate_up_t", None)), a)
-                y = self._lin(a, lw.down, getattr(lw, "down_t", None), slabs=True)
+                y = self._lin(self._gelu_up(lw, h2), lw.down, getattr(lw, "down_t", None), slabs=True)
                 nw, nb = lw.norm2b, lw.norm2b_b
             else:
                 nw, nb = lw.norm1b, lw.norm1b_b

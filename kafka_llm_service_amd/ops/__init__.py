@@ -107,17 +107,17 @@ def gather_rows(table: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
     return table.index_select(0, idx)
 
 
-def silu_mul(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
-    """silu(x[..., :F]) * x[..., F:] (bf16 out); ``x`` may be a split-K slab [S, T, 2F]."""
+def silu_mul(x: torch.Tensor, out: torch.Tensor | None = None, act: str = "silu") -> torch.Tensor:
+    """silu(x[..., :F]) * x[..., F:] (bf16 out; ``act`` "gelu": its tanh form in SiLU's place); ``x`` may be a split-K slab [S, T, 2F]."""
     F = x.shape[-1] // 2
     slab = is_slab(x)
     if out is None:
         lead = (x.shape[1],) if slab else x.shape[:-1]
         out = torch.empty(*lead, F, dtype=torch.bfloat16 if slab else x.dtype, device=x.device)
     if _gpu(x):
-        ext().silu_mul(out.view(-1, F), x if slab else x.reshape(-1, 2 * F))
+        ext().silu_mul(out.view(-1, F), x if slab else x.reshape(-1, 2 * F), act == "gelu")
     else:
-        out.copy_(ref.silu_mul(x.sum(0) if slab else x))
+        out.copy_(ref.silu_mul(x.sum(0) if slab else x, act))
     return out
 
 
@@ -447,13 +447,14 @@ def tile_ok(x: torch.Tensor, wt: torch.Tensor | None) -> bool:
         x.stride(0) % 8 == 0 and x.stride(0) < 1 << 22 and x.data_ptr() % 16 == 0 and wt.is_contiguous()
 
 
-def linear_tile(x: torch.Tensor, wt: torch.Tensor, plan: tuple[int, int, int], glu: bool = False, relu2: bool = False) -> torch.Tensor:
+def linear_tile(x: torch.Tensor, wt: torch.Tensor, plan: tuple[int, int, int], glu: bool = False, relu2: bool = False,
+                act: str = "silu") -> torch.Tensor:
     """x @ W^T from the wave-tiled weight: bf16 [M, N] for a plan of one split (``glu``: W tiled with glu=True, silu(gate) * up
-    [M, N / 2]; ``relu2``: relu squared), else fp32 slabs [S, M, N] (gate | up order)."""
+    [M, N / 2], ``act`` as in ``silu_mul``; ``relu2``: relu squared), else fp32 slabs [S, M, N] (gate | up order)."""
     M, N, (mt, nt, s) = x.shape[0], wt.shape[0] * 32, plan
     if s == 1:
         y = torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
-        ext().tile_gemm(x, wt, y, None, mt, nt, 1, glu, relu2)
+        ext().tile_gemm(x, wt, y, None, mt, nt, 1, glu, relu2, glu and act == "gelu")
         return y
     p = torch.empty(s, M, N, dtype=torch.float32, device=x.device)
     ext().tile_gemm(x, wt, None, p, mt, nt, s, glu)
@@ -471,13 +472,14 @@ def linear_long(x: torch.Tensor, w: torch.Tensor | None, wt: torch.Tensor | None
     return linear_dense(x, w if w is not None else untile_weight(wt))
 
 
-def linear_glu_long(x: torch.Tensor, wt: torch.Tensor) -> torch.Tensor | None:
-    """silu(x @ Wg^T) * (x @ Wu^T) of a long step from GLU-tiled weights, None where the tile kernel does not take it."""
+def linear_glu_long(x: torch.Tensor, wt: torch.Tensor, act: str = "silu") -> torch.Tensor | None:
+    """silu(x @ Wg^T) * (x @ Wu^T) of a long step from GLU-tiled weights (``act`` as in ``silu_mul``), None where the tile kernel does
+    not take it."""
     plan = tile_plan(x.shape[0], wt.shape[0] * 32, x.shape[1], "glu") if tile_ok(x, wt) else None
     if plan is None:
         return None
-    y = linear_tile(x, wt, plan, glu=True)
-    return y if plan[2] == 1 else silu_mul(y)
+    y = linear_tile(x, wt, plan, glu=True, act=act)
+    return y if plan[2] == 1 else silu_mul(y, act=act)
 
 
 def linear_relu2_long(x: torch.Tensor, wt: torch.Tensor) -> torch.Tensor | None:
@@ -512,11 +514,11 @@ def linear_skinny(x: torch.Tensor, wt: torch.Tensor, max_splits: int = 8, glu: b
 
 
 def linear_stream(x: torch.Tensor, wt: torch.Tensor, max_splits: int = 8, nt: bool = True,
-                  glu: bool = False) -> torch.Tensor:
+                  glu: bool = False, act: str = "silu") -> torch.Tensor:
     """y = x @ W^T for decode-sized M (<= 128) from the wave-tiled weight ``wt``: the weight-streaming MFMA kernel.
     Returns bf16 [M, N] when the plan has one split, else the fp32 split-K slabs [S, M, N] (a slab; the consumer
     kernels sum it while loading). ``glu`` (wt tiled with glu=True): a one-split plan returns the ACTIVATED
-    silu(gate) * up [M, N/2] (fused epilogue); a split plan returns gate | up slabs as usual (see ``linear_glu``)."""
+    silu(gate) * up [M, N/2] (fused epilogue; ``act`` as in ``silu_mul``); a split plan returns gate | up slabs as usual (see ``linear_glu``)."""
     M, K = x.shape
     N = wt.shape[0] * 32
     plan = stream_plan(M, N, K, max_splits)
@@ -526,7 +528,7 @@ def linear_stream(x: torch.Tensor, wt: torch.Tensor, max_splits: int = 8, nt: bo
     if _gpu(x):
         if S == 1:
             y = torch.empty(M, N // 2 if glu else N, dtype=x.dtype, device=x.device)
-            ext().wstream_gemm(x, wt, y, None, int(max_splits), bool(nt), bool(glu))
+            ext().wstream_gemm(x, wt, y, None, int(max_splits), bool(nt), (2 if act == "gelu" else 1) if glu else 0)
             return y
         p = torch.empty(S, M, N, dtype=torch.float32, device=x.device)
         ext().wstream_gemm(x, wt, None, p, int(max_splits), bool(nt), bool(glu))
@@ -536,19 +538,19 @@ def linear_stream(x: torch.Tensor, wt: torch.Tensor, max_splits: int = 8, nt: bo
     if S == 1:
         y = xf @ w.t()
         if glu:
-            return ref.silu_mul(y).to(x.dtype)
+            return ref.silu_mul(y, act).to(x.dtype)
         return y.to(x.dtype)
     ks = K // S
     return torch.stack([xf[:, s * ks:(s + 1) * ks] @ w[:, s * ks:(s + 1) * ks].t() for s in range(S)])
 
 
-def linear_glu(x: torch.Tensor, wt: torch.Tensor, max_splits: int = 8) -> torch.Tensor:
+def linear_glu(x: torch.Tensor, wt: torch.Tensor, max_splits: int = 8, act: str = "silu") -> torch.Tensor:
     """silu(x @ Wg^T) * (x @ Wu^T) from GLU-tiled gate_up weights: fused into the GEMM epilogue when the plan has one
-    split, else the GEMM's slabs go through silu_mul."""
+    split, else the GEMM's slabs go through silu_mul (``act`` as there)."""
     N = wt.shape[0] * 32
     plan = stream_plan(x.shape[0], N, x.shape[1], max_splits)
-    y = linear_stream(x, wt, max_splits, glu=True)
-    return y if plan is not None and plan[2] == 1 else silu_mul(y)
+    y = linear_stream(x, wt, max_splits, glu=True, act=act)
+    return y if plan is not None and plan[2] == 1 else silu_mul(y, act=act)
 
 
 # ---- fused decode layer (csrc/wstream_gemm.hip FIN_*): deferred RMSNorm + split-K finishers ----------------------

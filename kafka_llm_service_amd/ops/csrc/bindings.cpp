@@ -19,8 +19,8 @@ hipError_t kafka_launch_rows_norm(bf16* out, int64_t os, const bf16* x, int64_t 
                                   hipStream_t st);
 hipError_t kafka_launch_gather_rows(void* out, int64_t out_bytes, const void* src, int64_t src_bytes, const int64_t* idx,
                                     int64_t n_src, int n, int row_bytes, hipStream_t st);
-hipError_t kafka_launch_silu_mul(bf16* out, const bf16* x, int64_t xs, int T, int F, hipStream_t st);
-hipError_t kafka_launch_silu_mul_slab(bf16* out, const float* xp, int S, int64_t ps, int T, int F, hipStream_t st);
+hipError_t kafka_launch_silu_mul(bf16* out, const bf16* x, int64_t xs, int T, int F, int gelu, hipStream_t st);
+hipError_t kafka_launch_silu_mul_slab(bf16* out, const float* xp, int S, int64_t ps, int T, int F, int gelu, hipStream_t st);
 hipError_t kafka_launch_rope_kv(const bf16* qkv, const float* qp, int S, int64_t ps, int64_t qkv_stride,
                                 const int64_t* positions, const float* cos_sin, bf16* q_out, int64_t q_stride,
                                 bf16* k_cache, bf16* v_cache, const int64_t* slot_mapping, int T, int Hq, int Hkv,
@@ -223,8 +223,8 @@ static void gather_rows(at::Tensor out, at::Tensor src, at::Tensor idx) {
                                      src.size(0), (int)idx.size(0), (int)row, cur_stream()));
 }
 
-// x: bf16 [T, 2F] or slab [S, T, 2F]
-static void silu_mul(at::Tensor out, at::Tensor x) {
+// x: bf16 [T, 2F] or slab [S, T, 2F]; gelu: its tanh form in SiLU's place
+static void silu_mul(at::Tensor out, at::Tensor x, bool gelu) {
   CHECK_CUDA(x); CHECK_DT(out, at::kBFloat16);
   const bool slab = is_slab(x);
   if (slab) check_slab(x); else CHECK_DT(x, at::kBFloat16);
@@ -234,9 +234,9 @@ static void silu_mul(at::Tensor out, at::Tensor x) {
   const int64_t T = x.size(slab ? 1 : 0);
   TORCH_CHECK(x.size(slab ? 2 : 1) == 2 * F && F % 8 == 0 && out.size(0) == T, "silu_mul: bad shapes");
   if (slab)
-    CHECK_HIP(kafka_launch_silu_mul_slab(bptr(out), x.data_ptr<float>(), x.size(0), T * 2 * F, T, F, cur_stream()));
+    CHECK_HIP(kafka_launch_silu_mul_slab(bptr(out), x.data_ptr<float>(), x.size(0), T * 2 * F, T, F, gelu ? 1 : 0, cur_stream()));
   else
-    CHECK_HIP(kafka_launch_silu_mul(bptr(out), bptr(x), x.stride(0), T, F, cur_stream()));
+    CHECK_HIP(kafka_launch_silu_mul(bptr(out), bptr(x), x.stride(0), T, F, gelu ? 1 : 0, cur_stream()));
 }
 
 // Paged KV caches: bf16 K[blocks, Hkv, 16, 128] / V[blocks, Hkv, 128, 16], or fp8 (e4m3 + per-token exponents,
@@ -546,13 +546,14 @@ static std::vector<int64_t> wstream_plan(int64_t M, int64_t N, int64_t K, int64_
 // x [M, K] bf16 . W^T with W given wave-tiled as wt [N/32, K/16, 64, 8] (ops.tile_weight). Writes bf16 y [M, N]
 // (splits == 1) or fp32 slabs p [splits, M, N].
 static void wstream_gemm(at::Tensor x, at::Tensor wt, c10::optional<at::Tensor> y, c10::optional<at::Tensor> p,
-                         int64_t max_splits, bool nt, bool glu) {
+                         int64_t max_splits, bool nt, int64_t glu) {
   CHECK_CUDA(x); CHECK_DT(x, at::kBFloat16); CHECK_DT(wt, at::kBFloat16); CHECK_LASTDIM(x);
   TORCH_CHECK(x.dim() == 2 && x.stride(0) % 8 == 0, "wstream_gemm: x must be [M, K] with 16-B rows");
   TORCH_CHECK(wt.dim() == 4 && wt.is_contiguous() && wt.size(2) == 64 && wt.size(3) == 8,
               "wstream_gemm: wt must be contiguous [N/32, K/16, 64, 8]");
   const int M = x.size(0), K = x.size(1), N = wt.size(0) * 32;
   TORCH_CHECK(wt.size(1) * 16 == K, "wstream_gemm: K mismatch");
+  TORCH_CHECK(glu >= 0 && glu <= 2, "wstream_gemm: glu 0 (none), 1 (SiLU) or 2 (GELU)");
   TORCH_CHECK(!glu || N % 64 == 0, "wstream_gemm: GLU weights need N % 64 == 0");
   int mt = 0, kc = 0, s = 0;
   TORCH_CHECK(kafka_wstream_plan(M, N, K, (int)max_splits, &mt, &kc, &s) == 0, "wstream_gemm: unsupported shape");
@@ -583,7 +584,7 @@ static void wstream_gemm(at::Tensor x, at::Tensor wt, c10::optional<at::Tensor> 
   // (profiles/r05/wstream_sweep_pin.jsonl)
   const int pin = mt != 3 && K / s / kc >= 3 ? 1 : 0;
   CHECK_HIP(kafka_launch_wstream_gemm(bptr(x), x.stride(0), bptr(wt), M, N, K, mt, kc, s, nt ? 1 : 0, kw, pin,
-                                      glu ? 1 : 0,
+                                      (int)glu,
                                       yp, ldy, pp, cur_stream()));
 }
 
@@ -728,14 +729,14 @@ static void small_gemm(at::Tensor x, at::Tensor w, at::Tensor out, c10::optional
 // Dense products of long steps (csrc/tile_gemm.hip) on tiles of 32 mt x 32 nt: y bf16 [M, N] (glu: [M, N / 2] activated) or
 // fp32 split-K slabs p [splits, M, N]; relu2: y's elements through relu, squared
 static void tile_gemm(at::Tensor x, at::Tensor wt, c10::optional<at::Tensor> y, c10::optional<at::Tensor> p, int64_t mt,
-                      int64_t nt, int64_t splits, bool glu, bool relu2) {
+                      int64_t nt, int64_t splits, bool glu, bool relu2, bool gelu) {
   CHECK_CUDA(x); CHECK_DT(x, at::kBFloat16); CHECK_CUDA(wt); CHECK_DT(wt, at::kBFloat16); CHECK_LASTDIM(x);
   TORCH_CHECK(x.dim() == 2, "tile_gemm: x must be [M, K]");
   TORCH_CHECK(wt.dim() == 4 && wt.is_contiguous() && wt.size(2) == 64 && wt.size(3) == 8,
               "tile_gemm: wt must be contiguous [N/32, K/16, 64, 8]");
   const int64_t M = x.size(0), K = x.size(1), N = wt.size(0) * 32;
   TORCH_CHECK(wt.size(1) * 16 == K && M < (1 << 28) && (M < 2 || x.stride(0) >= K), "tile_gemm: shape");
-  TORCH_CHECK(y.has_value() != p.has_value() && !(relu2 && (glu || p.has_value())), "tile_gemm: one output, one activation");
+  TORCH_CHECK(y.has_value() != p.has_value() && !(relu2 && (glu || p.has_value())) && !(gelu && !glu), "tile_gemm: one output, one activation");
   bf16* yp = nullptr; float* pp = nullptr; int64_t ldy = 0;
   if (y.has_value()) {
     CHECK_DT(y.value(), at::kBFloat16); CHECK_CUDA(y.value()); CHECK_LASTDIM(y.value());
@@ -748,7 +749,7 @@ static void tile_gemm(at::Tensor x, at::Tensor wt, c10::optional<at::Tensor> y, 
     pp = p->data_ptr<float>();
   }
   CHECK_HIP(kafka_launch_tile_gemm(bptr(x), x.stride(0), bptr(wt), (int)M, (int)N, (int)K, (int)mt, (int)nt, (int)splits,
-                                   glu ? 1 : relu2 ? 2 : 0, yp, ldy, pp, cur_stream()));
+                                   glu ? (gelu ? 3 : 1) : relu2 ? 2 : 0, yp, ldy, pp, cur_stream()));
 }
 
 static void skinny_gemm(at::Tensor x, at::Tensor wt, c10::optional<at::Tensor> y, c10::optional<at::Tensor> p,
@@ -1220,7 +1221,7 @@ PYBIND11_MODULE(_kafka_ops, m) {
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
   m.def("rows_norm", &rows_norm);
   m.def("gather_rows", &gather_rows);
-  m.def("silu_mul", &silu_mul);
+  m.def("silu_mul", &silu_mul, py::arg("out"), py::arg("x"), py::arg("gelu") = false);
   m.def("rope_kv_write", &rope_kv_write);
   m.def("attn_decode", &attn_decode, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
         py::arg("items"), py::arg("out_part"), py::arg("lse_part"), py::arg("scale"), py::arg("out"),
@@ -1245,7 +1246,7 @@ PYBIND11_MODULE(_kafka_ops, m) {
         py::arg("stamps") = py::none());
   m.def("skinny_plan", &skinny_plan);
   m.def("tile_gemm", &tile_gemm, py::arg("x"), py::arg("wt"), py::arg("y"), py::arg("p"), py::arg("mt"), py::arg("nt"), py::arg("splits"),
-        py::arg("glu"), py::arg("relu2") = false);
+        py::arg("glu"), py::arg("relu2") = false, py::arg("gelu") = false);
   m.def("small_gemm", &small_gemm, py::arg("x"), py::arg("w"), py::arg("out"), py::arg("bias") = c10::nullopt);
   m.def("skinny_gemm", &skinny_gemm);
   m.def("wstream_gemm_cfg", &wstream_gemm_cfg);

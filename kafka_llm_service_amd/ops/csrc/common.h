@@ -163,6 +163,12 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+// act(g) = g / (1 + e^-s) of the gated feed-forwards: s = g (SiLU), or with gelu that of the tanh form of GELU
+__device__ __forceinline__ float gate_act(float g, bool gelu) {
+  const float s = gelu ? 1.5957691216057308f * (g + 0.044715f * g * g * g) : g;
+  return g / (1.0f + __expf(-s));
+}
+
 // Counter-based RNG (splitmix64 finaliser): deterministic given (seed, stream, index).
 __device__ __forceinline__ uint64_t mix64(uint64_t z) {
   z += 0x9E3779B97F4A7C15ull;

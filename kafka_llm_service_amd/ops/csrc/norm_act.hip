@@ -76,7 +76,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(bf16* __restrict__ out, int
 // out[t, :] = silu(x[t, :F]) * x[t, F:]   (x: [T, 2F] row stride xs (bf16 or slabs), out: [T, F] contiguous)
 __global__ __launch_bounds__(256) void silu_mul_kernel(bf16* __restrict__ out, const bf16* __restrict__ x,
                                                         const float* __restrict__ xp, int S, int64_t ps,
-                                                        int64_t xs, int F) {
+                                                        int64_t xs, int F, bool gelu) {
   const int64_t row = blockIdx.y;
   const int nvec = F >> 3;
   for (int vi = blockIdx.x * 256 + threadIdx.x; vi < nvec; vi += gridDim.x * 256) {
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(bf16* __restrict__ out, c
     load_in8(u, x, xp, S, ps, row * xs + F + vi * 8);
     bf16x8 o;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = (bf16)(g[j] / (1.0f + __expf(-g[j])) * u[j]);
+    for (int j = 0; j < 8; ++j) o[j] = (bf16)(gate_act(g[j], gelu) * u[j]);
     store_bf16x8(out + row * (int64_t)F + vi * 8, o);
   }
 }
@@ -241,23 +241,23 @@ extern "C" hipError_t kafka_launch_fused_add_rmsnorm_slab(bf16* out, int64_t os,
   return launch_rmsnorm_t<true>(out, os, nullptr, xp, S, ps, d, resid, rs, w, T, d, eps, st);
 }
 
-extern "C" hipError_t kafka_launch_silu_mul(bf16* out, const bf16* x, int64_t xs, int T, int F, hipStream_t st) {
+extern "C" hipError_t kafka_launch_silu_mul(bf16* out, const bf16* x, int64_t xs, int T, int F, int gelu, hipStream_t st) {
   if (T == 0) return hipSuccess;
   const int nvec = F / 8;
   int gx = (nvec + 255) / 256;
   if (gx > 64) gx = 64;
-  silu_mul_kernel<<<dim3(gx, T), dim3(256), 0, st>>>(out, x, nullptr, 0, 0, xs, F);
+  silu_mul_kernel<<<dim3(gx, T), dim3(256), 0, st>>>(out, x, nullptr, 0, 0, xs, F, gelu != 0);
   return hipGetLastError();
 }
 
 // SwiGLU over S fp32 split-K slabs [S][T][2F]
 extern "C" hipError_t kafka_launch_silu_mul_slab(bf16* out, const float* xp, int S, int64_t ps, int T, int F,
-                                                hipStream_t st) {
+                                                int gelu, hipStream_t st) {
   if (T == 0) return hipSuccess;
   const int nvec = F / 8;
   int gx = (nvec + 255) / 256;
   if (gx > 64) gx = 64;
-  silu_mul_kernel<<<dim3(gx, T), dim3(256), 0, st>>>(out, nullptr, xp, S, ps, 2 * (int64_t)F, F);
+  silu_mul_kernel<<<dim3(gx, T), dim3(256), 0, st>>>(out, nullptr, xp, S, ps, 2 * (int64_t)F, F, gelu != 0);
   return hipGetLastError();
 }
 

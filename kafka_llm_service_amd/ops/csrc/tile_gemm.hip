@@ -12,7 +12,7 @@
 namespace kafka {
 namespace tg {
 
-enum { OUT_BF16 = 0, OUT_SLAB = 1, OUT_GLU = 2, OUT_SLAB_GLU = 3, OUT_RELU2 = 4 };
+enum { OUT_BF16 = 0, OUT_SLAB = 1, OUT_GLU = 2, OUT_SLAB_GLU = 3, OUT_RELU2 = 4, OUT_GELU = 5 };
 
 // MT, NT: 16-row and 16-column parts of a wave's tile (2 x 2 waves); OCC workgroups on a CU
 template <int MT, int NT, int OCC>
@@ -66,13 +66,13 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const bf16* __restr
           o[i] = (bf16)(mode == OUT_RELU2 ? p * p : a);
         }
         *reinterpret_cast<bf16x8*>(Y + (int64_t)(row0 + m) * ldy + (nb + t) * 32 + 8 * q) = o;
-      } else if (mode == OUT_GLU) {                // tiles of 32: gate, up, gate, up
+      } else if (mode == OUT_GLU || mode == OUT_GELU) {                // tiles of 32: gate, up, gate, up
         if (t & 1) continue;
         bf16x8 o;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const float a = acc[mt][2 * t + (i >> 2)][i & 3], b = acc[mt][(2 * t + 2 + (i >> 2)) % NT][i & 3];
-          o[i] = (bf16)(a / (1.0f + __expf(-a)) * b);
+          o[i] = (bf16)(gate_act(a, mode == OUT_GELU) * b);
         }
         *reinterpret_cast<bf16x8*>(Y + (int64_t)(row0 + m) * ldy + ((nb + t) >> 1) * 32 + 8 * q) = o;
       } else {
@@ -86,18 +86,18 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const bf16* __restr
   }
 }
 
-// act: 1 W tiled as gate, up pairs (silu(gate) * up into Y, slabs in gate | up order), 2 relu squared into Y
+// act: 1, 3 W tiled as gate, up pairs (silu or gelu(gate) * up into Y, slabs in gate | up order), 2 relu squared into Y
 extern "C" hipError_t kafka_launch_tile_gemm(const bf16* X, int64_t ldx, const bf16* Wt, int M, int N, int K, int mt, int nt,
                                              int splits, int act, bf16* Y, int64_t ldy, float* P, hipStream_t st) {
   if (M <= 0) return hipSuccess;
-  const bool glu = act == 1;
-  if (act < 0 || act > 2 || (act == 2 && P)) return hipErrorInvalidValue;
+  const bool glu = act & 1;
+  if (act < 0 || act > 3 || (act == 2 && P)) return hipErrorInvalidValue;
   if (N < 32 || N % 32 || K % 64 || splits < 1 || K / 64 < 2 * splits || ldx % 8 || (glu && N % 64)) return hipErrorInvalidValue;
   if ((Y != nullptr) == (P != nullptr) || (Y && (splits != 1 || ldy % 8 || reinterpret_cast<uintptr_t>(Y) % 16)))
     return hipErrorInvalidValue;
   if (reinterpret_cast<uintptr_t>(X) % 16 || 256 * ldx * 2 > (int64_t)0xffff0000 || (int64_t)N * K * 2 > (int64_t)0xffff0000)
     return hipErrorInvalidValue;
-  const int mode = P ? (glu ? OUT_SLAB_GLU : OUT_SLAB) : (glu ? OUT_GLU : act ? OUT_RELU2 : OUT_BF16);
+  const int mode = P ? (glu ? OUT_SLAB_GLU : OUT_SLAB) : (act == 1 ? OUT_GLU : act == 2 ? OUT_RELU2 : act == 3 ? OUT_GELU : OUT_BF16);
   const int64_t total = (int64_t)((M + 32 * mt - 1) / (32 * mt)) * ((N + 32 * nt - 1) / (32 * nt)) * splits;
   if (total > 0x0fffffff) return hipErrorInvalidValue;
   const unsigned grid = (unsigned)((total + 7) / 8 * 8);

@@ -538,7 +538,7 @@ __global__ __launch_bounds__(256 * KW) void wstream_gemm_kernel(const bf16* __re
     return;
   }
   if (glu && P == nullptr) {
-    // fused SwiGLU epilogue (weight tiles GLU-interleaved: tile 2j = gate rows [32j, 32j+32), tile 2j+1 = the
+    // fused SwiGLU (glu = 2: GELU-gated) epilogue (weight tiles GLU-interleaved: tile 2j = gate rows [32j, 32j+32), tile 2j+1 = the
     // matching up rows): odd waves hand their up tile to the even wave of the pair through LDS, which writes
     // silu(gate) * up straight from the fp32 accumulators into Y [M, N/2]
     float* red = reinterpret_cast<float*>(&xs[0][0]);
@@ -572,7 +572,7 @@ __global__ __launch_bounds__(256 * KW) void wstream_gemm_kernel(const bf16* __re
             const int m = mt * 32 + (i & 3) + 8 * (i >> 2) + 4 * h;
             const float rr = rrow(m);
             const float g = acc[mt][i] * rr, u = red[(((ct >> 1) * MT + mt) * 16 + i) * 64 + lane] * rr;
-            ty[m * 64 + (ct >> 1) * 32 + r] = (bf16)(g / (1.0f + __expf(-g)) * u);
+            ty[m * 64 + (ct >> 1) * 32 + r] = (bf16)(gate_act(g, glu == 2) * u);
           }
       }
       __syncthreads();
@@ -593,7 +593,7 @@ __global__ __launch_bounds__(256 * KW) void wstream_gemm_kernel(const bf16* __re
           if (m < M) {
             const float rr = rrow(m);
             const float g = acc[mt][i] * rr, u = red[(((ct >> 1) * MT + mt) * 16 + i) * 64 + lane] * rr;
-            Y[(int64_t)m * ldy + n] = (bf16)(g / (1.0f + __expf(-g)) * u);
+            Y[(int64_t)m * ldy + n] = (bf16)(gate_act(g, glu == 2) * u);
           }
         }
     }

@@ -119,10 +119,11 @@ def fused_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, w: torch.Tensor, 
     return rmsnorm(s, w, eps), s
 
 
-def silu_mul(x: torch.Tensor) -> torch.Tensor:
+def silu_mul(x: torch.Tensor, act: str = "silu") -> torch.Tensor:
     F = x.shape[-1] // 2
     g, u = x[..., :F].float(), x[..., F:].float()
-    return (torch.nn.functional.silu(g) * u).to(x.dtype)
+    a = torch.nn.functional.gelu(g, approximate="tanh") if act == "gelu" else torch.nn.functional.silu(g)
+    return (a * u).to(x.dtype)
 
 
 def rope_kv_write(qkv, positions, cos_sin, q_out, k_cache, v_cache, slot_mapping, Hq: int, Hkv: int) -> None:

@@ -44,6 +44,10 @@ def test_long_products_on_the_cpu():
     assert ops.linear_glu_long(torch.randn(150, 128), ops.tile_weight(torch.randn(128, 128), glu=True)) is None
 
 
+def _gelu(z):
+    return torch.nn.functional.gelu(z, approximate="tanh")
+
+
 def _close(got, want, K):
     # sums of K terms of size ~ 1 / sqrt(K) in fp32 (errors of 1e-6 of them) rounded to bf16, 2^-9 of a value
     assert ((got.float() - want).abs() <= 2 ** -8 * want.abs() + 1e-3).all()
@@ -76,8 +80,28 @@ def test_tiles_against_fp32(mt, nt):
         if N % 64 == 0 and nt % 4 == 0:
             gt, F = ops.tile_weight(w, glu=True), N // 2
             _close(ops.linear_tile(x, gt, (mt, nt, 1), glu=True), torch.nn.functional.silu(want[:, :F]) * want[:, F:], K)
+            _close(ops.linear_tile(x, gt, (mt, nt, 1), glu=True, act="gelu"), _gelu(want[:, :F]) * want[:, F:], K)
             if s > 1:
                 assert ((ops.linear_tile(x, gt, (mt, nt, s), glu=True).sum(0) - want).abs() <= 1e-4).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 31, 64, 65, 128, 129, 300])
+def test_gelu_gated_products(M):
+    """The same activation in the weight-streaming kernel's epilogue (one split), over its slabs, and of steps beyond it."""
+    g = torch.Generator().manual_seed(M)
+    for N, K in ((256, 256), (96 * 64, 512), (448 * 64, 256)):
+        w = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
+        x, wt, F = (torch.randn(M, K, generator=g) * 2).to(torch.bfloat16).cuda(), ops.tile_weight(w, glu=True), N // 2
+        want = x.float() @ w.float().t()
+        want = _gelu(want[:, :F]) * want[:, F:]
+        if M <= ops.STREAM_MAX_M:
+            _close(ops.linear_glu(x, wt, act="gelu"), want, K)
+            _close(ops.linear_glu(x, wt, 1, act="gelu"), want, K)
+        a = ops.linear_glu_long(x, wt, act="gelu")
+        if a is not None:
+            _close(a, want, K)
+        _close(ops.silu_mul((x.float() @ w.float().t()).expand(2, M, N).contiguous() / 2, act="gelu"), want, K)
 
 
 @pytest.mark.gpu

@@ -524,12 +524,17 @@ class FurapelLM:
 
     def _experts(self, lw, h):
         """The routed experts' weighted sum, fp32 [T, d], or of a long step its rows (``hops.ExpertRows``)."""
-        tw, te, _ = hops.moe_router_grouped(h, lw.router, None, lw.top, 1, 1, norm=False, w_act=lw.router_a)
         T, up_t, down_t = h.shape[0], getattr(lw, "w_up_t", None), getattr(lw, "w_down_t", None)
-        if up_t is not None and hops.moe_wide(T, lw.top, lw.E):
+        wide = up_t is not None and hops.moe_wide(T, lw.top, lw.E)
+        out = None if wide else torch.empty(T, self.cfg.hidden_size, dtype=torch.float32, device=self.device)
+        r = None if wide else hops.moe_route_sorted(h, lw.router_a, lw.top, False, out)
+        if r is not None:
+            tw, te = r.topk_w, r.topk_e
+        else:
+            tw, te, _ = hops.moe_router_grouped(h, lw.router, None, lw.top, 1, 1, norm=False, w_act=lw.router_a)
+        if wide:
             return hops.moe_expert_rows(h, up_t, down_t, tw, te, lw.E)
-        out = torch.empty(T, self.cfg.hidden_size, dtype=torch.float32, device=self.device)
-        hops.moe_experts(h, lw.w_up, lw.w_down, tw, te, out, up_t, down_t, act="relu2")
+        hops.moe_experts(h, lw.w_up, lw.w_down, tw, te, out, up_t, down_t, act="relu2", routing=r)
         return out
 
 

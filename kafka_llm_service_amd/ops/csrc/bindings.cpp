@@ -99,6 +99,10 @@ int kafka_narrow_ok(int N, int K, int64_t xs);
 int kafka_narrow_max_k();
 hipError_t kafka_launch_narrow_linear(const bf16* x, int64_t xs, const bf16* w, const float* bias, int N, int K,
                                       float* out, int64_t os, int64_t T, hipStream_t st);
+int kafka_narrow_sort_ok(int N, int64_t T);
+hipError_t kafka_launch_narrow_route_sort(const bf16* x, int64_t xs, const bf16* w, int N, int K, int k, int norm, float scale,
+                                          float* tw, int* te, int64_t T, int bm, int* perm_tok, float* perm_w, int* expert_off,
+                                          int* tile_off, float* zero, int64_t nzero, hipStream_t st);
 hipError_t kafka_launch_narrow_route(const bf16* x, int64_t xs, const bf16* w, int N, int K, int k, int norm, float scale,
                                      float* tw, int* te, int64_t T, hipStream_t st);
 hipError_t kafka_launch_grouped_gemm(const bf16* X, int64_t ldx, const bf16* W, int N, int Kd, const int* perm_tok,
@@ -954,6 +958,27 @@ static void moe_route(at::Tensor logits, int64_t k, int64_t bm, at::Tensor topk_
                                    cur_stream()));
 }
 
+// narrow_route and moe_sort of few rows in one launch
+static void narrow_route_sort(at::Tensor x, at::Tensor w, bool norm, double scale, int64_t bm, at::Tensor tw, at::Tensor te,
+                              at::Tensor perm_tok, at::Tensor perm_w, at::Tensor expert_off, at::Tensor tile_off,
+                              c10::optional<at::Tensor> zero) {
+  narrow_args(x, w);
+  const int64_t T = x.size(0), N = w.size(0);
+  CHECK_DT(tw, at::kFloat); CHECK_DT(perm_w, at::kFloat);
+  CHECK_DT(te, at::kInt); CHECK_DT(perm_tok, at::kInt); CHECK_DT(expert_off, at::kInt); CHECK_DT(tile_off, at::kInt);
+  TORCH_CHECK(tw.dim() == 2 && tw.is_contiguous() && te.is_contiguous() && te.sizes() == tw.sizes() && tw.size(0) == T &&
+                  tw.size(1) >= 1 && tw.size(1) <= N && tw.size(1) <= kafka_narrow_max_k() && T >= 1 && kafka_narrow_sort_ok((int)N, T),
+              "narrow_route_sort: choices [T, k] of up to 16 rows and 32 experts");
+  TORCH_CHECK(perm_tok.numel() == tw.numel() && perm_w.numel() == tw.numel() && expert_off.numel() == N + 1 &&
+                  tile_off.numel() == N + 1 && perm_tok.is_contiguous() && perm_w.is_contiguous() && expert_off.is_contiguous() &&
+                  tile_off.is_contiguous(), "narrow_route_sort: output sizes");
+  const int64_t nz = clear_pieces(zero, true);
+  CHECK_HIP(kafka_launch_narrow_route_sort(bptr(x), x.stride(0), bptr(w), (int)N, (int)w.size(1), (int)tw.size(1), norm ? 1 : 0,
+                                           (float)scale, tw.data_ptr<float>(), te.data_ptr<int>(), T, (int)bm, perm_tok.data_ptr<int>(),
+                                           perm_w.data_ptr<float>(), expert_off.data_ptr<int>(), tile_off.data_ptr<int>(),
+                                           nz ? zero->data_ptr<float>() : nullptr, nz, cur_stream()));
+}
+
 // the sort of moe_route alone, for entries routed elsewhere (topk_w / topk_e [T, k] are inputs; expert ids in [0, E));
 // inv [T, k]: every entry's place in the sorted order
 static void moe_sort(at::Tensor topk_w, at::Tensor topk_e, int64_t E, int64_t bm, at::Tensor perm_tok,
@@ -1256,6 +1281,8 @@ PYBIND11_MODULE(_kafka_ops, m) {
         py::arg("pin") = true, py::arg("glu_limit") = 0.0, py::arg("glu_alpha") = 1.0, py::arg("relu2") = false);
   m.def("moe_sort", &moe_sort, py::arg("topk_w"), py::arg("topk_e"), py::arg("E"), py::arg("bm"), py::arg("perm_tok"),
         py::arg("perm_w"), py::arg("expert_off"), py::arg("tile_off"), py::arg("inv") = py::none(), py::arg("zero") = py::none());
+  m.def("narrow_sort_ok", [](int64_t N, int64_t T) { return kafka_narrow_sort_ok((int)N, T) != 0; });
+  m.def("narrow_route_sort", &narrow_route_sort);
   m.def("moe_route", &moe_route, py::arg("logits"), py::arg("k"), py::arg("bm"), py::arg("topk_w"), py::arg("topk_e"), py::arg("perm_tok"),
         py::arg("perm_w"), py::arg("expert_off"), py::arg("tile_off"), py::arg("zero") = py::none());
   m.def("cu_mask_stream", &cu_mask_stream);

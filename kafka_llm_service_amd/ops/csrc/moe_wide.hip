@@ -540,14 +540,26 @@ __device__ __forceinline__ float row16(float v, OP op) {
 }
 
 // up to 16 experts live in the first 16 lanes (the others run along): exchanges without LDS, 16 rows of 4096 12.2 -> 10.9 us
+// what a routing launch of up to NR_ROWS rows does beside: the stable sort of its choices by expert, and clearing the experts' sums
+struct RouteSort {
+  int bits, bm;
+  int *perm_tok, *expert_off, *tile_off;
+  float *perm_w, *zero;
+  int64_t nzero;
+};
+
 // softmax over all N experts, the k largest (ties: the lower index), their scores as weights (norm: divided by their sum)
-// times scale; lane = expert
-template <int TN>
+// times scale; lane = expert. SORT: one workgroup, with the sort (a launch of its own: 4.7 us of 16 rows) and, in further ones, the clearing
+template <int TN, bool SORT>
 __global__ __launch_bounds__(64 * nr_waves(TN)) void narrow_route_kernel(const bf16* __restrict__ x, int64_t xs,
                                                            const bf16* __restrict__ wt, int N, int K, int k, bool norm,
                                                            float scale, float* __restrict__ tw, int* __restrict__ te,
-                                                           int64_t T) {
+                                                           int64_t T, RouteSort so) {
   __shared__ float part[nr_waves(TN)][NR_ROWS][nr_ld(TN)];
+  if (SORT && blockIdx.x > 0) {
+    clear(so.zero, so.nzero, blockIdx.x - 1, gridDim.x - 1);
+    return;
+  }
   narrow_product<TN>(x, xs, T, wt, N, K, part);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll 1
@@ -592,6 +604,13 @@ __global__ __launch_bounds__(64 * nr_waves(TN)) void narrow_route_kernel(const b
       tw[t * k + lane] = (norm ? mine / sum : mine) * scale;
       te[t * k + lane] = me;
     }
+  }
+  if constexpr (SORT) {
+    static_assert(nr_waves(TN) == SORT_W, "the sort's waves");
+    __shared__ int cnt[SORT_W][64];
+    __syncthreads();   // (the sort reads what other threads of the workgroup wrote)
+    sort_few_experts(tw, te, 0, (int)T * k, k, N, so.bits, so.bm, so.perm_tok, so.perm_w, so.expert_off, so.tile_off, nullptr, nullptr,
+                     0, 1, cnt);
   }
 }
 
@@ -699,12 +718,29 @@ hipError_t kafka_launch_narrow_route(const bf16* x, int64_t xs, const bf16* w, i
   if (!kafka_narrow_ok(N, K, xs) || k < 1 || k > N || k > NR_MAXK) return hipErrorInvalidValue;
   const unsigned g = (unsigned)((T + NR_ROWS - 1) / NR_ROWS);
   auto a = [&](auto kern, int tn) {
-    kern<<<g, 64 * nr_waves(tn), 0, st>>>(x, xs, w, N, K, k, norm != 0, scale, tw, te, T);
+    kern<<<g, 64 * nr_waves(tn), 0, st>>>(x, xs, w, N, K, k, norm != 0, scale, tw, te, T, RouteSort{});
   };
-  if (N <= 16) a(narrow_route_kernel<1>, 1);
-  else if (N <= 32) a(narrow_route_kernel<2>, 2);
-  else if (N <= 48) a(narrow_route_kernel<3>, 3);
-  else a(narrow_route_kernel<4>, 4);
+  if (N <= 16) a(narrow_route_kernel<1, false>, 1);
+  else if (N <= 32) a(narrow_route_kernel<2, false>, 2);
+  else if (N <= 48) a(narrow_route_kernel<3, false>, 3);
+  else a(narrow_route_kernel<4, false>, 4);
+  return hipGetLastError();
+}
+
+// rows and experts whose routing takes the sort along
+int kafka_narrow_sort_ok(int N, int64_t T) { return N <= 32 && T <= NR_ROWS; }
+
+hipError_t kafka_launch_narrow_route_sort(const bf16* x, int64_t xs, const bf16* w, int N, int K, int k, int norm, float scale,
+                                          float* tw, int* te, int64_t T, int bm, int* perm_tok, float* perm_w, int* expert_off,
+                                          int* tile_off, float* zero, int64_t nzero, hipStream_t st) {
+  if (T <= 0) return hipSuccess;
+  if (!kafka_narrow_ok(N, K, xs) || !kafka_narrow_sort_ok(N, T) || k < 1 || k > N || k > NR_MAXK || bm < 1) return hipErrorInvalidValue;
+  RouteSort so{0, bm, perm_tok, expert_off, tile_off, perm_w, zero, nzero};
+  while ((1 << so.bits) < N) ++so.bits;
+  const unsigned g = 1 + (zero != nullptr ? clear_blocks(nzero) : 0);
+  auto a = [&](auto kern) { kern<<<g, SORT_NT, 0, st>>>(x, xs, w, N, K, k, norm != 0, scale, tw, te, T, so); };
+  if (N <= 16) a(narrow_route_kernel<1, true>);
+  else a(narrow_route_kernel<2, true>);
   return hipGetLastError();
 }
 

@@ -673,20 +673,20 @@ def moe_wide(T: int, k: int, n_experts: int) -> bool:
 
 
 def moe_experts(h, w_gu, w_down, topk_w, topk_e, out, w_gu_t=None, w_down_t=None, act: str = "silu",
-                limit: float = 0.0, alpha: float = 1.0) -> None:
+                limit: float = 0.0, alpha: float = 1.0, routing=None) -> None:
     """out (fp32 [T, d]) = the routed experts' weighted sum for every row. Sizes the framework's expert-sorted
     matrix-core kernels take (bf16) go through them - entries sorted by expert (``ops.moe_sort``), gate/up GEMM on
     gathered rows, silu * up, down GEMM with the weighted combine in its epilogue (fp32 adds, two entries per row
     commute), or with tiled expert weights the grouped weight-streaming kernels (steps of few rows) and the wide ones -
     everything else is evaluated per (row, expert) pair by ``moe_rows``. ``act`` as in ``moe_rows`` (the kernels on tiled
     weights apply it in their epilogue; between the two expert-sorted GEMMs it is a launch of its own, "relu2" is part
-    of the first)."""
+    of the first). ``routing``: the choices sorted and ``out`` cleared already (``moe_route_sorted``)."""
     from kafka_llm_service_amd import ops
 
     T = h.shape[0]
     glu = act != "relu2"
     if T and moe_grouped_ok(h, w_gu, w_down, glu):
-        r = ops.moe_sort(topk_w, topk_e, w_gu.shape[0], zero=out)
+        r = ops.moe_sort(topk_w, topk_e, w_gu.shape[0], zero=out) if routing is None else routing
         if w_gu_t is not None and w_down_t is not None:
             lim, al = _glu_act(act, limit, alpha) if glu else (0.0, 1.0)
             if moe_wide(T, topk_e.shape[1], w_gu.shape[0]):
@@ -901,6 +901,23 @@ def moe_router_grouped(h, w, correction, k: int, groups: int, keep: int, eps: fl
     else:
         ref.moe_router_grouped(h, w, E, correction, k, groups, keep, eps, tw, te, gate, score, group_score, norm, scale)
     return tw, te, gate
+
+
+def moe_route_sorted(h, w_act, k: int, norm: bool, out, scale: float = 1.0):
+    """The plain choice of ``moe_router_grouped`` (softmax over all experts, one group, no correction; ``w_act`` as there), the sort
+    of its entries by expert and out = 0 in one launch: an ``ops.MoERouting``, or None for steps and routers that it does not take
+    (up to 16 rows and 32 experts)."""
+    from kafka_llm_service_amd import ops
+
+    if w_act is None or not 0 < h.shape[0] <= 16 or h.dim() != 2 or not 1 <= k <= min(16, w_act.shape[0]) or not narrow_ok(h, w_act) or \
+            not ext().narrow_sort_ok(w_act.shape[0], h.shape[0]):
+        return None
+    T, E, dev = h.shape[0], w_act.shape[0], h.device
+    tw, pw = torch.empty(T, k, dtype=torch.float32, device=dev), torch.empty(T * k, dtype=torch.float32, device=dev)
+    te, pt = torch.empty(T, k, dtype=torch.int32, device=dev), torch.empty(T * k, dtype=torch.int32, device=dev)
+    eo, to = (torch.empty(E + 1, dtype=torch.int32, device=dev) for _ in range(2))
+    ext().narrow_route_sort(h, w_act, bool(norm), float(scale), ops.GG_BM, tw, te, pt, pw, eo, to, out)
+    return ops.MoERouting(tw, te, pt, pw, eo, to, E)
 
 
 # ---- gated recurrences beside attention (minGRU, HGRN2), rotation + head mix + paged store --------------------------

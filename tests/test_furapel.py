@@ -1188,3 +1188,29 @@ def test_shared_keys_past_a_run_of_pages():
     assert not torch.isnan(out).any()
     want = _attend(q[rows].to(dev), kv[0], torch.tensor([p0 + r for r in rows], device=dev), 0)
     assert torch.allclose(out[rows].double().view_as(want), want, atol=2e-2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,k", [(1, 1), (5, 2), (16, 4), (16, 16), (17, 3), (32, 8)])
+def test_routing_with_the_sort(E, k):
+    """Choice, sort and cleared sums in one launch are those of the launches apart, bit for bit, for every number of rows it takes; what
+    it does not take (17 rows, 33 experts, weights in fp32) is left to them."""
+    from kafka_llm_service_amd import ops
+
+    g = torch.Generator().manual_seed(E)
+    w = (torch.randn(E, 512, generator=g) / 8).to(torch.bfloat16).cuda()
+    for T in (1, 2, 15, 16):
+        h = torch.randn(T, 520, generator=g).to(torch.bfloat16).cuda()[:, :512]
+        for norm, d in ((False, 4096), (True, 6)):
+            out = torch.full((T, d), 7.0, device="cuda")
+            r = hops.moe_route_sorted(h, w, k, norm, out, 1.5)
+            tw, te, _ = hops.moe_router_grouped(h, w.float(), None, k, 1, 1, norm=norm, scale=1.5, w_act=w)
+            s = ops.moe_sort(tw, te, E)
+            for a in ("topk_w", "topk_e", "perm_tok", "perm_w", "expert_off", "tile_off"):
+                assert torch.equal(getattr(r, a), getattr(s, a)), (a, T)
+            assert (out == 0).all()
+    h = torch.randn(17, 512, generator=g).to(torch.bfloat16).cuda()
+    out = torch.full((17, 8), 7.0, device="cuda")
+    assert hops.moe_route_sorted(h, w, k, True, out) is None and hops.moe_route_sorted(h[:16], w.float(), k, True, out) is None
+    assert hops.moe_route_sorted(h[:16], torch.zeros(33, 512, dtype=torch.bfloat16, device="cuda"), 2, True, out) is None
+    assert hops.moe_route_sorted(h[:16].cpu(), w.cpu(), k, True, out.cpu()) is None and (out == 7).all()

@@ -1279,7 +1279,7 @@ void add_tanh_norm(at::Tensor x, OptT y1, OptT y2, bool assign, std::vector<doub
   TORCH_CHECK(n <= 2 && alpha.size() == n && w.size() == n && b.size() == n, "add_tanh_norm: up to two norms");
   TORCH_CHECK(y1.has_value() || (!assign && !y2.has_value() && !rows.has_value()),
               "add_tanh_norm: y2 and assign need y1");
-  int f32 = -1;   // the activation dtype: that of the outputs, else of y1
+  int f32 = -1;   // the activation dtype: that of the outputs, else of the experts' rows, else of y1
   float al[2]; const float *wp[2], *bp[2]; void* op[2]; int64_t os[2];
   auto dest = [&](const at::Tensor& o) {
     rows2d(o, "output");
@@ -1307,7 +1307,7 @@ void add_tanh_norm(at::Tensor x, OptT y1, OptT y2, bool assign, std::vector<doub
       TORCH_CHECK(y1->size(0) == T && y1->size(1) == d, "add_tanh_norm: y1 shape");
       s1 = y1->stride(0);
     }
-    if (f32 < 0) f32 = y1f;
+    if (f32 < 0) f32 = rows.has_value() ? act_f32(*rows) : y1f;
     TORCH_CHECK(y1f || !f32, "add_tanh_norm: y1 is fp32 or of the activation dtype");
     p1 = y1->data_ptr();
   }

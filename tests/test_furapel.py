@@ -1214,3 +1214,23 @@ def test_routing_with_the_sort(E, k):
     assert hops.moe_route_sorted(h, w, k, True, out) is None and hops.moe_route_sorted(h[:16], w.float(), k, True, out) is None
     assert hops.moe_route_sorted(h[:16], torch.zeros(33, 512, dtype=torch.bfloat16, device="cuda"), 2, True, out) is None
     assert hops.moe_route_sorted(h[:16].cpu(), w.cpu(), k, True, out.cpu()) is None and (out == 7).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 70])
+def test_add_slabs_and_expert_rows_without_outputs(T):
+    """What the last layer of a long step adds: a projection's fp32 slabs and the experts' bf16 rows, with nothing to write beside the
+    stream; fp32 sums of ten terms of size 1 (2^-22 of them)."""
+    g = torch.Generator().manual_seed(T)
+    d, k = 256, 4
+    x, y = torch.randn(T, d, generator=g), torch.randn(4, T, d, generator=g)
+    rows, inv = torch.randn(T * k, d, generator=g).to(torch.bfloat16), torch.randperm(T * k, generator=g).view(T, k)
+    want = x.double() + y.double().sum(0) + rows.double()[inv].sum(1)
+    for y1 in (y, y.sum(0)):
+        got = x.cuda()
+        hops.add_tanh_norm(got, y1.cuda(), hops.ExpertRows(rows.cuda(), inv.to(torch.int32).cuda()))
+        assert ((got.cpu().double() - want).abs() <= 1e-5).all()
+    low = y[0].to(torch.bfloat16)
+    got = x.cuda()
+    hops.add_tanh_norm(got, low.cuda(), hops.ExpertRows(rows.cuda(), inv.to(torch.int32).cuda()))
+    assert ((got.cpu().double() - x.double() - low.double() - rows.double()[inv].sum(1)).abs() <= 1e-5).all()

@@ -402,6 +402,12 @@ class BuduraxLM:
             hops.gelu_mul(self._lin(h, lw.gate_up, wt), a)
         return a
 
+    def _logits(self, hf):
+        """hf @ head^T as fp32."""
+        t = getattr(self, "head_t", None)
+        y = ops.stream_logits(hf, t, self.stream_max_m) if self.stream else None
+        return self._lin(hf, self.head, t).float() if y is None else y
+
     def weight_bytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self._tensors)
 
@@ -594,7 +600,7 @@ class BuduraxLM:
         xs = ops.gather_rows(x, inp.logit_rows)
         hf = torch.empty(xs.shape[0], d, dtype=dt, device=dev)
         hops.ln_shift(xs, self.final_norm, self.final_norm_b, eps, hf)
-        return self._lin(hf, self.head, getattr(self, "head_t", None)).float()[:, :cfg.vocab_size]
+        return self._logits(hf)[:, :cfg.vocab_size]
 
     def _latent_attention(self, i: int, lw, h, inp, m: SegMeta, pages: list) -> torch.Tensor:
         mm = lw.m

@@ -271,6 +271,12 @@ class FurapelLM:
             return ops.slab_reduce(y) if ops.is_slab(y) and not slabs else y
         return ops.linear_long(x, w, wt if self.stream else None, slabs)
 
+    def _logits(self, hf):
+        """hf @ head^T as fp32."""
+        t = getattr(self, "head_t", None)
+        y = ops.stream_logits(hf, t, self.stream_max_m) if self.stream else None
+        return self._lin(hf, self.head, t).float() if y is None else y
+
     def weight_bytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self._tensors)
 
@@ -468,7 +474,7 @@ class FurapelLM:
         xs = ops.gather_rows(x, inp.logit_rows)
         hf = torch.empty(xs.shape[0], d, dtype=dt, device=dev)
         hops.add_tanh_norm(xs, norms=[self.final_norm], outs=[hf])
-        logits = self._lin(hf, self.head, getattr(self, "head_t", None)).float()
+        logits = self._logits(hf)
         if cfg.logit_scale != 1.0:
             logits.mul_(cfg.logit_scale)
         return logits[:, :cfg.vocab_size]   # (a view: the padded row stride is what the sampler reads)

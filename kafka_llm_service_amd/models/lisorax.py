@@ -271,6 +271,12 @@ class LisoraxLM:
             return ops.linear_long(x, w, wt)
         return F.linear(x, w, bias)
 
+    def _logits(self, hf):
+        """hf @ head^T as fp32."""
+        t = getattr(self, "head_t", None)
+        y = ops.stream_logits(hf, t, self.stream_max_m) if self.stream else None
+        return self._lin(hf, self.head, t).float() if y is None else y
+
     def weight_bytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self._tensors)
 
@@ -451,7 +457,7 @@ class LisoraxLM:
         xs = ops.gather_rows(x, inp.logit_rows)
         hf = torch.empty(xs.shape[0], d, dtype=dt, device=dev)
         hops.rms_norm(xs, self.final_norm, eps, hf)
-        return self._lin(hf, self.head, getattr(self, "head_t", None)).float()[:, :cfg.vocab_size]
+        return self._logits(hf)[:, :cfg.vocab_size]
 
     def _attention(self, i: int, lw, hm, inp, m: SegMeta, pages: list, st: dict) -> torch.Tensor:
         mm = lw.m

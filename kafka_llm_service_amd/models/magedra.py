@@ -296,6 +296,12 @@ class MagedraLM:
             return ops.linear_long(x, w, wt)
         return F.linear(x, w, bias)
 
+    def _logits(self, hf):
+        """hf @ head^T as fp32."""
+        t = getattr(self, "head_t", None)
+        y = ops.stream_logits(hf, t, self.stream_max_m) if self.stream else None
+        return self._lin(hf, self.head, t).float() if y is None else y
+
     def weight_bytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self._tensors)
 
@@ -526,7 +532,7 @@ class MagedraLM:
         xsel = xs.index_select(1, inp.logit_rows)
         hf = torch.empty(xsel.shape[1], d, dtype=dt, device=dev)
         hops.stream_step(xsel, read=self.sum_in, norm_w=self.final_norm, eps=eps, out=hf, center=True)
-        logits = self._lin(hf, self.head, getattr(self, "head_t", None)).float()
+        logits = self._logits(hf)
         if cfg.logit_scale != 1.0:
             logits.mul_(cfg.logit_scale)
         return logits[:, :cfg.vocab_size]   # (a view: the padded row stride is what the sampler reads)

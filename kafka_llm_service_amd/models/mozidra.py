@@ -280,6 +280,12 @@ class MozidraLM:
             return ops.linear_long(x, w, wt)
         return F.linear(x, w, bias)
 
+    def _logits(self, hf):
+        """hf @ head^T as fp32."""
+        t = getattr(self, "head_t", None)
+        y = ops.stream_logits(hf, t, self.stream_max_m) if self.stream else None
+        return self._lin(hf, self.head, t).float() if y is None else y
+
     def weight_bytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in self._tensors)
 
@@ -479,7 +485,7 @@ class MozidraLM:
         xsel = xs.index_select(1, inp.logit_rows)
         hf = torch.empty(xsel.shape[1], d, dtype=dt, device=dev)
         hops.stream_step(xsel, read=self.sum_in, norm_w=self.final_norm, eps=eps, out=hf)
-        return self._lin(hf, self.head, getattr(self, "head_t", None)).float()[:, :cfg.vocab_size]
+        return self._logits(hf)[:, :cfg.vocab_size]
 
     def _attention(self, i: int, lw, h, inp, m: SegMeta, pages: list, step: dict) -> torch.Tensor:
         mm = lw.m

@@ -544,6 +544,20 @@ def linear_stream(x: torch.Tensor, wt: torch.Tensor, max_splits: int = 8, nt: bo
     return torch.stack([xf[:, s * ks:(s + 1) * ks] @ w[:, s * ks:(s + 1) * ks].t() for s in range(S)])
 
 
+def stream_logits(x: torch.Tensor, wt: torch.Tensor | None, max_m: int) -> torch.Tensor | None:
+    """x @ W^T in fp32 from the weight-streaming kernel's sums, None for shapes that it does not take in one split: logits, which
+    are read as fp32 (as bf16, a launch to widen them again: 5 us)."""
+    if wt is None or not _gpu(x) or not 0 < x.shape[0] <= max_m or x.dtype != torch.bfloat16 or x.stride(0) % 8 or x.stride(1) != 1:
+        return None
+    M, N = x.shape[0], wt.shape[0] * 32
+    plan = stream_plan(M, N, x.shape[1])
+    if plan is None or plan[2] != 1:
+        return None
+    p = torch.empty(1, M, N, dtype=torch.float32, device=x.device)
+    ext().wstream_gemm(x, wt, None, p, 8, True, 0)
+    return p[0]
+
+
 def linear_glu(x: torch.Tensor, wt: torch.Tensor, max_splits: int = 8, act: str = "silu") -> torch.Tensor:
     """silu(x @ Wg^T) * (x @ Wu^T) from GLU-tiled gate_up weights: fused into the GEMM epilogue when the plan has one
     split, else the GEMM's slabs go through silu_mul (``act`` as there)."""

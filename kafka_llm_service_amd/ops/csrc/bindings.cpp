@@ -564,15 +564,15 @@ static void wstream_gemm(at::Tensor x, at::Tensor wt, c10::optional<at::Tensor> 
   bf16* yp = nullptr;
   int64_t ldy = 0;
   float* pp = nullptr;
-  if (s == 1) {
+  if (s == 1 && !p.has_value()) {
     // glu + one split: y is the activated [M, N/2]; otherwise [M, N] in gate | up column order
     TORCH_CHECK(y.has_value(), "wstream_gemm: y required for a single split");
     CHECK_DT(y.value(), at::kBFloat16); CHECK_LASTDIM(y.value());
     TORCH_CHECK(y->dim() == 2 && y->size(0) == M && y->size(1) == (glu ? N / 2 : N), "wstream_gemm: y shape");
     yp = bptr(y.value());
     ldy = y->stride(0);
-  } else {
-    TORCH_CHECK(p.has_value(), "wstream_gemm: slab output required");
+  } else {   // slabs (one: the fp32 result)
+    TORCH_CHECK(p.has_value() && (s > 1 || !glu), "wstream_gemm: slab output required");
     CHECK_DT(p.value(), at::kFloat);
     TORCH_CHECK(p->is_contiguous() && p->dim() == 3 && p->size(0) == s && p->size(1) == M && p->size(2) == N,
                 "wstream_gemm: slab shape must be [splits, M, N]");

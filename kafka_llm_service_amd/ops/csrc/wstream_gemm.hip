@@ -899,7 +899,7 @@ extern "C" hipError_t kafka_launch_wstream_gemm(const bf16* X, int64_t ldx, cons
   const dim3 grid((rt > 1 ? (nblk + 7) / 8 * 8 : nblk) * rt, splits);  // (row tiles: column blocks padded to 8)
   const int ks = K / splits;
   const auto* wt = reinterpret_cast<const bf16x8*>(Wt);
-  float* p = splits > 1 ? P : nullptr;
+  float* p = splits > 1 || Y == nullptr ? P : nullptr;   // (one split into P: the fp32 result)
   // split-K slabs leave as 16-B sc1 stores through an LDS transpose (was one 4-B store per accumulator, the lines
   // kept dirty in the XCD's L2): +2.0 % on the headline, in-step GPU time 7.50 vs 7.65 ms
   // (profiles/r05/bench_ab_wstream_slab16_sc1.jsonl); KAFKA_WSTREAM_SLAB16=0 restores the old epilogue

@@ -97,3 +97,22 @@ def test_router_logits_of_long_steps(E, K, gate):
         assert ((got[0] - want[0]).abs()[same] <= 1e-4).all()
         if gate:
             assert ((got[2] - want[2]).abs() <= 1e-4).all()
+
+
+@pytest.mark.gpu
+def test_logits_in_fp32():
+    """The weight-streaming kernel's sums as they are (fp32 sums of K terms of size 1 / sqrt(K)), rows and columns that end inside its
+    tiles; None for what it would split or not take."""
+    g = torch.Generator().manual_seed(7)
+    for N, K in ((32000, 256), (24608, 512)):
+        w = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
+        wt = ops.tile_weight(w)
+        for M in (1, 31, 33, 64, 100, 128):
+            x = torch.randn(M, K + 8, generator=g).to(torch.bfloat16).cuda()[:, :K]
+            y = ops.stream_logits(x, wt, 128)
+            assert y.dtype == torch.float32 and ((y - x.float() @ w.float().t()).abs() <= 2e-5).all()
+    assert ops.stream_logits(x, wt, 127) is None and ops.stream_logits(x, None, 128) is None and ops.stream_logits(x.cpu(), wt, 128) is None
+    assert ops.stream_logits(x[:, ::2], wt, 128) is None and ops.stream_logits(x.float(), wt, 128) is None
+    few = ops.tile_weight(torch.zeros(64, 4096, dtype=torch.bfloat16, device="cuda"))
+    x = torch.zeros(4, 4096, dtype=torch.bfloat16, device="cuda")
+    assert ops.stream_plan(4, 64, 4096)[2] > 1 and ops.stream_logits(x, few, 128) is None

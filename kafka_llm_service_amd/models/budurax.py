@@ -588,9 +588,7 @@ class BuduraxLM:
             ys = None
             if lw.side_gate is not None:
                 hops.add_ln(x, y, nw, nb, eps, h2)  # h2 = the new x in the model dtype (the gate GEMM's input)
-                g = torch.empty(T, cfg.token_side_dim, dtype=dt, device=dev)
-                hops.side_gate(ops.linear_small(h2, lw.side_gate), inp.tokens, self.side_embed, i * cfg.token_side_dim, g)
-                ys = ops.linear_small(g, lw.side_proj)
+                ys = ops.linear_small(hops.side_gate_product(h2, lw.side_gate, inp.tokens, self.side_embed, i * cfg.token_side_dim), lw.side_proj)
             else:
                 hops.add_ln(x, y, nw, nb, eps)
             if ys is not None or stack is not None:

@@ -128,7 +128,8 @@ hipError_t kafka_launch_ep_recv_route(const bf16* img, int ep, int C, int MR, in
 hipError_t kafka_launch_ep_combine(const bf16* back, const int* slot_map, const float* topk_w, int lo, int n_own,
                                    int k, int d, bf16* out, int64_t ldo, hipStream_t st);
 hipError_t kafka_launch_small_gemm(const bf16* X, const bf16* W, int B, int M, int N, int K, int64_t xb, int64_t xm, int64_t wb,
-                                   int64_t wn, const float* bias, int f32, void* Y, int64_t yb, int64_t ym, hipStream_t st);
+                                   int64_t wn, const float* bias, int f32, void* Y, int64_t yb, int64_t ym,
+                                   const int64_t* tok, const bf16* emb, int64_t emb_stride, int64_t emb_rows, hipStream_t st);
 hipError_t kafka_launch_tile_gemm(const bf16* X, int64_t ldx, const bf16* Wt, int M, int N, int K, int mt, int nt, int splits,
                                   int glu, bf16* Y, int64_t ldy, float* P, hipStream_t st);
 int kafka_skinny_plan(int M, int N, int K, int max_splits, int* splits);
@@ -727,7 +728,22 @@ static void small_gemm(at::Tensor x, at::Tensor w, at::Tensor out, c10::optional
   CHECK_HIP(kafka_launch_small_gemm(bptr(x), bptr(w), (int)B, (int)M, (int)N, (int)K, d == 3 ? x.stride(0) : 0, x.stride(-2),
                                     d == 3 ? w.stride(0) : 0, w.stride(-2),
                                     bias.has_value() ? bias->data_ptr<float>() : nullptr, f32 ? 1 : 0, out.data_ptr(),
-                                    d == 3 ? out.stride(0) : 0, out.stride(-2), cur_stream()));
+                                    d == 3 ? out.stride(0) : 0, out.stride(-2), nullptr, nullptr, 0, 0, cur_stream()));
+}
+
+// out[m, n] = gelu(x[m, :] . w[n, :]) * emb[tokens[m], col0 + n] of bf16 rows, K from 1024 on; rows of unknown tokens are NaN
+static void small_gate(at::Tensor x, at::Tensor w, at::Tensor tokens, at::Tensor emb, int64_t col0, at::Tensor out) {
+  for (const at::Tensor* t : {&x, &w, &emb, &out}) {
+    CHECK_CUDA(*t); CHECK_DT(*t, at::kBFloat16); CHECK_LASTDIM(*t);
+    TORCH_CHECK(t->dim() == 2, "small_gate: matrices");
+  }
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  CHECK_CUDA(tokens); CHECK_DT(tokens, at::kLong);
+  TORCH_CHECK(w.size(1) == K && out.size(0) == M && out.size(1) == N && M < (1 << 28) && N < (1 << 20) && K < (1 << 20) && K >= 1024 &&
+                  col0 >= 0 && col0 + N <= emb.size(1) && tokens.is_contiguous() && tokens.numel() == M, "small_gate: shapes");
+  CHECK_HIP(kafka_launch_small_gemm(bptr(x), bptr(w), 1, (int)M, (int)N, (int)K, 0, x.stride(0), 0, w.stride(0), nullptr, 0, out.data_ptr(),
+                                    0, out.stride(0), tokens.data_ptr<int64_t>(), bptr(emb) + col0, emb.stride(0), emb.size(0),
+                                    cur_stream()));
 }
 
 // Dense products of long steps (csrc/tile_gemm.hip) on tiles of 32 mt x 32 nt: y bf16 [M, N] (glu: [M, N / 2] activated) or
@@ -1272,6 +1288,7 @@ PYBIND11_MODULE(_kafka_ops, m) {
   m.def("skinny_plan", &skinny_plan);
   m.def("tile_gemm", &tile_gemm, py::arg("x"), py::arg("wt"), py::arg("y"), py::arg("p"), py::arg("mt"), py::arg("nt"), py::arg("splits"),
         py::arg("glu"), py::arg("relu2") = false, py::arg("gelu") = false);
+  m.def("small_gate", &small_gate);
   m.def("small_gemm", &small_gemm, py::arg("x"), py::arg("w"), py::arg("out"), py::arg("bias") = c10::nullopt);
   m.def("skinny_gemm", &skinny_gemm);
   m.def("wstream_gemm_cfg", &wstream_gemm_cfg);

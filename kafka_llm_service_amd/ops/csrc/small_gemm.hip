@@ -18,13 +18,19 @@ typedef float f32x4v __attribute__((ext_vector_type(4)));
 struct Strides {
   int64_t xb, xm, wb, wn, yb, ym;
 };
+// what a gate product's rows are multiplied with: gelu(sum) * emb[tok[m]][n] (rows outside the table: NaN)
+struct Gate {
+  const int64_t* tok;
+  const bf16* emb;
+  int64_t stride, rows;
+};
 
 // A wave: 16 rows x 16 NT columns over its share of K. KW waves of a workgroup share K (their sums meet in LDS), the other
 // 4 / KW (KW up to 4) take further columns. Products are taken with the weights first: a lane holds four columns of one row.
-template <int NT, int KW, bool F32>
+template <int NT, int KW, bool F32, bool GATE = false>
 __global__ __launch_bounds__(64 * (KW > 4 ? KW : 4)) void small_gemm_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W,
                                                                             int M, int N, int K, const float* __restrict__ bias,
-                                                                            void* __restrict__ Y, Strides st) {
+                                                                            void* __restrict__ Y, Strides st, Gate gate) {
   constexpr int NW = KW > 4 ? KW : 4, CW = NW / KW;   // waves; column parts
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, q = lane >> 4;
   const int kw = w % KW, m0 = blockIdx.x * 16, n0 = (blockIdx.y * CW + w / KW) * 16 * NT, b = blockIdx.z;
@@ -76,6 +82,8 @@ __global__ __launch_bounds__(64 * (KW > 4 ? KW : 4)) void small_gemm_kernel(cons
   }
   const int m = m0 + r;
   if (m >= M) return;
+  const int64_t tok = GATE ? gate.tok[m] : 0;
+  const bool known = tok >= 0 && tok < gate.rows;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int n = n0 + 16 * t + 4 * q;               // (N is a multiple of 4)
@@ -87,14 +95,23 @@ __global__ __launch_bounds__(64 * (KW > 4 ? KW : 4)) void small_gemm_kernel(cons
     } else {
       bf16x4 o;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = (bf16)acc[t][i];
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (GATE)
+          o[i] = known ? (bf16)(gate_act(acc[t][i], true) * (float)gate.emb[tok * gate.stride + n + i]) : (bf16)__builtin_nanf("");
+        else
+          o[i] = (bf16)acc[t][i];
+      }
       *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(Y) + at) = o;
     }
   }
 }
 
 extern "C" hipError_t kafka_launch_small_gemm(const bf16* X, const bf16* W, int B, int M, int N, int K, int64_t xb, int64_t xm,
-                                              int64_t wb, int64_t wn, const float* bias, int f32, void* Y, int64_t yb, int64_t ym, hipStream_t st) {
+                                              int64_t wb, int64_t wn, const float* bias, int f32, void* Y, int64_t yb, int64_t ym,
+                                              const int64_t* tok, const bf16* emb, int64_t emb_stride, int64_t emb_rows,
+                                              hipStream_t st) {
+  const Gate gate{tok, emb, emb_stride, emb_rows};
+  if (tok != nullptr && (f32 || bias || B != 1 || K < 1024)) return hipErrorInvalidValue;
   if (B < 1 || M < 1 || N < 1) return hipSuccess;
   const uintptr_t ya = reinterpret_cast<uintptr_t>(Y);
   if (N % 4 || K < 8 || K % 8 || xb % 8 || xm % 8 || wb % 8 || wn % 8 || yb % 4 || ym % 4 || reinterpret_cast<uintptr_t>(X) % 16 ||
@@ -105,11 +122,12 @@ extern "C" hipError_t kafka_launch_small_gemm(const bf16* X, const bf16* W, int 
   const int rows = (M + 15) / 16;
   auto go = [&](auto kern, int nt, int kw) {
     const int cols = 16 * nt * (kw >= 4 ? 1 : 4 / kw);
-    kern<<<dim3(rows, (N + cols - 1) / cols, B), 64 * (kw > 4 ? kw : 4), 0, st>>>(X, W, M, N, K, bias, Y, s);
+    kern<<<dim3(rows, (N + cols - 1) / cols, B), 64 * (kw > 4 ? kw : 4), 0, st>>>(X, W, M, N, K, bias, Y, s, gate);
     return hipGetLastError();
   };
   // Long K: 16 waves share it, a workgroup per 16 columns (64 columns of 4096 in one workgroup of 8 waves 19.7 us at 64 rows, so 8.8);
   // in between 4 waves; short K: a wave takes 64 columns alone.
+  if (tok != nullptr) return go(small_gemm_kernel<1, 16, false, true>, 1, 16);
   if (K >= 1024) return f32 ? go(small_gemm_kernel<1, 16, true>, 1, 16) : go(small_gemm_kernel<1, 16, false>, 1, 16);
   if (K >= 256) return f32 ? go(small_gemm_kernel<2, 4, true>, 2, 4) : go(small_gemm_kernel<2, 4, false>, 2, 4);
   return f32 ? go(small_gemm_kernel<4, 1, true>, 4, 1) : go(small_gemm_kernel<4, 1, false>, 4, 1);

@@ -72,6 +72,19 @@ def side_gate(sg, tokens, side_embed, col0: int, out) -> None:
         ref.side_gate(sg, tokens, side_embed, col0, out)
 
 
+def side_gate_product(h, w, tokens, side_embed, col0: int) -> torch.Tensor:
+    """gelu_tanh(h @ w^T) * side_embed[token, col0 : col0 + dim]: steps of few rows in one launch, the product's fp32 sums activated."""
+    from kafka_llm_service_amd import ops
+
+    g = torch.empty(h.shape[0], w.shape[0], dtype=h.dtype, device=h.device)
+    if h.shape[1] >= 1024 and side_embed.dtype == h.dtype and side_embed.stride(1) == 1 and tokens.dtype == torch.int64 and \
+            tokens.is_contiguous() and ops.small_ok(h, w, ops.small_rows(w.shape[0], w.shape[1])):
+        ext().small_gate(h, w, tokens, side_embed, int(col0), g)
+    else:
+        side_gate(ops.linear_small(h, w), tokens, side_embed, col0, g)
+    return g
+
+
 def side_dwa(x, y, side_w, eps, stack, layer: int, dwa) -> None:
     """x += y / rms(y) * side_w (when y is given); stack[layer + 1] = x; with ``dwa`` x = sum_j dwa[j] stack[j]."""
     if _gpu(x):

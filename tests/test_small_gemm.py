@@ -116,3 +116,23 @@ def test_logits_in_fp32():
     few = ops.tile_weight(torch.zeros(64, 4096, dtype=torch.bfloat16, device="cuda"))
     x = torch.zeros(4, 4096, dtype=torch.bfloat16, device="cuda")
     assert ops.stream_plan(4, 64, 4096)[2] > 1 and ops.stream_logits(x, few, 128) is None
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_gate_times_token_rows(device):
+    """gelu(product) times the tokens' rows: in the product's kernel and, for short or too many rows, apart (the product rounded to bf16
+    between, 2^-8 of it more), columns from the middle of the table."""
+    g = torch.Generator().manual_seed(9)
+    for M, N, K in ((1, 4, 1024), (17, 64, 2048), (40, 64, 512), (1030, 64, 1024)):
+        x, w = torch.randn(M, K + 8, generator=g).to(torch.bfloat16)[:, :K], (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16)
+        emb, tok = torch.randn(11, 3 * N, generator=g).to(torch.bfloat16), torch.randint(0, 11, (M,), generator=g)
+        got = hops.side_gate_product(x.to(device), w.to(device), tok.to(device), emb.to(device), N).float().cpu()
+        z = x.float() @ w.float().t()
+        e = emb[tok, N:2 * N].float()
+        # (the slope of gelu is below 1.13)
+        assert ((got - torch.nn.functional.gelu(z, approximate="tanh") * e).abs() <= 2 ** -8 * (got.abs() + 1.2 * z.abs() * e.abs()) + 1e-3).all()
+    if device == "cuda":
+        tok = torch.tensor([3, -1, 11, 0], device=device)
+        y = hops.side_gate_product(torch.ones(4, 1024, dtype=torch.bfloat16, device=device), torch.ones(8, 1024, dtype=torch.bfloat16, device=device),
+                                   tok, emb.to(device), 0)
+        assert y[1:3].isnan().all() and y[[0, 3]].isfinite().all()

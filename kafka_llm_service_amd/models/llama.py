@@ -156,13 +156,13 @@ class TransformerLM:
 
     def enable_stream_weights(self, tiled_only: bool = False) -> int:
         """Keep a wave-tiled copy of every dense projection and of the lm_head (ops.tile_weight) so decode-sized
-        steps (T <= ops.STREAM_MAX_M) run the weight-streaming MFMA GEMM (csrc/wstream_gemm.hip) instead of
-        hipBLASLt; prefill-sized steps keep the row-major weights. Costs one more copy of those weights (16 GB for
+        steps (T <= ops.STREAM_MAX_M) run the weight-streaming MFMA GEMM (csrc/wstream_gemm.hip) and longer ones the tile
+        kernel (csrc/tile_gemm.hip), instead of hipBLASLt on the row-major weights. Costs one more copy of those weights (16 GB for
         Llama-3-8B: the HBM of an MI355X has room, and the KV pool is sized after this). Returns the added bytes.
 
         ``tiled_only``: when the second copy does not fit (Llama-3-70B on one GPU), the row-major dense projections
-        and the lm_head are dropped after tiling (no extra memory) and prefill-sized steps untile one weight at a
-        time into a transient buffer for hipBLASLt (``_dense``); MoE experts keep their row-major layout only
+        and the lm_head are dropped after tiling (no extra memory); prefill-sized steps run on the tiled weights too (the
+        tile kernel), but for shapes that it does not take, untiled one at a time into a transient buffer (``_dense``); MoE experts keep their row-major layout only
         (grouped GEMM at every step size — a tiled expert copy would be the 90 GB second copy this mode avoids)."""
         added = 0
         for lw in self.layers:
@@ -192,9 +192,8 @@ class TransformerLM:
                 added += self.lm_head_t.numel() * self.lm_head_t.element_size()
         self.stream = True
         self.tiled_only = tiled_only
-        # tiled-only: any larger step would untile every projection for hipBLASLt, so the streaming kernel takes
-        # steps up to its 256-row limit (two row tiles beyond 128) — slower than hipBLASLt there, far cheaper than
-        # untiling
+        # tiled-only: a larger step untiles the projections that the tile kernel does not take, so the streaming kernel takes
+        # steps up to its 256-row limit (two row tiles beyond 128), far cheaper than untiling
         self.stream_max_m = ops.STREAM_KERNEL_MAX_M if tiled_only else ops.STREAM_MAX_M
         if tiled_only and self.device.type == "cuda":
             torch.cuda.empty_cache()
@@ -280,7 +279,7 @@ class TransformerLM:
                 if ops.is_slab(a):
                     a = ops.silu_mul(a)
             else:
-                a = ops.linear_glu_long(x, lw.gate_up_t) if self.stream and lw.glu else None
+                a = ops.linear_glu_long(x, lw.gate_up_t, library=lw.gate_up is not None) if self.stream and lw.glu else None
                 if a is None:
                     a = ops.silu_mul(F.linear(x, self._dense(lw.gate_up, lw.gate_up_t, bool(lw.glu))))
             if tp and self._can_overlap(T, lw.down_t) and i + 1 < len(self.layers):

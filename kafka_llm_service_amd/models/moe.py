@@ -6,8 +6,8 @@ its own experts over the tokens routed to them and the per-rank partial outputs 
 that a dense row-parallel MLP would use (one collective per layer, [T, d] bf16). With ep = 1 the whole block is
 local (Mixtral 8x7B bf16 = 93 GB fits one 288 GB MI355X).
 
-Per layer: router GEMM (hipBLASLt) -> ``ops.moe_route`` (HIP, one workgroup: softmax + top-k + renormalise + stable
-expert sort, no host sync) -> ``ops.grouped_gemm`` gate_up (HIP MFMA, A rows gathered through the permutation) ->
+Per layer: router GEMM (``ops.linear_small``) -> ``ops.moe_route`` (HIP, one workgroup: softmax + top-k + renormalise + stable
+expert sort, no host sync; further ones clear the combine buffer) -> ``ops.grouped_gemm`` gate_up (HIP MFMA, A rows gathered through the permutation) ->
 ``ops.silu_mul`` -> ``ops.grouped_gemm`` down with the routing-weighted scatter-combine fused into its epilogue
 (fp32 atomics onto a zeroed [T, d] buffer). On CPU the same calls run the fp32 references of ``ops/reference.py``.
 """

@@ -472,10 +472,10 @@ def linear_long(x: torch.Tensor, w: torch.Tensor | None, wt: torch.Tensor | None
     return linear_dense(x, w if w is not None else untile_weight(wt))
 
 
-def linear_glu_long(x: torch.Tensor, wt: torch.Tensor, act: str = "silu") -> torch.Tensor | None:
+def linear_glu_long(x: torch.Tensor, wt: torch.Tensor, act: str = "silu", library: bool = True) -> torch.Tensor | None:
     """silu(x @ Wg^T) * (x @ Wu^T) of a long step from GLU-tiled weights (``act`` as in ``silu_mul``), None where the tile kernel does
-    not take it."""
-    plan = tile_plan(x.shape[0], wt.shape[0] * 32, x.shape[1], "glu") if tile_ok(x, wt) else None
+    not take it or, with a row-major weight for it (``library``), the library is as fast."""
+    plan = tile_plan(x.shape[0], wt.shape[0] * 32, x.shape[1], "glu", library) if tile_ok(x, wt) else None
     if plan is None:
         return None
     y = linear_tile(x, wt, plan, glu=True, act=act)

@@ -173,6 +173,13 @@ DECODE_TARGET_ITEMS = 1344  # (768 / 1536 / 2304 lose to it: profiles/r04/bench_
 # 64 rows of 1344 keys 844 / 818 (592 workgroups 833, 736 830), 16 of 3000 608 / 585, fp8 29 of 7900 768 / 745 (376 workgroups 787, 752 775), fp8 8 of 8000 611 / 570,
 # 90 of 700 793 / 775 (three a CU); 128 rows are more than that either way (1333 / 1336 on one piece each).
 DECODE_ROUNDS = (512, 768)
+# ... where the round's longest piece is at most this often the mean share, plus one shortest piece: a round lasts as long as its longest
+# piece, and with few pieces beside the rows a long row stays whole. A step of four layers, 63 rows of 500 keys and one of 60000: 5155 us in one
+# round, 780 else; 64 rows of 100 - 8000 1051, 815. us of the attention alone, 1344 workgroups / one round: 64
+# rows of 1344 keys, +- 17 % 67.7 / 59.8, 50 % 70.6 / 66.5, 70 % 60.2 / 66.8, one row eight times as long 74 / 186, contexts log-uniform over a factor of 60 69 / 104;
+# 300 keys +- 90 % 24.2 / 21.2; 4500 keys, 33 % 201 / 195, 70 % 200 / 211, 32 rows of them +- 33 % 99.7 / 101.5. Over 363 batches of 4 - 96 rows
+# this line takes 6.8 % off the attention, always one round 3.6 %, the better plan of each batch 7.1 %.
+ROUND_SHARE = 1.25
 
 
 def decode_round(n: int) -> int:
@@ -317,11 +324,25 @@ def prefix_groups(bt: np.ndarray, nfull: np.ndarray, min_blocks: int) -> tuple[l
     return order, [(len(rows), p) for rows, p in groups]
 
 
+def round_pieces(nb: np.ndarray, n: int, cap: np.ndarray) -> np.ndarray | None:
+    """Pieces of every row (``nb`` 32-key blocks, at most ``cap`` pieces) of a launch of at most ``n``, as short as 16 tried lengths
+    get them; None where the longest would be past its bound (ROUND_SHARE)."""
+    share, short = int(nb.sum()) / n, MIN_DECODE_KEYS // 32
+    top = int(ROUND_SHARE * share) + short
+    k = np.linspace(max(short, math.ceil(share)), top, 16).astype(np.int64)
+    fits = np.minimum(-(-nb // k[:, None]), cap).sum(1) <= n
+    if not fits[-1]:
+        return None
+    ns = np.minimum(-(-nb // k[int(fits.argmax())]), cap)
+    return ns if int((-(-nb // ns)).max()) <= top else None
+
+
 def decode_items(seq_lens: np.ndarray, kv_start: np.ndarray, npre: np.ndarray, hkv: int,
                  target: int = DECODE_TARGET_ITEMS, min_keys: int = MIN_DECODE_KEYS) -> np.ndarray:
     """Work items (b, lo, hi, split, nsplit, npre, 0, 0) of the decode kernel: every row's keys [kv_start, len) in
     32-key-aligned pieces of about ``ch`` keys, ``ch`` chosen so the launch has ~``target`` workgroups (x Hkv) of
-    about equal bytes (long histories are split, short ones stay whole); at most MAX_PARTIALS - npre pieces."""
+    about equal bytes (long histories are split, short ones stay whole); at most MAX_PARTIALS - npre pieces. Where that is more than
+    the round that the rows leave room in (``decode_round``), pieces for that round if they come out balanced (``round_pieces``)."""
     B = seq_lens.shape[0]
     suffix = np.maximum(seq_lens - kv_start, 1).astype(np.int64)
     # fewer rows than it takes to fill the GPU (B x Hkv < 512 workgroups): split so the launch still has ~512
@@ -336,11 +357,11 @@ def decode_items(seq_lens: np.ndarray, kv_start: np.ndarray, npre: np.ndarray, h
     bps = -(-nb // ns)
     ns = -(-nb // bps)  # no empty trailing piece
     whole = decode_round(B * hkv) if target > 0 else 0
-    while whole and int(ns.sum()) * hkv > whole:     # (rounding up gave the rows more pieces than the round has)
-        ch += max(32, ch // 16 // 32 * 32)
-        ns = np.minimum(np.maximum(1, -(-suffix // ch)), MAX_PARTIALS - npre)
-        bps = -(-nb // ns)
-        ns = -(-nb // bps)
+    if whole and int(ns.sum()) * hkv > whole:
+        even = round_pieces(nb, whole // hkv, MAX_PARTIALS - npre)
+        if even is not None:
+            bps = -(-nb // even)
+            ns = -(-nb // bps)
     rows = np.repeat(np.arange(B), ns)
     first = np.cumsum(ns) - ns
     split = np.arange(rows.shape[0]) - np.repeat(first, ns)
@@ -837,8 +858,10 @@ class ModelRunner:
     def _plan_decode_items(self, h: HostStep, seq_lens: np.ndarray, kv_start: np.ndarray, npre: np.ndarray,
                            i32_parts: list) -> None:
         if self.graphs is not None or self.fixed_decode_items:  # graph replay: the decode grid depends on B alone
+            # (one round where it has three pieces a row: rows of any lengths are balanced then. us of the attention, 1344 workgroups / one
+            # round: 16 rows of 1344 keys 25.1 / 19.9, one of them eight times as long 36.3 / 27.8, 32 rows of 4500 102 / 96, 122 / 116)
             ditems = decode_items_fixed(seq_lens, kv_start, npre, self.model.hkv,
-                                        decode_round(len(seq_lens) * self.model.hkv) or DECODE_TARGET_ITEMS)
+                                        decode_round(3 * len(seq_lens) * self.model.hkv) or DECODE_TARGET_ITEMS)
         else:
             ditems = decode_items(seq_lens, kv_start, npre, self.model.hkv)
         h.n_dec_items = int(ditems.shape[0])

@@ -440,6 +440,50 @@ def test_prefix_groups_and_decode_items():
             assert len(rows) + npre[b] <= MAX_PARTIALS
 
 
+@pytest.mark.parametrize("lens", [[500] * 63 + [60000], [500] * 63 + [8000], [300] * 89 + [30000], [100] * 63 + [100000],
+                                  [1000] * 63 + [20000], list(range(200, 2600, 37))[:64], list(range(100, 8000, 123))[:64],
+                                  list(range(100, 8000, 82))[:96], list(range(100, 8000, 250))[:32], [500] * 94 + [30000] * 2])
+def test_decode_pieces_balanced_on_uneven_contexts(lens, monkeypatch):
+    """A launch lasts as long as its longest piece: on contexts that differ it is no longer than that of the pieces for
+    DECODE_TARGET_ITEMS workgroups, or than the bound of a whole round; plans of captured steps have a size by the rows alone."""
+    import numpy as np
+
+    from kafka_llm_service_amd.engine import model_runner as mr
+
+    lens, z, hkv = np.array(lens), np.zeros(len(lens), dtype=np.int64), 8
+    it = mr.decode_items(lens, z, z, hkv)
+    whole = mr.decode_round(len(lens) * hkv)
+    share = -(-lens // 32).sum() * 32 * hkv / whole
+    longest = (it[:, 2] - it[:, 1]).max()
+    assert np.bincount(it[:, 0], weights=it[:, 2] - it[:, 1]).tolist() == lens.tolist() and (it[:, 2] > it[:, 1]).all()
+    monkeypatch.setattr(mr, "DECODE_ROUNDS", ())
+    parts = mr.decode_items(lens, z, z, hkv)
+    assert longest <= max((parts[:, 2] - parts[:, 1]).max(), 1.25 * share + 256)
+    monkeypatch.undo()
+    r = mr.ModelRunner.__new__(mr.ModelRunner)
+    r.graphs, r.fixed_decode_items, r.model = None, True, type("M", (), {"hkv": hkv})
+    n = set()
+    for x in (lens, np.full(len(lens), int(lens.mean()))):
+        h, out = mr.HostStep(B=len(x)), []
+        r._plan_decode_items(h, x, z, z, out)
+        f = out[0].reshape(-1, 8)
+        n.add(len(f))
+        assert (f[:, 2] - f[:, 1]).max() <= max(2 * -(-x // 32).sum() * 32 / len(f), -(-x.max() // mr.MAX_PARTIALS) + 32)
+    assert len(n) == 1
+
+
+@pytest.mark.parametrize("rows, keys, workgroups", [(64, 1344, 512), (61, 1344, 512), (16, 3000, 512), (8, 8000, 512),
+                                                    (29, 7900, 512), (90, 700, 768)])
+def test_decode_pieces_of_even_contexts_fill_one_round(rows, keys, workgroups):
+    import numpy as np
+
+    from kafka_llm_service_amd.engine import model_runner as mr
+
+    lens = keys - np.arange(rows) * 613 % (keys // 3 + 1)
+    it = mr.decode_items(lens, np.zeros_like(lens), np.zeros_like(lens), 8)
+    assert 0.9 * workgroups < len(it) * 8 <= workgroups
+
+
 def test_tiled_only_mixtral_and_export(tmp_path):
     """Tiled-only mode on an MoE model: experts stay row-major (no second expert copy), the lm_head keeps only its
     tiled copy, generation equals the two-copy stream mode, and safetensors export untiles what was dropped."""

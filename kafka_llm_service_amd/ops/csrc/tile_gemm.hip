@@ -92,6 +92,7 @@ extern "C" hipError_t kafka_launch_tile_gemm(const bf16* X, int64_t ldx, const b
   if (M <= 0) return hipSuccess;
   const bool glu = act & 1;
   if (act < 0 || act > 3 || (act == 2 && P)) return hipErrorInvalidValue;
+  if (glu && Y && nt % 4) return hipErrorInvalidValue;   // (a wave holds whole gate, up pairs)
   if (N < 32 || N % 32 || K % 64 || splits < 1 || K / 64 < 2 * splits || ldx % 8 || (glu && N % 64)) return hipErrorInvalidValue;
   if ((Y != nullptr) == (P != nullptr) || (Y && (splits != 1 || ldy % 8 || reinterpret_cast<uintptr_t>(Y) % 16)))
     return hipErrorInvalidValue;

@@ -105,6 +105,20 @@ def test_gelu_gated_products(M):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mt,nt", [t for t in sorted(ops.TILES) if t[1] % 4])
+def test_gates_need_whole_pairs_in_a_wave(mt, nt):
+    """Tiles whose waves hold three 32-column tiles cannot activate gate, up pairs: refused; their slabs are in gate | up order."""
+    x, w = torch.randn(65, 128).to(torch.bfloat16).cuda(), torch.randn(384, 128).to(torch.bfloat16).cuda() / 12
+    wt = ops.tile_weight(w, glu=True)
+    for act in ("silu", "gelu"):
+        with pytest.raises(RuntimeError):
+            ops.linear_tile(x, wt, (mt, nt, 1), glu=True, act=act)
+    p = torch.empty(1, 65, 384, device="cuda")
+    ops.ext().tile_gemm(x, wt, None, p, mt, nt, 1, True)
+    assert ((p[0] - x.float() @ w.float().t()).abs() <= 1e-4).all()
+
+
+@pytest.mark.gpu
 def test_relu_squared_of_what_is_not_finite():
     """NaN stays, minus infinity is zero, plus infinity infinite."""
     x = torch.ones(200, 128, dtype=torch.bfloat16, device="cuda")

@@ -310,8 +310,8 @@ __global__ __launch_bounds__(256, 1) void grouped_ring_kernel(const bf16* __rest
   const int seg0 = expert_off[e] + rt * BM, rows = min(BM, expert_off[e + 1] - seg0);
   const RingArgs A{X, ldx, Wt, N, K, perm_tok, perm_w, Y, ldy, out, ldo, glu_limit, glu_alpha};
   // an expert's last rows on a lower tile where they fit one: the weights' way is then what it takes, a third of a whole tile
-  // (sums added to memory take as long either way)
-  if (rows > 128 || EPI == EPI_COMBINE) ring_tile<8, GATHER, EPI>(A, smem, e, seg0, rows, nt);
+  // (22 rows an expert, us, whole / low tile of the combined product: 8 experts 2304 -> 2048 46 / 22, 4608 -> 4096 85 / 64, 64 of 768 -> 2048 50 / 40)
+  if (rows > 128) ring_tile<8, GATHER, EPI>(A, smem, e, seg0, rows, nt);
   else if (rows > 64) ring_tile<4, GATHER, EPI>(A, smem, e, seg0, rows, nt);
   else ring_tile<2, GATHER, EPI>(A, smem, e, seg0, rows, nt);
 }
@@ -659,15 +659,21 @@ hipError_t kafka_launch_grouped_wide(const bf16* X, int64_t ldx, const bf16* Wt,
                        (int64_t)N * K * 2 < (int64_t)0xffff0000 &&
                        (epi == EPI_COMBINE || (ldy % 8 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0));
   if (bm == 0) {
-    // Which tiles, from the mean rows of an expert. Up to 128 rows the ring kernel's low tiles (us, 128-row kernel / ring, 40 - 100 rows
-    // of each of 8 experts: 4096 -> 2 x 4608 148 - 154 / 142 - 158, 4608 -> 4096 79 - 86 / 68 - 82, 2048 -> 2 x 2304 39 / 30,
-    // 2304 -> 2048 42 / 26). Beyond, by rounds: one is 256 tiles of 256 x 256 or 512 of 128 x 256, the same products; the ring
+    // Which tiles, from the mean rows r of an expert. Few rows: the ring kernel's low tiles, up to 96 rows (an expert of more than 128
+    // takes a whole tile) in the first product and 128 in the second. us, 128-row kernel / ring: 8 experts 2048 -> 2 x 2304 40 rows 37 / 27,
+    // 90 40 / 31, 110 42 / 50; 4096 -> 2 x 4608 40 rows 147 / 143, 90 152 / 156, 110 150 / 182; 4608 -> 4096 rows 77 / 67, 95 / 83 combined, 110 87 / 88;
+    // 16 experts 1536 -> 4096 combined 40 rows 42 / 37, 110 72 / 57; 64 experts 4096 -> 2 x 1536 4 rows 269 / 264, 40 282 / 275, 1536 -> 4096 combined 40
+    // rows 164 / 160, 110 249 / 220; 256 of them 4 rows 529 / 540, 40 672 / 673, 110 939 / 888. Very short rows of many tiles wait for a tile's start,
+    // which two workgroups a CU hide: 256 experts 512 -> 2048 combined 4 rows 103 / 115, 22 125 / 136, 40 152 / 155; 16 experts 22 rows 19 / 12.
+    // Beyond, by rounds: one is 256 tiles of 256 x 256 or 512 of 128 x 256, the same products; the ring
     // kernel does them 1.4 times as fast, but in whole rounds, the other one's last round thins out (a quarter of one on
-    // average): 2048 -> 2 x 2304 280 rows 63 / 99, 600 rows 100 / 100, 1300 rows 218 / 208; 4096 -> 2 x 14336 140 rows 504 / 446, 600 rows 1143 / 1025.
+    // average); a mean of 128 rows is 1.6 tiles of 128: 2048 -> 2 x 2304 280 rows 63 / 99, 600 rows 100 / 100, 1300 rows 218 / 208;
+    // 4096 -> 2 x 14336 140 rows 454 / 428, 600 rows 1143 / 1025.
     const int64_t r = ((int64_t)n_ent + E - 1) / E, ct = (N + BN - 1) / BN * (int64_t)E;
+    const bool low = r <= (epi == EPI_GLU || epi == EPI_RELU2 ? 96 : 128) && (K >= 768 || r >= 32 || ct <= 512);
     const double ring_rounds = (double)(((r + 255) / 256 * ct + 255) / 256) / 1.4;
-    const double wide_rounds = (double)((r + 127) / 128 * ct) / 512 + 0.25;
-    bm = ring_ok && (r <= 128 || ring_rounds < wide_rounds) ? 256 : 128;
+    const double wide_rounds = (r <= 128 ? r / 128.0 + 0.6 : (double)((r + 127) / 128)) * ct / 512 + 0.25;
+    bm = ring_ok && (low || ring_rounds < wide_rounds) ? 256 : 128;
   }
   if ((bm != 128 && bm != 256) || (bm == 256 && N % 128)) return hipErrorInvalidValue;
   if (bm == 256 && !ring_ok) bm = 128;

@@ -1051,6 +1051,28 @@ def test_wide_expert_products_on_low_row_tiles(rows, N, K):
     test_wide_expert_products_on_256_row_tiles(rows, N, K)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,N,K", [(3, 256, 256), (5, 384, 768), (130, 1024, 256)])
+@pytest.mark.parametrize("rows", [1, 31, 33, 96, 98, 128, 130])
+def test_expert_products_on_either_side_of_the_tile_choice(E, N, K, rows):
+    """About ``rows`` rows of each expert, of sizes that differ: what the launcher picks is one of the two kernels' results (sums of the
+    same products in another order, rounded to bf16; the combined rows in fp32)."""
+    from kafka_llm_service_amd import ops
+
+    g = torch.Generator().manual_seed(rows)
+    te = torch.multinomial(torch.rand(E, generator=g) + 0.5, rows * E, replacement=True, generator=g).int()[:, None]
+    n = te.shape[0]
+    r = ops.moe_sort(torch.rand(n, 1, generator=g).cuda(), te.cuda(), E)
+    x = torch.randn(n, K, generator=g).to(torch.bfloat16).cuda()
+    wt = ops.tile_experts((torch.randn(E, N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda())
+    for epi in ("relu2", "rows", "combine"):
+        y = []
+        for tile in (0, 128, 256):
+            out = torch.zeros(n, N, device="cuda") if epi == "combine" else None
+            y.append(ops.grouped_wide(x, wt, r, epi, True, out, tile=tile).float())
+        assert all(((y[0] - z).abs() <= (2 ** -7 * z.abs() + 1e-3 if out is None else 1e-4)).all() for z in y[1:])
+
+
 def test_items_that_share_keys():
     """Which of a step's attention items count for the kernel that shares keys among eight of them: all of prompt portions, those of
     more than one token beside decoded ones (160 of one token and 2 portions of 5 items of 8: 10), none where items of one token

@@ -387,6 +387,26 @@ TILE_WHOLE_GAIN = 0.8
 
 
 @lru_cache(maxsize=4096)
+def _tile_best(M: int, N: int, K: int, form: str) -> tuple[float, tuple[int, int, int]]:
+    """(us, plan) of the fastest launch of ``tile_plan`` by the figures above."""
+    best = None
+    for (mt, nt), (launch, rnd, unit, out) in TILES.items():
+        if form == "glu" and nt % 4:
+            continue                # (a wave holds whole gate, up pairs)
+        items = -(-M // (32 * mt)) * -(-N // (32 * nt))
+        for s in TILE_SPLITS:
+            if K // 64 < 2 * s or s > 1 and (form == "relu2" or 4 * s * M * N > TILE_SLAB_BYTES):
+                break
+            mb = M * N / 4.5e6
+            t = launch + -(-items * s // 256) * (rnd + unit * (K // 64) / s) + out * mb * (4 * s if s > 1 else 2)
+            if s > 1:               # the slabs' way back in, beside that of a bf16 output; a launch of its own but for "slabs"
+                t += mb * (4 * s - 2) if form == "slabs" else 6 + mb * (4 * s + 2)
+            if best is None or t < best[0]:
+                best = (t, (mt, nt, s))
+    return best
+
+
+@lru_cache(maxsize=4096)
 def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) -> tuple[int, int, int] | None:
     """(16-row parts, 16-column parts, splits) of the tile kernel for x [M, K] @ W^T [N, K], None where it does not take the shape or
     the library is as fast. ``form``: "slabs" (the consumer sums the split-K slabs as it loads them), "bf16" (slabs go
@@ -416,20 +436,8 @@ def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) 
     if library and M > TILE_MAX_M and \
             (M > (TILE_GLU_M if act else TILE_RAGGED_M if N % 256 else TILE_EVEN_M) or tiles <= (512 if act else 256)):
         return None
-    best = None
-    for (mt, nt), (launch, rnd, unit, out) in TILES.items():
-        if form == "glu" and nt % 4:
-            continue                # (a wave holds whole gate, up pairs)
-        items = -(-M // (32 * mt)) * -(-N // (32 * nt))
-        for s in TILE_SPLITS:
-            if K // 64 < 2 * s or s > 1 and (form == "relu2" or 4 * s * M * N > TILE_SLAB_BYTES):
-                break
-            mb = M * N / 4.5e6
-            t = launch + -(-items * s // 256) * (rnd + unit * (K // 64) / s) + out * mb * (4 * s if s > 1 else 2)
-            if s > 1:               # the slabs' way back in, beside that of a bf16 output; a launch of its own but for "slabs"
-                t += mb * (4 * s - 2) if form == "slabs" else 6 + mb * (4 * s + 2)
-            if best is None or t < best[0]:
-                best = (t, (mt, nt, s))
+    # (tiles are multiples of 64 rows high: sizes up to the next 64 share a search, 15 us of the host, else each new length of a prompt pays it)
+    best = _tile_best(-(-M // 64) * 64, N, K, form)
     if library and M > (768 if tiles > 256 else 1024):
         rows = M // DENSE_BLOCK * DENSE_BLOCK if dense_cut(M, N, K) else M
         lib = 4 + -(-(-(-rows // 256) * -(-N // 256)) // 256) * 1.42 * (K // 64) + (20 if rows < M else 0)

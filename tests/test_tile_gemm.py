@@ -33,6 +33,24 @@ def test_plans_are_launches():
     assert ops.tile_plan(300, 28672, 4096) is None and ops.tile_plan(300, 28672, 4096, "glu") is not None
 
 
+def test_lengths_share_a_search():
+    """A prompt of a length that had none before asks for a plan once per 64 rows, not once per length, and gets the plan that its own length
+    would or one behind by no more than the rows between."""
+    ops._tile_best.cache_clear()
+    for M in range(1985, 2049):
+        for form in ("slabs", "glu"):
+            assert ops.tile_plan(M, 6144, 1984, form, library=False) is not None
+    assert ops._tile_best.cache_info().misses == 2
+    rng = random.Random(5)
+    for _ in range(400):
+        M, N, K = rng.randint(129, 9000), 64 * rng.randint(1, 450), 64 * rng.randint(2, 230)
+        form = rng.choice(["slabs", "bf16", "glu", "relu2"])
+        own, up = ops._tile_best(M, N, K, form), ops._tile_best(-(-M // 64) * 64, N, K, form)
+        assert own[0] <= up[0]
+        if own[1] != up[1]:
+            assert up[0] <= own[0] * (1 + 64 / M)
+
+
 def test_long_products_on_the_cpu():
     """Without a GPU linear_long is the plain product, from either weight, whatever the strides of x."""
     w = torch.randn(96, 128)

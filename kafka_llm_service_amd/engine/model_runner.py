@@ -539,8 +539,9 @@ class ModelRunner:
         self.variant = int(os.environ.get("KAFKA_TILE_VARIANT", "0" if fp8 else "3"))
         if fp8 and self.variant == 3:
             raise ValueError("tile variant 3 reads bf16 KV pages only")
-        # mixed steps of 129..256 rows padded away from hipBLASLt's slow sizes (dense TP = 1 GPU models)
-        self.pad_rows = (self.device.type == "cuda" and model.tp == 1 and not getattr(model, "tiled_only", False)
+        # mixed steps of 129..256 rows padded away from hipBLASLt's slow sizes (TP = 1 GPU models whose products are the library's: with
+        # tiled weights they are the tile kernel's, which has none)
+        self.pad_rows = (self.device.type == "cuda" and model.tp == 1 and not getattr(model, "stream", False)
                          and os.environ.get("KAFKA_PAD_ROWS", "1") == "1")
         self.tile = ops.tile_rows(self.variant) // self.G  # tokens per attention work item
         # the v3 cascade hands its prefix partials to the decode kernel as bf16 (normalised O, fp32 lse): ~33 MB

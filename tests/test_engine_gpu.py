@@ -117,3 +117,23 @@ def _run_logits(e, prompts, sps):
     finally:
         e.runner.sample_device = orig
     return outs, seen
+
+
+@pytest.mark.parametrize("rows", [129, 150, 192, 255])
+def test_steps_of_129_to_256_rows_run_as_they_are(eng, rows):
+    """No inert rows beside those of a step whose products are the tile kernel's; the library's keep them."""
+    prompt = _prompts(rows, rows, (0,))
+    seen, orig = [], eng.runner.build_host
+
+    def build_host(batch):
+        h, ss = orig(batch)
+        seen.append(h.T)
+        return h, ss
+    eng.runner.build_host = build_host
+    outs = eng.generate(prompt, GREEDY)
+    eng.runner.build_host = orig
+    assert rows in seen
+    _oracle_ok(eng.model, prompt, outs)
+    if rows == 129:
+        blas = LLMEngine(EngineConfig(model="tiny-llama", device="cuda:0", num_kv_blocks=64, max_model_len=512, decode_gemm="blas"))
+        assert blas.runner.pad_rows and not eng.runner.pad_rows

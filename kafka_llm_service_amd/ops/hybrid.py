@@ -1141,7 +1141,8 @@ def linear_f32(x, w, bias=None) -> torch.Tensor:
         from kafka_llm_service_amd import ops
 
         if x.dim() == 2 and ops.small_ok(x, w, SMALL_F32_ROWS) and 1024 <= w.shape[1] and w.shape[0] <= 64 and \
-                (bias is None or bias.data_ptr() % 16 == 0):
+                (bias is None or bias.dtype == torch.float32 and bias.shape == w.shape[:1] and bias.is_contiguous() and
+                 bias.data_ptr() % 16 == 0):
             out = torch.empty(x.shape[0], w.shape[0], dtype=torch.float32, device=x.device)
             ext().small_gemm(x, w, out, bias)
             return out

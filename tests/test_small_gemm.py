@@ -48,6 +48,20 @@ def test_against_fp32(K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K", [1032, 2056])
+def test_biases_of_other_forms(K):
+    """Rows that the kernel for few weight rows does not take (K in steps of 8) have taken any bias that adds to the result: bf16, every second
+    element, one for all columns, one a row."""
+    g = torch.Generator().manual_seed(K)
+    for M, N in ((3, 16), (40, 64)):
+        x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+        w = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
+        want, b = x.float() @ w.float().t(), torch.randn(2 * N, generator=g).cuda()
+        for bias in (b[:N].to(torch.bfloat16), b[::2], b[:1], b[:N].expand(M, N), b[:M, None] if M <= 2 * N else b[:1, None]):
+            assert ((hops.linear_f32(x, w, bias) - want - bias).abs() <= 2e-5).all()
+
+
+@pytest.mark.gpu
 def test_rows_beyond_and_forms_of_the_library():
     """One row past each limit, and operands that the kernel does not take (odd columns, odd strides, a shifted start)."""
     g = torch.Generator().manual_seed(1)

@@ -348,12 +348,12 @@ def skinny_plan(M: int, N: int, K: int, max_splits: int = 8) -> int:
 # ---- small products (csrc/small_gemm.hip) -----------------------------------------------------------------------------
 def small_ok(x: torch.Tensor, w: torch.Tensor, rows: int) -> bool:
     """Whether x [.., M, K] @ w [.., N, K]^T of up to ``rows`` rows runs on the kernel for small products: bf16 operands of one
-    order, whole 16-byte pieces."""
+    order, whole 16-byte pieces, extents of its grid."""
     d, K = x.dim(), x.shape[-1]
     return x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and d == w.dim() and w.shape[-1] == K and \
-        0 < x.shape[-2] <= rows and K % 8 == 0 and K > 0 and w.shape[-2] % 4 == 0 and w.shape[-2] > 0 and \
+        0 < x.shape[-2] <= rows and K % 8 == 0 and 0 < K < 1 << 20 and w.shape[-2] % 4 == 0 and 0 < w.shape[-2] < 1 << 19 and \
         x.stride(-1) == 1 and w.stride(-1) == 1 and x.stride(-2) % 8 == 0 and w.stride(-2) % 8 == 0 and \
-        (d == 2 or d == 3 and x.shape[0] == w.shape[0] and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0) and \
+        (d == 2 or d == 3 and x.shape[0] == w.shape[0] < 1 << 16 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0) and \
         x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
 
 

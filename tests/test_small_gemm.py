@@ -79,6 +79,21 @@ def test_rows_beyond_and_forms_of_the_library():
 
 
 @pytest.mark.gpu
+def test_extents_beyond_the_kernels_grid():
+    """Columns, depth and heads that its launch refuses, and the last ones that it takes: the library's or the kernel's, the same product."""
+    for M, N, K in ((2, 4, 1 << 20), (2, 4, (1 << 20) - 8), (2, 1 << 20, 8), (2, 1 << 19, 8), (2, (1 << 19) - 4, 8)):
+        x, w = torch.ones(M, K, dtype=torch.bfloat16, device="cuda"), torch.ones(N, K, dtype=torch.bfloat16, device="cuda")
+        w[-1] = 2
+        y = ops.linear_small(x, w).float()
+        assert (y[:, :-1] == x[:1].float().sum().to(torch.bfloat16).float()).all() and (y[:, -1] == 2 * y[:, 0]).all()
+    for H in ((1 << 16) - 1, 1 << 16):
+        x, w = torch.ones(H, 1, 8, dtype=torch.bfloat16, device="cuda"), torch.ones(H, 4, 8, dtype=torch.bfloat16, device="cuda")
+        w[-1] = 2
+        y = head_product(x, w, w.transpose(1, 2).contiguous())
+        assert (y[:-1] == 8).all() and (y[-1] == 16).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 16, 63, 64, 65])
 def test_heads(n):
     """Products per head into the head's columns of a wider row and into rows of their own, queries as slices of a fused row."""

@@ -74,10 +74,15 @@ def _whole_rows(t: torch.Tensor, idx: torch.Tensor) -> bool:
         t.data_ptr() % 16 == 0
 
 
+def _whole_norm(w: torch.Tensor, d: int) -> bool:
+    """A norm's weight that the row kernels read in 16-byte pieces."""
+    return w.dtype == torch.bfloat16 and w.shape == (d,) and w.is_contiguous() and w.data_ptr() % 16 == 0
+
+
 def embed_rmsnorm(table: torch.Tensor, tokens: torch.Tensor, w: torch.Tensor, eps: float) -> tuple[torch.Tensor, torch.Tensor]:
     """(rows = table[tokens], rmsnorm(rows) * w), both new: a step's residual stream and its first layer's input."""
     n, d = tokens.shape[0], table.shape[1]
-    if n and _whole_rows(table, tokens) and table.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and d <= 16384:
+    if n and _whole_rows(table, tokens) and table.dtype == torch.bfloat16 and _whole_norm(w, d) and d <= 16384:
         r = torch.empty(n, d, dtype=table.dtype, device=table.device)
         x = torch.empty_like(r)
         ext().rows_norm(x, table, r, tokens, w, float(eps), True)
@@ -90,7 +95,7 @@ def rows_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, rows: torch.Tensor
     """rmsnorm(x[rows] + residual[rows]) * w (``x`` bf16 or a slab); neither is written."""
     slab = is_slab(x)
     if rows.shape[0] and _whole_rows(x, rows) and _whole_rows(residual, rows) and residual.shape[1] <= 16384 and \
-            residual.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and (slab or x.dtype == torch.bfloat16):
+            residual.dtype == torch.bfloat16 and _whole_norm(w, residual.shape[1]) and (x.is_contiguous() if slab else x.dtype == torch.bfloat16):
         out = torch.empty(rows.shape[0], residual.shape[1], dtype=residual.dtype, device=x.device)
         ext().rows_norm(out, x, residual, rows, w, float(eps), False)
         return out

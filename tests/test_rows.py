@@ -44,3 +44,18 @@ def test_on_the_gpu():
     for t in (r, x, f, y):
         assert torch.isnan(t[1:3]).all() and torch.isfinite(t[0]).all() and torch.isfinite(t[3]).all()
     assert torch.equal(r[[0, 3]], table[[4, 0]])
+
+
+@pytest.mark.parametrize("dev,dtype", [("cpu", torch.float32), pytest.param("cuda", torch.bfloat16, marks=pytest.mark.gpu)])
+def test_weights_and_slabs_that_the_kernels_do_not_read(dev, dtype):
+    """A norm's weight that starts between two 16-byte pieces, and slabs that are a view: the separate operations take them."""
+    g = torch.Generator().manual_seed(4)
+    table, w = torch.randn(11, 256, generator=g).to(dtype).to(dev), torch.rand(257, generator=g).to(dtype).to(dev)[1:]
+    idx = torch.randint(0, 11, (5,), generator=g).to(dev)
+    r, x = ops.embed_rmsnorm(table, idx, w, 1e-5)
+    assert torch.equal(r, table[idx]) and torch.equal(x, ops.rmsnorm(table[idx], w, 1e-5))
+    want = ops.fused_add_rmsnorm(table[idx], table[idx], w, 1e-5)
+    assert torch.equal(ops.rows_add_rmsnorm(table, table, idx, w, 1e-5), want)
+    even, wide = w.clone(), torch.randn(2, 14, 256, generator=g).to(dev)[:, 1:12]
+    want = ops.fused_add_rmsnorm(wide.index_select(1, idx), table[idx], even, 1e-5)
+    assert torch.equal(ops.rows_add_rmsnorm(wide, table, idx, even, 1e-5), want)

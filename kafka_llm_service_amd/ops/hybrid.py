@@ -49,7 +49,12 @@ def add_ln(x, y, w, b, eps, out2=None, w2=None, b2=None) -> None:
     out2's dtype when no second norm is given. y [T, d] in the weights' dtype, or the fp32 split-K slabs [S, T, d] of a
     projection (summed here)."""
     if y.dim() == 3 and not (_gpu(x) and x.shape[1] <= 4096 and w.dtype == torch.bfloat16 and y.is_contiguous()):
-        y = y.sum(0).to(w.dtype)
+        if w.dtype == torch.bfloat16 and y.is_contiguous() and y.shape[2] % 8 == 0:   # (rows wider than the kernel's registers hold)
+            from kafka_llm_service_amd import ops
+
+            y = ops.slab_reduce(y)
+        else:
+            y = y.sum(0).to(w.dtype)
     if _gpu(x):
         ext().hy_add_ln(x, y, w, b, float(eps), out2, w2, b2)
     else:

@@ -1140,6 +1140,18 @@ def test_add_norm_of_slabs(device, d, T):
             assert ((o.cpu().double() - want).abs() <= (2 ** -8 + d * 2.0 ** -24 + 1e-5) * (want.abs() + 1)).all()
 
 
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("d", [4104, 8192])
+def test_add_norm_of_wide_slabs_reduces_them_in_one_pass(device, d, monkeypatch):
+    """Rows wider than the kernel takes slabs of: the reduction that a projection's own output goes through, not a sum and a conversion."""
+    from kafka_llm_service_amd import ops
+
+    calls, orig = [], ops.slab_reduce
+    monkeypatch.setattr(ops, "slab_reduce", lambda y: calls.append(y.shape) or orig(y))
+    test_add_norm_of_slabs(device, d, 3)
+    assert calls == [(S, 3, d) for S in (1, 2, 3, 4, 8) for _ in range(2)]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("d,T", [(4, 3), (1024, 3), (1028, 5), (1030, 5), (4096, 7), (4096, 600), (4100, 3), (1022, 2)])

@@ -153,12 +153,12 @@ class LLMEngine:
                 self.model.enable_stream_weights()  # before the KV pool is sized from the free memory
             else:  # e.g. Llama-3-70B on one GPU: a second copy of 140 GB would starve the KV pool
                 log.warning("wave-tiled weight copy (%.1f GB) does not fit next to the KV pool (%.1f GB free): "
-                            "keeping tiled weights only (prefill untiles per projection)", need / 1e9, free / 1e9)
+                            "keeping tiled weights only (long steps untile the projections that the tile kernel does not take)", need / 1e9, free / 1e9)
                 self.model.enable_stream_weights(tiled_only=True)
         elif mode == "stream_only" and not self.model.stream:
             self.model.enable_stream_weights(tiled_only=True)
         if self.model.tiled_only and cfg.max_num_seqs > self.model.stream_max_m:
-            # decode batches beyond the streaming kernel's rows would untile every projection every step
+            # decode batches beyond the streaming kernel's rows would untile what the tile kernel does not take in every step
             log.info("tiled-only weights: max_num_seqs %d -> %d", cfg.max_num_seqs, self.model.stream_max_m)
             cfg.max_num_seqs = self.model.stream_max_m
         self.load_s = time.perf_counter() - t0
@@ -337,9 +337,9 @@ class LLMEngine:
 
     def _step_rows_fit(self) -> int:
         """Row fit of the scheduler (engine/scheduler.py): explicit config, else env KAFKA_STEP_ROWS_FIT, else on
-        (ops.STREAM_MAX_M) only for tiled-only weights — there a step beyond the streaming kernel's rows untiles
-        every projection for hipBLASLt, which costs far more than splitting a new turn over two steps (Llama-3-70B
-        on one GPU: profiles/r02/bench_70b_tp1_*), while with both weight copies the fit measured slower
+        (ops.STREAM_MAX_M) only for tiled-only weights — drawn when a step beyond the streaming kernel's rows untiled
+        every projection for hipBLASLt, which cost far more than splitting a new turn over two steps (Llama-3-70B
+        on one GPU: profiles/r02/bench_70b_tp1_*; most run on the tile kernel now, not measured there), while with both weight copies the fit measured slower
         (profiles/r02/step_rows_fit_rejected.jsonl)."""
         if self.cfg.step_rows_fit is not None:
             return self.cfg.step_rows_fit

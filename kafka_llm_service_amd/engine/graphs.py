@@ -7,7 +7,7 @@ write / cascade + split-K paged attention / merge, final norm, lm_head, sampler)
 cost drops from ~2 ms to ~20 us, which is what lets the host keep up with short decode steps (small batches, TP
 shards) and leaves the CPU free for the API loop.
 
-Layout key: (B, decode work items (padded to a power of two), partial slots, prefix work items, cascade on/off, packed-buffer sizes,
+Layout key: (B, decode work items (a number by B alone), partial slots, prefix work items, cascade on/off, packed-buffer sizes,
 greedy, logits processing on/off). Everything that changes from step to step — token ids, positions, KV slots, block
 tables, sequence lengths, cascade work items, sampling parameters, seeds and the rows' logits-processing entries
 (grammar mask rows / forced tokens / penalty slots, engine/logits_proc.py: the mask and count tables sit at fixed

@@ -36,9 +36,8 @@ class SchedulerConfig:
     tpot_guard_decodes: int = 16
     # Row fit: while the guard holds, prefill is also capped so the whole step stays within `step_rows_fit` rows
     # (0 = off) as long as that leaves at least `step_rows_fit_min` prefill tokens. Steps of <= 128 rows run the
-    # weight-streaming decode GEMM (ops.STREAM_MAX_M); a 64-stream step that admits 100 new-turn tokens would
-    # otherwise take hipBLASLt at M = 164 (~172 vs ~128 us of GEMM per Llama-3-8B layer, profiles/wstream_sweep_r01.log,
-    # profiles/r02/gemm_sweep_M129_320.log). A new turn longer than the room is chunked over two steps.
+    # weight-streaming decode GEMM (ops.STREAM_MAX_M); a 64-stream step that admits 100 new-turn tokens
+    # takes the tile kernel (~136 us of GEMM per Llama-3-8B layer at 200 rows, ~89 at 64). A new turn longer than the room is chunked over two steps.
     step_rows_fit: int = 0
     step_rows_fit_min: int = 32
     # Burst splitting: new prefills admitted into one step may cost at most this many token-equivalents, a token at

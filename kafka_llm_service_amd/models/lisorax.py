@@ -234,8 +234,8 @@ class LisoraxLM:
 
     def enable_stream_weights(self, tiled_only: bool = False) -> int:
         """Wave-tiled copies of the projections (ops.tile_weight) so that decode-sized steps (<= ops.STREAM_MAX_M
-        rows) run them on the framework's weight-streaming MFMA GEMM; prefill-sized steps and shapes the kernel does
-        not take stay on hipBLASLt. bf16 only. Returns the added bytes."""
+        rows) run them on the framework's weight-streaming MFMA GEMM and longer ones on its tile kernel; shapes that they do
+        not take, biases and sizes that the library is as fast at stay on hipBLASLt. bf16 only. Returns the added bytes."""
         added = 0
         for lw in self.layers:
             for n in self.STREAMED:

@@ -243,8 +243,8 @@ class MozidraLM:
     def enable_stream_weights(self, tiled_only: bool = False) -> int:
         """Wave-tiled copies of the projections (ops.tile_weight) and of the experts (ops.tile_experts) so that
         decode-sized steps (<= ops.STREAM_MAX_M rows; experts: <= hops.MOE_STREAM_MAX_T) run them on the framework's
-        weight-streaming MFMA kernels; prefill-sized steps and shapes the kernels do not take stay on hipBLASLt and
-        the expert-sorted GEMMs. bf16 only. Returns the added bytes."""
+        weight-streaming MFMA kernels and longer ones on its tile kernel and the wide expert kernels; shapes that they do not take,
+        biases and sizes that the library is as fast at stay on hipBLASLt and the expert-sorted GEMMs. bf16 only. Returns the added bytes."""
         added = 0
         for lw in self.layers:
             for n in self.STREAMED:

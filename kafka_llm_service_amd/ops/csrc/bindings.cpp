@@ -942,7 +942,6 @@ static void slab_reduce(at::Tensor p, at::Tensor y) {
                                      cur_stream()));
 }
 
-// softmax -> top-k -> renormalise + stable expert sort (one kernel, no host sync)
 // an fp32 tensor that a routing launch clears: its 16-byte pieces, 0 where it has to be cleared by itself (and is, here)
 static int64_t clear_pieces(const c10::optional<at::Tensor>& zero, bool in_launch) {
   if (!zero.has_value()) return 0;
@@ -953,6 +952,7 @@ static int64_t clear_pieces(const c10::optional<at::Tensor>& zero, bool in_launc
   return 0;
 }
 
+// softmax -> top-k -> renormalise + stable expert sort (one kernel, no host sync)
 static void moe_route(at::Tensor logits, int64_t k, int64_t bm, at::Tensor topk_w, at::Tensor topk_e,
                       at::Tensor perm_tok, at::Tensor perm_w, at::Tensor expert_off, at::Tensor tile_off,
                       c10::optional<at::Tensor> zero) {

@@ -539,7 +539,6 @@ __device__ __forceinline__ float row16(float v, OP op) {
   return op(v, dpp<0x140>(v));
 }
 
-// up to 16 experts live in the first 16 lanes (the others run along): exchanges without LDS, 16 rows of 4096 12.2 -> 10.9 us
 // what a routing launch of up to NR_ROWS rows does beside: the stable sort of its choices by expert, and clearing the experts' sums
 struct RouteSort {
   int bits, bm;
@@ -549,7 +548,8 @@ struct RouteSort {
 };
 
 // softmax over all N experts, the k largest (ties: the lower index), their scores as weights (norm: divided by their sum)
-// times scale; lane = expert. SORT: one workgroup, with the sort (a launch of its own: 4.7 us of 16 rows) and, in further ones, the clearing
+// times scale; lane = expert: up to 16 live in the first 16 lanes (the others run along), exchanges without LDS, 16 rows of 4096 12.2 -> 10.9 us.
+// SORT: one workgroup, with the sort (a launch of its own: 4.7 us of 16 rows) and, in further ones, the clearing
 template <int TN, bool SORT>
 __global__ __launch_bounds__(64 * nr_waves(TN)) void narrow_route_kernel(const bf16* __restrict__ x, int64_t xs,
                                                            const bf16* __restrict__ wt, int N, int K, int k, bool norm,

@@ -4,9 +4,9 @@ y = x W^T via F.linear). Result (profiles/r02/tunableop_mixed_step_gemms_rejecte
 rocBLAS solutions nothing beats the library's default pick at these shapes (tuned = default within noise, several
 worse), so the engine does not load a tuning file.
 
-Mixed steps (64 decode rows + a new turn's prompt tokens, 129..256 rows padded to 16 k + 8 by
-``model_runner.pad_step_rows``) are ~20 % of the headline bench's steps and their four projections on hipBLASLt's
-default picks take ~167 us per layer (profiles/r02/kernel breakdown). For each shape this prints the default time,
+Mixed steps (64 decode rows + a new turn's prompt tokens, 129..256 rows; without tiled weights padded to 16 k + 8 by
+``model_runner.pad_step_rows``) are ~20 % of the headline bench's steps; their four projections on hipBLASLt's
+default picks took ~167 us per layer (profiles/r02/kernel breakdown). For each shape this prints the default time,
 tunes (all hipBLASLt + rocBLAS solutions, cold weights: copies rotated past the 256 MB MALL), and prints the tuned
 time. Usage: python scripts/tune_gemm.py --ms 168,184,200,216,232,248 --out <csv>
 """

@@ -48,6 +48,7 @@ class HostStep:
     prefill_splits: int = 0
     n_merge: int = 0        # prefill row ranges whose tiles were split: i32[-2 n_merge:] = (lo, hi) pairs
     prefix_joined: int = 0  # prefill tiles that ride in the cascade prefix pass (alt partials into prefill_part)
+    mixed: int = 0          # rows that one launch of the prefix items and the decode items merges (ops.attn_mixed), 0: two launches
     i64: np.ndarray | None = None
     i32: np.ndarray | None = None
     # (row, seq, position): decode inputs whose token was still being sampled at planning time, filled at launch
@@ -78,7 +79,7 @@ class SampleParams:
 
 
 _PLAN_SCALARS = ("B", "T", "nbt", "bt_w", "n_rows", "s_total", "n_dec_items", "n_prefix_items", "cascade_prefix",
-                 "n_items", "prefill_splits", "n_merge", "n_late", "late_off", "bt_need", "prefix_joined", "n_seg")
+                 "n_items", "prefill_splits", "n_merge", "n_late", "late_off", "bt_need", "prefix_joined", "n_seg", "mixed")
 PLAN_HDR = 32  # int64 header of a broadcast step plan
 PLAN_PAYLOAD_IDX = 1 + len(_PLAN_SCALARS) + 4  # header word holding the payload size (pack_plan)
 
@@ -187,6 +188,15 @@ def decode_round(n: int) -> int:
     return next((r for r in DECODE_ROUNDS if n <= r), 0)
 
 
+# One launch of prefix tiles and decode pieces (ops.attn_mixed): workgroups that its tiles and pieces share in proportion to their keys (a
+# tile's key takes as long as a piece's; 512 fit the chip at once), and those that its pieces are sized for. us of the launch, 18000 shared keys:
+# 64 rows of 1344 keys 96 tile workgroups 79, 128 68.3, 192 67.4, 256 72.6 with 1024 of pieces, 74.4 with 512, 70.2 with 1536; 222 rows (161 of
+# new turns) 224 tile workgroups 107, 336 95, 448 100, 672 104. Tiles of short launches get at least 5 / 4 of the mean share of a workgroup (30
+# rows of 1344 keys: 128 tile workgroups 46.5, 192 50, 256 50). Steps of four layers, us, two launches / one: 64 rows 823 / 769, with new turns
+# 1345 / 1262, 30 rows 662 / 642, 64 of 400 keys 700 / 688, 96 of 900 990 / 908, 16 of 2000 behind 3000 602 / 570, 2 - 8 rows 1 % less,
+# 64 rows and new turns of 800 3701 / 3211.
+MIXED_WGS, MIXED_PIECES = 560, 768
+MIXED_JOINED = 2048         # rows of new turns that such a launch takes along (their partials stay under 2 GiB)
 MAX_PARTIALS = 64           # partial slots per row that the decode kernel's fused merge reads (one lane each)
 MAX_PREFIX_CHUNKS = 32
 
@@ -338,11 +348,11 @@ def round_pieces(nb: np.ndarray, n: int, cap: np.ndarray) -> np.ndarray | None:
 
 
 def decode_items(seq_lens: np.ndarray, kv_start: np.ndarray, npre: np.ndarray, hkv: int,
-                 target: int = DECODE_TARGET_ITEMS, min_keys: int = MIN_DECODE_KEYS) -> np.ndarray:
+                 target: int = DECODE_TARGET_ITEMS, min_keys: int = MIN_DECODE_KEYS, rounds: bool = True) -> np.ndarray:
     """Work items (b, lo, hi, split, nsplit, npre, 0, 0) of the decode kernel: every row's keys [kv_start, len) in
     32-key-aligned pieces of about ``ch`` keys, ``ch`` chosen so the launch has ~``target`` workgroups (x Hkv) of
     about equal bytes (long histories are split, short ones stay whole); at most MAX_PARTIALS - npre pieces. Where that is more than
-    the round that the rows leave room in (``decode_round``), pieces for that round if they come out balanced (``round_pieces``)."""
+    the round that the rows leave room in (``decode_round``), pieces for that round if they come out balanced (``round_pieces``; not without ``rounds``)."""
     B = seq_lens.shape[0]
     suffix = np.maximum(seq_lens - kv_start, 1).astype(np.int64)
     # fewer rows than it takes to fill the GPU (B x Hkv < 512 workgroups): split so the launch still has ~512
@@ -356,7 +366,7 @@ def decode_items(seq_lens: np.ndarray, kv_start: np.ndarray, npre: np.ndarray, h
     ns = np.minimum(np.maximum(1, -(-suffix // ch)), MAX_PARTIALS - npre)
     bps = -(-nb // ns)
     ns = -(-nb // bps)  # no empty trailing piece
-    whole = decode_round(B * hkv) if target > 0 else 0
+    whole = decode_round(B * hkv) if target > 0 and rounds else 0
     if whole and int(ns.sum()) * hkv > whole:
         even = round_pieces(nb, whole // hkv, MAX_PARTIALS - npre)
         if even is not None:
@@ -548,6 +558,10 @@ class ModelRunner:
         # less HBM traffic per Llama-3-8B layer at 64 threads on an 18k prefix (+1.4 %,
         # profiles/r03/bench_ab_cascade_bf16_partials.jsonl)
         self.cascade_bf16 = self.variant == 3
+        # the prefix pass and the decode pieces in one launch, on tiles of 128 query rows
+        self.mixed_attn = self.variant == 3 and self.G in (1, 2, 4, 8) and model.D == 128 and \
+            os.environ.get("KAFKA_MIXED_ATTN", "1") == "1"
+        self.mixed_tile = 128 // self.G
         self.cascade_min_prefix = cascade_min_prefix
         self.target_wgs = target_wgs  # workgroups the prefill / cascade tile launches are balanced for
         self.prefill_kv_chunk = int(os.environ.get("KAFKA_PREFILL_KV_CHUNK", prefill_kv_chunk))
@@ -747,31 +761,39 @@ class ModelRunner:
         # system prompt every new turn of a thread re-attends): their tokens join the group's prefix pass — one read
         # of the prefix pages per step for all rows — and their own tiles attend only the keys behind the prefix
         joins = self._prefix_joins(bt, B, pre, groups, tiles) if groups and self.variant == 3 else {}
-        sfx_slots, sfx_rows = 0, []  # joined tiles whose own keys are planned into the prefix pass: slots, rows
+        sfx_slots, sfx_rows, sfx_parts = 0, [], []  # joined tiles whose own keys are planned into the prefix pass: slots, rows, parts
         if B:
             kv_start = np.zeros(B, dtype=np.int64)
             npre = np.zeros(B, dtype=np.int64)
             pit = []
             if groups:
+                mixed = self._mixed_plan(sum(tiles[ti][1] for js in joins.values() for ti in js))
+                tile = self.mixed_tile if mixed else self.tile
                 # joined tiles' own key spans (behind the prefix): with join_suffix they are items of this launch too
                 spans = {ti: tiles[ti][3] - groups[gi][1] * PAGE for gi, js in joins.items() for ti in js} \
                     if self.join_suffix else {}
                 # the joined rows' prefix-pass tiles: the group's joined tokens re-tiled at token granularity (a burst
                 # of short new turns fills 64-token tiles instead of one mostly empty tile per turn; every key of the
                 # prefix is below every joined token's position, so tokens of different turns share a tile)
-                jt = {gi: retile([tiles[ti][:2] for ti in js], self.tile if self.retile_joins else 0)
+                jt = {gi: retile([tiles[ti][:2] for ti in js], tile if self.retile_joins else 0)
                       for gi, js in joins.items()}
                 # key chunks sized so the prefix pass launches ~target_wgs workgroups over all groups together
-                work = sum(-(-n // self.tile) * p * PAGE for n, p in groups) + \
-                    sum(len(t) * groups[gi][1] * PAGE for gi, t in jt.items()) + sum(spans.values())
-                want = max(1, self.target_wgs // self.model.hkv)
-                chunk = min(MAX_ITEM_KEYS, max(256, -(-work // (want * 32)) * 32))
+                parts = {ti: -(-tiles[ti][1] // tile) for ti in spans}  # (row tiles of a joined tile's own keys)
+                work = sum(-(-n // tile) * p * PAGE for n, p in groups) + \
+                    sum(len(t) * groups[gi][1] * PAGE for gi, t in jt.items()) + sum(k * spans[ti] for ti, k in parts.items())
+                wgs, least = self.target_wgs, 256
+                if mixed:
+                    own = int(seq_lens.sum()) - sum(n * p * PAGE for n, p in groups)
+                    wgs = max(128, MIXED_WGS * work // max(1, work + own))
+                    least = max(256, min(1024, 5 * (work + own) * self.model.hkv // 2048))
+                want = max(1, wgs // self.model.hkv)
+                chunk = min(MAX_ITEM_KEYS, max(least, -(-work // (want * 32)) * 32))
                 # one round of workgroups: per-group rounding up can overshoot the target by a few items, and a
                 # second round of a handful of workgroups doubles the launch
-                tiles_per_group = [-(-n // self.tile) + len(jt.get(gi, ())) for gi, (n, _) in enumerate(groups)]
+                tiles_per_group = [-(-n // tile) + len(jt.get(gi, ())) for gi, (n, _) in enumerate(groups)]
                 while chunk < MAX_ITEM_KEYS and sum(t * -(-(p * PAGE) // chunk) for t, (_, p) in
                                                     zip(tiles_per_group, groups)) + \
-                        sum(-(-sp // chunk) for sp in spans.values()) > want:
+                        sum(k * -(-spans[ti] // chunk) for ti, k in parts.items()) > want:
                     chunk += 32
                 r0 = 0
                 for gi, (n, p) in enumerate(groups):
@@ -782,8 +804,8 @@ class ModelRunner:
                         ck = -(-P // (MAX_PREFIX_CHUNKS * 32)) * 32
                         nc = -(-P // ck)
                     for c in range(nc):  # chunk-major: the row tiles of one chunk run together (L2 sharing)
-                        for g0 in range(r0, r0 + n, self.tile):
-                            pit.append((g0, min(self.tile, r0 + n - g0), r0, c * ck, min(P, (c + 1) * ck), c, 0, 0))
+                        for g0 in range(r0, r0 + n, tile):
+                            pit.append((g0, min(tile, r0 + n - g0), r0, c * ck, min(P, (c + 1) * ck), c, 0, nc))
                         for q0, cnt in jt.get(gi, ()):  # joined prefill rows: q rows B + q0, fp32 alt partials
                             pit.append((B + q0, cnt, r0, c * ck, min(P, (c + 1) * ck), c, 1, 0))
                     for ti in joins.get(gi, ()):
@@ -796,18 +818,26 @@ class ModelRunner:
                             nsp = max(1, -(-spans[ti] // chunk))
                             ps = -(-spans[ti] // (nsp * 32)) * 32
                             nsp = -(-spans[ti] // ps)
-                            pit += [(B + q0, cnt, btr, P + c * ps, min(hi, P + (c + 1) * ps), nc + c, 1, 0)
-                                    for c in range(nsp)]
+                            pit += [(B + q0 + t0, min(tile, cnt - t0), btr, P + c * ps, min(hi, P + (c + 1) * ps), nc + c, 1, 0)
+                                    for c in range(nsp) for t0 in range(0, cnt, tile)]
                             sfx_slots = max(sfx_slots, nc + nsp)
                             sfx_rows.append((q0, q0 + cnt))
+                            sfx_parts.append(nc + nsp)
                     kv_start[r0:r0 + n] = P
                     npre[r0:r0 + n] = nc
                     h.cascade_prefix = max(h.cascade_prefix, P)
                     r0 += n
-            self._plan_decode_items(h, seq_lens, kv_start, npre, i32_parts)
+                h.mixed = B + max((hi for _, hi in sfx_rows), default=0) if mixed else 0
+            ditems = self._plan_decode_items(h, seq_lens, kv_start, npre, i32_parts)
             if pit:
                 h.n_prefix_items = len(pit)
                 i32_parts.append(np.asarray(pit, dtype=np.int32).reshape(-1))
+            if h.mixed:  # parts of every row that the launch merges, and above them how many of them are the prefix tiles'
+                row_parts = np.zeros(h.mixed, dtype=np.int32)
+                row_parts[ditems[:, 0]] = ditems[:, 4] + ditems[:, 5] + (ditems[:, 5] << 16)
+                for (lo, hi), n in zip(sfx_rows, sfx_parts):
+                    row_parts[B + lo:B + hi] = n
+                i32_parts.append(row_parts)
         if sfx_rows:  # (their suffix items are in the prefix pass)
             done = {ti for js in joins.values() for ti in js}
             tiles = [t for ti, t in enumerate(tiles) if ti not in done]
@@ -818,7 +848,7 @@ class ModelRunner:
                                                                  min(256, self.prefill_kv_chunk))
             if sfx_rows:
                 h.prefill_splits = max(h.prefill_splits, sfx_slots)
-                ranges = merge_ranges(ranges + sfx_rows)
+                ranges = merge_ranges(ranges + sfx_rows) if not h.mixed else ranges
             h.n_items = len(items)
             i32_parts.append(np.asarray(items, dtype=np.int32).reshape(-1))
             if ranges:
@@ -829,9 +859,14 @@ class ModelRunner:
         h.prefix_joined = sum(len(v) for v in joins.values())
         h.stats = {"B": B, "T": T, "cascade_prefix": h.cascade_prefix, "cascade_groups": len(groups),
                    "prefix_joined_tiles": h.prefix_joined,
-                   "decode_items": h.n_dec_items, "prefix_items": h.n_prefix_items, "s_total": h.s_total,
+                   "decode_items": h.n_dec_items, "prefix_items": h.n_prefix_items, "mixed": h.mixed, "s_total": h.s_total,
                    "prefill_splits": h.prefill_splits, "prefill_items": h.n_items}
         return h, sample_seqs
+
+    def _mixed_plan(self, joined: int) -> bool:
+        """Whether a step's prefix tiles and decode pieces go out as one launch (ops.attn_mixed), with ``joined`` rows of new turns."""
+        return self.mixed_attn and self.cascade_bf16 and self.graphs is None and not self.fixed_decode_items and \
+            (joined == 0 or self.retile_joins and self.join_suffix and joined <= MIXED_JOINED)
 
     @staticmethod
     def _prefix_joins(bt: np.ndarray, B: int, pre: list, groups: list[tuple[int, int]],
@@ -857,12 +892,14 @@ class ModelRunner:
         return joins
 
     def _plan_decode_items(self, h: HostStep, seq_lens: np.ndarray, kv_start: np.ndarray, npre: np.ndarray,
-                           i32_parts: list) -> None:
+                           i32_parts: list) -> np.ndarray:
         if self.graphs is not None or self.fixed_decode_items:  # graph replay: the decode grid depends on B alone
             # (one round where it has three pieces a row: rows of any lengths are balanced then. us of the attention, 1344 workgroups / one
             # round: 16 rows of 1344 keys 25.1 / 19.9, one of them eight times as long 36.3 / 27.8, 32 rows of 4500 102 / 96, 122 / 116)
             ditems = decode_items_fixed(seq_lens, kv_start, npre, self.model.hkv,
                                         decode_round(3 * len(seq_lens) * self.model.hkv) or DECODE_TARGET_ITEMS)
+        elif h.mixed:
+            ditems = decode_items(seq_lens, kv_start, npre, self.model.hkv, MIXED_PIECES, rounds=False)
         else:
             ditems = decode_items(seq_lens, kv_start, npre, self.model.hkv)
         h.n_dec_items = int(ditems.shape[0])
@@ -873,6 +910,7 @@ class ModelRunner:
             # partial buffers' unused slots are never touched)
             h.s_total = min(MAX_PARTIALS, -(-h.s_total // 8) * 8)
         i32_parts.append(ditems.reshape(-1))
+        return ditems
 
     def to_device(self, h: HostStep, sp: "SampleParams | None" = None) -> StepInput:
         """One H2D copy of the packed buffers (and of the step's sampling parameters when ``sp`` samples with
@@ -922,13 +960,16 @@ class ModelRunner:
             if h.n_prefix_items:
                 meta.prefix_items = d32[o:o + h.n_prefix_items * 8].view(-1, 8)
                 o += h.n_prefix_items * 8
+            if h.mixed:
+                meta.row_parts = d32[o:o + h.mixed]
+                o += h.mixed
             meta.s_total = h.s_total
             meta.part = torch.empty(B, Hq, h.s_total, D, dtype=torch.float32, device=self.device)
             meta.lse = torch.empty(B, Hq, h.s_total, dtype=torch.float32, device=self.device)
             if h.n_prefix_items and self.cascade_bf16:
                 meta.pre_part = torch.empty(B, Hq, h.s_total, D, dtype=torch.bfloat16, device=self.device)
             meta.extra["cascade_prefix"] = h.cascade_prefix
-        if h.n_items or h.n_merge:
+        if h.n_items or h.n_merge or h.prefill_splits:
             if h.n_items:
                 meta.prefill_items = d32[o:o + h.n_items * 8].view(-1, 8)
                 o += h.n_items * 8

@@ -52,6 +52,7 @@ class AttnMeta:
     prefill_part: torch.Tensor | None = None
     prefill_lse: torch.Tensor | None = None
     prefill_merge: list = field(default_factory=list)  # (lo, hi) prefill row ranges of split tiles
+    row_parts: torch.Tensor | None = None      # int32: prefix_items and decode_items are one launch's (ops.attn_mixed), parts by row
     prefix_joined: bool = False                # prefill rows take part in the cascade prefix pass (alt partials)
     scale: float = 1.0
     variant: int = 0                           # tile-kernel variant (ops.tile_rows): 0 = 8 waves / 256 rows
@@ -73,7 +74,13 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                     out: torch.Tensor) -> None:
     """q [T, Hq, D] (post-RoPE) -> out [T, Hq, D] bf16."""
     B = meta.num_decode
-    if B > 0:
+    if B > 0 and meta.row_parts is not None:
+        # prefix items and decode items (and the new turns' rows that they cover) in one launch
+        n = meta.row_parts.numel()
+        ops.attn_mixed(meta.prefix_items, meta.decode_items, q[:n], k_cache, v_cache, meta.block_tables, meta.q_limit, meta.part,
+                       meta.lse, meta.pre_part, meta.row_parts, meta.scale, out[:n],
+                       *((meta.prefill_part, meta.prefill_lse) if n > B else ()))
+    elif B > 0:
         qd = q[:B]
         if meta.prefix_items is not None:
             # new-turn prefill rows that share the prefix ride along (items flagged alt: fp32 partials in their own

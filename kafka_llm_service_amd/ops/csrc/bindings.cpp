@@ -35,6 +35,11 @@ hipError_t kafka_launch_attn_decode(const bf16* q, int64_t q_stride, const void*
                                     bf16* out, int64_t out_stride, int* tickets, const bf16* pre_bf16,
                                     const float* m_part, const float* m_lse, int m_S, int m_rows, bf16* m_out,
                                     int64_t m_out_stride, hipStream_t st);
+hipError_t kafka_launch_attn_mixed(const int* titems, int n_tiles, const int* ditems, int n_pieces, const int* row_parts,
+                                   int n_rows, const bf16* q, int64_t q_stride, const void* k_cache, const void* v_cache, int Hkv, int G,
+                                   const int* block_tables, int bt_stride, const int* q_limit, int B, float* part, float* lse,
+                                   bf16* pre, int S_total, float scale, bf16* out, int64_t out_stride, int* counters,
+                                   float* alt_part, float* alt_lse, int alt_S, int alt_tok_off, hipStream_t st);
 hipError_t kafka_launch_attn_prefill(const void* items, int n_items, const bf16* q, int64_t q_stride,
                                      const void* k_cache, const void* v_cache, int fp8, int Hkv, int G, int D,
                                      const int* block_tables, int bt_stride, const int* q_limit, bf16* out,
@@ -389,6 +394,56 @@ static void attn_decode(at::Tensor q, at::Tensor k_cache, at::Tensor v_cache, at
                                       items.data_ptr<int>(), out_part.data_ptr<float>(), lse_part.data_ptr<float>(),
                                       S_total, scale, op, ostride, tp, pre, mp, ml, mS, mrows, mo, mstride,
                                       cur_stream()));
+}
+
+// prefix tiles and decode pieces of a step in one launch (attn_mixed.hip): q [T, Hq, 128], rows [0, B) of it (part's) the
+// decode rows; out and row_parts: the rows that it merges
+static void attn_mixed(at::Tensor prefix_items, at::Tensor decode_items, at::Tensor q, at::Tensor k_cache, at::Tensor v_cache,
+                       at::Tensor block_tables, at::Tensor q_limit, at::Tensor part, at::Tensor lse, at::Tensor pre,
+                       at::Tensor row_parts, double scale, at::Tensor out, at::Tensor counters, c10::optional<at::Tensor> alt_part, c10::optional<at::Tensor> alt_lse,
+                       int64_t alt_tok_off) {
+  CHECK_CUDA(q); CHECK_DT(q, at::kBFloat16); check_cache_pair(k_cache, v_cache);
+  CHECK_DT(block_tables, at::kInt); CHECK_DT(part, at::kFloat); CHECK_DT(lse, at::kFloat); CHECK_DT(pre, at::kBFloat16);
+  CHECK_DT(out, at::kBFloat16); CHECK_DT(q_limit, at::kInt);
+  TORCH_CHECK(!is_fp8_cache(k_cache), "attn_mixed reads bf16 pages only");
+  TORCH_CHECK(q.dim() == 3 && q.stride(2) == 1 && q.stride(1) == 128 && q.size(2) == 128, "q must be [T, Hq, 128]");
+  const int T = q.size(0), Hq = q.size(1), Hkv = k_cache.size(1), R = out.size(0), B = part.size(0);
+  TORCH_CHECK(Hq % Hkv == 0 && Hq / Hkv <= 8 && 128 % (Hq / Hkv) == 0, "attn_mixed needs Hq/Hkv of 1, 2, 4 or 8");
+  for (const auto* it : {&prefix_items, &decode_items})
+    TORCH_CHECK(it->is_cuda() && it->scalar_type() == at::kInt && it->is_contiguous() && it->dim() == 2 && it->size(1) == 8,
+                "attn_mixed: items must be device int32 [n, 8]");
+  TORCH_CHECK(row_parts.is_cuda() && row_parts.scalar_type() == at::kInt && row_parts.is_contiguous() && row_parts.numel() == R && R >= B,
+              "attn_mixed: row_parts must be a device int32 [rows of out]");
+  TORCH_CHECK(T >= R && q_limit.is_contiguous() && q_limit.numel() >= T, "attn_mixed: q_limit");
+  TORCH_CHECK(block_tables.dim() == 2 && block_tables.size(0) >= B && block_tables.stride(1) == 1, "block_tables");
+  TORCH_CHECK(part.is_contiguous() && part.dim() == 4 && part.size(1) == Hq && part.size(3) == 128 &&
+                  part.numel() * 4 < 0x7fffffffLL, "attn_mixed: part must be [B, Hq, S, 128] of less than 2 GiB");
+  TORCH_CHECK(pre.is_contiguous() && pre.sizes() == part.sizes(), "attn_mixed: pre must have part's shape");
+  const int S = part.size(2);
+  TORCH_CHECK(lse.is_contiguous() && lse.numel() >= part.size(0) * Hq * S, "attn_mixed: lse");
+  TORCH_CHECK(out.dim() == 3 && out.size(1) == Hq && out.size(2) == 128 && out.stride(2) == 1 && out.stride(1) == 128 &&
+                  out.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0, "attn_mixed: out must be [B, Hq, 128]");
+  TORCH_CHECK(counters.is_cuda() && counters.scalar_type() == at::kInt && counters.is_contiguous() &&
+                  counters.numel() >= (int64_t)R * Hkv, "attn_mixed: counters must be int32, >= rows * Hkv zeros");
+  float *ap = nullptr, *al = nullptr;
+  int S2 = 0;
+  TORCH_CHECK(R == B || alt_part.has_value(), "attn_mixed: rows past part's need alt partials");
+  if (alt_part.has_value()) {
+    TORCH_CHECK(alt_lse.has_value(), "attn_mixed: alt partials need alt_lse");
+    CHECK_DT(alt_part.value(), at::kFloat); CHECK_DT(alt_lse.value(), at::kFloat);
+    TORCH_CHECK(alt_part->is_contiguous() && alt_part->dim() == 4 && alt_part->size(1) == Hq && alt_part->size(3) == 128 &&
+                    alt_tok_off == B && alt_part->size(0) + B >= R &&
+                    alt_part->numel() * 4 < 0x7fffffffLL, "attn_mixed: alt_part must be [>= rows - B, Hq, S, 128] of less than 2 GiB");
+    S2 = alt_part->size(2);
+    TORCH_CHECK(alt_lse->is_contiguous() && alt_lse->numel() >= alt_part->size(0) * Hq * S2, "attn_mixed: alt_lse");
+    ap = alt_part->data_ptr<float>();
+    al = alt_lse->data_ptr<float>();
+  }
+  CHECK_HIP(kafka_launch_attn_mixed(prefix_items.data_ptr<int>(), prefix_items.size(0), decode_items.data_ptr<int>(),
+                                     decode_items.size(0), row_parts.data_ptr<int>(), R, bptr(q), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), Hkv, Hq / Hkv,
+                                     block_tables.data_ptr<int>(), block_tables.stride(0), q_limit.data_ptr<int>(), B,
+                                     part.data_ptr<float>(), lse.data_ptr<float>(), bptr(pre), S, scale, bptr(out), out.stride(0),
+                                     counters.data_ptr<int>(), ap, al, S2, (int)alt_tok_off, cur_stream()));
 }
 
 static void attn_prefill(at::Tensor items, at::Tensor q, at::Tensor k_cache, at::Tensor v_cache,
@@ -1268,6 +1323,10 @@ PYBIND11_MODULE(_kafka_ops, m) {
         py::arg("items"), py::arg("out_part"), py::arg("lse_part"), py::arg("scale"), py::arg("out"),
         py::arg("tickets"), py::arg("pre_part") = py::none(), py::arg("m_part") = py::none(),
         py::arg("m_lse") = py::none(), py::arg("m_out") = py::none());
+  m.def("attn_mixed", &attn_mixed, py::arg("prefix_items"), py::arg("decode_items"), py::arg("q"), py::arg("k_cache"),
+        py::arg("v_cache"), py::arg("block_tables"), py::arg("q_limit"), py::arg("part"), py::arg("lse"), py::arg("pre"),
+        py::arg("row_parts"), py::arg("scale"), py::arg("out"), py::arg("counters"), py::arg("alt_part") = py::none(), py::arg("alt_lse") = py::none(),
+        py::arg("alt_tok_off") = 0);
   m.def("attn_prefill", &attn_prefill, py::arg("items"), py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
         py::arg("block_tables"), py::arg("q_limit"), py::arg("out"), py::arg("out_part"), py::arg("lse_part"),
         py::arg("scale"), py::arg("variant") = 0, py::arg("alt_part") = py::none(), py::arg("alt_lse") = py::none(),

@@ -1,0 +1,179 @@
+"""Prefix tiles and decode pieces in one launch (``ops.attn_mixed``): rows against fp32 attention over their whole context, and the
+engine's plans for it."""
+import math
+import os
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+from kafka_llm_service_amd import ops
+from kafka_llm_service_amd.engine.model_runner import decode_items
+from kafka_llm_service_amd.ops import reference as ref
+
+sys.path.insert(0, os.path.dirname(__file__))
+
+
+def _case(groups, own, hkv, G, seed, dev, loose=0, alt=0):
+    """Rows of ``groups`` ((rows, prefix pages, prefix parts) each), then ``loose`` rows without one; ``own`` keys behind the
+    prefix per row, in order; ``alt`` new tokens behind the first group's prefix."""
+    g = torch.Generator().manual_seed(seed)
+    B = sum(n for n, _, _ in groups) + loose
+    pages = sum(p for _, p, _ in groups) + sum(-(-n // 16) for n in own) + 4 + alt // 16
+    W = max([p for _, p, _ in groups] + [0]) + max(-(-n // 16) for n in own) + 4 + alt // 16
+    perm = torch.randperm(pages, generator=g).tolist()
+    bt = torch.zeros(B + 1, W, dtype=torch.int32)
+    kv0, npre, items, at, r0 = np.zeros(B, np.int64), np.zeros(B, np.int64), [], 0, 0
+    tile = 128 // G
+    for gi, (n, p, nc) in enumerate(groups):
+        shared = perm[at:at + p]
+        at += p
+        ck = -(-p * 16 // (nc * 32)) * 32
+        nc = -(-p * 16 // ck)
+        for c in range(nc):
+            rows = [(r, min(tile, r0 + n - r), 0) for r in range(r0, r0 + n, tile)]
+            if gi == 0:
+                rows += [(B + t, min(tile, alt - t), 1) for t in range(0, alt, tile)]
+            items += [(r, k, r0, c * ck, min(p * 16, (c + 1) * ck), c, a, nc) for r, k, a in rows]
+        for r in list(range(r0, r0 + n)) + ([B] if gi == 0 else []):
+            bt[r, :p] = torch.tensor(shared, dtype=torch.int32)
+        kv0[r0:r0 + n], npre[r0:r0 + n] = p * 16, nc
+        r0 += n
+    for b in range(B):
+        p, k = int(kv0[b]) // 16, -(-own[b] // 16)
+        bt[b, p:p + k] = torch.tensor(perm[at:at + k], dtype=torch.int32)
+        at += k
+    k = torch.randn(pages, hkv, 16, 128, generator=g).to(torch.bfloat16)
+    v = torch.randn(pages, hkv, 128, 16, generator=g).to(torch.bfloat16)
+    q = torch.randn(B + alt, hkv * G, 128, generator=g).to(torch.bfloat16)
+    lens = kv0 + np.asarray(own)
+    lim = torch.tensor(list(lens - 1) + [int(groups[0][1]) * 16 + 5] * alt, dtype=torch.int32)
+    return dict(B=B, q=q.to(dev), k=k.to(dev), v=v.to(dev), bt=bt.to(dev), lens=lens, kv0=kv0, npre=npre, lim=lim.to(dev),
+                items=torch.tensor(items, dtype=torch.int32).reshape(-1, 8).to(dev))
+
+
+def _run(c, target=1344, dec=None):
+    dev, B, Hq = c["q"].device, c["B"], c["q"].shape[1]
+    if dec is None:
+        dec = decode_items(c["lens"], c["kv0"], c["npre"], c["k"].shape[1], target)
+    S = int((dec[:, 4] + dec[:, 5]).max())
+    part = torch.full((B, Hq, S, 128), float("nan"), device=dev)
+    lse = torch.full((B, Hq, S), float("nan"), device=dev)
+    pre = torch.full((B, Hq, S, 128), float("nan"), device=dev, dtype=torch.bfloat16)
+    T = c["q"].shape[0]
+    out = torch.full((T, Hq, 128), float("nan"), device=dev, dtype=torch.bfloat16)
+    parts = torch.zeros(T, dtype=torch.int32)
+    for b, _, _, _, n, npre, _, _ in dec.tolist():
+        parts[b] = n + npre | npre << 16
+    parts[B:] = int(c["npre"][0])
+    alt = (torch.zeros(T - B, Hq, S, 128, device=dev), torch.full((T - B, Hq, S), float("-inf"), device=dev)) if T > B else ()
+    ops.attn_mixed(c["items"], torch.tensor(dec, device=dev), c["q"], c["k"], c["v"], c["bt"], c["lim"], part, lse, pre, parts.to(dev),
+                   128 ** -0.5, out, *alt)
+    return out
+
+
+def _whole(c, b, n):
+    """fp32 attention of row b over its first n keys."""
+    hkv = c["k"].shape[1]
+    kk, vv = ref.gather_kv(c["k"].cpu(), c["v"].cpu(), c["bt"][min(b, c["B"])].cpu(), n)
+    q = c["q"][b].float().cpu().view(hkv, -1, 128)
+    s = torch.einsum("hgd,nhd->hgn", q, kk.float()) / math.sqrt(128)
+    return torch.einsum("hgn,nhd->hgd", s.softmax(-1), vv.float()).reshape(-1, 128)
+
+
+def _check(c, out):
+    # bf16 probabilities, prefix partials and rows: each 2^-9 of values of about sqrt(1/n), so 3 * 2^-9 of the largest; taken twice
+    tol = 6 * 2.0 ** -9
+    for b in list(range(c["B"])) + [r for r in (c["B"], c["B"] + 37, out.shape[0] - 1) if c["B"] <= r < out.shape[0]]:
+        want = _whole(c, b, int(c["lens"][b] if b < c["B"] else c["kv0"][0]))
+        assert (out[b].float().cpu() - want).abs().max() <= tol * max(1e-3, want.abs().max()), b
+
+
+#: (groups, own keys by row, kv heads, G, loose rows, new tokens): whole and ragged row tiles, one row of a tile, one prefix part,
+#: several groups, rows without a group, pieces of one row, every G
+CASES = [([(5, 40, 3)], [1, 17, 33, 500, 64], 2, 4, 0, 0), ([(33, 34, 2)], [20 + 7 * i for i in range(33)], 2, 4, 0, 0),
+         ([(2, 32, 1), (3, 64, 4)], [300, 5, 31, 32, 1200], 2, 8, 0, 0), ([(2, 40, 5)], [600, 40, 900, 16], 1, 2, 2, 0),
+         ([(3, 48, 2)], [90, 1, 700], 3, 1, 0, 0), ([(4, 130, 32)], [50, 9000, 3, 77], 2, 4, 0, 70)]
+
+
+@pytest.mark.parametrize("groups,own,hkv,G,loose,alt", CASES)
+def test_rows_equal_whole_attention_cpu(groups, own, hkv, G, loose, alt):
+    c = _case(groups, own, hkv, G, 3, "cpu", loose, alt)
+    _check(c, _run(c))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("groups,own,hkv,G,loose,alt", CASES + [([(64, 70, 8)], [40 + 11 * i for i in range(64)], 8, 4, 0, 130)])
+def test_rows_equal_whole_attention(cuda, groups, own, hkv, G, loose, alt):
+    """... and again: the counters are back at zero; pieces of other lengths (many of a row, one of each)."""
+    c = _case(groups, own, hkv, G, 3, cuda, loose, alt)
+    _check(c, _run(c))
+    for target in (1344, 1344, 64, 8):
+        _check(c, _run(c, target))
+    stream = torch.cuda.current_stream(cuda).cuda_stream
+    assert not ops._TICKETS[(c["q"].device, f"mixed {stream}")].any()
+
+
+@pytest.mark.gpu
+def test_keys_that_are_no_numbers_reach_their_rows_only(cuda):
+    c = _case([(6, 40, 3)], [50, 60, 700, 80, 90, 100], 2, 4, 5, cuda)
+    want = _run(c)
+    c["k"][c["bt"][2, 41]] = float("nan")          # a page of row 2's own keys
+    out = _run(c)
+    rest = [0, 1, 3, 4, 5]
+    assert torch.equal(out[rest], want[rest])
+    c["v"][c["bt"][0, 3]] = float("nan")           # a page that all share
+    out = _run(c)
+    assert out.isnan().any(-1).all()
+
+
+def test_plans_of_a_cascade_step_cover_every_key_once():
+    """The engine's plan for one launch: every key of every row in exactly one tile or piece, at most 128 query rows a tile, and a
+    prefix tile names as many parts as its rows' pieces do."""
+    from kafka_llm_service_amd.engine.engine import EngineConfig, LLMEngine
+    from kafka_llm_service_amd.engine.sequence import SamplingParams, Sequence
+
+    eng = LLMEngine(EngineConfig(model="tiny-llama", device="cpu", num_kv_blocks=700, max_num_seqs=48, max_model_len=2400))
+    r = eng.runner
+    if not r.mixed_attn:                           # (the small preset's head size: the plan alone)
+        r.mixed_attn, r.mixed_tile = True, 128 // r.G
+    shared = list(range(1, 1 + 64 * 16))
+    seqs = [Sequence(f"r{i}", shared + [5 + i] * (3 + 29 * i % 400), SamplingParams(max_tokens=4)) for i in range(41)]
+    first = Sequence("shared", list(shared), SamplingParams(max_tokens=1))
+    for s in [first] + seqs:                       # (the pages that the rest of them share)
+        batch = eng.sched.replay([(s, s.total_len)])
+        for x, _, b in batch.prefill:
+            x.num_computed = b
+            eng.kvm.commit(x.seq_id, b)
+        for x in batch.decode:
+            x.num_computed = x.total_len
+    for s in seqs:
+        s.prompt_ids.append(7)
+        eng.kvm.append_tokens(s.seq_id, [7])
+    new = seqs[-1]
+    for t in range(90):
+        new.prompt_ids.append(9)
+    eng.kvm.append_tokens(new.seq_id, [9] * 90)
+    host, _ = r.build_host(eng.sched.replay([(s, s.total_len - s.num_computed) for s in seqs]))
+    assert host.mixed and host.n_prefix_items and host.B == 40 and host.prefix_joined
+    o = host.nbt * host.bt_w + host.T
+    dec = host.i32[o:o + 8 * host.n_dec_items].reshape(-1, 8)
+    pre = host.i32[o + 8 * host.n_dec_items:][:8 * host.n_prefix_items].reshape(-1, 8)
+    assert (pre[:, 1] * r.G <= 128).all()
+    seen = {b: [] for b in range(host.T)}
+    for b, lo, hi, split, n, npre, _, _ in dec:
+        seen[b].append((lo, hi, npre + split))
+        assert all(t[7] == npre for t in pre if t[0] <= b < t[0] + t[1] and not t[6])
+    for q0, cnt, _, lo, hi, split, alt, _ in pre:
+        for t in range(q0, q0 + cnt):
+            seen[t].append((lo, hi, split))
+            assert bool(alt) == (t >= host.B)
+    limit = host.i32[host.nbt * host.bt_w:][:host.T]
+    parts = host.i32[o + 8 * (host.n_dec_items + host.n_prefix_items):][:host.mixed]
+    assert host.mixed == host.T and not host.n_merge and host.prefill_splits
+    for b, spans in seen.items():
+        spans.sort()
+        assert [a[0] for a in spans] == [0] + [a[1] for a in spans[:-1]] and spans[-1][1] > limit[b]
+        assert {a[2] for a in spans} == set(range(len(spans))) and parts[b] & 0xffff == len(spans)
+        assert parts[b] >> 16 == (sum(a[1] <= 1024 for a in spans) if b < host.B else 0)

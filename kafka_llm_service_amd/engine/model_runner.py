@@ -188,15 +188,26 @@ def decode_round(n: int) -> int:
     return next((r for r in DECODE_ROUNDS if n <= r), 0)
 
 
-# One launch of prefix tiles and decode pieces (ops.attn_mixed): workgroups that its tiles and pieces share in proportion to their keys (a
-# tile's key takes as long as a piece's; 512 fit the chip at once), and those that its pieces are sized for. us of the launch, 18000 shared keys:
-# 64 rows of 1344 keys 96 tile workgroups 79, 128 68.3, 192 67.4, 256 72.6 with 1024 of pieces, 74.4 with 512, 70.2 with 1536; 222 rows (161 of
-# new turns) 224 tile workgroups 107, 336 95, 448 100, 672 104. Tiles of short launches get at least 5 / 4 of the mean share of a workgroup (30
-# rows of 1344 keys: 128 tile workgroups 46.5, 192 50, 256 50). Steps of four layers, us, two launches / one: 64 rows 823 / 769, with new turns
-# 1345 / 1262, 30 rows 662 / 642, 64 of 400 keys 700 / 688, 96 of 900 990 / 908, 16 of 2000 behind 3000 602 / 570, 2 - 8 rows 1 % less,
-# 64 rows and new turns of 800 3701 / 3211.
-MIXED_WGS, MIXED_PIECES = 560, 768
+# One launch of prefix tiles and decode pieces (ops.attn_mixed): workgroups that its pieces are sized for.
+MIXED_PIECES = 768
 MIXED_JOINED = 2048         # rows of new turns that such a launch takes along (their partials stay under 2 GiB)
+MIXED_FEW = 6               # prefix keys of its tiles beside a row's own, past which the two launches of before stay (one round of them)
+
+
+def mixed_tile_wgs(work: int, own: int, tiles: int, hkv: int) -> int:
+    """Workgroups of the prefix tiles of such a launch: ``work`` keys of ``tiles`` row tiles (of each of ``hkv`` heads) beside ``own`` keys of
+    decode pieces. A tile a CU where the tiles have more to do than the pieces, three for four CUs where the pieces have (us, 18000 shared keys,
+    tile workgroups 128 / 192 / 256 / 384: 64 rows of 1344 keys 68 / 67 / 72 / 77, 96 of 900 76 / 75 / 79 / 85, of 700 60 / 52 / 51 / 58, of 400
+    57 / 47 / 45 / 49); two a CU where the pieces hardly matter (61 rows of 100 with 161 new turns' 256 / 512: 97 / 85; of 1344 110 / 128), or
+    where one a CU would leave up to half of them idle (461 rows: 240 / 480 197 / 178); whole rounds where the row tiles alone are more
+    than a CU each (a step of 5 rows and 1094 of new turns 288 / 864: 3810 / 3468)."""
+    if work < own:
+        return 192
+    if tiles * hkv > 128:
+        return 512 if tiles * hkv <= 256 else 1024
+    return 512 if 2 * work > 7 * own and work * hkv > 2000 * 256 else 256
+
+
 MAX_PARTIALS = 64           # partial slots per row that the decode kernel's fused merge reads (one lane each)
 MAX_PREFIX_CHUNKS = 32
 
@@ -767,7 +778,7 @@ class ModelRunner:
             npre = np.zeros(B, dtype=np.int64)
             pit = []
             if groups:
-                mixed = self._mixed_plan(sum(tiles[ti][1] for js in joins.values() for ti in js))
+                mixed = self._mixed_plan(seq_lens, groups, sum(tiles[ti][1] for js in joins.values() for ti in js))
                 tile = self.mixed_tile if mixed else self.tile
                 # joined tiles' own key spans (behind the prefix): with join_suffix they are items of this launch too
                 spans = {ti: tiles[ti][3] - groups[gi][1] * PAGE for gi, js in joins.items() for ti in js} \
@@ -779,21 +790,22 @@ class ModelRunner:
                       for gi, js in joins.items()}
                 # key chunks sized so the prefix pass launches ~target_wgs workgroups over all groups together
                 parts = {ti: -(-tiles[ti][1] // tile) for ti in spans}  # (row tiles of a joined tile's own keys)
+                # (beside decode pieces the joined rows' own keys do not count: short items, done long before the prefix tiles)
+                sized = {} if mixed else parts
                 work = sum(-(-n // tile) * p * PAGE for n, p in groups) + \
-                    sum(len(t) * groups[gi][1] * PAGE for gi, t in jt.items()) + sum(k * spans[ti] for ti, k in parts.items())
-                wgs, least = self.target_wgs, 256
+                    sum(len(t) * groups[gi][1] * PAGE for gi, t in jt.items()) + sum(k * spans[ti] for ti, k in sized.items())
+                tiles_per_group = [-(-n // tile) + len(jt.get(gi, ())) for gi, (n, _) in enumerate(groups)]
+                wgs = self.target_wgs
                 if mixed:
                     own = int(seq_lens.sum()) - sum(n * p * PAGE for n, p in groups)
-                    wgs = max(128, MIXED_WGS * work // max(1, work + own))
-                    least = max(256, min(1024, 5 * (work + own) * self.model.hkv // 2048))
+                    wgs = mixed_tile_wgs(work, own, sum(tiles_per_group), self.model.hkv)
                 want = max(1, wgs // self.model.hkv)
-                chunk = min(MAX_ITEM_KEYS, max(least, -(-work // (want * 32)) * 32))
+                chunk = min(MAX_ITEM_KEYS, max(256, -(-work // (want * 32)) * 32))
                 # one round of workgroups: per-group rounding up can overshoot the target by a few items, and a
                 # second round of a handful of workgroups doubles the launch
-                tiles_per_group = [-(-n // tile) + len(jt.get(gi, ())) for gi, (n, _) in enumerate(groups)]
                 while chunk < MAX_ITEM_KEYS and sum(t * -(-(p * PAGE) // chunk) for t, (_, p) in
                                                     zip(tiles_per_group, groups)) + \
-                        sum(k * -(-spans[ti] // chunk) for ti, k in parts.items()) > want:
+                        sum(k * -(-spans[ti] // chunk) for ti, k in sized.items()) > want:
                     chunk += 32
                 r0 = 0
                 for gi, (n, p) in enumerate(groups):
@@ -863,10 +875,18 @@ class ModelRunner:
                    "prefill_splits": h.prefill_splits, "prefill_items": h.n_items}
         return h, sample_seqs
 
-    def _mixed_plan(self, joined: int) -> bool:
-        """Whether a step's prefix tiles and decode pieces go out as one launch (ops.attn_mixed), with ``joined`` rows of new turns."""
-        return self.mixed_attn and self.cascade_bf16 and self.graphs is None and not self.fixed_decode_items and \
-            (joined == 0 or self.retile_joins and self.join_suffix and joined <= MIXED_JOINED)
+    def _mixed_plan(self, seq_lens: np.ndarray, groups: list[tuple[int, int]], joined: int) -> bool:
+        """Whether a step's prefix tiles and decode pieces go out as one launch (ops.attn_mixed), with ``joined`` rows of new turns. us of a
+        layer's attention, two launches / one (18000 shared keys): 64 rows of 1344 keys 84 / 67, 96 of 900 99 / 75, 128 of 300 83 / 63, 30 of 1344
+        53 / 47, 61 of 1344 and 161 rows of new turns 135 / 110, 64 of 300 behind 3000 35 / 25, 20 of 300 33.5 / 32, 8 of 1000 behind
+        9000 27 / 26.5; the tiles alone are as fast in one launch of 256 rows each: 64 of 100 36.6 / 37.9, 40 of 60 33 / 37."""
+        if not (self.mixed_attn and self.cascade_bf16 and self.graphs is None and not self.fixed_decode_items):
+            return False
+        if joined:
+            return self.retile_joins and self.join_suffix and joined <= MIXED_JOINED
+        work = sum(-(-n // self.mixed_tile) * p * PAGE for n, p in groups)
+        own = int(seq_lens.sum()) - sum(n * p * PAGE for n, p in groups)
+        return work <= MIXED_FEW * own or work * self.model.hkv > 300000
 
     @staticmethod
     def _prefix_joins(bt: np.ndarray, B: int, pre: list, groups: list[tuple[int, int]],

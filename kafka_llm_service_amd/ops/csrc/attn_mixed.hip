@@ -13,7 +13,7 @@
 // of heads to merge alone, 20 - 40 us; 64 rows of 1344 keys 82 -> 85 us, 30 rows 54 -> 77.)
 //
 // us of a layer's attention, tile and decode launch / this one (Llama-3-8B heads, 18000 shared keys; caches not resident): 64 rows of 1344
-// keys 83 / 67, 96 of 900 99 / 73, 30 of 1344 55 / 46, 64 of 400 50 / 43, 64 of 5000 210 / 186. The first moves 370 MB: 5.5 TB/s, where the
+// keys 84 / 67, 96 of 900 99 / 75, 30 of 1344 53 / 47, 64 of 400 48 / 45, 64 of 5000 210 / 186. The first moves 370 MB: 5.5 TB/s, where the
 // decode kernel alone reaches 6.4; the rest is the merges at its end (5 us) and tiles that go on beside the last pieces.
 #include "attn_decode.h"
 #include "attn_tile.h"

@@ -401,10 +401,25 @@ def linear_small(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 # ---- dense products of long steps on wave-tiled weights (csrc/tile_gemm.hip) -------------------------------------------
 # (16-row parts, 16-column parts) of a wave's tile, 2 x 2 waves a workgroup -> us: of a launch, of a round of 256 workgroups, of 64 of K
-# in it, and of a MB/us of what is written, over 4.5. Fitted to 6200 timings (19 shapes of width 2048 and 4096, 136 - 4099 rows,
-# every tile, one to eight splits; weights from memory): a time is off by 5 % (the worst by a third), the tile and split that the
-# figures pick by 0.5 % on average from the best.
-TILES = {(8, 8): (3.3, 7.6, 1.24, 0.64), (8, 6): (3.7, 4.6, 0.96, 0.82), (6, 8): (2.9, 7.5, 0.94, 0.55), (6, 6): (2.9, 5.9, 0.75, 0.73), (8, 4): (2.8, 3.6, 0.71, 1.00), (4, 8): (3.1, 4.4, 0.76, 0.81), (4, 6): (2.8, 3.9, 0.61, 0.98), (4, 4): (4.9, 0.2, 0.45, 1.01)}
+# in it, and of a MB/us of what is written, over 4.5; then the same of steps of up to 256 rows, where one row tile's weights pass the caches by. Fitted to
+# 11936 timings (14 shapes of width 2048 and 4096, 70 - 4099 rows, every tile, one to eight splits; weights from memory): a time is off by 3 - 5 %
+# (the worst by a third), the tile and split that the figures pick by 0.5 % on average from the best. Heights of 160 and 224 rows and the weights past
+# the caches take 1 - 2 % off steps of 129 - 1024 rows and 3 - 4 % off longer ones (129 rows of 14336 -> 4096 35 -> 30, 1300 of 4096 -> 14336 15 %).
+TILES = {
+    (8, 8): ((1.8, 8.8, 1.208, 0.60), (1.4, 7.2, 1.173, 0.97)),
+    (8, 6): ((2.3, 5.1, 0.982, 0.78), (2.7, 4.0, 0.957, 1.13)),
+    (7, 8): ((2.2, 6.8, 1.096, 0.66), (1.0, 6.6, 1.089, 1.01)),
+    (6, 8): ((2.2, 5.8, 0.978, 0.72), (1.8, 5.5, 0.979, 1.13)),
+    (7, 6): ((2.5, 5.4, 0.873, 0.86), (1.9, 5.4, 0.878, 1.25)),
+    (6, 6): ((2.1, 4.3, 0.789, 0.93), (2.2, 4.0, 0.793, 1.40)),
+    (5, 8): ((2.2, 4.0, 0.865, 0.85), (2.3, 4.2, 0.869, 1.23)),
+    (8, 4): ((1.4, 3.8, 0.734, 0.96), (2.0, 3.0, 0.723, 1.32)),
+    (7, 4): ((1.2, 4.7, 0.661, 1.00), (1.7, 4.1, 0.665, 1.43)),
+    (5, 4): ((1.2, 2.2, 0.550, 1.33), (1.8, 2.9, 0.554, 1.37)),
+    (4, 8): ((1.5, 2.3, 0.808, 1.09), (1.4, 4.1, 0.833, 1.19)),
+    (4, 6): ((1.5, 2.5, 0.648, 1.24), (1.6, 3.9, 0.663, 1.25)),
+    (4, 4): ((3.3, 0.0, 0.464, 1.05), (3.9, 0.0, 0.504, 1.18)),
+}
 TILE_SPLITS = (1, 2, 4, 8)      # what the consumers of slabs load with all slabs in flight
 TILE_SLAB_BYTES = 1 << 28
 TILE_LIBRARY_N, TILE_MAX_M = 24576, 2560
@@ -412,13 +427,13 @@ TILE_GLU_M, TILE_EVEN_M, TILE_RAGGED_M = 3600, 5600, 8448
 TILE_WHOLE_GAIN = 0.8
 
 
-@lru_cache(maxsize=4096)
-def _tile_best(M: int, N: int, K: int, form: str) -> tuple[float, tuple[int, int, int]]:
-    """(us, plan) of the fastest launch of ``tile_plan`` by the figures above."""
+def _tile_search(M: int, N: int, K: int, form: str, odd: int) -> tuple[float, tuple[int, int, int]]:
+    """(us, plan) of the fastest launch of ``tile_plan`` by the figures above, on tiles of an even or ``odd`` number of 32 rows."""
     best = None
-    for (mt, nt), (launch, rnd, unit, out) in TILES.items():
-        if form == "glu" and nt % 4:
+    for (mt, nt), figures in TILES.items():
+        if mt & 1 != odd or form == "glu" and nt % 4:
             continue                # (a wave holds whole gate, up pairs)
+        launch, rnd, unit, out = figures[M <= 256]
         items = -(-M // (32 * mt)) * -(-N // (32 * nt))
         for s in TILE_SPLITS:
             if K // 64 < 2 * s or s > 1 and (form == "relu2" or 4 * s * M * N > TILE_SLAB_BYTES):
@@ -430,6 +445,16 @@ def _tile_best(M: int, N: int, K: int, form: str) -> tuple[float, tuple[int, int
             if best is None or t < best[0]:
                 best = (t, (mt, nt, s))
     return best
+
+
+@lru_cache(maxsize=4096)
+def _tile_best(M: int, N: int, K: int, form: str) -> tuple[float, tuple[int, int, int]]:
+    return _tile_search(M, N, K, form, 0)
+
+
+@lru_cache(maxsize=4096)
+def _tile_odd(M: int, N: int, K: int, form: str) -> tuple[float, tuple[int, int, int]]:
+    return _tile_search(M, N, K, form, 1)
 
 
 @lru_cache(maxsize=4096)
@@ -462,8 +487,10 @@ def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) 
     if library and M > TILE_MAX_M and \
             (M > (TILE_GLU_M if act else TILE_RAGGED_M if N % 256 else TILE_EVEN_M) or tiles <= (512 if act else 256)):
         return None
-    # (tiles are multiples of 64 rows high: sizes up to the next 64 share a search, 15 us of the host, else each new length of a prompt pays it)
-    best = _tile_best(-(-M // 64) * 64, N, K, form)
+    # (sizes up to the next multiple of the heights' 64 or 32 rows share a search, 15 us of the host, else each new length of a prompt pays it)
+    best, odd = _tile_best(-(-M // 64) * 64, N, K, form), _tile_odd(-(-M // 32) * 32, N, K, form)
+    if odd[0] < 0.98 * best[0]:     # (about what the figures cannot tell apart: 359 rows of 14336 -> 4096, 53.4 and 53.9 by them, a step takes 1 % more)
+        best = odd
     if library and M > (768 if tiles > 256 else 1024):
         rows = M // DENSE_BLOCK * DENSE_BLOCK if dense_cut(M, N, K) else M
         lib = 4 + -(-(-(-rows // 256) * -(-N // 256)) // 256) * 1.42 * (K // 64) + (20 if rows < M else 0)

@@ -228,9 +228,9 @@ __device__ __forceinline__ void ring_tile(const RingArgs& A, char* smem, int e, 
   const int N = A.N, K = A.K;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, q = lane >> 4;
   const int nb = nt * 8 + 4 * (w & 1);             // this wave's first 32-column tile (N is a multiple of 128)
-  unsigned xo[2 * R::DX], wo[R::DW];
+  unsigned xo[R::PX], wo[R::DW];
 #pragma unroll
-  for (int u = 0; u < 2 * R::DX; ++u) {
+  for (int u = 0; u < R::PX; ++u) {
     const int row = R::xrow(w, u, lane), m = min(row, rows - 1);   // rows past the segment reload a valid row, never stored
     const unsigned at = GATHER ? (unsigned)A.perm_tok[seg0 + m] : (unsigned)m;
     xo[u] = at * (unsigned)(A.ldx * 2) + R::xbyte(row, lane);
@@ -311,7 +311,10 @@ __global__ __launch_bounds__(256, 1) void grouped_ring_kernel(const bf16* __rest
   const RingArgs A{X, ldx, Wt, N, K, perm_tok, perm_w, Y, ldy, out, ldo, glu_limit, glu_alpha};
   // an expert's last rows on a lower tile where they fit one: the weights' way is then what it takes, a third of a whole tile
   // (22 rows an expert, us, whole / low tile of the combined product: 8 experts 2304 -> 2048 46 / 22, 4608 -> 4096 85 / 64, 64 of 768 -> 2048 50 / 40)
-  if (rows > 128) ring_tile<8, GATHER, EPI>(A, smem, e, seg0, rows, nt);
+  if (rows > 224) ring_tile<8, GATHER, EPI>(A, smem, e, seg0, rows, nt);
+  else if (rows > 192) ring_tile<7, GATHER, EPI>(A, smem, e, seg0, rows, nt);
+  else if (rows > 160) ring_tile<6, GATHER, EPI>(A, smem, e, seg0, rows, nt);
+  else if (rows > 128) ring_tile<5, GATHER, EPI>(A, smem, e, seg0, rows, nt);
   else if (rows > 64) ring_tile<4, GATHER, EPI>(A, smem, e, seg0, rows, nt);
   else ring_tile<2, GATHER, EPI>(A, smem, e, seg0, rows, nt);
 }

@@ -46,24 +46,27 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const void* p) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, -1, 0x00020000);
 }
 
-template <int MT_, int NT_, bool SWAP_>
+// WNT: weights that one row tile reads are asked for past the caches' retention (nt), so that the activations, which every column
+// tile reads, stay in the L2s: 222 rows of 4096 -> 28672 64 -> 61 us, of 14336 -> 4096 in eight splits 41 -> 36.
+template <int MT_, int NT_, bool SWAP_, bool WNT = false>
 struct Ring {
   static constexpr int MT = MT_, NT = NT_;
   static constexpr bool SWAP = SWAP_;
   static constexpr int BM = 32 * MT, BN = 32 * NT;
   static constexpr int NX = 3, NW = 4, XU = BM * 2 * BK * 2, WS = BN * BK * 2, LDS = NX * XU + NW * WS;   // bytes
-  static constexpr int DX = BM / 64, DW = BN / 64, DPS = DX + DW;   // 1 KB pieces a wave moves per stage (activations: half a unit)
+  // 1 KB pieces a wave moves: of a unit of activations (the first DO of them in an odd step, DE in the even one after it), of a stage of weights
+  static constexpr int PX = MT, DO = (PX + 1) / 2, DE = PX / 2, DW = BN / 64;
   static constexpr int NM = MT * NT, NR = MT + NT;                  // products and fragments of a stage
-  static constexpr int RST = NM * 3 / 4 / NR > 0 ? NM * 3 / 4 / NR : 1, DST = NM * 3 / 4 / DPS;
-  static_assert(BM % 64 == 0 && BN % 64 == 0 && 1 + (DPS - 1) * DST < NM && (NR - 1) * RST < NM, "ring");
+  static constexpr int RST = NM * 3 / 4 / NR > 0 ? NM * 3 / 4 / NR : 1, DST = NM * 3 / 4 / (DO + DW);
+  static_assert(BN % 64 == 0 && 1 + (DO + DW - 1) * DST < NM && (NR - 1) * RST < NM && LDS <= 163840, "ring");
 
   // what a lane adds to a weight piece's place: its 16 bytes of the tile
   static __device__ __forceinline__ unsigned wlane(int lane) {
     const int l = lane & 31;
     return ((lane & 32) + (SWAP ? 8 * ((l & 15) >> 2) + 4 * (l >> 4) + (l & 3) : l)) * 16;
   }
-  // row of the tile whose 16 bytes a lane moves in wave w's u-th piece of a unit (u < 2 DX), and where in the row's 128 bytes they start
-  static __device__ __forceinline__ int xrow(int w, int u, int lane) { return 8 * (2 * DX * w + u) + (lane >> 3); }
+  // row of the tile whose 16 bytes a lane moves in wave w's u-th piece of a unit (u < PX), and where in the row's 128 bytes they start
+  static __device__ __forceinline__ int xrow(int w, int u, int lane) { return 8 * (PX * w + u) + (lane >> 3); }
   static __device__ __forceinline__ int xbyte(int row, int lane) { return 16 * ((lane & 7) ^ (row & 7)); }
   // (32-column tile, 16-deep block) of wave w's u-th weight piece
   static __device__ __forceinline__ int wtile(int w, int u) { return (DW * w + u) / KB; }
@@ -72,22 +75,23 @@ struct Ring {
   // acc += the tile's products over nst stages (even, at least 4). xo: byte offsets of this lane's activation pieces in xr, wo: of
   // this wave's weight pieces in wr (behind which wl is the lane's), both at the first stage.
   static __device__ __forceinline__ void multiply(f32x4v (&acc)[MT][NT], char* smem, __amdgpu_buffer_rsrc_t xr,
-                                                  const unsigned (&xo)[2 * DX], __amdgpu_buffer_rsrc_t wr, unsigned wl,
+                                                  const unsigned (&xo)[PX], __amdgpu_buffer_rsrc_t wr, unsigned wl,
                                                   const unsigned (&wo)[DW], int nst, int lane, int w) {
     const int r = lane & 15, q = lane >> 4;
     char* const wsm = smem + NX * XU;
     auto xpiece = [&](int v, int slot, int u) {      // u-th piece of unit v
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_t*)(smem + slot * XU + (2 * DX * w + u) * 1024), 16, xo[u],
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_t*)(smem + slot * XU + (PX * w + u) * 1024), 16, xo[u],
                                                v * (4 * BK), 0, 0);
     };
     auto wpiece = [&](int s, int u) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_t*)(wsm + (s & (NW - 1)) * WS + (DW * w + u) * 1024), 16, wl,
-                                               wo[u] + s * (KB * 1024), 0, 0);
+                                               wo[u] + s * (KB * 1024), 0, WNT ? 2 : 0);
     };
     // what step s asks for: weights of stage s + 4, a half (the second where s is even) of the unit of stage s + 4 or s + 5
     auto piece = [&](int s, int odd, int slot, int u) {
-      if (u < DX) xpiece((s + 4 + odd) >> 1, slot, (odd ? 0 : DX) + u);
-      else wpiece(s + 4, u - DX);
+      const int dx = odd ? DO : DE;
+      if (u < dx) xpiece((s + 4 + odd) >> 1, slot, (odd ? 0 : DO) + u);
+      else wpiece(s + 4, u - dx);
     };
     // where this lane's fragments lie: rows 16 i + r, 8-deep piece q of the stage's half of a unit; columns 16 j + r, piece q of
     // tile j / 2
@@ -101,26 +105,26 @@ struct Ring {
     };
     // all that was asked for up to step s - 3 has arrived, everywhere: stage s + 1 is there, stage s read
     auto turn = [&](int s) {
-      if (s <= nst - 5) vmcnt<2 * DPS>();
-      else if (s == nst - 4) vmcnt<DPS + DW>();
+      if (s <= nst - 5) vmcnt<PX + 2 * DW>();
+      else if (s == nst - 4) vmcnt<DE + 2 * DW>();   // (an even step's, and the weights alone)
       else if (s == nst - 3) vmcnt<DW>();
       else vmcnt<0>();
       asm volatile("s_barrier" ::: "memory");
     };
     bf16x8 a0[MT], b0[NT], a1[MT], b1[NT];
 #pragma unroll
-    for (int u = 0; u < 2 * DX; ++u) xpiece(0, 0, u);
+    for (int u = 0; u < PX; ++u) xpiece(0, 0, u);
 #pragma unroll
     for (int u = 0; u < DW; ++u) wpiece(0, u);
 #pragma unroll
-    for (int u = 0; u < DPS; ++u) piece(-3, 1, 1, u);
+    for (int u = 0; u < DO + DW; ++u) piece(-3, 1, 1, u);
 #pragma unroll
-    for (int u = 0; u < DPS; ++u) piece(-2, 0, 1, u);
+    for (int u = 0; u < DE + DW; ++u) piece(-2, 0, 1, u);
 #pragma unroll
-    for (int u = 0; u < DPS; ++u)
-      if (u >= DX || nst > 4) piece(-1, 1, 2, u);
-    if (nst > 4) vmcnt<3 * DPS>();
-    else vmcnt<2 * DPS + DW>();
+    for (int u = 0; u < DO + DW; ++u)
+      if (u >= DO || nst > 4) piece(-1, 1, 2, u);
+    if (nst > 4) vmcnt<PX + DO + 3 * DW>();
+    else vmcnt<PX + 3 * DW>();
     asm volatile("s_barrier" ::: "memory");
 #pragma unroll
     for (int i = 0; i < NR; ++i) read(a0, b0, smem + xa0, wsm + wa, i);
@@ -129,13 +133,13 @@ struct Ring {
     auto step = [&](auto full, auto is_odd, int s, const bf16x8(&a)[MT], const bf16x8(&b)[NT], bf16x8(&an)[MT],
                     bf16x8(&bn)[NT]) {
       constexpr bool load = decltype(full)::value;
-      constexpr int odd = decltype(is_odd)::value ? 1 : 0;
+      constexpr int odd = decltype(is_odd)::value ? 1 : 0, DX = odd ? DO : DE, DPS = DX + DW;
       const int next = slot == NX - 1 ? 0 : slot + 1, third = next == NX - 1 ? 0 : next + 1;
       const int to = odd ? slot : third;             // the unit that step s fills
       __builtin_amdgcn_s_waitcnt(LGKM0);             // (this stage's fragments)
       const bool more = load || s + 1 < nst;
       if constexpr (load) {
-        vmcnt<2 * DPS>();
+        vmcnt<PX + 2 * DW>();
         asm volatile("s_barrier" ::: "memory");
       } else {
         if (more) turn(s);

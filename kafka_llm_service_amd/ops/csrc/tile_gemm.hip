@@ -14,13 +14,13 @@ namespace tg {
 
 enum { OUT_BF16 = 0, OUT_SLAB = 1, OUT_GLU = 2, OUT_SLAB_GLU = 3, OUT_RELU2 = 4, OUT_GELU = 5 };
 
-// MT, NT: 16-row and 16-column parts of a wave's tile (2 x 2 waves); OCC workgroups on a CU
-template <int MT, int NT, int OCC>
+// MT, NT: 16-row and 16-column parts of a wave's tile (2 x 2 waves); OCC workgroups on a CU; WNT: of one row tile
+template <int MT, int NT, int OCC, bool WNT>
 __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const bf16* __restrict__ X, int64_t ldx,
                                                              const bf16x8* __restrict__ Wt, int M, int N, int K, int S,
                                                              bf16* __restrict__ Y, int64_t ldy, float* __restrict__ P,
                                                              int mode) {
-  using R = ring::Ring<MT, NT, true>;
+  using R = ring::Ring<MT, NT, true, WNT>;
   __shared__ __attribute__((aligned(1024))) char smem[R::LDS];
   // item -> (split, rows, columns): an XCD takes one contiguous stretch of them: of a split the row tiles of up to 2048 rows
   // side by side, then the next column tile, so that its weights leave memory once
@@ -33,9 +33,9 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const bf16* __restr
   // K in units of 64, split as evenly as they go
   const int units = K >> 6, u0 = (int)((int64_t)units * sp / S), u1 = (int)((int64_t)units * (sp + 1) / S);
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, q = lane >> 4;
-  unsigned xo[2 * R::DX], wo[R::DW];
+  unsigned xo[R::PX], wo[R::DW];
 #pragma unroll
-  for (int u = 0; u < 2 * R::DX; ++u) {            // rows past M reload the last, never stored
+  for (int u = 0; u < R::PX; ++u) {            // rows past M reload the last, never stored
     const int row = R::xrow(w, u, lane);
     xo[u] = (unsigned)min(row, rows - 1) * (unsigned)(ldx * 2) + R::xbyte(row, lane);
   }
@@ -104,16 +104,27 @@ extern "C" hipError_t kafka_launch_tile_gemm(const bf16* X, int64_t ldx, const b
   const unsigned grid = (unsigned)((total + 7) / 8 * 8);
   const auto* wt = reinterpret_cast<const bf16x8*>(Wt);
   auto a = [&](auto kern) { kern<<<grid, 256, 0, st>>>(X, ldx, wt, M, N, K, splits, Y, ldy, P, mode); };
-  if (mt == 8 && nt == 8) a(tile_gemm_kernel<8, 8, 1>);
-  else if (mt == 8 && nt == 4) a(tile_gemm_kernel<8, 4, 1>);
-  else if (mt == 8 && nt == 6) a(tile_gemm_kernel<8, 6, 1>);
-  else if (mt == 6 && nt == 8) a(tile_gemm_kernel<6, 8, 1>);
-  else if (mt == 6 && nt == 6) a(tile_gemm_kernel<6, 6, 1>);
-  else if (mt == 4 && nt == 6) a(tile_gemm_kernel<4, 6, 1>);
-  else if (mt == 4 && nt == 8) a(tile_gemm_kernel<4, 8, 1>);
-  else if (mt == 4 && nt == 4) a(tile_gemm_kernel<4, 4, 2>);
-  else return hipErrorInvalidValue;
-  return hipGetLastError();
+#define TILE(MT, NT, OCC)                                        \
+  if (mt == MT && nt == NT) {                                    \
+    if (M <= 32 * MT) a(tile_gemm_kernel<MT, NT, OCC, true>);    \
+    else a(tile_gemm_kernel<MT, NT, OCC, false>);                \
+    return hipGetLastError();                                    \
+  }
+  TILE(8, 8, 1)
+  TILE(8, 4, 1)
+  TILE(8, 6, 1)
+  TILE(7, 8, 1)
+  TILE(7, 6, 1)
+  TILE(7, 4, 1)
+  TILE(6, 8, 1)
+  TILE(6, 6, 1)
+  TILE(5, 8, 1)
+  TILE(5, 4, 1)
+  TILE(4, 6, 1)
+  TILE(4, 8, 1)
+  TILE(4, 4, 2)
+#undef TILE
+  return hipErrorInvalidValue;
 }
 
 }  // namespace tg

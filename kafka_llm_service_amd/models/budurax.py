@@ -385,8 +385,7 @@ class BuduraxLM:
         M = x.shape[0]
         if self.stream and wt is not None and 0 < M <= self.stream_max_m and \
                 ops.stream_plan(M, w.shape[0], w.shape[1]) is not None:
-            y = ops.linear_stream(x, wt)
-            return ops.slab_reduce(y) if ops.is_slab(y) and not slabs else y
+            return ops.linear_stream(x, wt) if slabs else ops.linear_stream_rounded(x, wt)
         return ops.linear_long(x, w, wt if self.stream else None, slabs)
 
     def _gelu_up(self, lw, h):

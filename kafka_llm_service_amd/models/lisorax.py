@@ -264,8 +264,7 @@ class LisoraxLM:
         M = x.shape[0]
         if self.stream and wt is not None and 0 < M <= self.stream_max_m and \
                 ops.stream_plan(M, w.shape[0], w.shape[1]) is not None:
-            y = ops.linear_stream(x, wt)
-            y = ops.slab_reduce(y) if ops.is_slab(y) else y
+            y = ops.linear_stream_rounded(x, wt)
             return y if bias is None else y.add_(bias)
         if self.stream and wt is not None and bias is None and x.is_cuda:
             return ops.linear_long(x, w, wt)

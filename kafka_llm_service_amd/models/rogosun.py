@@ -303,8 +303,7 @@ class RogosunLM:
         """x @ w^T: the weight-streaming kernel for decode-sized steps when the weight has a tiled copy, else
         the tile kernel or the library (ops.linear_long). ``slabs``: the caller takes the split-K slabs [S, T, N] as they are."""
         if self._streams(x.shape[0], w, wt):
-            y = ops.linear_stream(x, wt)
-            return ops.slab_reduce(y) if ops.is_slab(y) and not slabs else y
+            return ops.linear_stream(x, wt) if slabs else ops.linear_stream_rounded(x, wt)
         return ops.linear_long(x, w, wt if self.stream else None, slabs)
 
     def _logits(self, hf):

@@ -352,8 +352,7 @@ def stream_plan(M: int, N: int, K: int, max_splits: int = 8) -> tuple[int, int, 
     if K % kc or K <= 0:
         return None
     nx, chunks, s = (N + 127) // 128 * ((M + 32 * mt - 1) // (32 * mt)), K // kc, 1
-    target = 192
-    while s * 2 <= max_splits and s * 2 <= 8 and chunks % (s * 2) == 0 and nx * s < target:
+    while s * 2 <= max_splits and s * 2 <= 8 and chunks % (s * 2) == 0 and (nx * s <= 128 or s == 1 and nx < 192):
         s *= 2
     return mt, kc, s
 
@@ -605,6 +604,18 @@ def linear_stream(x: torch.Tensor, wt: torch.Tensor, max_splits: int = 8, nt: bo
     return torch.stack([xf[:, s * ks:(s + 1) * ks] @ w[:, s * ks:(s + 1) * ks].t() for s in range(S)])
 
 
+def _one_split(wt: torch.Tensor) -> int:
+    """Most splits of a product whose caller has no use for slabs: one of 129 - 191 column tiles is faster whole (18560 columns of 4096, us, two
+    splits / one: 1 row 32.3 / 27.0, 64 39.1 / 34.3, 128 50.9 / 46.7, and the slabs' sum, 5, beside the former)."""
+    return 1 if 128 < (wt.shape[0] + 3) // 4 < 192 else 8
+
+
+def linear_stream_rounded(x: torch.Tensor, wt: torch.Tensor) -> torch.Tensor:
+    """``linear_stream`` in the activations' type, [M, N]."""
+    y = linear_stream(x, wt, _one_split(wt))
+    return slab_reduce(y) if is_slab(y) else y
+
+
 def stream_logits(x: torch.Tensor, wt: torch.Tensor | None, max_m: int) -> torch.Tensor | None:
     """x @ W^T in fp32 from the weight-streaming kernel's sums, None for shapes that it does not take in one split: logits, which
     are read as fp32 (as bf16, a launch to widen them again: 5 us)."""
@@ -622,7 +633,7 @@ def stream_logits(x: torch.Tensor, wt: torch.Tensor | None, max_m: int) -> torch
 def linear_glu(x: torch.Tensor, wt: torch.Tensor, max_splits: int = 8, act: str = "silu") -> torch.Tensor:
     """silu(x @ Wg^T) * (x @ Wu^T) from GLU-tiled gate_up weights: fused into the GEMM epilogue when the plan has one
     split, else the GEMM's slabs go through silu_mul (``act`` as there)."""
-    N = wt.shape[0] * 32
+    N, max_splits = wt.shape[0] * 32, min(max_splits, _one_split(wt))
     plan = stream_plan(x.shape[0], N, x.shape[1], max_splits)
     y = linear_stream(x, wt, max_splits, glu=True, act=act)
     return y if plan is not None and plan[2] == 1 else silu_mul(y, act=act)

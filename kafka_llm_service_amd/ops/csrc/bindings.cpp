@@ -634,15 +634,17 @@ static void wstream_gemm(at::Tensor x, at::Tensor wt, c10::optional<at::Tensor> 
                 "wstream_gemm: slab shape must be [splits, M, N]");
     pp = p->data_ptr<float>();
   }
-  // two K halves per chunk (8 waves) for 64-row tiles with >= 6 chunks per split: the long streams (gate_up unsplit
+  // two K halves per chunk (8 waves) for 64-row tiles with >= 4 chunks per split: the long streams (gate_up unsplit
   // with its fused SwiGLU, down) ran 1.6-2.8 % faster in the config sweep, the short ones (qkv, o) slower; headline
-  // +0.24 % (3 / 3 interleaved pairs, profiles/r04/bench_ab_wstream_kw2.jsonl)
-  const int kw = mt == 2 && kc == 256 && K / s / kc >= 6 ? 2 : 1;
+  // +0.24 % (3 / 3 interleaved pairs, profiles/r04/bench_ab_wstream_kw2.jsonl). Of 4 chunks, us, one / two: 4096 -> 6144 13.0 / 12.5,
+  // -> 8192 15.9 / 15.2, 8192 -> 4096 15.1 / 14.7, 2048 -> 9344 12.2 / 11.8, -> 14336 15.1 / 15.3; of 2 the same.
+  const int kw = mt == 2 && kc == 256 && K / s / kc >= 4 ? 2 : 1;
   // weight prefetch pinned ahead of the MFMAs (wstream_gemm_kernel PIN) when a split streams >= 3 chunks: -1..-4 us
   // per projection at 64 rows, -4..-7 us at 97..128 rows; not for 96-row tiles (their 348 registers leave one wave
   // per SIMD and the longer live ranges lose) nor 2-chunk splits (o at 64 rows: +0.9 us)
-  // (profiles/r05/wstream_sweep_pin.jsonl)
-  const int pin = mt != 3 && K / s / kc >= 3 ? 1 : 0;
+  // (profiles/r05/wstream_sweep_pin.jsonl); and not for up to 32 rows where nearly every CU has a workgroup (us, pinned / not, 4096 -> 28672
+  // 37.0 / 36.1, -> 32000 41.8 / 40.3, -> 14336 in two 21.0 / 20.3; with fewer of them 18560 27.0 / 28.9)
+  const int pin = mt != 3 && K / s / kc >= 3 && !(mt == 1 && (N + 127) / 128 * s > 192) ? 1 : 0;
   CHECK_HIP(kafka_launch_wstream_gemm(bptr(x), x.stride(0), bptr(wt), M, N, K, mt, kc, s, nt ? 1 : 0, kw, pin,
                                       (int)glu,
                                       yp, ldy, pp, cur_stream()));
@@ -690,7 +692,7 @@ static void wstream_fin(int64_t fin, at::Tensor x, at::Tensor wt, c10::optional<
     fa.nss = ss_in->size(0);
     fa.ss_ld = ss_in->stride(0);
   }
-  const int kw = mt == 2 && kc == 256 && K / s / kc >= 6 ? 2 : 1;  // (the wstream_gemm rules above)
+  const int kw = mt == 2 && kc == 256 && K / s / kc >= 4 ? 2 : 1;  // (the wstream_gemm rules above)
   const int pin = mt != 3 && K / s / kc >= 3 ? 1 : 0;
   bf16* yp = nullptr;
   int64_t ldy = 0;

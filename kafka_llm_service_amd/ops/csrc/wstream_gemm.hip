@@ -878,9 +878,12 @@ extern "C" int kafka_wstream_plan(int M, int N, int K, int max_splits, int* mt, 
   // unsplit and qkv (N = 6144) with S = 4. With the pinned prefetch, gate_up at 97..128 rows also runs fastest
   // unsplit (53.3 us at 114 rows with its fused SwiGLU vs 60.4 + a SwiGLU pass split in two;
   // profiles/r05/wstream_sweep_pin.jsonl), so MT = 4 shares the target (it was 256).
-  const int target = 192;
+  // Past one split never more than one round of the chip (256): the workgroups of a second, partial one run beside the first ones' and
+  // take from their share. us, splits for 192 workgroups / these: 10816 columns of 4096 (340 workgroups / 170) 1 row 18.2 / 15.4, 64 23.5 / 20.3, 128
+  // 30.5 / 26.2; 9344 of 2048 (292 / 146) 1 row 10.1 / 9.0, 64 13.8 / 11.8, 128 19.7 / 15.7. (129 - 191 column tiles: in two for
+  // consumers of fp32 slabs, whole for others, ops.linear_stream_rounded.)
   int s = 1;
-  while (s * 2 <= max_splits && s * 2 <= 8 && chunks % (s * 2) == 0 && nx * s < target) s *= 2;
+  while (s * 2 <= max_splits && s * 2 <= 8 && chunks % (s * 2) == 0 && (nx * s <= 128 || (s == 1 && nx < 192))) s *= 2;
   *mt = MT;
   *kc = KC;
   *splits = s;

@@ -12,6 +12,7 @@ constexpr int CH = 128;         // tokens per chunk
 constexpr int VSL = 64;         // value columns of a workgroup
 constexpr int LDJ = CH + 8;     // row length of a transposed tile in LDS
 constexpr int DS = 128;         // key channels staged at a time
+constexpr int LDD = DS + 8;     // row length of a tile of an entry state's part in LDS
 
 // v = a + b + c with bf16 parts that hold all its bits
 struct Split {
@@ -47,12 +48,14 @@ __device__ __forceinline__ bool chunk_item(int items, int slices, int& item, int
 }
 __host__ __device__ __forceinline__ int chunk_grid(int items, int slices) { return (items + 7) / 8 * 8 * slices; }
 
-// rows row0 .. row0 + 127 (past n: the last one), columns c0 .. c0 + nc - 1 of the head's part at col -> tile[column][row]
+// rows row0 .. row0 + 127 (past n: the last one), columns c0 .. c0 + nc - 1 of the head's part at col -> tile[column][row].
+// A wave moves 4 x 8 columns of 16 x 4 rows: 64 bytes in a run from memory, pairs of banks in LDS (all columns of 8 x 4 rows: eight on one bank).
 __device__ __forceinline__ void stage_transposed(const bf16* src, int64_t stride, int n, int c0, int nc, int ncols,
                                                  bf16* tile, int tid) {
-  const int cgs = nc >> 3;
-  for (int u = tid; u < cgs * (CH / 4); u += NT) {
-    const int cg = u % cgs, rq = u / cgs, c = c0 + 8 * cg;
+  const int cgs = nc >> 3, blocks = (cgs + 3) >> 2;
+  for (int u = tid; u < blocks * CH; u += NT) {
+    const int q = u >> 6, half = q >= blocks, cg = 4 * (q - half * blocks) + (u & 3), rq = 16 * half + ((u >> 2) & 15), c = c0 + 8 * cg;
+    if (cg >= cgs) continue;
     bf16x8 x[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -65,6 +68,38 @@ __device__ __forceinline__ void stage_transposed(const bf16* src, int64_t stride
       const bf16x4 y = {x[0][e], x[1][e], x[2][e], x[3][e]};
       *reinterpret_cast<bf16x4*>(tile + (8 * cg + e) * LDJ + 4 * rq) = y;
     }
+  }
+}
+
+// channels 0 .. nd - 1 (nd <= DS) of VSL fp32 rows (past nv: zeros) in three bf16 parts -> buf[part][row][channel]. All of a thread's
+// loads go out together.
+__device__ __forceinline__ void stage_split(const float* src, int64_t stride, int nd, int nv, bf16* buf, int tid) {
+  typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
+  constexpr int RQ = DS / 4, NU = VSL * RQ / NT;
+  static_assert(NT % RQ == 0 && VSL * RQ % NT == 0, "whole rows");
+  const int v = tid / RQ, d = 4 * (tid % RQ);
+  if (d >= nd) return;
+  f32x4 x[NU];
+#pragma unroll
+  for (int k = 0; k < NU; ++k) {
+    const int r = v + k * (NT / RQ);
+    x[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (r < nv) x[k] = *reinterpret_cast<const f32x4*>(src + r * stride + d);
+  }
+#pragma unroll
+  for (int k = 0; k < NU; ++k) {
+    bf16x4 p[3];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bf16 a = (bf16)x[k][e];
+      const float rr = x[k][e] - (float)a;
+      const bf16 b = (bf16)rr;
+      p[0][e] = a;
+      p[1][e] = b;
+      p[2][e] = (bf16)(rr - (float)b);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x4*>(buf + (i * VSL + v + k * (NT / RQ)) * LDD + d) = p[i];
   }
 }
 

@@ -18,6 +18,8 @@
 //     chunk_state   U^T and its normaliser for every chunk in parallel
 //     chunk_carry   the chunks' entry states in order (in place of U), the sequence's state advanced
 //     chunk_out     the read-outs for every chunk in parallel
+//   What bounds the chunks is as in hybrid_ssd.hip, and three workgroups share a CU in the same way: 8192 tokens x 16 heads of 128 x 256,
+//   one layer: 86 + 60 + 138 us (two workgroups a CU, one element of the carry a thread: 113 + 77 + 205).
 //   All products run on the bf16 matrix cores: q, k and v are bf16, the fp32 factor of a product (scaled keys, weights,
 //   entry states) is split into three bf16 parts that hold all 24 bits of it, one product each.
 #include "chunk_common.h"
@@ -140,11 +142,13 @@ struct ChunkIn {
   float* U;             // [chunks][H][Dv][D]: own contribution, then entry state
   float* un;            // [chunks][H][D]: the same for the normaliser
   float* sc;            // [chunks][H][4] = F_end, M, m0
+  float* sums;          // [chunks][H][3][CH]: what chunk_gates finds
 };
 
-// The chunk's gates by one wave: a_t, its running maximum c_t and F_t to LDS (rows past n: f = 0, a = -inf).
+// The chunk's gates by one wave: a_t, its running maximum c_t and F_t to LDS (rows past n: f = 0, a = -inf). They are
+// kept (unless nullptr) for chunk_out, whose waves would wait for them.
 __device__ __forceinline__ void chunk_gates(const ChunkIn& in, int row0, int n, int h, int lane, float* a_s, float* c_s,
-                                            float* F_s) {
+                                            float* F_s, float* keep) {
   float f[2], g[2];
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
@@ -171,6 +175,10 @@ __device__ __forceinline__ void chunk_gates(const ChunkIn& in, int row0, int n, 
     c[k] = g[k] - f[k];
     a_s[64 * k + lane] = c[k];
     F_s[64 * k + lane] = f[k];
+    if (keep) {
+      keep[64 * k + lane] = c[k];
+      keep[2 * CH + 64 * k + lane] = f[k];
+    }
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const float u = __shfl_up(c[k], o, 64);
@@ -179,10 +187,13 @@ __device__ __forceinline__ void chunk_gates(const ChunkIn& in, int row0, int n, 
   }
   c[1] = fmaxf(c[1], __shfl(c[0], 63, 64));
 #pragma unroll
-  for (int k = 0; k < 2; ++k) c_s[64 * k + lane] = c[k];
+  for (int k = 0; k < 2; ++k) {
+    c_s[64 * k + lane] = c[k];
+    if (keep) keep[CH + 64 * k + lane] = c[k];
+  }
 }
 
-__global__ __launch_bounds__(NT) void mlstm_chunk_state_kernel(ChunkIn in, int n_chunks, int slices) {
+__global__ __launch_bounds__(NT, 3) void mlstm_chunk_state_kernel(ChunkIn in, int n_chunks, int slices) {
   __shared__ __attribute__((aligned(16))) bf16 Kt[DS * LDJ];
   __shared__ __attribute__((aligned(16))) bf16 Vt[VSL * LDJ];
   __shared__ float a_s[CH], c_s[CH], F_s[CH];
@@ -193,7 +204,7 @@ __global__ __launch_bounds__(NT) void mlstm_chunk_state_kernel(ChunkIn in, int n
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int D = in.D, Dv = in.Dv, H = in.H;
   const bf16* rows = in.qkv + (int64_t)row0 * in.qs;
-  if (w == 0) chunk_gates(in, row0, n, h, lane, a_s, c_s, F_s);
+  if (w == 0) chunk_gates(in, row0, n, h, lane, a_s, c_s, F_s, slice == 0 ? in.sums + (int64_t)item * 3 * CH : nullptr);
   stage_transposed(rows + 2 * (int64_t)H * D + (int64_t)h * Dv, in.qs, n, v0, VSL, Dv, Vt, tid);
   for (int db = 0; db < D; db += DS) {
     if (db) __syncthreads();
@@ -245,8 +256,47 @@ __global__ __launch_bounds__(NT) void mlstm_chunk_state_kernel(ChunkIn in, int n
   }
 }
 
-// grid (element blocks of Dv * D (+ one block of the normaliser and the maximum), H, segments): cs[r] = (first chunk,
-// chunks, first position, state slot)
+// grid (blocks of 4 NT elements of Dv * D (+ one block of the normaliser and the maximum), H, segments): cs[r] = (first chunk,
+// chunks, first position, state slot). V neighbouring elements a thread: el those of the first chunk, st theirs in the slot.
+template <int V>
+__device__ __forceinline__ void carry_chunks(const ChunkIn& in, int h, int first, int last, int p0, float m, float* el, int64_t step,
+                                             float* st, int64_t st_step, bool keep) {
+  typedef float fv __attribute__((ext_vector_type(V)));
+  const int H = in.H;
+  fv S;
+#pragma unroll
+  for (int e = 0; e < V; ++e) S[e] = p0 > 0 ? st[e * st_step] : 0.f;
+  auto at = [&](int c) { return reinterpret_cast<fv*>(el + (int64_t)c * step); };
+  constexpr int PF = 4;
+  fv u[PF];
+#pragma unroll
+  for (int k = 0; k < PF; ++k)
+    if (first + k < last) u[k] = *at(first + k);
+  for (int c0 = first; c0 < last; c0 += PF) {
+    fv nx[PF];
+#pragma unroll
+    for (int k = 0; k < PF; ++k)
+      if (c0 + PF + k < last) nx[k] = *at(c0 + PF + k);
+#pragma unroll
+    for (int k = 0; k < PF; ++k) {
+      const int c = c0 + k;
+      if (c < last) {
+        const float* sc = in.sc + 4 * ((int64_t)c * H + h);
+        const float F = sc[0], M = sc[1], mu = fmaxf(m, M);
+        *at(c) = S;                                      // the chunk's entry state
+        if (keep) in.sc[4 * ((int64_t)c * H + h) + 2] = m;
+        S = expf(m - mu) * S + expf(M - mu) * u[k];
+        m = F + mu;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < PF; ++k) u[k] = nx[k];
+  }
+#pragma unroll
+  for (int e = 0; e < V; ++e) st[e * st_step] = S[e];
+  if (keep) in.sc[4 * ((int64_t)(last - 1) * H + h) + 3] = m;
+}
+
 __global__ __launch_bounds__(NT) void mlstm_chunk_carry_kernel(ChunkIn in, const int* __restrict__ cs,
                                                                float* __restrict__ Sst, float* __restrict__ nst,
                                                                float* __restrict__ mst) {
@@ -255,61 +305,30 @@ __global__ __launch_bounds__(NT) void mlstm_chunk_carry_kernel(ChunkIn in, const
   const int64_t head = (int64_t)slot * H + h;
   // (the block of the normaliser is the only writer of m; the others read it before: it writes m to sc and mlstm_commit
   // stores it in the end)
-  float m = p0 > 0 ? mst[head] : 0.f;
-  const bool norm = blockIdx.x + 1 == gridDim.x;
-  float* st;
-  float* el;
-  int64_t step;
-  if (norm) {
-    if ((int)threadIdx.x >= D) return;
-    st = nst + head * D + threadIdx.x;
-    el = in.un + (int64_t)h * D + threadIdx.x;
-    step = (int64_t)H * D;
-  } else {
-    const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;   // element v * D + d
-    if (i >= (int64_t)Dv * D) return;
-    const int v = (int)(i / D), d = (int)(i - (int64_t)v * D);
-    st = Sst + head * D * Dv + (int64_t)d * Dv + v;
-    el = in.U + (int64_t)h * Dv * D + i;
-    step = (int64_t)H * Dv * D;
+  const float m = p0 > 0 ? mst[head] : 0.f;
+  if (blockIdx.x + 1 == gridDim.x) {
+    const int d = threadIdx.x;
+    if (d < D) carry_chunks<1>(in, h, first, last, p0, m, in.un + (int64_t)h * D + d, (int64_t)H * D, nst + head * D + d, 1, d == 0);
+    return;
   }
-  float S = p0 > 0 ? *st : 0.f;
-  constexpr int PF = 4;
-  float u[PF];
-#pragma unroll
-  for (int k = 0; k < PF; ++k) u[k] = first + k < last ? el[(int64_t)(first + k) * step] : 0.f;
-  for (int c0 = first; c0 < last; c0 += PF) {
-    float nx[PF];
-#pragma unroll
-    for (int k = 0; k < PF; ++k) nx[k] = c0 + PF + k < last ? el[(int64_t)(c0 + PF + k) * step] : 0.f;
-#pragma unroll
-    for (int k = 0; k < PF; ++k) {
-      const int c = c0 + k;
-      if (c < last) {
-        const float* sc = in.sc + 4 * ((int64_t)c * H + h);
-        const float F = sc[0], M = sc[1], mu = fmaxf(m, M);
-        el[(int64_t)c * step] = S;                       // the chunk's entry state
-        if (norm && threadIdx.x == 0) in.sc[4 * ((int64_t)c * H + h) + 2] = m;
-        S = expf(m - mu) * S + expf(M - mu) * u[k];
-        m = F + mu;
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < PF; ++k) u[k] = nx[k];
-  }
-  *st = S;
-  if (norm && threadIdx.x == 0) in.sc[4 * ((int64_t)(last - 1) * H + h) + 3] = m;
+  const int64_t i = 4 * ((int64_t)blockIdx.x * NT + threadIdx.x);   // element v * D + d (D is a multiple of 16)
+  if (i >= (int64_t)Dv * D) return;
+  const int v = (int)(i / D), d = (int)(i - (int64_t)v * D);
+  carry_chunks<4>(in, h, first, last, p0, m, in.U + (int64_t)h * Dv * D + i, (int64_t)H * Dv * D,
+                  Sst + head * D * Dv + (int64_t)d * Dv + v, Dv, false);
 }
 
 // NKS: 16-channel steps of a head held in registers (D <= 16 NKS; the steps past D multiply by zero queries)
 template <int NKS>
-__global__ __launch_bounds__(NT) void mlstm_chunk_out_kernel(ChunkIn in, const int* __restrict__ cs, int n_segs,
+__global__ __launch_bounds__(NT, NKS <= 8 ? 3 : 2) void mlstm_chunk_out_kernel(ChunkIn in, const int* __restrict__ cs, int n_segs,
                                                              float* __restrict__ mst, int n_chunks, int slices,
                                                              float* __restrict__ out, int64_t os) {
   // one buffer, first for the entry state's three parts [3][VSL][DS + 8], then for the values [VSL][LDJ]
-  constexpr int LDD = DS + 8;
   __shared__ __attribute__((aligned(16))) bf16 buf[3 * VSL * LDD];
-  __shared__ float a_s[CH], c_s[CH], F_s[CH], n_s[256];
+  __shared__ float sum_s[3 * CH];
+  const float *a_s = sum_s, *c_s = sum_s + CH, *F_s = sum_s + 2 * CH;
+  // the normaliser's entry state lies in the 16 bytes behind the first rows of buf (with 1 KB of its own two workgroups share a CU, not three)
+  auto n_s = [&](int d) { return reinterpret_cast<float*>(buf + (d >> 2) * LDD + DS) + (d & 3); };
   // the sequences' maxima: read by every block of the carry kernel, written only now
   for (int i = blockIdx.x * NT + threadIdx.x; i < n_segs * in.H; i += gridDim.x * NT) {
     const int r = i / in.H, h = i - r * in.H;
@@ -319,12 +338,12 @@ __global__ __launch_bounds__(NT) void mlstm_chunk_out_kernel(ChunkIn in, const i
   if (!chunk_item(n_chunks * in.H, slices, item, slice)) return;   // (uniform)
   const int ch = item / in.H, h = item - ch * in.H, v0 = slice * VSL;
   const int row0 = in.vseg[4 * ch], n = in.vseg[4 * ch + 1];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int D = in.D, Dv = in.Dv, H = in.H, nks = D >> 4;
   const bf16* rows = in.qkv + (int64_t)row0 * in.qs;
   const float m0 = in.sc[4 * (int64_t)item + 2];
-  if (w == 0) chunk_gates(in, row0, n, h, lane, a_s, c_s, F_s);
-  for (int d = tid; d < D; d += NT) n_s[d] = in.un[(int64_t)item * D + d];
+  for (int i = tid; i < 3 * CH; i += NT) sum_s[i] = in.sums[(int64_t)item * 3 * CH + i];
+  for (int d = tid; d < D; d += NT) *n_s(d) = in.un[(int64_t)item * D + d];
   const int t = 32 * w + lr;                       // this lane's row
   const bf16* qrow = rows + (int64_t)min(t, n - 1) * in.qs + (int64_t)h * D + 8 * lh;
   bf16x8 qf[NKS], kf[NKS];
@@ -338,7 +357,6 @@ __global__ __launch_bounds__(NT) void mlstm_chunk_out_kernel(ChunkIn in, const i
     qf[ks] = load_bf16x8(qrow + 16 * min(ks, nks - 1));
     if (ks >= nks) qf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
   }
-  fetch_keys(0);
   f32x16 acc[2];
 #pragma unroll
   for (int vt = 0; vt < 2; ++vt)
@@ -347,26 +365,9 @@ __global__ __launch_bounds__(NT) void mlstm_chunk_out_kernel(ChunkIn in, const i
   float nq = 0.f;
   // ---- the entry state: acc = S_0^T q
   for (int db = 0; db < D; db += DS) {
-    const int nd = min(DS, D - db), d4s = nd >> 2;
+    const int nd = min(DS, D - db);
     if (db) __syncthreads();
-    for (int u = tid; u < VSL * d4s; u += NT) {
-      const int v = u / d4s, d = 4 * (u - v * d4s);
-      f32x4 x = {0.f, 0.f, 0.f, 0.f};
-      if (v0 + v < Dv) x = *reinterpret_cast<const f32x4*>(in.U + ((int64_t)item * Dv + v0 + v) * D + db + d);
-      typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
-      bf16x4 p[3];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bf16 a = (bf16)x[e];
-        const float rr = x[e] - (float)a;
-        const bf16 b = (bf16)rr;
-        p[0][e] = a;
-        p[1][e] = b;
-        p[2][e] = (bf16)(rr - (float)b);
-      }
-#pragma unroll
-      for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x4*>(buf + (k * VSL + v) * LDD + d) = p[k];
-    }
+    stage_split(in.U + ((int64_t)item * Dv + v0) * D + db, D, nd, Dv - v0, buf, tid);
     __syncthreads();
     if (32 * w < n) {   // (uniform per wave)
 #pragma unroll
@@ -374,7 +375,7 @@ __global__ __launch_bounds__(NT) void mlstm_chunk_out_kernel(ChunkIn in, const i
         const int d = 16 * ks - db;   // (uniform) the step's channels in this block
         if (d >= 0 && d < nd) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) nq += n_s[db + d + 8 * lh + e] * (float)qf[ks][e];
+          for (int e = 0; e < 8; ++e) nq += *n_s(db + d + 8 * lh + e) * (float)qf[ks][e];
 #pragma unroll
           for (int vt = 0; vt < 2; ++vt)
 #pragma unroll
@@ -386,6 +387,7 @@ __global__ __launch_bounds__(NT) void mlstm_chunk_out_kernel(ChunkIn in, const i
       mfma_settle();
     }
   }
+  fetch_keys(0);
   __syncthreads();
   stage_transposed(rows + 2 * (int64_t)H * D + (int64_t)h * Dv, in.qs, n, v0, VSL, Dv, buf, tid);
   __syncthreads();
@@ -494,7 +496,7 @@ int kafka_hy_mlstm_chunk_ok(int H, int D, int Dv, int64_t qs) {
   return D >= 16 && D % 16 == 0 && D <= 256 && Dv >= 8 && Dv % 8 == 0 && qs % 8 == 0;
 }
 // floats of scratch per (chunk, head)
-int64_t kafka_hy_mlstm_chunk_scratch(int D, int Dv) { return (int64_t)D * Dv + D + 4; }
+int64_t kafka_hy_mlstm_chunk_scratch(int D, int Dv) { return (int64_t)D * Dv + D + 4 + 3 * CH; }
 
 // the segments of cs in chunks (vseg: all their chunks in order)
 hipError_t kafka_hy_mlstm_chunked(const void* qkv, int64_t qs, const float* gates, int64_t gs, int H, int D, int Dv,
@@ -506,10 +508,10 @@ hipError_t kafka_hy_mlstm_chunked(const void* qkv, int64_t qs, const float* gate
   const int slices = (Dv + VSL - 1) / VSL;
   if ((items + 8) * slices > 0x7fffffff) return hipErrorInvalidValue;
   ChunkIn in{(const bf16*)qkv, qs, gates, gs, H, D, Dv, cap, vseg, scratch, scratch + items * D * Dv,
-             scratch + items * ((int64_t)D * Dv + D)};
+             scratch + items * ((int64_t)D * Dv + D), scratch + items * ((int64_t)D * Dv + D + 4)};
   const unsigned g = (unsigned)chunk_grid((int)items, slices);
   mlstm_chunk_state_kernel<<<g, NT, 0, st>>>(in, n_chunks, slices);
-  const dim3 gc((unsigned)(((int64_t)D * Dv + NT - 1) / NT + 1), H, R);
+  const dim3 gc((unsigned)(((int64_t)D * Dv + 4 * NT - 1) / (4 * NT) + 1), H, R);
   mlstm_chunk_carry_kernel<<<gc, NT, 0, st>>>(in, cs, S, nrm, mx);
   if (D <= 64) mlstm_chunk_out_kernel<4><<<g, NT, 0, st>>>(in, cs, R, mx, n_chunks, slices, out, os);
   else if (D <= 128) mlstm_chunk_out_kernel<8><<<g, NT, 0, st>>>(in, cs, R, mx, n_chunks, slices, out, os);

@@ -15,9 +15,11 @@
 // difference of two of them is good to its own last bit however long the chunk's sum has become. A token's exponent is held
 // at SSD_FLOOR or above: every decay over such a token is zero in fp32 either way, and the sums stay finite where A or dt do not.
 //
-// What bounds it: the chunks' contributions and entry states through memory (67 MB written, read and written by the
-// carry, read at 2048 tokens x 128 heads of 128 x 64) and the LDS reads of the split products. Measured there, one layer of a
-// step: 55 + 33 + 108 us; the token-by-token form in two passes over chunks of 256 took 2 x 1196 + 87 us.
+// What bounds it: a workgroup is a chain of loads, LDS exchanges and products, so as many of them on a CU as LDS allows: three, when the
+// registers are held to 168 (left to itself the compiler uses 200 and two fit). Beside that the chunks' contributions and entry
+// states through memory (67 MB written, read and written by the carry, read at 2048 tokens x 128 heads of 128 x 64). Measured there,
+// one layer of a step: 45 + 25 + 71 us; with two workgroups on a CU, the entry state loaded piece by piece, the sums formed twice
+// and the carry an element a thread 50 + 33 + 99. The token-by-token form in two passes over chunks of 256 took 2 x 1196 + 87 us.
 #include "chunk_common.h"
 
 namespace kafka {
@@ -36,14 +38,15 @@ struct SsdIn {
   const int* vseg;      // [chunks][4] = (first row, rows, -, -)
   float* U;             // [chunks][H][P][N]: own contribution, then entry state
   float* dec;           // [chunks][H]: e^(c_end)
+  float* sums;          // [chunks][H][3][CH]: what ssd_sums finds
 };
 
 constexpr double SSD_FLOOR = -1000.0;   // (e^-1000 is far below the smallest fp32 number)
 
 // The chunk's step sizes and running sums (times log2 e, as a float and what the float leaves out) by one wave; rows past n:
-// dt = 0, the sum stays.
+// dt = 0, the sum stays. They are kept (unless nullptr) for ssd_out, whose waves would wait for them (9 of its 100 us).
 __device__ __forceinline__ void ssd_sums(const SsdIn& in, int row0, int n, int h, int lane, float* dt_s, float* ch_s,
-                                         float* cl_s) {
+                                         float* cl_s, float* keep) {
   const float A = -expf(in.A_log[h]), bias = in.dt_bias[h];
   double c[2];
 #pragma unroll
@@ -57,6 +60,7 @@ __device__ __forceinline__ void ssd_sums(const SsdIn& in, int row0, int n, int h
       a = (double)A * (double)dt;
     }
     dt_s[t] = dt;
+    if (keep) keep[t] = dt;
     c[k] = a < SSD_FLOOR ? SSD_FLOOR : a;   // (NaN stays NaN)
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -69,8 +73,13 @@ __device__ __forceinline__ void ssd_sums(const SsdIn& in, int row0, int n, int h
   for (int k = 0; k < 2; ++k) {
     const double v = c[k] * 1.4426950408889634;
     const float hi = (float)v;
+    const float lo = (float)(v - (double)hi);
     ch_s[64 * k + lane] = hi;
-    cl_s[64 * k + lane] = (float)(v - (double)hi);
+    cl_s[64 * k + lane] = lo;
+    if (keep) {
+      keep[CH + 64 * k + lane] = hi;
+      keep[2 * CH + 64 * k + lane] = lo;
+    }
   }
 }
 
@@ -79,7 +88,7 @@ __device__ __forceinline__ float ssd_decay(float ha, float la, float hb, float l
   return fast_exp2((ha - hb) + (la - lb));
 }
 
-__global__ __launch_bounds__(NT) void ssd_state_kernel(SsdIn in, int n_chunks, int slices) {
+__global__ __launch_bounds__(NT, 3) void ssd_state_kernel(SsdIn in, int n_chunks, int slices) {
   __shared__ __attribute__((aligned(16))) bf16 Bt[DS * LDJ];
   __shared__ __attribute__((aligned(16))) bf16 Xt[VSL * LDJ];
   __shared__ __attribute__((aligned(16))) float f_s[CH];
@@ -91,7 +100,7 @@ __global__ __launch_bounds__(NT) void ssd_state_kernel(SsdIn in, int n_chunks, i
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int P = in.P, N = in.N, H = in.H, grp = h / (H / in.G);
   const bf16* rows = in.xbc + (int64_t)row0 * in.xs;
-  if (w == 0) ssd_sums(in, row0, n, h, lane, f_s, ch_s, cl_s);
+  if (w == 0) ssd_sums(in, row0, n, h, lane, f_s, ch_s, cl_s, slice == 0 ? in.sums + (int64_t)item * 3 * CH : nullptr);
   stage_transposed(rows + (int64_t)h * P, in.xs, n, v0, VSL, P, Xt, tid);
   for (int db = 0; db < N; db += DS) {
     if (db) __syncthreads();
@@ -137,56 +146,63 @@ __global__ __launch_bounds__(NT) void ssd_state_kernel(SsdIn in, int n_chunks, i
   if (slice == 0 && tid == 0) in.dec[item] = fast_exp2(ch_s[CH - 1] + cl_s[CH - 1]);
 }
 
-// grid (element blocks of P * N, H, segments): cs[r] = (first chunk, chunks, first position, state slot). A thread owns an
-// element of the state; the next four chunks' contributions are in flight while four are added up.
+// grid (blocks of 4 NT elements of P * N, H, segments): cs[r] = (first chunk, chunks, first position, state slot). A thread owns four
+// neighbouring elements of the state; the next chunks' contributions are in flight while PF are added up.
 __global__ __launch_bounds__(NT) void ssd_carry_kernel(SsdIn in, const int* __restrict__ cs, float* __restrict__ state) {
   const int r = blockIdx.z, h = blockIdx.y, N = in.N, P = in.P, H = in.H;
   const int first = cs[4 * r], last = first + cs[4 * r + 1], p0 = cs[4 * r + 2], slot = cs[4 * r + 3];
-  const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;   // element p * N + d
+  const int64_t i = 4 * ((int64_t)blockIdx.x * NT + threadIdx.x);   // element p * N + d (N is a multiple of 16)
   if (i >= (int64_t)P * N) return;
   const int p = (int)(i / N), d = (int)(i - (int64_t)p * N);
   float* st = state + (((int64_t)slot * H + h) * N + d) * P + p;
   float* el = in.U + (int64_t)h * P * N + i;
   const int64_t step = (int64_t)H * P * N;
-  float S = p0 > 0 ? *st : 0.f;
+  f32x4 S = {0.f, 0.f, 0.f, 0.f};
+  if (p0 > 0)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) S[e] = st[(int64_t)e * P];
+  auto at = [&](int c) { return reinterpret_cast<f32x4*>(el + (int64_t)c * step); };
   constexpr int PF = 4;
-  float u[PF];
+  f32x4 u[PF];
 #pragma unroll
-  for (int k = 0; k < PF; ++k) u[k] = first + k < last ? el[(int64_t)(first + k) * step] : 0.f;
+  for (int k = 0; k < PF; ++k)
+    if (first + k < last) u[k] = *at(first + k);
   for (int c0 = first; c0 < last; c0 += PF) {
-    float nx[PF];
+    f32x4 nx[PF];
 #pragma unroll
-    for (int k = 0; k < PF; ++k) nx[k] = c0 + PF + k < last ? el[(int64_t)(c0 + PF + k) * step] : 0.f;
+    for (int k = 0; k < PF; ++k)
+      if (c0 + PF + k < last) nx[k] = *at(c0 + PF + k);
 #pragma unroll
     for (int k = 0; k < PF; ++k)
       if (c0 + k < last) {
-        el[(int64_t)(c0 + k) * step] = S;                       // the chunk's entry state
+        *at(c0 + k) = S;                       // the chunk's entry state
         S = in.dec[(int64_t)(c0 + k) * H + h] * S + u[k];
       }
 #pragma unroll
     for (int k = 0; k < PF; ++k) u[k] = nx[k];
   }
-  *st = S;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) st[(int64_t)e * P] = S[e];
 }
 
 // NKS: 16-channel steps of a head's state rows held in registers (N <= 16 NKS; the steps past N multiply by zeros)
 template <int NKS>
-__global__ __launch_bounds__(NT) void ssd_out_kernel(SsdIn in, int n_chunks, int slices, const float* __restrict__ Dp,
+__global__ __launch_bounds__(NT, NKS <= 8 ? 3 : 2) void ssd_out_kernel(SsdIn in, int n_chunks, int slices, const float* __restrict__ Dp,
                                                      float* __restrict__ y, int64_t ys) {
   // one buffer, first for the entry state's three parts [3][VSL][DS + 8], then for the x columns [VSL][LDJ]
-  constexpr int LDD = DS + 8;
   typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
   __shared__ __attribute__((aligned(16))) bf16 buf[3 * VSL * LDD];
-  __shared__ float dt_s[CH], ch_s[CH], cl_s[CH];
+  __shared__ float sum_s[3 * CH];
+  const float *dt_s = sum_s, *ch_s = sum_s + CH, *cl_s = sum_s + 2 * CH;
   int item, slice;
   if (!chunk_item(n_chunks * in.H, slices, item, slice)) return;   // (uniform)
   const int ch = item / in.H, h = item - ch * in.H, v0 = slice * VSL;
   const int row0 = in.vseg[4 * ch], n = in.vseg[4 * ch + 1];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int P = in.P, N = in.N, H = in.H, nks = N >> 4, grp = h / (H / in.G);
   const bf16* rows = in.xbc + (int64_t)row0 * in.xs;
   const bf16* Bc = rows + (int64_t)H * P + (int64_t)grp * N + 8 * lh;
-  if (w == 0) ssd_sums(in, row0, n, h, lane, dt_s, ch_s, cl_s);
+  for (int i = tid; i < 3 * CH; i += NT) sum_s[i] = in.sums[(int64_t)item * 3 * CH + i];
   const int t = 32 * w + lr;                       // this lane's row
   const bf16* crow = Bc + (int64_t)in.G * N + (int64_t)min(t, n - 1) * in.xs;
   bf16x8 qf[NKS], kf[NKS];
@@ -200,7 +216,6 @@ __global__ __launch_bounds__(NT) void ssd_out_kernel(SsdIn in, int n_chunks, int
     qf[ks] = load_bf16x8(crow + 16 * min(ks, nks - 1));
     if (ks >= nks) qf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
   }
-  fetch_keys(0);
   f32x16 acc[2];
 #pragma unroll
   for (int vt = 0; vt < 2; ++vt)
@@ -208,25 +223,9 @@ __global__ __launch_bounds__(NT) void ssd_out_kernel(SsdIn in, int n_chunks, int
     for (int i = 0; i < 16; ++i) acc[vt][i] = 0.f;
   // ---- the entry state: acc = S_0^T C
   for (int db = 0; db < N; db += DS) {
-    const int nd = min(DS, N - db), d4s = nd >> 2;
+    const int nd = min(DS, N - db);
     if (db) __syncthreads();
-    for (int u = tid; u < VSL * d4s; u += NT) {
-      const int v = u / d4s, d = 4 * (u - v * d4s);
-      f32x4 x = {0.f, 0.f, 0.f, 0.f};
-      if (v0 + v < P) x = *reinterpret_cast<const f32x4*>(in.U + ((int64_t)item * P + v0 + v) * N + db + d);
-      bf16x4 p[3];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bf16 a = (bf16)x[e];
-        const float rr = x[e] - (float)a;
-        const bf16 b = (bf16)rr;
-        p[0][e] = a;
-        p[1][e] = b;
-        p[2][e] = (bf16)(rr - (float)b);
-      }
-#pragma unroll
-      for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x4*>(buf + (k * VSL + v) * LDD + d) = p[k];
-    }
+    stage_split(in.U + ((int64_t)item * P + v0) * N + db, N, nd, P - v0, buf, tid);
     __syncthreads();
     if (32 * w < n) {   // (uniform per wave)
 #pragma unroll
@@ -244,6 +243,7 @@ __global__ __launch_bounds__(NT) void ssd_out_kernel(SsdIn in, int n_chunks, int
       mfma_settle();
     }
   }
+  fetch_keys(0);
   __syncthreads();
   stage_transposed(rows + (int64_t)h * P, in.xs, n, v0, VSL, P, buf, tid);
   __syncthreads();
@@ -353,7 +353,7 @@ int kafka_hy_ssd_ok(int H, int P, int N, int G, int64_t xs) {
   return H >= 1 && G >= 1 && H % G == 0 && N >= 16 && N % 16 == 0 && N <= 256 && P >= 8 && P % 8 == 0 && xs % 8 == 0;
 }
 // floats of scratch per (chunk, head)
-int64_t kafka_hy_ssd_scratch(int P, int N) { return (int64_t)P * N + 1; }
+int64_t kafka_hy_ssd_scratch(int P, int N) { return (int64_t)P * N + 1 + 3 * CH; }
 
 // the segments of cs in chunks (vseg: all their chunks in order)
 hipError_t kafka_hy_ssd_scan(const void* xbc, int64_t xs, const void* dt, int64_t ds, const float* dt_bias,
@@ -364,10 +364,11 @@ hipError_t kafka_hy_ssd_scan(const void* xbc, int64_t xs, const void* dt, int64_
   const int64_t items = (int64_t)n_chunks * H;
   const int slices = (P + VSL - 1) / VSL;
   if ((items + 8) * slices > 0x7fffffff) return hipErrorInvalidValue;
-  SsdIn in{(const bf16*)xbc, xs, (const bf16*)dt, ds, dt_bias, A_log, H, P, N, G, vseg, scratch, scratch + items * P * N};
+  SsdIn in{(const bf16*)xbc, xs, (const bf16*)dt, ds, dt_bias, A_log, H, P, N, G, vseg, scratch, scratch + items * P * N,
+           scratch + items * ((int64_t)P * N + 1)};
   const unsigned g = (unsigned)chunk_grid((int)items, slices);
   ssd_state_kernel<<<g, NT, 0, st>>>(in, n_chunks, slices);
-  ssd_carry_kernel<<<dim3((unsigned)(((int64_t)P * N + NT - 1) / NT), H, R), NT, 0, st>>>(in, cs, state);
+  ssd_carry_kernel<<<dim3((unsigned)(((int64_t)P * N + 4 * NT - 1) / (4 * NT)), H, R), NT, 0, st>>>(in, cs, state);
   if (N <= 64) ssd_out_kernel<4><<<g, NT, 0, st>>>(in, n_chunks, slices, Dp, y, ys);
   else if (N <= 128) ssd_out_kernel<8><<<g, NT, 0, st>>>(in, n_chunks, slices, Dp, y, ys);
   else ssd_out_kernel<16><<<g, NT, 0, st>>>(in, n_chunks, slices, Dp, y, ys);

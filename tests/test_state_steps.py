@@ -110,3 +110,61 @@ def test_memory_step(D, Dv, dtype):
         close(out[t].view(H, Dv), num / den[:, None], 1.01 * (dn / den[:, None] + (num / den[:, None]).abs() * (dd / den)[:, None]) +
               8 * EPS * (num / den[:, None]).abs())
     assert torch.equal(gS[0].cpu(), S[0])
+
+
+@pytest.mark.parametrize("n,p0", [(128 * 4 + 1, 0), (128 * 9 + 5, 7), (128 * 12, 3)])   # chunks that the carry asks for in one, three and three goes
+def test_chunks_carried(n, p0):
+    """Segments of more chunks than the carry keeps in flight, against 64-bit sums. A result is a sum of at most 128 rows, 128 channels
+    and one entry state per chunk in fp32: as many roundings of the sum of its parts' magnitudes, and a few for each decay."""
+    torch.manual_seed(n)
+    H, P, N, D, Dv, cap, dev = 2, 24, 32, 32, 40, 6.0, "cuda:0"
+    seg, tok = torch.tensor([(0, n, p0, 1)], dtype=torch.int32), torch.zeros(n, dtype=torch.int32, device=dev)
+    bound = (128 + 128 + n // 128 + 40) * EPS
+
+    xbc, proj = (torch.randn(n, H * P + 2 * N) / 2).bfloat16(), torch.randn(n, H).bfloat16()
+    bias, A, Dp = torch.randn(H) - 4, torch.rand(H) - 2, torch.randn(H)
+    state, y = torch.randn(2, H, N, P), torch.empty(n, H * P, device=dev)
+    gs = state.cuda()
+    tabs = tuple(torch.from_numpy(t).to(dev) for t in hops.chunk_tables(seg.numpy(), hops.SSD_CHUNK, hops.SSD_CHUNK_MIN))
+    hops.ssm_scan(xbc.cuda(), proj.cuda(), 0, bias.cuda(), A.cuda(), Dp.cuda(), H, P, N, 1, tok, seg.cuda(), gs, y, chunks=tabs, rows=None)
+    S = state[1].double() * (p0 > 0)
+    mag = S.abs()
+    want, most = [], []
+    for t in range(n):
+        x = xbc[t].double()
+        xv, B, C = x[:H * P].view(H, P), x[H * P:H * P + N], x[H * P + N:]
+        dt = torch.nn.functional.softplus(proj[t].double() + bias.double())
+        dec, new = torch.exp(-torch.exp(A.double()) * dt)[:, None, None], B[None, :, None] * (dt[:, None] * xv)[:, None]
+        S, mag = dec * S + new, dec * mag + new.abs()
+        want.append((S * C[:, None]).sum(1) + Dp.double()[:, None] * xv)
+        most.append((mag * C.abs()[:, None]).sum(1) + (Dp.double()[:, None] * xv).abs())
+    close(y.view(n, H, P), torch.stack(want), bound * torch.stack(most))
+    close(gs[1], S, bound * mag)
+
+    qkv, gates = torch.randn(n, H * (2 * D + Dv)).bfloat16(), 4 * torch.randn(n, 2 * H)
+    M, nrm, mx = torch.randn(2, H, D, Dv), torch.randn(2, H, D), torch.randn(2, H)
+    gM, gn, gm, out = M.cuda(), nrm.cuda(), mx.cuda(), torch.empty(n, H * Dv, device=dev)
+    tabs = tuple(torch.from_numpy(t).to(dev) for t in hops.chunk_tables(seg.numpy(), hops.MLSTM_CHUNK, hops.MLSTM_CHUNK_MIN))
+    hops.mlstm_scan(qkv.cuda(), gates.cuda(), H, D, Dv, cap, tok, seg.cuda(), gM, gn, gm, out, chunks=tabs, rows=None)
+    S, v0, m = (a[1].double() * (p0 > 0) for a in (M, nrm, mx))
+    magS, magn = S.abs(), v0.abs()
+    want, most = [], []
+    for t in range(n):
+        x = qkv[t].double()
+        q, k, v = x[:H * D].view(H, D) * D ** -0.5, x[H * D:2 * H * D].view(H, D), x[2 * H * D:].view(H, Dv)
+        c = cap * torch.tanh(gates[t].double() / cap)
+        ig, fg = c[:H], torch.nn.functional.logsigmoid(c[H:])
+        m1 = torch.maximum(fg + m, ig)
+        dec, gain, m = torch.exp(fg + m - m1), torch.exp(ig - m1), m1
+        kv = gain[:, None, None] * k[:, :, None] * v[:, None]
+        S, magS = dec[:, None, None] * S + kv, dec[:, None, None] * magS + kv.abs()
+        v0, magn = dec[:, None] * v0 + gain[:, None] * k, dec[:, None] * magn + gain[:, None] * k.abs()
+        den = torch.maximum((v0 * q).sum(1).abs(), torch.exp(-m)) + 1e-6
+        o = (S * q[:, :, None]).sum(1) / den[:, None]
+        want.append(o)
+        # (a log gate's roundings, a few of cap, enter as an exponent's; running sums of 128 of them as 128)
+        most.append(((magS * q.abs()[:, :, None]).sum(1) + o.abs() * (magn * q.abs()).sum(1)[:, None]) / den[:, None] + o.abs())
+    gate = bound + 128 * 2 * cap * EPS
+    close(out.view(n, H, Dv), torch.stack(want), gate * torch.stack(most))
+    close(gM[1], S, gate * magS)
+    close(gn[1], v0, gate * magn)

@@ -370,237 +370,46 @@ __global__ __launch_bounds__(NT) void window_attn_kernel(const AT* __restrict__ 
 }
 
 // ---- windowed softmax attention on the matrix cores (bf16) --------------------------------------------------------
-// One workgroup (4 waves) per (tile, key/value head): a tile is 32 query rows = (token, query head of this key/value
-// head) pairs of consecutive tokens of one segment (floor(32 / rep) tokens, rep = H / G query heads per key/value
-// head). Keys go by in blocks of 128, from the block that holds the first key the tile's first row sees:
-//   scores   wave w takes keys 32 w .. 32 w + 31 of the block: S = Q K^T as D / 16 MFMA steps (32x32x16), the Q tile
-//            read from LDS, the key rows straight from the paged cache (lane = key, 16 bytes per step), the next
-//            block's rows requested before this block's softmax;
-//   softmax  keys ahead of the row or behind its window count as -inf; row maxima within the wave by lane exchange
-//            and across the four waves through LDS; P = 2^(S - m) goes to LDS as bf16; the row sums stay per lane
-//            and are combined once at the end;
-//   values   wave w owns output columns [32 TW w, 32 TW (w + 1)): O += P V with V read from the page-wise transposed
-//            values (lane = column, 8 consecutive keys = 16 bytes), one page per MFMA step.
-// Scores, maxima, sums and accumulators are fp32. The sink joins the denominator once, at the end. With
-// gridDim.z > 1 the tile's key blocks are dealt to gridDim.z workgroups in contiguous ranges; each leaves its
-// unnormalised accumulators in po [z][T][H Dv] and (row maximum, row sum) in pml [z][T][H][2] for window_merge.
-// Needs 16-token pages, D % 16 == 0, at most 32 query heads per key/value head.
-// What bounds it: a block's chain of key loads, maxima, weights and value loads. A decoded token fills few of the 32 rows, and
-// the others' softmax is left out (their weights in LDS stay zero); maxima go lane to lane without LDS. With the merge, operands from
-// memory, before / now, us: 16 sequences x 1700 keys, 32 heads over 8, 61 / 57, 64 sequences 159 / 153, one x 8000 50 / 37,
-// 16 sequences, 32 over 2, 32 / 27 (from a warm cache 43 / 34, 111 / 105, 45 / 28, 27 / 22).
-constexpr int WM_ROWS = 32;
-
-// the largest of a lane half's 32 values, in each of its lanes: neighbours, pairs, mirrored eights and sixteens, the other sixteen
-__device__ __forceinline__ float max32(float v) {
-  auto dpp = [](float x, auto c) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(c)::value, 0xf, 0xf, false));
-  };
-  v = fmaxf(v, dpp(v, std::integral_constant<int, 0xB1>()));
-  v = fmaxf(v, dpp(v, std::integral_constant<int, 0x4E>()));
-  v = fmaxf(v, dpp(v, std::integral_constant<int, 0x141>()));
-  v = fmaxf(v, dpp(v, std::integral_constant<int, 0x140>()));
-  return fmaxf(v, __shfl_xor(v, 16, 64));
-}
-
-template <int TW, int NKSC>
-__global__ __launch_bounds__(256) void window_attn_mfma_kernel(
-    const bf16* __restrict__ q, int64_t qs, const bf16* __restrict__ kc, const bf16* __restrict__ vt,
-    const int* __restrict__ bt, int bt_stride, const int* __restrict__ items, const int64_t* __restrict__ positions,
-    int H, int G, int D, int Dv, int Ck, int kstep, float scale_log2e, int window, const float* __restrict__ sink,
-    const bf16* __restrict__ gate, int64_t gs, bf16* __restrict__ out, int64_t os, float* __restrict__ po,
-    float* __restrict__ pml, int64_t T, float out_scale, int max_tok) {
-  // (D, Ck, kstep as in window_attn_kernel: kstep = 0 and D = Ck when every query row meets the whole key row)
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int nks = D >> 4, qstride = D + 8;
-  bf16* Qs = reinterpret_cast<bf16*>(smem);                       // [32][D + 8]
-  bf16* Ps = Qs + WM_ROWS * qstride;                              // [32][128 + 8]
-  float* mloc = reinterpret_cast<float*>(Ps + WM_ROWS * 136);     // [4][32]
-  int* prow_s = reinterpret_cast<int*>(mloc + 4 * WM_ROWS);       // [32]
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 31, lh = lane >> 5;
-  const int t0 = items[4 * blockIdx.x], ntok = items[4 * blockIdx.x + 1], sg = items[4 * blockIdx.x + 2];
-  if (ntok > max_tok) return;   // (uniform) an item of window_attn_rows
-  const int g = blockIdx.y, rep = H / G;
-  const int nrows = ntok * rep;
-  for (int i = threadIdx.x; i < WM_ROWS * 136 / 8; i += 256) store_bf16x8(Ps + 8 * i, bf16x8{0, 0, 0, 0, 0, 0, 0, 0});
-  for (int i = threadIdx.x; i < WM_ROWS * (D >> 3); i += 256) {
-    const int r = i / (D >> 3), d0 = (i - r * (D >> 3)) << 3;
-    bf16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (r < nrows) v = load_bf16x8(q + (int64_t)(t0 + r / rep) * qs + (int64_t)(g * rep + r % rep) * D + d0);
-    store_bf16x8(Qs + r * qstride + d0, v);
-  }
-  // a row beyond the tile sees no key
-  if (threadIdx.x < WM_ROWS) prow_s[threadIdx.x] = threadIdx.x < nrows ? (int)positions[t0 + threadIdx.x / rep] : -1;
-  const int maxpos = (int)positions[t0 + ntok - 1];
-  __syncthreads();
-  int prow[16];
-  float m[16], lsum[16];
-  f32x16 O[TW];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    prow[i] = prow_s[(i & 3) + 8 * (i >> 2) + 4 * lh];
-    m[i] = -INFINITY;
-    lsum[i] = 0.f;
-  }
-#pragma unroll
-  for (int tw = 0; tw < TW; ++tw)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) O[tw][i] = 0.f;
-  const int* btr = bt + (int64_t)sg * bt_stride;
-  const int Cv = G * Dv;
-  const int nblocks = (maxpos >> 7) + 1;
-  const int kbmin = window > 0 ? max(0, (int)positions[t0] - window + 1) >> 7 : 0;
-  const bf16* qrow = Qs + lr * qstride + 8 * lh;
-  bf16x8 kf[NKSC];
-  auto fetch_keys = [&](int kb) {
-    const int kcix = min(kb * 128 + 32 * w + lr, maxpos);  // past the tile's last position: a valid row, masked below
-    const bf16* krow = kc + ((int64_t)btr[kcix >> 4] * PAGE + (kcix & 15)) * Ck + (int64_t)g * kstep + 8 * lh;
-#pragma unroll
-    for (int ks = 0; ks < NKSC; ++ks)
-      if (ks < nks) kf[ks] = load_bf16x8(krow + 16 * ks);
-  };
-  const int nsplit = gridDim.z;
-  const int bps = (nblocks - kbmin + nsplit - 1) / nsplit;
-  const int kb0 = kbmin + blockIdx.z * bps, kb1 = min(nblocks, kb0 + bps);
-  if (kb0 < kb1 && kb0 * 128 + 32 * w <= maxpos) fetch_keys(kb0);
-  for (int kb = kb0; kb < kb1; ++kb) {
-    const int key = kb * 128 + 32 * w + lr;
-    f32x16 S;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) S[i] = 0.f;
-    const bool any = kb * 128 + 32 * w <= maxpos;  // (uniform per wave)
-    if (any) {
-#pragma unroll
-      for (int ks = 0; ks < NKSC; ++ks)
-        if (ks < nks) S = mfma32(load_bf16x8(qrow + 16 * ks), kf[ks], S);
-    }
-    if (kb + 1 < kb1 && (kb + 1) * 128 + 32 * w <= maxpos) fetch_keys(kb + 1);
-    float s[16], mx[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      if (8 * (i >> 2) >= nrows) break;   // (uniform) a decoded token has few rows
-      s[i] = (any && key <= prow[i] && (window == 0 || key > prow[i] - window)) ? S[i] * scale_log2e : -INFINITY;
-      mx[i] = max32(s[i]);
-    }
-    if (lr == 0) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        if (8 * (i >> 2) >= nrows) break;
-        mloc[w * 32 + (i & 3) + 8 * (i >> 2) + 4 * lh] = mx[i];
-      }
-    }
-    lds_barrier();
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      if (8 * (i >> 2) >= nrows) break;
-      const int r = (i & 3) + 8 * (i >> 2) + 4 * lh;
-      const float mn = fmaxf(fmaxf(m[i], fmaxf(mloc[r], mloc[32 + r])), fmaxf(mloc[64 + r], mloc[96 + r]));
-      // first block: m = -inf -> corr 0. A range may lie wholly outside a row's window: then mn is still -inf and
-      // the row stays empty (the guards keep inf - inf out)
-      const float corr = mn == -INFINITY ? 0.f : fast_exp2(m[i] - mn);
-      const float p = mn == -INFINITY ? 0.f : fast_exp2(s[i] - mn);
-      lsum[i] = lsum[i] * corr + p;
-      m[i] = mn;
-      Ps[r * 136 + 32 * w + lr] = (bf16)p;
-#pragma unroll
-      for (int tw = 0; tw < TW; ++tw) O[tw][i] *= corr;
-    }
-    lds_barrier();
-    // ---- values: one page (16 keys) per step
-#pragma unroll
-    for (int k0 = 0; k0 < 8; k0 += 4) {
-      bf16x8 vf[4][TW];  // four pages' value operands in flight together
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        if ((kb * 8 + k0 + kk) * 16 > maxpos) break;  // (uniform) pages past the last position
-        const bf16* vp = vt + ((int64_t)btr[kb * 8 + k0 + kk] * Cv + (int64_t)g * Dv) * PAGE + 8 * lh;
-#pragma unroll
-        for (int tw = 0; tw < TW; ++tw) {
-          const int col = (w * TW + tw) * 32 + lr;
-          bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-          vf[kk][tw] = col < Dv ? load_bf16x8(vp + (int64_t)col * PAGE) : z;
-        }
-      }
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        if ((kb * 8 + k0 + kk) * 16 > maxpos) break;
-        const bf16x8 a = load_bf16x8(Ps + lr * 136 + 16 * (k0 + kk) + 8 * lh);
-#pragma unroll
-        for (int tw = 0; tw < TW; ++tw)
-          if ((w * TW + tw) * 32 < Dv) O[tw] = mfma32(a, vf[kk][tw], O[tw]);
-      }
-    }
-    lds_barrier();
-  }
-  // ---- row sums: across the lanes of a half, then across the waves
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    float v = lsum[i];
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    lsum[i] = v;
-  }
-  if (lr == 0) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) mloc[w * 32 + (i & 3) + 8 * (i >> 2) + 4 * lh] = lsum[i];
-  }
-  lds_barrier();
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int r = (i & 3) + 8 * (i >> 2) + 4 * lh;
-    if (r >= nrows) continue;
-    float l = mloc[r] + mloc[32 + r] + mloc[64 + r] + mloc[96 + r];
-    const int64_t t = t0 + r / rep;
-    const int h = g * rep + r % rep;
-    if (nsplit == 1) {
-      if (sink != nullptr) l += fast_exp2(sink[h] * LOG2E - m[i]);
-      float inv = out_scale / l;
-      if (gate != nullptr) inv *= head_gate(gate + t * gs + h);
-#pragma unroll
-      for (int tw = 0; tw < TW; ++tw) {
-        const int col = (w * TW + tw) * 32 + lr;
-        if (col < Dv) out[t * os + (int64_t)h * Dv + col] = (bf16)(O[tw][i] * inv);
-      }
-    } else {
-      const int64_t row = ((int64_t)blockIdx.z * T + t) * H + h;
-      if (w == 0 && lr == 0) {
-        pml[2 * row] = m[i];
-        pml[2 * row + 1] = l;
-      }
-#pragma unroll
-      for (int tw = 0; tw < TW; ++tw) {
-        const int col = (w * TW + tw) * 32 + lr;
-        if (col < Dv) po[row * Dv + col] = O[tw][i];
-      }
-    }
-  }
-}
-
-// ---- the same for prompt portions: a wave per item ------------------------------------------------------------------
-// A wave takes one item's 32 (token, head) rows of one key/value head and walks their keys 32 at a time:
+// An item is 32 query rows = (token, query head) pairs of consecutive tokens of one segment for one key/value head
+// (floor(32 / rep) tokens, rep = H / G query heads per key/value head). A wave walks keys 32 at a time:
 //   scores   S^T = K Q^T: lane = row, a lane's 16 registers = its half of the block's keys. The key rows are loaded with
 //            bits 2 and 3 of their numbers swapped, which leaves lane half lh with keys 8 lh .. + 7 of each page;
 //   softmax  a row's maximum, sum and weights live in its two lanes; the accumulators are rescaled only when a row's
 //            maximum has moved;
 //   values   O^T += V^T P^T: the weights are the right operand as they lie in the registers, the left one is a channel's
 //            8 consecutive tokens of a transposed page (16 bytes).
-// No LDS and no barriers; the four waves of a workgroup are neighbouring items (the same keys, from the cache), a key/value
-// head's workgroups go to one XCD where there are eight of them, the items with the most keys first. NKS, NVT: steps of
-// 16 key channels and tiles of 32 value channels held in registers (queries past D are zero).
-template <int NKS, int NVT>
+// Keys ahead of the row or behind its window count as -inf; scores, maxima, sums and accumulators are fp32; the sink joins the
+// denominator once, at the end. Needs 16-token pages, D % 16 == 0, at most 32 query heads per key/value head. NKS, NVT: steps of 16
+// key channels and tiles of 32 value channels held in registers (queries past D are zero).
+//   prompt portions: a wave per item, no LDS and no barriers; the four waves of a workgroup are neighbouring items (the same
+//     keys, from the cache), a key/value head's workgroups go to one XCD where there are eight of them, the items with the most
+//     keys first.
+//   SPLIT, decoded tokens: a workgroup per item (one key/value head's side by side), its blocks of keys dealt to the four waves in turn, the waves' maxima, sums and
+//     accumulators met in LDS at the end. With gridDim.z > 1 the item's blocks are dealt to that many workgroups in contiguous
+//     ranges; each leaves its unnormalised accumulators in po [z][T][H Dv] and (row maximum, row sum) in pml [z][T][H][2] for
+//     window_merge. What bounds it: the round trips of a block, which is why no wave waits for another in the walk: with the scores
+//     of 128 keys shared through LDS, three barriers a block and the values asked for behind them, us (operands from memory, with the
+//     merge; before / now): 16 sequences x 1700 keys, 32 heads over 8, 38 / 28, 64 sequences 102 / 86 (4.6 TB/s), one x 8000 28 / 19, 128 x
+//     300 43 / 34; 32 over 2, 128 x 1700, 70 / 44; 64 channels, 64 x 1700, 65 / 46; 256 channels, 16 over 4, 16 x 1700 52 / 34. Two
+//     blocks in flight a wave (one wave a SIMD) 31, 84, 21, 48, 47, 47, 37; past the caches' retention 42, 110, 28, 42 (a line
+//     of keys is four loads).
+constexpr int WM_ROWS = 32;
+
+template <int NKS, int NVT, bool SPLIT>
 __global__ __launch_bounds__(256, NKS * 4 + NVT * 16 <= 96 ? 2 : 1) void window_attn_rows_kernel(
     const bf16* __restrict__ q, int64_t qs, const bf16* __restrict__ kc, const bf16* __restrict__ vt,
     const int* __restrict__ bt, int bt_stride, const int* __restrict__ items, int n_items,
     const int64_t* __restrict__ positions, int H, int G, int D, int Dv, int Ck, int kstep, float scale_log2e, int window,
     const float* __restrict__ sink, const bf16* __restrict__ gate, int64_t gs, bf16* __restrict__ out, int64_t os,
-    float out_scale, int min_tok, bool vec4) {
-  const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
+    float out_scale, int tok_lim, bool vec4, float* __restrict__ po, float* __restrict__ pml, int64_t T) {
+  constexpr int STEP = SPLIT ? 4 : 1;   // blocks from a wave's one to its next
+  const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int item = __builtin_amdgcn_readfirstlane(
-      n_items - 1 - ((int)blockIdx.y * (int)(blockDim.x >> 6) + (int)(threadIdx.x >> 6)));
-  if (item < 0) return;   // whole waves leave; nothing below synchronises across waves
+      SPLIT ? (int)(blockIdx.x % (unsigned)n_items) : n_items - 1 - ((int)blockIdx.y * (int)(blockDim.x >> 6) + (int)(threadIdx.x >> 6)));
+  if (item < 0) return;   // whole waves leave; nothing below synchronises across waves unless SPLIT
   const int t0 = items[4 * item], ntok = items[4 * item + 1], sg = items[4 * item + 2];   // (uniform)
-  if (ntok < min_tok) return;
-  const int g = blockIdx.x, rep = H / G, nks = D >> 4, nrows = ntok * rep;
+  if (SPLIT ? ntok > tok_lim : ntok < tok_lim) return;   // (an item of the other form)
+  const int g = SPLIT ? blockIdx.x / (unsigned)n_items : blockIdx.x, rep = H / G, nks = D >> 4, nrows = ntok * rep;
   const bool live = lr < nrows;
   const int row = min(lr, nrows - 1), h = g * rep + row % rep;
   const int64_t t = t0 + row / rep;
@@ -628,11 +437,17 @@ __global__ __launch_bounds__(256, NKS * 4 + NVT * 16 <= 96 ? 2 : 1) void window_
   for (int v = 0; v < NVT; ++v)
 #pragma unroll
     for (int i = 0; i < 16; ++i) O[v][i] = 0.f;
-  const int kb0 = window > 0 ? max(0, minpos - window + 1) >> 5 : 0, kb1 = (maxpos >> 5) + 1;
-  int pa = page_of(kb0, 0), pb = page_of(kb0, 1), na = page_of(kb0 + 1, 0), nb = page_of(kb0 + 1, 1);
+  int kb0 = window > 0 ? max(0, minpos - window + 1) >> 5 : 0, kb1 = (maxpos >> 5) + 1;
+  if constexpr (SPLIT) {   // of the z-th of gridDim.z ranges, every fourth
+    const int per = (kb1 - kb0 + (int)gridDim.z - 1) / (int)gridDim.z;
+    kb0 += (int)blockIdx.z * per;
+    kb1 = min(kb1, kb0 + per);
+    kb0 += w;
+  }
+  int pa = page_of(kb0, 0), pb = page_of(kb0, 1), na = page_of(kb0 + STEP, 0), nb = page_of(kb0 + STEP, 1);
   fetch_keys(pa, pb);
-  for (int kb = kb0; kb < kb1; ++kb) {
-    const int fa = page_of(kb + 2, 0), fb = page_of(kb + 2, 1);   // (two blocks ahead)
+  for (int kb = kb0; kb < kb1; kb += STEP) {
+    const int fa = page_of(kb + 2 * STEP, 0), fb = page_of(kb + 2 * STEP, 1);   // (two blocks ahead)
     bf16x8 vf[2][NVT];
 #pragma unroll
     for (int pg = 0; pg < 2; ++pg) {
@@ -693,6 +508,51 @@ __global__ __launch_bounds__(256, NKS * 4 + NVT * 16 <= 96 ? 2 : 1) void window_
   asm volatile("s_nop 15");
   __builtin_amdgcn_sched_barrier(0);
   l += __shfl_xor(l, 32, 64);
+  if constexpr (SPLIT) {
+    constexpr int LO = 32 * NVT + 4;
+    __shared__ __attribute__((aligned(16))) float part[4 * WM_ROWS * LO];   // [wave][row]
+    __shared__ float ml[4][WM_ROWS][2];
+    if (live) {
+      if (lh == 0) {
+        ml[w][lr][0] = m;
+        ml[w][lr][1] = l;
+      }
+#pragma unroll
+      for (int v = 0; v < NVT; ++v)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4)
+          *reinterpret_cast<f32x4*>(part + (w * WM_ROWS + lr) * LO + 32 * v + 8 * i4 + 4 * lh) =
+              f32x4{O[v][4 * i4], O[v][4 * i4 + 1], O[v][4 * i4 + 2], O[v][4 * i4 + 3]};
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < nrows * Dv; i += 256) {
+      const int r = i / Dv, c = i - r * Dv, hr = g * rep + r % rep;
+      const int64_t tr = t0 + r / rep;
+      const float mn = fmaxf(fmaxf(ml[0][r][0], ml[1][r][0]), fmaxf(ml[2][r][0], ml[3][r][0]));
+      // (a range may lie wholly outside a row's window: then mn is -inf and the row stays empty)
+      float o = 0.f, lt = 0.f;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float f = ml[k][r][0] == -INFINITY ? 0.f : fast_exp2(ml[k][r][0] - mn);
+        lt += f * ml[k][r][1];
+        o += f * part[(k * WM_ROWS + r) * LO + c];
+      }
+      if (gridDim.z == 1) {
+        if (sink != nullptr) lt += fast_exp2(sink[hr] * LOG2E - mn);
+        float inv = out_scale / lt;
+        if (gate != nullptr) inv *= head_gate(gate + tr * gs + hr);
+        out[tr * os + (int64_t)hr * Dv + c] = (bf16)(o * inv);
+      } else {
+        const int64_t at = ((int64_t)blockIdx.z * T + tr) * H + hr;
+        if (c == 0) {
+          pml[2 * at] = mn;
+          pml[2 * at + 1] = lt;
+        }
+        po[at * Dv + c] = o;
+      }
+    }
+    return;
+  }
   if (!live) return;
   if (sink != nullptr) l += fast_exp2(sink[h] * LOG2E - m);
   float inv = out_scale / l;
@@ -1245,7 +1105,7 @@ hipError_t kafka_hy_window_attn_mfma(const void* q, int64_t qs, const void* kc, 
     auto b = [&](auto k) {
       k<<<gr, 64 * waves, 0, st>>>((const bf16*)q, qs, (const bf16*)kc, (const bf16*)vt, bt, bt_stride, items, n_items,
                                    positions, H, G, D, Dv, Ck, kstep, scale * LOG2E, window, sink, (const bf16*)gate, gs,
-                                   (bf16*)out, os, out_scale, min_rows_tok, vec4);
+                                   (bf16*)out, os, out_scale, min_rows_tok, vec4, nullptr, nullptr, T);
     };
     const bool al = ((reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vt)) & 15) == 0;
     if (D == 128 && Dv == 128 && al && scale > 0.f && (int64_t)tile_items * G >= WT_MIN_WAVES) {
@@ -1253,34 +1113,34 @@ hipError_t kafka_hy_window_attn_mfma(const void* q, int64_t qs, const void* kc, 
           (const bf16*)q, qs, (const bf16*)kc, (const bf16*)vt, bt, bt_stride, items, n_items, positions, H, G, Ck, kstep,
           scale * LOG2E, window, sink, (const bf16*)gate, gs, (bf16*)out, os, out_scale, min_rows_tok, vec4);
     } else if (D <= 64) {
-      if (Dv <= 64) b(window_attn_rows_kernel<4, 2>);
-      else if (Dv <= 128) b(window_attn_rows_kernel<4, 4>);
-      else b(window_attn_rows_kernel<4, 8>);
+      if (Dv <= 64) b(window_attn_rows_kernel<4, 2, false>);
+      else if (Dv <= 128) b(window_attn_rows_kernel<4, 4, false>);
+      else b(window_attn_rows_kernel<4, 8, false>);
     } else if (D <= 128) {
-      if (Dv <= 64) b(window_attn_rows_kernel<8, 2>);
-      else if (Dv <= 128) b(window_attn_rows_kernel<8, 4>);
-      else b(window_attn_rows_kernel<8, 8>);
+      if (Dv <= 64) b(window_attn_rows_kernel<8, 2, false>);
+      else if (Dv <= 128) b(window_attn_rows_kernel<8, 4, false>);
+      else b(window_attn_rows_kernel<8, 8, false>);
     } else {
-      if (Dv <= 64) b(window_attn_rows_kernel<16, 2>);
-      else if (Dv <= 128) b(window_attn_rows_kernel<16, 4>);
-      else b(window_attn_rows_kernel<16, 8>);
+      if (Dv <= 64) b(window_attn_rows_kernel<16, 2, false>);
+      else if (Dv <= 128) b(window_attn_rows_kernel<16, 4, false>);
+      else b(window_attn_rows_kernel<16, 8, false>);
     }
   }
   if (max_tok <= 0) return hipGetLastError();
   if (nsplit > 1 && min_rows_tok > 0) return hipErrorInvalidValue;   // (the merge pass takes every row)
-  const size_t lds = (size_t)WM_ROWS * (D + 8) * 2 + WM_ROWS * 136 * 2 + 5 * WM_ROWS * 4;
-  const dim3 grid((unsigned)n_items, (unsigned)G, (unsigned)nsplit);
+  const dim3 grid((unsigned)n_items * (unsigned)G, 1, (unsigned)nsplit);
   auto a = [&](auto k) {
-    k<<<grid, 256, lds, st>>>((const bf16*)q, qs, (const bf16*)kc, (const bf16*)vt, bt, bt_stride, items, positions, H,
-                              G, D, Dv, Ck, kstep, scale * LOG2E, window, sink, (const bf16*)gate, gs, (bf16*)out, os, po, pml,
-                              T, out_scale, max_tok);
+    k<<<grid, 256, 0, st>>>((const bf16*)q, qs, (const bf16*)kc, (const bf16*)vt, bt, bt_stride, items, n_items, positions, H, G, D,
+                            Dv, Ck, kstep, scale * LOG2E, window, sink, (const bf16*)gate, gs, (bf16*)out, os, out_scale, max_tok,
+                            false, po, pml, T);
   };
-  const int nks = D / 16, tw = ((Dv + 31) / 32 + 3) / 4;
-  if (tw == 1 && nks <= 4) a(window_attn_mfma_kernel<1, 4>);
-  else if (tw == 1 && nks <= 8) a(window_attn_mfma_kernel<1, 8>);
-  else if (tw == 1) a(window_attn_mfma_kernel<1, 16>);
-  else if (nks <= 8) a(window_attn_mfma_kernel<2, 8>);
-  else a(window_attn_mfma_kernel<2, 16>);
+  auto by_dv = [&](auto k2, auto k4, auto k8) { Dv <= 64 ? a(k2) : Dv <= 128 ? a(k4) : a(k8); };
+  if (D <= 64)
+    by_dv(window_attn_rows_kernel<4, 2, true>, window_attn_rows_kernel<4, 4, true>, window_attn_rows_kernel<4, 8, true>);
+  else if (D <= 128)
+    by_dv(window_attn_rows_kernel<8, 2, true>, window_attn_rows_kernel<8, 4, true>, window_attn_rows_kernel<8, 8, true>);
+  else
+    by_dv(window_attn_rows_kernel<16, 2, true>, window_attn_rows_kernel<16, 4, true>, window_attn_rows_kernel<16, 8, true>);
   if (nsplit > 1)
     window_merge_kernel<<<(unsigned)(T * H), 64, 0, st>>>(po, pml, nsplit, T, H, Dv, sink, (const bf16*)gate, gs,
                                                           (bf16*)out, os, out_scale);

@@ -801,8 +801,14 @@ def qk_norm_rope_store(qkv, H: int, G: int, D: int, Dv: int, q_w, k_w, eps, posi
                                lam, k_cache, v_cache_t, slot_mapping, q_out)
 
 
-WINDOW_SPLIT_WGS = 512    # workgroups a windowed-attention launch is split towards (two per CU) ...
-SHARED_SPLIT_WGS = 1024   # ... and one with shared keys
+WINDOW_SPLIT_WGS = 256    # workgroups a windowed-attention launch of decoded tokens is split towards (one per CU)
+
+
+def window_splits(wgs: int, max_keys: int) -> int:
+    """Key-range splits of a windowed-attention launch of ``wgs`` workgroups, each of at least two blocks of 128 keys.
+    One a CU: more are more partial sums of shorter walks (16 sequences of 1700 keys, 32 heads over 8, us with the merge: two splits 28, four
+    33, one 31; 256 channels, 16 heads over 4, four splits 34, eight 43, two 40)."""
+    return max(1, min(SIG_SPLIT_MAX, WINDOW_SPLIT_WGS // max(1, wgs), -(-max_keys // 128) // 2))
 
 
 def window_attn_mfma_ok(q, k_cache, v_cache_t, H: int, G: int, shared_keys: bool = False) -> bool:
@@ -860,9 +866,7 @@ def window_attn(q, k_cache, v_cache_t, block_tables, tok_seg, positions, H: int,
             share = shared_items(q.shape[0], tiles.shape[0], tt, kinds, max_keys) if kinds[1] else 0
             if window and max_keys:  # a tile's key range is at most the window and its own tokens long
                 max_keys = min(max_keys, window + tt)
-            # (shared keys: few key/value heads, every workgroup walks the whole key row - more, shorter ranges)
-            ns = sig_splits(tiles.shape[0] * G, max_keys, SHARED_SPLIT_WGS if shared_keys else WINDOW_SPLIT_WGS) \
-                if max_keys and not kinds[1] else 1
+            ns = window_splits(tiles.shape[0] * G, max_keys) if max_keys and not kinds[1] else 1
             # tiles of up to mt tokens here, the others a wave each
             mt = 32 if not kinds[1] else 1 if kinds[0] and tt > 1 else 0
             po = pml = None

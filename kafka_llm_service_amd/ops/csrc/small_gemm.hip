@@ -127,7 +127,12 @@ extern "C" hipError_t kafka_launch_small_gemm(const bf16* X, const bf16* W, int 
   };
   // Long K: 16 waves share it, a workgroup per 16 columns (64 columns of 4096 in one workgroup of 8 waves 19.7 us at 64 rows, so 8.8);
   // in between 4 waves; short K: a wave takes 64 columns alone.
-  if (tok != nullptr) return go(small_gemm_kernel<1, 16, false, true>, 1, 16);
+  // Gates of more rows than one round of such workgroups: 32 columns each, one round again. us at 2048 rows of 64 columns, the library and the gate's
+  // launch / 16 columns / 32: K = 4096 21.6 / 18.7 / 15.5, 2048 11.5 / 11.3 / 9.9; at 3000 (two rounds) 21.1 / 27.2 / 29.0; 32 columns, 3000 rows
+  // 14.0 / 18.9 / 15.5.
+  if (tok != nullptr)
+    return N > 32 && (int64_t)rows * ((N + 15) / 16) > 256 ? go(small_gemm_kernel<2, 16, false, true>, 2, 16)
+                                                           : go(small_gemm_kernel<1, 16, false, true>, 1, 16);
   if (K >= 1024) return f32 ? go(small_gemm_kernel<1, 16, true>, 1, 16) : go(small_gemm_kernel<1, 16, false>, 1, 16);
   if (K >= 256) return f32 ? go(small_gemm_kernel<2, 4, true>, 2, 4) : go(small_gemm_kernel<2, 4, false>, 2, 4);
   return f32 ? go(small_gemm_kernel<4, 1, true>, 4, 1) : go(small_gemm_kernel<4, 1, false>, 4, 1);

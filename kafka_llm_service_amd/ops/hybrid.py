@@ -83,7 +83,7 @@ def side_gate_product(h, w, tokens, side_embed, col0: int) -> torch.Tensor:
 
     g = torch.empty(h.shape[0], w.shape[0], dtype=h.dtype, device=h.device)
     if h.shape[1] >= 1024 and side_embed.dtype == h.dtype and side_embed.stride(1) == 1 and tokens.dtype == torch.int64 and \
-            tokens.is_contiguous() and ops.small_ok(h, w, ops.small_rows(w.shape[0], w.shape[1])):
+            tokens.is_contiguous() and ops.small_ok(h, w, max(ops.small_rows(w.shape[0], w.shape[1]), 2048 if w.shape[0] <= 64 else 0)):
         ext().small_gate(h, w, tokens, side_embed, int(col0), g)
     else:
         side_gate(ops.linear_small(h, w), tokens, side_embed, col0, g)

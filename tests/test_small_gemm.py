@@ -165,3 +165,22 @@ def test_gate_times_token_rows(device):
         y = hops.side_gate_product(torch.ones(4, 1024, dtype=torch.bfloat16, device=device), torch.ones(8, 1024, dtype=torch.bfloat16, device=device),
                                    tok, emb.to(device), 0)
         assert y[1:3].isnan().all() and y[[0, 3]].isfinite().all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1025, 64, 1024), (2048, 64, 4096), (2047, 36, 1096), (1366, 48, 2048), (2048, 32, 1024), (2048, 4, 1024)])
+def test_gate_of_long_steps(M, N, K):
+    """One launch up to 2048 rows, of 32 columns a workgroup past 256 workgroups of 16: the same bound as above, fp32 sums of K terms beside it."""
+    from unittest import mock
+
+    g = torch.Generator().manual_seed(M + N)
+    x, w = torch.randn(M, K, generator=g).to(torch.bfloat16), (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16)
+    emb, tok = torch.randn(7, 3 * N, generator=g).to(torch.bfloat16), torch.randint(-1, 8, (M,), generator=g)
+    with mock.patch.object(ops, "linear_small", side_effect=AssertionError("two launches")):
+        got = hops.side_gate_product(x.cuda(), w.cuda(), tok.cuda(), emb.cuda(), N).double().cpu()
+    known = (tok >= 0) & (tok < 7)
+    assert got[~known].isnan().all()
+    z, mag = x[known].double() @ w.double().t(), x[known].double().abs() @ w.double().abs().t()
+    e = emb[tok[known], N:2 * N].double()
+    want = torch.nn.functional.gelu(z, approximate="tanh") * e
+    assert ((got[known] - want).abs() <= 2 ** -8 * want.abs() + 1.13 * K * 2.0 ** -24 * mag * e.abs() + 1e-5 * e.abs()).all()

@@ -17,11 +17,11 @@
 //                       for the scores (the query row broadcast from LDS), online softmax over 64-key blocks, then
 //                       lane = value channel reading its channel's 16 consecutive tokens of a transposed page; a
 //                       row's keys are visited in order, whatever the batch
-//   window_attn_mfma    the same attention on the matrix cores (bf16): 32 (token, head) rows of one key/value head per
-//                       workgroup, 128-key blocks, online softmax, key-range splits with a merge pass
-//   window_attn_rows    the same attention for prompt portions (bf16): a wave per 32 (token, head) rows of one key/value
-//                       head, scores transposed so that rows are lanes - maxima, sums and weights stay in a lane's
-//                       registers, no LDS and no barriers
+//   window_attn_rows    the same attention on the matrix cores (bf16): 32 (token, head) rows of one key/value head, scores
+//                       transposed so that rows are lanes - maxima, sums and weights stay in a lane's registers. Prompt portions: a
+//                       wave each, no LDS and no barriers; decoded tokens: keys over the waves of a workgroup, and over several
+//                       workgroups with a merge pass
+//   window_attn_tile    the same for long portions of 128 channels, eight items on one walk over keys in LDS
 //   moe_topk_grouped    softmax or sigmoid scores, choice among the best groups (by their largest score or the sum of
 //                       their two largest) by corrected score, weights normalised or as they are, times a scale
 #include "common.h"

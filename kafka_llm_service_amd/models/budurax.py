@@ -570,8 +570,11 @@ class BuduraxLM:
         sh = m.seg_host
         last = None if sh is not None and bool(((sh[:, 1] == 1) | (sh[:, 2] == 0)).all()) else \
             torch.empty(m.num_segs, d, dtype=torch.float32, device=dev)
+        one_row = last is None and m.num_segs == T   # (decoded tokens alone)
+        normed = False
         for i, lw in enumerate(self.layers):
-            hops.ln_shift(x, lw.norm1, lw.norm1_b, eps, h, lw.shift, m.tok_seg, m.seg, state.shift[i], last)
+            if not normed:
+                hops.ln_shift(x, lw.norm1, lw.norm1_b, eps, h, lw.shift, m.tok_seg, m.seg, state.shift[i], last)
             if lw.shift is not None and last is not None:
                 hops.scatter_rows(state.shift[i], m.seg, last)
             if lw.type == "latent_attention":
@@ -590,8 +593,12 @@ class BuduraxLM:
                 ys = ops.linear_small(hops.side_gate_product(h2, lw.side_gate, inp.tokens, self.side_embed, i * cfg.token_side_dim), lw.side_proj)
             else:
                 hops.add_ln(x, y, nw, nb, eps)
+            normed = False
             if ys is not None or stack is not None:
-                hops.side_dwa(x, ys, lw.side_norm, eps, stack, i, lw.dwa)
+                nl = self.layers[i + 1] if i + 1 < len(self.layers) else None
+                normed = one_row and nl is not None and nl.shift is not None
+                hops.side_dwa(x, ys, lw.side_norm, eps, stack, i, lw.dwa,
+                              (nl.norm1, nl.norm1_b, eps, h, nl.shift, m.tok_seg, m.seg, state.shift[i + 1]) if normed else None)
             if layers_out is not None:
                 layers_out.append(x.clone())
         xs = ops.gather_rows(x, inp.logit_rows)

@@ -343,15 +343,44 @@ __global__ __launch_bounds__(NTH) void add_ln_reg_kernel(float* __restrict__ x, 
   }
 }
 
-template <typename AT, int VEC, int NTH, int NV>
+// The next layer's norm and token shift where every segment is one row (its previous row is its slot's, whose place it takes)
+struct NextNorm {
+  const void *w, *b, *mu;
+  float eps;
+  const int *tok_seg, *seg;
+  float* state;
+  void* out;
+  int64_t os;
+};
+
+// NEXT: with that norm, from the registers that hold the row (a launch of its own: 5 us of 64 rows of 4096, here 1.5)
+template <typename AT, int VEC, int NTH, int NV, bool NEXT = false>
 __global__ __launch_bounds__(NTH) void side_dwa_reg_kernel(float* __restrict__ x, const AT* __restrict__ y, int64_t ys,
                                                            const AT* __restrict__ sw, float eps,
                                                            float* __restrict__ stack, int layer,
-                                                           const float* __restrict__ dwa, int64_t T, int d) {
+                                                           const float* __restrict__ dwa, int64_t T, int d, NextNorm nx) {
   __shared__ float red[NTH / 64];
   const int64_t t = blockIdx.x;
   const int64_t plane = T * d;
   float xv[NV][VEC], yv[NV][VEC], a[NV][VEC];
+  float nw[NEXT ? NV : 1][VEC], nb[NEXT ? NV : 1][VEC], mu[NEXT ? NV : 1][VEC], pv[NEXT ? NV : 1][VEC];
+  float* slot = nullptr;
+  if constexpr (NEXT) {
+    const int* sg = nx.seg + 4 * nx.tok_seg[t];
+    const int p0 = sg[2];
+    slot = nx.state + (int64_t)sg[3] * d;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int i = (threadIdx.x + k * NTH) * VEC;
+      zero<VEC>(pv[k]);
+      if (i < d) {
+        ldv<VEC>(reinterpret_cast<const AT*>(nx.w) + i, nw[k]);
+        ldv<VEC>(reinterpret_cast<const AT*>(nx.b) + i, nb[k]);
+        ldv<VEC>(reinterpret_cast<const AT*>(nx.mu) + i, mu[k]);
+        if (p0 > 0) ldv<VEC>(slot + i, pv[k]);
+      }
+    }
+  }
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     const int i = (threadIdx.x + k * NTH) * VEC;
@@ -411,6 +440,23 @@ __global__ __launch_bounds__(NTH) void side_dwa_reg_kernel(float* __restrict__ x
         }
       }
       stv<VEC>(x + t * d + i, xv[k]);
+    }
+  }  if constexpr (NEXT) {
+    float mean, rstd;
+    reg_stats<VEC, NTH, NV>(xv, d, nx.eps, red, mean, rstd);
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int i = (threadIdx.x + k * NTH) * VEC;
+      if (i < d) {
+        float h[VEC], o[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          h[e] = (xv[k][e] - mean) * rstd * nw[k][e] + nb[k][e];
+          o[e] = h[e] + (pv[k][e] - h[e]) * mu[k][e];
+        }
+        stv<VEC>(reinterpret_cast<AT*>(nx.out) + t * nx.os + i, o);
+        stv<VEC>(slot + i, h);
+      }
     }
   }
 }
@@ -1543,11 +1589,30 @@ hipError_t kafka_hy_side_dwa(int f32, float* x, const void* y, int64_t ys, const
     const bool v4 = d % 4 == 0 && ys % 4 == 0 && al16(x) && al16(y) && al16(sw) && al16(stack);
     if (!row_shape(T, d, v4, [&](auto V, auto N, auto K) {
           side_dwa_reg_kernel<AT, V.value, N.value, K.value><<<(unsigned)T, N.value, 0, st>>>(
-              x, (const AT*)y, ys, (const AT*)sw, eps, stack, layer, dwa, T, d);
+              x, (const AT*)y, ys, (const AT*)sw, eps, stack, layer, dwa, T, d, NextNorm{});
         }))
       side_dwa_kernel<AT><<<(int)T, NT, 0, st>>>(x, (const AT*)y, ys, (const AT*)sw, eps, stack, layer, dwa, T, d);
   });
   return hipGetLastError();
+}
+
+// the same, then out = ln_shift(x) of segments of one row each
+hipError_t kafka_hy_side_dwa_ln(int f32, float* x, const void* y, int64_t ys, const void* sw, float eps, float* stack, int layer,
+                                const float* dwa, int64_t T, int d, const void* w, const void* b, float eps2, void* out, int64_t os,
+                                const void* mu, const int* tok_seg, const int* seg, float* state, hipStream_t st) {
+  if (T <= 0) return hipSuccess;
+  bool done = false;
+  DISPATCH_AT(f32, {
+    const bool v4 = d % 4 == 0 && ys % 4 == 0 && os % 4 == 0 && al16(x) && al16(y) && al16(sw) && al16(stack) && al16(w) && al16(b) &&
+                    al16(mu) && al16(state) && al16(out);
+    done = row_shape(T, d, v4, [&](auto V, auto N, auto K) {
+      side_dwa_reg_kernel<AT, V.value, N.value, K.value, true><<<(unsigned)T, N.value, 0, st>>>(
+          x, (const AT*)y, ys, (const AT*)sw, eps, stack, layer, dwa, T, d, NextNorm{w, b, mu, eps2, tok_seg, seg, state, out, os});
+    });
+  });
+  if (done) return hipGetLastError();
+  const hipError_t e = kafka_hy_side_dwa(f32, x, y, ys, sw, eps, stack, layer, dwa, T, d, st);
+  return e != hipSuccess ? e : kafka_hy_ln_shift(f32, x, d, w, b, eps2, out, os, (int)T, d, mu, tok_seg, seg, state, nullptr, st);
 }
 
 hipError_t kafka_hy_latent_prep(int f32, const void* qgd, int64_t qs, int T, int H, int dim, int rd, int R, int dkv_off,

@@ -15,6 +15,9 @@ hipError_t kafka_hy_add_ln(int f32, float* x, int64_t xs, const void* y, int64_t
 hipError_t kafka_hy_gelu_mul(int f32, const void* gu, int64_t gs, void* out, int64_t T, int F, hipStream_t st);
 hipError_t kafka_hy_side_gate(int f32, const void* sg, int64_t ss, const int64_t* tokens, const void* emb, int64_t es,
                               int col0, void* out, int64_t T, int dim, hipStream_t st);
+hipError_t kafka_hy_side_dwa_ln(int f32, float* x, const void* y, int64_t ys, const void* sw, float eps, float* stack, int layer,
+                                const float* dwa, int64_t T, int d, const void* w, const void* b, float eps2, void* out, int64_t os,
+                                const void* mu, const int* tok_seg, const int* seg, float* state, hipStream_t st);
 hipError_t kafka_hy_side_dwa(int f32, float* x, const void* y, int64_t ys, const void* sw, float eps, float* stack,
                              int layer, const float* dwa, int64_t T, int d, hipStream_t st);
 hipError_t kafka_hy_latent_prep(int f32, const void* qgd, int64_t qs, int T, int H, int dim, int rd, int R, int dkv_off,
@@ -325,7 +328,11 @@ void side_gate(at::Tensor sg, at::Tensor tokens, at::Tensor emb, int64_t col0, a
                             emb.stride(0), (int)col0, out.data_ptr(), T, (int)dim, stream()));
 }
 
-void side_dwa(at::Tensor x, OptT y, OptT sw, double eps, OptT stack, int64_t layer, OptT dwa) {
+struct SideNext {
+  at::Tensor w, b, out, mu, tok_seg, seg, state;
+  double eps;
+};
+void side_dwa_next(at::Tensor x, OptT y, OptT sw, double eps, OptT stack, int64_t layer, OptT dwa, const SideNext* nx) {
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kFloat && x.is_contiguous() && x.dim() == 2,
               "side_dwa: x fp32 [T, d] contiguous");
   const int64_t T = x.size(0), d = x.size(1);
@@ -350,7 +357,30 @@ void side_dwa(at::Tensor x, OptT y, OptT sw, double eps, OptT stack, int64_t lay
       dp = dwa->data_ptr<float>();
     }
   }
+  if (nx != nullptr) {   // the next layer's ln_shift, of segments of one row each
+    const int of32 = act_f32(nx->out);
+    TORCH_CHECK(!y.has_value() || of32 == f32, "side_dwa: one activation type");
+    rows2d(nx->out, "out");
+    same_act(of32, {&nx->w, &nx->b, &nx->mu});
+    vec(nx->w, d, "w"); vec(nx->b, d, "b"); vec(nx->mu, d, "mu");
+    segs(nx->tok_seg, nx->seg, T);
+    TORCH_CHECK(nx->out.size(0) == T && nx->out.size(1) == d && nx->seg.size(0) == T, "side_dwa: a segment a row");
+    TORCH_CHECK(nx->state.is_cuda() && nx->state.scalar_type() == at::kFloat && nx->state.is_contiguous() && nx->state.dim() == 2 &&
+                    nx->state.size(1) == d, "side_dwa: state fp32 [slots, d]");
+    HY_HIP(kafka_hy_side_dwa_ln(of32, x.data_ptr<float>(), yp, ys, swp, (float)eps, sp, (int)layer, dp, T, (int)d, nx->w.data_ptr(),
+                                nx->b.data_ptr(), (float)nx->eps, nx->out.data_ptr(), nx->out.stride(0), nx->mu.data_ptr(),
+                                nx->tok_seg.data_ptr<int>(), nx->seg.data_ptr<int>(), nx->state.data_ptr<float>(), stream()));
+    return;
+  }
   HY_HIP(kafka_hy_side_dwa(f32, x.data_ptr<float>(), yp, ys, swp, (float)eps, sp, (int)layer, dp, T, (int)d, stream()));
+}
+void side_dwa(at::Tensor x, OptT y, OptT sw, double eps, OptT stack, int64_t layer, OptT dwa) {
+  side_dwa_next(x, y, sw, eps, stack, layer, dwa, nullptr);
+}
+void side_dwa_ln(at::Tensor x, OptT y, OptT sw, double eps, OptT stack, int64_t layer, OptT dwa, at::Tensor w, at::Tensor b, double eps2,
+                 at::Tensor out, at::Tensor mu, at::Tensor tok_seg, at::Tensor seg, at::Tensor state) {
+  const SideNext nx{w, b, out, mu, tok_seg, seg, state, eps2};
+  side_dwa_next(x, y, sw, eps, stack, layer, dwa, &nx);
 }
 
 void latent_prep(at::Tensor qgd, int64_t H, int64_t dim, int64_t rd, int64_t R, int64_t dkv_off, OptT dkv_w, double eps,
@@ -1404,6 +1434,7 @@ void kafka_bind_hybrid(pybind11::module_& m) {
   m.def("hy_gelu_mul", &gelu_mul);
   m.def("hy_side_gate", &side_gate);
   m.def("hy_side_dwa", &side_dwa);
+  m.def("hy_side_dwa_ln", &side_dwa_ln);
   m.def("hy_latent_prep", &latent_prep, py::arg("qgd"), py::arg("H"), py::arg("dim"), py::arg("rd"), py::arg("R"),
         py::arg("dkv_off"), py::arg("dkv_w"), py::arg("eps"), py::arg("positions"), py::arg("cos_sin"),
         py::arg("dims"), py::arg("cache"), py::arg("slots"), py::arg("q_rot"), py::arg("cache_t") = py::none());

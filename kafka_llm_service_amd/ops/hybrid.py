@@ -90,12 +90,18 @@ def side_gate_product(h, w, tokens, side_embed, col0: int) -> torch.Tensor:
     return g
 
 
-def side_dwa(x, y, side_w, eps, stack, layer: int, dwa) -> None:
-    """x += y / rms(y) * side_w (when y is given); stack[layer + 1] = x; with ``dwa`` x = sum_j dwa[j] stack[j]."""
-    if _gpu(x):
-        ext().hy_side_dwa(x, y, side_w, float(eps), stack, int(layer), dwa)
-    else:
+def side_dwa(x, y, side_w, eps, stack, layer: int, dwa, nxt=None) -> None:
+    """x += y / rms(y) * side_w (when y is given); stack[layer + 1] = x; with ``dwa`` x = sum_j dwa[j] stack[j]. ``nxt``: (w, b, eps,
+    out, mu, tok_seg, seg, state) of an ``ln_shift`` of the new x behind it, for steps whose segments are one row each."""
+    if not _gpu(x):
         ref.side_dwa(x, y, side_w, eps, stack, layer, dwa)
+        if nxt is not None:
+            ln_shift(x, *nxt)
+    elif nxt is not None:
+        w, b, e, *more = nxt
+        ext().hy_side_dwa_ln(x, y, side_w, float(eps), stack, int(layer), dwa, w, b, float(e), *more)
+    else:
+        ext().hy_side_dwa(x, y, side_w, float(eps), stack, int(layer), dwa)
 
 
 def latent_prep(qgd, H, dim, rd, R, dkv_off, dkv_w, eps, positions, cos_sin, rot_dims, cache, slot_mapping,

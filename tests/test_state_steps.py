@@ -168,3 +168,41 @@ def test_chunks_carried(n, p0):
     close(out.view(n, H, Dv), torch.stack(want), gate * torch.stack(most))
     close(gM[1], S, gate * magS)
     close(gn[1], v0, gate * magn)
+
+
+@pytest.mark.parametrize("T,d,off", [(1, 64, 0), (5, 1024, 0), (5, 1028, 0), (64, 4096, 0), (3, 4100, 0), (5, 7, 0), (5, 1030, 0), (5, 1024, 1),
+                                     (600, 4096, 0)])   # threads and pieces a row, single elements, a width and rows that the registers do not take
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_layer_end_with_the_next_norm(T, d, off, dtype):
+    """One launch of a layer's end and the next one's shifted norm against the two: the same operations on the same values, whose products
+    and sums may be contracted differently (2 roundings of a value of the row's scale), and in bf16 half a unit of the result."""
+    torch.manual_seed(T + d)
+    dev, layer = "cuda:0", 1
+    segs = [(t, 1, 0 if t % 3 == 1 else 4, T - t) for t in range(T)]
+    seg, tok = torch.tensor(segs, dtype=torch.int32, device=dev), torch.arange(T, dtype=torch.int32, device=dev)
+    x, y, stack = torch.randn(T, d, device=dev), torch.randn(T, d, device=dev).to(dtype), torch.randn(3, T, d, device=dev)
+    w, b, mu, sw = (torch.randn(d, device=dev).to(dtype) for _ in range(4))
+    dwa = torch.rand(layer + 2, device=dev)
+    state = torch.randn(T + 1, d, device=dev)
+    for _, _, p0, slot in segs:
+        if p0 == 0:
+            state[slot] = float("nan")   # (not read)
+    for yy, ss, dd in ((y, stack, dwa), (y, None, None), (None, stack, dwa), (y, stack, None)):
+        res = []
+        for joined in (False, True):
+            xs, st, sk = x.clone(), state.clone(), ss.clone() if ss is not None else None
+            out = torch.full((T, d + 8), 7.0, dtype=dtype, device=dev)
+            rows = out[:, off:off + d]
+            nxt = (w, b, 1e-5, rows, mu, tok, seg, st)
+            hops.side_dwa(xs, yy, sw if yy is not None else None, 1e-6, sk, layer, dd, nxt if joined else None)
+            if not joined:
+                hops.ln_shift(xs, *nxt)
+            assert (out[:, :off] == 7).all() and (out[:, off + d:] == 7).all()
+            res.append((xs, rows.float(), st, sk))
+        for k, (a, c) in enumerate(zip(*res)):
+            if a is not None:
+                assert torch.equal(a.isnan(), c.isnan())
+                a, c = a.nan_to_num(), c.nan_to_num()
+                unit = 2.0 ** -8 if k == 1 and dtype == torch.bfloat16 else 0.0
+                assert ((a - c).abs() <= unit * a.abs() + 8 * EPS * a.abs().amax()).all(), k
+        assert torch.equal(res[1][2][0], state[0])   # (no segment's slot)

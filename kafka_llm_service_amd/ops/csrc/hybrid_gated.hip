@@ -48,6 +48,28 @@ constexpr int PAGE = 16;
 // would drain them as well. This wave's LDS reads and writes are complete (lgkmcnt 0) before it arrives.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// rows of up to 4096 aligned elements in registers: one round trip to memory, not three (us: 1 row of 4096 5.6 -> 2.9, 64 6.0 -> 3.1,
+// 512 6.6 -> 4.4; 64 of 2048 4.2 -> 2.8)
+template <typename AT>
+__global__ __launch_bounds__(1024) void rms_norm_reg_kernel(const float* __restrict__ x, int64_t xs, const AT* __restrict__ w, float eps,
+                                                            AT* __restrict__ out, int64_t os, int d) {
+  typedef AT atx4 __attribute__((ext_vector_type(4)));
+  __shared__ float red[16];
+  const int i = 4 * (int)threadIdx.x;
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  atx4 g = {};
+  if (i < d) {
+    v = *reinterpret_cast<const f32x4*>(x + (int64_t)blockIdx.x * xs + i);
+    g = *reinterpret_cast<const atx4*>(w + i);
+  }
+  const float rs = 1.0f / sqrtf(block_sum<1024>(v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3], red) / (float)d + eps);
+  if (i >= d) return;
+  atx4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = (AT)(v[e] * rs * (float)g[e]);
+  *reinterpret_cast<atx4*>(out + (int64_t)blockIdx.x * os + i) = o;
+}
+
 template <typename AT>
 __global__ __launch_bounds__(NT) void rms_norm_kernel(const float* __restrict__ x, int64_t xs, const AT* __restrict__ w,
                                                       float eps, AT* __restrict__ out, int64_t os, int d) {
@@ -876,7 +898,12 @@ extern "C" {
 hipError_t kafka_hy_rms_norm(int f32, const float* x, int64_t xs, const void* w, float eps, void* out, int64_t os,
                              int T, int d, hipStream_t st) {
   if (T <= 0) return hipSuccess;
-  DISPATCH_AT(f32, { rms_norm_kernel<AT><<<T, NT, 0, st>>>(x, xs, (const AT*)w, eps, (AT*)out, os, d); });
+  auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  const bool v4 = T <= 512 && d <= 4096 && d % 4 == 0 && xs % 4 == 0 && os % 4 == 0 && al(x) && al(w) && al(out);
+  DISPATCH_AT(f32, {
+    if (v4) rms_norm_reg_kernel<AT><<<T, 1024, 0, st>>>(x, xs, (const AT*)w, eps, (AT*)out, os, d);
+    else rms_norm_kernel<AT><<<T, NT, 0, st>>>(x, xs, (const AT*)w, eps, (AT*)out, os, d);
+  });
   return hipGetLastError();
 }
 

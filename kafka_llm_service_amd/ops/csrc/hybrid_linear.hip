@@ -49,7 +49,7 @@ constexpr int NA_MAXS = 8;   // split-K slabs of y1
 // One workgroup per row. VEC consecutive columns per thread and round, NV rounds in registers (d <= NT VEC NV): every
 // load of the row is in flight before the statistics, the sublayer's output and the residual stay in registers. S: slabs of
 // an fp32 y1, 0 = y1 in the activation dtype.
-template <typename AT, int VEC, int NV, int S>
+template <typename AT, int VEC, int NV, int S, int NT>
 __global__ __launch_bounds__(NT) void norm_add_kernel(float* __restrict__ x, int64_t xs, const void* __restrict__ y1,
                                                       int64_t y1s, int64_t slab,
                                                       const AT* __restrict__ y2, int64_t y2s,
@@ -978,23 +978,26 @@ hipError_t kafka_hy_norm_add(int f32, float* x, int64_t xs, const void* y1, int6
   auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   const bool v4 = d % 4 == 0 && xs % 4 == 0 && y1s % 4 == 0 && slab % 4 == 0 && y2s % 4 == 0 && os % 4 == 0 && al(x) &&
                   al(y1) && al(y2) && al(w) && al(out);
-#define NA_LAUNCH(VEC, NV, SL) \
-  norm_add_kernel<AT, VEC, NV, SL><<<(unsigned)T, NT, 0, st>>>(x, xs, y1, y1s, slab, (const AT*)y2, y2s, w, eps, (AT*)out, os, d)
-#define NA_S(VEC, NV)                         \
-  do {                                        \
-    if (!y1_f32) NA_LAUNCH(VEC, NV, 0);       \
-    else if (S == 1) NA_LAUNCH(VEC, NV, 1);   \
-    else if (S == 2) NA_LAUNCH(VEC, NV, 2);   \
-    else if (S == 4) NA_LAUNCH(VEC, NV, 4);   \
-    else NA_LAUNCH(VEC, NV, 8);               \
+#define NA_LAUNCH(VEC, NV, SL, W) \
+  norm_add_kernel<AT, VEC, NV, SL, W><<<(unsigned)T, W, 0, st>>>(x, xs, y1, y1s, slab, (const AT*)y2, y2s, w, eps, (AT*)out, os, d)
+#define NA_S(VEC, NV, W)                         \
+  do {                                           \
+    if (!y1_f32) NA_LAUNCH(VEC, NV, 0, W);       \
+    else if (S == 1) NA_LAUNCH(VEC, NV, 1, W);   \
+    else if (S == 2) NA_LAUNCH(VEC, NV, 2, W);   \
+    else if (S == 4) NA_LAUNCH(VEC, NV, 4, W);   \
+    else NA_LAUNCH(VEC, NV, 8, W);               \
   } while (0)
   const bool s8 = !y1_f32 || S == 1 || S == 2 || S == 4 || S == 8;
   DISPATCH_AT(f32, {
-    if (v4 && s8 && d <= NT * 4) NA_S(4, 1);
-    else if (v4 && s8 && d <= NT * 8) NA_S(4, 2);
-    else if (v4 && s8 && d <= NT * 16) NA_S(4, 4);
-    else if (v4 && s8 && d <= NT * 32) NA_S(4, 8);
-    else if (s8 && d <= NT * 4) NA_S(1, 4);
+    // (few rows wait for their own chain: a piece a thread. us, 256 threads / 1024, a bf16 y1 and one of eight slabs: 64 rows of 4096 4.2 / 3.2 and 5.2 /
+    // 4.0, 512 6.1 / 5.6 and 15.2 / 14.3; 2048 columns 3.3 / 2.9, 512 rows 4.2 / 4.3)
+    if (v4 && s8 && d <= 1024) NA_S(4, 1, 256);
+    else if (v4 && s8 && d <= 4096 && T <= 512) NA_S(4, 1, 1024);
+    else if (v4 && s8 && d <= 2048) NA_S(4, 2, 256);
+    else if (v4 && s8 && d <= 4096) NA_S(4, 4, 256);
+    else if (v4 && s8 && d <= 8192) NA_S(4, 8, 256);
+    else if (s8 && d <= 1024) NA_S(1, 4, 256);
     else
       norm_add_wide_kernel<AT><<<(unsigned)T, NT, 0, st>>>(x, xs, y1, y1s, y1_f32, S, slab, (const AT*)y2, y2s, w, eps,
                                                            (AT*)out, os, d);

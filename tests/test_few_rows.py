@@ -1,0 +1,58 @@
+"""Row kernels of short steps: norms with a piece a thread, routing with an expert a lane."""
+import pytest
+import torch
+
+from kafka_llm_service_amd.ops import hybrid as hops
+
+pytestmark = pytest.mark.gpu
+EPS = 2.0 ** -24
+
+
+@pytest.mark.parametrize("T,d,off", [(1, 4, 0), (3, 1020, 0), (3, 4096, 0), (512, 4092, 0), (513, 4096, 0), (2, 4100, 0), (5, 7, 0), (3, 1024, 1)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rms_norm(T, d, off, dtype):
+    """Against 64-bit sums: a row's mean square is a sum of d squares in fp32, its root and the two products round once each."""
+    torch.manual_seed(T + d)
+    x, w = torch.randn(T, d + 4, device="cuda")[:, off:off + d], torch.randn(d, device="cuda").to(dtype)
+    out = torch.full((T, d + 4), 7.0, dtype=dtype, device="cuda")
+    hops.rms_norm(x, w, 1e-5, out[:, off:off + d])
+    want = x.double() / (x.double().pow(2).mean(1, keepdim=True) + 1e-5).sqrt() * w.double()
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    assert ((out[:, off:off + d].double() - want).abs() <= (unit + (d + 8) * EPS) * want.abs()).all()
+    assert (out[:, :off] == 7).all() and (out[:, off + d:] == 7).all()
+
+
+@pytest.mark.parametrize("T,d", [(3, 1028), (512, 2048), (2, 4096), (513, 4092), (3, 4104), (4, 1024)])   # 256 and 1024 threads a row
+@pytest.mark.parametrize("S", [0, 1, 2, 4, 8])
+def test_norm_add(T, d, S):
+    torch.manual_seed(T + d + S)
+    x, w = torch.randn(T, d, device="cuda"), torch.randn(d, device="cuda")
+    y1 = torch.randn(S, T, d, device="cuda") if S else torch.randn(T, d, device="cuda").bfloat16()
+    y2 = torch.randn(T, d, device="cuda").bfloat16() if S in (0, 2) else None
+    y = (y1.double().sum(0) if S else y1.double()) + (y2.double() if y2 is not None else 0.0)
+    mag = (y1.double().abs().sum(0) if S else y1.double().abs()) + (y2.double().abs() if y2 is not None else 0.0)
+    r = 1 / (y.pow(2).mean(1, keepdim=True) + 1e-5).sqrt()
+    want = x.double() + y * r * w.double()
+    out = torch.empty(T, d, dtype=torch.bfloat16, device="cuda")
+    hops.norm_add(x, y1, y2, w, 1e-5, out)
+    bound = EPS * (12 * mag * r * w.double().abs() + (d + 8) * (y * r * w.double()).abs() + 2 * want.abs())
+    # (a row's scale carries the elements' errors as their mean, less than their largest)
+    bound = bound + 12 * EPS * (mag.amax(1, keepdim=True) * r) * (y * r * w.double()).abs()
+    assert ((x.double() - want).abs() <= bound).all()
+    assert ((out.double() - x.double()).abs() <= 2.0 ** -8 * x.double().abs()).all()
+
+
+@pytest.mark.parametrize("E,k,groups,keep", [(4, 2, 1, 1), (8, 3, 4, 2), (63, 6, 9, 4), (64, 8, 8, 3), (66, 6, 6, 2), (128, 4, 64, 7), (512, 8, 8, 4)])
+@pytest.mark.parametrize("score,group_score", [("softmax", "max"), ("sigmoid", "top2")])
+def test_router_choice(E, k, groups, keep, score, group_score):
+    """One and eight experts a lane, against the choice on the CPU: weights to the few roundings of an exponential and a sum of E, the same
+    experts (random scores, no ties)."""
+    torch.manual_seed(E + k)
+    T, d = 37, 64
+    h, w = torch.randn(T, d).bfloat16(), torch.randn(E, d).bfloat16()
+    corr = torch.rand(E) / 4
+    args = dict(score=score, group_score=group_score, scale=1.5)
+    a = hops.moe_router_grouped(h, w.float(), corr, k, groups, keep, **args)
+    b = hops.moe_router_grouped(h.cuda(), w.float().cuda(), corr.cuda(), k, groups, keep, **args)
+    assert torch.equal(a[1], b[1].cpu())
+    assert ((a[0] - b[0].cpu()).abs() <= (E + 40) * 4 * EPS * a[0].abs()).all()

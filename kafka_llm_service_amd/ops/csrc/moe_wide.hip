@@ -466,36 +466,55 @@ __device__ __forceinline__ f32x4v mfma16(bf16x8 a, bf16x8 b, f32x4v c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// z[row][n] = x[row] . w[n] for 16 rows, the waves' parts summed through LDS -> z in part[0]
+// z[row][n] = x[row] . w[n] for 16 rows, the waves' parts summed through LDS -> z in part[0]. A wave's operands go through LDS of its
+// own (ring), ST steps at a time, so that a load takes whole cache lines of a row: straight to the registers each took half a line of
+// 16 rows, and what a CU takes in is what these products wait for. A row's 16-byte pieces are turned by its number, so that reading a
+// fragment meets all banks. us, K = 4096, before / now: 16 columns 16 rows 9.0 / 4.3, 2048 9.6 / 6.0, 8192 18.8 / 14.8; 32 columns 12.4 /
+// 5.4, 13.1 / 7.5, 27.1 / 18.2; 64 columns 20.6 / 8.4, 21.4 / 9.6, 40.8 / 24.3; the choice and sort of 16 rows, 16 experts 13.4 / 8.8.
+constexpr int nr_steps(int TN) { return TN == 1 ? 4 : 2; }
+constexpr int nr_ring(int TN) { return (1 + TN) * NR_ROWS * 64 * nr_steps(TN); }   // bytes a wave
+typedef __attribute__((address_space(3))) void nr_lds_t;
 template <int TN>
 __device__ __forceinline__ void narrow_product(const bf16* __restrict__ x, int64_t xs, int64_t T, const bf16* __restrict__ wt,
                                                int N, int K, float (*part)[NR_ROWS][nr_ld(TN)]) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
-  const int64_t t = min((int64_t)blockIdx.x * NR_ROWS + r, T - 1);
-  const bf16* xp = x + t * xs + 8 * q;
-  const bf16* wp[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) wp[j] = wt + (int64_t)min(16 * j + r, N - 1) * K + 8 * q;
+  constexpr int ST = nr_steps(TN), ROW = 64 * ST, PCS = 4 * ST, TILE = NR_ROWS * ROW;   // bytes and 16-byte pieces of a row
+  constexpr int NW = nr_waves(TN), PF = TN <= 2 ? 8 : 4;   // steps of a wave in a run
+  __shared__ __attribute__((aligned(16))) unsigned char ring[NW * nr_ring(TN)];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, q = lane >> 4;
+  unsigned char* const my = ring + w * nr_ring(TN);
   f32x4v acc[TN];
 #pragma unroll
   for (int j = 0; j < TN; ++j) acc[j] = f32x4v{0.f, 0.f, 0.f, 0.f};
-  constexpr int PF = TN <= 2 ? 8 : 4;              // steps in flight
   const int ns = K / 32;
-  constexpr int NW = nr_waves(TN);
   for (int s0 = w * PF; s0 < ns; s0 += NW * PF) {
-    bf16x8 a[PF], b[PF][TN];
 #pragma unroll
-    for (int p = 0; p < PF; ++p) {
-      const int s = min(s0 + p, ns - 1);
-      a[p] = load_bf16x8(xp + 32 * s);
-      if (s0 + p >= ns) a[p] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    for (int h = 0; h < PF; h += ST) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j) b[p][j] = load_bf16x8(wp[j] + 32 * s);
+      for (int i = 0; i < TILE / 1024; ++i) {
+        const int row = i * (64 / PCS) + lane / PCS, at = min((s0 + h) * 32 + ((lane ^ row) & (PCS - 1)) * 8, K - 8);
+        const int64_t t = min((int64_t)blockIdx.x * NR_ROWS + row, T - 1);
+        __builtin_amdgcn_global_load_lds(x + t * xs + at, (nr_lds_t*)(my + i * 1024), 16, 0, 0);
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          __builtin_amdgcn_global_load_lds(wt + (int64_t)min(16 * j + row, N - 1) * K + at,
+                                           (nr_lds_t*)(my + (1 + j) * TILE + i * 1024), 16, 0, 0);
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      bf16x8 a[ST], b[ST][TN];
+#pragma unroll
+      for (int p = 0; p < ST; ++p) {
+        const unsigned char* f = my + r * ROW + (((4 * p + q) ^ r) & (PCS - 1)) * 16;
+        a[p] = *reinterpret_cast<const bf16x8*>(f);
+        if (s0 + h + p >= ns) a[p] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < TN; ++j) b[p][j] = *reinterpret_cast<const bf16x8*>(f + (1 + j) * TILE);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (read, before the next loads land there)
+#pragma unroll
+      for (int p = 0; p < ST; ++p)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[j] = mfma16(a[p], b[p][j], acc[j]);
     }
-#pragma unroll
-    for (int p = 0; p < PF; ++p)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) acc[j] = mfma16(a[p], b[p][j], acc[j]);
   }
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("s_nop 15");
@@ -551,7 +570,7 @@ struct RouteSort {
 };
 
 // softmax over all N experts, the k largest (ties: the lower index), their scores as weights (norm: divided by their sum)
-// times scale; lane = expert: up to 16 live in the first 16 lanes (the others run along), exchanges without LDS, 16 rows of 4096 12.2 -> 10.9 us.
+// times scale; lane = expert: up to 16 live in the first 16 lanes (the others run along), exchanges without LDS (1.3 us of 16 rows).
 // SORT: one workgroup, with the sort (a launch of its own: 4.7 us of 16 rows) and, in further ones, the clearing
 template <int TN, bool SORT>
 __global__ __launch_bounds__(64 * nr_waves(TN)) void narrow_route_kernel(const bf16* __restrict__ x, int64_t xs,

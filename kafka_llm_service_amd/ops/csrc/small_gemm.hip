@@ -2,11 +2,12 @@
 // (gfx950). Gates and routers (few columns, long rows), low-rank projections (short rows, many columns) and the products of
 // latent attention's heads (a small product per head): what has neither a tiled copy nor the size for one.
 //
-// What bounds it: a round trip to memory, a launch, and with long rows of a power of two that all 16 of a load lie in one cache
-// channel. So the loads of a wave's whole share of K (16 waves share it) are in flight together. The library's kernels take as long here, but
-// its call costs the host 17 us and this one 3, which is what steps of few rows wait for.
-// us, library on the GPU / this kernel: 64 columns of K = 4096, 64 rows 7.6 / 8.8, 900 8.1 / 9.4, 2048 15.2 / 16.9, 4096 15.9 / 31.9; 8 columns 1900 rows 15.3 / 7.9,
-// with the call 18.8 / 7.9, 8192 21 / 15.6; 32 columns 1900 rows 20 / 9.5, 2805 20 / 17; 4096 columns of
+// What bounds it: a round trip to memory, a launch, and with long rows what a CU takes in: 16 waves share K, and their operands come
+// through LDS in whole cache lines of a row (straight to the registers a load takes half a line of 16 rows). us, K = 4096, before / now:
+// 8 columns 16 rows 7.5 / 4.1, 2048 8.1 / 5.8, 8192 15.6 / 14.0; 64 columns 64 rows 9.1 / 4.8, 300 9.4 / 5.6, 2048 17.1 / 10.3, 4096 32 / 20.4; 32 columns
+// 4096 rows 17.2 / 12.3. The library's call costs the host 17 us and this one 3, which is what steps of few rows wait for.
+// us, library on the GPU / this kernel: 64 columns of K = 4096, 64 rows 7.6 / 4.8, 2048 15.2 / 10.3, 4096 15.9 / 20.4; 8 columns of 1900 rows
+// 15.3 / 5.8, with the call 18.8, 8192 21 / 14; 32 columns of 1900 rows 20 / 6.3; 4096 columns of
 // K = 64, 64 rows 3.6 / 3.3, 300 5.4 / 4.7, 900 5.8 / 8.4; 2048 of K = 16, 64 rows 4.0 / 2.8, 4096 10.1 / 8.9; 8192 of K = 128, 128 rows
 // 4.7 / 4.6, 300 6.3 / 9.8; 32 heads of 128 -> 512, 64 rows 4.6 / 4.6, 128 5.5 / 7.9, of 512 -> 128, 64 rows 8.6 / 4.7, 300 15.3 / 16.1.
 #include "common.h"
@@ -15,6 +16,7 @@ namespace kafka {
 namespace sg {
 
 typedef float f32x4v __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_t;
 struct Strides {
   int64_t xb, xm, wb, wn, yb, ym;
 };
@@ -52,8 +54,39 @@ __global__ __launch_bounds__(64 * (KW > 4 ? KW : 4)) void small_gemm_kernel(cons
   };
   const int whole = min(s1, K >> 5);                 // (a last step of 8, 16 or 24: the lanes past K bring zeros)
   int s = s0;
-  constexpr int U = KW == 16 ? 8 : 4;                // steps whose loads are in flight together
-  for (; s + U <= whole; s += U) {
+  if constexpr (KW == 16) {
+    // ST steps at a time through LDS of the wave's own, a load whole cache lines of a row; a row's 16-byte pieces turned by its number
+    constexpr int ST = NT == 1 ? 4 : 2, ROW = 64 * ST, PCS = 4 * ST, TILE = 16 * ROW;   // bytes and pieces of a row
+    __shared__ __attribute__((aligned(16))) unsigned char ring[NW * (1 + NT) * TILE];
+    unsigned char* const my = ring + w * (1 + NT) * TILE;
+    for (; s + ST <= whole; s += ST) {
+#pragma unroll
+      for (int i = 0; i < TILE / 1024; ++i) {
+        const int row = i * (64 / PCS) + lane / PCS, at = 32 * s + ((lane ^ row) & (PCS - 1)) * 8;
+        __builtin_amdgcn_global_load_lds(X + b * st.xb + (int64_t)min(m0 + row, M - 1) * st.xm + at, (lds_t*)(my + i * 1024), 16, 0, 0);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          __builtin_amdgcn_global_load_lds(W + b * st.wb + (int64_t)min(n0 + 16 * t + row, N - 1) * st.wn + at,
+                                           (lds_t*)(my + (1 + t) * TILE + i * 1024), 16, 0, 0);
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      bf16x8 xv[ST], wv[ST][NT];
+#pragma unroll
+      for (int j = 0; j < ST; ++j) {
+        const unsigned char* f = my + r * ROW + (((4 * j + q) ^ r) & (PCS - 1)) * 16;
+        xv[j] = *reinterpret_cast<const bf16x8*>(f);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) wv[j][t] = *reinterpret_cast<const bf16x8*>(f + (1 + t) * TILE);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (read, before the next loads land there)
+#pragma unroll
+      for (int j = 0; j < ST; ++j)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[j][t], xv[j], acc[t], 0, 0, 0);
+    }
+  }
+  constexpr int U = 4;                               // steps whose loads are in flight together
+  for (; KW < 16 && s + U <= whole; s += U) {
     bf16x8 xv[U], wv[U][NT];
 #pragma unroll
     for (int j = 0; j < U; ++j) {
@@ -125,11 +158,11 @@ extern "C" hipError_t kafka_launch_small_gemm(const bf16* X, const bf16* W, int 
     kern<<<dim3(rows, (N + cols - 1) / cols, B), 64 * (kw > 4 ? kw : 4), 0, st>>>(X, W, M, N, K, bias, Y, s, gate);
     return hipGetLastError();
   };
-  // Long K: 16 waves share it, a workgroup per 16 columns (64 columns of 4096 in one workgroup of 8 waves 19.7 us at 64 rows, so 8.8);
+  // Long K: 16 waves share it, a workgroup per 16 columns (64 columns of 4096 in one workgroup of 8 waves 9.0 us at 64 rows, so 4.8);
   // in between 4 waves; short K: a wave takes 64 columns alone.
   // Gates of more rows than one round of such workgroups: 32 columns each, one round again. us at 2048 rows of 64 columns, the library and the gate's
-  // launch / 16 columns / 32: K = 4096 21.6 / 18.7 / 15.5, 2048 11.5 / 11.3 / 9.9; at 3000 (two rounds) 21.1 / 27.2 / 29.0; 32 columns, 3000 rows
-  // 14.0 / 18.9 / 15.5.
+  // launch / 16 columns / 32: K = 4096 21.6 / 11.0 / 8.9, 2048 11.5 / 7.9 / 6.6; 3000 rows (two rounds)
+  // of K = 4096 18.5, 17.1 on 32 columns, of 2048 11.8, 12.1.
   if (tok != nullptr)
     return N > 32 && (int64_t)rows * ((N + 15) / 16) > 256 ? go(small_gemm_kernel<2, 16, false, true>, 2, 16)
                                                            : go(small_gemm_kernel<1, 16, false, true>, 1, 16);

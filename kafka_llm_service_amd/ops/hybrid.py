@@ -1144,8 +1144,8 @@ def narrow_ok(x, w) -> bool:
 
 
 # Gate products of long rows: the kernel for small products gives 16 columns a workgroup, the narrow one all of them to one, which
-# waits longer for few rows and reads the rows once (32 columns of K = 4096, us, narrow / small: 16 rows 12.3 / 8.6, 2048 12.8 /
-# 9.4, 4096 13.3 / 16.4).
+# waits longer for few rows and reads the rows once (K = 4096, us, narrow / small: 32 columns 16 rows 5.4 / 4.3, 2048 7.5 / 6.3, 4096 8.9 / 12.7;
+# 8 columns 4.2 / 4.2, 5.9 / 5.8, 8.0 / 8.0; 64 columns 8.4 / 4.3, 9.6 / 10.5).
 SMALL_F32_ROWS = 2048
 
 

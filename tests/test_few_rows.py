@@ -56,3 +56,22 @@ def test_router_choice(E, k, groups, keep, score, group_score):
     b = hops.moe_router_grouped(h.cuda(), w.float().cuda(), corr.cuda(), k, groups, keep, **args)
     assert torch.equal(a[1], b[1].cpu())
     assert ((a[0] - b[0].cpu()).abs() <= (E + 40) * 4 * EPS * a[0].abs()).all()
+
+
+@pytest.mark.parametrize("K", [32, 64, 96, 160, 544, 1024, 2080, 4096, 8224])   # runs of steps that end inside, at and past a wave's share
+def test_narrow_products_by_whole_lines(K):
+    """Rows and columns at the edges of 16, in buffers whose neighbours are not numbers: sums of K products of bf16, each rounded in fp32."""
+    torch.manual_seed(K)
+    for T, N in ((1, 1), (15, 16), (16, 17), (17, 33), (33, 48), (40, 64)):
+        x = torch.full((T, K + 16), float("nan"), device="cuda", dtype=torch.bfloat16)
+        x[:, 8:8 + K] = torch.randn(T, K, device="cuda").bfloat16()
+        x = x[:, 8:8 + K]
+        w = torch.randn(N, K, device="cuda").bfloat16()
+        want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+        z = torch.empty(T, N, device="cuda")
+        hops.ext().narrow_linear(x, w, None, z)
+        assert ((z.double() - want).abs() <= (K + 16) * EPS * size).all(), (T, N)
+        if N % 4 == 0:
+            s = torch.empty(T, N, device="cuda")
+            hops.ext().small_gemm(x, w, s)
+            assert ((s.double() - want).abs() <= (K + 16) * EPS * size).all(), (T, N)

@@ -554,6 +554,9 @@ __device__ __forceinline__ float rot_elem(const AT* v, int j, int dims, const fl
   return a * cs[j - half] + ldf(v + j - half) * cs[j];  // cs[half + (j - half)] = sin
 }
 
+// A workgroup per row for the latent, gridDim.y - 1 for the queries' rotation: one after the other in the threads of one they are a chain
+// of trips to memory. us, 32 heads of 64 beside a latent of 512, one workgroup a row / now: 1 row 6.1 / 3.0, 64 6.5 / 3.2, 512 7.8 / 4.9, 1024
+// 11.4 / 8.2, 2048 16.7 / 15.7, 4096 29.2 / 28.0.
 template <typename AT>
 __global__ __launch_bounds__(NT) void latent_prep_kernel(const AT* __restrict__ qgd, int64_t qs, int H, int dim, int rd,
                                                          int R, int dkv_off, const AT* __restrict__ dkv_w, float eps,
@@ -566,9 +569,12 @@ __global__ __launch_bounds__(NT) void latent_prep_kernel(const AT* __restrict__ 
   const int64_t t = blockIdx.x;
   const AT* row = qgd + t * qs;
   const float* cs = cos_sin + positions[t] * dims;
-  for (int i = threadIdx.x; i < H * rd; i += NT) {
-    const int h = i / rd, j = i - h * rd;
-    stf(q_rot + (t * H + h) * rd + j, rot_elem(row + (int64_t)h * (dim + rd) + dim, j, dims, cs));
+  if (blockIdx.y > 0) {
+    for (int i = (blockIdx.y - 1) * NT + threadIdx.x; i < H * rd; i += NT * (gridDim.y - 1)) {
+      const int h = i / rd, j = i - h * rd;
+      stf(q_rot + (t * H + h) * rd + j, rot_elem(row + (int64_t)h * (dim + rd) + dim, j, dims, cs));
+    }
+    return;
   }
   if (dkv_off < 0) return;
   const int64_t slot = slots[t];
@@ -1620,7 +1626,10 @@ hipError_t kafka_hy_latent_prep(int f32, const void* qgd, int64_t qs, int T, int
                                 void* cache, void* cache_t, int page, const int64_t* slots, void* q_rot,
                                 hipStream_t st) {
   if (T <= 0) return hipSuccess;
-  DISPATCH_AT(f32, latent_prep_kernel<AT><<<T, NT, 0, st>>>((const AT*)qgd, qs, H, dim, rd, R, dkv_off,
+  // PREPFIG
+  // as many as the queries fill, up to two rounds of the chip (a thread takes more elements then)
+  const int64_t need = ((int64_t)H * rd + NT - 1) / NT, parts = std::min<int64_t>(need, std::max(4096 / T, 1));
+  DISPATCH_AT(f32, latent_prep_kernel<AT><<<dim3((unsigned)T, 1 + (unsigned)parts), NT, 0, st>>>((const AT*)qgd, qs, H, dim, rd, R, dkv_off,
                                                            (const AT*)dkv_w, eps, positions, cos_sin, dims, (AT*)cache,
                                                            (AT*)cache_t, page, slots, (AT*)q_rot));
   return hipGetLastError();

@@ -75,3 +75,26 @@ def test_narrow_products_by_whole_lines(K):
             s = torch.empty(T, N, device="cuda")
             hops.ext().small_gemm(x, w, s)
             assert ((s.double() - want).abs() <= (K + 16) * EPS * size).all(), (T, N)
+
+
+@pytest.mark.parametrize("T", [1, 512, 635])   # as many workgroups for the queries as they fill, and fewer
+@pytest.mark.parametrize("H,dim,rd,dims,R", [(32, 64, 64, 64, 512), (3, 16, 64, 32, 40), (33, 8, 8, 4, 64), (130, 8, 128, 128, 64), (4, 16, 0, 0, 64)])
+def test_latent_prep(T, H, dim, rd, dims, R):
+    """Against the same in fp32 on the CPU: two products and a sum an element, the norm a sum of R squares; every fourth row without
+    a slot, and queries alone."""
+    g = torch.Generator().manual_seed(T + H)
+    off, page, cap = H * (dim + rd), 16, 640
+    row = torch.randn(T, off + R + rd + 8, generator=g)
+    w, cs = torch.rand(R, generator=g), torch.randn(700, max(dims, 1), generator=g)
+    pos, slots = torch.randint(0, 700, (T,), generator=g), torch.randperm(cap, generator=g)[:T]
+    slots[3::4] = -1
+    for o in (off, -1):
+        got = []
+        for dev in ("cpu", "cuda"):
+            c, ct = torch.full((cap // page, page, R + rd), 7.0, device=dev), torch.full((cap // page, R, page), 7.0, device=dev)
+            q = torch.full((T, H, rd), 7.0, device=dev)
+            hops.latent_prep(row.to(dev), H, dim, rd, R, o, w.to(dev), 1e-5, pos.to(dev), cs.to(dev) if dims else None, dims, c, slots.to(dev), q, ct)
+            got.append([t.cpu() for t in (c, ct, q)])
+        big = 8 * (row.abs().max() * cs.abs().max()).item()
+        for a, b in zip(*got):
+            assert ((a - b).abs() <= (R + 8) * EPS * a.abs() + 4 * EPS * big).all()

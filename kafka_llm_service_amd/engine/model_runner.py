@@ -10,7 +10,7 @@ batches run eagerly.
 from __future__ import annotations
 
 import bisect
-
+import heapq
 import math
 import os
 from collections import deque
@@ -206,6 +206,20 @@ def mixed_tile_wgs(work: int, own: int, tiles: int, hkv: int) -> int:
     if tiles * hkv > 128:
         return 512 if tiles * hkv <= 256 else 1024
     return 512 if 2 * work > 7 * own and work * hkv > 2000 * 256 else 256
+
+
+# A new turn's own keys do not count in the size of its pieces up to this many of the prefix's chunks ...
+MIXED_SHORT = 3
+MIXED_LONG = 2000           # ... and keys of a piece past which they take two workgroups a CU
+
+
+def tile_rounds(items: list[tuple[int, int]], slots: int) -> int:
+    """Keys that the last of ``slots`` workgroups at a time has walked when ``items`` (how many, keys of each; in their order) are done."""
+    ends = [0] * slots
+    for n, k in items:
+        for _ in range(n):
+            heapq.heapreplace(ends, ends[0] + k)
+    return max(ends)
 
 
 MAX_PARTIALS = 64           # partial slots per row that the decode kernel's fused merge reads (one lane each)
@@ -536,6 +550,16 @@ class _Stager:
         dst.copy_(buf[base:base + n], non_blocking=True)
 
 
+@dataclass
+class CascadePlan:
+    """A step's pass over the shared prefixes (``ModelRunner._plan_cascade``)."""
+    kv_start: np.ndarray                                        # by decode row: keys that the pass attends ...
+    npre: np.ndarray                                            # ... and partial slots that it fills
+    items: list[tuple] = field(default_factory=list)
+    behind: dict[int, tuple[int, int]] = field(default_factory=dict)          # joined tile: (keys, partial slots) that the pass has of it
+    own_rows: list[tuple[int, int, int]] = field(default_factory=list)        # joined rows wholly in the pass: (first, last + 1, parts)
+
+
 class ModelRunner:
     def __init__(self, model: TransformerLM, k_caches, v_caches, kvm, max_num_seqs: int, max_blocks_per_seq: int,
                  cascade_min_prefix: int = 512, use_cascade: bool = True, target_wgs: int = 256,
@@ -772,95 +796,38 @@ class ModelRunner:
         # system prompt every new turn of a thread re-attends): their tokens join the group's prefix pass — one read
         # of the prefix pages per step for all rows — and their own tiles attend only the keys behind the prefix
         joins = self._prefix_joins(bt, B, pre, groups, tiles) if groups and self.variant == 3 else {}
-        sfx_slots, sfx_rows, sfx_parts = 0, [], []  # joined tiles whose own keys are planned into the prefix pass: slots, rows, parts
+        own_rows: list[tuple[int, int, int]] = []  # joined rows whose own keys are planned into the prefix pass: first, last + 1, parts
         if B:
-            kv_start = np.zeros(B, dtype=np.int64)
-            npre = np.zeros(B, dtype=np.int64)
-            pit = []
+            kv_start, npre, cp, plan = np.zeros(B, dtype=np.int64), np.zeros(B, dtype=np.int64), None, []
+            h.mixed = int(bool(groups) and self._mixed_plan(seq_lens, groups, sum(tiles[ti][1] for js in joins.values() for ti in js)))
             if groups:
-                mixed = self._mixed_plan(seq_lens, groups, sum(tiles[ti][1] for js in joins.values() for ti in js))
-                tile = self.mixed_tile if mixed else self.tile
-                # joined tiles' own key spans (behind the prefix): with join_suffix they are items of this launch too
-                spans = {ti: tiles[ti][3] - groups[gi][1] * PAGE for gi, js in joins.items() for ti in js} \
-                    if self.join_suffix else {}
-                # the joined rows' prefix-pass tiles: the group's joined tokens re-tiled at token granularity (a burst
-                # of short new turns fills 64-token tiles instead of one mostly empty tile per turn; every key of the
-                # prefix is below every joined token's position, so tokens of different turns share a tile)
-                jt = {gi: retile([tiles[ti][:2] for ti in js], tile if self.retile_joins else 0)
-                      for gi, js in joins.items()}
-                # key chunks sized so the prefix pass launches ~target_wgs workgroups over all groups together
-                parts = {ti: -(-tiles[ti][1] // tile) for ti in spans}  # (row tiles of a joined tile's own keys)
-                # (beside decode pieces the joined rows' own keys do not count: short items, done long before the prefix tiles)
-                sized = {} if mixed else parts
-                work = sum(-(-n // tile) * p * PAGE for n, p in groups) + \
-                    sum(len(t) * groups[gi][1] * PAGE for gi, t in jt.items()) + sum(k * spans[ti] for ti, k in sized.items())
-                tiles_per_group = [-(-n // tile) + len(jt.get(gi, ())) for gi, (n, _) in enumerate(groups)]
-                wgs = self.target_wgs
-                if mixed:
-                    own = int(seq_lens.sum()) - sum(n * p * PAGE for n, p in groups)
-                    wgs = mixed_tile_wgs(work, own, sum(tiles_per_group), self.model.hkv)
-                want = max(1, wgs // self.model.hkv)
-                chunk = min(MAX_ITEM_KEYS, max(256, -(-work // (want * 32)) * 32))
-                # one round of workgroups: per-group rounding up can overshoot the target by a few items, and a
-                # second round of a handful of workgroups doubles the launch
-                while chunk < MAX_ITEM_KEYS and sum(t * -(-(p * PAGE) // chunk) for t, (_, p) in
-                                                    zip(tiles_per_group, groups)) + \
-                        sum(k * -(-spans[ti] // chunk) for ti, k in sized.items()) > want:
-                    chunk += 32
-                r0 = 0
-                for gi, (n, p) in enumerate(groups):
-                    P = p * PAGE
-                    nc = -(-P // chunk)
-                    ck = chunk
-                    if nc > MAX_PREFIX_CHUNKS:
-                        ck = -(-P // (MAX_PREFIX_CHUNKS * 32)) * 32
-                        nc = -(-P // ck)
-                    for c in range(nc):  # chunk-major: the row tiles of one chunk run together (L2 sharing)
-                        for g0 in range(r0, r0 + n, tile):
-                            pit.append((g0, min(tile, r0 + n - g0), r0, c * ck, min(P, (c + 1) * ck), c, 0, nc))
-                        for q0, cnt in jt.get(gi, ()):  # joined prefill rows: q rows B + q0, fp32 alt partials
-                            pit.append((B + q0, cnt, r0, c * ck, min(P, (c + 1) * ck), c, 1, 0))
-                    for ti in joins.get(gi, ()):
-                        tiles[ti] = tiles[ti][:5] + (P, nc)
-                        if ti in spans:
-                            # the tile's keys [P, extent) in pieces of ~chunk keys: alt partials at slots nc, nc + 1..
-                            # (beside its prefix pieces' slots 0..nc-1), so the step needs no separate prefill launch
-                            # for it; attn_merge combines all of the row's slots as before
-                            q0, cnt, btr, ext, hi = tiles[ti][:5]
-                            nsp = max(1, -(-spans[ti] // chunk))
-                            ps = -(-spans[ti] // (nsp * 32)) * 32
-                            nsp = -(-spans[ti] // ps)
-                            pit += [(B + q0 + t0, min(tile, cnt - t0), btr, P + c * ps, min(hi, P + (c + 1) * ps), nc + c, 1, 0)
-                                    for c in range(nsp) for t0 in range(0, cnt, tile)]
-                            sfx_slots = max(sfx_slots, nc + nsp)
-                            sfx_rows.append((q0, q0 + cnt))
-                            sfx_parts.append(nc + nsp)
-                    kv_start[r0:r0 + n] = P
-                    npre[r0:r0 + n] = nc
-                    h.cascade_prefix = max(h.cascade_prefix, P)
-                    r0 += n
-                h.mixed = B + max((hi for _, hi in sfx_rows), default=0) if mixed else 0
-            ditems = self._plan_decode_items(h, seq_lens, kv_start, npre, i32_parts)
-            if pit:
-                h.n_prefix_items = len(pit)
-                i32_parts.append(np.asarray(pit, dtype=np.int32).reshape(-1))
+                cp = self._plan_cascade(seq_lens, groups, joins, tiles, bool(h.mixed))
+                kv_start, npre = cp.kv_start, cp.npre
+            ditems = self._plan_decode_items(h, seq_lens, kv_start, npre, plan)
+            i32_parts += plan
+            if cp:
+                own_rows, h.cascade_prefix, h.n_prefix_items = cp.own_rows, int(kv_start.max()), len(cp.items)
+                i32_parts.append(np.asarray(cp.items, dtype=np.int32).reshape(-1))
+                for ti, at in cp.behind.items():
+                    tiles[ti] = tiles[ti][:5] + at
             if h.mixed:  # parts of every row that the launch merges, and above them how many of them are the prefix tiles'
+                h.mixed = B + max((hi for _, hi, _ in own_rows), default=0)
                 row_parts = np.zeros(h.mixed, dtype=np.int32)
                 row_parts[ditems[:, 0]] = ditems[:, 4] + ditems[:, 5] + (ditems[:, 5] << 16)
-                for (lo, hi), n in zip(sfx_rows, sfx_parts):
+                for lo, hi, n in own_rows:
                     row_parts[B + lo:B + hi] = n
                 i32_parts.append(row_parts)
-        if sfx_rows:  # (their suffix items are in the prefix pass)
+        if own_rows:  # (their suffix items are in the prefix pass)
             done = {ti for js in joins.values() for ti in js}
             tiles = [t for ti, t in enumerate(tiles) if ti not in done]
-        if tiles or sfx_rows:
+        if tiles or own_rows:
             # long tiles (a new turn against a ~20k-token cached context, the late tiles of a causal prompt) are
             # split along the key range so the launch is balanced; their partials are merged afterwards
             items, h.prefill_splits, ranges = plan_prefill_items(tiles, self.model.hkv, self.target_wgs,
                                                                  min(256, self.prefill_kv_chunk))
-            if sfx_rows:
-                h.prefill_splits = max(h.prefill_splits, sfx_slots)
-                ranges = merge_ranges(ranges + sfx_rows) if not h.mixed else ranges
+            if own_rows:
+                h.prefill_splits = max(h.prefill_splits, max(n for _, _, n in own_rows))
+                ranges = merge_ranges(ranges + [r[:2] for r in own_rows]) if not h.mixed else ranges
             h.n_items = len(items)
             i32_parts.append(np.asarray(items, dtype=np.int32).reshape(-1))
             if ranges:
@@ -874,6 +841,101 @@ class ModelRunner:
                    "decode_items": h.n_dec_items, "prefix_items": h.n_prefix_items, "mixed": h.mixed, "s_total": h.s_total,
                    "prefill_splits": h.prefill_splits, "prefill_items": h.n_items}
         return h, sample_seqs
+
+    def _plan_cascade(self, seq_lens: np.ndarray, groups: list[tuple[int, int]], joins: dict[int, list[int]], tiles: list[tuple],
+                      mixed: bool) -> CascadePlan:
+        """Work items of the pass over the groups' shared prefixes (the decode rows' by group from row 0 on) and, with ``joins`` (of prefill
+        ``tiles``), of the new turns that read the same pages; ``mixed``: for one launch beside the decode pieces."""
+        B, tile = seq_lens.shape[0], self.mixed_tile if mixed else self.tile
+        cp = CascadePlan(np.zeros(B, dtype=np.int64), np.zeros(B, dtype=np.int64))
+        # joined tiles' own key spans (behind the prefix): with join_suffix they are items of this launch too
+        spans = {ti: tiles[ti][3] - groups[gi][1] * PAGE for gi, js in joins.items() for ti in js} if self.join_suffix else {}
+        # the joined rows' prefix-pass tiles: the group's joined tokens re-tiled at token granularity (a burst
+        # of short new turns fills 64-token tiles instead of one mostly empty tile per turn; every key of the
+        # prefix is below every joined token's position, so tokens of different turns share a tile)
+        jt = {gi: retile([tiles[ti][:2] for ti in js], tile if self.retile_joins else 0) for gi, js in joins.items()}
+        # key chunks sized so the prefix pass launches ~target_wgs workgroups over all groups together
+        parts = {ti: -(-tiles[ti][1] // tile) for ti in spans}  # (row tiles of a joined tile's own keys)
+        tiles_per_group = [-(-n // tile) + len(jt.get(gi, ())) for gi, (n, _) in enumerate(groups)]
+        prefix_work = sum(t * p * PAGE for t, (_, p) in zip(tiles_per_group, groups))
+        own = int(seq_lens.sum()) - sum(n * p * PAGE for n, p in groups)
+
+        def key_work(sized: dict[int, int]) -> int:
+            return prefix_work + sum(k * spans[ti] for ti, k in sized.items())
+
+        def key_chunk(sized: dict[int, int], least: int = 0) -> int:
+            work = key_work(sized)
+            wgs = max(mixed_tile_wgs(work, own, sum(tiles_per_group), self.model.hkv), least) if mixed else self.target_wgs
+            want = max(1, wgs // self.model.hkv)
+            chunk = min(MAX_ITEM_KEYS, max(256, -(-work // (want * 32)) * 32))
+            # one round of workgroups: per-group rounding up can overshoot the target by a few items, and a
+            # second round of a handful of workgroups doubles the launch (the first chunk of them that has no more; the items fall with it)
+            lo, hi = 0, (MAX_ITEM_KEYS - chunk) // 32
+            while lo < hi:
+                mid = (lo + hi) // 2
+                ck = chunk + 32 * mid
+                if sum(t * -(-(p * PAGE) // ck) for t, (_, p) in zip(tiles_per_group, groups)) + \
+                        sum(k * -(-spans[ti] // ck) for ti, k in sized.items()) > want:
+                    lo = mid + 1
+                else:
+                    hi = mid
+            return chunk + 32 * lo
+
+        chunk = key_chunk({} if mixed else parts)
+        if mixed and spans:
+            # Beside decode pieces the joined rows' own keys do not count while they make up to three pieces: done long before the prefix tiles.
+            # Longer ones do (then also two workgroups a CU, where pieces of one round would be long and do not go evenly over it) ...
+            n_tiles, slots = sum(tiles_per_group) * self.model.hkv, max(1, 512 // self.model.hkv)
+            long = {ti: k for ti, k in parts.items() if spans[ti] > MIXED_SHORT * chunk}
+            if long:
+                chunk = key_chunk(long)
+                if chunk > MIXED_LONG and key_work(long) > own and n_tiles >= 48:
+                    chunk = key_chunk(long, 512)
+            # ... and all of them where they begin a round of their own (two workgroups a CU) and it is done sooner with them.
+            # us of a layer's attention, two launches / none counted / so: 61 rows of 1344 keys behind 18000, two turns of 83 behind 900 of their own
+            # 140 / 117 / 117 (all counted 139), one of 90 behind 9000 142 / 113 / 119; 30 rows, 1024 shared, a turn of 90 behind 3000 54 / 49 / 41, 9000
+            # 68 / 73 / 47, 30000 113 / 124 / 90, four of 30 behind 9000 78 / 92 / 64; 2 rows, 18000 shared, 300 behind 3000 149 / 176 / 148, 90 behind 3000
+            # 76 / 81 / 61; 2 rows, 1024 shared, two of 180 behind 3000 51 / 51 / 44 (one a CU 69). Over 480 steps of 2 - 128 rows with 4 and 8 heads 1 / 0.88 /
+            # 0.80, the worst 1 / 1.8 / 1.02.
+            def pieces(ck: int) -> list[tuple[int, int]]:
+                spread = [(t, p * PAGE) for t, (_, p) in zip(tiles_per_group, groups)] + [(k, spans[ti]) for ti, k in parts.items()]
+                return [(n * -(-keys // ck), -(-keys // -(-keys // ck))) for n, keys in spread]
+
+            if sum(n for n, _ in pieces(chunk)) > slots:
+                full = key_chunk(parts)
+                if tile_rounds(pieces(full), slots) < tile_rounds(pieces(chunk), slots):
+                    chunk = full
+        r0 = 0
+        for gi, (n, p) in enumerate(groups):
+            P = p * PAGE
+            nc = -(-P // chunk)
+            ck = chunk
+            if nc > MAX_PREFIX_CHUNKS:
+                ck = -(-P // (MAX_PREFIX_CHUNKS * 32)) * 32
+                nc = -(-P // ck)
+            for c in range(nc):  # chunk-major: the row tiles of one chunk run together (L2 sharing)
+                for g0 in range(r0, r0 + n, tile):
+                    cp.items.append((g0, min(tile, r0 + n - g0), r0, c * ck, min(P, (c + 1) * ck), c, 0, nc))
+                for q0, cnt in jt.get(gi, ()):  # joined prefill rows: q rows B + q0, fp32 alt partials
+                    cp.items.append((B + q0, cnt, r0, c * ck, min(P, (c + 1) * ck), c, 1, 0))
+            for ti in joins.get(gi, ()):
+                cp.behind[ti] = (P, nc)
+                if ti in spans:
+                    # the tile's keys [P, extent) in pieces of ~chunk keys: alt partials at slots nc, nc + 1..
+                    # (beside its prefix pieces' slots 0..nc-1), so the step needs no separate prefill launch
+                    # for it; attn_merge combines all of the row's slots as before
+                    # (no more slots than one launch merges: of a single turn behind 30000 tokens and few heads there would be 100)
+                    q0, cnt, btr, _, hi = tiles[ti][:5]
+                    nsp = min(max(1, -(-spans[ti] // chunk)), MAX_PARTIALS - nc) if mixed else max(1, -(-spans[ti] // chunk))
+                    ps = -(-spans[ti] // (nsp * 32)) * 32
+                    nsp = -(-spans[ti] // ps)
+                    cp.items += [(B + q0 + t0, min(tile, cnt - t0), btr, P + c * ps, min(hi, P + (c + 1) * ps), nc + c, 1, 0)
+                                 for c in range(nsp) for t0 in range(0, cnt, tile)]
+                    cp.own_rows.append((q0, q0 + cnt, nc + nsp))
+            cp.kv_start[r0:r0 + n] = P
+            cp.npre[r0:r0 + n] = nc
+            r0 += n
+        return cp
 
     def _mixed_plan(self, seq_lens: np.ndarray, groups: list[tuple[int, int]], joined: int) -> bool:
         """Whether a step's prefix tiles and decode pieces go out as one launch (ops.attn_mixed), with ``joined`` rows of new turns. us of a

@@ -4,11 +4,14 @@ import math
 import os
 import sys
 
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 import torch
 
 from kafka_llm_service_amd import ops
+from kafka_llm_service_amd.engine import model_runner as mr
 from kafka_llm_service_amd.engine.model_runner import decode_items
 from kafka_llm_service_amd.ops import reference as ref
 
@@ -177,3 +180,89 @@ def test_plans_of_a_cascade_step_cover_every_key_once():
         assert [a[0] for a in spans] == [0] + [a[1] for a in spans[:-1]] and spans[-1][1] > limit[b]
         assert {a[2] for a in spans} == set(range(len(spans))) and parts[b] & 0xffff == len(spans)
         assert parts[b] >> 16 == (sum(a[1] <= 1024 for a in spans) if b < host.B else 0)
+
+
+class _Tables:
+    """The pages of a step's sequences, as a plan asks for them."""
+
+    def __init__(self):
+        self.pages, self.n = {}, 0
+
+    def sequence(self, sid, prefix, own):
+        k = -(-own // 16)
+        self.pages[sid] = np.concatenate([np.arange(prefix), np.arange(self.n, self.n + k)])
+        self.n += k
+        return SimpleNamespace(seq_id=sid, total_len=prefix * 16 + own, token_at=lambda p: 1, tokens_range=lambda a, b: [1] * (b - a))
+
+    def fill_block_tables(self, ids, bt):
+        for row, sid in zip(bt, ids):
+            row[:len(self.pages[sid])] = self.pages[sid][:len(row)]
+
+    def fill_slots(self, sid, a, b, slots, at):
+        slots[at:at + b - a] = 0
+
+
+def _planned(hkv, G, shared, rows, own, portions):
+    """(runner, plan) of a step: ``rows`` decoding sequences of ``own`` keys behind ``shared`` ones, beside ``portions`` (new tokens, own
+    history) behind the same prefix, history None: a prompt with nothing in common."""
+    t = _Tables()
+    t.n = shared // 16
+    r = mr.ModelRunner.__new__(mr.ModelRunner)
+    r.device, r.kvm, r.model, r.G = torch.device("cpu"), t, SimpleNamespace(hkv=hkv, hq=hkv * G, D=128, scale=128 ** -0.5), G
+    r.segments = r.pad_rows = r.fixed_decode_items = False
+    r.graphs, r.variant, r.tile, r.mixed_tile, r.max_blocks, r.target_wgs, r.prefill_kv_chunk = None, 3, 256 // G, 128 // G, 16384, 256, 256
+    r.cascade_bf16 = r.mixed_attn = r.use_cascade = r.join_suffix = r.retile_joins = True
+    r.cascade_min_prefix, r.stager = 512, mr._Stager(torch.device("cpu"))
+    dec = [t.sequence(f"d{i}", shared // 16, max(1, own - 7 * i)) for i in range(rows)]
+    pre = []
+    for j, (n, hist) in enumerate(portions):
+        first = 0 if hist is None else shared // 16 * 16 + hist
+        pre.append((t.sequence(f"p{j}", 0 if hist is None else shared // 16, n + (hist or 0)), first, first + n))
+    return r, r.build_host(SimpleNamespace(decode=dec, prefill=pre))[0]
+
+
+def _check_plan(r, h):
+    """Every key of every row in one part, the parts of a row in slots of their own from 0 on, no more than one launch merges, and within
+    the buffers that the step makes."""
+    o = h.nbt * h.bt_w
+    limit, B = h.i32[o:o + h.T], h.B
+    o += h.T
+    dec = h.i32[o:o + 8 * h.n_dec_items].reshape(-1, 8)
+    o += dec.size
+    pre = h.i32[o:o + 8 * h.n_prefix_items].reshape(-1, 8)
+    o += pre.size
+    parts = h.i32[o:o + h.mixed]
+    meta = r.views(torch.zeros(3 * h.T + h.n_rows, dtype=torch.int64), torch.from_numpy(h.i32), h).attn
+    seen = [[] for _ in range(h.T)]
+    for b, lo, hi, split, _, npre, _, _ in dec.tolist():
+        assert npre + split < meta.part.shape[2]
+        seen[b].append((lo, hi, npre + split))
+    for q0, n, _, lo, hi, slot, alt, _ in pre.tolist():
+        assert 1 <= n <= r.mixed_tile and hi - lo <= mr.MAX_ITEM_KEYS
+        for t in range(q0, q0 + n):
+            assert bool(alt) == (t >= B)
+            seen[t].append((lo, hi, slot))
+    for t, spans in enumerate(seen[:h.mixed]):
+        assert len(spans) == parts[t] & 0xffff and len(spans) <= mr.MAX_PARTIALS
+        if spans:
+            spans.sort()
+            assert [a[0] for a in spans] == [0] + [a[1] for a in spans[:-1]] and spans[-1][1] > limit[t]
+            assert [a[2] for a in spans] == list(range(len(spans)))
+    assert not any(seen[h.mixed:])
+    if meta.prefill_items is not None:             # rows of no joined turn: launches of their own
+        for q0, n, *_ in meta.prefill_items.tolist():
+            assert not any(seen[B + q0:B + q0 + n])
+    return meta
+
+
+@pytest.mark.parametrize("hkv,G", [(8, 4), (4, 8), (2, 4), (1, 8), (8, 1)])
+def test_new_turns_behind_long_histories_have_as_many_parts_as_one_launch_merges(hkv, G):
+    longest = 0
+    for shared in (512, 1024, 2048, 18000):
+        for rows, own in ((2, 300), (30, 1344)):
+            for n, hist in ((90, 500), (90, 6000), (33, 16500), (83, 30000), (500, 9000), (5, 120000), (1, 60000)):
+                r, h = _planned(hkv, G, shared, rows, own, [(n, hist)])
+                assert h.mixed
+                _check_plan(r, h)
+                longest = max(longest, h.prefill_splits)
+    assert longest > 20 and (hkv > 2 or longest == mr.MAX_PARTIALS)     # (the bound is met where few heads share the launch)

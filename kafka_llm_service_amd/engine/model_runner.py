@@ -49,6 +49,9 @@ class HostStep:
     n_merge: int = 0        # prefill row ranges whose tiles were split: i32[-2 n_merge:] = (lo, hi) pairs
     prefix_joined: int = 0  # prefill tiles that ride in the cascade prefix pass (alt partials into prefill_part)
     mixed: int = 0          # rows that one launch of the prefix items and the decode items merges (ops.attn_mixed), 0: two launches
+    alt_lo: int = 0         # ... the first new turns' row among them (relative to B), 0 slots: none ...
+    alt_slots: int = 0      # ... their partial slots, in a buffer of rows alt_lo .. mixed - B ...
+    tile_splits: int = 0    # ... and those of the prefill tiles beside it
     i64: np.ndarray | None = None
     i32: np.ndarray | None = None
     # (row, seq, position): decode inputs whose token was still being sampled at planning time, filled at launch
@@ -79,7 +82,8 @@ class SampleParams:
 
 
 _PLAN_SCALARS = ("B", "T", "nbt", "bt_w", "n_rows", "s_total", "n_dec_items", "n_prefix_items", "cascade_prefix",
-                 "n_items", "prefill_splits", "n_merge", "n_late", "late_off", "bt_need", "prefix_joined", "n_seg", "mixed")
+                 "n_items", "prefill_splits", "n_merge", "n_late", "late_off", "bt_need", "prefix_joined", "n_seg", "mixed",
+                 "alt_lo", "alt_slots", "tile_splits")
 PLAN_HDR = 32  # int64 header of a broadcast step plan
 PLAN_PAYLOAD_IDX = 1 + len(_PLAN_SCALARS) + 4  # header word holding the payload size (pack_plan)
 
@@ -190,7 +194,9 @@ def decode_round(n: int) -> int:
 
 # One launch of prefix tiles and decode pieces (ops.attn_mixed): workgroups that its pieces are sized for.
 MIXED_PIECES = 768
-MIXED_JOINED = 2048         # rows of new turns that such a launch takes along (their partials stay under 2 GiB)
+MIXED_JOINED = 2048         # rows of new turns that such a launch takes along
+MIXED_PART_BYTES = 1 << 31  # ... which takes the decode rows' partials below this (its merge's 32-bit offsets) ...
+MIXED_ALT_BYTES = 1 << 30   # ... and those of the new turns' rows, and what lies between them, up to this
 MIXED_FEW = 6               # prefix keys of its tiles beside a row's own, past which the two launches of before stay (one round of them)
 
 
@@ -798,12 +804,17 @@ class ModelRunner:
         joins = self._prefix_joins(bt, B, pre, groups, tiles) if groups and self.variant == 3 else {}
         own_rows: list[tuple[int, int, int]] = []  # joined rows whose own keys are planned into the prefix pass: first, last + 1, parts
         if B:
-            kv_start, npre, cp, plan = np.zeros(B, dtype=np.int64), np.zeros(B, dtype=np.int64), None, []
+            kv_start, npre, cp = np.zeros(B, dtype=np.int64), np.zeros(B, dtype=np.int64), None
             h.mixed = int(bool(groups) and self._mixed_plan(seq_lens, groups, sum(tiles[ti][1] for js in joins.values() for ti in js)))
-            if groups:
-                cp = self._plan_cascade(seq_lens, groups, joins, tiles, bool(h.mixed))
-                kv_start, npre = cp.kv_start, cp.npre
-            ditems = self._plan_decode_items(h, seq_lens, kv_start, npre, plan)
+            while True:
+                if groups:
+                    cp = self._plan_cascade(seq_lens, groups, joins, tiles, bool(h.mixed))
+                    kv_start, npre = cp.kv_start, cp.npre
+                plan: list[np.ndarray] = []
+                ditems = self._plan_decode_items(h, seq_lens, kv_start, npre, plan)
+                if not h.mixed or self._mixed_fits(h, cp):
+                    break
+                h.mixed = 0                # (too much for one launch: two of them)
             i32_parts += plan
             if cp:
                 own_rows, h.cascade_prefix, h.n_prefix_items = cp.own_rows, int(kv_start.max()), len(cp.items)
@@ -811,7 +822,9 @@ class ModelRunner:
                 for ti, at in cp.behind.items():
                     tiles[ti] = tiles[ti][:5] + at
             if h.mixed:  # parts of every row that the launch merges, and above them how many of them are the prefix tiles'
-                h.mixed = B + max((hi for _, hi, _ in own_rows), default=0)
+                h.mixed = B
+                if own_rows:
+                    h.alt_lo, h.mixed, h.alt_slots = own_rows[0][0], B + own_rows[-1][1], max(n for _, _, n in own_rows)
                 row_parts = np.zeros(h.mixed, dtype=np.int32)
                 row_parts[ditems[:, 0]] = ditems[:, 4] + ditems[:, 5] + (ditems[:, 5] << 16)
                 for lo, hi, n in own_rows:
@@ -825,6 +838,7 @@ class ModelRunner:
             # split along the key range so the launch is balanced; their partials are merged afterwards
             items, h.prefill_splits, ranges = plan_prefill_items(tiles, self.model.hkv, self.target_wgs,
                                                                  min(256, self.prefill_kv_chunk))
+            h.tile_splits = h.prefill_splits
             if own_rows:
                 h.prefill_splits = max(h.prefill_splits, max(n for _, _, n in own_rows))
                 ranges = merge_ranges(ranges + [r[:2] for r in own_rows]) if not h.mixed else ranges
@@ -935,7 +949,16 @@ class ModelRunner:
             cp.kv_start[r0:r0 + n] = P
             cp.npre[r0:r0 + n] = nc
             r0 += n
+        cp.own_rows.sort()
         return cp
+
+    def _mixed_fits(self, h: HostStep, cp: CascadePlan) -> bool:
+        """Whether the partials, parts and workgroups of such a launch are what it takes."""
+        row = self.model.hq * self.model.D * 4
+        rows, slots = (cp.own_rows[-1][1] - cp.own_rows[0][0], max(n for _, _, n in cp.own_rows)) if cp.own_rows else (0, 0)
+        merges = -(-(h.B + (cp.own_rows[-1][1] if cp.own_rows else 0)) * self.G // 16)
+        return max(slots, h.s_total) <= MAX_PARTIALS and h.B * h.s_total * row < MIXED_PART_BYTES and \
+            rows * slots * row <= MIXED_ALT_BYTES and len(cp.items) + h.n_dec_items + merges <= 65535
 
     def _mixed_plan(self, seq_lens: np.ndarray, groups: list[tuple[int, int]], joined: int) -> bool:
         """Whether a step's prefix tiles and decode pieces go out as one launch (ops.attn_mixed), with ``joined`` rows of new turns. us of a
@@ -1045,25 +1068,29 @@ class ModelRunner:
             if h.mixed:
                 meta.row_parts = d32[o:o + h.mixed]
                 o += h.mixed
+                if h.alt_slots:
+                    rows = h.mixed - B - h.alt_lo
+                    meta.alt_part = torch.empty(rows, Hq, h.alt_slots, D, dtype=torch.float32, device=self.device)
+                    meta.alt_lse = torch.empty(rows, Hq, h.alt_slots, dtype=torch.float32, device=self.device)
+                    meta.alt_off = B + h.alt_lo
             meta.s_total = h.s_total
             meta.part = torch.empty(B, Hq, h.s_total, D, dtype=torch.float32, device=self.device)
             meta.lse = torch.empty(B, Hq, h.s_total, dtype=torch.float32, device=self.device)
             if h.n_prefix_items and self.cascade_bf16:
                 meta.pre_part = torch.empty(B, Hq, h.s_total, D, dtype=torch.bfloat16, device=self.device)
             meta.extra["cascade_prefix"] = h.cascade_prefix
-        if h.n_items or h.n_merge or h.prefill_splits:
+        if h.n_items or h.n_merge:
             if h.n_items:
                 meta.prefill_items = d32[o:o + h.n_items * 8].view(-1, 8)
                 o += h.n_items * 8
-            if h.prefill_splits:
+            splits = h.tile_splits if h.mixed else h.prefill_splits
+            if splits:
                 Tp = T - B
-                meta.prefill_splits = h.prefill_splits
+                meta.prefill_splits = splits
                 mr = h.i32[h.i32.size - 2 * h.n_merge:].reshape(-1, 2)  # host copy of the plan (every TP rank)
                 meta.prefill_merge = [(int(lo), int(hi)) for lo, hi in mr]
-                meta.prefill_part = torch.empty(Tp, Hq, h.prefill_splits, D, dtype=torch.float32,
-                                                device=self.device)
-                meta.prefill_lse = torch.full((Tp, Hq, h.prefill_splits), float("-inf"), dtype=torch.float32,
-                                              device=self.device)
+                meta.prefill_part = torch.empty(Tp, Hq, splits, D, dtype=torch.float32, device=self.device)
+                meta.prefill_lse = torch.full((Tp, Hq, splits), float("-inf"), dtype=torch.float32, device=self.device)
                 meta.prefix_joined = h.prefix_joined > 0
         if h.n_late:
             L, n = h.late_off, h.n_late

@@ -173,24 +173,26 @@ def attn_decode_items(q, k_cache, v_cache, block_tables, items, out_part, lse_pa
 
 
 def attn_mixed(prefix_items, decode_items, q, k_cache, v_cache, block_tables, q_limit, part, lse, pre, row_parts, scale: float, out,
-               alt_part=None, alt_lse=None) -> None:
+               alt_part=None, alt_lse=None, alt_off: int | None = None) -> None:
     """``attn_prefill`` of the cascade's prefix items (bf16 partials into ``pre``, items flagged alt into ``alt_part``) and
     ``attn_decode_items`` with all merges, as one launch on pages in bf16: tiles of at most 128 query rows beside the decode pieces.
-    Rows [0, B) of q and out are the decode rows (B = part's), those behind them new turns' rows. ``row_parts`` int32 [rows of out]: the
-    parts of every row (its prefix items and pieces, from slot 0 on; 0: not this launch's), those that are in ``pre`` once more in
-    the upper 16 bits."""
+    Rows [0, B) of q and out are the decode rows (B = part's), those behind them new turns' rows, whose partials from row ``alt_off`` on
+    (B unless given) are in ``alt_part``. ``row_parts`` int32 [rows of out]: the parts of every row (its prefix items and pieces, from
+    slot 0 on; 0: not this launch's), those that are in ``pre`` once more in the upper 16 bits."""
+    B = part.shape[0]
+    off = B if alt_off is None or alt_part is None else int(alt_off)
     if _gpu(q):
         n = out.shape[0] * k_cache.shape[1]
         counters = _tickets(q.device, n, f"mixed {torch.cuda.current_stream(q.device).cuda_stream}")
         ext().attn_mixed(prefix_items, decode_items, q, k_cache, v_cache, block_tables, q_limit, part, lse, pre, row_parts, float(scale),
-                         out, counters, alt_part, alt_lse, part.shape[0])
+                         out, counters, alt_part, alt_lse, off)
         return
-    B = part.shape[0]
-    ref.attn_prefill_items(prefix_items, q, k_cache, v_cache, block_tables, q_limit, scale, None, pre, lse, alt_part, alt_lse, B)
+    ref.attn_prefill_items(prefix_items, q, k_cache, v_cache, block_tables, q_limit, scale, None, pre, lse, alt_part, alt_lse, off)
     ref.attn_decode_items(q[:B], k_cache, v_cache, block_tables, decode_items, part, lse, scale, out[:B], pre)
-    for r in range(B, out.shape[0]):
-        if row_parts[r]:
-            ref.attn_merge(alt_part[r - B:r - B + 1], alt_lse[r - B:r - B + 1], out[r:r + 1])
+    for r in range(off, out.shape[0]):
+        n, a = int(row_parts[r]), r - off
+        if n:
+            ref.attn_merge(alt_part[a:a + 1, :, :n], alt_lse[a:a + 1, :, :n], out[r:r + 1])
 
 
 def uniform_decode_items(seq_lens: torch.Tensor, kv_start: torch.Tensor | None, num_splits: int,

@@ -168,7 +168,8 @@ __global__ __launch_bounds__(256, 2) void attn_mixed_kernel(const TileItem* __re
   if (tid < tw) {
     const int row = row0 + tid;
     int need = row < n_rows ? row_parts[row] & ((1 << PRE) - 1) : 0;
-    const bool fits = need <= min(MAXS, row < B ? S_total : ap.S);   // (a host bug otherwise: nothing is read)
+    // (a host bug otherwise: nothing is read; rows between the decode rows and the new turns' have no parts)
+    const bool fits = need <= min(MAXS, row < B ? S_total : ap.S) && (row < B || row >= ap.tok_off);
     need = fits ? need : 0;
     int* c = counters + (int64_t)min(row, n_rows - 1) * Hkv + kvh;
     int polls = POLLS;
@@ -205,7 +206,7 @@ extern "C" hipError_t kafka_launch_attn_mixed(const int* titems, int n_tiles, co
   const int n_merge = (n_rows + 16 / G - 1) / (16 / G);
   if ((int64_t)n_tiles + n_pieces + n_merge > 65535) return hipErrorInvalidValue;
   if (!part || !lse || !pre || !out || !counters || out_stride % 8 || reinterpret_cast<uintptr_t>(out) % 16 || S_total < 1 ||
-      (n_rows > B && (!alt_part || alt_tok_off != B)))
+      (n_rows > B && (!alt_part || alt_tok_off < B || alt_tok_off > n_rows)))
     return hipErrorInvalidValue;
   attn_mixed_kernel<<<dim3(Hkv, n_tiles + n_pieces + n_merge), 256, 0, st>>>(
       reinterpret_cast<const TileItem*>(titems), n_tiles, reinterpret_cast<const DecodeItem*>(ditems), n_pieces, row_parts, n_rows, q,

@@ -397,7 +397,7 @@ static void attn_decode(at::Tensor q, at::Tensor k_cache, at::Tensor v_cache, at
 }
 
 // prefix tiles and decode pieces of a step in one launch (attn_mixed.hip): q [T, Hq, 128], rows [0, B) of it (part's) the
-// decode rows; out and row_parts: the rows that it merges
+// decode rows; out and row_parts: the rows that it merges (from alt_tok_off on those whose partials are in alt_part)
 static void attn_mixed(at::Tensor prefix_items, at::Tensor decode_items, at::Tensor q, at::Tensor k_cache, at::Tensor v_cache,
                        at::Tensor block_tables, at::Tensor q_limit, at::Tensor part, at::Tensor lse, at::Tensor pre,
                        at::Tensor row_parts, double scale, at::Tensor out, at::Tensor counters, c10::optional<at::Tensor> alt_part, c10::optional<at::Tensor> alt_lse,
@@ -432,8 +432,8 @@ static void attn_mixed(at::Tensor prefix_items, at::Tensor decode_items, at::Ten
     TORCH_CHECK(alt_lse.has_value(), "attn_mixed: alt partials need alt_lse");
     CHECK_DT(alt_part.value(), at::kFloat); CHECK_DT(alt_lse.value(), at::kFloat);
     TORCH_CHECK(alt_part->is_contiguous() && alt_part->dim() == 4 && alt_part->size(1) == Hq && alt_part->size(3) == 128 &&
-                    alt_tok_off == B && alt_part->size(0) + B >= R &&
-                    alt_part->numel() * 4 < 0x7fffffffLL, "attn_mixed: alt_part must be [>= rows - B, Hq, S, 128] of less than 2 GiB");
+                    alt_tok_off >= B && alt_tok_off <= R && alt_part->size(0) + alt_tok_off >= R &&
+                    alt_part->numel() * 4 < 0x7fffffffLL, "attn_mixed: alt_part must be [>= rows - alt_tok_off, Hq, S, 128] of less than 2 GiB");
     S2 = alt_part->size(2);
     TORCH_CHECK(alt_lse->is_contiguous() && alt_lse->numel() >= alt_part->size(0) * Hq * S2, "attn_mixed: alt_lse");
     ap = alt_part->data_ptr<float>();

@@ -13,6 +13,7 @@ import torch
 from kafka_llm_service_amd import ops
 from kafka_llm_service_amd.engine import model_runner as mr
 from kafka_llm_service_amd.engine.model_runner import decode_items
+from kafka_llm_service_amd.models.attention import paged_attention
 from kafka_llm_service_amd.ops import reference as ref
 
 sys.path.insert(0, os.path.dirname(__file__))
@@ -202,17 +203,17 @@ class _Tables:
         slots[at:at + b - a] = 0
 
 
-def _planned(hkv, G, shared, rows, own, portions):
+def _planned(hkv, G, shared, rows, own, portions, dev="cpu"):
     """(runner, plan) of a step: ``rows`` decoding sequences of ``own`` keys behind ``shared`` ones, beside ``portions`` (new tokens, own
     history) behind the same prefix, history None: a prompt with nothing in common."""
     t = _Tables()
     t.n = shared // 16
     r = mr.ModelRunner.__new__(mr.ModelRunner)
-    r.device, r.kvm, r.model, r.G = torch.device("cpu"), t, SimpleNamespace(hkv=hkv, hq=hkv * G, D=128, scale=128 ** -0.5), G
+    r.device, r.kvm, r.model, r.G = torch.device(dev), t, SimpleNamespace(hkv=hkv, hq=hkv * G, D=128, scale=128 ** -0.5), G
     r.segments = r.pad_rows = r.fixed_decode_items = False
     r.graphs, r.variant, r.tile, r.mixed_tile, r.max_blocks, r.target_wgs, r.prefill_kv_chunk = None, 3, 256 // G, 128 // G, 16384, 256, 256
     r.cascade_bf16 = r.mixed_attn = r.use_cascade = r.join_suffix = r.retile_joins = True
-    r.cascade_min_prefix, r.stager = 512, mr._Stager(torch.device("cpu"))
+    r.cascade_min_prefix, r.stager = 512, mr._Stager(torch.device(dev))
     dec = [t.sequence(f"d{i}", shared // 16, max(1, own - 7 * i)) for i in range(rows)]
     pre = []
     for j, (n, hist) in enumerate(portions):
@@ -235,13 +236,17 @@ def _check_plan(r, h):
     meta = r.views(torch.zeros(3 * h.T + h.n_rows, dtype=torch.int64), torch.from_numpy(h.i32), h).attn
     seen = [[] for _ in range(h.T)]
     for b, lo, hi, split, _, npre, _, _ in dec.tolist():
-        assert npre + split < meta.part.shape[2]
+        assert npre + split < meta.part.shape[2] and meta.part.numel() * 4 < 1 << 31
         seen[b].append((lo, hi, npre + split))
     for q0, n, _, lo, hi, slot, alt, _ in pre.tolist():
         assert 1 <= n <= r.mixed_tile and hi - lo <= mr.MAX_ITEM_KEYS
         for t in range(q0, q0 + n):
             assert bool(alt) == (t >= B)
             seen[t].append((lo, hi, slot))
+    joined = [t for t in range(B, h.T) if seen[t]]
+    if joined:                                     # (their partials lie in a buffer of their rows)
+        assert meta.alt_off == joined[0] and meta.alt_part.shape[0] == joined[-1] + 1 - joined[0] and h.mixed == joined[-1] + 1
+        assert max(a[2] for t in joined for a in seen[t]) < meta.alt_part.shape[2] and meta.alt_part.numel() * 4 <= 1 << 30
     for t, spans in enumerate(seen[:h.mixed]):
         assert len(spans) == parts[t] & 0xffff and len(spans) <= mr.MAX_PARTIALS
         if spans:
@@ -252,7 +257,6 @@ def _check_plan(r, h):
     if meta.prefill_items is not None:             # rows of no joined turn: launches of their own
         for q0, n, *_ in meta.prefill_items.tolist():
             assert not any(seen[B + q0:B + q0 + n])
-    return meta
 
 
 @pytest.mark.parametrize("hkv,G", [(8, 4), (4, 8), (2, 4), (1, 8), (8, 1)])
@@ -266,3 +270,85 @@ def test_new_turns_behind_long_histories_have_as_many_parts_as_one_launch_merges
                 _check_plan(r, h)
                 longest = max(longest, h.prefill_splits)
     assert longest > 20 and (hkv > 2 or longest == mr.MAX_PARTIALS)     # (the bound is met where few heads share the launch)
+
+
+@pytest.mark.parametrize("hkv,G", [(8, 4), (1, 8), (8, 1)])
+@pytest.mark.parametrize("rows,portions", [
+    (12, [(6000, None), (90, 6000)]), (4, [(5000, None), (90, 9000)]), (8, [(7000, None), (100, 6000)]), (8, [(8000, None), (100, 8000)]),
+    (8, [(6000, None), (2000, 4000)]), (8, [(90, 6000), (300, None), (41, 3000)]), (4, [(90, 30000), (7000, None), (90, 30000)]), (30, [(2048, 60000)])])
+def test_partials_of_new_turns_beside_cold_prompts(rows, portions, hkv, G):
+    """Rows that are not the launch's take no part in its buffers, which stay within what its merge addresses; what would not is two launches."""
+    one = 0
+    for shared in (1024, 6000):
+        r, h = _planned(hkv, G, shared, rows, 300, portions)
+        between = len(portions) == 3 and portions[1][0] > 1000
+        assert h.mixed or between and hkv * G > 8
+        if h.mixed:
+            one += 1
+            _check_plan(r, h)
+        assert bool(h.prefix_joined)
+    assert one or between
+
+
+def test_partials_past_what_one_launch_addresses_are_two_launches(monkeypatch):
+    batch = (8, 4, 1024, 40, 300, [(90, 3000)])
+    h = _planned(*batch)[1]
+    assert h.mixed and h.alt_slots
+    row, alt = 32 * 128 * 4, (h.mixed - h.B - h.alt_lo) * h.alt_slots
+    for name, n in (("MIXED_ALT_BYTES", alt * row - 1), ("MIXED_PART_BYTES", h.B * h.s_total * row)):
+        with monkeypatch.context() as m:
+            m.setattr(mr, name, n)
+            two = _planned(*batch)[1]
+        assert not two.mixed and two.n_merge and two.prefix_joined and not two.alt_slots
+    with monkeypatch.context() as m:
+        m.setattr(mr, "MIXED_ALT_BYTES", alt * row)
+        m.setattr(mr, "MIXED_PART_BYTES", h.B * h.s_total * row + 1)
+        assert _planned(*batch)[1].mixed
+
+
+#: (kv heads, G, shared, decode rows, their own keys, portions, parts of the longest row): as many parts as a launch merges; a turn's tile cut
+#: into several, some of whose pieces lie past the first ones' limits; a cold prompt between and before joined turns, both kinds of splits
+#: beside each other; whole tiles of one head
+STEPS = [(1, 8, 512, 2, 300, [(33, 60000)], 64), (2, 4, 640, 3, 100, [(70, 20)], 2), (2, 4, 1024, 5, 200, [(90, 6000), (300, None), (41, 3000)], 20),
+         (2, 4, 1024, 5, 200, [(2000, None), (90, 6000)], 20), (8, 1, 1024, 4, 90, [(150, 1200)], 4)]
+
+
+def _steps(hkv, G, shared, rows, own, portions, parts, dev):
+    r, h = _planned(hkv, G, shared, rows, own, portions, dev)
+    assert h.mixed and max(h.alt_slots, h.tile_splits) >= parts
+    g = torch.Generator().manual_seed(5)
+    n = r.kvm.n
+    k = torch.randn(n, hkv, 16, 128, generator=g).to(torch.bfloat16)
+    v = torch.randn(n, hkv, 128, 16, generator=g).to(torch.bfloat16)
+    q = torch.randn(h.T, hkv * G, 128, generator=g).to(torch.bfloat16)
+    meta = r.to_device(h).attn
+    out = torch.full(q.shape, float("nan"), dtype=torch.bfloat16, device=dev)
+    paged_attention(q.to(dev), k.to(dev), v.to(dev), meta, out)
+    if dev != "cpu":
+        first = out.clone()
+        paged_attention(q.to(dev), k.to(dev), v.to(dev), meta, out)
+        assert torch.equal(first, out)
+    assert not out.isnan().any()
+    o, starts = h.nbt * h.bt_w, [h.B]
+    bt, limit = torch.from_numpy(h.i32[:o].reshape(h.nbt, -1)), h.i32[o:o + h.T]
+    for m, _ in portions:
+        starts.append(starts[-1] + m)
+    picks = {b: b for b in range(h.B)}
+    for j, (a, b) in enumerate(zip(starts, starts[1:])):
+        picks.update({t: h.B + j for t in (a, a + 31, a + 33, a + 64, (a + b) // 2, b - 1) if a <= t < b})
+    for t, row in picks.items():                   # (as _check: 3 roundings of 2^-9, taken twice)
+        kk, vv = ref.gather_kv(k, v, bt[row], int(limit[t]) + 1)
+        s = torch.einsum("hgd,nhd->hgn", q[t].float().view(hkv, G, 128), kk.float()) / math.sqrt(128)
+        want = torch.einsum("hgn,nhd->hgd", s.softmax(-1), vv.float()).reshape(-1, 128)
+        assert (out[t].float().cpu() - want).abs().max() <= 6 * 2.0 ** -9 * want.abs().max(), t
+
+
+@pytest.mark.parametrize("step", STEPS)
+def test_steps_with_new_turns_equal_whole_attention_cpu(step):
+    _steps(*step, "cpu")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("step", STEPS)
+def test_steps_with_new_turns_equal_whole_attention(cuda, step):
+    _steps(*step, cuda)

@@ -829,7 +829,8 @@ class ModelRunner:
                 row_parts[ditems[:, 0]] = ditems[:, 4] + ditems[:, 5] + (ditems[:, 5] << 16)
                 for lo, hi, n in own_rows:
                     row_parts[B + lo:B + hi] = n
-                i32_parts.append(row_parts)
+                # (and the launch's counters: the step's own, clear with its upload)
+                i32_parts += [row_parts, np.zeros(h.mixed * self.model.hkv, dtype=np.int32)]
         if own_rows:  # (their suffix items are in the prefix pass)
             done = {ti for js in joins.values() for ti in js}
             tiles = [t for ti, t in enumerate(tiles) if ti not in done]
@@ -1068,6 +1069,8 @@ class ModelRunner:
             if h.mixed:
                 meta.row_parts = d32[o:o + h.mixed]
                 o += h.mixed
+                meta.counters = d32[o:o + h.mixed * self.model.hkv]
+                o += h.mixed * self.model.hkv
                 if h.alt_slots:
                     rows = h.mixed - B - h.alt_lo
                     meta.alt_part = torch.empty(rows, Hq, h.alt_slots, D, dtype=torch.float32, device=self.device)

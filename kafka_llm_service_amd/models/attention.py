@@ -53,6 +53,7 @@ class AttnMeta:
     prefill_lse: torch.Tensor | None = None
     prefill_merge: list = field(default_factory=list)  # (lo, hi) prefill row ranges of split tiles
     row_parts: torch.Tensor | None = None      # int32: prefix_items and decode_items are one launch's (ops.attn_mixed), parts by row
+    counters: torch.Tensor | None = None       # int32 zeros [rows of that launch, kv heads]
     alt_part: torch.Tensor | None = None       # f32 [new turns' rows of that launch, Hq, slots, D], from row alt_off of q on
     alt_lse: torch.Tensor | None = None
     alt_off: int = 0
@@ -82,7 +83,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         n = meta.row_parts.numel()
         ops.attn_mixed(meta.prefix_items, meta.decode_items, q[:n], k_cache, v_cache, meta.block_tables, meta.q_limit, meta.part,
                        meta.lse, meta.pre_part, meta.row_parts, meta.scale, out[:n],
-                       meta.alt_part, meta.alt_lse, meta.alt_off)
+                       meta.alt_part, meta.alt_lse, meta.alt_off, meta.counters)
     elif B > 0:
         qd = q[:B]
         if meta.prefix_items is not None:

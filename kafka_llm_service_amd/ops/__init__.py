@@ -172,20 +172,27 @@ def attn_decode_items(q, k_cache, v_cache, block_tables, items, out_part, lse_pa
         ref.attn_merge(*merge)
 
 
+MIXED_POLLS = 1 << 24  # looks (of about a us) that a row of such a launch waits for its parts
+MIXED_PARTS = 64       # parts of a row that its merge reads
+
+
 def attn_mixed(prefix_items, decode_items, q, k_cache, v_cache, block_tables, q_limit, part, lse, pre, row_parts, scale: float, out,
-               alt_part=None, alt_lse=None, alt_off: int | None = None) -> None:
+               alt_part=None, alt_lse=None, alt_off: int | None = None, counters=None, polls: int = MIXED_POLLS) -> None:
     """``attn_prefill`` of the cascade's prefix items (bf16 partials into ``pre``, items flagged alt into ``alt_part``) and
     ``attn_decode_items`` with all merges, as one launch on pages in bf16: tiles of at most 128 query rows beside the decode pieces.
     Rows [0, B) of q and out are the decode rows (B = part's), those behind them new turns' rows, whose partials from row ``alt_off`` on
     (B unless given) are in ``alt_part``. ``row_parts`` int32 [rows of out]: the parts of every row (its prefix items and pieces, from
-    slot 0 on; 0: not this launch's), those that are in ``pre`` once more in the upper 16 bits."""
+    slot 0 on; 0: not this launch's; more than 64, or more than come: the row is not a number), those that are in ``pre`` once more in
+    the upper 16 bits. ``counters``: int32 zeros [rows of out, kv heads] that belong to the caller's step, whose launches leave them
+    zero but for rows that were no numbers, which stay so; one per device and stream, cleared here, without."""
     B = part.shape[0]
     off = B if alt_off is None or alt_part is None else int(alt_off)
     if _gpu(q):
-        n = out.shape[0] * k_cache.shape[1]
-        counters = _tickets(q.device, n, f"mixed {torch.cuda.current_stream(q.device).cuda_stream}")
+        if counters is None:
+            counters = _tickets(q.device, out.shape[0] * k_cache.shape[1], f"mixed {torch.cuda.current_stream(q.device).cuda_stream}")
+            counters.zero_()
         ext().attn_mixed(prefix_items, decode_items, q, k_cache, v_cache, block_tables, q_limit, part, lse, pre, row_parts, float(scale),
-                         out, counters, alt_part, alt_lse, off)
+                         out, counters, alt_part, alt_lse, off, polls)
         return
     ref.attn_prefill_items(prefix_items, q, k_cache, v_cache, block_tables, q_limit, scale, None, pre, lse, alt_part, alt_lse, off)
     ref.attn_decode_items(q[:B], k_cache, v_cache, block_tables, decode_items, part, lse, scale, out[:B], pre)
@@ -193,6 +200,7 @@ def attn_mixed(prefix_items, decode_items, q, k_cache, v_cache, block_tables, q_
         n, a = int(row_parts[r]), r - off
         if n:
             ref.attn_merge(alt_part[a:a + 1, :, :n], alt_lse[a:a + 1, :, :n], out[r:r + 1])
+    out[(row_parts & 0xffff) > MIXED_PARTS] = float("nan")
 
 
 def uniform_decode_items(seq_lens: torch.Tensor, kv_start: torch.Tensor | None, num_splits: int,

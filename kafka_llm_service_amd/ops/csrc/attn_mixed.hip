@@ -9,7 +9,8 @@
 // and then counts itself in at each of its (row, kv head) counters. The last workgroups of the grid merge: each waits until its rows' counters
 // have reached the number of their parts, reads these agent-coherently, writes the final rows and sets the counters back to zero. Workgroups are
 // dispatched in the grid's order, so whatever they wait for is running or done when they start, and waits for nothing itself; the wait is
-// bounded all the same, a row past it is not a number. (Merged by whichever part comes last instead: a tile that comes last has up to 128 rows
+// bounded all the same: a row past it is not a number, here and in every launch on the same counters, whose parts of before may yet come.
+// So counters are a step's own (or cleared before the launch). (Merged by whichever part comes last instead: a tile that comes last has up to 128 rows
 // of heads to merge alone, 20 - 40 us; 64 rows of 1344 keys 82 -> 85 us, 30 rows 54 -> 77.)
 //
 // us of a layer's attention, tile and decode launch / this one (Llama-3-8B heads, 18000 shared keys; caches not resident): 64 rows of 1344
@@ -25,7 +26,7 @@ constexpr int NW = 4, NSLOT = 2, ROWS = 32 * NW;             // a tile's waves, 
 constexpr int TILE_LDS = tile3::lds_bytes<NSLOT>();
 constexpr int MAXS = 64;                                     // parts of a row
 constexpr int PRE = 16;                                      // row_parts: a row's parts, and above this bit those that tiles left in bf16
-constexpr int POLLS = 1 << 24;                               // (of about a us: seconds)
+constexpr int LOST = -(1 << 30);                             // a counter whose row was given up: parts that come later leave it below zero
 }  // namespace mixed
 
 // a row's parts: [rows, Hq, S, 128] and lse [rows, Hq, S]
@@ -128,7 +129,7 @@ __global__ __launch_bounds__(256, 2) void attn_mixed_kernel(const TileItem* __re
                                                             float* __restrict__ part, float* __restrict__ lse,
                                                             bf16* __restrict__ pre, int S_total, float scale_log2,
                                                             bf16* __restrict__ out, int64_t out_stride,
-                                                            int* __restrict__ counters, AltPart ap) {
+                                                            int* __restrict__ counters, int polls, AltPart ap) {
   using namespace mixed;
   __shared__ __attribute__((aligned(16))) char smem[TILE_LDS];
   static_assert(sizeof(DecodeSmem<128>) <= TILE_LDS, "a piece's LDS is a tile's");
@@ -167,15 +168,21 @@ __global__ __launch_bounds__(256, 2) void attn_mixed_kernel(const TileItem* __re
   int* s_ok = reinterpret_cast<int*>(smem);
   if (tid < tw) {
     const int row = row0 + tid;
-    int need = row < n_rows ? row_parts[row] & ((1 << PRE) - 1) : 0;
-    // (a host bug otherwise: nothing is read; rows between the decode rows and the new turns' have no parts)
-    const bool fits = need <= min(MAXS, row < B ? S_total : ap.S) && (row < B || row >= ap.tok_off);
-    need = fits ? need : 0;
-    int* c = counters + (int64_t)min(row, n_rows - 1) * Hkv + kvh;
-    int polls = POLLS;
-    while (need > 0 && __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need && --polls > 0) __builtin_amdgcn_s_sleep(8);
-    if (need > 0) __hip_atomic_store(c, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_ok[tid] = need > 0 ? (polls > 0 ? need : -1) : 0;
+    int n = row < n_rows ? row_parts[row] & ((1 << PRE) - 1) : 0;
+    if (n > 0) {
+      // (parts that do not fit, a host bug: nothing of them is read. Rows between the decode rows and the new turns' have none.)
+      const bool fits = n <= min(MAXS, row < B ? S_total : ap.S) && (row < B || row >= ap.tok_off);
+      int* c = counters + (int64_t)row * Hkv + kvh;
+      int left = fits ? polls : 0, got = 0;
+      while (left > 0 && (got = __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >= 0 && got < n) {
+        --left;
+        __builtin_amdgcn_s_sleep(8);
+      }
+      const bool ok = left > 0 && got >= n;
+      __hip_atomic_store(c, ok ? 0 : LOST, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      n = ok ? n : -1;
+    }
+    s_ok[tid] = n;
   }
   __syncthreads();
   const int i = tid >> 4, row = row0 + i / G, head = kvh * G + i % G, n = s_ok[i / G];
@@ -185,7 +192,7 @@ __global__ __launch_bounds__(256, 2) void attn_mixed_kernel(const TileItem* __re
 #pragma unroll
     for (int j = 0; j < 8; ++j) o[8 * (tid & 15) + j] = (bf16)__builtin_nanf("");
   } else if (row < B) {
-    mixed_merge_row(MixedParts{part, pre, lse, S_total}, (int64_t)row * Hq + head, row_parts[row] >> PRE, n, o);
+    mixed_merge_row(MixedParts{part, pre, lse, S_total}, (int64_t)row * Hq + head, min(row_parts[row] >> PRE, n), n, o);
   } else {
     mixed_merge_row(MixedParts{ap.part, nullptr, ap.lse, ap.S}, (int64_t)(row - ap.tok_off) * Hq + head, 0, n, o);
   }
@@ -193,13 +200,13 @@ __global__ __launch_bounds__(256, 2) void attn_mixed_kernel(const TileItem* __re
 
 // titems: int32 [n_tiles, 8] as attn_tile.h, ditems [n_pieces, 8] as attn_decode.h; row_parts [n_rows]: parts of every row that this launch
 // merges (0: none of it; the parts of a row of new turns are tiles flagged alt), and above bit 16 those that tiles leave in bf16.
-// counters: [n_rows, Hkv] zeros.
+// counters: [n_rows, Hkv] zeros, zeros again behind it but for rows that were given up. polls: looks at a counter (of about a us) before that.
 extern "C" hipError_t kafka_launch_attn_mixed(const int* titems, int n_tiles, const int* ditems, int n_pieces,
                                              const int* row_parts, int n_rows, const bf16* q, int64_t q_stride,
                                              const void* k_cache, const void* v_cache, int Hkv, int G,
                                              const int* block_tables, int bt_stride, const int* q_limit, int B,
                                              float* part, float* lse, bf16* pre, int S_total, float scale, bf16* out,
-                                             int64_t out_stride, int* counters, float* alt_part, float* alt_lse, int alt_S,
+                                             int64_t out_stride, int* counters, int polls, float* alt_part, float* alt_lse, int alt_S,
                                              int alt_tok_off, hipStream_t st) {
   if (n_tiles + n_pieces == 0 || n_rows == 0) return hipSuccess;
   if (G < 1 || G > 8 || 16 % G || n_tiles < 0 || n_pieces < 0 || n_rows < B) return hipErrorInvalidValue;
@@ -211,7 +218,7 @@ extern "C" hipError_t kafka_launch_attn_mixed(const int* titems, int n_tiles, co
   attn_mixed_kernel<<<dim3(Hkv, n_tiles + n_pieces + n_merge), 256, 0, st>>>(
       reinterpret_cast<const TileItem*>(titems), n_tiles, reinterpret_cast<const DecodeItem*>(ditems), n_pieces, row_parts, n_rows, q,
       q_stride, static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), Hkv, G, block_tables, bt_stride, q_limit, B, part,
-      lse, pre, S_total, scale * 1.4426950408889634f, out, out_stride, counters, AltPart{alt_part, alt_lse, alt_S, alt_tok_off});
+      lse, pre, S_total, scale * 1.4426950408889634f, out, out_stride, counters, polls, AltPart{alt_part, alt_lse, alt_S, alt_tok_off});
   return hipGetLastError();
 }
 

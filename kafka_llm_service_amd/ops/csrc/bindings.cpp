@@ -38,7 +38,7 @@ hipError_t kafka_launch_attn_decode(const bf16* q, int64_t q_stride, const void*
 hipError_t kafka_launch_attn_mixed(const int* titems, int n_tiles, const int* ditems, int n_pieces, const int* row_parts,
                                    int n_rows, const bf16* q, int64_t q_stride, const void* k_cache, const void* v_cache, int Hkv, int G,
                                    const int* block_tables, int bt_stride, const int* q_limit, int B, float* part, float* lse,
-                                   bf16* pre, int S_total, float scale, bf16* out, int64_t out_stride, int* counters,
+                                   bf16* pre, int S_total, float scale, bf16* out, int64_t out_stride, int* counters, int polls,
                                    float* alt_part, float* alt_lse, int alt_S, int alt_tok_off, hipStream_t st);
 hipError_t kafka_launch_attn_prefill(const void* items, int n_items, const bf16* q, int64_t q_stride,
                                      const void* k_cache, const void* v_cache, int fp8, int Hkv, int G, int D,
@@ -401,7 +401,7 @@ static void attn_decode(at::Tensor q, at::Tensor k_cache, at::Tensor v_cache, at
 static void attn_mixed(at::Tensor prefix_items, at::Tensor decode_items, at::Tensor q, at::Tensor k_cache, at::Tensor v_cache,
                        at::Tensor block_tables, at::Tensor q_limit, at::Tensor part, at::Tensor lse, at::Tensor pre,
                        at::Tensor row_parts, double scale, at::Tensor out, at::Tensor counters, c10::optional<at::Tensor> alt_part, c10::optional<at::Tensor> alt_lse,
-                       int64_t alt_tok_off) {
+                       int64_t alt_tok_off, int64_t polls) {
   CHECK_CUDA(q); CHECK_DT(q, at::kBFloat16); check_cache_pair(k_cache, v_cache);
   CHECK_DT(block_tables, at::kInt); CHECK_DT(part, at::kFloat); CHECK_DT(lse, at::kFloat); CHECK_DT(pre, at::kBFloat16);
   CHECK_DT(out, at::kBFloat16); CHECK_DT(q_limit, at::kInt);
@@ -443,7 +443,7 @@ static void attn_mixed(at::Tensor prefix_items, at::Tensor decode_items, at::Ten
                                      decode_items.size(0), row_parts.data_ptr<int>(), R, bptr(q), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), Hkv, Hq / Hkv,
                                      block_tables.data_ptr<int>(), block_tables.stride(0), q_limit.data_ptr<int>(), B,
                                      part.data_ptr<float>(), lse.data_ptr<float>(), bptr(pre), S, scale, bptr(out), out.stride(0),
-                                     counters.data_ptr<int>(), ap, al, S2, (int)alt_tok_off, cur_stream()));
+                                     counters.data_ptr<int>(), (int)std::min<int64_t>(polls, 1 << 24), ap, al, S2, (int)alt_tok_off, cur_stream()));
 }
 
 static void attn_prefill(at::Tensor items, at::Tensor q, at::Tensor k_cache, at::Tensor v_cache,
@@ -1328,7 +1328,7 @@ PYBIND11_MODULE(_kafka_ops, m) {
   m.def("attn_mixed", &attn_mixed, py::arg("prefix_items"), py::arg("decode_items"), py::arg("q"), py::arg("k_cache"),
         py::arg("v_cache"), py::arg("block_tables"), py::arg("q_limit"), py::arg("part"), py::arg("lse"), py::arg("pre"),
         py::arg("row_parts"), py::arg("scale"), py::arg("out"), py::arg("counters"), py::arg("alt_part") = py::none(), py::arg("alt_lse") = py::none(),
-        py::arg("alt_tok_off") = 0);
+        py::arg("alt_tok_off") = 0, py::arg("polls") = 1 << 24);
   m.def("attn_prefill", &attn_prefill, py::arg("items"), py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
         py::arg("block_tables"), py::arg("q_limit"), py::arg("out"), py::arg("out_part"), py::arg("lse_part"),
         py::arg("scale"), py::arg("variant") = 0, py::arg("alt_part") = py::none(), py::arg("alt_lse") = py::none(),

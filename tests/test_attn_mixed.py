@@ -57,7 +57,7 @@ def _case(groups, own, hkv, G, seed, dev, loose=0, alt=0):
                 items=torch.tensor(items, dtype=torch.int32).reshape(-1, 8).to(dev))
 
 
-def _run(c, target=1344, dec=None):
+def _run(c, target=1344, dec=None, edit=None, **kw):
     dev, B, Hq = c["q"].device, c["B"], c["q"].shape[1]
     if dec is None:
         dec = decode_items(c["lens"], c["kv0"], c["npre"], c["k"].shape[1], target)
@@ -72,8 +72,10 @@ def _run(c, target=1344, dec=None):
         parts[b] = n + npre | npre << 16
     parts[B:] = int(c["npre"][0])
     alt = (torch.zeros(T - B, Hq, S, 128, device=dev), torch.full((T - B, Hq, S), float("-inf"), device=dev)) if T > B else ()
+    if edit:
+        edit(parts)
     ops.attn_mixed(c["items"], torch.tensor(dec, device=dev), c["q"], c["k"], c["v"], c["bt"], c["lim"], part, lse, pre, parts.to(dev),
-                   128 ** -0.5, out, *alt)
+                   128 ** -0.5, out, *alt, **kw)
     return out
 
 
@@ -130,6 +132,38 @@ def test_keys_that_are_no_numbers_reach_their_rows_only(cuda):
     c["v"][c["bt"][0, 3]] = float("nan")           # a page that all share
     out = _run(c)
     assert out.isnan().any(-1).all()
+
+
+def _more(row, n):
+    def edit(parts):
+        parts[row] += n
+    return edit
+
+
+@pytest.mark.gpu
+def test_rows_whose_parts_do_not_come_are_no_numbers_and_stay_alone(cuda):
+    """More parts than a merge reads (nothing waits for them), one part more than comes (after a bounded wait): that row is not a number, in this
+    launch and in the next ones on its counters, and no other row is touched; on clear counters all is as before."""
+    c = _case([(6, 40, 3)], [50, 60, 900, 80, 90, 100], 2, 4, 5, cuda)
+    want, rest = _run(c), [0, 1, 3, 4, 5]
+    assert not want.isnan().any()
+    for row, n in ((2, 70), (1, 1)):
+        rest = [r for r in range(6) if r != row]
+        counters = torch.zeros(6 * 2, dtype=torch.int32, device=cuda)
+        for edit in (_more(row, n), None, None):
+            out = _run(c, edit=edit, counters=counters, polls=1 << 16)
+            assert torch.equal(out[rest], want[rest]) and out[row].isnan().all()
+            lost = counters.view(6, 2)
+            assert (lost[row] < -(1 << 29)).all() and not lost[rest].any()
+        assert torch.equal(_run(c, edit=_more(row, n), polls=1 << 16)[rest], want[rest])
+        assert torch.equal(_run(c), want)          # (the stream's counters, cleared before each launch)
+        assert torch.equal(_run(c, counters=counters.zero_()), want) and not counters.any()
+
+
+def test_rows_of_more_parts_than_a_merge_reads_are_no_numbers():
+    c = _case([(6, 40, 3)], [50, 60, 700, 80, 90, 100], 2, 4, 5, "cpu")
+    want, out = _run(c), _run(c, edit=_more(2, 70))
+    assert out[2].isnan().all() and torch.equal(out[[0, 1, 3, 4, 5]], want[[0, 1, 3, 4, 5]])
 
 
 def test_plans_of_a_cascade_step_cover_every_key_once():
@@ -244,6 +278,7 @@ def _check_plan(r, h):
             assert bool(alt) == (t >= B)
             seen[t].append((lo, hi, slot))
     joined = [t for t in range(B, h.T) if seen[t]]
+    assert not meta.counters.any() and meta.counters.numel() == h.mixed * r.model.hkv
     if joined:                                     # (their partials lie in a buffer of their rows)
         assert meta.alt_off == joined[0] and meta.alt_part.shape[0] == joined[-1] + 1 - joined[0] and h.mixed == joined[-1] + 1
         assert max(a[2] for t in joined for a in seen[t]) < meta.alt_part.shape[2] and meta.alt_part.numel() * 4 <= 1 << 30
@@ -327,7 +362,7 @@ def _steps(hkv, G, shared, rows, own, portions, parts, dev):
     if dev != "cpu":
         first = out.clone()
         paged_attention(q.to(dev), k.to(dev), v.to(dev), meta, out)
-        assert torch.equal(first, out)
+        assert torch.equal(first, out) and not meta.counters.any()
     assert not out.isnan().any()
     o, starts = h.nbt * h.bt_w, [h.B]
     bt, limit = torch.from_numpy(h.i32[:o].reshape(h.nbt, -1)), h.i32[o:o + h.T]

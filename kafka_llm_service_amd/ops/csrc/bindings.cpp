@@ -692,7 +692,8 @@ static void wstream_fin(int64_t fin, at::Tensor x, at::Tensor wt, c10::optional<
     fa.nss = ss_in->size(0);
     fa.ss_ld = ss_in->stride(0);
   }
-  const int kw = mt == 2 && kc == 256 && K / s / kc >= 4 ? 2 : 1;  // (the wstream_gemm rules above)
+  // (wstream_gemm's rules, but for its exception of up to 32 rows, whose prefetch stays pinned here: timed without a finisher only)
+  const int kw = mt == 2 && kc == 256 && K / s / kc >= 4 ? 2 : 1;
   const int pin = mt != 3 && K / s / kc >= 3 ? 1 : 0;
   bf16* yp = nullptr;
   int64_t ldy = 0;

@@ -441,7 +441,8 @@ __global__ __launch_bounds__(NTH) void side_dwa_reg_kernel(float* __restrict__ x
       }
       stv<VEC>(x + t * d + i, xv[k]);
     }
-  }  if constexpr (NEXT) {
+  }
+  if constexpr (NEXT) {
     float mean, rstd;
     reg_stats<VEC, NTH, NV>(xv, d, nx.eps, red, mean, rstd);
 #pragma unroll
@@ -1626,7 +1627,6 @@ hipError_t kafka_hy_latent_prep(int f32, const void* qgd, int64_t qs, int T, int
                                 void* cache, void* cache_t, int page, const int64_t* slots, void* q_rot,
                                 hipStream_t st) {
   if (T <= 0) return hipSuccess;
-  // PREPFIG
   // as many as the queries fill, up to two rounds of the chip (a thread takes more elements then)
   const int64_t need = ((int64_t)H * rd + NT - 1) / NT, parts = std::min<int64_t>(need, std::max(4096 / T, 1));
   DISPATCH_AT(f32, latent_prep_kernel<AT><<<dim3((unsigned)T, 1 + (unsigned)parts), NT, 0, st>>>((const AT*)qgd, qs, H, dim, rd, R, dkv_off,

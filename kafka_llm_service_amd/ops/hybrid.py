@@ -856,7 +856,7 @@ def window_attn(q, k_cache, v_cache_t, block_tables, tok_seg, positions, H: int,
     (int32 [n, 4] = (first row, tokens, segment, 0), at most ``sig_tile_tokens(H, G)`` tokens of one segment each) and
     sizes it takes, bf16 runs on the matrix cores; else one wave per (row, head) on the vector units, keys in order,
     whatever the batch. ``max_keys`` (the step's longest context) lets a launch of few tiles split its key ranges
-    over more workgroups (``sig_splits``); a merge pass combines them.
+    over more workgroups (``window_splits``); a merge pass combines them.
     ``shared_keys``: q is [T, H G D] - every query head is a row of the whole key row's size and its score is the
     product with ALL G key heads of a token (queries that hold a mix over the heads, see ``rope_kv_store``); values
     stay per key/value head. The result is multiplied by ``out_scale``; ``out`` may be a column slice.

@@ -965,7 +965,9 @@ class ModelRunner:
         """Whether a step's prefix tiles and decode pieces go out as one launch (ops.attn_mixed), with ``joined`` rows of new turns. us of a
         layer's attention, two launches / one (18000 shared keys): 64 rows of 1344 keys 84 / 67, 96 of 900 99 / 75, 128 of 300 83 / 63, 30 of 1344
         53 / 47, 61 of 1344 and 161 rows of new turns 135 / 110, 64 of 300 behind 3000 35 / 25, 20 of 300 33.5 / 32, 8 of 1000 behind
-        9000 27 / 26.5; the tiles alone are as fast in one launch of 256 rows each: 64 of 100 36.6 / 37.9, 40 of 60 33 / 37."""
+        9000 27 / 26.5; the tiles alone are as fast in one launch of 256 rows each: 64 of 100 36.6 / 37.9, 40 of 60 33 / 37. One row tile of 8 heads
+        is even on average behind 9000 - 18000 keys (157 steps of 4 - 32 rows with 300 - 2600 keys of their own 0.87 - 1.19), 0.85 of two launches
+        behind up to 8200; 0.9 with 4 heads behind any. With new turns: ``_plan_cascade``."""
         if not (self.mixed_attn and self.cascade_bf16 and self.graphs is None and not self.fixed_decode_items):
             return False
         if joined:

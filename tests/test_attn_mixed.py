@@ -341,6 +341,15 @@ def test_partials_past_what_one_launch_addresses_are_two_launches(monkeypatch):
         assert _planned(*batch)[1].mixed
 
 
+def test_plans_of_one_launch_travel_whole():
+    h = _planned(8, 4, 1024, 5, 200, [(90, 6000), (300, None), (41, 3000)])[1]
+    z = np.zeros(0, np.float32)
+    got, _ = mr.unpack_plan(*mr.pack_plan(h, mr.SampleParams(z, z, z.astype(np.int32), z.astype(np.int64), None, True)))
+    assert h.mixed and h.alt_slots
+    assert all(getattr(got, f) == getattr(h, f) for f in mr._PLAN_SCALARS)
+    assert np.array_equal(got.i32, h.i32) and np.array_equal(got.i64, h.i64)
+
+
 #: (kv heads, G, shared, decode rows, their own keys, portions, parts of the longest row): as many parts as a launch merges; a turn's tile cut
 #: into several, some of whose pieces lie past the first ones' limits; a cold prompt between and before joined turns, both kinds of splits
 #: beside each other; whole tiles of one head

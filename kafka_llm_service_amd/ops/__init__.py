@@ -414,8 +414,6 @@ def linear_small(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 # 11936 timings (14 shapes of width 2048 and 4096, 70 - 4099 rows, every tile, one to eight splits; weights from memory): a time is off by 3 - 5 %
 # (the worst by a third), the tile and split that the figures pick by 0.5 % on average from the best. Heights of 160 and 224 rows and the weights past
 # the caches take 1 - 2 % off steps of 129 - 1024 rows and 3 - 4 % off longer ones (129 rows of 14336 -> 4096 35 -> 30, 1300 of 4096 -> 14336 15 %).
-# (5, 4) of one row tile by 2000 timings more, with K of 7168 and 14336 and 10240 - 18560 columns, where a CU takes in less: 0.554 of them by the former ones
-# alone (129 rows of 7168 -> 18560 83 us, 73 now as before those heights, -> 4096 29.1, 27.7; 10240 columns are 10 % behind).
 TILES = {
     (8, 8): ((1.8, 8.8, 1.208, 0.60), (1.4, 7.2, 1.173, 0.97)),
     (8, 6): ((2.3, 5.1, 0.982, 0.78), (2.7, 4.0, 0.957, 1.13)),
@@ -426,7 +424,7 @@ TILES = {
     (5, 8): ((2.2, 4.0, 0.865, 0.85), (2.3, 4.2, 0.869, 1.23)),
     (8, 4): ((1.4, 3.8, 0.734, 0.96), (2.0, 3.0, 0.723, 1.32)),
     (7, 4): ((1.2, 4.7, 0.661, 1.00), (1.7, 4.1, 0.665, 1.43)),
-    (5, 4): ((1.2, 2.2, 0.550, 1.33), (1.8, 2.9, 0.600, 1.37)),
+    (5, 4): ((1.2, 2.2, 0.550, 1.33), (1.8, 2.9, 0.554, 1.37)),
     (4, 8): ((1.5, 2.3, 0.808, 1.09), (1.4, 4.1, 0.833, 1.19)),
     (4, 6): ((1.5, 2.5, 0.648, 1.24), (1.6, 3.9, 0.663, 1.25)),
     (4, 4): ((3.3, 0.0, 0.464, 1.05), (3.9, 0.0, 0.504, 1.18)),

@@ -51,12 +51,6 @@ def test_lengths_share_a_search():
             assert up[0] <= own[0] * (1 + 64 / M)
 
 
-@pytest.mark.parametrize("M", [129, 145, 160])
-def test_deep_wide_products_of_one_row_tile_stay_in_two_splits(M):
-    """Measured with the slabs' sum, us at 129 / 160 rows of 7168 -> 18560: (6, 6) in two splits 64 / 68, (5, 4) whole 76 / 80, (5, 8) in two 72 / 77."""
-    assert ops.tile_plan(M, 18560, 7168) == ops.tile_plan(M, 18560, 7168, "slabs") == (6, 6, 2)
-
-
 def test_long_products_on_the_cpu():
     """Without a GPU linear_long is the plain product, from either weight, whatever the strides of x."""
     w = torch.randn(96, 128)

@@ -1316,8 +1316,10 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(const AT* __restrict__ xb
 // The same, four columns a thread. What bounds it is the state, read and written: a workgroup asks for 32 KB of its head's (N P <= 8192: all of
 // it) in 16-byte loads before anything else, B, C and the step size arrive meanwhile, and the state goes past the caches'
 // retention both ways (it is next read a step later). 64 segments of 128 heads of 64 x 128: 127 -> 93 us (4.2 -> 5.8 TB/s; without the hints 104),
-// 16 segments 36 -> 25, one 11 -> 5.2, 200 of 16 heads of 32 x 16 10.6 -> 8.3.
-template <typename AT>
+// 16 segments 36 -> 25, one 11 -> 5.2, 200 of 16 heads of 32 x 16 10.6 -> 7.0.
+// RN: rows a thread has in flight, as many as it has at all up to eight. (With eight always the loads of rows that are not there are more than
+// the state of 16 rows: us, the kernel above / so / as many: 39 segments of 128 heads of 64 x 16 16.9 / 18.6 / 14.3, 147 of 64 heads 29.3 / 31.4 / 23.8.)
+template <typename AT, int RN>
 __global__ __launch_bounds__(256) void ssm_step_vec4_kernel(const AT* __restrict__ xbc, int64_t xs,
                                                             const AT* __restrict__ proj, int64_t ps, int dt_off,
                                                             const float* __restrict__ dt_bias,
@@ -1325,7 +1327,6 @@ __global__ __launch_bounds__(256) void ssm_step_vec4_kernel(const AT* __restrict
                                                             int heads, int P, int N, int G, int NG,
                                                             const int* __restrict__ seg, float* __restrict__ state,
                                                             float* __restrict__ y, int64_t ys) {
-  constexpr int RN = 8;
   __shared__ __attribute__((aligned(16))) float part[1024];
   const int sgi = blockIdx.x / heads, h = blockIdx.x - sgi * heads;
   const int64_t row = seg[4 * sgi];
@@ -1795,8 +1796,12 @@ hipError_t kafka_hy_ssm_scan(int f32, const void* xbc, int64_t xs, const void* p
         k<<<R * heads, threads, 0, st>>>((const AT*)xbc, xs, (const AT*)proj, ps, dt_off, dt_bias, A_log, Dp, heads, P, N, G, NG, seg,
                                          state, y, ys);
       };
-      if (v4) a(ssm_step_vec4_kernel<AT>, P / 4 * NG);
-      else a(ssm_step_kernel<AT>, P * NG);
+      const int rows = (N + NG - 1) / NG;   // of a thread
+      if (!v4) a(ssm_step_kernel<AT>, P * NG);
+      else if (rows == 1) a(ssm_step_vec4_kernel<AT, 1>, P / 4 * NG);
+      else if (rows == 2) a(ssm_step_vec4_kernel<AT, 2>, P / 4 * NG);
+      else if (rows <= 4) a(ssm_step_vec4_kernel<AT, 4>, P / 4 * NG);
+      else a(ssm_step_vec4_kernel<AT, 8>, P / 4 * NG);
     });
     min_n = 2;
   }

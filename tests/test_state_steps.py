@@ -27,6 +27,7 @@ def close(got, want, bound):
     (4, 1, 0), (4, 300, 0),            # 256 row groups, more rows than one piece of them
     (8, 7, 0), (12, 128, 0),           # columns that do not divide the workgroup
     (64, 128, 0), (64, 129, 0), (64, 257, 0),   # one piece, one row more, two and one row
+    (64, 16, 0), (64, 17, 0), (64, 32, 0), (64, 33, 0), (64, 64, 0), (64, 65, 0),   # one, two, up to four rows a thread, and one more
     (252, 5, 0), (256, 32, 0), (256, 33, 0),    # the widest head
     (64, 128, 1), (30, 20, 0), (255, 9, 0)])    # a state off 16 bytes, odd columns: the kernel of single columns
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

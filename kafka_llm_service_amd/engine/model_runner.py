@@ -197,7 +197,7 @@ MIXED_PIECES = 768
 MIXED_JOINED = 2048         # rows of new turns that such a launch takes along
 MIXED_PART_BYTES = 1 << 31  # ... which takes the decode rows' partials below this (its merge's 32-bit offsets) ...
 MIXED_ALT_BYTES = 1 << 30   # ... and those of the new turns' rows, and what lies between them, up to this
-MIXED_FEW = 6               # prefix keys of its tiles beside a row's own, past which the two launches of before stay (one round of them)
+MIXED_FEW = 6               # prefix keys of its tiles beside rows' own, past which the two launches of before stay (one round of them)
 
 
 def mixed_tile_wgs(work: int, own: int, tiles: int, hkv: int) -> int:
@@ -965,16 +965,24 @@ class ModelRunner:
         """Whether a step's prefix tiles and decode pieces go out as one launch (ops.attn_mixed), with ``joined`` rows of new turns. us of a
         layer's attention, two launches / one (18000 shared keys): 64 rows of 1344 keys 84 / 67, 96 of 900 99 / 75, 128 of 300 83 / 63, 30 of 1344
         53 / 47, 61 of 1344 and 161 rows of new turns 135 / 110, 64 of 300 behind 3000 35 / 25, 20 of 300 33.5 / 32, 8 of 1000 behind
-        9000 27 / 26.5; the tiles alone are as fast in one launch of 256 rows each: 64 of 100 36.6 / 37.9, 40 of 60 33 / 37. One row tile of 8 heads
-        is even on average behind 9000 - 18000 keys (157 steps of 4 - 32 rows with 300 - 2600 keys of their own 0.87 - 1.19), 0.85 of two launches
-        behind up to 8200; 0.9 with 4 heads behind any. With new turns: ``_plan_cascade``."""
+        9000 27 / 26.5; the tiles alone are as fast in one launch of 256 rows each: 64 of 100 36.6 / 37.9, 40 of 60 33 / 37.
+        One row tile in as many parts as there can be, which are a workgroup a CU, stays with two launches unless the pieces are most of the work
+        (a step of four Llama layers of 8 heads, 2 - 32 rows, one launch / two: 8300 shared keys 0.96, 9000 1.02, 12000 1.02, 18000 1.01, the worst 1.06, up to
+        three times as many keys of their own as shared ones, 0.99 beyond; 8 rows of 2600 behind 18000 602 / 633 us; 16 and 32 heads, or 4, which do not
+        fill the chip so, 0.8 - 1 of the attention); so do two row tiles of nearly as much work and few pieces (33 - 64 rows behind 18000: 1.01 below half as many, 0.96
+        beyond; behind 9000 0.99). With new turns: ``_plan_cascade``."""
         if not (self.mixed_attn and self.cascade_bf16 and self.graphs is None and not self.fixed_decode_items):
             return False
         if joined:
             return self.retile_joins and self.join_suffix and joined <= MIXED_JOINED
+        tiles = sum(-(-n // self.mixed_tile) for n, _ in groups)
         work = sum(-(-n // self.mixed_tile) * p * PAGE for n, p in groups)
         own = int(seq_lens.sum()) - sum(n * p * PAGE for n, p in groups)
-        return work <= MIXED_FEW * own or work * self.model.hkv > 300000
+        if tiles == 1 and work > 256 * MAX_PREFIX_CHUNKS and 256 <= self.model.hkv * MAX_PREFIX_CHUNKS < 512:
+            return own >= 3 * work
+        if work * self.model.hkv > 300000:
+            return True
+        return work <= (2 if work * self.model.hkv > 200000 else MIXED_FEW) * own
 
     @staticmethod
     def _prefix_joins(bt: np.ndarray, B: int, pre: list, groups: list[tuple[int, int]],

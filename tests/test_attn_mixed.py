@@ -341,6 +341,18 @@ def test_partials_past_what_one_launch_addresses_are_two_launches(monkeypatch):
         assert _planned(*batch)[1].mixed
 
 
+@pytest.mark.parametrize("hkv,G,shared,rows,own,one", [
+    (8, 4, 8192, 8, 900, True), (8, 4, 8224, 8, 900, False), (8, 4, 9000, 2, 2600, False), (8, 4, 18000, 28, 900, False),   # one row tile in 32 parts
+    (8, 4, 9000, 32, 1344, True), (8, 4, 9000, 33, 300, True), (8, 8, 9000, 16, 900, False), (8, 8, 9000, 17, 900, True),   # ... beside enough pieces; two
+    (4, 8, 9000, 8, 900, True), (16, 2, 9000, 8, 900, True), (2, 4, 18000, 8, 900, True),   # parts that leave CUs idle, or are fewer
+    (8, 4, 18000, 40, 500, False), (8, 4, 18000, 40, 700, True), (8, 4, 9000, 40, 400, True), (8, 4, 18000, 96, 60, True)])
+def test_few_rows_behind_long_prefixes_take_two_launches(hkv, G, shared, rows, own, one):
+    r, h = _planned(hkv, G, shared, rows, own, [])
+    assert bool(h.mixed) == one and h.n_prefix_items
+    if one:
+        _check_plan(r, h)
+
+
 def test_plans_of_one_launch_travel_whole():
     h = _planned(8, 4, 1024, 5, 200, [(90, 6000), (300, None), (41, 3000)])[1]
     z = np.zeros(0, np.float32)

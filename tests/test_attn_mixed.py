@@ -279,6 +279,8 @@ def _check_plan(r, h):
             seen[t].append((lo, hi, slot))
     joined = [t for t in range(B, h.T) if seen[t]]
     assert not meta.counters.any() and meta.counters.numel() == h.mixed * r.model.hkv
+    at = meta.counters.storage_offset()            # (in cache lines of their own)
+    assert at % 64 == 0 and at >= o + h.mixed and not h.i32[at:at + -(-h.mixed * r.model.hkv // 64) * 64].any()
     if joined:                                     # (their partials lie in a buffer of their rows)
         assert meta.alt_off == joined[0] and meta.alt_part.shape[0] == joined[-1] + 1 - joined[0] and h.mixed == joined[-1] + 1
         assert max(a[2] for t in joined for a in seen[t]) < meta.alt_part.shape[2] and meta.alt_part.numel() * 4 <= 1 << 30

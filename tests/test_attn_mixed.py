@@ -1,5 +1,6 @@
 """Prefix tiles and decode pieces in one launch (``ops.attn_mixed``): rows against fp32 attention over their whole context, and the
 engine's plans for it."""
+import dataclasses
 import math
 import os
 import sys
@@ -387,6 +388,11 @@ def _steps(hkv, G, shared, rows, own, portions, parts, dev):
         paged_attention(q.to(dev), k.to(dev), v.to(dev), meta, out)
         assert torch.equal(first, out) and not meta.counters.any()
     assert not out.isnan().any()
+    alone = torch.full_like(out, float("nan"))     # (without the cold prompts' launch: their rows, between the joined ones too, are left alone)
+    paged_attention(q.to(dev), k.to(dev), v.to(dev), dataclasses.replace(meta, prefill_items=None, prefill_merge=[]), alone)
+    mine = torch.zeros(h.T, dtype=torch.bool)
+    mine[:h.mixed] = meta.row_parts.cpu() > 0
+    assert mine[:h.B].all() and torch.equal(alone[mine], out[mine]) and alone[~mine].isnan().all()
     o, starts = h.nbt * h.bt_w, [h.B]
     bt, limit = torch.from_numpy(h.i32[:o].reshape(h.nbt, -1)), h.i32[o:o + h.T]
     for m, _ in portions:

@@ -228,23 +228,23 @@ __device__ __forceinline__ void ring_tile(const RingArgs& A, char* smem, int e, 
   const int N = A.N, K = A.K;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, q = lane >> 4;
   const int nb = nt * 8 + 4 * (w & 1);             // this wave's first 32-column tile (N is a multiple of 128)
-  unsigned xo[R::PX], wo[R::DW];
+  unsigned xo[R::PX], wo[R::WR];
 #pragma unroll
   for (int u = 0; u < R::PX; ++u) {
     const int row = R::xrow(w, u, lane), m = min(row, rows - 1);   // rows past the segment reload a valid row, never stored
     const unsigned at = GATHER ? (unsigned)A.perm_tok[seg0 + m] : (unsigned)m;
-    xo[u] = at * (unsigned)(A.ldx * 2) + R::xbyte(row, lane);
+    xo[u] = at * (unsigned)(A.ldx * 2) + R::xbyte(row, u, lane);
   }
 #pragma unroll
-  for (int u = 0; u < R::DW; ++u)                  // (tiles past N reload the last, never stored)
+  for (int u = 0; u < R::WR; ++u)                  // (tiles past N reload the last, never stored)
     wo[u] = (unsigned)(min(nt * 8 + R::wtile(w, u), (N >> 5) - 1) * (K >> 4) + R::wblock(w, u)) * 1024u;
   ring::f32x4v acc[MT][8];
 #pragma unroll
   for (int a = 0; a < MT; ++a)
 #pragma unroll
     for (int b = 0; b < 8; ++b) acc[a][b] = ring::f32x4v{0.f, 0.f, 0.f, 0.f};
-  R::multiply(acc, smem, ring::buffer(GATHER ? A.X : A.X + (int64_t)seg0 * A.ldx), xo,
-              ring::buffer(A.Wt + (int64_t)e * (N >> 5) * (K >> 4) * 64), R::wlane(lane), wo, K / ring::BK, lane, w);
+  R::multiply(acc, smem, R::xbuffer(GATHER ? A.X : A.X + (int64_t)seg0 * A.ldx), xo,
+              ring::buffer(A.Wt + (int64_t)e * (N >> 5) * (K >> 4) * 64), R::wlane(lane), wo, K / R::BK, lane, w);
   if (nb >= (N >> 5)) return;
   if constexpr (EPI == EPI_COMBINE) {
 #pragma unroll

@@ -20,7 +20,7 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const bf16* __restr
                                                              const bf16x8* __restrict__ Wt, int M, int N, int K, int S,
                                                              bf16* __restrict__ Y, int64_t ldy, float* __restrict__ P,
                                                              int mode) {
-  using R = ring::Ring<MT, NT, true, WNT>;
+  using R = ring::Ring<MT, NT, true, WNT, OCC>;
   __shared__ __attribute__((aligned(1024))) char smem[R::LDS];
   // item -> (split, rows, columns): an XCD takes one contiguous stretch of them: of a split the row tiles of up to 2048 rows
   // side by side, then the next column tile, so that its weights leave memory once
@@ -33,22 +33,22 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const bf16* __restr
   // K in units of 64, split as evenly as they go
   const int units = K >> 6, u0 = (int)((int64_t)units * sp / S), u1 = (int)((int64_t)units * (sp + 1) / S);
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, q = lane >> 4;
-  unsigned xo[R::PX], wo[R::DW];
+  unsigned xo[R::PX], wo[R::WR];
 #pragma unroll
   for (int u = 0; u < R::PX; ++u) {            // rows past M reload the last, never stored
     const int row = R::xrow(w, u, lane);
-    xo[u] = (unsigned)min(row, rows - 1) * (unsigned)(ldx * 2) + R::xbyte(row, lane);
+    xo[u] = (unsigned)min(row, rows - 1) * (unsigned)(ldx * 2) + R::xbyte(row, u, lane);
   }
 #pragma unroll
-  for (int u = 0; u < R::DW; ++u)                  // (tiles past N reload the last, never stored)
+  for (int u = 0; u < R::WR; ++u)                  // (tiles past N reload the last, never stored)
     wo[u] = (unsigned)(min(nt * NT + R::wtile(w, u), (N >> 5) - 1) * (K >> 4) + R::wblock(w, u)) * 1024u;
   ring::f32x4v acc[MT][NT];
 #pragma unroll
   for (int a = 0; a < MT; ++a)
 #pragma unroll
     for (int b = 0; b < NT; ++b) acc[a][b] = ring::f32x4v{0.f, 0.f, 0.f, 0.f};
-  R::multiply(acc, smem, ring::buffer(X + (int64_t)row0 * ldx + 64 * u0), xo, ring::buffer(Wt + (int64_t)u0 * 4 * 64),
-              R::wlane(lane), wo, 2 * (u1 - u0), lane, w);
+  R::multiply(acc, smem, R::xbuffer(X + (int64_t)row0 * ldx + 64 * u0), xo, ring::buffer(Wt + (int64_t)u0 * 4 * 64),
+              R::wlane(lane), wo, u1 - u0, lane, w);
   // this lane: row 16 mt + r, columns 8 q .. of every 32-column tile
   const int nb = nt * NT + NT / 2 * (w & 1), nall = N >> 5;
 #pragma unroll

@@ -202,11 +202,9 @@ __global__ __launch_bounds__(256, 2) void grouped_wide_kernel(const bf16* __rest
 // leave in 16-byte pieces. An expert's last rows go on a tile of 64 or 128 rows where they fit one (the weights' way is then what it
 // takes, a third of a whole tile). What bounds it: the card lowers its clock to 1.9 - 2.0 GHz under these products, and the last
 // round of the chip.
-// Measured, us, before (stages of 32 for both operands, 64-bit addresses, whole tiles only, 2-byte stores) / now (random routing
-// and values, rows of 128 bytes a piece): 32768 entries of 16 experts, 4096 -> 5376 relu2 1325 / 1260, 5376 -> 4096 rows 1295 /
-// 1147; 3800 of 8, 4096 -> 2 x 14336 glu 887 / 847, 14336 -> 4096 rows 660 / 606; 5386 of 8, 4096 -> 2 x 4608 glu 423 / 404, 4608 -> 4096
-// rows 223 / 211. Activations in 64-byte pieces alone (half a cache line: twice the lines asked of the cache) 1303 and 1254 for the first
-// two. A workgroup that goes on to its next tile with the ring kept full gained nothing (the clock), its branches in the loop cost 5 %.
+// Measured, us, stages of 32 and 64 bytes of a row a store / units of 64 and results in whole cache lines (random routing
+// and values): 32768 entries of 16 experts, 4096 -> 5376 relu2 1132 / 1077, 5376 -> 4096 rows 1123 / 1084; 3800 of 8, 4096 -> 2 x 14336 glu 750 /
+// 732, 14336 -> 4096 rows 360 / 350, combined 382 / 375; 5386 of 8, 4096 -> 2 x 4608 glu 366 / 353, 4608 -> 4096 rows 196 / 188, combined 243 / 233.
 struct RingArgs {
   const bf16* X;
   int64_t ldx;
@@ -259,38 +257,32 @@ __device__ __forceinline__ void ring_tile(const RingArgs& A, char* smem, int e, 
         for (int j = 0; j < 8; ++j) atomicAdd(o + 16 * j, pw * acc[mt][j][i]);
       }
   } else {
-    // this lane: row 16 mt + r, columns 8 q .. of every tile
+    bf16* const y = A.Y + (int64_t)seg0 * A.ldy + (EPI == EPI_GLU ? nb * 16 : nb * 32);
+    const int tiles = EPI == EPI_GLU ? ((N >> 5) - nb) / 2 : (N >> 5) - nb;
+    float pw[MT];
+    if constexpr (EPI == EPI_ROWS) {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = 16 * (MT * (w >> 1) + mt) + r;
-      if (m >= rows) continue;
-      bf16* y = A.Y + (int64_t)(seg0 + m) * A.ldy + 8 * q;
-      const float pw = EPI == EPI_ROWS ? A.perm_w[seg0 + m] : 1.0f;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        if (EPI == EPI_GLU && (t & 1)) continue;   // tiles of 32: gate, up, gate, up
-        bf16x8 o;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float v = acc[mt][2 * t + (i >> 2)][i & 3];
-          if constexpr (EPI == EPI_ROWS) {
-            o[i] = (bf16)(pw * v);
-          } else if constexpr (EPI == EPI_RELU2) {
-            const float a = fmaxf(v, 0.f);
-            o[i] = (bf16)(a * a);
-          } else {
-            float g = v, u = acc[mt][(2 * t + 2 + (i >> 2)) & 7][i & 3], al = 1.0f;
-            if (A.glu_limit > 0.f) {   // (uniform) the clamped form
-              g = fminf(g, A.glu_limit);
-              u = fminf(fmaxf(u, -A.glu_limit), A.glu_limit) + 1.0f;
-              al = A.glu_alpha;
-            }
-            o[i] = (bf16)(g / (1.0f + __expf(-al * g)) * u);
-          }
-        }
-        *reinterpret_cast<bf16x8*>(y + (EPI == EPI_GLU ? (nb + t) >> 1 : nb + t) * 32) = o;
-      }
+      for (int mt = 0; mt < MT; ++mt) pw[mt] = A.perm_w[seg0 + min(16 * (MT * (w >> 1) + mt) + r, rows - 1)];
     }
+    auto value = [&](auto mc, auto c, int i) {
+      constexpr int mt = decltype(mc)::value, t = decltype(c)::value * (EPI == EPI_GLU ? 2 : 1);
+      const float v = acc[mt][2 * t + (i >> 2)][i & 3];
+      if constexpr (EPI == EPI_ROWS) {
+        return pw[mt] * v;
+      } else if constexpr (EPI == EPI_RELU2) {
+        const float a = fmaxf(v, 0.f);
+        return a * a;
+      } else {                                       // tiles of 32: gate, up, gate, up
+        float g = v, u = acc[mt][(2 * t + 2 + (i >> 2)) & 7][i & 3], al = 1.0f;
+        if (A.glu_limit > 0.f) {                     // (uniform) the clamped form
+          g = fminf(g, A.glu_limit);
+          u = fminf(fmaxf(u, -A.glu_limit), A.glu_limit) + 1.0f;
+          al = A.glu_alpha;
+        }
+        return g / (1.0f + __expf(-al * g)) * u;
+      }
+    };
+    R::template rows_bf16<EPI == EPI_GLU ? 2 : 4>(y, A.ldy, rows, tiles, lane, w, value);
   }
 }
 

@@ -169,13 +169,6 @@ struct Ring {
       ws = wn;
       ++v;
     };
-    // the zeros are in the accumulation registers before anything else: the compiler would write them in front of the first product of
-    // each, and knows of no wait between the two
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int j = 0; j < NT; ++j) asm volatile("" : "+a"(acc[i][j]));
-    __builtin_amdgcn_sched_barrier(0);
     each<NW>([&](auto first) {
       constexpr int f = decltype(first)::value;
       if (f < 2 || f < nu) {
@@ -183,6 +176,14 @@ struct Ring {
         each<PW>([&](auto u) { wpiece(u, f, f); });
       }
     });
+    __builtin_amdgcn_sched_barrier(0);
+    // the zeros are in the accumulation registers while the first pieces are on their way: the compiler would write them in front of the first
+    // product of each, and knows of no wait between the two
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) asm volatile("" : "+a"(acc[i][j]));
+    __builtin_amdgcn_sched_barrier(0);
     if (nu >= NW) vmcnt<NX * PX + NW * PW - P>();
     else vmcnt<0>();
     asm volatile("s_barrier" ::: "memory");
@@ -222,6 +223,68 @@ struct Ring {
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 15");
     __builtin_amdgcn_sched_barrier(0);
+  }
+
+  // The tile's results (SWAP). A lane holds eight columns in a run of one row, 16 rows x 4 runs a fragment; pairs of lanes (rows m, m + 1) trade
+  // pieces, so that a store takes eight rows of 128 bytes, whole cache lines, where 16 rows of 64 would take every line twice. Each kind of
+  // result is code of its own in one run: with the choice between them inside the loops a workgroup jumped through 60 KB of instructions
+  // that no cache held (256 x 256 bf16: 18.6 k cycles, 4.3 k so; 8192 rows of 4096 -> 4096 193 -> 181 us).
+  static __device__ __forceinline__ void trade(int odd, const f32x4v& p0, const f32x4v& p1, f32x4v& even_row, f32x4v& odd_row) {
+    f32x4v got;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)                      // (the neighbouring lane's)
+      got[i] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, odd ? p0[i] : p1[i]), 0xB1, 0xf, 0xf, true));
+    even_row = odd ? got : p0;
+    odd_row = odd ? p1 : got;
+  }
+  // value(mt, t, i): column i of the run in the wave's t-th 32-column tile of results; y: row 0, the wave's first column; rows, tiles: how many there are
+  template <int TILES, typename V>
+  static __device__ __forceinline__ void rows_bf16(bf16* y, int64_t ld, int rows, int tiles, int lane, int w, V&& value) {
+    const int r = lane & 15, q = lane >> 4, odd = r & 1;
+    auto run = [&](auto mt, auto t) {
+      bf16x8 o;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = (bf16)value(mt, t, i);
+      return __builtin_bit_cast(f32x4v, o);
+    };
+    each<MT>([&](auto mt) {
+      const int m = 16 * (MT * (w >> 1) + decltype(mt)::value) + (r & ~1);
+      bf16* const p = y + m * ld + 8 * q;
+      each<TILES / 2>([&](auto pair) {
+        constexpr int t = 2 * decltype(pair)::value;
+        f32x4v a, b;
+        trade(odd, run(mt, Num<t>()), run(mt, Num<t + 1>()), a, b);
+        if (t + odd < tiles) {
+          bf16* const c = p + 32 * (t + odd);
+          if (m < rows) *reinterpret_cast<f32x4v*>(c) = a;
+          if (m + 1 < rows) *reinterpret_cast<f32x4v*>(c + ld) = b;
+        }
+      });
+      if constexpr (TILES % 2) {
+        const f32x4v a = run(mt, Num<TILES - 1>());
+        if (TILES - 1 < tiles && m + odd < rows) *reinterpret_cast<f32x4v*>(p + odd * ld + 32 * (TILES - 1)) = a;
+      }
+    });
+  }
+  // the sums themselves; column(t): where the wave's t-th tile begins in a row of p
+  template <typename F>
+  static __device__ __forceinline__ void rows_f32(const f32x4v (&acc)[MT][NT], float* p, int64_t ld, int rows, int tiles, int lane,
+                                                  int w, F&& column) {
+    const int r = lane & 15, q = lane >> 4, odd = r & 1;
+    each<MT>([&](auto mt) {
+      constexpr int i = decltype(mt)::value;
+      const int m = 16 * (MT * (w >> 1) + i) + (r & ~1);
+      each<NT / 2>([&](auto tile) {
+        constexpr int t = decltype(tile)::value;
+        f32x4v a, b;
+        trade(odd, acc[i][2 * t], acc[i][2 * t + 1], a, b);
+        if (t < tiles) {
+          float* const c = p + m * ld + column(t) + 8 * q + 4 * odd;
+          if (m < rows) *reinterpret_cast<f32x4v*>(c) = a;
+          if (m + 1 < rows) *reinterpret_cast<f32x4v*>(c + ld) = b;
+        }
+      });
+    });
   }
 };
 

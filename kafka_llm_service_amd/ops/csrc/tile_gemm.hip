@@ -49,40 +49,33 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const bf16* __restr
     for (int b = 0; b < NT; ++b) acc[a][b] = ring::f32x4v{0.f, 0.f, 0.f, 0.f};
   R::multiply(acc, smem, R::xbuffer(X + (int64_t)row0 * ldx + 64 * u0), xo, ring::buffer(Wt + (int64_t)u0 * 4 * 64),
               R::wlane(lane), wo, u1 - u0, lane, w);
-  // this lane: row 16 mt + r, columns 8 q .. of every 32-column tile
-  const int nb = nt * NT + NT / 2 * (w & 1), nall = N >> 5;
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int m = 16 * (MT * (w >> 1) + mt) + r;
-    if (m >= rows) continue;
-#pragma unroll
-    for (int t = 0; t < NT / 2; ++t) {
-      if (nb + t >= nall) continue;
-      if (mode == OUT_BF16 || mode == OUT_RELU2) {
-        bf16x8 o;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float a = acc[mt][2 * t + (i >> 2)][i & 3], p = a < 0.f ? 0.f : a;   // (not a number stays)
-          o[i] = (bf16)(mode == OUT_RELU2 ? p * p : a);
-        }
-        *reinterpret_cast<bf16x8*>(Y + (int64_t)(row0 + m) * ldy + (nb + t) * 32 + 8 * q) = o;
-      } else if (mode == OUT_GLU || mode == OUT_GELU) {                // tiles of 32: gate, up, gate, up
-        if (t & 1) continue;
-        bf16x8 o;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float a = acc[mt][2 * t + (i >> 2)][i & 3], b = acc[mt][(2 * t + 2 + (i >> 2)) % NT][i & 3];
-          o[i] = (bf16)(gate_act(a, mode == OUT_GELU) * b);
-        }
-        *reinterpret_cast<bf16x8*>(Y + (int64_t)(row0 + m) * ldy + ((nb + t) >> 1) * 32 + 8 * q) = o;
-      } else {
-        // (gate | up order of interleaved tiles)
-        const int c = mode == OUT_SLAB ? (nb + t) * 32 : (((nb + t) & 1) ? N >> 1 : 0) + ((nb + t) >> 1) * 32;
-        float* p = P + ((int64_t)sp * M + row0 + m) * N + c + 8 * q;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) *reinterpret_cast<ring::f32x4v*>(p + 4 * h) = acc[mt][2 * t + h];
-      }
-    }
+  const int nb = nt * NT + NT / 2 * (w & 1), nall = N >> 5;   // this wave's first tile of 32 columns, all of them
+  if (nb >= nall) return;
+  auto sum = [&](auto m, auto c, int i) { return acc[decltype(m)::value][2 * decltype(c)::value + (i >> 2)][i & 3]; };
+  if (mode == OUT_SLAB || mode == OUT_SLAB_GLU) {
+    float* const p = P + ((int64_t)sp * M + row0) * N;
+    // (gate | up order of interleaved tiles)
+    if (mode == OUT_SLAB) R::rows_f32(acc, p, N, rows, nall - nb, lane, w, [&](int t) { return (nb + t) * 32; });
+    else R::rows_f32(acc, p, N, rows, nall - nb, lane, w, [&](int t) { return (((nb + t) & 1) ? N >> 1 : 0) + ((nb + t) >> 1) * 32; });
+    return;
+  }
+  bf16* const y = Y + (int64_t)row0 * ldy;
+  if (mode == OUT_BF16) {
+    R::template rows_bf16<NT / 2>(y + nb * 32, ldy, rows, nall - nb, lane, w, sum);
+  } else if (mode == OUT_RELU2) {
+    R::template rows_bf16<NT / 2>(y + nb * 32, ldy, rows, nall - nb, lane, w, [&](auto m, auto c, int i) {
+      const float a = sum(m, c, i), p = a < 0.f ? 0.f : a;   // (not a number stays)
+      return p * p;
+    });
+  } else if constexpr (NT % 4 == 0) {                        // tiles of 32: gate, up, gate, up
+    auto gated = [&](auto m, auto c, int i, bool gelu) {
+      constexpr int t = 2 * decltype(c)::value;
+      return gate_act(sum(m, ring::Num<t>(), i), gelu) * sum(m, ring::Num<t + 1>(), i);
+    };
+    if (mode == OUT_GLU)
+      R::template rows_bf16<NT / 4>(y + nb * 16, ldy, rows, (nall - nb) / 2, lane, w, [&](auto m, auto c, int i) { return gated(m, c, i, false); });
+    else
+      R::template rows_bf16<NT / 4>(y + nb * 16, ldy, rows, (nall - nb) / 2, lane, w, [&](auto m, auto c, int i) { return gated(m, c, i, true); });
   }
 }
 

@@ -411,24 +411,26 @@ def linear_small(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 # ---- dense products of long steps on wave-tiled weights (csrc/tile_gemm.hip) -------------------------------------------
 # (16-row parts, 16-column parts) of a wave's tile, 2 x 2 waves a workgroup -> us: of a launch, of a round of 256 workgroups, of 64 of K
 # in it, and of a MB/us of what is written, over 4.5; then the same of steps of up to 256 rows, where one row tile's weights pass the caches by. Fitted to
-# 11936 timings (14 shapes of width 2048 and 4096, 70 - 4099 rows, every tile, one to eight splits; weights from memory): a time is off by 3 - 5 %
-# (the worst by a third), the tile and split that the figures pick by 0.5 % on average from the best. Heights of 160 and 224 rows and the weights past
-# the caches take 1 - 2 % off steps of 129 - 1024 rows and 3 - 4 % off longer ones (129 rows of 14336 -> 4096 35 -> 30, 1300 of 4096 -> 14336 15 %).
+# 17197 timings (17 shapes of width 2048 and 4096, 129 - 4099 rows, every tile, one to eight splits; weights from memory), then to the choice that they
+# make: the tile and split that the figures pick take 1.0 % (slabs) and 1.7 % (bf16) longer than the best on average (1.8 and 2.4 by the figures
+# of the loop before; 222 rows of 14336 -> 4096 41 -> 36.5 us).
 TILES = {
-    (8, 8): ((1.8, 8.8, 1.208, 0.60), (1.4, 7.2, 1.173, 0.97)),
-    (8, 6): ((2.3, 5.1, 0.982, 0.78), (2.7, 4.0, 0.957, 1.13)),
-    (7, 8): ((2.2, 6.8, 1.096, 0.66), (1.0, 6.6, 1.089, 1.01)),
-    (6, 8): ((2.2, 5.8, 0.978, 0.72), (1.8, 5.5, 0.979, 1.13)),
-    (7, 6): ((2.5, 5.4, 0.873, 0.86), (1.9, 5.4, 0.878, 1.25)),
-    (6, 6): ((2.1, 4.3, 0.789, 0.93), (2.2, 4.0, 0.793, 1.40)),
-    (5, 8): ((2.2, 4.0, 0.865, 0.85), (2.3, 4.2, 0.869, 1.23)),
-    (8, 4): ((1.4, 3.8, 0.734, 0.96), (2.0, 3.0, 0.723, 1.32)),
-    (7, 4): ((1.2, 4.7, 0.661, 1.00), (1.7, 4.1, 0.665, 1.43)),
-    (5, 4): ((1.2, 2.2, 0.550, 1.33), (1.8, 2.9, 0.554, 1.37)),
-    (4, 8): ((1.5, 2.3, 0.808, 1.09), (1.4, 4.1, 0.833, 1.19)),
-    (4, 6): ((1.5, 2.5, 0.648, 1.24), (1.6, 3.9, 0.663, 1.25)),
-    (4, 4): ((3.3, 0.0, 0.464, 1.05), (3.9, 0.0, 0.504, 1.18)),
+    (8, 8): ((0.6, 0.0, 1.19, 1.06), (2.1, 5.0, 1.00, 0.92)),
+    (8, 6): ((1.0, 2.5, 0.974, 0.79), (3.5, 2.2, 0.876, 0.90)),
+    (7, 8): ((0.8, 0.8, 1.08, 1.01), (3.8, 1.9, 0.954, 1.01)),
+    (6, 8): ((0.6, 0.8, 0.951, 1.02), (4.4, 0.0, 0.845, 1.21)),
+    (7, 6): ((0.4, 2.2, 0.877, 0.95), (3.3, 2.0, 0.800, 0.98)),
+    (6, 6): ((0.8, 1.1, 0.791, 1.03), (2.9, 0.75, 0.746, 0.98)),
+    (5, 8): ((0.4, 0.3, 0.842, 1.17), (4.0, 0.0, 0.800, 1.22)),
+    (8, 4): ((0.3, 1.8, 0.688, 1.00), (2.5, 1.4, 0.679, 1.15)),
+    (7, 4): ((0.2, 1.5, 0.602, 1.18), (3.0, 0.0, 0.655, 1.32)),
+    (5, 4): ((0.2, 1.5, 0.519, 1.20), (1.0, 0.86, 0.544, 1.78)),
+    (4, 8): ((0.0, 0.3, 0.729, 1.14), (0.7, 0.1, 0.849, 1.33)),
+    (4, 6): ((1.0, 0.3, 0.620, 1.09), (1.4, 2.4, 0.602, 0.94)),
+    (4, 4): ((2.85, 0.57, 0.434, 0.65), (2.8, 0.0, 0.507, 0.74)),
 }
+# rows up to which the last row tile is a low one (tiles of more than 128 rows), and us of a round of those and 64 of K by the 16-column parts
+TILE_LOW, TILE_LOW_UNIT = 64, {8: 0.43, 6: 0.26, 4: 0.21}
 TILE_SPLITS = (1, 2, 4, 8)      # what the consumers of slabs load with all slabs in flight
 TILE_SLAB_BYTES = 1 << 28
 TILE_LIBRARY_N, TILE_MAX_M = 24576, 2560
@@ -443,12 +445,16 @@ def _tile_search(M: int, N: int, K: int, form: str, odd: int) -> tuple[float, tu
         if mt & 1 != odd or form == "glu" and nt % 4:
             continue                # (a wave holds whole gate, up pairs)
         launch, rnd, unit, out = figures[M <= 256]
-        items = -(-M // (32 * mt)) * -(-N // (32 * nt))
+        cols = -(-N // (32 * nt))
+        low = mt > 4 and M > 32 * mt and 0 < M % (32 * mt) <= TILE_LOW
+        items = (M // (32 * mt) if low else -(-M // (32 * mt))) * cols
         for s in TILE_SPLITS:
             if K // 64 < 2 * s or s > 1 and (form == "relu2" or 4 * s * M * N > TILE_SLAB_BYTES):
                 break
             mb = M * N / 4.5e6
-            t = launch + -(-items * s // 256) * (rnd + unit * (K // 64) / s) + out * mb * (4 * s if s > 1 else 2)
+            rounds = -(-items * s // 256)
+            more = -(-max(0, cols * s - (256 * rounds - items * s)) // 256) if low else 0   # rounds of low tiles past the last whole one
+            t = launch + (rounds + more) * rnd + (rounds * unit + more * TILE_LOW_UNIT[nt]) * (K // 64) / s + out * mb * (4 * s if s > 1 else 2)
             if s > 1:               # the slabs' way back in, beside that of a bf16 output; a launch of its own but for "slabs"
                 t += mb * (4 * s - 2) if form == "slabs" else 6 + mb * (4 * s + 2)
             if best is None or t < best[0]:
@@ -496,18 +502,45 @@ def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) 
     if library and M > TILE_MAX_M and \
             (M > (TILE_GLU_M if act else TILE_RAGGED_M if N % 256 else TILE_EVEN_M) or tiles <= (512 if act else 256)):
         return None
-    # (sizes up to the next multiple of the heights' 64 or 32 rows share a search, 15 us of the host, else each new length of a prompt pays it)
-    best, odd = _tile_best(-(-M // 64) * 64, N, K, form), _tile_odd(-(-M // 32) * 32, N, K, form)
-    if odd[0] < 0.98 * best[0]:     # (about what the figures cannot tell apart: 359 rows of 14336 -> 4096, 53.4 and 53.9 by them, a step takes 1 % more)
-        best = odd
+    best = _tile_pick(M, N, K, form)
     if library and M > (768 if tiles > 256 else 1024):
-        rows = M // DENSE_BLOCK * DENSE_BLOCK if dense_cut(M, N, K) else M
-        lib = 4 + -(-(-(-rows // 256) * -(-N // 256)) // 256) * 1.42 * (K // 64) + (20 if rows < M else 0)
-        if act:                     # (the activation's launch and its way to memory and back)
-            lib += 5 + (3 if form == "glu" else 4) * M * N / 4.5e6
-        if best[0] > lib * gain:
+        if best[0] > _library_us(M, N, K, form) * gain:
             return None
     return best[1]
+
+
+def _tile_pick(M: int, N: int, K: int, form: str) -> tuple[float, tuple[int, int, int]]:
+    # (sizes up to the next multiple of the heights' 64 or 32 rows share a search, 15 us of the host, else each new length of a prompt pays it)
+    best, odd = _tile_best(-(-M // 64) * 64, N, K, form), _tile_odd(-(-M // 32) * 32, N, K, form)
+    # (2 %: about what the figures cannot tell apart: 359 rows of 14336 -> 4096, 53.4 and 53.9 by them, a step takes 1 % more)
+    return odd if odd[0] < 0.98 * best[0] else best
+
+
+def _library_us(M: int, N: int, K: int, form: str) -> float:
+    """About what the library takes for a product of long steps: rounds of its 256 x 256 tiles, and the activation's launch."""
+    rows = M // DENSE_BLOCK * DENSE_BLOCK if dense_cut(M, N, K) else M
+    us = 4 + -(-(-(-rows // 256) * -(-N // 256)) // 256) * 1.42 * (K // 64) + (20 if rows < M else 0)
+    if form in ("glu", "relu2"):    # (the activation's launch and its way to memory and back)
+        us += 5 + (3 if form == "glu" else 4) * M * N / 4.5e6
+    return us
+
+
+@lru_cache(maxsize=4096)
+def long_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) -> tuple[int, int, int] | None:
+    """``tile_plan``, and past one round of the library's tiles what it leaves to the library where this kernel is faster since its loop has
+    one meeting of the waves per 64 of K. With an activation that is everywhere: us, library and activation / this kernel, 4096 -> 28672
+    2048 rows 375 / 360, 4099 745 / 690, 5600 1078 / 891, 8192 1369 / 1284; 4096 -> 9216 2700 rows 173 / 158, 5600 418 / 311; 2048 -> 14336 2048
+    rows 109 / 100, 6500 416 / 297; over 134 sizes of 1100 - 8192 rows 9 % less than by ``tile_plan`` alone (3072 rows of 4096 -> 10752, the
+    worst, 194 / 194). Without one, where the figures say so, and not where the library takes blocks of 4096 rows (4099 of 4096 -> 4096 101 /
+    113): 5600 rows of 4096 -> 9216 394 / 296, 2700 of 4096 -> 28672 552 / 451, 8192 of 4096 -> 12320 631 / 589; over 194 sizes 2 % less, the worst
+    2304 of 2048 -> 14336 99 / 106."""
+    plan = tile_plan(M, N, K, form, library)
+    if plan is not None or not library or M <= 768 or -(-M // 256) * -(-N // 256) <= 256 or \
+            tile_plan(M, N, K, form, False) is None:
+        return plan
+    if form in ("glu", "relu2") or M > 1024 and not dense_cut(M, N, K) and _tile_pick(M, N, K, form)[0] < _library_us(M, N, K, form):
+        return tile_plan(M, N, K, form, False)
+    return None
 
 
 def tile_ok(x: torch.Tensor, wt: torch.Tensor | None) -> bool:
@@ -535,7 +568,7 @@ def linear_long(x: torch.Tensor, w: torch.Tensor | None, wt: torch.Tensor | None
     """x @ w^T of a long step: on the tile kernel where the weight has a tiled copy ``wt`` (or is only that) and the plan says so, else
     the library. bf16, or with ``slabs`` maybe the split-K slabs (is_slab)."""
     if tile_ok(x, wt):
-        plan = tile_plan(x.shape[0], wt.shape[0] * 32, x.shape[1], "slabs" if slabs else "bf16", w is not None)
+        plan = long_plan(x.shape[0], wt.shape[0] * 32, x.shape[1], "slabs" if slabs else "bf16", w is not None)
         if plan is not None:
             y = linear_tile(x, wt, plan)
             return y if slabs or plan[2] == 1 else slab_reduce(y)
@@ -545,7 +578,7 @@ def linear_long(x: torch.Tensor, w: torch.Tensor | None, wt: torch.Tensor | None
 def linear_glu_long(x: torch.Tensor, wt: torch.Tensor, act: str = "silu", library: bool = True) -> torch.Tensor | None:
     """silu(x @ Wg^T) * (x @ Wu^T) of a long step from GLU-tiled weights (``act`` as in ``silu_mul``), None where the tile kernel does
     not take it or, with a row-major weight for it (``library``), the library is as fast."""
-    plan = tile_plan(x.shape[0], wt.shape[0] * 32, x.shape[1], "glu", library) if tile_ok(x, wt) else None
+    plan = long_plan(x.shape[0], wt.shape[0] * 32, x.shape[1], "glu", library) if tile_ok(x, wt) else None
     if plan is None:
         return None
     y = linear_tile(x, wt, plan, glu=True, act=act)
@@ -554,7 +587,7 @@ def linear_glu_long(x: torch.Tensor, wt: torch.Tensor, act: str = "silu", librar
 
 def linear_relu2_long(x: torch.Tensor, wt: torch.Tensor) -> torch.Tensor | None:
     """relu(x @ W^T)^2 of a long step, None where the tile kernel does not take it."""
-    plan = tile_plan(x.shape[0], wt.shape[0] * 32, x.shape[1], "relu2") if tile_ok(x, wt) else None
+    plan = long_plan(x.shape[0], wt.shape[0] * 32, x.shape[1], "relu2") if tile_ok(x, wt) else None
     return None if plan is None else linear_tile(x, wt, plan, relu2=True)
 
 

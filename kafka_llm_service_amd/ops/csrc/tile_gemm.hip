@@ -1,12 +1,13 @@
 // Dense products of long steps on wave-tiled weights: Y[M, N] = X[M, K] W[N, K]^T, bf16, fp32 sums (gfx950).
 //
-// Tiles of 128, 192 and 256 rows and columns (ring.h), K split over workgroups into fp32 slabs where a step has few rows: the host
-// picks by a model of the launch (ops.tile_plan). What bounds it: a whole round of 256 x 256 tiles takes 1.24 us per 64 of K
-// (1.7 PFLOP/s) and 7.6 us for its start and its results; smaller tiles are bound by what the L2s give the CUs, 65 - 72 GB/s each
-// whatever the tile (17 - 18 TB/s): 192 x 192 0.75 us per 64 of K, 256 x 128 0.71, 128 x 128 (two workgroups a CU) 0.45 each. So a tile is as
-// large as leaves no round of the chip half empty, and sizes between 128 and 256 pay: 2048 rows of 4096 -> 6144 on 256 x 256 91 us, on
-// 256 x 192 78; 2800 rows on 192 x 192 120, on 256 x 256 150. Tried: two of the four waves moving the weights alone, eight stages ahead
-// (3 % more: their latency is not what a step of 136 - 256 rows waits for).
+// Tiles of 128 - 256 rows and columns (ring.h), K split over workgroups into fp32 slabs where a step has few rows: the host
+// picks by a model of the launch (ops.tile_plan). What bounds it: a whole round of 256 x 256 tiles takes 1.2 - 1.35 us per 64 of K
+// (1.6 - 1.8 PFLOP/s, the card's clock under the values) and about 10 us for its start and its results; smaller tiles are bound by what the L2s
+// give the CUs, 65 - 75 GB/s each whatever the tile (17 - 19 TB/s): 192 x 192 0.79 us per 64 of K, 256 x 128 0.69, 128 x 128 (two workgroups a CU)
+// 0.43 each. So a tile is as large as leaves no round of the chip half empty, and sizes between 128 and 256 pay: 2048 rows of 4096 -> 6144 on
+// 256 x 256 95 us, on 256 x 192 74. Tried: workgroups that go on to their next tiles with the ring kept full (0.5 - 1.8 % of two to seven rounds:
+// the card lowers its clock by what the gaps were); K begun at another place for every column tile (0 - 2 %); two of the four waves moving the
+// weights alone, eight stages ahead (3 % more: their latency is not what a step of 136 - 256 rows waits for).
 #include "ring.h"
 
 namespace kafka {
@@ -14,25 +15,26 @@ namespace tg {
 
 enum { OUT_BF16 = 0, OUT_SLAB = 1, OUT_GLU = 2, OUT_SLAB_GLU = 3, OUT_RELU2 = 4, OUT_GELU = 5 };
 
-// MT, NT: 16-row and 16-column parts of a wave's tile (2 x 2 waves); OCC workgroups on a CU; WNT: of one row tile
+struct TileArgs {
+  const bf16* X;
+  int64_t ldx;
+  const bf16x8* Wt;
+  int M, N, K, S;
+  bf16* Y;
+  int64_t ldy;
+  float* P;
+  int mode;
+};
+
+// rows (at most 32 MT) rows from row0 on, 32 NT columns from tile nt on, split sp
 template <int MT, int NT, int OCC, bool WNT>
-__global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const bf16* __restrict__ X, int64_t ldx,
-                                                             const bf16x8* __restrict__ Wt, int M, int N, int K, int S,
-                                                             bf16* __restrict__ Y, int64_t ldy, float* __restrict__ P,
-                                                             int mode) {
+__device__ __forceinline__ void tile(const TileArgs& A, char* smem, int sp, int nt, int row0, int rows) {
   using R = ring::Ring<MT, NT, true, WNT, OCC>;
-  __shared__ __attribute__((aligned(1024))) char smem[R::LDS];
-  // item -> (split, rows, columns): an XCD takes one contiguous stretch of them: of a split the row tiles of up to 2048 rows
-  // side by side, then the next column tile, so that its weights leave memory once
-  const int rts = (M + R::BM - 1) / R::BM, nts = (N + R::BN - 1) / R::BN, tiles = rts * nts, total = tiles * S;
-  const int per = (total + 7) >> 3, k8 = blockIdx.x >> 3, item = (blockIdx.x & 7) * per + k8;
-  if (k8 >= per || item >= total) return;          // (uniform)
-  constexpr int GR = 2048 / R::BM;
-  const int sp = item / tiles, it = item - sp * tiles, g = it / (GR * nts), j = it - g * GR * nts, in_g = min(GR, rts - g * GR);
-  const int nt = j / in_g, row0 = (g * GR + j - nt * in_g) * R::BM, rows = min(R::BM, M - row0);
+  const int N = A.N, K = A.K, mode = A.mode;
+  const int64_t ldx = A.ldx, ldy = A.ldy;
   // K in units of 64, split as evenly as they go
-  const int units = K >> 6, u0 = (int)((int64_t)units * sp / S), u1 = (int)((int64_t)units * (sp + 1) / S);
-  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, q = lane >> 4;
+  const int units = K >> 6, u0 = (int)((int64_t)units * sp / A.S), u1 = (int)((int64_t)units * (sp + 1) / A.S);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   unsigned xo[R::PX], wo[R::WR];
 #pragma unroll
   for (int u = 0; u < R::PX; ++u) {            // rows past M reload the last, never stored
@@ -47,19 +49,19 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const bf16* __restr
   for (int a = 0; a < MT; ++a)
 #pragma unroll
     for (int b = 0; b < NT; ++b) acc[a][b] = ring::f32x4v{0.f, 0.f, 0.f, 0.f};
-  R::multiply(acc, smem, R::xbuffer(X + (int64_t)row0 * ldx + 64 * u0), xo, ring::buffer(Wt + (int64_t)u0 * 4 * 64),
+  R::multiply(acc, smem, R::xbuffer(A.X + (int64_t)row0 * ldx + 64 * u0), xo, ring::buffer(A.Wt + (int64_t)u0 * 4 * 64),
               R::wlane(lane), wo, u1 - u0, lane, w);
   const int nb = nt * NT + NT / 2 * (w & 1), nall = N >> 5;   // this wave's first tile of 32 columns, all of them
   if (nb >= nall) return;
   auto sum = [&](auto m, auto c, int i) { return acc[decltype(m)::value][2 * decltype(c)::value + (i >> 2)][i & 3]; };
   if (mode == OUT_SLAB || mode == OUT_SLAB_GLU) {
-    float* const p = P + ((int64_t)sp * M + row0) * N;
+    float* const p = A.P + ((int64_t)sp * A.M + row0) * N;
     // (gate | up order of interleaved tiles)
     if (mode == OUT_SLAB) R::rows_f32(acc, p, N, rows, nall - nb, lane, w, [&](int t) { return (nb + t) * 32; });
     else R::rows_f32(acc, p, N, rows, nall - nb, lane, w, [&](int t) { return (((nb + t) & 1) ? N >> 1 : 0) + ((nb + t) >> 1) * 32; });
     return;
   }
-  bf16* const y = Y + (int64_t)row0 * ldy;
+  bf16* const y = A.Y + (int64_t)row0 * ldy;
   if (mode == OUT_BF16) {
     R::template rows_bf16<NT / 2>(y + nb * 32, ldy, rows, nall - nb, lane, w, sum);
   } else if (mode == OUT_RELU2) {
@@ -79,6 +81,41 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const bf16* __restr
   }
 }
 
+// A last row tile of at most LOW rows is one of that height: its weights' way is then what it takes, a third of a whole tile. The whole tiles are
+// dealt out first, evenly, then those. us, before / now: 4099 rows of 4096 -> 28672 698 / 669, of 4096 -> 4096 152 / 112, of 14336 -> 4096 504 / 376;
+// 2060 rows of 4096 -> 4096 on 256 x 128 87 / 65. (One row tile alone, WNT, has a height that fits; tiles of 128 rows are low enough.)
+constexpr int LOW = 64;
+template <int MT>
+__host__ __device__ constexpr int low_rows(int M) {
+  return MT > 4 && M > 32 * MT && M % (32 * MT) <= LOW ? M % (32 * MT) : 0;
+}
+
+// MT, NT: 16-row and 16-column parts of a wave's tile (2 x 2 waves); OCC workgroups on a CU; WNT: of one row tile
+template <int MT, int NT, int OCC, bool WNT>
+__global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const TileArgs A) {
+  using R = ring::Ring<MT, NT, true, WNT, OCC>;
+  using L = ring::Ring<LOW / 32, NT, true, WNT, OCC>;
+  constexpr bool HAS_LOW = MT > 4 && !WNT;
+  __shared__ __attribute__((aligned(1024))) char smem[HAS_LOW && L::LDS > R::LDS ? L::LDS : R::LDS];
+  // item -> (split, rows, columns): an XCD takes one contiguous stretch of them: of a split the row tiles of up to 2048 rows
+  // side by side, then the next column tile, so that its weights leave memory once
+  const int low = HAS_LOW ? low_rows<MT>(A.M) : 0, rts = low ? A.M / R::BM : (A.M + R::BM - 1) / R::BM;
+  const int nts = (A.N + R::BN - 1) / R::BN, tiles = rts * nts, total = tiles * A.S;
+  const int per = (total + 7) >> 3, k8 = blockIdx.x >> 3, x8 = blockIdx.x & 7;
+  if (k8 < per) {
+    const int item = x8 * per + k8;
+    if (item >= total) return;                       // (uniform)
+    constexpr int GR = 2048 / R::BM;
+    const int sp = item / tiles, it = item - sp * tiles, g = it / (GR * nts), j = it - g * GR * nts, in_g = min(GR, rts - g * GR);
+    const int nt = j / in_g, row0 = (g * GR + j - nt * in_g) * R::BM;
+    tile<MT, NT, OCC, WNT>(A, smem, sp, nt, row0, min(R::BM, A.M - row0));
+  } else if constexpr (HAS_LOW) {
+    const int all = nts * A.S, lper = (all + 7) >> 3, item = x8 * lper + k8 - per;
+    if (!low || k8 - per >= lper || item >= all) return;
+    tile<LOW / 32, NT, OCC, WNT>(A, smem, item / nts, item % nts, rts * R::BM, low);
+  }
+}
+
 // act: 1, 3 W tiled as gate, up pairs (silu or gelu(gate) * up into Y, slabs in gate | up order), 2 relu squared into Y
 extern "C" hipError_t kafka_launch_tile_gemm(const bf16* X, int64_t ldx, const bf16* Wt, int M, int N, int K, int mt, int nt,
                                              int splits, int act, bf16* Y, int64_t ldy, float* P, hipStream_t st) {
@@ -92,15 +129,17 @@ extern "C" hipError_t kafka_launch_tile_gemm(const bf16* X, int64_t ldx, const b
   if (reinterpret_cast<uintptr_t>(X) % 16 || 256 * ldx * 2 > (int64_t)0xffff0000 || (int64_t)N * K * 2 > (int64_t)0xffff0000)
     return hipErrorInvalidValue;
   const int mode = P ? (glu ? OUT_SLAB_GLU : OUT_SLAB) : (act == 1 ? OUT_GLU : act == 2 ? OUT_RELU2 : act == 3 ? OUT_GELU : OUT_BF16);
-  const int64_t total = (int64_t)((M + 32 * mt - 1) / (32 * mt)) * ((N + 32 * nt - 1) / (32 * nt)) * splits;
-  if (total > 0x0fffffff) return hipErrorInvalidValue;
-  const unsigned grid = (unsigned)((total + 7) / 8 * 8);
-  const auto* wt = reinterpret_cast<const bf16x8*>(Wt);
-  auto a = [&](auto kern) { kern<<<grid, 256, 0, st>>>(X, ldx, wt, M, N, K, splits, Y, ldy, P, mode); };
+  const TileArgs A{X, ldx, reinterpret_cast<const bf16x8*>(Wt), M, N, K, splits, Y, ldy, P, mode};
+  const int64_t nts = (int64_t)((N + 32 * nt - 1) / (32 * nt)) * splits;
+  if ((M + 32 * mt - 1) / (32 * mt) * nts > 0x0fffffff) return hipErrorInvalidValue;
+  auto a = [&](auto kern, int low) {
+    const int64_t total = (low ? M / (32 * mt) : (M + 32 * mt - 1) / (32 * mt)) * nts;
+    kern<<<(unsigned)((total + 7) / 8 * 8 + (low ? (nts + 7) / 8 * 8 : 0)), 256, 0, st>>>(A);
+  };
 #define TILE(MT, NT, OCC)                                        \
   if (mt == MT && nt == NT) {                                    \
-    if (M <= 32 * MT) a(tile_gemm_kernel<MT, NT, OCC, true>);    \
-    else a(tile_gemm_kernel<MT, NT, OCC, false>);                \
+    if (M <= 32 * MT) a(tile_gemm_kernel<MT, NT, OCC, true>, 0); \
+    else a(tile_gemm_kernel<MT, NT, OCC, false>, low_rows<MT>(M)); \
     return hipGetLastError();                                    \
   }
   TILE(8, 8, 1)

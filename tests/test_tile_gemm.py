@@ -166,3 +166,41 @@ def test_long_products_by_their_plans():
                 a = ops.linear_glu_long(x, ops.tile_weight(w, glu=True))
                 if a is not None:
                     _close(a, torch.nn.functional.silu(want[:, :N // 2]) * want[:, N // 2:], K)
+
+
+def test_long_plans_take_more_from_the_library():
+    """Past one round of the library's tiles a product with an activation is the tile kernel's, a plain one where the figures say so; all that
+    tile_plan takes stays as it is, so do shapes that the kernel does not take and products within a round."""
+    rng = random.Random(11)
+    for _ in range(400):
+        M, N, K = rng.randint(129, 12000), 32 * rng.randint(1, 900), 64 * rng.randint(2, 230)
+        form = rng.choice(["slabs", "bf16", "glu", "relu2"])
+        had, plan, own = ops.tile_plan(M, N, K, form), ops.long_plan(M, N, K, form), ops.tile_plan(M, N, K, form, library=False)
+        assert ops.long_plan(M, N, K, form, library=False) == own and plan in (had, own) and (had is None or plan == had)
+        past = -(-M // 256) * -(-N // 256) > 256
+        if form in ("glu", "relu2") and M > 768 and past:
+            assert plan == own
+        if had is None and (M <= 768 or not past or form in ("slabs", "bf16") and (M <= 1024 or ops.dense_cut(M, N, K))):
+            assert plan is None
+    assert ops.long_plan(4099, 28672, 4096, "glu") is not None and ops.long_plan(4099, 4096, 4096) is None
+    assert ops.long_plan(5600, 9216, 4096) is not None and ops.long_plan(5600, 9216 + 16, 4096) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mt,nt", sorted(ops.TILES))
+def test_low_last_row_tiles_and_short_loops(mt, nt):
+    """A last row tile on both sides of the low one's height, behind one and several whole ones, columns past the last tile, K from two units
+    (fewer than the ring holds) to more than twice what it holds, even and uneven splits; rows beyond stay as they were."""
+    g = torch.Generator().manual_seed(mt * 100 + nt)
+    bm = 32 * mt
+    for M, N, K, s in ((bm + 1, 64, 128, 1), (bm + 63, 32 * nt + 32, 192, 1), (2 * bm + 64, 96, 256, 2), (2 * bm + 65, 64, 320, 1), (bm + 64, 64, 384, 3),
+                       (9 * bm + 3, 32, 448, 1), (bm + 17, 64 * nt, 640, 2), (bm + 33, 64, 704, 1), (bm + 2, 128, 832, 5)):
+        x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+        w = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
+        want, wt = x.float() @ w.float().t(), ops.tile_weight(w)
+        y = torch.full((M + 70, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.ext().tile_gemm(x, wt, y[:M], None, mt, nt, 1, False)
+        _close(y[:M], want, K)
+        assert (y[M:] == 7).all()
+        if s > 1:
+            assert ((ops.linear_tile(x, wt, (mt, nt, s)).sum(0) - want).abs() <= 1e-4).all()

@@ -163,10 +163,17 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+// 1 / (1 + e^-s): the hardware's exponential and reciprocal (1 ulp each), the exponent's rounding error given back in a product. A quotient behind
+// an exponential of a rounded argument takes a quarter longer (2048 rows of 4096 -> 28672 with silu * up 366 us, so 358) and is further off: g / (1 + e^-g)
+// over -90 .. 90 within 3.7e-6 of 64 bits, rms 6.0e-7, where this one is within 2.5e-7, rms 4.3e-8. Past |s| = 88 as at 88, where the result is 1, or 0 for normal numbers.
+__device__ __forceinline__ float sigmoid_of(float s) {
+  const float x = __builtin_amdgcn_fmed3f(-s, -88.f, 88.f), t = x * 1.44269504f;
+  const float lo = fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269504f, -t)), p = __builtin_amdgcn_exp2f(t);
+  return __builtin_amdgcn_rcpf(1.0f + fmaf(p, 0.69314718f * lo, p));
+}
 // act(g) = g / (1 + e^-s) of the gated feed-forwards: s = g (SiLU), or with gelu that of the tanh form of GELU
 __device__ __forceinline__ float gate_act(float g, bool gelu) {
-  const float s = gelu ? 1.5957691216057308f * (g + 0.044715f * g * g * g) : g;
-  return g / (1.0f + __expf(-s));
+  return g * sigmoid_of(gelu ? 1.5957691216057308f * (g + 0.044715f * g * g * g) : g);
 }
 
 // Counter-based RNG (splitmix64 finaliser): deterministic given (seed, stream, index).

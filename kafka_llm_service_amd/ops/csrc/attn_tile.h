@@ -1,25 +1,28 @@
 // Tile attention v3 for gfx950: the cascade prefix pass (all decode rows of a batch against the shared system
-// prompt's KV, SURVEY.md §2.6 `shared_prefix_decode_attention`) and chunked / causal prefill
+// prompt's KV, `shared_prefix_decode_attention`) and chunked / causal prefill
 // (`prefill_flash_attention`). Same work items, page layouts and outputs as attn_prefill_kernel (attention.hip);
 // selected as tile variant 3 (ops.tile_rows(3) = 256 rows).
 //
-// Structure (one workgroup = 8 waves = two waves per SIMD, 256 query rows of one KV head):
-//   * each wave owns 32 query rows (one 32-row MFMA block); the partner wave's MFMAs run beside this wave's softmax
-//     VALU (a 4-wave / 64-row layout with one wave per SIMD halves the LDS reads but hides no latency: -3.8 % on the
-//     headline, profiles/r04/bench_ab_tile_prologue.jsonl);
-//   * K/V arrive by LDS-DMA (global_load_lds_dwordx4, 1 KiB per wave-instruction) in 64-key tiles (4 pages: 16 KB
-//     K + 16 KB V) into a 3-slot ring: tile j+2 is issued right after the barrier that retires tile j, so two
-//     tiles (64 KB per CU) stay in flight across every barrier. No register round trip, no ds_write pass, and one
-//     counted `s_waitcnt vmcnt(8)` + one `s_barrier` per 64 keys (v2: a vmcnt + ds_write pass + barrier per 32);
+// Structure (one workgroup = 4 or 8 waves, two waves per SIMD, 128 or 256 query rows of one KV head):
+//   * each wave owns 32 query rows (one 32-row MFMA block). A wave is a pipeline over 64-key tiles (4 pages): between the products
+//     of the next tile's keys stand the exponentials of this one, between the products of this one's values the rest of
+//     them and the next one's maxima, each product behind the LDS reads of the eight fragments after it. Waves of a SIMD
+//     are mostly at the same place, so what stood one after the other in a wave (products, then softmax, then products,
+//     reads in front of each) did so on the SIMD. What bounds it now: LDS, 32 KB of fragments a wave and tile (without the
+//     reads 389 us, without the exponentials 480, without the copies 464, of 497: 4096 rows of 32 heads against 8192
+//     keys, 525 before), and the clock that the card holds. (64 rows a wave on one wave per SIMD halve the reads,
+//     but 256 + 256 registers did not hold it without scratch in the loop: 574 us.);
+//   * K/V arrive by LDS-DMA (1 KiB per wave-instruction), 16 KB each per tile, into 2 or 3 slots for each: the keys run a
+//     tile ahead of the values, and both slots that a step has read are filled again in its middle, behind its one counted
+//     `s_waitcnt vmcnt` and one `s_barrier`;
 //   * the DMA destination is lane-linear, so layouts are chosen on the SOURCE side: a K page (plane-major, see
 //     rope_kv.hip) is copied verbatim — its plane-major order already makes the A-fragment reads of a 16-lane
 //     ds_read_b128 group hit 16 distinct bank slots; the V^T page is copied with the 16-B halves of rows 8..15 of
 //     every 16-row group swapped (source lane permutation L ^ ((L >> 4) & 1)), which makes the V^T fragment reads
-//     conflict-free too (cdna_hip_programming.md §5.4 rule 21: linear destination, permuted source, same
-//     permutation on the read);
+//     conflict-free too (linear destination, permuted source, same permutation on the read);
 //   * softmax in the S^T layout (lane = query column: row max / sum are lane-local plus one permlane32 swap) with a
 //     deferred rescale (T13): O and l are rescaled only when some row's max grew by more than 2^THR, so the 64-wide
-//     O rescale almost never runs; the row sums run on the matrix pipe (an MFMA against a ones operand).
+//     O rescale almost never runs.
 #pragma once
 #include "common.h"
 
@@ -55,9 +58,14 @@ struct AltPart {
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 
-template <int AUX = 0>
-__device__ __forceinline__ void dma16(const void* g, char* lds) {
-  __builtin_amdgcn_global_load_lds(g, (lds_void_t*)lds, 16, 0, AUX);
+// N pieces of 1 KiB from g on (uniform; lane_bytes: this lane's 16 bytes of a piece) to lds on. Buffer loads: the immediate moves both sides, and
+// the compiler knows that they leave the waits for LDS reads alone (behind global_load_lds, a FLAT form, it waits for every read there is)
+template <int N, int AUX, int C = 0>
+__device__ __forceinline__ void dma_pieces(const bf16* g, int lane_bytes, char* lds) {
+  if constexpr (C < N) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(buf_rsrc(g), (lds_void_t*)lds, 16, lane_bytes, 0, 1024 * C, AUX);
+    dma_pieces<N, AUX, C + 1>(g, lane_bytes, lds);
+  }
 }
 
 // max without fmaxf's NaN-quieting: IEEE-mode v_max_f32 needs each MFMA result canonicalised first (a v_max x, x
@@ -221,102 +229,88 @@ __device__ __forceinline__ void tile_item(char* smem, const TileItem it, int kvh
 
   const int jf = (lo > base && ntiles > 0) ? 1 : 0;  // (= j0 below)
   auto tile_of = [&](int i) { return i < ntiles - jf ? i + jf : 0; };
-  // ---- DMA of processing index i (tile t(i)) into ring slot i % NSLOT: wave w copies page w of the tile
-  auto issue = [&](int i) {
-    const int j = i;
-    // wave w: page (w * 4) / NW of the tile, its 1-KiB pieces c0 .. c0 + DPT/2 - 1 of K and of V
-    const int pw = (w * 4) / NW, c0 = (w % (NW / 4)) * (DPT / 2);
-    const int pg = s_pages[min(4 * tile_of(i) + pw, npg - 1)];
-    const int64_t poff = ((int64_t)pg * Hkv + kvh) * (tile3::PAGE * D);
-    const bf16* kp = k_cache + poff;
-    const bf16* vp = v_cache + poff;
-    char* kd = smem + (j % NSLOT) * SLOT + pw * 4096;
-    char* vd = kd + KBYTES;
-#pragma unroll
-    for (int cc = 0; cc < DPT / 2; ++cc) {
-      const int c = c0 + cc;
-      const int L = c * 64 + lane;
-      dma16<KVAUX>(kp + L * 8, kd + c * 1024);
-      dma16<KVAUX>(vp + (L ^ ((L >> 4) & 1)) * 8, vd + c * 1024);
-    }
+  // ---- DMA: keys and values have NSLOT slots each; group g is the keys of processing index g (tile t(g)) and the values of g - 1, which are
+  // needed a tile later: wave w copies page w of both
+  const int pw = (w * 4) / NW, c0 = (w % (NW / 4)) * (DPT / 2);   // its page of the tile, its 1-KiB pieces of K and of V
+  const int kl = 16 * lane, vl = 16 * (lane ^ ((lane >> 4) & 1));
+  auto page_of = [&](int i) { return s_pages[min(4 * tile_of(min(i, ntiles - 1)) + pw, npg - 1)]; };
+  auto issue = [&](int g, int kpage, int vpage) {
+    char* const kd = smem + (g % NSLOT) * KBYTES + pw * 4096 + c0 * 1024;
+    char* const vd = smem + (NSLOT + (g + NSLOT - 1) % NSLOT) * KBYTES + pw * 4096 + c0 * 1024;
+    if (g < ntiles) dma_pieces<DPT / 2, KVAUX>(k_cache + ((int64_t)kpage * Hkv + kvh) * (tile3::PAGE * D) + c0 * 512, kl, kd);
+    if (g > 0) dma_pieces<DPT / 2, KVAUX>(v_cache + ((int64_t)vpage * Hkv + kvh) * (tile3::PAGE * D) + c0 * 512, vl, vd);
   };
+  int last_page = 0;                                 // of the keys of the group that was issued last: the next one's values'
+  if (ntiles > 0) {
 #pragma unroll
-  for (int j = 0; j < NSLOT - 1; ++j)
-    if (j < ntiles) issue(j);
+    for (int g = 0; g < NSLOT; ++g) {
+      const int pg = __builtin_amdgcn_readfirstlane(page_of(g));
+      if (g <= ntiles) issue(g, pg, last_page);
+      last_page = pg;
+    }
+  }
   load_q();
 
-  // Running state per row block: O^T accumulators; row sums `ls` as an MFMA accumulator (every register of a lane
-  // holds its column's sum ones . P: 8 MFMAs per tile instead of 64 adds); the running max m (exp2 domain).
+  // Running state per row block: O^T accumulators; this lane's half of the row sums (of the rounded weights, as the products take them: two a
+  // dot product; as products with ones they were an eighth of the matrix cores' work); the running max m (exp2 domain).
   // (Folding -m into the QK^T accumulator init would save the per-score FMA too, but needs Q prescaled by
   // scale * log2(e) in bf16: +0.4 % relative score error, 0.037 abs on a peaked row vs 0.02 tolerance — rejected.)
-  f32x16 o[RB][D / 32], ls[RB];
-  float m[RB];
+  f32x16 o[RB][D / 32];
+  float m[RB], ls[RB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
 #pragma unroll
     for (int t = 0; t < D / 32; ++t)
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[rb][t][i] = 0.f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) ls[rb][i] = 0.f;
+    ls[rb] = 0.f;
     m[rb] = -INFINITY;
   }
-  bf16x8 ones;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) ones[j] = (bf16)1.f;
 
-  // ---- one 64-key tile (processing index j) from ring slot j % NSLOT
-  auto tile_body = [&](auto masked_c, int j, int key0) {
-    constexpr bool MASKED = decltype(masked_c)::value;
-    const char* Ks = smem + (j % NSLOT) * SLOT;  // [page 4][plane 16][key 16][16 B]
-    const char* Vs = Ks + KBYTES;                // [page 4][d 128][2 x 16 B] (halves swapped on rows 8..15 of 16)
-    // S^T = K . Q^T for both 32-key halves (kb) and both row blocks
-    f32x16 s[RB][2];
+  // Processing order: the interior tiles first, then the edge tiles (range ends, causal diagonal): online softmax does not care about key
+  // order. Index i -> tile t(i): tiles j0 .. ntiles-1, then tile 0 when it starts below lo.
+  const int j0 = (lo > base && ntiles > 0) ? 1 : 0;
+  const int wmin_all = min(wmin_b[0], wmin_b[1]);
+  const int clean_end = min(hi_e, wmin_all == 0x7fffffff ? 0x7fffffff : wmin_all + 1);  // keys below: no mask
+  const int j_e = clean_end > base ? min(ntiles, (clean_end - base) / TK) : 0;
+  const int n_int = max(0, j_e - j0);
+
+  // The loop is a pipeline over tiles within the wave: step j multiplies the keys of tile j + 1 between the exponentials of tile j, then
+  // the values of tile j between the rest of them and the maxima of tile j + 1. The eight fragments ahead of a product are on their way from LDS
+  // (fr): 16 of keys (kb = f & 1, depth f >> 1), 16 of values (32 keys' half, 16 keys, 32 columns).
+  const char* const Kl = smem + (r >> 4) * 4096 + (h * 16 + (r & 15)) * 16;                 // [slot][page 4][plane 16][key 16][16 B]
+  const char* const Vl = smem + NSLOT * KBYTES + r * 32 + 16 * (h ^ ((r >> 3) & 1));        // [slot][page 4][d 128][2 x 16 B] (halves swapped)
+  bf16x8 fr[8];
+  f32x16 sa[RB][2], sb[RB][2];
+  auto kfrag = [&](const char* k, int f) { return *reinterpret_cast<const bf16x8*>(k + (f & 1) * 8192 + (f >> 1) * 512); };
+  auto vfrag = [&](const char* v, int f) { return *reinterpret_cast<const bf16x8*>(v + (f >> 2) * 4096 + (f & 3) * 1024); };
+  auto kslot = [&](int i) { return Kl + (i % NSLOT) * KBYTES; };
+  auto vslot = [&](int i) { return Vl + (i % NSLOT) * KBYTES; };
+  auto mask = [&](f32x16(&s)[RB][2], int i) {        // wave-uniform per 32-key half: range edges and the causal diagonal
+    const int key0 = base + TK * tile_of(i);
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      bf16x8 kf[D / 16];
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-      for (int kk = 0; kk < D / 16; ++kk)
-        kf[kk] = *reinterpret_cast<const bf16x8*>(Ks + (2 * kb + (r >> 4)) * 4096 + ((2 * kk + h) * 16 + (r & 15)) * 16);
+      for (int kb = 0; kb < 2; ++kb) {
+        const int k0 = key0 + 32 * kb;
+        if ((k0 < lo) | (k0 + 32 > hi_b[rb]) | (k0 + 31 > wmin_b[rb])) {
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        f32x16 acc = {};
-#pragma unroll
-        for (int kk = 0; kk < D / 16; ++kk) acc = mfma32(kf[kk], qf[rb][kk], acc);
-        s[rb][kb] = acc;
-      }
-    }
-    if constexpr (MASKED) {  // wave-uniform per 32-key half: range edges and the causal diagonal
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-          const int k0 = key0 + 32 * kb;
-          if ((k0 < lo) | (k0 + 32 > hi_b[rb]) | (k0 + 31 > wmin_b[rb])) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              const int key = k0 + (i & 3) + 8 * (i >> 2) + 4 * h;
-              if (!((key >= lo) & (key < hi_b[rb]) & (key <= limit[rb]))) s[rb][kb][i] = -INFINITY;
-            }
+          for (int e = 0; e < 16; ++e) {
+            const int key = k0 + (e & 3) + 8 * (e >> 2) + 4 * h;
+            if (!((key >= lo) & (key < hi_b[rb]) & (key <= limit[rb]))) s[rb][kb][e] = -INFINITY;
           }
         }
-    }
-    // row max; deferred rescale, rare: only when a row's max passed m + THR (or at its first finite scores)
-    float smax[2];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      // two chains of v_maximum3_f32 (m = max3(m, a, b)): 16 VALU ops for the 32 scores of a lane
-      float ma = t3_max(s[rb][0][0], s[rb][1][0]), mb = t3_max(s[rb][0][1], s[rb][1][1]);
-#pragma unroll
-      for (int i = 2; i < 16; i += 2) {
-        ma = t3_max(t3_max(ma, s[rb][0][i]), s[rb][1][i]);
-        mb = t3_max(t3_max(mb, s[rb][0][i + 1]), s[rb][1][i + 1]);
       }
-      smax[rb] = t3_xor32_max(t3_max(ma, mb)) * scale_log2;
-    }
+  };
+  // deferred rescale, rare: only when a row's max passed m + THR (or at its first finite scores)
+  auto rescale = [&](const float (&mx)[RB]) {
+    float smax[RB];
     bool need = false;
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) need = need | !(smax[rb] <= m[rb] + THR);
+    for (int rb = 0; rb < RB; ++rb) {
+      smax[rb] = t3_xor32_max(mx[rb]) * scale_log2;
+      need = need | !(smax[rb] <= m[rb] + THR);
+    }
     if (__any(need)) {
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
@@ -328,80 +322,165 @@ __device__ __forceinline__ void tile_item(char* smem, const TileItem it, int kvh
         m[rb] = mn;
       }
     }
-    // P = exp2(S scale - m) (<= 2^THR), O^T += V^T . P, row sums += ones . P (both on the matrix pipe). V^T fragments (A
-    // operand: lane (r, h) = row d = 32 t + r, keys 8h .. 8h+7 of a page) are read per 32-key half (32 VGPRs live).
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      bf16x8 vf[2][D / 32];
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-        for (int t = 0; t < D / 32; ++t) {
-          const int d = 32 * t + r;
-          vf[s2][t] = *reinterpret_cast<const bf16x8*>(Vs + (2 * kb + s2) * 4096 + d * 32 + 16 * (h ^ ((d >> 3) & 1)));
-        }
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        const float mu = (m[rb] == -INFINITY) ? 0.f : m[rb];
-        bf16x8 pf[2];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const float x = fmaf(s[rb][kb][i], scale_log2, -mu);
-          pf[i >> 3][i & 7] = (bf16)fast_exp2(x);
-        }
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-#pragma unroll
-          for (int t = 0; t < D / 32; ++t) o[rb][t] = mfma32(vf[s2][t], pf[s2], o[rb][t]);
-          ls[rb] = mfma32(ones, pf[s2], ls[rb]);
-        }
-      }
+  };
+  int next_page = 0;                                 // page of the keys of the group that is issued next, on its way from LDS
+  // every wave has read the keys of tile j + 1 and the values of tile j, and group j + 2 has landed: their slots are filled again
+  auto meet = [&](int j) {
+    __builtin_amdgcn_s_waitcnt(0xC07F);              // lgkmcnt(0): this wave's reads of those slots
+    t3_wait_tiles<DPT>(min(NSLOT - 2, max(0, ntiles - 1 - (j + 2))));
+    t3_barrier();
+    const int g = j + 1 + NSLOT;
+    if (g <= ntiles) {
+      const int pg = __builtin_amdgcn_readfirstlane(next_page);
+      issue(g, pg, last_page);
+      last_page = pg;
+      next_page = page_of(g + 1);
     }
   };
-
-  // Processing order: the interior tiles first, then the edge tiles (range ends, causal diagonal), so each kind runs
-  // in a loop of its own with its own body — interior tiles without any masking code (one straight-line block up to
-  // the rare rescale branch and one after it: the scheduler can put the max of one row block beside the other's QK^T
-  // MFMAs and the exp of one beside the other's PV MFMAs). Online softmax does not care about key order; the DMA
-  // ring streams in processing order. Index i -> tile t(i): tiles j0 .. ntiles-1, then tile 0 when it starts below lo.
-  const int j0 = (lo > base && ntiles > 0) ? 1 : 0;
-  const int wmin_all = min(wmin_b[0], wmin_b[1]);
-  const int clean_end = min(hi_e, wmin_all == 0x7fffffff ? 0x7fffffff : wmin_all + 1);  // keys below: no mask
-  const int j_e = clean_end > base ? min(ntiles, (clean_end - base) / TK) : 0;
-  const int n_int = max(0, j_e - j0);
-  auto step = [&](int i) {
-    // tile i landed (this wave's pieces; the NSLOT - 2 younger tiles stay in flight), then every wave's: the
-    // barrier also retires every read of slot (i + NSLOT - 1) % NSLOT (index i - 1's)
-    t3_wait_tiles<DPT>(min(NSLOT - 2, ntiles - 1 - i));
-    t3_barrier();
-    if (i + NSLOT - 1 < ntiles) issue(i + NSLOT - 1);
+  // step j: s the scores of tile j, sn those of the next one (unless LAST)
+  auto tile_step = [&](auto last_c, int j, f32x16(&s)[RB][2], f32x16(&sn)[RB][2]) {
+    constexpr bool LAST = decltype(last_c)::value;
+    const f32x16 zero = {};
+    const char *kc = kslot(j + 1), *vc = vslot(j);
+    float mu[RB];
+    bf16x8 pf[RB][2], pg[RB][2];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) mu[rb] = (m[rb] == -INFINITY) ? 0.f : m[rb];
+    auto prob = [&](int rb, float x) { return (bf16)fast_exp2(fmaf(x, scale_log2, -mu[rb])); };
+    auto add = [&](int rb, const bf16x8& p) {        // the row sums' share of eight weights
+      const bf16x2 one = {(bf16)1.f, (bf16)1.f};
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) {
+        const bf16x2 two = {p[i], p[i + 1]};
+        ls[rb] = __builtin_amdgcn_fdot2_f32_bf16(two, one, ls[rb], false);
+      }
+    };
+    if constexpr (LAST) {
+#pragma unroll
+      for (int p = 0; p < 8; ++p) fr[p] = vfrag(vc, p);
+#pragma unroll
+      for (int p = 0; p < 16; ++p)
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) pf[rb][p >> 3][p & 7] = prob(rb, s[rb][0][p]);
+    } else {
+#pragma unroll
+      for (int p = 0; p < 16; ++p) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+          sn[rb][p & 1] = mfma32(fr[p & 7], qf[rb][p >> 1], p < 2 ? zero : sn[rb][p & 1]);
+          pf[rb][p >> 3][p & 7] = prob(rb, s[rb][0][p]);
+        }
+        fr[p & 7] = p < 8 ? kfrag(kc, p + 8) : vfrag(vc, p - 8);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        o[rb][p & 3] = mfma32(fr[p], pf[rb][p >> 2], o[rb][p & 3]);
+        pg[rb][p >> 2][2 * (p & 3)] = prob(rb, s[rb][1][2 * p]);
+        pg[rb][p >> 2][2 * (p & 3) + 1] = prob(rb, s[rb][1][2 * p + 1]);
+        if ((p & 3) == 0) add(rb, pf[rb][p >> 2]);
+      }
+      fr[p] = vfrag(vc, p + 8);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    float ma[RB], mb[RB];
+    const char* kn = kslot(j + 2);
+    if constexpr (!LAST) {
+      // (the compiler would move the exponentials to the products that take them)
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) asm volatile("" : "+v"(pg[rb][0]), "+v"(pg[rb][1]));
+      meet(j);
+      if (j + 1 >= n_int) mask(sn, j + 1);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        ma[rb] = t3_max(sn[rb][0][0], sn[rb][1][0]);
+        mb[rb] = t3_max(sn[rb][0][1], sn[rb][1][1]);
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        o[rb][p & 3] = mfma32(fr[p], pg[rb][p >> 2], o[rb][p & 3]);
+        if (!LAST && p > 0) {
+          ma[rb] = t3_max(t3_max(ma[rb], sn[rb][0][2 * p]), sn[rb][1][2 * p]);
+          mb[rb] = t3_max(t3_max(mb[rb], sn[rb][0][2 * p + 1]), sn[rb][1][2 * p + 1]);
+        }
+        if ((p & 3) == 0) add(rb, pg[rb][p >> 2]);
+      }
+      if constexpr (!LAST) fr[p] = kfrag(kn, p);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (!LAST) {
+      float mx[RB];
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) mx[rb] = t3_max(ma[rb], mb[rb]);
+      rescale(mx);
+    }
   };
-  for (int i = 0; i < n_int; ++i) {
-    step(i);
-    if constexpr (ABL == 8)
-      if (i == 0) ph[2] = t3_rt();
-    tile_body(std::false_type{}, i, base + TK * tile_of(i));
+  if (ntiles > 0) {
+    t3_wait_vmcnt<0>();                              // (the rows came last)
+    t3_barrier();
+    if constexpr (ABL == 8) ph[2] = t3_rt();
+    next_page = page_of(NSLOT);
+#pragma unroll
+    for (int p = 0; p < 8; ++p) fr[p] = kfrag(Kl, p);
+#pragma unroll
+    for (int p = 0; p < 16; ++p) {
+      const f32x16 zero = {};
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) sa[rb][p & 1] = mfma32(fr[p & 7], qf[rb][p >> 1], p < 2 ? zero : sa[rb][p & 1]);
+      if (p < 8) fr[p] = kfrag(Kl, p + 8);
+    }
+    meet(-1);
+#pragma unroll
+    for (int p = 0; p < 8; ++p) fr[p] = kfrag(kslot(1), p);
+    if (n_int < 1) mask(sa, 0);
+    float mx[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      mx[rb] = t3_max(sa[rb][0][0], sa[rb][1][0]);
+#pragma unroll
+      for (int i = 1; i < 16; ++i) mx[rb] = t3_max(t3_max(mx[rb], sa[rb][0][i]), sa[rb][1][i]);
+    }
+    rescale(mx);
+    int j = 0;
+    for (; j + 2 < ntiles; j += 2) {
+      tile_step(std::false_type{}, j, sa, sb);
+      tile_step(std::false_type{}, j + 1, sb, sa);
+    }
+    if (j + 1 < ntiles) {
+      tile_step(std::false_type{}, j, sa, sb);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        sa[rb][0] = sb[rb][0];
+        sa[rb][1] = sb[rb][1];
+      }
+      ++j;
+    }
+    tile_step(std::true_type{}, j, sa, sb);
   }
-  for (int i = n_int; i < ntiles; ++i) {
-    step(i);
-    tile_body(std::true_type{}, i, base + TK * tile_of(i));
-  }
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) ls[rb] = t3_xor32_sum(ls[rb]);
 
   if constexpr (ABL == 8) ph[3] = t3_rt();
-  // ---- epilogue: through a per-wave LDS transpose (slot ntiles % NSLOT is idle: its last tile was read before the
-  // barrier every wave passed NSLOT - 1 tiles ago), so every store instruction writes whole 128-B lines
+  // ---- epilogue: through a per-wave LDS transpose (the keys' slots are idle: every wave has read the last ones before it passed the last
+  // meeting, and nothing more is on its way there), so every store instruction writes whole 128-B lines
   const bool part = it.split >= 0;
   const bool alt = part && it.alt != 0 && ap.part != nullptr;  // (workgroup-uniform)
   float* const opart = alt ? ap.part : out_part;
   float* const lpart = alt ? ap.lse : lse_part;
   const int Sx = alt ? ap.S : S_total, toff = alt ? ap.tok_off : 0;
   const bool pbf = part_bf16 && !alt;
-  char* slab = smem + (ntiles % NSLOT) * SLOT + w * (4096 * RB);
+  char* slab = smem + w * (4096 * RB);
   const int cc = lane & 7;
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     if (!__any(valid[rb])) continue;  // wave-uniform
-    const float ll = fits ? ls[rb][0] : __builtin_nanf("");
+    const float ll = fits ? ls[rb] : __builtin_nanf("");
     const float inv = ll > 0.f ? 1.f / ll : (fits ? 0.f : ll);
     if (ABL != 8 && part && valid[rb] && h == 0) {
       float* lp = lpart + ((int64_t)(token[rb] - toff) * Hq + head[rb]) * Sx + it.split;

@@ -5,20 +5,28 @@
 
 namespace kafka {
 
-// three ring slots (4: 30.9 vs 29.9 us per cascade launch, profiles/r05/cascade/cascade_nslot_*.jsonl)
-template <int ABL = 0, int KVAUX = 0, int PST = 0>
-__global__ __launch_bounds__(512, 2) void attn_tile_kernel(const TileItem* __restrict__ items,
-                                                           const bf16* __restrict__ q, int64_t q_stride,
-                                                           const bf16* __restrict__ k_cache,
-                                                           const bf16* __restrict__ v_cache, int Hkv, int G,
-                                                           const int* __restrict__ block_tables, int bt_stride,
-                                                           const int* __restrict__ q_limit, bf16* __restrict__ out,
-                                                           int64_t out_stride, float* __restrict__ out_part,
-                                                           float* __restrict__ lse_part, int S_total,
-                                                           float scale_log2, int part_bf16, AltPart ap) {
-  __shared__ __attribute__((aligned(16))) char smem[tile3::lds_bytes<3>()];
-  tile_item<ABL, KVAUX, PST, 8, 3>(smem, items[blockIdx.y], blockIdx.x, q, q_stride, k_cache, v_cache, Hkv, G, block_tables,
-                                   bt_stride, q_limit, out, out_stride, out_part, lse_part, S_total, scale_log2, part_bf16, ap);
+// An item (256 query rows) is 8 / NW workgroups of one key/value head. Prompts: two of four waves and two ring slots each, two workgroups a CU, whose
+// waves do not wait for each other and whose halves of a causal item end where their own rows do; 4096 rows against 8192 keys, us, 8 waves 497, two
+// of 4 482 (528 before the loop was a pipeline; 8 waves 514). A cascade's prefix pass (few row tiles, keys from memory) reads the keys once an item:
+// 8 waves, three slots (4: 30.9 vs 29.9 us per cascade launch, profiles/r05/cascade/cascade_nslot_*.jsonl)
+template <int ABL, int KVAUX, int PST, int NW, int NSLOT>
+__global__ __launch_bounds__(64 * NW, 2) void attn_tile_kernel(const TileItem* __restrict__ items,
+                                                               const bf16* __restrict__ q, int64_t q_stride,
+                                                               const bf16* __restrict__ k_cache,
+                                                               const bf16* __restrict__ v_cache, int Hkv, int G,
+                                                               const int* __restrict__ block_tables, int bt_stride,
+                                                               const int* __restrict__ q_limit, bf16* __restrict__ out,
+                                                               int64_t out_stride, float* __restrict__ out_part,
+                                                               float* __restrict__ lse_part, int S_total,
+                                                               float scale_log2, int part_bf16, AltPart ap) {
+  __shared__ __attribute__((aligned(16))) char smem[tile3::lds_bytes<NSLOT>()];
+  TileItem it = items[blockIdx.y];
+  const int share = blockIdx.x / Hkv, tok = 32 * NW / G;
+  it.q_start += share * tok;
+  it.q_count = min(it.q_count - share * tok, NW == 8 ? it.q_count : tok);
+  if (it.q_count <= 0) return;
+  tile_item<ABL, KVAUX, PST, NW, NSLOT>(smem, it, blockIdx.x - share * Hkv, q, q_stride, k_cache, v_cache, Hkv, G, block_tables,
+                                        bt_stride, q_limit, out, out_stride, out_part, lse_part, S_total, scale_log2, part_bf16, ap);
 }
 
 // Host launcher (bf16 KV only; the fp8 cache keeps tile variant 0). Items: int32 [n, 8] as attn_prefill_kernel.
@@ -40,11 +48,15 @@ extern "C" hipError_t kafka_launch_attn_tile(const void* items, int n_items, con
   // (profiles/r05/cascade/bench_ab_kv_nt.jsonl). Prefill launches keep the default policy: their query tiles re-read
   // the same keys.
   // Its bf16 partials are stored sc1 (16-B stores that leave this XCD's L2: +0.2..0.6 %, bench_ab_part_sc1.jsonl).
-  auto kern = stamps ? attn_tile_kernel<8> : part_bf16 ? attn_tile_kernel<0, 2, 1> : attn_tile_kernel<0>;
-  kern<<<dim3(Hkv, n_items), 512, 0, st>>>(reinterpret_cast<const TileItem*>(items), q, q_stride,
-                                           static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), Hkv,
-                                           G, block_tables, bt_stride, q_limit, out, out_stride, out_part, lse_part,
-                                           S_total, scale_log2, part_bf16, AltPart{alt_part, alt_lse, alt_S, alt_tok_off});
+  auto go = [&](auto kern, int shares) {
+    kern<<<dim3(Hkv * shares, n_items), 512 / shares, 0, st>>>(
+        reinterpret_cast<const TileItem*>(items), q, q_stride, static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), Hkv, G,
+        block_tables, bt_stride, q_limit, out, out_stride, out_part, lse_part, S_total, scale_log2, part_bf16,
+        AltPart{alt_part, alt_lse, alt_S, alt_tok_off});
+  };
+  if (stamps) go(attn_tile_kernel<8, 0, 0, 8, 3>, 1);
+  else if (part_bf16) go(attn_tile_kernel<0, 2, 1, 8, 3>, 1);
+  else go(attn_tile_kernel<0, 0, 0, 4, 2>, 2);
   return hipGetLastError();
 }
 

@@ -237,19 +237,23 @@ __device__ __forceinline__ void tile_item(char* smem, const TileItem it, int kvh
   auto issue = [&](int g, int kpage, int vpage) {
     char* const kd = smem + (g % NSLOT) * KBYTES + pw * 4096 + c0 * 1024;
     char* const vd = smem + (NSLOT + (g + NSLOT - 1) % NSLOT) * KBYTES + pw * 4096 + c0 * 1024;
-    if (g < ntiles) dma_pieces<DPT / 2, KVAUX>(k_cache + ((int64_t)kpage * Hkv + kvh) * (tile3::PAGE * D) + c0 * 512, kl, kd);
+    if (g < ntiles || g == 1) dma_pieces<DPT / 2, KVAUX>(k_cache + ((int64_t)kpage * Hkv + kvh) * (tile3::PAGE * D) + c0 * 512, kl, kd);
     if (g > 0) dma_pieces<DPT / 2, KVAUX>(v_cache + ((int64_t)vpage * Hkv + kvh) * (tile3::PAGE * D) + c0 * 512, vl, vd);
   };
   int last_page = 0;                                 // of the keys of the group that was issued last: the next one's values'
   if (ntiles > 0) {
+    last_page = __builtin_amdgcn_readfirstlane(page_of(0));
+    issue(0, last_page, 0);
+  }
+  load_q();                                          // (the first products take the rows and the first keys, no more)
+  if (ntiles > 0) {
 #pragma unroll
-    for (int g = 0; g < NSLOT; ++g) {
+    for (int g = 1; g < NSLOT; ++g) {
       const int pg = __builtin_amdgcn_readfirstlane(page_of(g));
       if (g <= ntiles) issue(g, pg, last_page);
       last_page = pg;
     }
   }
-  load_q();
 
   // Running state per row block: O^T accumulators; this lane's half of the row sums (of the rounded weights, as the products take them: two a
   // dot product; as products with ones they were an eighth of the matrix cores' work); the running max m (exp2 domain).
@@ -422,7 +426,7 @@ __device__ __forceinline__ void tile_item(char* smem, const TileItem it, int kvh
     }
   };
   if (ntiles > 0) {
-    t3_wait_vmcnt<0>();                              // (the rows came last)
+    t3_wait_vmcnt<DPT>();                            // (group 1 is whole whatever there is: its keys are the last ones' again where they are past them)
     t3_barrier();
     if constexpr (ABL == 8) ph[2] = t3_rt();
     next_page = page_of(NSLOT);

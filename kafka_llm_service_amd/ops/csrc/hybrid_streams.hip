@@ -578,17 +578,21 @@ __global__ __launch_bounds__(256, NKS * 4 + NVT * 16 <= 96 ? 2 : 1) void window_
     }
 }
 
-// ---- the same for long portions, 128 channels: eight items share their keys in LDS -----------------------------------------
-// A workgroup takes eight neighbouring items of one key/value head, a wave each (as above: S^T = K Q^T, the weights stay in
-// registers, O^T += V^T P^T), and walks the union of their keys 64 at a time: K and V^T pages go to a ring of three slots in LDS
-// without a register on the way, two tiles ahead. Chunk c (16 bytes) of key row k lies at c ^ k of its page, the halves of
-// channels 8 .. 15 of every 16 in a V^T page are swapped: every operand read meets all banks once. Items of different segments
-// go one segment after the other, the rest of the workgroup helps loading. The accumulators are rescaled only when a row's
-// maximum has grown by more than 2^WT_THR.
-// What bounds it: products and softmax of two waves a SIMD; above, each wave's operands came through the caches. 8192 fresh rows
-// x 32 heads over 8 1287 -> 649 us (0.85 PFLOP/s), 3 x 1100 rows, 32 over 2, 108 -> 65, 4096 rows with a window of 1024 175 -> 97.
-constexpr int WT_WAVES = 8, WT_KEYS = 64, WT_SLOTS = 3, WT_RUN = 512;   // WT_RUN: tiles whose page ids lie in LDS at a time
-constexpr int WT_KB = WT_KEYS * 256, WT_SLOT = 2 * WT_KB;
+// ---- the same for long portions, 128 channels: four items share their keys in LDS ------------------------------------------
+// A workgroup takes four neighbouring items of one key/value head, a wave each (as above: S^T = K Q^T, the weights stay in
+// registers, O^T += V^T P^T), and walks the union of their keys 64 at a time; two workgroups share a CU. Chunk c (16 bytes) of key row k lies
+// at c ^ k of its page, the halves of channels 8 .. 15 of every 16 in a V^T page are swapped: every operand read meets all banks once. Items
+// of different segments go one segment after the other, the rest of the workgroup helps loading. The accumulators are rescaled only
+// when a row's maximum has grown by more than 2^WT_THR.
+// A wave is a pipeline over the tiles, as in attn_tile.h: the next tile's products with the keys stand between this one's exponentials, its
+// products with the values between the rest of them and the next maxima, and eight fragments are on their way from LDS at any time. K and V^T
+// pages have two slots each, without a register on the way (buffer loads); the keys run a tile ahead, and both slots that a step has read are
+// filled again in its middle, where the waves meet.
+// What bounds it: LDS (32 KB of fragments a wave and tile) and the clock. us in a step, products and softmax of a tile one after the other and
+// eight waves a workgroup / now: 8192 fresh rows x 32 heads over 8 594 / 518 (1.06 PFLOP/s), 1100, 843 and 862 rows, 32 over 2, 48.4 / 43.2. (Before
+// that a wave's operands came through the caches, twice as long.)
+constexpr int WT_WAVES = 4, WT_KEYS = 64, WT_SLOTS = 2, WT_RUN = 512;   // WT_RUN: tiles whose page ids lie in LDS at a time
+constexpr int WT_KB = WT_KEYS * 256, WT_PIECES = 16 / WT_WAVES;         // bytes of a tile's keys; 1-KiB pieces of them that a wave copies
 constexpr float WT_THR = 8.f;
 // Items (those that it works on, not the single tokens between them) x key/value heads from which it runs: a wave each on 256 CUs, fewer leave whole CUs idle that the form above still uses.
 // us there / here: 1000 waves (1000 rows) 33 / 40, 1024 (2048 rows, 4 heads) 62 / 66, 1200 47 / 45, 1500 63 / 60, 2048 with a
@@ -596,22 +600,26 @@ constexpr float WT_THR = 8.f;
 constexpr int WT_MIN_WAVES = 1280;
 
 typedef __attribute__((address_space(3))) void wt_lds_t;
-template <int OFF>
-__device__ __forceinline__ void wt_dma16(const void* g, void* lds) {
-  __builtin_amdgcn_global_load_lds(g, (wt_lds_t*)lds, 16, OFF, 0);
+// pieces C .. of a page from g on (uniform), this lane's bytes of each less 1 KiB a piece, which the immediate adds on both sides
+template <int C = 0>
+__device__ __forceinline__ void wt_dma(const char* g, const int (&at)[WT_PIECES], unsigned char* lds) {
+  if constexpr (C < WT_PIECES) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(buf_rsrc(g), (wt_lds_t*)lds, 16, at[C], 0, 1024 * C, 0);
+    wt_dma<C + 1>(g, at, lds);
+  }
 }
 __device__ __forceinline__ float wt_max(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 
-__global__ __launch_bounds__(512, 2) void window_attn_tile_kernel(
+__global__ __launch_bounds__(64 * WT_WAVES, 2) void window_attn_tile_kernel(
     const bf16* __restrict__ q, int64_t qs, const bf16* __restrict__ kc, const bf16* __restrict__ vt,
     const int* __restrict__ bt, int bt_stride, const int* __restrict__ items, int n_items,
     const int64_t* __restrict__ positions, int H, int G, int Ck, int kstep, float scale_log2e, int window,
     const float* __restrict__ sink, const bf16* __restrict__ gate, int64_t gs, bf16* __restrict__ out, int64_t os,
     float out_scale, int min_tok, bool vec4) {
   constexpr int D = 128, Dv = 128, NKS = 8, NVT = 4;
-  __shared__ __attribute__((aligned(16))) unsigned char smem[WT_SLOTS * WT_SLOT + 4 * WT_RUN * 4 + WT_WAVES * 16];
-  int* pg_s = reinterpret_cast<int*>(smem + WT_SLOTS * WT_SLOT);   // [4 WT_RUN]
-  int4* who = reinterpret_cast<int4*>(pg_s + 4 * WT_RUN);          // [waves] (segment or -1, first tile, end tile, last page)
+  __shared__ __attribute__((aligned(16))) unsigned char smem[2 * WT_SLOTS * WT_KB + 4 * WT_RUN * 4 + WT_WAVES * 16];
+  int* pg_s = reinterpret_cast<int*>(smem + 2 * WT_SLOTS * WT_KB);   // [4 WT_RUN]
+  int4* who = reinterpret_cast<int4*>(pg_s + 4 * WT_RUN);            // [waves] (segment or -1, first tile, end tile, last page)
   const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int item = n_items - 1 - ((int)blockIdx.y * WT_WAVES + w);
   int t0 = 0, ntok = 0, sg = -1;
@@ -638,36 +646,39 @@ __global__ __launch_bounds__(512, 2) void window_attn_tile_kernel(
   const int jb = window > 0 ? max(0, minpos - window + 1) / WT_KEYS : 0, je = maxpos / WT_KEYS + 1;   // tiles of this wave
   if (lane == 0) who[w] = int4{sg, jb, je, maxpos >> 4};
   const int krow = (lr & 19) | ((lr & 4) << 1) | ((lr & 8) >> 1), kk = krow & 15;   // bits 2 and 3 swapped
-  int kat[NKS], vat[NVT];   // operands' places in a slot
+  int kat[NKS];             // operands' places in a slot
 #pragma unroll
   for (int ks = 0; ks < NKS; ++ks) kat[ks] = (krow >> 4) * 4096 + kk * 256 + 16 * ((2 * ks + lh) ^ kk);
+  const int vat = WT_SLOTS * WT_KB + lr * 32 + 16 * (lh ^ ((lr >> 3) & 1));
+  // wave w copies WT_PIECES 1-KiB pieces of K and of V^T of page pw of a tile
+  constexpr int PW = 4 / WT_PIECES;                 // waves of a page
+  const int pw = w / PW, c0 = (w % PW) * WT_PIECES;
+  int ksrc[WT_PIECES], vsrc[WT_PIECES];
 #pragma unroll
-  for (int v = 0; v < NVT; ++v) vat[v] = WT_KB + (32 * v + lr) * 32 + 16 * (lh ^ ((lr >> 3) & 1));
-  // wave w copies half w & 1 of page w >> 1 of a tile: two 1-KiB pieces of K and of V^T
-  const int pw = w >> 1, c0 = (w & 1) * 2048;
-  const int vsrc = c0 + (lane ^ ((lane >> 4) & 1)) * 16;
-  int ksrc[2];
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const int k = 8 * (w & 1) + 4 * c + (lane >> 4);
-    ksrc[c] = k * Ck * 2 + 16 * ((lane & 15) ^ k);
+  for (int c = 0; c < WT_PIECES; ++c) {
+    const int k = 4 * (c0 + c) + (lane >> 4);
+    ksrc[c] = k * Ck * 2 + 16 * ((lane & 15) ^ k) - 1024 * c;   // (Ck >= 128: not below zero)
+    vsrc[c] = c0 * 1024 + (lane ^ ((lane >> 4) & 1)) * 16;
   }
-  auto issue = [&](int j) {   // tile j of the run
-    const int64_t pg = __builtin_amdgcn_readfirstlane(pg_s[4 * j + pw]);
-    const char* kp = reinterpret_cast<const char*>(kc + pg * PAGE * Ck + (int64_t)g * kstep);
-    const char* vp = reinterpret_cast<const char*>(vt + (pg * Cv + (int64_t)g * Dv) * PAGE);
-    unsigned char* dst = smem + (j % WT_SLOTS) * WT_SLOT + pw * 4096 + c0;
-    wt_dma16<0>(kp + ksrc[0], dst);
-    wt_dma16<0>(kp + ksrc[1], dst + 1024);
-    wt_dma16<0>(vp + vsrc, dst + WT_KB);
-    wt_dma16<1024>(vp + vsrc, dst + WT_KB);
+  // group i of the run: the keys of tile i and the values of tile i - 1
+  auto page_of = [&](int i, int n) { return pg_s[4 * min(i, n - 1) + pw]; };
+  auto issue = [&](int i, int n, int64_t kpage, int64_t vpage) {
+    unsigned char* const dst = smem + pw * 4096 + c0 * 1024;
+    if (i < n)
+      wt_dma(reinterpret_cast<const char*>(kc + kpage * PAGE * Ck + (int64_t)g * kstep), ksrc, dst + (i % WT_SLOTS) * WT_KB);
+    if (i > 0)
+      wt_dma(reinterpret_cast<const char*>(vt + (vpage * Cv + (int64_t)g * Dv) * PAGE), vsrc,
+             dst + (WT_SLOTS + (i + WT_SLOTS - 1) % WT_SLOTS) * WT_KB);
   };
   float m = -INFINITY, l = 0.f;
-  f32x16 O[NVT];
+  f32x16 O[NVT], sa[2], sb[2];
 #pragma unroll
   for (int v = 0; v < NVT; ++v)
 #pragma unroll
     for (int i = 0; i < 16; ++i) O[v][i] = 0.f;
+  bf16x8 fr[8];             // fragments on their way: 16 of keys (32-key half f & 1, depth f >> 1), 16 of values (page f >> 2, channels f & 3)
+  auto kfrag = [&](const unsigned char* k, int f) { return *reinterpret_cast<const bf16x8*>(k + kat[f >> 1] + (f & 1) * 8192); };
+  auto vfrag = [&](const unsigned char* v, int f) { return *reinterpret_cast<const bf16x8*>(v + vat + (f >> 2) * 4096 + (f & 3) * 1024); };
   __builtin_amdgcn_s_waitcnt(0x0F70);   // (vmcnt(0): left open, the queries' loads are waited for, with the tiles', in every step)
   lds_barrier();
   for (int a = 0; a < WT_WAVES;) {   // (uniform) waves a .. b - 1 walk one segment
@@ -688,83 +699,139 @@ __global__ __launch_bounds__(512, 2) void window_attn_tile_kernel(
     const int* btr = bt + (int64_t)seg * bt_stride;
     for (int run = lo; run < hi; run += WT_RUN) {
       const int n = min(hi - run, WT_RUN);
-      for (int i = threadIdx.x; i < 4 * n; i += 512) pg_s[i] = btr[min(4 * run + i, lastpg)];   // (past the last page: it again)
+      for (int i = threadIdx.x; i < 4 * n; i += 64 * WT_WAVES) pg_s[i] = btr[min(4 * run + i, lastpg)];   // (past the last page: it again)
       lds_barrier();
-      issue(0);
-      if (n > 1) issue(1);
-      for (int j = 0; j < n; ++j) {
-        // this wave's pieces of the tile have landed (the next tile's stay on their way), then everyone's; everyone has left
-        // the tile before, whose slot the one after next takes
-        if (j + 1 < n)
-          asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-        else
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      int last_page = 0, next_page = 0;              // of the keys of the group issued last; of the next one's, on its way
+#pragma unroll
+      for (int i = 0; i < WT_SLOTS; ++i) {
+        const int pg = __builtin_amdgcn_readfirstlane(page_of(i, n));
+        if (i <= n) issue(i, n, pg, last_page);
+        last_page = pg;
+      }
+      next_page = page_of(WT_SLOTS, n);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_barrier();
+      // this wave's reads of the keys of tile j + 1 and the values of tile j are done, group j + 2 has landed; then everyone's: the slots are
+      // filled again
+      auto meet = [&](int j) {
+        static_assert(WT_SLOTS == 2, "the wait");
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         lds_barrier();
-        if (j + 2 < n) issue(j + 2);
-        const int key0 = (run + j) * WT_KEYS;
-        if (!on || run + j < jb || run + j >= je) continue;
-        const unsigned char* sl = smem + (j % WT_SLOTS) * WT_SLOT;
-        f32x16 S[2];
-#pragma unroll
-        for (int sb = 0; sb < 2; ++sb) {
-          bf16x8 kf[NKS];
-#pragma unroll
-          for (int ks = 0; ks < NKS; ++ks) kf[ks] = *reinterpret_cast<const bf16x8*>(sl + kat[ks] + sb * 8192);
-          f32x16 acc = {};
-#pragma unroll
-          for (int ks = 0; ks < NKS; ++ks) acc = mfma32(kf[ks], qf[ks], acc);
-          S[sb] = acc;
+        const int i = j + 1 + WT_SLOTS;
+        if (i <= n) {
+          const int pg = __builtin_amdgcn_readfirstlane(next_page);
+          issue(i, n, pg, last_page);
+          last_page = pg;
+          next_page = page_of(i + 1, n);
         }
-        // (uniform) a tile that every row sees whole needs no mask
-        if (key0 + WT_KEYS - 1 > minpos || (window > 0 && key0 <= maxpos - window)) {
+      };
+      // step j: CUR: tile j, whose scores S holds, is this wave's; NXT: tile j + 1 is, its scores go to T
+      auto step = [&](auto cur_c, auto nxt_c, int j, f32x16(&S)[2], f32x16(&T)[2]) {
+        constexpr bool CUR = decltype(cur_c)::value, NXT = decltype(nxt_c)::value;
+        const unsigned char *kc1 = smem + ((j + 1) % WT_SLOTS) * WT_KB, *kc2 = smem + ((j + 2) % WT_SLOTS) * WT_KB,
+                            *vc = smem + (max(j, 0) % WT_SLOTS) * WT_KB;
+        const float base = m == -INFINITY ? 0.f : m;   // nothing visible yet: every weight is 2^-inf = 0
+        bf16x8 pf[2], pg[2];
+        auto prob = [&](float x) {
+          const float e = fast_exp2(fmaf(x, scale_log2e, -base));
+          l += e;
+          return (bf16)e;
+        };
+        if constexpr (!CUR && NXT) {
 #pragma unroll
-          for (int sb = 0; sb < 2; ++sb)
+          for (int f = 0; f < 8; ++f) fr[f] = kfrag(kc1, f);
+        }
+        if constexpr (CUR && !NXT) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              const int key = key0 + 32 * sb + 16 * (i >> 3) + 8 * lh + (i & 7);
-              if (key > p || (window > 0 && key <= p - window)) S[sb][i] = -INFINITY;
+          for (int f = 0; f < 8; ++f) fr[f] = vfrag(vc, f);
+#pragma unroll
+          for (int i = 0; i < 16; ++i) pf[i >> 3][i & 7] = prob(S[0][i]);
+        }
+        if constexpr (NXT) {
+#pragma unroll
+          for (int f = 0; f < 16; ++f) {
+            const f32x16 zero = {};
+            T[f & 1] = mfma32(fr[f & 7], qf[f >> 1], f < 2 ? zero : T[f & 1]);
+            if (f < 8) fr[f] = kfrag(kc1, f + 8);
+            else if (CUR) fr[f - 8] = vfrag(vc, f - 8);
+            if (CUR) pf[f >> 3][f & 7] = prob(S[0][f]);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        if constexpr (CUR) {
+#pragma unroll
+          for (int f = 0; f < 8; ++f) {
+            O[f & 3] = mfma32(fr[f], pf[f >> 2], O[f & 3]);
+            fr[f] = vfrag(vc, f + 8);
+            pg[f >> 2][2 * (f & 3)] = prob(S[1][2 * f]);
+            pg[f >> 2][2 * (f & 3) + 1] = prob(S[1][2 * f + 1]);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          // (the compiler would move the exponentials to the products that take them)
+          asm volatile("" : "+v"(pg[0]), "+v"(pg[1]));
+        }
+        meet(j);
+        float ma = 0.f, mb = 0.f;
+        if constexpr (NXT) {
+          const int key0 = (run + j + 1) * WT_KEYS;
+          // (uniform) a tile that every row sees whole needs no mask
+          if (key0 + WT_KEYS - 1 > minpos || (window > 0 && key0 <= maxpos - window)) {
+#pragma unroll
+            for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+              for (int i = 0; i < 16; ++i) {
+                const int key = key0 + 32 * s2 + 16 * (i >> 3) + 8 * lh + (i & 7);
+                if (key > p || (window > 0 && key <= p - window)) T[s2][i] = -INFINITY;
+              }
+          }
+          ma = wt_max(T[0][0], T[1][0]), mb = wt_max(T[0][1], T[1][1]);
+        }
+#pragma unroll
+        for (int f = 0; f < 8; ++f) {
+          if constexpr (CUR) O[f & 3] = mfma32(fr[f], pg[f >> 2], O[f & 3]);
+          if constexpr (NXT) {
+            fr[f] = kfrag(kc2, f);                     // (past the run's last tile: not used)
+            if (f > 0) {
+              ma = wt_max(wt_max(ma, T[0][2 * f]), T[1][2 * f]);
+              mb = wt_max(wt_max(mb, T[0][2 * f + 1]), T[1][2 * f + 1]);
             }
+          }
+          __builtin_amdgcn_sched_barrier(0);
         }
-        float ma = wt_max(S[0][0], S[1][0]), mb = wt_max(S[0][1], S[1][1]);
-#pragma unroll
-        for (int i = 2; i < 16; i += 2) {
-          ma = wt_max(wt_max(ma, S[0][i]), S[1][i]);
-          mb = wt_max(wt_max(mb, S[0][i + 1]), S[1][i + 1]);
-        }
-        float mx = wt_max(ma, mb);
-        {
+        if constexpr (NXT) {
+          float mx = wt_max(ma, mb);
           const auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
           mx = wt_max(__uint_as_float(r2[0]), __uint_as_float(r2[1])) * scale_log2e;   // (the scale is positive)
-        }
-        if (__any(!(mx <= m + WT_THR))) {
-          const float mn = fmaxf(m, mx);
-          const float corr = mn == -INFINITY ? 1.f : fast_exp2(m - mn);
-          l *= corr;
+          if (__any(!(mx <= m + WT_THR))) {
+            const float mn = fmaxf(m, mx);
+            const float corr = mn == -INFINITY ? 1.f : fast_exp2(m - mn);
+            l *= corr;
 #pragma unroll
-          for (int v = 0; v < NVT; ++v) O[v] *= corr;
-          m = mn;
-        }
-        const float base = m == -INFINITY ? 0.f : m;   // nothing visible yet: every weight is 2^-inf = 0
-#pragma unroll
-        for (int sb = 0; sb < 2; ++sb) {
-          bf16x8 vf[2][NVT];
-#pragma unroll
-          for (int pg = 0; pg < 2; ++pg)
-#pragma unroll
-            for (int v = 0; v < NVT; ++v) vf[pg][v] = *reinterpret_cast<const bf16x8*>(sl + vat[v] + sb * 8192 + pg * 4096);
-          bf16x8 pf[2];
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const float e = fast_exp2(fmaf(S[sb][i], scale_log2e, -base));
-            l += e;
-            pf[i >> 3][i & 7] = (bf16)e;
+            for (int v = 0; v < NVT; ++v) O[v] *= corr;
+            m = mn;
           }
-#pragma unroll
-          for (int pg = 0; pg < 2; ++pg)
-#pragma unroll
-            for (int v = 0; v < NVT; ++v) O[v] = mfma32(vf[pg][v], pf[pg], O[v]);
         }
+      };
+      const int first = on ? max(jb - run, 0) : n, end = on ? min(je - run, n) : 0;   // this wave's tiles of the run
+      int j = -1;
+      if (first < end) {
+        for (; j + 1 < first; ++j) meet(j);
+        step(std::false_type{}, std::true_type{}, j, sb, sa);
+        ++j;
+        for (; j + 2 < end; j += 2) {
+          step(std::true_type{}, std::true_type{}, j, sa, sb);
+          step(std::true_type{}, std::true_type{}, j + 1, sb, sa);
+        }
+        if (j + 1 < end) {
+          step(std::true_type{}, std::true_type{}, j, sa, sb);
+          sa[0] = sb[0];
+          sa[1] = sb[1];
+          ++j;
+        }
+        step(std::true_type{}, std::false_type{}, j, sa, sb);
+        ++j;
       }
+      for (; j < n; ++j) meet(j);
       lds_barrier();   // (the run's page ids and slots have been read)
     }
   }

@@ -466,8 +466,8 @@ _NP2TORCH = {np.dtype(np.int64): torch.int64, np.dtype(np.int32): torch.int32, n
 
 class _Stager:
     """Per-step host->device uploads through a ring of pinned staging arenas (one arena per launch, bump-allocated):
-    no pinned allocation and no pageable copy on the step path, so every upload is a plain async DMA in stream
-    order. An arena is reused ``depth`` launches later, when at most two steps can be in flight — its copies have
+    no pinned allocation and no pageable copy on the step path, so every upload runs in stream order without the host
+    (a kernel that reads the arena, a copy engine for large ones: ``ops.host_copy``). An arena is reused ``depth`` launches later, when at most two steps can be in flight — its copies have
     executed by then."""
 
     def __init__(self, device: torch.device, nbytes: int = 8 << 20, depth: int = 4):
@@ -492,7 +492,7 @@ class _Stager:
 
     def upload_many(self, arrays: list[np.ndarray]) -> list[torch.Tensor]:
         """Several arrays staged back to back (256-B aligned) and moved by ONE async copy into one device buffer —
-        a step's plan and sampling parameters cost one copy launch instead of one each; returns device views."""
+        a step's plan and sampling parameters cost one launch instead of one each; returns device views."""
         arrays = [np.ascontiguousarray(a) for a in arrays]
         if self.device.type != "cuda":
             return [torch.from_numpy(a) for a in arrays]
@@ -510,7 +510,7 @@ class _Stager:
             host[base + o:base + o + a.nbytes] = a.reshape(-1).view(np.uint8)
         self.off = base + off
         dev = torch.empty(off, dtype=torch.uint8, device=self.device)
-        dev.copy_(buf[base:base + off], non_blocking=True)
+        ops.host_copy(dev, buf[base:base + off])
         return [dev[o:o + a.nbytes].view(_NP2TORCH[a.dtype]).view(a.shape) for a, o in zip(arrays, offs)]
 
     def upload(self, a: np.ndarray) -> torch.Tensor:
@@ -528,7 +528,7 @@ class _Stager:
         stage.numpy()[:] = a.reshape(-1).view(np.uint8)
         self.off = off + nb
         dev = torch.empty(a.size, dtype=_NP2TORCH[a.dtype], device=self.device)
-        dev.view(torch.uint8).copy_(stage, non_blocking=True)
+        ops.host_copy(dev.view(torch.uint8).view(-1), stage)
         return dev.view(a.shape)
 
     def upload_into(self, arrays: list[np.ndarray | None], offs: list[int], dst: torch.Tensor) -> None:
@@ -554,7 +554,7 @@ class _Stager:
                 a = np.ascontiguousarray(a)
                 host[base + o:base + o + a.nbytes] = a.reshape(-1).view(np.uint8)
         self.off = base + n
-        dst.copy_(buf[base:base + n], non_blocking=True)
+        ops.host_copy(dst, buf[base:base + n])
 
 
 @dataclass

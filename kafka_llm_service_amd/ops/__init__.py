@@ -102,6 +102,18 @@ def rows_add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, rows: torch.Tensor
     return fused_add_rmsnorm(x.index_select(1 if slab else 0, rows), residual.index_select(0, rows), w, eps)
 
 
+# Uploads by a kernel up to here, by a copy engine beyond: eight small kernels and an upload take, engine / kernel, us, 41.7 / 40.2 at
+# 300 KB, 45.1 / 40.0 at 512 KB, 53 / 41 at 1 MiB (the host's 36 - 40 us of launches cover the rest), and beyond that both follow the
+# link (69 / 57 at 2 MiB, 105 / 92 at 4), where an engine leaves the CUs to other streams. A decoding step's plan: see host_copy_kernel.
+HOST_COPY_MAX = 1 << 20
+
+
+def host_copy(dst: torch.Tensor, src: torch.Tensor) -> None:
+    """dst <- src, bytes in pinned host memory, in stream order; the host does not wait."""
+    if src.numel() > HOST_COPY_MAX or not ext().host_copy(dst, src):
+        dst.copy_(src, non_blocking=True)
+
+
 def gather_rows(table: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
     """table[idx] for rows of a matrix."""
     if idx.shape[0] and table.dim() == 2 and _whole_rows(table, idx) and table.dtype in (torch.float32, torch.bfloat16) and \

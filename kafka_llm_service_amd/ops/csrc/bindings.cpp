@@ -2,6 +2,7 @@
 // Python bindings for the CDNA4 kernels. Host-side shape / dtype / device checks live here so that a malformed
 // call fails with a Python exception instead of launching a kernel on a shape it does not assume.
 #include <torch/extension.h>
+#include <ATen/core/CachingHostAllocator.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 
@@ -19,6 +20,7 @@ hipError_t kafka_launch_rows_norm(bf16* out, int64_t os, const bf16* x, int64_t 
                                   hipStream_t st);
 hipError_t kafka_launch_gather_rows(void* out, int64_t out_bytes, const void* src, int64_t src_bytes, const int64_t* idx,
                                     int64_t n_src, int n, int row_bytes, hipStream_t st);
+hipError_t kafka_launch_host_copy(void* dst, const void* src, int64_t n, hipStream_t st);
 hipError_t kafka_launch_silu_mul(bf16* out, const bf16* x, int64_t xs, int T, int F, int gelu, hipStream_t st);
 hipError_t kafka_launch_silu_mul_slab(bf16* out, const float* xp, int S, int64_t ps, int T, int F, int gelu, hipStream_t st);
 hipError_t kafka_launch_rope_kv(const bf16* qkv, const float* qp, int S, int64_t ps, int64_t qkv_stride,
@@ -231,6 +233,29 @@ static void gather_rows(at::Tensor out, at::Tensor src, at::Tensor idx) {
   TORCH_CHECK(row % 16 == 0 && row > 0 && row < (1 << 24) && al(src) && al(out), "gather_rows: rows of whole 16-byte pieces");
   CHECK_HIP(kafka_launch_gather_rows(out.data_ptr(), out.stride(0) * e, src.data_ptr(), src.stride(0) * e, idx.data_ptr<int64_t>(),
                                      src.size(0), (int)idx.size(0), (int)row, cur_stream()));
+}
+
+// dst <- src (bytes) by a kernel on the current stream that reads the pinned memory itself; false (and nothing done) where src is not
+// memory of torch's pinned allocator that the device sees at the host's address. The allocator keeps a freed block until the
+// stream has passed the kernel, as for its own copies.
+static bool host_copy(at::Tensor dst, at::Tensor src) {
+  CHECK_CUDA(dst); CHECK_DT(dst, at::kByte); CHECK_DT(src, at::kByte);
+  TORCH_CHECK(src.device().is_cpu() && dst.is_contiguous() && src.is_contiguous() && dst.numel() == src.numel(), "host_copy: operands");
+  const int64_t n = src.numel();
+  if (n == 0) return true;
+  if (reinterpret_cast<uintptr_t>(dst.data_ptr()) % 8 || reinterpret_cast<uintptr_t>(src.data_ptr()) % 8 || n >= (int64_t)1 << 40) return false;
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, src.data_ptr()) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (a.type != hipMemoryTypeHost || a.devicePointer != src.data_ptr()) return false;
+  const auto& store = src.storage().data_ptr();
+  const auto stream = c10::hip::getCurrentHIPStream();
+  if (!at::getHostAllocator(at::kCUDA)->record_event(store.get(), store.get_context(), c10::Stream(c10::Stream::UNSAFE, c10::Device(at::kCUDA, stream.device_index()), stream.id())))
+    return false;
+  CHECK_HIP(kafka_launch_host_copy(dst.data_ptr(), src.data_ptr(), n, stream.stream()));
+  return true;
 }
 
 // x: bf16 [T, 2F] or slab [S, T, 2F]; gelu: its tanh form in SiLU's place
@@ -1320,6 +1345,7 @@ PYBIND11_MODULE(_kafka_ops, m) {
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
   m.def("rows_norm", &rows_norm);
   m.def("gather_rows", &gather_rows);
+  m.def("host_copy", &host_copy);
   m.def("silu_mul", &silu_mul, py::arg("out"), py::arg("x"), py::arg("gelu") = false);
   m.def("rope_kv_write", &rope_kv_write);
   m.def("attn_decode", &attn_decode, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),

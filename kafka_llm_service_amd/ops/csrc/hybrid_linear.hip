@@ -38,7 +38,23 @@ constexpr int NT = 256;
 constexpr float LOG2E = 1.4426950408889634f;
 
 __device__ __forceinline__ float sigmoidf(float z) { return 1.0f / (1.0f + expf(-z)); }
-__device__ __forceinline__ float softplusf(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
+// max(z, 0) + log(1 + u), u = e^-|z| <= 1: log(1 + u) as u + u^2 Q(u) with a minimax fit Q of degree 9 over 0 .. 1 (relative
+// error of the sum 8e-10; 1.15 ulp at most and 0.30 rms of what u is exact for, as the library's function, which takes 130
+// instructions and a branch to 11 here)
+__device__ __forceinline__ float softplusf(float z) {
+  const float u = expf(-fabsf(z));
+  float q = 0.0020729179959744215f;
+  q = __builtin_fmaf(q, u, -0.013631332665681839f);
+  q = __builtin_fmaf(q, u, 0.0419810488820076f);
+  q = __builtin_fmaf(q, u, -0.0830736979842186f);
+  q = __builtin_fmaf(q, u, 0.12467096000909805f);
+  q = __builtin_fmaf(q, u, -0.16129323840141296f);
+  q = __builtin_fmaf(q, u, 0.19897928833961487f);
+  q = __builtin_fmaf(q, u, -0.24988578259944916f);
+  q = __builtin_fmaf(q, u, 0.33332690596580505f);
+  q = __builtin_fmaf(q, u, -0.49999988079071045f);
+  return fmaxf(z, 0.f) + __builtin_fmaf(u * u, q, u);
+}
 // Workgroup barrier for LDS hand-overs that leaves global loads (a prefetched next block) in flight: __syncthreads()
 // would drain them as well. This wave's LDS reads and writes are complete (lgkmcnt 0) before it arrives.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -384,7 +400,7 @@ struct ChunkBuf {
   float* W;    // [2][Dp / 16] fragments: rows t, columns d of W (delta rule)
   float* K;    // [Dp / 16][2] fragments: rows d, columns t of k_t e^(b_end - b_t)
   float* E;    // [Dp]         e^(b_end)
-  float* P;    // [32][32]
+  float* P;    // [4][64][4]   per wave w and lane l of the scan: rows l % 16 and 16 + l % 16, columns 16 (w / 2) + 4 (l / 16) + 2 (w % 2) and the next
   float* U;    // [2][NV] tiles of U0 in the accumulator layout: lane l holds rows 4 (l / 16) .. + 3 of column l % 16
 };
 
@@ -460,23 +476,40 @@ __global__ __launch_bounds__(NT) void lin_chunk_prep_kernel(LinIn<AT> in, const 
     Ps[i] = 0.f;
     if (DELTA) As[i] = 0.f;
   }
+  float nf = 0.f;   // delta rule, unit vectors: lanes 4 i .. + 3 the factor of query row i, of key row i - 8
+  if constexpr (DELTA) {
+    float v[16];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      v[j] = v[8 + j] = 0.f;
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        if (8 * w + j >= n || DS * s + lane >= D) qv[s][j] = kv[s][j] = 0.f;
+        v[j] += qv[s][j] * qv[s][j];
+        v[8 + j] += kv[s][j] * kv[s][j];
+      }
+    }
+#pragma unroll
+    for (int k = 8; k > 0; k >>= 1) {   // sixteen sums over the wave, half of them handed over in each exchange
+      const bool up = lane & (4 * k);
+#pragma unroll
+      for (int i = 0; i < k; ++i) {
+        const float lo = v[i], hi = v[i + k];
+        v[i] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, 4 * k, 64);
+      }
+    }
+    v[0] += __shfl_xor(v[0], 2, 64);
+    v[0] += __shfl_xor(v[0], 1, 64);
+    nf = (lane < 32 ? in.qscale : 1.0f) / sqrtf(v[0] + UNIT_EPS);
+  }
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const bool ok = 8 * w + j < n;
-    float sq = 0.f, sk = 0.f;
+    const float fq = DELTA ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(nf), 4 * j)) : in.qscale;
+    const float fk = DELTA ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(nf), 32 + 4 * j)) : 1.0f;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       if (!ok || DS * s + lane >= D) qv[s][j] = kv[s][j] = 0.f;
-      sq += qv[s][j] * qv[s][j];
-      sk += kv[s][j] * kv[s][j];
-    }
-    float fq = in.qscale, fk = 1.0f;
-    if (DELTA) {   // unit vectors
-      fq = in.qscale / sqrtf(wave_sum(sq) + UNIT_EPS);
-      fk = 1.0f / sqrtf(wave_sum(sk) + UNIT_EPS);
-    }
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
       qv[s][j] *= fq;
       kv[s][j] *= fk;
       const float lg = ok && DS * s + lane < D ? log_decay<DELTA>(b[s][j] + zb[s], rate, in.inv_tau) * LOG2E : 0.f;
@@ -592,7 +625,7 @@ __global__ __launch_bounds__(NT) void lin_chunk_prep_kernel(LinIn<AT> in, const 
   __syncthreads();
   if (!DELTA || w > 0) {
     for (int i = DELTA ? threadIdx.x - 64 : threadIdx.x; i < CH * CH; i += DELTA ? NT - 64 : NT)
-      cb.P[ch * CH * CH + i] = Ps[(i >> 5) * LA + (i & 31)];
+      cb.P[ch * CH * CH + i] = Ps[(8 * (i & 2) + ((i >> 2) & 15)) * LA + 16 * (i >> 9) + 4 * ((i >> 6) & 3) + 2 * ((i >> 8) & 1) + (i & 1)];
   }
   if constexpr (DELTA) {
     if (w == 0) {
@@ -694,7 +727,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NTL > 2 || D
 void lin_chunk_scan_kernel(
     LinIn<AT> in, const int* __restrict__ vseg, const int* __restrict__ cs, ChunkBuf cb, float* __restrict__ Sst,
     float* __restrict__ out, int64_t os) {
-  __shared__ f32x4 red[4][2][64];
+  __shared__ f32x4 red[DELTA ? 4 : 2][2][64];
   __shared__ __attribute__((aligned(16))) f32x4 redo[2][4][2][64];
   const int D = in.D, Dv = in.Dv, Dp = (D + 15) & ~15, NV = (Dv + 15) >> 4, ndt = Dp >> 4;
   int vt, h;
@@ -709,7 +742,7 @@ void lin_chunk_scan_kernel(
   const int r = blockIdx.y;
   const int first = cs[4 * r], cnt = cs[4 * r + 1], p0 = cs[4 * r + 2], slot = cs[4 * r + 3];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, m = lane & 15, kq = lane >> 4;
-  const int vcol = vt * 16 + m;
+  const int vcol = vt * 16 + m, vrow = 16 * (w >> 1) + 4 * kq + 2 * (w & 1);
   float* Sp = Sst + (((int64_t)slot * in.H + h) * D) * Dv + vcol;
   f32x4 S[NTL];
 #pragma unroll
@@ -719,9 +752,10 @@ void lin_chunk_scan_kernel(
       const int d = (w * NTL + a) * 16 + 4 * kq + i;
       S[a][i] = (p0 > 0 && d < D && vcol < Dv) ? Sp[(int64_t)d * Dv] : 0.f;
     }
+  // values as they lie in memory: converted while they are read, they would be waited for where they are asked for
   struct Ops {
-    f32x4 W[2][NTL], Q[2][NTL], K[NTL][2], E[NTL], U[2];
-    f32x2 P[2];
+    f32x4 W[2][NTL], Q[2][NTL], K[NTL][2], E[NTL], U[2], P;
+    AT V[2];
   };
   Ops ops[2];
   // a segment's chunks are consecutive rows, all whole but the last
@@ -751,10 +785,7 @@ void lin_chunk_scan_kernel(
       for (int tt = 0; tt < 2; ++tt) o.K[a][tt] = *reinterpret_cast<const f32x4*>(Kp + (tile(a) * 2 + tt) * 256);
       o.E[a] = *reinterpret_cast<const f32x4*>(cb.E + ch * Dp + tile(a) * 16 + 4 * kq);
     }
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
-      o.P[rt] = *reinterpret_cast<const f32x2*>(cb.P + ch * CH * CH + (16 * rt + m) * CH + 16 * (w >> 1) + 4 * kq +
-                                                2 * (w & 1));
+    o.P = *reinterpret_cast<const f32x4*>(cb.P + ch * CH * CH + (w * 64 + lane) * 4);
     if constexpr (DELTA) {
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt)
@@ -763,12 +794,18 @@ void lin_chunk_scan_kernel(
       const int rows = c + 1 < last ? CH : tail;
       const AT* vp = in.v + (int64_t)(row0 + CH * (c - first)) * in.v_s + (int64_t)h * Dv + min(vcol, Dv - 1);
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o.U[tt][i] = ldf(vp + (int64_t)min(16 * tt + 4 * kq + i, rows - 1) * in.v_s);
+      for (int e = 0; e < 2; ++e) o.V[e] = vp[(int64_t)min(vrow + e, rows - 1) * in.v_s];
     }
   };
-  auto step = [&](Ops& o, int c) {
+  // without the delta rule U is V: a wave brings its quarter (rows vrow, + 1 of the lane's column) for all, a chunk ahead
+  float uq[2] = {0.f, 0.f};
+  auto put = [&](const Ops& o, int c) {
+    const int n = c + 1 < last ? CH : tail;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) uq[e] = vrow + e >= n || vcol >= Dv ? 0.f : (float)o.V[e];
+    *reinterpret_cast<f32x2*>(reinterpret_cast<float*>(&red[c & 1][w >> 1][lane]) + 2 * (w & 1)) = f32x2{uq[0], uq[1]};
+  };
+  auto step = [&](Ops& o, const Ops& next, int c) {
     f32x4 ws[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, ow[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll
     for (int a = 0; a < NTL; ++a)
@@ -781,7 +818,7 @@ void lin_chunk_scan_kernel(
         }
     mfma_settle();
     const int t0 = row0 + CH * (c - first), n = c + 1 < last ? CH : tail;
-    if (c + 2 < last) load_a(o, c + 2);
+    load_a(o, min(c + 2, last - 1));   // (always: behind a branch, waits would be for everything that is on its way)
     if constexpr (DELTA) {
       red[w][0][lane] = ws[0];
       red[w][1][lane] = ws[1];
@@ -789,21 +826,17 @@ void lin_chunk_scan_kernel(
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt)
         o.U[tt] -= (red[0][tt][lane] + red[1][tt][lane]) + (red[2][tt][lane] + red[3][tt][lane]);
+      const f32x4 us = (w >> 1) ? o.U[1] : o.U[0];
+      uq[0] = (w & 1) ? us[2] : us[0];
+      uq[1] = (w & 1) ? us[3] : us[1];
     } else {
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (16 * tt + 4 * kq + i >= n || vcol >= Dv) o.U[tt][i] = 0.f;
+      for (int tt = 0; tt < 2; ++tt) o.U[tt] = red[c & 1][tt][lane];
     }
-    {
-      const f32x4 us = (w >> 1) ? o.U[1] : o.U[0];
-      const float u0 = (w & 1) ? us[2] : us[0], u1 = (w & 1) ? us[3] : us[1];
 #pragma unroll
-      for (int rt = 0; rt < 2; ++rt) {
-        ow[rt] = mfma16f(o.P[rt][0], u0, ow[rt]);
-        ow[rt] = mfma16f(o.P[rt][1], u1, ow[rt]);
-      }
+    for (int rt = 0; rt < 2; ++rt) {
+      ow[rt] = mfma16f(o.P[2 * rt], uq[0], ow[rt]);
+      ow[rt] = mfma16f(o.P[2 * rt + 1], uq[1], ow[rt]);
     }
     f32x4* ro = &redo[c & 1][0][0][0];
     ro[(w * 2 + 0) * 64 + lane] = ow[0];
@@ -820,7 +853,8 @@ void lin_chunk_scan_kernel(
         }
     }
     mfma_settle();
-    if (c + 2 < last) load_b(o, c + 2);
+    if constexpr (!DELTA) put(next, c + 1);
+    load_b(o, min(c + 2, last - 1));
     lds_barrier();
     {
       const int rt = threadIdx.x >> 7, l2 = (threadIdx.x & 127) >> 1, part = threadIdx.x & 1;
@@ -833,15 +867,22 @@ void lin_chunk_scan_kernel(
       }
     }
   };
+  if (cnt > 0) {   // (uniform)
 #pragma unroll
-  for (int k = 0; k < 2; ++k)
-    if (k < cnt) {
-      load_a(ops[k], first + k);
-      load_b(ops[k], first + k);
+    for (int k = 0; k < 2; ++k) {
+      load_a(ops[k], min(first + k, last - 1));
+      load_b(ops[k], min(first + k, last - 1));
     }
-  for (int c = first; c < last; c += 2) {
-    step(ops[0], c);
-    if (c + 1 < last) step(ops[1], c + 1);
+    if constexpr (!DELTA) {
+      put(ops[0], first);
+      lds_barrier();
+    }
+    int c = first;
+    for (; c + 1 < last; c += 2) {
+      step(ops[0], ops[1], c);
+      step(ops[1], ops[0], c + 1);
+    }
+    if (c < last) step(ops[0], ops[1], c);
   }
 #pragma unroll
   for (int a = 0; a < NTL; ++a)

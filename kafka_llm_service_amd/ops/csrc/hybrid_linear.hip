@@ -719,11 +719,12 @@ __global__ __launch_bounds__(NT) void lin_chunk_prep_kernel(LinIn<AT> in, const 
 // (Q e^b) S over the wave's rows; the waves' parts of W S are summed through LDS to U; the state's update; a quarter of
 // P U per wave; the waves' parts of the output summed through LDS. The operands of the next two chunks are in flight.
 // The column tiles of a head are given to workgroups of one XCD where the heads divide by 8: they read the same operands.
-// What bounds it: half the time fp32 products, else a chunk's chain of loads and exchanges. Up to 128 channels without the delta rule
-// three workgroups fit a CU when the registers are held to 160 (2529 rows of three segments, 32 heads: 156 -> 117 us; left
-// to itself the compiler aims at two); with it that costs 34 spilled registers (181 -> 244), so two.
-template <typename AT, int NTL, bool FULL, bool DELTA>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NTL > 2 || DELTA ? 1 : 3, NTL > 2 ? 1 : DELTA ? 2 : 3)))
+// What bounds it: fp32 products (two fifths of the time their units are busy; 42 of 92 us below), each chunk's exchanges and its 52 KB of operands.
+// Up to 128 channels without the delta rule three workgroups fit a CU when the registers are held to 168: 2805 rows of three
+// segments, 16 heads of 256 value columns 92 us (108 with every wave waiting for all values where it asked for them). With it two do,
+// or three with one chunk's operands on their way (DEPTH 1); the rule is where it is launched.
+template <typename AT, int NTL, bool FULL, bool DELTA, int DEPTH>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NTL > 2 || (DELTA && DEPTH > 1) ? 1 : 3, NTL > 2 ? 1 : DELTA && DEPTH > 1 ? 2 : 3)))
 void lin_chunk_scan_kernel(
     LinIn<AT> in, const int* __restrict__ vseg, const int* __restrict__ cs, ChunkBuf cb, float* __restrict__ Sst,
     float* __restrict__ out, int64_t os) {
@@ -757,7 +758,8 @@ void lin_chunk_scan_kernel(
     f32x4 W[2][NTL], Q[2][NTL], K[NTL][2], E[NTL], U[2], P;
     AT V[2];
   };
-  Ops ops[2];
+  static_assert(DEPTH == 2 || DELTA, "values are handed over a chunk ahead");
+  Ops ops[DEPTH];
   // a segment's chunks are consecutive rows, all whole but the last
   const int last = first + cnt, row0 = cnt > 0 ? vseg[4 * first] : 0;
   const int tail = cnt > 0 ? vseg[4 * (last - 1) + 1] : 0;
@@ -818,7 +820,7 @@ void lin_chunk_scan_kernel(
         }
     mfma_settle();
     const int t0 = row0 + CH * (c - first), n = c + 1 < last ? CH : tail;
-    load_a(o, min(c + 2, last - 1));   // (always: behind a branch, waits would be for everything that is on its way)
+    load_a(o, min(c + DEPTH, last - 1));   // (always: behind a branch, waits would be for everything that is on its way)
     if constexpr (DELTA) {
       red[w][0][lane] = ws[0];
       red[w][1][lane] = ws[1];
@@ -854,7 +856,7 @@ void lin_chunk_scan_kernel(
     }
     mfma_settle();
     if constexpr (!DELTA) put(next, c + 1);
-    load_b(o, min(c + 2, last - 1));
+    load_b(o, min(c + DEPTH, last - 1));
     lds_barrier();
     {
       const int rt = threadIdx.x >> 7, l2 = (threadIdx.x & 127) >> 1, part = threadIdx.x & 1;
@@ -869,7 +871,7 @@ void lin_chunk_scan_kernel(
   };
   if (cnt > 0) {   // (uniform)
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < DEPTH; ++k) {
       load_a(ops[k], min(first + k, last - 1));
       load_b(ops[k], min(first + k, last - 1));
     }
@@ -877,12 +879,16 @@ void lin_chunk_scan_kernel(
       put(ops[0], first);
       lds_barrier();
     }
-    int c = first;
-    for (; c + 1 < last; c += 2) {
-      step(ops[0], ops[1], c);
-      step(ops[1], ops[0], c + 1);
+    if constexpr (DEPTH == 1) {
+      for (int c = first; c < last; ++c) step(ops[0], ops[0], c);
+    } else {
+      int c = first;
+      for (; c + 1 < last; c += 2) {
+        step(ops[0], ops[1], c);
+        step(ops[1], ops[0], c + 1);
+      }
+      if (c < last) step(ops[0], ops[1], c);
     }
-    if (c < last) step(ops[0], ops[1], c);
   }
 #pragma unroll
   for (int a = 0; a < NTL; ++a)
@@ -1144,24 +1150,30 @@ hipError_t kafka_hy_lin_chunked(int f32, const void* qk, int64_t qk_s, int q_off
                        q_off, k_off, H, G, D, Dv, qscale, inv_tau};
     auto p = [&](auto k) { k<<<g1, NT, 0, st>>>(in, vseg, cb); };
     auto b = [&](auto k) { k<<<g2, NT, 0, st>>>(in, vseg, cs, cb, S, out, os); };
+    // The delta rule up to 128 channels: two workgroups a CU with two chunks' operands on their way, three with one. Three where they need
+    // fewer rounds of the chip's 256 CUs. Preparation and scan, us, two / three a CU, 128 channels and value columns, 32 heads:
+    // segments of 1100, 843 and 862 (768 workgroups) 221 / 194, seven of 300 (1792) 156 / 151; four of 700 (1024) 189 / 202,
+    // one of 4000 (256) 295 / 364, 500 and 600 (512) 83 / 85.
+    const int64_t wgs = (int64_t)g2.x * g2.y;
+    const bool three = (wgs + 767) / 768 < (wgs + 511) / 512;
     if (rate != nullptr) {
       if (D <= 64) p(lin_chunk_prep_kernel<AT, 1, true>);
       else if (D <= 128) p(lin_chunk_prep_kernel<AT, 2, true>);
       else p(lin_chunk_prep_kernel<AT, 4, true>);
-      if (D == 64) b(lin_chunk_scan_kernel<AT, 1, true, true>);
-      else if (D == 128) b(lin_chunk_scan_kernel<AT, 2, true, true>);
-      else if (D < 64) b(lin_chunk_scan_kernel<AT, 1, false, true>);
-      else if (D < 128) b(lin_chunk_scan_kernel<AT, 2, false, true>);
-      else b(lin_chunk_scan_kernel<AT, 4, false, true>);
+      if (D == 64) b(lin_chunk_scan_kernel<AT, 1, true, true, 2>);
+      else if (D == 128) (three ? b(lin_chunk_scan_kernel<AT, 2, true, true, 1>) : b(lin_chunk_scan_kernel<AT, 2, true, true, 2>));
+      else if (D < 64) b(lin_chunk_scan_kernel<AT, 1, false, true, 2>);
+      else if (D < 128) (three ? b(lin_chunk_scan_kernel<AT, 2, false, true, 1>) : b(lin_chunk_scan_kernel<AT, 2, false, true, 2>));
+      else b(lin_chunk_scan_kernel<AT, 4, false, true, 2>);
     } else {
       if (D <= 64) p(lin_chunk_prep_kernel<AT, 1, false>);
       else if (D <= 128) p(lin_chunk_prep_kernel<AT, 2, false>);
       else p(lin_chunk_prep_kernel<AT, 4, false>);
-      if (D == 64) b(lin_chunk_scan_kernel<AT, 1, true, false>);
-      else if (D == 128) b(lin_chunk_scan_kernel<AT, 2, true, false>);
-      else if (D < 64) b(lin_chunk_scan_kernel<AT, 1, false, false>);
-      else if (D < 128) b(lin_chunk_scan_kernel<AT, 2, false, false>);
-      else b(lin_chunk_scan_kernel<AT, 4, false, false>);
+      if (D == 64) b(lin_chunk_scan_kernel<AT, 1, true, false, 2>);
+      else if (D == 128) b(lin_chunk_scan_kernel<AT, 2, true, false, 2>);
+      else if (D < 64) b(lin_chunk_scan_kernel<AT, 1, false, false, 2>);
+      else if (D < 128) b(lin_chunk_scan_kernel<AT, 2, false, false, 2>);
+      else b(lin_chunk_scan_kernel<AT, 4, false, false, 2>);
     }
   });
   return hipGetLastError();

@@ -559,11 +559,8 @@ class BuduraxLM:
         cfg, dt, dev = self.cfg, self.dtype, self.device
         m: SegMeta = inp.attn
         T, d, eps = inp.tokens.shape[0], cfg.hidden_size, cfg.norm_eps
-        x = ops.gather_rows(self.embed, inp.tokens)  # fp32 [T, d] residual stream
-        stack = None
-        if self.has_dwa:
-            stack = torch.empty(len(self.layers) + 1, T, d, dtype=torch.float32, device=dev)
-            stack[0].copy_(x)
+        stack = torch.empty(len(self.layers) + 1, T, d, dtype=torch.float32, device=dev) if self.has_dwa else None
+        x = ops.gather_rows(self.embed, inp.tokens, None if stack is None else stack[0])  # fp32 [T, d] residual stream
         h = torch.empty(T, d, dtype=dt, device=dev)
         h2 = torch.empty(T, d, dtype=dt, device=dev)
         # the slots' shift rows: written in place unless a portion of several rows goes on from its slot

@@ -435,12 +435,11 @@ class FurapelLM:
         cfg, dt, dev = self.cfg, self.dtype, self.device
         m: SegMeta = inp.attn
         T, d = inp.tokens.shape[0], cfg.hidden_size
-        x = ops.gather_rows(self.embed, inp.tokens)       # fp32 [T, d] residual (the table holds the scale)
         h1, h2 = (torch.empty(T, d, dtype=dt, device=dev) for _ in range(2))
         both = None                                   # the loop product's input [residual | embedding rows]
         if self.loop_in is not None:
             both = torch.empty(T, 2 * d, dtype=dt, device=dev)
-            both[:, d:] = x
+        x = ops.gather_rows(self.embed, inp.tokens, None if both is None else both[:, d:])   # fp32 [T, d] residual (the table holds the scale)
 
         def outputs(r):
             """What the element-wise pass in front of run r leaves: the norms of its layer, or - where a pass of the

@@ -478,9 +478,8 @@ class RogosunLM:
         cfg, dt, dev = self.cfg, self.dtype, self.device
         m: SegMeta = inp.attn
         d, eps = cfg.hidden_size, cfg.norm_eps
-        x = ops.gather_rows(self.embed, inp.tokens)       # fp32 [T, d] residual
-        h = torch.empty(x.shape, dtype=dt, device=dev)
-        h.copy_(x)                                    # what the sublayers read: x in the model dtype
+        h = torch.empty(inp.tokens.shape[0], d, dtype=dt, device=dev)   # what the sublayers read: x in the model dtype
+        x = ops.gather_rows(self.embed, inp.tokens, h)    # fp32 [T, d] residual
         for i, lw in enumerate(self.layers):
             st = state.layers[i]
             last = i + 1 == len(self.layers)

@@ -114,14 +114,21 @@ def host_copy(dst: torch.Tensor, src: torch.Tensor) -> None:
         dst.copy_(src, non_blocking=True)
 
 
-def gather_rows(table: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
-    """table[idx] for rows of a matrix."""
+def gather_rows(table: torch.Tensor, idx: torch.Tensor, also: torch.Tensor | None = None) -> torch.Tensor:
+    """table[idx] for rows of a matrix; ``also`` [n, d] gets them as well, in its own type."""
     if idx.shape[0] and table.dim() == 2 and _whole_rows(table, idx) and table.dtype in (torch.float32, torch.bfloat16) and \
             table.shape[1] * table.element_size() < 1 << 24:
         out = torch.empty(idx.shape[0], table.shape[1], dtype=table.dtype, device=table.device)
-        ext().gather_rows(out, table, idx)
+        fused = also is not None and also.stride(1) == 1 and also.stride(0) % 8 == 0 and also.data_ptr() % 16 == 0 and \
+            (also.dtype == table.dtype or also.dtype == torch.bfloat16)
+        ext().gather_rows(out, table, idx, also if fused else None)
+        if also is not None and not fused:
+            also.copy_(out)
         return out
-    return table.index_select(0, idx)
+    out = table.index_select(0, idx)
+    if also is not None:
+        also.copy_(out)
+    return out
 
 
 def silu_mul(x: torch.Tensor, out: torch.Tensor | None = None, act: str = "silu") -> torch.Tensor:

@@ -19,7 +19,8 @@ hipError_t kafka_launch_rows_norm(bf16* out, int64_t os, const bf16* x, int64_t 
                                   int64_t rs, const int64_t* idx, int64_t n_src, const bf16* w, int n, int d, float eps, int embed,
                                   hipStream_t st);
 hipError_t kafka_launch_gather_rows(void* out, int64_t out_bytes, const void* src, int64_t src_bytes, const int64_t* idx,
-                                    int64_t n_src, int n, int row_bytes, hipStream_t st);
+                                    int64_t n_src, int n, int row_bytes, void* also, int64_t also_bytes, int also_half,
+                                    hipStream_t st);
 hipError_t kafka_launch_host_copy(void* dst, const void* src, int64_t n, hipStream_t st);
 hipError_t kafka_launch_silu_mul(bf16* out, const bf16* x, int64_t xs, int T, int F, int gelu, hipStream_t st);
 hipError_t kafka_launch_silu_mul_slab(bf16* out, const float* xp, int S, int64_t ps, int T, int F, int gelu, hipStream_t st);
@@ -222,8 +223,8 @@ static void rows_norm(at::Tensor out, at::Tensor x, at::Tensor residual, at::Ten
                                    cur_stream()));
 }
 
-// out[i] = src[idx[i]]: fp32 or bf16 rows of whole 16-byte pieces
-static void gather_rows(at::Tensor out, at::Tensor src, at::Tensor idx) {
+// out[i] = src[idx[i]]: fp32 or bf16 rows of whole 16-byte pieces; also: a second output of the same type, or bf16 of fp32 rows
+static void gather_rows(at::Tensor out, at::Tensor src, at::Tensor idx, c10::optional<at::Tensor> also) {
   CHECK_CUDA(src); CHECK_CUDA(out); CHECK_CUDA(idx); CHECK_DT(idx, at::kLong); CHECK_LASTDIM(src); CHECK_LASTDIM(out);
   TORCH_CHECK(src.dim() == 2 && out.dim() == 2 && idx.dim() == 1 && idx.is_contiguous() && src.scalar_type() == out.scalar_type() &&
                   (src.scalar_type() == at::kFloat || src.scalar_type() == at::kBFloat16) && out.size(0) == idx.size(0) &&
@@ -231,8 +232,22 @@ static void gather_rows(at::Tensor out, at::Tensor src, at::Tensor idx) {
   const int64_t e = src.element_size(), row = src.size(1) * e;
   auto al = [&](const at::Tensor& t) { return t.stride(0) * e % 16 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
   TORCH_CHECK(row % 16 == 0 && row > 0 && row < (1 << 24) && al(src) && al(out), "gather_rows: rows of whole 16-byte pieces");
+  void* ap = nullptr;
+  int64_t as = 0;
+  bool half = false;
+  if (also) {
+    const at::Tensor& t = *also;
+    CHECK_CUDA(t); CHECK_LASTDIM(t);
+    half = t.scalar_type() != src.scalar_type();
+    const int64_t piece = half ? 8 : 16;
+    as = t.stride(0) * t.element_size();
+    ap = t.data_ptr();
+    TORCH_CHECK(t.dim() == 2 && t.size(0) == out.size(0) && t.size(1) == out.size(1) &&
+                    (!half || (src.scalar_type() == at::kFloat && t.scalar_type() == at::kBFloat16)) && as % piece == 0 &&
+                    reinterpret_cast<uintptr_t>(ap) % piece == 0, "gather_rows: the second output");
+  }
   CHECK_HIP(kafka_launch_gather_rows(out.data_ptr(), out.stride(0) * e, src.data_ptr(), src.stride(0) * e, idx.data_ptr<int64_t>(),
-                                     src.size(0), (int)idx.size(0), (int)row, cur_stream()));
+                                     src.size(0), (int)idx.size(0), (int)row, ap, as, half ? 1 : 0, cur_stream()));
 }
 
 // dst <- src (bytes) by a kernel on the current stream that reads the pinned memory itself; false (and nothing done) where src is not

@@ -59,3 +59,16 @@ def test_weights_and_slabs_that_the_kernels_do_not_read(dev, dtype):
     even, wide = w.clone(), torch.randn(2, 14, 256, generator=g).to(dev)[:, 1:12]
     want = ops.fused_add_rmsnorm(wide.index_select(1, idx), table[idx], even, 1e-5)
     assert torch.equal(ops.rows_add_rmsnorm(wide, table, idx, even, 1e-5), want)
+
+
+@pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("d", [4, 64, 4096, 4104, 5000])
+def test_rows_gathered_twice(dev, d):
+    """The second output in the rows' type and in bf16, whole, as a part of wider rows, and where the kernel does not write it."""
+    g = torch.Generator().manual_seed(d)
+    table = torch.randn(9, d, generator=g).to(dev)
+    idx = torch.randint(0, 9, (5,), generator=g).to(dev)
+    for also in (torch.empty(5, d, device=dev), torch.empty(5, d, device=dev, dtype=torch.bfloat16),
+                 torch.empty(5, 2 * d, device=dev, dtype=torch.bfloat16)[:, d:], torch.empty(5, d + 3, device=dev)[:, 3:],
+                 torch.empty(5, d, device=dev, dtype=torch.float16)):
+        assert torch.equal(ops.gather_rows(table, idx, also), table[idx]) and torch.equal(also, table[idx].to(also.dtype))

@@ -292,12 +292,18 @@ class _Layer:
 HEAD_ROWS = 64   # rows up to which the heads' products run on the kernel for small products (figures: csrc/small_gemm.hip)
 
 
-def head_product(x, w, wt, out=None):
-    """Per head x [H, n, K] @ w [H, N, K]^T; ``wt``: the same weights [H, K, N], ``w`` None: those alone."""
+def head_product(x, w, wt, out=None, gate=None):
+    """Per head x [H, n, K] @ w [H, N, K]^T; ``wt``: the same weights [H, K, N], ``w`` None: those alone. ``gate`` [n, H N]: times its
+    sigmoid, into ``out`` [H, n, N], a view of [n, H N] rows."""
+    if gate is not None and not (gate.stride(0) % 4 == 0 and gate.stride(1) == 1 and gate.data_ptr() % 8 == 0 and gate.dtype == x.dtype):
+        w = None
     if w is not None and ops.small_ok(x, w, HEAD_ROWS) and (out is None or out.stride(0) % 4 == 0 and out.stride(1) % 4 == 0 and out.data_ptr() % 8 == 0):
         if out is None:
             out = torch.empty(x.shape[0], x.shape[1], w.shape[1], dtype=x.dtype, device=x.device)
-        ops.ext().small_gemm(x, w, out)
+        ops.ext().small_gemm(x, w, out, gate=gate)
+        return out
+    if gate is not None:
+        hops.sigmoid_mul(torch.bmm(x, wt), gate, out.transpose(0, 1).view(out.shape[1], -1))
         return out
     return torch.bmm(x, wt) if out is None else torch.bmm(x, wt, out=out)
 
@@ -319,10 +325,8 @@ def latent_mix(q, q_rot, cache, cache_t, lw, inp, m: SegMeta, ao, window: int = 
             tiles, keys = tiles[:n], int(m.seg_host[:n, 2].max()) + 1             # (single tokens: a tile each)
         hops.latent_attn(q_lat, q_rot[:n], cache, m.block_tables, m.tok_seg[:n], m.seg, inp.positions[:n], lw.scale, o_lat,
                          cache_t, tiles, keys, window=window, sink=sink)
-        if gate is None:
-            head_product(o_lat, lw.uv.view(H, Dv, R), lw.uv_ht, ao[:n].view(n, H, Dv).transpose(0, 1))  # head h -> its vdim columns
-        else:
-            hops.sigmoid_mul(head_product(o_lat, lw.uv.view(H, Dv, R), lw.uv_ht), gate[:n], ao[:n])
+        head_product(o_lat, lw.uv.view(H, Dv, R), lw.uv_ht, ao[:n].view(n, H, Dv).transpose(0, 1),  # head h -> its vdim columns
+                     None if gate is None else gate[:n])
     if n < T:
         hops.latent_attn_portions(q, q_rot, cache, lw.uk_h.view(H * D, R), lw.uv, tables, m.block_tables, lw.scale, ao, window,
                                   sink, gate)
@@ -598,9 +602,8 @@ class BuduraxLM:
                               (nl.norm1, nl.norm1_b, eps, h, nl.shift, m.tok_seg, m.seg, state.shift[i + 1]) if normed else None)
             if layers_out is not None:
                 layers_out.append(x.clone())
-        xs = ops.gather_rows(x, inp.logit_rows)
-        hf = torch.empty(xs.shape[0], d, dtype=dt, device=dev)
-        hops.ln_shift(xs, self.final_norm, self.final_norm_b, eps, hf)
+        hf = torch.empty(inp.logit_rows.shape[0], d, dtype=dt, device=dev)
+        hops.ln_rows(x, inp.logit_rows, self.final_norm, self.final_norm_b, eps, hf)
         return self._logits(hf)[:, :cfg.vocab_size]
 
     def _latent_attention(self, i: int, lw, h, inp, m: SegMeta, pages: list) -> torch.Tensor:

@@ -810,7 +810,7 @@ static int64_t skinny_plan(int64_t M, int64_t N, int64_t K, int64_t max_splits) 
 }
 
 // Small products (csrc/small_gemm.hip): out[b, m, n] = x[b, m, :] . w[b, n, :] of 2-D or 3-D operands, bf16 rows, out bf16 or fp32
-static void small_gemm(at::Tensor x, at::Tensor w, at::Tensor out, c10::optional<at::Tensor> bias) {
+static void small_gemm(at::Tensor x, at::Tensor w, at::Tensor out, c10::optional<at::Tensor> bias, c10::optional<at::Tensor> gate) {
   CHECK_CUDA(x); CHECK_DT(x, at::kBFloat16); CHECK_LASTDIM(x);
   CHECK_CUDA(w); CHECK_DT(w, at::kBFloat16); CHECK_LASTDIM(w);
   CHECK_CUDA(out); CHECK_LASTDIM(out);
@@ -823,10 +823,15 @@ static void small_gemm(at::Tensor x, at::Tensor w, at::Tensor out, c10::optional
     CHECK_DT(bias.value(), at::kFloat);
     TORCH_CHECK(bias->is_cuda() && bias->is_contiguous() && bias->numel() == N && f32, "small_gemm: bias [N] of an fp32 result");
   }
+  if (gate.has_value()) {   // [M, B N]: head b's columns b N ..
+    CHECK_CUDA(gate.value()); CHECK_DT(gate.value(), at::kBFloat16); CHECK_LASTDIM(gate.value());
+    TORCH_CHECK(gate->dim() == 2 && gate->size(0) == M && gate->size(1) == B * N && !f32 && !bias.has_value(), "small_gemm: gate [M, B N] of a bf16 result");
+  }
   CHECK_HIP(kafka_launch_small_gemm(bptr(x), bptr(w), (int)B, (int)M, (int)N, (int)K, d == 3 ? x.stride(0) : 0, x.stride(-2),
                                     d == 3 ? w.stride(0) : 0, w.stride(-2),
                                     bias.has_value() ? bias->data_ptr<float>() : nullptr, f32 ? 1 : 0, out.data_ptr(),
-                                    d == 3 ? out.stride(0) : 0, out.stride(-2), nullptr, nullptr, 0, 0, cur_stream()));
+                                    d == 3 ? out.stride(0) : 0, out.stride(-2), nullptr, gate.has_value() ? bptr(gate.value()) : nullptr,
+                                    gate.has_value() ? gate->stride(0) : 0, gate.has_value() ? N : 0, cur_stream()));
 }
 
 // out[m, n] = gelu(x[m, :] . w[n, :]) * emb[tokens[m], col0 + n] of bf16 rows, K from 1024 on; rows of unknown tokens are NaN
@@ -1392,7 +1397,8 @@ PYBIND11_MODULE(_kafka_ops, m) {
   m.def("tile_gemm", &tile_gemm, py::arg("x"), py::arg("wt"), py::arg("y"), py::arg("p"), py::arg("mt"), py::arg("nt"), py::arg("splits"),
         py::arg("glu"), py::arg("relu2") = false, py::arg("gelu") = false);
   m.def("small_gate", &small_gate);
-  m.def("small_gemm", &small_gemm, py::arg("x"), py::arg("w"), py::arg("out"), py::arg("bias") = c10::nullopt);
+  m.def("small_gemm", &small_gemm, py::arg("x"), py::arg("w"), py::arg("out"), py::arg("bias") = c10::nullopt,
+        py::arg("gate") = c10::nullopt);
   m.def("skinny_gemm", &skinny_gemm);
   m.def("wstream_gemm_cfg", &wstream_gemm_cfg);
   m.def("slab_reduce", &slab_reduce);

@@ -208,10 +208,11 @@ __global__ __launch_bounds__(NTH) void ln_shift_reg_kernel(const float* __restri
                                                            AT* __restrict__ out, int64_t os, int d,
                                                            const AT* __restrict__ mu, const int* __restrict__ tok_seg,
                                                            const int* __restrict__ seg, float* state,
-                                                           float* __restrict__ last) {
+                                                           float* __restrict__ last, const int64_t* __restrict__ idx, int64_t n_src) {
   __shared__ float red[NTH / 64];
-  const int64_t t = blockIdx.x;
-  const float* xr = x + t * xs;
+  const int64_t t = blockIdx.x, from = idx != nullptr ? idx[t] : t;
+  const bool in = from >= 0 && from < n_src;   // (a row outside comes out as NaN)
+  const float* xr = x + (in ? from : 0) * xs;
   bool first = true, is_last = false;
   int sg = 0, p0 = 0, slot = 0;
   if (mu != nullptr) {
@@ -242,6 +243,7 @@ __global__ __launch_bounds__(NTH) void ln_shift_reg_kernel(const float* __restri
   }
   float mean, rstd, mean2 = 0.f, rstd2 = 0.f;
   reg_stats<VEC, NTH, NV>(v, d, eps, red, mean, rstd);
+  if (!in) mean = __builtin_nanf("");
   if (mu != nullptr && !first) reg_stats<VEC, NTH, NV>(pv, d, eps, red, mean2, rstd2);  // (uniform per workgroup)
   float* keep = last != nullptr ? last + (int64_t)sg * d : state + (int64_t)slot * d;
 #pragma unroll
@@ -1515,17 +1517,20 @@ hipError_t kafka_hy_latent_decode(const void* q_lat, int64_t ql_h, int64_t ql_t,
 
 hipError_t kafka_hy_ln_shift(int f32, const float* x, int64_t xs, const void* w, const void* b, float eps, void* out,
                              int64_t os, int T, int d, const void* mu, const int* tok_seg, const int* seg,
-                             float* state, float* last, hipStream_t st) {
+                             float* state, float* last, const int64_t* idx, int64_t n_src, hipStream_t st) {
   if (T <= 0) return hipSuccess;
+  if (idx != nullptr && mu != nullptr) return hipErrorInvalidValue;
   DISPATCH_AT(f32, {
     const bool v4 = d % 4 == 0 && xs % 4 == 0 && os % 4 == 0 && al16(x) && al16(w) && al16(b) && al16(out) && al16(mu) &&
                     al16(state) && al16(last);
     if (!row_shape(T, d, v4, [&](auto V, auto N, auto K) {
           ln_shift_reg_kernel<AT, V.value, N.value, K.value><<<T, N.value, 0, st>>>(
-              x, xs, (const AT*)w, (const AT*)b, eps, (AT*)out, os, d, (const AT*)mu, tok_seg, seg, state, last);
-        }))
+              x, xs, (const AT*)w, (const AT*)b, eps, (AT*)out, os, d, (const AT*)mu, tok_seg, seg, state, last, idx, idx != nullptr ? n_src : T);
+        })) {
+      if (idx != nullptr) return hipErrorInvalidValue;
       ln_shift_kernel<AT><<<T, NT, 0, st>>>(x, xs, (const AT*)w, (const AT*)b, eps, (AT*)out, os, d, (const AT*)mu, tok_seg,
                                             seg, state, last);
+    }
   });
   return hipGetLastError();
 }
@@ -1620,7 +1625,7 @@ hipError_t kafka_hy_side_dwa_ln(int f32, float* x, const void* y, int64_t ys, co
   });
   if (done) return hipGetLastError();
   const hipError_t e = kafka_hy_side_dwa(f32, x, y, ys, sw, eps, stack, layer, dwa, T, d, st);
-  return e != hipSuccess ? e : kafka_hy_ln_shift(f32, x, d, w, b, eps2, out, os, (int)T, d, mu, tok_seg, seg, state, nullptr, st);
+  return e != hipSuccess ? e : kafka_hy_ln_shift(f32, x, d, w, b, eps2, out, os, (int)T, d, mu, tok_seg, seg, state, nullptr, nullptr, 0, st);
 }
 
 hipError_t kafka_hy_latent_prep(int f32, const void* qgd, int64_t qs, int T, int H, int dim, int rd, int R, int dkv_off,

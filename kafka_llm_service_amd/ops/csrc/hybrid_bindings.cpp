@@ -7,7 +7,7 @@
 extern "C" {
 hipError_t kafka_hy_ln_shift(int f32, const float* x, int64_t xs, const void* w, const void* b, float eps, void* out,
                              int64_t os, int T, int d, const void* mu, const int* tok_seg, const int* seg,
-                             float* state, float* last, hipStream_t st);
+                             float* state, float* last, const int64_t* idx, int64_t n_src, hipStream_t st);
 hipError_t kafka_hy_scatter_rows(float* dst, const int* seg, const float* src, int R, int d, hipStream_t st);
 hipError_t kafka_hy_add_ln(int f32, float* x, int64_t xs, const void* y, int64_t ys, int S, int64_t slab, const void* w, const void* b,
                            float eps, int T, int d, void* out2, int64_t os, const void* w2, const void* b2,
@@ -240,14 +240,16 @@ void segs(const at::Tensor& tok_seg, const at::Tensor& seg, int64_t T) {
 }
 
 void ln_shift(at::Tensor x, at::Tensor w, at::Tensor b, double eps, at::Tensor out, OptT mu, OptT tok_seg, OptT seg,
-              OptT state, OptT last) {
+              OptT state, OptT last, OptT rows) {
   rows2d(x, "x"); rows2d(out, "out");
   TORCH_CHECK(x.scalar_type() == at::kFloat, "ln_shift: x is the fp32 stream");
   const int f32 = act_f32(out);
-  const int64_t T = x.size(0), d = x.size(1);
+  const int64_t T = rows.has_value() ? rows->numel() : x.size(0), d = x.size(1);
   same_act(f32, {&w, &b});
   vec(w, d, "w"); vec(b, d, "b");
   TORCH_CHECK(out.size(0) == T && out.size(1) == d, "ln_shift: out shape");
+  TORCH_CHECK(!rows.has_value() || (rows->is_cuda() && rows->scalar_type() == at::kLong && rows->dim() == 1 && rows->is_contiguous() &&
+                                    x.size(0) > 0 && d <= 4096 && !mu.has_value()), "ln_shift: picked rows, int64, without a shift");
   const void* mup = nullptr; const int *tsp = nullptr, *sgp = nullptr; float *stp = nullptr, *lp = nullptr;
   if (mu.has_value()) {
     TORCH_CHECK(tok_seg.has_value() && seg.has_value() && state.has_value(), "ln_shift: a shift needs tok_seg, seg and state");
@@ -262,7 +264,8 @@ void ln_shift(at::Tensor x, at::Tensor w, at::Tensor b, double eps, at::Tensor o
     stp = state->data_ptr<float>(); lp = last.has_value() ? last->data_ptr<float>() : nullptr;
   }
   HY_HIP(kafka_hy_ln_shift(f32, x.data_ptr<float>(), x.stride(0), w.data_ptr(), b.data_ptr(), (float)eps,
-                           out.data_ptr(), out.stride(0), (int)T, (int)d, mup, tsp, sgp, stp, lp, stream()));
+                           out.data_ptr(), out.stride(0), (int)T, (int)d, mup, tsp, sgp, stp, lp,
+                           rows.has_value() ? rows->data_ptr<int64_t>() : nullptr, x.size(0), stream()));
 }
 
 void scatter_rows(at::Tensor dst, at::Tensor seg, at::Tensor src) {
@@ -1427,7 +1430,7 @@ void kafka_bind_hybrid(pybind11::module_& m) {
   namespace py = pybind11;
   m.def("hy_ln_shift", &ln_shift, py::arg("x"), py::arg("w"), py::arg("b"), py::arg("eps"), py::arg("out"),
         py::arg("mu") = py::none(), py::arg("tok_seg") = py::none(), py::arg("seg") = py::none(),
-        py::arg("state") = py::none(), py::arg("last") = py::none());
+        py::arg("state") = py::none(), py::arg("last") = py::none(), py::arg("rows") = py::none());
   m.def("hy_scatter_rows", &scatter_rows);
   m.def("hy_add_ln", &add_ln, py::arg("x"), py::arg("y"), py::arg("w"), py::arg("b"), py::arg("eps"),
         py::arg("out2") = py::none(), py::arg("w2") = py::none(), py::arg("b2") = py::none());

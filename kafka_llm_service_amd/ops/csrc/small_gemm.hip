@@ -20,7 +20,9 @@ typedef __attribute__((address_space(3))) void lds_t;
 struct Strides {
   int64_t xb, xm, wb, wn, yb, ym;
 };
-// what a gate product's rows are multiplied with: gelu(sum) * emb[tok[m]][n] (rows outside the table: NaN)
+// what a product's rows meet. GELU_GATE: gelu(sum) * emb[tok[m]][n] (rows outside the table: NaN). SIGMOID_GATE: the sum as bf16, times
+// sigmoid(emb[m][b * rows + n]), head b's part of a row of gates (a launch of its own: 4.0 us of 64 rows of 32 heads of 128).
+enum { NO_GATE, GELU_GATE, SIGMOID_GATE };
 struct Gate {
   const int64_t* tok;
   const bf16* emb;
@@ -29,7 +31,7 @@ struct Gate {
 
 // A wave: 16 rows x 16 NT columns over its share of K. KW waves of a workgroup share K (their sums meet in LDS), the other
 // 4 / KW (KW up to 4) take further columns. Products are taken with the weights first: a lane holds four columns of one row.
-template <int NT, int KW, bool F32, bool GATE = false>
+template <int NT, int KW, bool F32, int GATE = NO_GATE>
 __global__ __launch_bounds__(64 * (KW > 4 ? KW : 4)) void small_gemm_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W,
                                                                             int M, int N, int K, const float* __restrict__ bias,
                                                                             void* __restrict__ Y, Strides st, Gate gate) {
@@ -115,7 +117,7 @@ __global__ __launch_bounds__(64 * (KW > 4 ? KW : 4)) void small_gemm_kernel(cons
   }
   const int m = m0 + r;
   if (m >= M) return;
-  const int64_t tok = GATE ? gate.tok[m] : 0;
+  const int64_t tok = GATE == GELU_GATE ? gate.tok[m] : 0;
   const bool known = tok >= 0 && tok < gate.rows;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
@@ -126,10 +128,13 @@ __global__ __launch_bounds__(64 * (KW > 4 ? KW : 4)) void small_gemm_kernel(cons
       if (bias) acc[t] += *reinterpret_cast<const f32x4v*>(bias + n);
       *reinterpret_cast<f32x4v*>(reinterpret_cast<float*>(Y) + at) = acc[t];
     } else {
-      bf16x4 o;
+      bf16x4 o, g;
+      if constexpr (GATE == SIGMOID_GATE) g = *reinterpret_cast<const bf16x4*>(gate.emb + m * gate.stride + b * gate.rows + n);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        if constexpr (GATE)
+        if constexpr (GATE == SIGMOID_GATE)
+          o[i] = (bf16)((float)(bf16)acc[t][i] * (1.0f / (1.0f + expf(-(float)g[i]))));
+        else if constexpr (GATE == GELU_GATE)
           o[i] = known ? (bf16)(gate_act(acc[t][i], true) * (float)gate.emb[tok * gate.stride + n + i]) : (bf16)__builtin_nanf("");
         else
           o[i] = (bf16)acc[t][i];
@@ -143,7 +148,10 @@ extern "C" hipError_t kafka_launch_small_gemm(const bf16* X, const bf16* W, int 
                                               int64_t wb, int64_t wn, const float* bias, int f32, void* Y, int64_t yb, int64_t ym,
                                               const int64_t* tok, const bf16* emb, int64_t emb_stride, int64_t emb_rows,
                                               hipStream_t st) {
+  // tok: a gelu gate; emb alone: a sigmoid gate of rows emb_stride apart, a head's part emb_rows wide
   const Gate gate{tok, emb, emb_stride, emb_rows};
+  const bool sig = tok == nullptr && emb != nullptr;
+  if (sig && (f32 || bias || emb_stride % 4 || emb_rows % 4 || reinterpret_cast<uintptr_t>(emb) % 8)) return hipErrorInvalidValue;
   if (tok != nullptr && (f32 || bias || B != 1 || K < 1024)) return hipErrorInvalidValue;
   if (B < 1 || M < 1 || N < 1) return hipSuccess;
   const uintptr_t ya = reinterpret_cast<uintptr_t>(Y);
@@ -164,8 +172,12 @@ extern "C" hipError_t kafka_launch_small_gemm(const bf16* X, const bf16* W, int 
   // launch / 16 columns / 32: K = 4096 21.6 / 11.0 / 8.9, 2048 11.5 / 7.9 / 6.6; 3000 rows (two rounds)
   // of K = 4096 18.5, 17.1 on 32 columns, of 2048 11.8, 12.1.
   if (tok != nullptr)
-    return N > 32 && (int64_t)rows * ((N + 15) / 16) > 256 ? go(small_gemm_kernel<2, 16, false, true>, 2, 16)
-                                                           : go(small_gemm_kernel<1, 16, false, true>, 1, 16);
+    return N > 32 && (int64_t)rows * ((N + 15) / 16) > 256 ? go(small_gemm_kernel<2, 16, false, GELU_GATE>, 2, 16)
+                                                           : go(small_gemm_kernel<1, 16, false, GELU_GATE>, 1, 16);
+  if (sig)
+    return K >= 1024  ? go(small_gemm_kernel<1, 16, false, SIGMOID_GATE>, 1, 16)
+           : K >= 256 ? go(small_gemm_kernel<2, 4, false, SIGMOID_GATE>, 2, 4)
+                      : go(small_gemm_kernel<4, 1, false, SIGMOID_GATE>, 4, 1);
   if (K >= 1024) return f32 ? go(small_gemm_kernel<1, 16, true>, 1, 16) : go(small_gemm_kernel<1, 16, false>, 1, 16);
   if (K >= 256) return f32 ? go(small_gemm_kernel<2, 4, true>, 2, 4) : go(small_gemm_kernel<2, 4, false>, 2, 4);
   return f32 ? go(small_gemm_kernel<4, 1, true>, 4, 1) : go(small_gemm_kernel<4, 1, false>, 4, 1);

@@ -72,3 +72,20 @@ def test_rows_gathered_twice(dev, d):
                  torch.empty(5, 2 * d, device=dev, dtype=torch.bfloat16)[:, d:], torch.empty(5, d + 3, device=dev)[:, 3:],
                  torch.empty(5, d, device=dev, dtype=torch.float16)):
         assert torch.equal(ops.gather_rows(table, idx, also), table[idx]) and torch.equal(also, table[idx].to(also.dtype))
+
+
+@pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d", [8, 100, 1000, 4096, 5000])
+def test_layer_norm_of_picked_rows(dev, dtype, d):
+    """As of the rows picked before, to the last bit, for every row length's kernel and those without one."""
+    from kafka_llm_service_amd.ops import hybrid as hops
+
+    g = torch.Generator().manual_seed(d)
+    x = torch.randn(40, d, generator=g).to(dev)
+    w, b = (torch.randn(d, generator=g).to(dtype).to(dev) for _ in range(2))
+    for idx in (torch.tensor([39]), torch.randint(0, 40, (25,), generator=g), torch.randint(0, 40, (600,), generator=g)):
+        got, want = (torch.empty(len(idx), d, dtype=dtype, device=dev) for _ in range(2))
+        hops.ln_rows(x, idx.to(dev), w, b, 1e-6, got)
+        hops.ln_shift(x.index_select(0, idx.to(dev)), w, b, 1e-6, want)
+        assert torch.equal(got, want)

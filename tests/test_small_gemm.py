@@ -184,3 +184,25 @@ def test_gate_of_long_steps(M, N, K):
     e = emb[tok[known], N:2 * N].double()
     want = torch.nn.functional.gelu(z, approximate="tanh") * e
     assert ((got[known] - want).abs() <= 2 ** -8 * want.abs() + 1.13 * K * 2.0 ** -24 * mag * e.abs() + 1e-5 * e.abs()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [64, 120, 512, 1024])
+@pytest.mark.parametrize("M,N", [(1, 128), (17, 36), (64, 128), (65, 64)])
+def test_heads_with_a_sigmoid_gate(K, M, N):
+    """The gate in the product's epilogue is the product and the gate's launch, to the last bit; a gate that the kernel does not read goes the
+    other way."""
+    H, g = 3, torch.Generator().manual_seed(K + M)
+    x, w = (torch.randn(H, n, K, generator=g).to(torch.bfloat16).cuda() for n in (M, N))
+    wt = w.transpose(1, 2).contiguous()
+    wide = (4 * torch.randn(M, 8 + H * N + 1, generator=g)).to(torch.bfloat16).cuda()
+    wide[0, 9:11] = torch.tensor([float("inf"), -float("inf")])
+    for gate in (wide[:, 8:8 + H * N].contiguous(), torch.nn.functional.pad(wide, (0, -(8 + H * N + 1) % 4))[:, 8:8 + H * N], wide[:, 9:]):
+        want = torch.empty(M, H * N, dtype=torch.bfloat16, device="cuda")
+        hops.sigmoid_mul(head_product(x, w, wt), gate, want)
+        got = torch.full_like(want, float("nan"))
+        head_product(x, w, wt, got.view(M, H, N).transpose(0, 1), gate)
+        if gate.stride(0) % 4 == 0 and gate.data_ptr() % 8 == 0:
+            assert torch.equal(got, want)
+        else:   # (the library's sums in another order: a bf16 step of the product)
+            assert (got.float() - want.float()).norm() < 2e-3 * want.float().norm()

@@ -467,8 +467,8 @@ _NP2TORCH = {np.dtype(np.int64): torch.int64, np.dtype(np.int32): torch.int32, n
 class _Stager:
     """Per-step host->device uploads through a ring of pinned staging arenas (one arena per launch, bump-allocated):
     no pinned allocation and no pageable copy on the step path, so every upload runs in stream order without the host
-    (a kernel that reads the arena, a copy engine for large ones: ``ops.host_copy``). An arena is reused ``depth`` launches later, when at most two steps can be in flight — its copies have
-    executed by then."""
+    (a kernel that reads the arena, a copy engine for large ones: ``ops.host_copy``). An arena is reused ``depth``
+    launches later, when at most two steps can be in flight — its copies have executed by then."""
 
     def __init__(self, device: torch.device, nbytes: int = 8 << 20, depth: int = 4):
         self.device = device

@@ -163,17 +163,20 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// 1 / (1 + e^-s): the hardware's exponential and reciprocal (1 ulp each), the exponent's rounding error given back in a product. A quotient behind
-// an exponential of a rounded argument takes a quarter longer (2048 rows of 4096 -> 28672 with silu * up 366 us, so 358) and is further off: g / (1 + e^-g)
-// over -90 .. 90 within 3.7e-6 of 64 bits, rms 6.0e-7, where this one is within 2.5e-7, rms 4.3e-8. Past |s| = 88 as at 88, where the result is 1, or 0 for normal numbers.
-__device__ __forceinline__ float sigmoid_of(float s) {
-  const float x = __builtin_amdgcn_fmed3f(-s, -88.f, 88.f), t = x * 1.44269504f;
-  const float lo = fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269504f, -t)), p = __builtin_amdgcn_exp2f(t);
-  return __builtin_amdgcn_rcpf(1.0f + fmaf(p, 0.69314718f * lo, p));
+// g / (1 + e^-s): the hardware's exponential and reciprocal (1 ulp each), the exponent's rounding error given back in a product. A
+// quotient behind an exponential of a rounded argument takes a quarter longer (2048 rows of 4096 -> 28672 with silu * up 366 us, so 358)
+// and is further off. Relative error of s = g against 64 bits, at most / rms, quotient and so: -88.72 .. -10 3.9e-6 / 1.4e-6 and
+// 2.2e-7 / 5.2e-8, -10 .. 10 5.4e-7 / 1.2e-7 and 2.0e-7 / 5.0e-8, 10 .. 90 1.1e-7 / 1.3e-8 both. The denominator is a quarter of itself,
+// so that its reciprocal is a normal number as far as e^-s is one. From s = -88.7228394 down, where the exponent rounds to 128 and its error is
+// not negative, the exponential is infinite and the result 0 (less than 3e-37 off for s = g; not a number for g = -infinity).
+__device__ __forceinline__ float times_sigmoid(float g, float s) {
+  const float x = __builtin_amdgcn_fmed3f(-s, -88.f, 88.7228394f), t = x * 1.44269504f;
+  const float lo = fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269504f, -t)), p = 0.25f * __builtin_amdgcn_exp2f(t);
+  return 0.25f * g * __builtin_amdgcn_rcpf(0.25f + fmaf(p, 0.69314718f * lo, p));
 }
 // act(g) = g / (1 + e^-s) of the gated feed-forwards: s = g (SiLU), or with gelu that of the tanh form of GELU
 __device__ __forceinline__ float gate_act(float g, bool gelu) {
-  return g * sigmoid_of(gelu ? 1.5957691216057308f * (g + 0.044715f * g * g * g) : g);
+  return times_sigmoid(g, gelu ? 1.5957691216057308f * (g + 0.044715f * g * g * g) : g);
 }
 
 // Counter-based RNG (splitmix64 finaliser): deterministic given (seed, stream, index).

@@ -191,7 +191,7 @@ __global__ __launch_bounds__(256, 2) void grouped_wide_kernel(const bf16* __rest
           u = fminf(fmaxf(u, -glu_limit), glu_limit) + 1.0f;
           al = glu_alpha;
         }
-        Y[(int64_t)ent * ldy + (nb >> 1) * 32 + r] = (bf16)(g * sigmoid_of(al * g) * u);
+        Y[(int64_t)ent * ldy + (nb >> 1) * 32 + r] = (bf16)(times_sigmoid(g, al * g) * u);
       }
     }
 }
@@ -279,7 +279,7 @@ __device__ __forceinline__ void ring_tile(const RingArgs& A, char* smem, int e, 
           u = fminf(fmaxf(u, -A.glu_limit), A.glu_limit) + 1.0f;
           al = A.glu_alpha;
         }
-        return g * sigmoid_of(al * g) * u;
+        return times_sigmoid(g, al * g) * u;
       }
     };
     R::template rows_bf16<EPI == EPI_GLU ? 2 : 4>(y, A.ldy, rows, tiles, lane, w, value);

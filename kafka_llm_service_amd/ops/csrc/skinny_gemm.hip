@@ -147,7 +147,7 @@ __global__ __launch_bounds__(512, OCC) void skinny_gemm_kernel(const bf16* __res
         const int m = 64 * rg + 32 * a + (i & 3) + 8 * (i >> 2) + 4 * h;
         if (m < M) {
           const float g = acc[a][0][i], u = acc[a][1][i];
-          Y[(int64_t)m * ldy + n] = (bf16)(g * sigmoid_of(g) * u);
+          Y[(int64_t)m * ldy + n] = (bf16)(times_sigmoid(g, g) * u);
         }
       }
     return;

@@ -820,7 +820,7 @@ __global__ __launch_bounds__(256, MT == 4 ? 2 : 1) void wstream_grouped_kernel(c
             u = fminf(fmaxf(u, -glu_limit), glu_limit) + 1.0f;
             a = glu_alpha;
           }
-          Y[(int64_t)(seg0 + row0 + m) * ldy + n] = (bf16)(g * sigmoid_of(a * g) * u);
+          Y[(int64_t)(seg0 + row0 + m) * ldy + n] = (bf16)(times_sigmoid(g, a * g) * u);
         }
       }
   } else {

@@ -204,3 +204,39 @@ def test_low_last_row_tiles_and_short_loops(mt, nt):
         assert (y[M:] == 7).all()
         if s > 1:
             assert ((ops.linear_tile(x, wt, (mt, nt, s)).sum(0) - want).abs() <= 1e-4).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["silu", "gelu"])
+def test_gates_against_64_bits(act):
+    """Gates over all that the exponential has normal numbers for, and far past it on both sides, of the element-wise launch and of the products' epilogues
+    (each sum is one term, so exact). The result is bf16 (8 bits: half a unit is up to 2^-8 of it), the gate's fp32 error at most 88 times a few 2^-24 (the
+    argument of the gelu form); beyond s = -88.7 the result may be 0, as may what is not a normal number."""
+    v = torch.arange(-90, 90.25, 0.25)
+    v = torch.cat([v, v / 8, torch.tensor([-3e38, -1e30, -1e4, -100.0, -10.06, 100.0, 1e4, 3e38, -0.0])]).to(torch.bfloat16)
+    g = v.double()
+    s = g if act == "silu" else 1.5957691216057308 * (g + 0.044715 * g ** 3)
+    want = torch.where(s < -700, torch.zeros_like(g), g / (1 + torch.exp(-s.clamp(min=-700))))
+    bound = (2 ** -8 + 2 ** -15) * want.abs() + torch.where((s < -88.7) & (s > -700), g.abs() * 3e-39, torch.zeros_like(g)) + 1.2e-38
+
+    def check(y):
+        off = (y.cpu().double() - want).abs() > bound
+        assert not off.any(), (g[off], want[off], y.cpu()[off])
+
+    n = len(v)
+    x = torch.ones(n, 16, dtype=torch.bfloat16)
+    x[:, :8] = v[:, None]
+    check(ops.silu_mul(x.cuda(), act=act)[:, 3])
+    check(ops.silu_mul(x.float().cuda().view(1, n, 16), act=act)[:, 3])
+    edge = torch.tensor([[float("inf")] * 8 + [1.0] * 8, [-float("inf")] * 8 + [1.0] * 8, [float("nan")] * 8 + [1.0] * 8]).to(torch.bfloat16).cuda()
+    y = ops.silu_mul(edge, act=act)
+    assert (y[0] == float("inf")).all() and y[1:].isnan().all()
+    K, F = 256, 128
+    w, x = torch.zeros(2 * F, K), torch.zeros(n, K, dtype=torch.bfloat16)
+    w[:F, 0] = w[F:, 1] = 1
+    x[:, 0], x[:, 1] = v, 1
+    wt, x = ops.tile_weight(w.to(torch.bfloat16).cuda(), glu=True), x.cuda()
+    for mt, nt in ((4, 4), (8, 8)):
+        check(ops.linear_tile(x, wt, (mt, nt, 1), glu=True, act=act)[:, 5])
+    rows = ops.STREAM_MAX_M
+    check(torch.cat([ops.linear_glu(x[i:i + rows], wt, 1, act=act) for i in range(0, n, rows)])[:, 5])

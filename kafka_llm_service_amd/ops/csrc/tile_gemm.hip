@@ -82,11 +82,13 @@ __device__ __forceinline__ void tile(const TileArgs& A, char* smem, int sp, int 
 }
 
 // A last row tile of at most LOW rows is one of that height: its weights' way is then what it takes, a third of a whole tile. The whole tiles are
-// dealt out first, evenly, then those. us, before / now: 4099 rows of 4096 -> 28672 698 / 669, of 4096 -> 4096 152 / 112, of 14336 -> 4096 504 / 376;
-// 2060 rows of 4096 -> 4096 on 256 x 128 87 / 65. (One row tile alone, WNT, has a height that fits; tiles of 128 rows are low enough.)
+// dealt out first, evenly, then those, to each XCD what it has fewer of the others. us, before / now: 4099 rows of 4096 -> 28672 698 / 669,
+// of 4096 -> 4096 152 / 112, of 14336 -> 4096 504 / 376; 2060 rows of 4096 -> 4096 on 256 x 128 87 / 65. (Dealt out evenly by themselves, an XCD
+// had 65 tiles for its 64 places in two rounds: 1024 rows of 4096 -> 18560 on 160 x 256 142, so 129.) One row tile alone, WNT, has a height
+// that fits; tiles of 128 rows are low enough.
 constexpr int LOW = 64;
 template <int MT>
-__host__ __device__ constexpr int low_rows(int M) {
+__device__ constexpr int low_rows(int M) {
   return MT > 4 && M > 32 * MT && M % (32 * MT) <= LOW ? M % (32 * MT) : 0;
 }
 
@@ -101,17 +103,17 @@ __global__ __launch_bounds__(256, OCC) void tile_gemm_kernel(const TileArgs A) {
   // side by side, then the next column tile, so that its weights leave memory once
   const int low = HAS_LOW ? low_rows<MT>(A.M) : 0, rts = low ? A.M / R::BM : (A.M + R::BM - 1) / R::BM;
   const int nts = (A.N + R::BN - 1) / R::BN, tiles = rts * nts, total = tiles * A.S;
-  const int per = (total + 7) >> 3, k8 = blockIdx.x >> 3, x8 = blockIdx.x & 7;
-  if (k8 < per) {
+  const int all = low ? nts * A.S : 0, per = (total + 7) >> 3, both = (total + all + 7) >> 3;   // low tiles; of an XCD: whole tiles, tiles
+  const int k8 = blockIdx.x >> 3, x8 = blockIdx.x & 7, whole = max(0, min(per, total - x8 * per));
+  if (k8 < whole) {                                  // (uniform)
     const int item = x8 * per + k8;
-    if (item >= total) return;                       // (uniform)
     constexpr int GR = 2048 / R::BM;
     const int sp = item / tiles, it = item - sp * tiles, g = it / (GR * nts), j = it - g * GR * nts, in_g = min(GR, rts - g * GR);
     const int nt = j / in_g, row0 = (g * GR + j - nt * in_g) * R::BM;
     tile<MT, NT, OCC, WNT>(A, smem, sp, nt, row0, min(R::BM, A.M - row0));
   } else if constexpr (HAS_LOW) {
-    const int all = nts * A.S, lper = (all + 7) >> 3, item = x8 * lper + k8 - per;
-    if (!low || k8 - per >= lper || item >= all) return;
+    const int item = x8 * both - min(x8 * per, total) + k8 - whole;
+    if (k8 >= both || item >= all) return;
     tile<LOW / 32, NT, OCC, WNT>(A, smem, item / nts, item % nts, rts * R::BM, low);
   }
 }
@@ -132,14 +134,14 @@ extern "C" hipError_t kafka_launch_tile_gemm(const bf16* X, int64_t ldx, const b
   const TileArgs A{X, ldx, reinterpret_cast<const bf16x8*>(Wt), M, N, K, splits, Y, ldy, P, mode};
   const int64_t nts = (int64_t)((N + 32 * nt - 1) / (32 * nt)) * splits;
   if ((M + 32 * mt - 1) / (32 * mt) * nts > 0x0fffffff) return hipErrorInvalidValue;
-  auto a = [&](auto kern, int low) {
-    const int64_t total = (low ? M / (32 * mt) : (M + 32 * mt - 1) / (32 * mt)) * nts;
-    kern<<<(unsigned)((total + 7) / 8 * 8 + (low ? (nts + 7) / 8 * 8 : 0)), 256, 0, st>>>(A);
+  auto a = [&](auto kern) {
+    const int64_t total = (M + 32 * mt - 1) / (32 * mt) * nts;   // (the low tiles among them)
+    kern<<<(unsigned)((total + 7) / 8 * 8), 256, 0, st>>>(A);
   };
 #define TILE(MT, NT, OCC)                                        \
   if (mt == MT && nt == NT) {                                    \
-    if (M <= 32 * MT) a(tile_gemm_kernel<MT, NT, OCC, true>, 0); \
-    else a(tile_gemm_kernel<MT, NT, OCC, false>, low_rows<MT>(M)); \
+    if (M <= 32 * MT) a(tile_gemm_kernel<MT, NT, OCC, true>);    \
+    else a(tile_gemm_kernel<MT, NT, OCC, false>);                \
     return hipGetLastError();                                    \
   }
   TILE(8, 8, 1)

@@ -138,6 +138,16 @@ extern "C" hipError_t kafka_launch_tile_gemm(const bf16* X, int64_t ldx, const b
     const int64_t total = (M + 32 * mt - 1) / (32 * mt) * nts;   // (the low tiles among them)
     kern<<<(unsigned)((total + 7) / 8 * 8), 256, 0, st>>>(A);
   };
+  // 128 x 128: two workgroups share a CU and its LDS, with two units of activations and three of weights each. Where each has a CU to itself five of
+  // both fit, which long loops without splits on 96 workgroups and more are the faster for (us, sharing / alone: 96 - 256 workgroups of K = 2048 17.4 - 19.6 /
+  // 14.9 - 17.9, of 7168 57 / 48, 1000 rows of 4096 -> 4096 37.0 / 35.9); 64 - 72 of them take 13.8 / 14.3, and short loops wait for all that is asked
+  // for in front of them (splits of 512 10.8 - 14 / 11.7 - 15, of 896 - 1024 16.4 - 19 / 17.1 - 20, of 3584 as long).
+  const int64_t wgs = (M + 127) / 128 * nts;
+  if (mt == 4 && nt == 4 && splits == 1 && K >= 2048 && wgs >= 96 && wgs <= 256) {
+    if (M <= 128) a(tile_gemm_kernel<4, 4, 1, true>);
+    else a(tile_gemm_kernel<4, 4, 1, false>);
+    return hipGetLastError();
+  }
 #define TILE(MT, NT, OCC)                                        \
   if (mt == MT && nt == NT) {                                    \
     if (M <= 32 * MT) a(tile_gemm_kernel<MT, NT, OCC, true>);    \

@@ -240,3 +240,17 @@ def test_gates_against_64_bits(act):
         check(ops.linear_tile(x, wt, (mt, nt, 1), glu=True, act=act)[:, 5])
     rows = ops.STREAM_MAX_M
     check(torch.cat([ops.linear_glu(x[i:i + rows], wt, 1, act=act) for i in range(0, n, rows)])[:, 5])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(128, 96 * 128, 2048), (97, 128 * 128 - 32, 2112), (130, 48 * 128, 2048), (257, 85 * 128, 2176), (300, 32 * 128 - 64, 2048),
+                                   (2048, 16 * 128, 2048), (129, 128 * 128, 2368), (2049, 16 * 128, 2048), (257, 31 * 128, 2048), (500, 24 * 128, 1984)])
+def test_small_tiles_alone_on_a_cu(M, N, K):
+    """128 x 128 tiles by themselves on a CU and, beyond the rule's lines, two to a CU: one row tile, ragged rows and columns, odd numbers of units."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16).cuda()
+    y = torch.full((M + 30, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    ops.ext().tile_gemm(x, ops.tile_weight(w), y[:M], None, 4, 4, 1, False)
+    _close(y[:M], x.float() @ w.float().t(), K)
+    assert (y[M:] == 7).all()

@@ -431,11 +431,11 @@ def linear_small(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 # (16-row parts, 16-column parts) of a wave's tile, 2 x 2 waves a workgroup -> us: of a launch, of a round of 256 workgroups, of 64 of K
 # in it, and of a MB/us of what is written, over 4.5; then the same of steps of up to 256 rows, where one row tile's weights pass the caches by. Fitted to
 # 17197 timings (17 shapes of width 2048 and 4096, 129 - 4099 rows, every tile, one to eight splits; weights from memory), then to the choice that they
-# make: the tile and split that the figures pick take 1.0 % (slabs) and 1.7 % (bf16) longer than the best on average (1.8 and 2.4 by the figures
-# of the loop before; 222 rows of 14336 -> 4096 41 -> 36.5 us).
+# make: the tile and split that the figures pick took 1.0 % (slabs) and 1.7 % (bf16) longer than the best on average (1.8 and 2.4 by the figures
+# of the loop before; 222 rows of 14336 -> 4096 41 -> 36.5 us), TILE_DEEP and 256 x 192 (0.974 before) corrected since.
 TILES = {
     (8, 8): ((0.6, 0.0, 1.19, 1.06), (2.1, 5.0, 1.00, 0.92)),
-    (8, 6): ((1.0, 2.5, 0.974, 0.79), (3.5, 2.2, 0.876, 0.90)),
+    (8, 6): ((1.0, 2.5, 0.985, 0.79), (3.5, 2.2, 0.876, 0.90)),
     (7, 8): ((0.8, 0.8, 1.08, 1.01), (3.8, 1.9, 0.954, 1.01)),
     (6, 8): ((0.6, 0.8, 0.951, 1.02), (4.4, 0.0, 0.845, 1.21)),
     (7, 6): ((0.4, 2.2, 0.877, 0.95), (3.3, 2.0, 0.800, 0.98)),
@@ -450,6 +450,9 @@ TILES = {
 }
 # rows up to which the last row tile is a low one (tiles of more than 128 rows), and us of a round of those and 64 of K by the 16-column parts
 TILE_LOW, TILE_LOW_UNIT = 64, {8: 0.43, 6: 0.26, 4: 0.21}
+# what loops of 6144 and more of K take longer on tiles of 128 columns: us, without / with two splits on 256: 14336 -> 4096 1100 rows 135 / 112, 1770 164 / 153
+# (a third as deep, 4096 -> 4096, 1100 rows 41 / 43, 1770 50 / 60)
+TILE_DEEP = 1.04
 TILE_SPLITS = (1, 2, 4, 8)      # what the consumers of slabs load with all slabs in flight
 TILE_SLAB_BYTES = 1 << 28
 TILE_LIBRARY_N, TILE_MAX_M = 24576, 2560
@@ -471,9 +474,10 @@ def _tile_search(M: int, N: int, K: int, form: str, odd: int) -> tuple[float, tu
             if K // 64 < 2 * s or s > 1 and (form == "relu2" or 4 * s * M * N > TILE_SLAB_BYTES):
                 break
             mb = M * N / 4.5e6
+            depth = K // 64 / s * (TILE_DEEP if nt == 4 and K // 64 >= 96 * s else 1)
             rounds = -(-items * s // 256)
             more = -(-max(0, cols * s - (256 * rounds - items * s)) // 256) if low else 0   # rounds of low tiles past the last whole one
-            t = launch + (rounds + more) * rnd + (rounds * unit + more * TILE_LOW_UNIT[nt]) * (K // 64) / s + out * mb * (4 * s if s > 1 else 2)
+            t = launch + (rounds + more) * rnd + (rounds * unit + more * TILE_LOW_UNIT[nt]) * depth + out * mb * (4 * s if s > 1 else 2)
             if s > 1:               # the slabs' way back in, beside that of a bf16 output; a launch of its own but for "slabs"
                 t += mb * (4 * s - 2) if form == "slabs" else 6 + mb * (4 * s + 2)
             if best is None or t < best[0]:
@@ -497,21 +501,19 @@ def tile_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) 
     the library is as fast. ``form``: "slabs" (the consumer sums the split-K slabs as it loads them), "bf16" (slabs go
     through slab_reduce, a launch), "glu" (silu(gate) * up, in the epilogue or from slabs) or "relu2" (relu squared, in the epilogue). ``library``: there is a row-major weight for it.
 
-    Against the library (us, library / this kernel): 450 rows of 14336 -> 4096 89 / 55, 2048 rows 202 / 178; 2048 rows of 4096 -> 18560 350 / 277,
-    200 rows 57 / 45; 900 rows of 2048 -> 9344 45 / 36; 450 rows of 2048 -> 2048 19 / 11; over all timed shapes 13 % less time with slabs,
-    9 % as bf16. The library's: very wide outputs of 257 - 1024 rows (28672 columns: 320 rows 74 / 78, 640 135 / 149); beyond
-    768, where its 256 x 256 tiles (1.42 us a round and 64 of K) fill their rounds: past one round whole columns (multiples of 256) take this
-    kernel only where the model says a fifth less (28672: 1536 rows 264 / 293, with the activation 272 / 304, 900 rows 189 / 198, 4099 722 / 774; 14336:
-    1903 rows 162 / 190; where the model says a fifth to a twentieth less, 11 % more over 20 sizes), ragged ones mostly (10816: 2048 rows
-    164 / 151).
+    The lines against the library were drawn with the loop before (two meetings of the waves per 64 of K); what they leave to it past one
+    round of its tiles ``long_plan``, which the callers ask, looks at again. us, library (and activation) / this kernel as it is now, from
+    captured launches with weights from memory: 450 rows of 14336 -> 4096 88 / 60, 2048 rows 205 / 178; 900 rows of 2048 -> 9344 41 / 34,
+    2048 83 / 70; 256 rows of 4096 -> 18560 58 / 51, 2048 335 / 250; 450 rows of 4096 -> 4096 27 / 26, 2048 61 / 57. Few rows of few columns
+    are the library's better sizes: 2048 -> 2048 450 rows 11 / 14, 900 15 / 16.
 
-    Beyond 2560 rows the library's choice of kernel decides. Where its tiles are one round or less it is as fast or faster (4096 -> 4096: 2716 rows
-    73 / 74, 4096 91 / 100). Beyond a round ragged columns take this kernel (4096 -> 18560: 3182 rows 500 / 378, 4096 560 / 461; 12320: 2593 333 /
-    221, 7583 538 / 576; 2048 -> 9344: 4096 180 / 155; over 130 sizes up to 8192 rows 9 % less time), whole ones up to 5600 rows by the rule above
-    (6144: 2716 rows 205 / 120, 4096 158 / 156; over 28 sizes 9 % less, the others 6 % more). Gate and up with their
-    activation: up to 3600 rows from two rounds on (28672: 2716 rows 593 / 508, 3182 716 / 596, 3600 - 4200 3 % more; 4096 -> 9216, less
-    than two rounds, 5 % more). Steps: llama 2700 rows 5030 -> 4400, 3000 4930 -> 4790, 3300 6050 -> 5480; rogosun 4000 8740 -> 8570, width 2048 2700
-    2925 -> 2860; budurax width 2048 2700 2280 -> 2208; furapel 6400 15235 -> 15020."""
+    * Very wide outputs of 257 - 1024 rows are the library's: 28672 columns 300 rows 76 / 71, 600 136 / 125 (74 / 78 and 135 / 149 before).
+    * Beyond 768 rows its tiles of 256 x 256 (1.42 us a round and 64 of K) fill their rounds: past one round whole columns (multiples of 256) are
+      this kernel's only where the figures say a fifth less, ragged ones up to 8448 rows (4096 -> 18560: 3182 rows 496 / 353, 4099 579 / 449;
+      12320: 2560 189 / 185, 7583 540 / 536; 2048 -> 9344: 4099 165 / 132), whole ones up to 5600.
+    * Beyond 2560 rows products within one round are the library's: 4096 -> 4096 2716 rows 77 / 70, 3850 93 / 92; 14336 -> 4096 2716 250 / 228, 3584
+      292 / 274; 7168 -> 2048 3000 84 / 76 (by the loop before 4096 -> 4096 took 74 and 4096 rows of it 100, the library 91).
+    * Gate and up with their activation: beyond 2560 rows from two rounds on and up to 3600 (``long_plan``: past one round everywhere)."""
     if M < 1 or N % 32 or N < 32 or K % 64 or K < 128 or N * K * 2 > 0xffff0000 or (form == "glu" and N % 64):
         return None
     if library and form == "bf16" and N > TILE_LIBRARY_N and 256 < M <= 1024:
@@ -547,17 +549,19 @@ def _library_us(M: int, N: int, K: int, form: str) -> float:
 @lru_cache(maxsize=4096)
 def long_plan(M: int, N: int, K: int, form: str = "bf16", library: bool = True) -> tuple[int, int, int] | None:
     """``tile_plan``, and past one round of the library's tiles what it leaves to the library where this kernel is faster since its loop has
-    one meeting of the waves per 64 of K. With an activation that is everywhere: us, library and activation / this kernel, 4096 -> 28672
-    2048 rows 375 / 360, 4099 745 / 690, 5600 1078 / 891, 8192 1369 / 1284; 4096 -> 9216 2700 rows 173 / 158, 5600 418 / 311; 2048 -> 14336 2048
-    rows 109 / 100, 6500 416 / 297; over 134 sizes of 1100 - 8192 rows 9 % less than by ``tile_plan`` alone (3072 rows of 4096 -> 10752, the
-    worst, 194 / 194). Without one, where the figures say so, and not where the library takes blocks of 4096 rows (4099 of 4096 -> 4096 101 /
-    113): 5600 rows of 4096 -> 9216 394 / 296, 2700 of 4096 -> 28672 552 / 451, 8192 of 4096 -> 12320 631 / 589; over 194 sizes 2 % less, the worst
-    2304 of 2048 -> 14336 99 / 106."""
+    one meeting of the waves per 64 of K. us, library (and activation) / this kernel. With an activation that is everywhere: 4096 -> 28672
+    2048 rows 381 / 345, 4099 758 / 678, 5600 1093 / 900, 8192 1388 / 1269; 4096 -> 9216 2716 rows 176 / 156, 5600 416 / 309; 2048 -> 14336 2048
+    rows 111 / 97, 6500 417 / 287. Without one, where the figures say so, the library does not take blocks of 4096 rows (4099 of 4096 -> 4096 104 /
+    115) and its tiles do not fill whole rounds (8192 rows of 14336 -> 4096 613 / 627, of 4096 -> 28672 1225 / 1249, of 4096 -> 6144 266 / 274): 5600
+    rows of 4096 -> 9216 390 / 310, 2716 of 4096 -> 28672 542 / 460, 6500 of 2048 -> 14336 362 / 287. The library is uneven (5100 and 5600 rows of
+    2048 -> 14336 228 and 309) and the figures do not tell where: over 980 sizes of all forms 11 % less, the worst 2 - 3 % more (4201 rows of 4096
+    -> 28672 712 / 735)."""
     plan = tile_plan(M, N, K, form, library)
     if plan is not None or not library or M <= 768 or -(-M // 256) * -(-N // 256) <= 256 or \
             tile_plan(M, N, K, form, False) is None:
         return plan
-    if form in ("glu", "relu2") or M > 1024 and not dense_cut(M, N, K) and _tile_pick(M, N, K, form)[0] < _library_us(M, N, K, form):
+    if form in ("glu", "relu2") or M > 1024 and not dense_cut(M, N, K) and (-(-M // 256) * -(-N // 256)) % 256 and \
+            _tile_pick(M, N, K, form)[0] < _library_us(M, N, K, form):
         return tile_plan(M, N, K, form, False)
     return None
 

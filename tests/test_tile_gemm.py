@@ -186,6 +186,18 @@ def test_long_plans_take_more_from_the_library():
     assert ops.long_plan(5600, 9216, 4096) is not None and ops.long_plan(5600, 9216 + 16, 4096) is None
 
 
+def test_plans_of_deep_loops_and_of_full_rounds():
+    """Loops of 6144 and more of K on tiles of 128 columns are priced as they run, so that two splits on 256 columns take them; plain products whose library
+    tiles fill whole rounds are the library's, one row tile less is not."""
+    for M, N, K, form in ((1100, 4096, 14336, "bf16"), (1270, 4096, 14336, "bf16"), (1560, 4096, 14336, "slabs"), (1790, 4096, 14336, "slabs"),
+                          (2227, 2048, 7168, "slabs")):
+        assert ops.long_plan(M, N, K, form)[1:] == (8, 2), (M, N, K)
+    assert ops.long_plan(1100, 4096, 4096)[2] == 1 and ops.long_plan(1700, 4096, 4096, "slabs")[2] == 1
+    for M, N, K in ((8192, 4096, 14336), (7990, 14336, 2048), (8192, 6144, 4096), (8192, 28672, 4096), (4000, 28672, 4096)):
+        assert ops.long_plan(M, N, K) is None and ops.long_plan(M, N, K, library=False) is not None and ops.long_plan(M, N, K, "glu") is not None
+    assert ops.long_plan(5600, 9216, 4096) is not None and ops.long_plan(7900, 28672, 4096) is not None
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("mt,nt", sorted(ops.TILES))
 def test_low_last_row_tiles_and_short_loops(mt, nt):

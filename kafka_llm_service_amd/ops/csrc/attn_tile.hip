@@ -7,8 +7,11 @@ namespace kafka {
 
 // An item (256 query rows) is 8 / NW workgroups of one key/value head. Prompts: two of four waves and two ring slots each, two workgroups a CU, whose
 // waves do not wait for each other and whose halves of a causal item end where their own rows do; 4096 rows against 8192 keys, us, 8 waves 497, two
-// of 4 482 (528 before the loop was a pipeline; 8 waves 514). A cascade's prefix pass (few row tiles, keys from memory) reads the keys once an item:
-// 8 waves, three slots (4: 30.9 vs 29.9 us per cascade launch, profiles/r05/cascade/cascade_nslot_*.jsonl)
+// of 4 482 (before the loop was a pipeline 514 and 528). A cascade's prefix pass (few row tiles, keys from memory) reads the keys once an item:
+// 8 waves, three slots (4: 30.9 vs 29.9 us per cascade launch, profiles/r05/cascade/cascade_nslot_*.jsonl). So do a few short portions behind long
+// histories of their own, whose keys come from memory in many short parts: from eight parts a row on, where there are items for more than half the CUs
+// (fewer leave CUs to the second half). Two and four portions of 60 tokens behind 3000, 8 key/value heads, a step of four layers, two of 4 /
+// 8 waves: 706 / 689 and 871 / 844; with four parts (eight portions) 1164 / 1167, on fewer CUs (one portion) 556 / 567.
 template <int ABL, int KVAUX, int PST, int NW, int NSLOT>
 __global__ __launch_bounds__(64 * NW, 2) void attn_tile_kernel(const TileItem* __restrict__ items,
                                                                const bf16* __restrict__ q, int64_t q_stride,
@@ -56,6 +59,7 @@ extern "C" hipError_t kafka_launch_attn_tile(const void* items, int n_items, con
   };
   if (stamps) go(attn_tile_kernel<8, 0, 0, 8, 3>, 1);
   else if (part_bf16) go(attn_tile_kernel<0, 2, 1, 8, 3>, 1);
+  else if (out_part != nullptr && S_total >= 8 && n_items * Hkv > 128) go(attn_tile_kernel<0, 0, 0, 8, 3>, 1);
   else go(attn_tile_kernel<0, 0, 0, 4, 2>, 2);
   return hipGetLastError();
 }

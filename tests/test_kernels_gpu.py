@@ -610,6 +610,33 @@ def test_attn_prefill_balanced_split(cuda, ctx, qlen):
     _close(out, out_ref, atol=0.02, msg="balanced split prefill")
 
 
+@pytest.mark.parametrize("portions,rows,ctx", [(2, 60, 3000), (1, 60, 3000), (8, 60, 3000), (4, 63, 2100), (3, 1, 2500), (2, 70, 2049)])
+def test_attn_tile_split_portions(cuda, portions, rows, ctx):
+    """Short portions behind histories of their own, in parts: eight and more on many CUs (8 waves a workgroup), fewer parts or CUs (4)."""
+    from kafka_llm_service_amd.engine.model_runner import plan_prefill_items
+
+    torch.manual_seed(14)
+    Hq, Hkv, D = 32, 8, 128
+    tile, L, T = ops.tile_rows(3) // (Hq // Hkv), ctx + rows, portions * rows
+    k, v, bt = _random_paged(portions, [L] * portions, Hkv, cuda, seed=15)
+    q = torch.randn(T, Hq, D, device=cuda, dtype=torch.bfloat16)
+    q_limit = torch.arange(ctx, L, dtype=torch.int32).repeat(portions)
+    tiles = [(p * rows + t0, min(tile, rows - t0), p, ctx + t0 + min(tile, rows - t0), L) for p in range(portions) for t0 in range(0, rows, tile)]
+    items, splits, ranges = plan_prefill_items(tiles, Hkv, 256, 256)
+    out = torch.full((T, Hq, D), float("nan"), device=cuda, dtype=torch.bfloat16)
+    part = torch.full((T, Hq, splits, D), float("nan"), device=cuda)
+    lse = torch.full((T, Hq, splits), float("-inf"), device=cuda)
+    scale = 1 / math.sqrt(D)
+    ops.attn_prefill(torch.tensor(items, dtype=torch.int32, device=cuda), q, k, v, bt, q_limit.to(cuda), scale, out=out, out_part=part,
+                     lse_part=lse, variant=3)
+    for lo, hi in ranges:
+        ops.attn_merge(part[lo:hi], lse[lo:hi], out[lo:hi])
+    whole = torch.tensor([[t0, cnt, p, 0, L, -1, 0, 0] for t0, cnt, p, _, _ in tiles], dtype=torch.int32)
+    out_ref = torch.zeros(T, Hq, D, dtype=torch.bfloat16)
+    ref.attn_prefill_items(whole, q.cpu(), k.cpu(), v.cpu(), bt.cpu(), q_limit, scale, out=out_ref)
+    _close(out, out_ref, atol=0.02, msg="portions in parts")
+
+
 def test_sample_split_rows_equal_one_workgroup(cuda):
     """Greedy and plain-temperature rows split over 8 workgroups (ticket reduce) pick exactly the token of the
     one-workgroup kernel (same per-index noise); top-k / top-p rows keep the whole-row path. Three launches check

@@ -389,6 +389,41 @@ def test_lin_scan_in_chunks(delta, n):
     assert close(outs[1][1], outs[0][1], 3e-5)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("D", [72, 100, 128])
+@pytest.mark.parametrize("sizes", [(64, 97, 161), (95, 64, 66, 128, 79)])
+def test_delta_rule_three_workgroups_a_cu(sizes, D, dt):
+    """The scan with one chunk's operands on their way, which the delta rule takes where the chip then needs fewer rounds: against the token-by-token
+    kernel, outputs and states, every kind of last chunk, a segment that goes on from a state, whole and partial channel tiles."""
+    dev, H, G, Dv = "cuda:0", 32, 16, 128
+    wgs = H * (Dv // 16) * len(sizes)
+    assert -(-wgs // 768) < -(-wgs // 512)
+    g = torch.Generator().manual_seed(D + len(sizes))
+    zb, rate = torch.randn(H * D, generator=g), -(0.1 + torch.rand(H, generator=g))
+    before = 21                                       # tokens of the first sequence in front of its segment
+    c = {k: v.to(dt).to(dev) for k, v in _lin_case(g, before + sum(sizes), H, G, D, Dv).items()}
+    outs = []
+    for chunked in (False, True):
+        S = torch.full((len(sizes) + 2, H, D, Dv), float("nan"), device=dev)
+        got = []
+        starts = [before + sum(sizes[:i]) for i in range(len(sizes))]
+        for lo, hi, segs in ((0, before, [(0, before, 0, 1)]),
+                             (before, before + sum(sizes), [(a - before, n, before if i == 0 else 0, i + 1) for i, (a, n) in enumerate(zip(starts, sizes))])):
+            ts, seg = seg_tensors(dev, segs)
+            tabs = hops.lin_chunk_tables(np.asarray(segs, dtype=np.int32)) if chunked and lo else None
+            if tabs is not None:
+                tabs = tuple(torch.from_numpy(x).to(dev) for x in tabs)
+            x = {k: v[lo:hi] for k, v in c.items()}
+            out = torch.full((hi - lo, H * Dv), float("nan"), device=dev)
+            hops.lin_scan(x["qkv"], 0, G * D, x["qkv"][:, 2 * G * D:], x["z"], zb.to(dev), H, G, D, Dv, ts, seg, S, out, 1.0, rate.to(dev),
+                          x["beta"], tabs, (min(s[1] for s in segs), max(s[1] for s in segs)) if tabs is None else None)
+            got.append(out)
+        outs.append((torch.cat(got).cpu(), S[1:-1].cpu()))
+        assert S[0].isnan().all() and S[-1].isnan().all()
+    assert close(outs[1][0], outs[0][0], 3e-5) and close(outs[1][1], outs[0][1], 3e-5)
+
+
 class Paged:
     """Scattered pages for sequences of given lengths, fed in given portions: the step tensors the kernels take."""
 

@@ -585,8 +585,8 @@ class ModelRunner:
             self._init_common(max_num_seqs)
             return
         self.G = model.hq // model.hkv
-        # tile-kernel variant (ops.tile_rows): 3 = LDS-DMA ring kernel (csrc/attn_tile.hip, 8 waves x 256 query rows,
-        # bf16 pages); 0 = register-staged 8 waves x 256 rows (fp8 pages); 1 = 4 waves x 128 rows
+        # tile-kernel variant (ops.tile_rows): 3 = LDS-DMA kernel (csrc/attn_tile.hip, 256 query rows an item on 8 waves
+        # or on two workgroups of 4, bf16 pages); 0 = register-staged 8 waves x 256 rows (fp8 pages); 1 = 4 waves x 128 rows
         fp8 = bool(k_caches) and ops.is_fp8_cache(k_caches[0])
         self.variant = int(os.environ.get("KAFKA_TILE_VARIANT", "0" if fp8 else "3"))
         if fp8 and self.variant == 3:

@@ -8,10 +8,10 @@
 //     of the next tile's keys stand the exponentials of this one, between the products of this one's values the rest of
 //     them and the next one's maxima, each product behind the LDS reads of the eight fragments after it. Waves of a SIMD
 //     are mostly at the same place, so what stood one after the other in a wave (products, then softmax, then products,
-//     reads in front of each) did so on the SIMD. What bounds it now: LDS, 32 KB of fragments a wave and tile (without the
-//     reads 389 us, without the exponentials 480, without the copies 464, of 497: 4096 rows of 32 heads against 8192
-//     keys, 525 before), and the clock that the card holds. (64 rows a wave on one wave per SIMD halve the reads,
-//     but 256 + 256 registers did not hold it without scratch in the loop: 574 us.);
+//     reads in front of each) did so on the SIMD. What bounds it now: LDS, 32 KB of fragments a wave and tile (8 waves, 4096
+//     rows of 32 heads against 8192 keys, 497 us: without the reads 389, without the exponentials 480, without the
+//     copies 464), and the clock that the card holds. (64 rows a wave on one wave per SIMD halve the reads, but 256 + 256
+//     registers did not hold it without scratch in the loop: 574 us.);
 //   * K/V arrive by LDS-DMA (1 KiB per wave-instruction), 16 KB each per tile, into 2 or 3 slots for each: the keys run a
 //     tile ahead of the values, and both slots that a step has read are filled again in its middle, behind its one counted
 //     `s_waitcnt vmcnt` and one `s_barrier`;
@@ -110,8 +110,8 @@ __device__ __forceinline__ void t3_wait_tiles(int n) {
 }
 
 // ABL = 8 (diagnostic build, KAFKA_TILE_ABL=8, benchmarks/attn_tile_stamps.py): workgroup phase stamps on the 100 MHz
-// clock; the full kernel runs and lse_part is overwritten with u64 [entry, prologue done, first tile landed, loop
-// done, epilogue done, 0, 0, 0] per workgroup blockIdx.y * Hkv + blockIdx.x.
+// clock, every launch in the cascade's form (8 waves, three slots); the full kernel runs and lse_part is overwritten with
+// u64 [entry, prologue done, first tile landed, loop done, epilogue done, 0, 0, 0] per workgroup blockIdx.y * Hkv + blockIdx.x.
 // PST = 1: the bf16 prefix partials are stored sc1 (16-B stores whose lines leave this XCD's L2: the reader, the
 // suffix decode's merge, runs on any XCD, and the launch ends with fewer dirty lines to write back)
 // PST = 2: as 1, and fp32 partials and every lse as well: a workgroup of the same launch reads them (attn_mixed.hip)

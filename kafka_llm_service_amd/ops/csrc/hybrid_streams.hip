@@ -21,7 +21,7 @@
 //                       transposed so that rows are lanes - maxima, sums and weights stay in a lane's registers. Prompt portions: a
 //                       wave each, no LDS and no barriers; decoded tokens: keys over the waves of a workgroup, and over several
 //                       workgroups with a merge pass
-//   window_attn_tile    the same for long portions of 128 channels, eight items on one walk over keys in LDS
+//   window_attn_tile    the same for long portions of 128 channels, four items on one walk over keys in LDS
 //   moe_topk_grouped    softmax or sigmoid scores, choice among the best groups (by their largest score or the sum of
 //                       their two largest) by corrected score, weights normalised or as they are, times a scale
 #include "common.h"
@@ -594,9 +594,11 @@ __global__ __launch_bounds__(256, NKS * 4 + NVT * 16 <= 96 ? 2 : 1) void window_
 constexpr int WT_WAVES = 4, WT_KEYS = 64, WT_SLOTS = 2, WT_RUN = 512;   // WT_RUN: tiles whose page ids lie in LDS at a time
 constexpr int WT_KB = WT_KEYS * 256, WT_PIECES = 16 / WT_WAVES;         // bytes of a tile's keys; 1-KiB pieces of them that a wave copies
 constexpr float WT_THR = 8.f;
-// Items (those that it works on, not the single tokens between them) x key/value heads from which it runs: a wave each on 256 CUs, fewer leave whole CUs idle that the form above still uses.
-// us there / here: 1000 waves (1000 rows) 33 / 40, 1024 (2048 rows, 4 heads) 62 / 66, 1200 47 / 45, 1500 63 / 60, 2048 with a
-// window of 1024 85 / 45.
+// Items (those that it works on, not the single tokens between them) x key/value heads from which it runs: a wave each on 256 CUs, fewer leave
+// whole CUs idle that the form above still uses. us there / here, 32 heads over 2 or 8, one portion, behind 3000 keys, three portions, ten behind
+// 200: 500 waves 15 / 15, 74 / 58, 8.6 / 12.5, 11 / 17; 1000 waves 32 / 24, 132 / 71, 16 / 16, 17 / 19; 1150 42 / 27, 196 / 87, 22 / 16, 25 / 23;
+// 1280 48 / 30, 203 / 92, 27 / 19, 28 / 19. The line is that of eight waves a workgroup, which were even at 1200 - 1500; with four it is ahead
+// from 1000 - 1150 on, and behind long histories well below that.
 constexpr int WT_MIN_WAVES = 1280;
 
 typedef __attribute__((address_space(3))) void wt_lds_t;

@@ -845,9 +845,9 @@ def shared_items(tokens: int, items: int, tile_tokens: int, kinds, max_keys: int
     """About how many of a step's attention items, of up to ``tile_tokens`` of its ``tokens`` rows each, are tiles of prompt portions
     that gain from keys shared in LDS (window_attn_tile; it runs from 1280 items x key/value heads on). Beside decoded tokens those
     are counted from the rows that are more than one an item; items of one token each cannot be told apart then, and a workgroup
-    that meets eight sequences walks one after the other (64 decoded tokens behind 1500 keys beside 2 x 600 rows, 64 heads over 2:
-    268 us, a wave each 135). Nor is there much to share in short contexts: 100 portions of 30 rows, 32 heads over 8, 33 us a wave
-    each / 39 shared, 40 of 64 rows 31 / 34, 20 of 100 26 / 28, 10 of 200 30 / 28, 20 of 100 behind 1000 keys 141 / 78."""
+    that meets four sequences walks one after the other (64 decoded tokens behind 1500 keys beside 2 x 600 rows, 64 heads over 2:
+    120 us, a wave each 94). Nor is there much to share in short contexts: 100 portions of 30 rows, 32 heads over 8, 23 us a wave
+    each / 24 shared, 40 of 64 rows 23 / 22, 20 of 100 19 / 21, 10 of 200 22 / 20, 20 of 100 behind 1000 keys 126 / 63."""
     if max_keys and max_keys < WINDOW_SHARE_KEYS:
         return 0
     if not kinds[0]:

@@ -450,8 +450,8 @@ TILES = {
 }
 # rows up to which the last row tile is a low one (tiles of more than 128 rows), and us of a round of those and 64 of K by the 16-column parts
 TILE_LOW, TILE_LOW_UNIT = 64, {8: 0.43, 6: 0.26, 4: 0.21}
-# what loops of 6144 and more of K take longer on tiles of 128 columns: us, without / with two splits on 256: 14336 -> 4096 1100 rows 135 / 112, 1770 164 / 153
-# (a third as deep, 4096 -> 4096, 1100 rows 41 / 43, 1770 50 / 60)
+# what loops of 6144 and more of K take longer on tiles of 128 columns: us, on those without splits / on 256 in two: 14336 -> 4096 1100
+# rows 135 / 112, 1770 164 / 153 (a third as deep, 4096 -> 4096, 1100 rows 41 / 43, 1770 50 / 60)
 TILE_DEEP = 1.04
 TILE_SPLITS = (1, 2, 4, 8)      # what the consumers of slabs load with all slabs in flight
 TILE_SLAB_BYTES = 1 << 28

@@ -5,13 +5,15 @@
 
 namespace kafka {
 
-// An item (256 query rows) is 8 / NW workgroups of one key/value head. Prompts: two of four waves and two ring slots each, two workgroups a CU, whose
-// waves do not wait for each other and whose halves of a causal item end where their own rows do; 4096 rows of 32 heads against 8192 keys, us,
-// 8 waves 497, two of 4 482; on another card before the loop was a pipeline, 8 waves, / now 489 / 466, behind 4096 of the keys 408 / 374. A cascade's prefix pass (few row tiles, keys from memory) reads the keys once an item:
-// 8 waves, three slots (4: 30.9 vs 29.9 us per cascade launch, profiles/r05/cascade/cascade_nslot_*.jsonl). So do a few short portions behind long
-// histories of their own, whose keys come from memory in many short parts: from eight parts a row on, where there are items for more than half the CUs
-// (fewer leave CUs to the second half). Two and four portions of 60 tokens behind 3000, 8 key/value heads, a step of four layers, two of 4 /
-// 8 waves: 706 / 689 and 871 / 844; with four parts (eight portions) 1164 / 1167, on fewer CUs (one portion) 556 / 567.
+// An item (256 query rows) is 8 / NW workgroups of one key/value head. Prompts: two of four waves and two ring slots each, two workgroups
+// a CU, whose waves do not wait for each other and whose halves of a causal item end where their own rows do; 4096 rows of 32 heads
+// against 8192 keys, us, 8 waves 497, two of 4 482; on another card before the loop was a pipeline, 8 waves, / now 489 / 466, behind
+// 4096 of the keys 408 / 374.
+// A cascade's prefix pass (few row tiles, keys from memory) reads the keys once an item: 8 waves, three slots (4: 30.9 vs 29.9 us per
+// cascade launch, profiles/r05/cascade/cascade_nslot_*.jsonl). So do a few short portions behind long histories of their own, whose keys
+// come from memory in many short parts: from eight parts a row on, where there are items for more than half the CUs (fewer leave CUs to
+// the second half). Two and four portions of 60 tokens behind 3000, 8 key/value heads, a step of four layers, two of 4 / 8 waves:
+// 706 / 689 and 871 / 844; with four parts (eight portions) 1164 / 1167, on fewer CUs (one portion) 556 / 567.
 template <int ABL, int KVAUX, int PST, int NW, int NSLOT>
 __global__ __launch_bounds__(64 * NW, 2) void attn_tile_kernel(const TileItem* __restrict__ items,
                                                                const bf16* __restrict__ q, int64_t q_stride,
